@@ -96,3 +96,37 @@ def test_projection_reads_and_writes_stay_inside_its_views(T, K, nq, nkv, D):
     for (buf, view), w in zip(outs, want):
         close(view, w[0])
         assert torch.isnan(buf[0]).all() and torch.isnan(buf[T + 1]).all() and torch.isnan(buf[:, view.shape[1]:]).all()
+
+
+# tokens, hidden, columns of Q and of K and V, head_dim, and the tile that the launcher's rule picks: 64 x 64 tiles up to
+# 256 of them, 128 x 64 and then 128 x 128 likewise, two 128 x 128 per CU beyond
+@pytest.mark.parametrize("T,K,nq,nkv,D", [(33, 64, 64, 64, 64), (64, 200, 128, 64, 64), (65, 328, 192, 128, 64),       # 64 x 64
+                                         (100, 1024, 4096, 1024, 128), (128, 8, 72, 8, 8),
+                                         (190, 136, 5504, 256, 128), (256, 264, 6144, 1024, 128),                   # 128 x 64
+                                         (385, 136, 6144, 1024, 128), (512, 72, 6144, 1024, 128),                   # 128 x 128
+                                         (700, 72, 6144, 1024, 128)])                                               # two per CU
+@pytest.mark.parametrize("norm", [False, "plain", "gamma"])
+def test_projection_tilings_between_decode_and_long_prompts(T, K, nq, nkv, D, norm):
+    """Edges of each tile (tokens, columns, ragged hidden, fewer k-tiles than ring stages) with operands cut out of
+    NaN-filled buffers and outputs checked for strays.  Tolerance: one fp16 rounding of the output and, with gamma, one of
+    each product gamma * w: 3.6e-4 of the output's spread measured and expected, so 8e-3 of it is more than 20 sigma."""
+    from triton_amd import ops
+    g = torch.Generator().manual_seed(T + K)
+    nan = float("nan")
+    x, ws = ref.randn_half((T, K), g), weights(g, K, nq, nkv, K ** -0.5)
+    gamma = ref.randn_half((K,), g, 1.0, 0.02) if norm == "gamma" else None
+
+    def padded(t):
+        b = torch.full((t.shape[0] + 2, t.shape[1] + 16), nan, dtype=torch.float16, device="cuda")
+        b[1:-1, 8:-8] = t.cuda()
+        return b[1:-1, 8:-8]
+    bufs = [torch.full((T + 2, n + 16), nan, dtype=torch.float16, device="cuda") for n in (nq, nkv, nkv)]
+    outs = [b[1:-1, 8:-8].unflatten(1, (n // D, D)).permute(1, 0, 2) for b, n in zip(bufs, (nq, nkv, nkv))]
+    ops.prenorm_qkv(padded(x), gamma.cuda() if gamma is not None else None, *[padded(w) for w in ws], *outs, 1e-5, bool(norm))
+    torch.cuda.synchronize()
+    one = torch.ones(K, dtype=torch.float16)
+    want = ref.qkv_project(x[None], gamma if gamma is not None else one, *ws, 1e-5, bool(norm))
+    for b, w in zip(bufs, want):
+        close(b[1:-1, 8:-8], w[0], atol=8e-3 * float(w.float().std()), rtol=1e-3)
+        b[1:-1, 8:-8] = nan
+        assert torch.isnan(b).all(), "written outside the output"

@@ -28,10 +28,15 @@ __device__ __forceinline__ int wswz(int r) { return ((r & 3) << 2) | ((r >> 2) &
 int launch_prenorm_qkv_wide(GemmArgs a, hipStream_t stream);
 int64_t prenorm_qkv_wide_tiles(const GemmArgs& a);
 
-// At most 32 tokens: 64-column panels streamed by four waves that split the contraction (prenorm_qkv_skinny.hip).
+// At most 32 tokens: 64-column panels streamed by eight waves that split the contraction (prenorm_qkv_skinny.hip).
 int launch_prenorm_qkv_skinny(GemmArgs a, hipStream_t stream);
 
-// The 128 x 128 tiling and the choice between the three (prenorm_qkv.hip).
+// 64 x 64, 128 x 64 or 128 x 128 tiles (tokens x columns) whose waves split the contraction, for problems that leave the
+// larger tilings with fewer tiles than CUs (prenorm_qkv_mid.hip); the number of such tiles.
+int launch_prenorm_qkv_mid(const GemmArgs& a, int mt, int nt, hipStream_t stream);
+int64_t prenorm_qkv_mid_tiles(const GemmArgs& a, int mt, int nt);
+
+// The 128 x 128 tiling with two workgroups per CU, and the choice between them all (prenorm_qkv.hip).
 int launch_projections(GemmArgs a, hipStream_t stream);
 
 }  // namespace trn

@@ -219,9 +219,15 @@ __global__ __launch_bounds__(256, 2) void prenorm_qkv_kernel(const GemmArgs a) {
 int launch_projections(GemmArgs a, hipStream_t stream) {
     // a handful of tokens (decode): the weight stream is everything
     if (a.T <= 32) return launch_prenorm_qkv_skinny(a, stream);
-    // 256-token tiles once they alone occupy at least half of the 256 CUs; 128 x 128 tiles below that (short
-    // prefills, where the number of workgroups matters more than the work per staged byte)
+    // 256-token tiles once they alone occupy at least half of the 256 CUs
     if (prenorm_qkv_wide_tiles(a) >= 128) return launch_prenorm_qkv_wide(a, stream);
+    // Below that, the smallest tile that still gives every CU at most one: a tile's time is its chain of k-tiles, nearly
+    // the same for all of them up to one per CU, and half as much again or more with a second one beside it (4096 -> 6144,
+    // us 64 x 64 / 128 x 64 / 128 x 128: 100 tokens 25 / 33 / 46, 256 tokens 45 / 37 / 47, 512 tokens 65 / 62 / 48).  When
+    // even 128 x 128 tiles exceed the CUs, the kernel of this file takes them two per CU (768 tokens 76 against 87 us).
+    if (prenorm_qkv_mid_tiles(a, 64, 64) <= 256) return launch_prenorm_qkv_mid(a, 64, 64, stream);
+    if (prenorm_qkv_mid_tiles(a, 128, 64) <= 256) return launch_prenorm_qkv_mid(a, 128, 64, stream);
+    if (prenorm_qkv_mid_tiles(a, 128, 128) <= 256) return launch_prenorm_qkv_mid(a, 128, 128, stream);
     a.n_mtiles = (a.T + GBM - 1) / GBM;
     int t0 = 0;
     for (int i = 0; i < 3; ++i) { a.p[i].tile0 = t0; t0 += (a.p[i].n + GBN - 1) / GBN; }
