@@ -130,3 +130,20 @@ def test_projection_tilings_between_decode_and_long_prompts(T, K, nq, nkv, D, no
         close(b[1:-1, 8:-8], w[0], atol=8e-3 * float(w.float().std()), rtol=1e-3)
         b[1:-1, 8:-8] = nan
         assert torch.isnan(b).all(), "written outside the output"
+
+
+@pytest.mark.parametrize("T", [1, 16, 17, 24, 25, 32])
+@pytest.mark.parametrize("K", [8, 64, 264, 1000])
+def test_weight_stream_at_token_and_hidden_edges(T, K):
+    """The three token groups of the decode tiling and contractions from less than one k-tile to several turns of the
+    eight waves, norm with gamma, ragged panels; tolerance as above."""
+    from triton_amd import ops
+    g = torch.Generator().manual_seed(T * K)
+    x, gamma = ref.randn_half((T, K), g), ref.randn_half((K,), g, 1.0, 0.02)
+    ws = weights(g, K, 200, 72, K ** -0.5)
+    outs = [torch.zeros(T, n, dtype=torch.float16, device="cuda") for n in (200, 72, 72)]
+    ops.prenorm_qkv(x.cuda(), gamma.cuda(), *[w.cuda() for w in ws],
+                    *[o.unflatten(1, (-1, 8)).permute(1, 0, 2) for o in outs], 1e-5, True)
+    torch.cuda.synchronize()
+    for o, w in zip(outs, ref.qkv_project(x[None], gamma, *ws, 1e-5, True)):
+        close(o, w[0], atol=8e-3 * float(w.float().std()), rtol=1e-3)
