@@ -16,7 +16,7 @@ struct AttnArgs {
     // decode kernel only: keys split over n_split workgroups per head, partial results and arrival counters in ws
     int n_split;
     float* ws;
-    // decode kernel only, one workgroup per head: per-key sums (and sums of squares) of the probabilities -- of the
+    // decode kernel only, at most 32 queries: per-key sums (and sums of squares) of the probabilities -- of the
     // perturbed ones when noise is given -- from a second sweep over the keys once the row normalisers are final
     float* col_sum; float* col_sumsq;
     // ... and the probabilities themselves, un-reduced: float [B, Hq, Sq, Skv] contiguous
@@ -31,9 +31,11 @@ int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const voi
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
                  bool io16 = false);
 
-// At most 32 queries per head (decode): one workgroup per head whose eight waves split the keys (attn_decode.hip).
+// One workgroup per head and 32 queries, whose eight waves split the keys (attn_decode.hip): at most 32 queries per head
+// (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.
+bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t workspace_bytes, hipStream_t stream);
-const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_kv, int head_dim, bool noise);
+const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 // Bytes of workspace with which launch_attn_decode splits the keys of this problem over several workgroups (0: it would not).
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);
 

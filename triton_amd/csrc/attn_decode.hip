@@ -1,7 +1,8 @@
-// Attention forward for at most 32 queries per head (decode-append: a few new tokens against a long cache).
+// Attention forward for at most 32 queries per head (decode-append: a few new tokens against a long cache), and for more
+// of them where tiles of 32 queries are what it takes to occupy the chip (attn_decode_suits).
 //
 // With so few queries there is one 32-query MFMA block per head and the kernel is a stream of K and V through HBM.
-// One workgroup per (batch, head); its eight waves take the 32-key blocks round-robin, each with its own running
+// One workgroup per (batch, head, 32-query tile); its eight waves take the 32-key blocks round-robin, each with its own running
 // max / normaliser / O^T accumulator, and the eight partial results are merged through LDS at the end (the usual
 // log-sum-exp merge).  Formulation and register layouts are those of the prefill kernel: S^T = K Q^T with Q^T
 // resident in registers, P^T taken from the S^T accumulator, V^T via the transposing LDS read.  K rows are what the
@@ -60,19 +61,20 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // workgroup id -> (batch x head j, key share, column share).  The column shares of a head read the same K: their
     // ids are 8 apart, so that they sit on one XCD (ids are dealt to the 8 XCDs in turn) and share its L2.
-    int j, split, dsl;
-    if constexpr (DS > 1) {
-        const int grp = blockIdx.x / (8 * DS), rem = blockIdx.x % (8 * DS);
-        j = grp * 8 + rem % 8; dsl = rem / 8; split = 0;
+    // So do the query tiles of a head; the last one, with the most keys under a causal mask, comes first.
+    int j, split = 0, dsl = 0, q0 = 0;
+    if (DS > 1 || a.n_qtiles > 1) {
+        const int per_grp = 8 * DS * a.n_qtiles, grp = blockIdx.x / per_grp, rem = blockIdx.x % per_grp;
+        j = grp * 8 + rem % 8; dsl = rem / 8 % DS; q0 = 32 * (a.n_qtiles - 1 - rem / (8 * DS));
         if (j >= a.B * a.Hq) return;                    // the last group of eight heads may be short
     } else {
-        j = blockIdx.x / a.n_split; split = blockIdx.x % a.n_split; dsl = 0;
+        j = blockIdx.x / a.n_split; split = blockIdx.x % a.n_split;
     }
     const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
     const int kvslot = j % nkv, g = j / nkv;
     const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
     const int off = a.Skv - a.Sq;                       // causal: query i sees keys <= i + off
-    const int qrow = c;                                 // this lane's query
+    const int qrow = q0 + c;                            // this lane's query
     const int qrow_ld = qrow < a.Sq ? qrow : a.Sq - 1;
 
     // ---- Q^T B-operands: lane holds Q[qrow][ks*16 + 8h .. +7]; optional fused per-head RMSNorm of the row
@@ -173,7 +175,9 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     };
 
     // this workgroup's blocks: a contiguous share of the keys when they are split over several workgroups
-    const int nblk_all = (a.Skv + 31) / 32, bps = (nblk_all + a.n_split - 1) / a.n_split;
+    int visible = a.Skv;                                // keys that some query of the tile sees
+    if (a.causal) visible = min(visible, min(q0 + 31, a.Sq - 1) + off + 1);
+    const int nblk_all = (visible + 31) / 32, bps = (nblk_all + a.n_split - 1) / a.n_split;
     const int blk0 = split * bps, nblk = max(0, min(nblk_all, blk0 + bps) - blk0);
     const int nmine = nblk > wave ? (nblk - wave + DNW - 1) / DNW : 0;          // blocks blk0 + wave, + 8, ...
     half8_t ka0[NS], ka1[NS];
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         for (int ks = 0; ks < NS; ++ks) s = mfma32(kc[ks], qB[ks], s);
         if constexpr (NOISE) fetch_k(blk + DNW, kc);
         // mask (wave-uniform test), block max, running max, probabilities
-        const bool masked = (key0 + 32 > a.Skv) || (a.causal && key0 + 31 > off);
+        const bool masked = (key0 + 32 > a.Skv) || (a.causal && key0 + 31 > q0 + off);
         if (masked) {
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -431,8 +435,8 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     }
     {
         const float inv = 1.0f / L;
-        half_t* orow = a.o + b * a.ob + head * a.oh + (int64_t)q * a.os + dsl * DV;
-        if (q < a.Sq) {
+        half_t* orow = a.o + b * a.ob + head * a.oh + (int64_t)(q0 + q) * a.os + dsl * DV;
+        if (q0 + q < a.Sq) {
 #pragma unroll
             for (int qi = 0; qi < NQD; ++qi) {
                 const half4_t ov = {(half_t)(acc[qi][0] * inv), (half_t)(acc[qi][1] * inv), (half_t)(acc[qi][2] * inv), (half_t)(acc[qi][3] * inv)};
@@ -440,16 +444,16 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
             }
         }
         // (every column share holds the same row normalisers: the first one writes them)
-        if (dg == 0 && dsl == 0 && q < a.Sq && a.lse) a.lse[(int64_t)bh * a.Sq + q] = (mstar + fast_log2(L)) * kLn2;
+        if (dg == 0 && dsl == 0 && q0 + q < a.Sq && a.lse) a.lse[(int64_t)bh * a.Sq + q0 + q] = (mstar + fast_log2(L)) * kLn2;
         if constexpr (NOISE) {
-            if (dg == 1 && dsl == 0 && q < a.Sq) a.lse_pert[(int64_t)bh * a.Sq + q] = (ms2 + fast_log2(L2)) * kLn2;
+            if (dg == 1 && dsl == 0 && q0 + q < a.Sq) a.lse_pert[(int64_t)bh * a.Sq + q0 + q] = (ms2 + fast_log2(L2)) * kLn2;
         }
     }
     // ---- column statistics (KeyFormer key scores, RoCo sums): a second sweep over this head's keys now that the
     // row normalisers are final.  The score block is formed the other way round, S[query][key] -- the same two
     // register operands with their roles swapped -- so that a lane owns one KEY and holds 16 of the 32 queries: the
     // sum over queries is in-lane plus one exchange with lane^32, and a block's 32 sums are one 128-byte store.
-    // (Not with the keys split over workgroups -- the statistics need the normalisers of the whole head; the column
+    // (One query tile only.  Not with the keys split over workgroups -- the statistics need the normalisers of the whole head; the column
     // shares of a head all have them, and take every DS-th round of blocks of the sweep each.)
     if (a.col_sum || a.col_sumsq || a.probs) {
         __syncthreads();                                   // every thread has read the merge arrays
@@ -549,16 +553,33 @@ int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq
     return ((n_bh + 63) / 64) * 256 + n_bh * ns * 32 * (head_dim + 4) * 4;
 }
 
-static int decode_col_shares(int64_t n_bh, int seq_kv, int head_dim) {
+// Column shares of a head for `units` = heads x query tiles: as many as leave 32 columns per workgroup and at most one
+// workgroup per CU.  (Two per CU do not fit, and a second round costs what the first did: 128 units of head_dim 128, us
+// 1 / 2 / 4 shares: 400 keys 10.3 / 8.7 / 13.7, 4100 keys 34 / 26 / 45.)
+static int decode_col_shares(int64_t units, int seq_q, int seq_kv, int head_dim) {
     int ds = 1;
-    if (seq_kv >= 256)
-        while (ds < 4 && head_dim / (ds * 2) >= 32 && n_bh * ds * 2 <= 256) ds *= 2;
+    if (seq_kv >= 256 || seq_q > 32)
+        while (ds < 4 && head_dim / (ds * 2) >= 32 && units * ds * 2 <= 256) ds *= 2;
     return ds;
 }
 
+// More than 32 queries per head: tiles of 32 queries, eight waves sharing out the keys of each, against the prefill
+// kernels' 128-query workgroups whose waves walk all the keys -- better as long as the tiles are no more than the CUs,
+// i.e. while the prefill kernels would leave most of the chip idle.  Measured, us prefill / here: 32 heads of 128: 100
+// queries on 4100 keys 63 / 26, on 400 12.6 / 8.7, causal 256 on 256 10.6 / 8.9 (256 tiles), causal 350 on 350 12.3 / 14.4
+// (352 tiles); 8 heads of 128, causal 777 on 777 17.6 / 12.2; 71 heads of 64: 64 queries on 4064 keys 41 / 19.  With more
+// tiles than CUs: head_dim 64 on long caches (71 heads, 100 queries: 4100 keys 42 / 35, 1124 keys 15.6 / 15.6, 164 keys
+// 6.8 / 10.2); with score perturbation, where the prefill kernel is slower, any (32 heads of 128, causal 350 on 350 22 /
+// 19; 71 heads of 64, 128 queries on 4128 keys 114 / 83; but 781 tiles 20 / 25).
+bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
+    if (seq_q <= 32) return true;
+    const int64_t tiles = (int64_t)batch * n_q_heads * ((seq_q + 31) / 32);
+    return tiles <= 256 || (tiles < 512 && (noise || (head_dim == 64 && seq_kv >= 1024)));
+}
+
 // Name of the instantiation launched for a problem without a workspace (a measurement aid: what a kernel trace shows).
-const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_kv, int head_dim, bool noise) {
-    const int ds = decode_col_shares((int64_t)batch * n_q_heads, seq_kv, head_dim);
+const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
+    const int ds = decode_col_shares((int64_t)batch * n_q_heads * ((seq_q + 31) / 32), seq_q, seq_kv, head_dim);
     if (head_dim == 128) {
         if (ds == 4) return noise ? "trn::attn_decode_kernel<128, 4, 1>" : "trn::attn_decode_kernel<128, 4, 0>";
         if (ds == 2) return noise ? "trn::attn_decode_kernel<128, 2, 1>" : "trn::attn_decode_kernel<128, 2, 0>";
@@ -576,11 +597,12 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
         a.ws = static_cast<float*>(workspace);
     }
     // Without a key split: share V's columns out over workgroups while that still leaves every workgroup 32 columns
-    // and the grid within one workgroup per CU (32 heads of 128: 4 shares; 71 heads of 64: 2).  Short caches are left
-    // alone: below some 8 blocks per wave-round the fixed part of a launch is all there is.
+    // and the grid within one workgroup per CU (32 heads of 128: 4 shares; 71 heads of 64: 2).  Few queries on a short
+    // cache are left alone: below some 8 blocks per wave-round the fixed part of a launch is all there is.
+    a.n_qtiles = (a.Sq + 31) / 32;
     const int64_t n_bh = (int64_t)a.B * a.Hq;
-    const int ds = a.n_split == 1 ? decode_col_shares(n_bh, a.Skv, head_dim) : 1;
-    const int64_t grid = ds > 1 ? ((n_bh + 7) / 8) * 8 * ds : n_bh * a.n_split;
+    const int ds = a.n_split == 1 ? decode_col_shares(n_bh * a.n_qtiles, a.Sq, a.Skv, head_dim) : 1;
+    const int64_t grid = ds > 1 || a.n_qtiles > 1 ? ((n_bh + 7) / 8) * 8 * ds * a.n_qtiles : n_bh * a.n_split;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)grid), t(DNW * 64);
 #define TRN_DEC(D_, DS_, N_) hipLaunchKernelGGL((attn_decode_kernel<D_, DS_, N_>), g, t, 0, stream, a)

@@ -432,7 +432,8 @@ extern "C" const char* trn_attn_fwd_kernel_name(const trn_attn_desc* d, int32_t 
     using namespace trn;
     if (!d || validate_attn(d, true) != TRN_OK) return "";
     const bool d128 = d->head_dim == 128;
-    if (d->seq_q <= 32) return attn_decode_kernel_name(d->batch, d->n_q_heads, d->seq_kv, d->head_dim, with_noise != 0);
+    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0))
+        return attn_decode_kernel_name(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
     if (!with_noise) return attn_fwd16_kernel_name(d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->head_dim, d->causal != 0));
     const bool wide = noise_kernel_wide(d);
     if (d128) return wide ? "trn::attn_fwd_kernel<128, 8, true>" : "trn::attn_fwd_kernel<128, 4, true>";
@@ -573,8 +574,8 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         return TRN_E_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
-    // a handful of queries per head (decode): one workgroup per head, its waves split the keys
-    if (d->seq_q <= 32)
+    // few queries per head (decode), or few query tiles in all: one workgroup per head and 32 queries, its waves split the keys
+    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, noise != nullptr))
         return launch_attn_decode(a, d->head_dim, workspace, workspace_bytes, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     // Without score perturbation: the 16x16x32 kernel, in the workgroup shape its launcher's rule picks.
     if (!noise)
