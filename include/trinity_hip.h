@@ -227,6 +227,23 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
                                 void* out_sum, void* out_sumsq, void* stream);
 
 /*
+ * Attention and per-key statistics for every shape and element type in one entry point: what the KeyFormer and RoCo
+ * modules call.  As trn_attn_fwd_stats_ws_f16 (one launch with at most 32 queries per head unless the workspace makes it
+ * split the keys, two launches otherwise), with
+ *   noise       nullable; fp16 when noise_half is set, float otherwise.  Rows at any pitch and any element alignment (the
+ *               reference's noise [.., M, P + M] is fp16 with any key count); desc's noise strides count elements.
+ *   rows        float [batch, n_q_heads, seq_q], required: receives the row normalisers of the scores the statistics are
+ *               of (perturbed with noise, plain without).
+ *   out1, out2  [batch, n_q_heads, seq_kv] contiguous, fp16 when out_half is set (the float result rounded once), float
+ *               otherwise: sum and sum of squares (one may be NULL) or, with mean_std (without noise; both required), mean
+ *               and standard deviation as trn_attn_colmeanstd_f16.
+ *   workspace   nullable: trn_attn_stats_workspace_bytes(desc) zero-initialised bytes, as trn_attn_fwd_stats_ws_f16.
+ */
+int trn_attn_key_scores_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v, void* o,
+                            const void* noise, int32_t noise_half, float* rows, void* out1, void* out2,
+                            int32_t out_half, int32_t mean_std, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * The decode-append form of KeyFormer as its reference class returns it (ref_rms.py:171-179): the attention output
  * and the UN-REDUCED probabilities  out_probs[b,h,i,j] = softmax_j((scale*QK^T + noise)/tau)  (plain softmax(scale*QK^T)
  * when noise is NULL), float [batch, n_q_heads, seq_q, seq_kv] contiguous, masked entries 0; optionally their sums

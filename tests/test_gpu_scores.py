@@ -308,3 +308,63 @@ def test_fp16_statistics_form_refuses_prefill_shapes():
     h1 = torch.zeros(1, 2, 64, device="cuda", dtype=torch.float16)
     with pytest.raises(ValueError):
         ops.attention_with_stats_half(qd, kd, vd, torch.zeros_like(qd), 0.125, True, h1)
+
+
+# ---- trn_attn_key_scores_f16: any noise element type, pitch and alignment, fp16 or fp32 statistics, every kernel behind it
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,ws", [
+    (1, 4, 2, 16, 333, 128, True, False), (1, 3, 3, 1, 35, 64, False, False), (1, 8, 2, 16, 8193, 128, False, True),   # decode, split keys
+    (2, 4, 2, 65, 129, 128, True, False), (1, 71, 1, 100, 131, 64, False, False),                                      # tiles of 32 queries
+    (4, 32, 8, 131, 131, 128, True, False), (2, 71, 1, 150, 217, 64, True, False), (8, 32, 8, 257, 257, 64, True, False)])  # prefill kernels
+@pytest.mark.parametrize("noise", ["fp16", "fp32"])
+def test_key_scores_for_noise_at_any_pitch(B, Hq, Hkv, Sq, Skv, D, causal, ws, noise):
+    """Rows of Skv (odd) elements without padding, the whole tensor starting one element into its buffer: held bit for bit to
+    the entry point that takes padded fp32 noise (and that the oracle tests above cover); fp16 statistics are the fp32
+    ones rounded once.  The words around the tensor are NaN."""
+    from triton_amd import ops
+    q, k, v = (t.cuda() for t in make(B, Hq, Hkv, Sq, Skv, D, seed=11))
+    dt = torch.float16 if noise == "fp16" else torch.float32
+    n = B * Hq * Sq * Skv
+    buf = torch.full((n + 9,), float("nan"), dtype=dt, device="cuda")
+    x = buf[1:n + 1].view(B, Hq, Sq, Skv)
+    x.copy_(torch.randn(B, Hq, Sq, Skv, generator=torch.Generator().manual_seed(2)))
+    pad = torch.full((B, Hq, Sq, (Skv + 3) // 4 * 4), float("nan"), device="cuda")
+    pad[..., :Skv] = x.float()
+    scale, stat = D ** -0.5, lambda dt=torch.float32: torch.full((B, Hq, Skv), -1.0, device="cuda", dtype=dt)
+    work = None
+    if ws:
+        nb = ops.attention_stats_workspace_bytes(q, k, v, q, scale, causal)
+        assert nb > 0
+        work = torch.zeros(nb, dtype=torch.uint8, device="cuda")
+    o1, o2, o3 = torch.zeros_like(q), torch.zeros_like(q), torch.zeros_like(q)
+    r1, r2 = torch.zeros(B, Hq, Sq, device="cuda"), torch.zeros(B, Hq, Sq, device="cuda")
+    a1, b1, a2, b2 = stat(), stat(), stat(), stat()
+    h1, h2 = stat(torch.float16), stat(torch.float16)
+    ops.attention_with_stats(q, k, v, o1, scale, causal, a1, b1, noise=pad[..., :Skv], tau=1.5, lse_pert=r1, workspace=work)
+    ops.attention_key_scores(q, k, v, o2, scale, causal, r2, a2, b2, noise=x, tau=1.5, workspace=work)
+    ops.attention_key_scores(q, k, v, o3, scale, causal, r2, h1, h2, noise=x, tau=1.5, workspace=work)
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2) and torch.equal(o1, o3) and torch.equal(r1, r2)
+    assert torch.equal(a1, a2) and torch.equal(b1, b2)
+    assert torch.equal(h1, a1.half()) and torch.equal(h2, b1.half())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sq,Skv", [(16, 100), (200, 200)])
+def test_key_scores_without_noise_and_as_mean_and_std(Sq, Skv):
+    from triton_amd import ops, _lib
+    q, k, v = (t.cuda() for t in make(1, 4, 2, Sq, Skv, 128, seed=12))
+    stat = lambda: torch.full((1, 4, Skv), -1.0, device="cuda")
+    lse, rows = torch.zeros(1, 4, Sq, device="cuda"), torch.zeros(1, 4, Sq, device="cuda")
+    o1, o2, s = torch.zeros_like(q), torch.zeros_like(q), [stat() for _ in range(8)]
+    ops.attention(q, k, v, o1, 0.1, True, lse=lse)
+    ops.attention_with_stats(q, k, v, o1, 0.1, True, s[0], s[1], lse=lse)
+    ops.attention_col_mean_std(q, k, lse, 0.1, True, s[2], s[3])
+    ops.attention_key_scores(q, k, v, o2, 0.1, True, rows, s[4], s[5])
+    ops.attention_key_scores(q, k, v, o2, 0.1, True, rows, s[6], s[7], mean_std=True)
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2) and torch.equal(lse, rows) and all(torch.equal(s[i], s[i + 4]) for i in range(4))
+    with pytest.raises(ValueError):
+        ops.attention_key_scores(q, k, v, o2, 0.1, True, rows, s[4], s[5].half())
+    with pytest.raises(_lib.TrnError):           # mean and standard deviation are defined without noise only
+        ops.attention_key_scores(q, k, v, o2, 0.1, True, rows, s[4], s[5], noise=torch.zeros(1, 4, Sq, Skv, device="cuda"), mean_std=True)

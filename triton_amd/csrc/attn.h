@@ -21,15 +21,49 @@ struct AttnArgs {
     float* col_sum; float* col_sumsq;
     // ... and the probabilities themselves, un-reduced: float [B, Hq, Sq, Skv] contiguous
     float* probs;
-    // decode kernel only: noise, col_sum and col_sumsq point at fp16 data (noise pitches in halfs)
-    int io16;
+    int n16;       // noise points at fp16 data (its pitches count halfs; any alignment: see HalfNoise)
+    int s16;       // decode kernel only: col_sum and col_sumsq point at fp16 data
 };
+
+// fp16 noise as the kernels fetch it.  Its rows may start at any element (the reference's [.., M, P + M] tensors have any
+// key count), so a lane reads the whole dwords around its 4 keys -- three of them cover both cases -- and shifts by half a
+// dword where its row starts on an odd element.  Nothing outside the dword that holds a row's last key is ever read: the
+// base is rounded down to a dword and the range up to one.
+#if defined(__HIP_DEVICE_COMPILE__)
+typedef uint32_t uint3_t __attribute__((ext_vector_type(3)));
+struct HalfNoise {
+    __amdgpu_buffer_rsrc_t rs;
+    int odd;           // 1: the base was rounded down by one element
+    __device__ __forceinline__ HalfNoise(const void* head_base, int64_t rows, int64_t pitch, int64_t cols) {
+        const uintptr_t p = reinterpret_cast<uintptr_t>(head_base);
+        odd = (int)(p >> 1) & 1;
+        rs = __builtin_amdgcn_make_buffer_rsrc((void*)(p & ~(uintptr_t)3), 0, (int)((((rows - 1) * pitch + cols + odd) * 2 + 3) & ~3), 0x00020000);
+    }
+    // byte offset of a row's (rounded down) start and the shift of its elements within the dwords
+    __device__ __forceinline__ int row(int64_t first_elem, int& shift) const {
+        const int64_t e = first_elem + odd;
+        shift = (int)(e & 1) * 16;
+        return (int)((e & ~(int64_t)1) * 2);
+    }
+};
+// the 4 values out of three dwords
+__device__ __forceinline__ half4_t half_noise4(const uint3_t& d, int shift) {
+    const uint2_t u = {__builtin_amdgcn_alignbit(d.y, d.x, shift), __builtin_amdgcn_alignbit(d.z, d.y, shift)};
+    return __builtin_bit_cast(half4_t, u);
+}
+#endif
 
 // Checks, argument block and kernel choice behind every attention entry point of the C ABI.
 int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                  const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
-                 bool io16 = false);
+                 bool n16 = false, bool s16 = false, bool any_pitch = false);
+
+// Checks, argument block and kernel choice behind the column statistics (attn_colstats.hip); mean_std: the two outputs
+// are the mean and standard deviation; n16 / s16: fp16 noise / outputs; any_pitch: fp32 noise on any dword (16-byte
+// buffer loads need no more).
+int attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise, float* out_sum,
+                  float* out_sumsq, int mean_std, void* stream, bool n16 = false, bool s16 = false, bool any_pitch = false);
 
 // One workgroup per head and 32 queries, whose eight waves split the keys (attn_decode.hip): at most 32 queries per head
 // (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.

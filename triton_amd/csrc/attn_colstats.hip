@@ -20,7 +20,7 @@
 // in a fixed order: the wait for a Q stage counts the loads issued behind it.  Masks (causal diagonal, ragged
 // ends) are evaluated only in the blocks that need them (a wave-uniform test).
 #include <type_traits>
-#include "common.h"
+#include "attn.h"
 
 namespace trn {
 
@@ -34,19 +34,29 @@ struct ColArgs {
     float c1;   // log2-domain multiplier of the raw score: scale*log2e (RoCo) or scale*log2e/tau (KeyFormer)
     float c3;   // log2e/tau multiplier of the noise
     int causal;
+    int n16;        // noise points at fp16 data (its pitches count halfs)
+    int s16;        // the outputs are fp16: the fp32 results rounded once
     int pair;       // (no-noise kernel) a workgroup takes key tiles i and n-1-i
     int mean_std;   // write the per-key mean and population standard deviation over the queries that see the key
                     // (into out_sum / out_sumsq) instead of the two sums
 };
+
+__device__ __forceinline__ void store_stat(const ColArgs& a, float* out, int64_t at, float v) {
+    if (!out) return;
+    if (a.s16) reinterpret_cast<half_t*>(out)[at] = (half_t)v;
+    else out[at] = v;
+}
 
 constexpr int CBN = 128;  // keys per workgroup
 [[maybe_unused]] constexpr int CBM = 64;   // queries per staged tile
 
 // SQ: the sums of squares are wanted too (RoCo); without them (KeyFormer) their accumulators and one of the five
 // VALU operations per score are not compiled in.
-template <int D, bool NOISE, bool SQ>
-__global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const ColArgs a) {
+// NZ: 1 fp32 noise, 2 fp16 noise
+template <int D, int NZ, bool SQ>
+__global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
+    constexpr bool N16 = NZ == 2;
     constexpr int NKS = D / 16;
     constexpr int CPR = D / 8;                 // 16-byte chunks per Q row
     constexpr int RPI = 64 / CPR;              // stage rows covered by one wave-wide 1 KB load
@@ -56,7 +66,7 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
     __shared__ __attribute__((aligned(1024))) half_t Qs2[CBM * D];
     // KeyFormer: the wave's 32 x 32 block of noise is fetched with whole 128-byte row pieces per 8 lanes (a load
     // instruction then touches 8 cache lines, not 32) and turned into the accumulator layout through this array
-    __shared__ __attribute__((aligned(1024))) float Ns[NOISE ? 4 * 1024 : 4];
+    __shared__ __attribute__((aligned(1024))) float Ns[4 * 1024];
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -98,15 +108,21 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
     // ---- per-tile register prefetch: row normalisers and noise of the tile's two 32-query blocks
     const __amdgpu_buffer_rsrc_t lrs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.lse + ((int64_t)b * a.Hq + head) * a.Sq), 0, a.Sq * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t nrs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(NOISE ? a.noise + b * a.nb + head * a.nh : a.lse), 0,
-        NOISE ? (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4) : 0, 0x00020000);
+    // (fp16 noise: three dwords around the 4 keys, shifted and widened when the block is consumed)
+    typedef typename std::conditional<N16, uint3_t, float4_t>::type noise_t;
+    constexpr int nsz = N16 ? 2 : 4;
+    const void* nbase = reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * nsz;
+    const HalfNoise hn(nbase, N16 ? a.Sq : 1, N16 ? a.ns : 0, N16 ? a.Skv : 0);
+    const __amdgpu_buffer_rsrc_t nrs = N16 ? hn.rs : __builtin_amdgcn_make_buffer_rsrc(
+        (void*)nbase, 0, (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4), 0x00020000);
     // load i of a block covers its query rows 8i .. 8i+7: lane -> row 8i + lane/8, keys 4*(lane%8) .. +3
-    const int nvo = NOISE ? (int)(((lane >> 3) * a.ns + wkey0 + 4 * (lane & 7)) * 4) : 0;
-    const int nrow8 = NOISE ? (int)(8 * a.ns * 4) : 0;
+    int nsh = 0;
+    const int64_t nfirst = (lane >> 3) * a.ns + wkey0 + 4 * (lane & 7);
+    const int nvo = N16 ? hn.row(nfirst, nsh) : (int)(nfirst * 4);
+    const int nrow8 = (int)(8 * a.ns * nsz);
     // transposer: the 16-byte chunk q of row r sits at chunk r*8 + (q ^ ((r/2) % 8)); written as loaded, read as
     // row c, chunks 2*r4 + h (both conflict-free)
-    float* nsw = Ns + (NOISE ? wave * 1024 : 0);
+    float* nsw = Ns + wave * 1024;
     int ns_wr[4], ns_rd[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -117,15 +133,15 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
     // Two register buffers, used by even and odd tiles in turn.  A block's half of a buffer is refilled, for the tile
     // after next, as soon as that block has been consumed, so between one and two tiles of noise (8 - 16 KB per
     // wave) are in flight at any time.
-    struct Pre { float lse[2]; float4_t g[2][4]; };
+    struct Pre { float lse[2]; noise_t g[2][4]; };
     Pre pa, pb;
     auto prefetch = [&](int t, int qb, Pre& p) __attribute__((always_inline)) {
         p.lse[qb] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lrs, c * 4, (t * CBM + qb * 32) * 4, 0));
-        if constexpr (NOISE) {
+        const int so = (int)((t * CBM + qb * 32) * a.ns * nsz);
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4)
-                p.g[qb][r4] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                    nrs, nvo + r4 * nrow8, (int)((t * CBM + qb * 32) * a.ns * 4), 0));
+        for (int r4 = 0; r4 < 4; ++r4) {
+            if constexpr (N16) p.g[qb][r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b96(nrs, nvo + r4 * nrow8, so, 0));
+            else p.g[qb][r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * nrow8, so, 0));
         }
     };
 
@@ -134,15 +150,19 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
 
     // The VALU part of a 32-query block.  Masked and plain blocks are separate loops (one wave-uniform branch
     // per block) so that the plain one is 4 instructions per score: fma, exp2, add, fma.
-    auto softmax_sums = [&](const float16_t& acc, int qfirst, float lse, const float4_t (&gl)[4]) __attribute__((always_inline)) {
+    auto softmax_sums = [&](const float16_t& acc, int qfirst, float lse, const noise_t (&gl)[4]) __attribute__((always_inline)) {
         const float lse2 = lse * kLog2e;
         float4_t gq[4];
-        if constexpr (NOISE) {       // (LDS operations of one wave execute in order: no barrier between the two)
+        // (LDS operations of one wave execute in order: no barrier between the two)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) *reinterpret_cast<float4_t*>(&nsw[ns_wr[i]]) = gl[i];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) gq[i] = *reinterpret_cast<const float4_t*>(&nsw[ns_rd[i]]);
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (N16) {
+                const half4_t hv = half_noise4(gl[i], nsh);
+                *reinterpret_cast<float4_t*>(&nsw[ns_wr[i]]) = float4_t{(float)hv[0], (float)hv[1], (float)hv[2], (float)hv[3]};
+            } else *reinterpret_cast<float4_t*>(&nsw[ns_wr[i]]) = gl[i];
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) gq[i] = *reinterpret_cast<const float4_t*>(&nsw[ns_rd[i]]);
         const bool masked = (qfirst + 31 >= a.Sq) || (wkey0 + 31 >= a.Skv) || (a.causal && wkey0 + 31 > qfirst + off);
         if (masked) {
             // last key this lane's query may count, as an offset from the lane's first key (-1: none)
@@ -151,7 +171,7 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 float t = __builtin_fmaf(acc[r], a.c1, -lse2);
-                if constexpr (NOISE) t = __builtin_fmaf(gq[r / 4][r % 4], a.c3, t);
+                t = __builtin_fmaf(gq[r / 4][r % 4], a.c3, t);
                 const float p = (8 * (r / 4) + (r % 4) <= last) ? fast_exp2(t) : 0.f;
                 s1[r] += p;
                 if constexpr (SQ) s2[r] = __builtin_fmaf(p, p, s2[r]);
@@ -160,7 +180,7 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 float t = __builtin_fmaf(acc[r], a.c1, -lse2);
-                if constexpr (NOISE) t = __builtin_fmaf(gq[r / 4][r % 4], a.c3, t);
+                t = __builtin_fmaf(gq[r / 4][r % 4], a.c3, t);
                 const float p = fast_exp2(t);
                 s1[r] += p;
                 if constexpr (SQ) s2[r] = __builtin_fmaf(p, p, s2[r]);
@@ -206,7 +226,7 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
     // sizes its own waits for prefetched registers by the loads it KNOWS follow them, and a conditional load counts
     // as absent, which would make every use of a prefetched value drain the refills too.
     auto tile = [&](int t, const half_t* Qc, half_t* Qf, Pre& pc) __attribute__((always_inline)) {
-        constexpr int kBehind = NI + 4 + (NOISE ? 16 : 0);
+        constexpr int kBehind = NI + 4 + 16;
         __builtin_amdgcn_s_waitcnt(0x0f70 | (kBehind & 15) | ((kBehind >> 4) << 14));
         __builtin_amdgcn_s_barrier();        // (a bare barrier: nothing else in flight needs draining)
         __builtin_amdgcn_sched_barrier(0);
@@ -253,8 +273,8 @@ __global__ __launch_bounds__(256, NOISE ? 2 : 3) void attn_colstats_kernel(const
             x = mean;
         }
         if (c == 0 && key < a.Skv) {
-            if (a.out_sum) a.out_sum[obase + key] = x;
-            if (SQ && a.out_sumsq) a.out_sumsq[obase + key] = y;
+            store_stat(a, a.out_sum, obase + key, x);
+            if (SQ) store_stat(a, a.out_sumsq, obase + key, y);
         }
     }
 #endif
@@ -477,8 +497,8 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
             x = mean;
         }
         if (c == 0 && key < a.Skv) {
-            if (a.out_sum) a.out_sum[obase + key] = x;
-            if (SQ && a.out_sumsq) a.out_sumsq[obase + key] = y;
+            store_stat(a, a.out_sum, obase + key, x);
+            if (SQ) store_stat(a, a.out_sumsq, obase + key, y);
         }
     }
     }   // pass
@@ -495,34 +515,29 @@ static hipError_t launch_col_plain(ColArgs a, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int D, bool NOISE>
+template <int D, int NZ>
 static hipError_t launch_col(const ColArgs& a, hipStream_t s) {
     const unsigned grid = (unsigned)a.n_kvtiles * a.B * a.Hq;
-    if (a.out_sumsq) hipLaunchKernelGGL((attn_colstats_kernel<D, NOISE, true>), dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((attn_colstats_kernel<D, NOISE, false>), dim3(grid), dim3(256), 0, s, a);
+    if (a.out_sumsq) hipLaunchKernelGGL((attn_colstats_kernel<D, NZ, true>), dim3(grid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((attn_colstats_kernel<D, NZ, false>), dim3(grid), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
 }  // namespace trn
 
-namespace trn {
-static int colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
-                    float* out_sum, float* out_sumsq, int mean_std, void* stream);
-}
-
 extern "C" int trn_attn_colstats_f16(const trn_attn_desc* d, const void* q, const void* k, const float* lse,
                                      const float* noise, float* out_sum, float* out_sumsq, void* stream) {
-    return trn::colstats(d, q, k, lse, noise, out_sum, out_sumsq, 0, stream);
+    return trn::attn_colstats(d, q, k, lse, noise, out_sum, out_sumsq, 0, stream);
 }
 
 extern "C" int trn_attn_colmeanstd_f16(const trn_attn_desc* d, const void* q, const void* k, const float* lse,
                                        float* out_mean, float* out_std, void* stream) {
     if (!out_mean || !out_std) return TRN_E_NULL;
-    return trn::colstats(d, q, k, lse, nullptr, out_mean, out_std, 1, stream);
+    return trn::attn_colstats(d, q, k, lse, nullptr, out_mean, out_std, 1, stream);
 }
 
-static int trn::colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
-                         float* out_sum, float* out_sumsq, int mean_std, void* stream) {
+int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
+                       float* out_sum, float* out_sumsq, int mean_std, void* stream, bool n16, bool s16, bool any_pitch) {
     if (!d || !q || !k || !lse) return TRN_E_NULL;
     if (!out_sum && !out_sumsq) return TRN_E_NULL;
     int st = validate_attn(d, false);
@@ -534,8 +549,8 @@ static int trn::colstats(const trn_attn_desc* d, const void* q, const void* k, c
         if (d->noise_stride_s < d->seq_kv) return TRN_E_STRIDE;
         // one head's noise is addressed with 32-bit byte offsets
         if (((int64_t)d->seq_q + 128) * d->noise_stride_s * 4 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
-        if (!aligned16(noise) || !pitch16(d->noise_stride_s, 4) || !pitch16(d->noise_stride_h, 4) ||
-            !pitch16(d->noise_stride_b, 4))
+        if (n16 || any_pitch ? (reinterpret_cast<uintptr_t>(noise) & (n16 ? 1u : 3u)) != 0
+                : !aligned16(noise) || !pitch16(d->noise_stride_s, 4) || !pitch16(d->noise_stride_h, 4) || !pitch16(d->noise_stride_b, 4))
             return TRN_E_ALIGN;
     }
     // Q tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base (with room for the tile requested
@@ -552,11 +567,11 @@ static int trn::colstats(const trn_attn_desc* d, const void* q, const void* k, c
     const float tau = noise ? d->tau : 1.f;
     a.c1 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.causal = d->causal ? 1 : 0;
-    a.mean_std = mean_std; a.pair = 0;
+    a.mean_std = mean_std; a.pair = 0; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
     if ((int64_t)a.n_kvtiles * a.B * a.Hq > 0x7fffffffLL) return TRN_E_SHAPE;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
-    if (d->head_dim == 128) e = noise ? launch_col<128, true>(a, s) : launch_col_plain<128>(a, s);
-    else e = noise ? launch_col<64, true>(a, s) : launch_col_plain<64>(a, s);
+    if (d->head_dim == 128) e = !noise ? launch_col_plain<128>(a, s) : n16 ? launch_col<128, 2>(a, s) : launch_col<128, 1>(a, s);
+    else e = !noise ? launch_col_plain<64>(a, s) : n16 ? launch_col<64, 2>(a, s) : launch_col<64, 1>(a, s);
     return e == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
 }

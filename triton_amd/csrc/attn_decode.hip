@@ -12,6 +12,7 @@
 // that the waits can be counted.
 #include "attn.h"
 #include <mutex>
+#include <type_traits>
 
 typedef unsigned long long ulong2_t __attribute__((ext_vector_type(2)));
 
@@ -149,28 +150,21 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         for (int r = 0; r < 16; ++r) oacc[i][r] = 0.f;
     float m = -INFINITY, l = 0.f;       // running max (log2 domain, shared by the lane pair) and this lane's partial sum
     float m2 = -INFINITY, l2 = 0.f;     // the same for the perturbed scores (KeyFormer)
-    // KeyFormer noise: this lane's query row, the 4 x 4 keys of its accumulator layout per block, one block ahead
-    // (fp16 noise: 8-byte pieces of 4 keys, widened as they arrive)
-    constexpr int nsz = N16 ? 2 : 4;     // bytes per noise element
-    const __amdgpu_buffer_rsrc_t nrs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(NOISE ? reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * nsz : nullptr), 0,
-        NOISE ? (int)(((int64_t)(a.Sq - 1) * a.ns + (N16 ? (a.Skv + 1) & ~1 : a.Skv)) * nsz) : 0, 0x00020000);
-    // (The range check works on whole dwords: with fp16 noise and an odd key count the last row's last key shares its
-    // dword with the first half of the row's padding, so the range ends behind that dword -- the rows are padded to
-    // 8 bytes -- and keys past the end are discarded by the mask, whatever the padding holds.)
-    const int nvo = NOISE ? (int)(((int64_t)qrow_ld * a.ns + 4 * h) * nsz) : 0;
-    float4_t g0[4], g1[4];
-    auto fetch_noise = [&](int blk, float4_t (&g)[4]) __attribute__((always_inline)) {
-        if constexpr (N16) {
+    // KeyFormer noise: this lane's query row, the 4 x 4 keys of its accumulator layout per block, one block ahead; kept as
+    // it arrives (three dwords per 4 keys of fp16 noise) and widened where it is used, so that nothing waits for it here
+    typedef typename std::conditional<N16, uint3_t, float4_t>::type noise_t;
+    const void* nbase = NOISE ? reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * (N16 ? 2 : 4) : nullptr;
+    const HalfNoise hn(nbase, N16 ? a.Sq : 1, N16 ? a.ns : 0, N16 ? a.Skv : 0);
+    const __amdgpu_buffer_rsrc_t nrs = N16 ? hn.rs : __builtin_amdgcn_make_buffer_rsrc(
+        (void*)nbase, 0, NOISE ? (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4) : 0, 0x00020000);
+    int nsh = 0;
+    const int nvo = N16 ? hn.row((int64_t)qrow_ld * a.ns + 4 * h, nsh) : NOISE ? (int)(((int64_t)qrow_ld * a.ns + 4 * h) * 4) : 0;
+    noise_t g0[4], g1[4];
+    auto fetch_noise = [&](int blk, noise_t (&g)[4]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                const half4_t hv = __builtin_bit_cast(half4_t, __builtin_amdgcn_raw_buffer_load_b64(nrs, nvo + r4 * 16, blk * 64, 0));
-                g[r4] = float4_t{(float)hv[0], (float)hv[1], (float)hv[2], (float)hv[3]};
-            }
-        } else {
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4)
-                g[r4] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * 32, blk * 128, 0));
+        for (int r4 = 0; r4 < 4; ++r4) {
+            if constexpr (N16) g[r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b96(nrs, nvo + r4 * 16, blk * 64, 0));
+            else g[r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * 32, blk * 128, 0));
         }
     };
 
@@ -183,8 +177,8 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     half8_t ka0[NS], ka1[NS];
 
     // One 32-key block whose K is in kc and whose V is in stage Vc; the next block's loads go to kn / Vn first.
-    auto block = [&](int it, half8_t (&kc)[NS], half8_t (&kn)[NS], const half_t* Vc, half_t* Vn, float4_t (&gc)[4],
-                     float4_t (&gn)[4]) __attribute__((always_inline)) {
+    auto block = [&](int it, half8_t (&kc)[NS], half8_t (&kn)[NS], const half_t* Vc, half_t* Vn, noise_t (&gc)[4],
+                     noise_t (&gn)[4]) __attribute__((always_inline)) {
         const int blk = blk0 + wave + it * DNW, key0 = blk * 32;
         // (with noise the registers are short: K is then single-buffered, refilled as soon as the scores are issued)
         if constexpr (!NOISE) fetch_k(blk + DNW, kn);
@@ -215,7 +209,16 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         if constexpr (NOISE) {          // row normaliser of z = (scale*s + g)/tau in the log2 domain
             float16_t z;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) z[r] = __builtin_fmaf(gc[r / 4][r % 4], a.c3, s[r] * a.c2);
+            for (int r4 = 0; r4 < 4; ++r4) {
+                if constexpr (N16) {
+                    const half4_t gv = half_noise4(gc[r4], nsh);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) z[r4 * 4 + e] = __builtin_fmaf((float)gv[e], a.c3, s[r4 * 4 + e] * a.c2);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) z[r4 * 4 + e] = __builtin_fmaf(gc[r4][e], a.c3, s[r4 * 4 + e] * a.c2);
+                }
+            }
             if (masked) {               // a select, not arithmetic: what lies past a row's last key (the padding of
                                         // the noise pitch) may be anything, NaN included
 #pragma unroll
@@ -472,7 +475,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
                     const int qr = 8 * (r / 4) + 4 * h + (r % 4);
                     if constexpr (N16)
                         g[r] = (float)__builtin_bit_cast(half_t, __builtin_amdgcn_raw_buffer_load_b16(
-                            nrs, (int)((qr * a.ns + c) * 2), blk * 64, 0));
+                            nrs, (int)((qr * a.ns + c + hn.odd) * 2), blk * 64, 0));
                     else
                         g[r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
                             nrs, (int)((qr * a.ns + c) * 4), blk * 128, 0));
@@ -508,7 +511,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
             x = half_sum(x); y = half_sum(y);
             if (h == 0 && key < a.Skv) {
                 const int64_t at = (int64_t)bh * a.Skv + key;
-                if (a.io16) {       // (the fp32 value rounded once, as a copy into the caller's fp16 tensor would)
+                if (a.s16) {        // (the fp32 value rounded once, as a copy into the caller's fp16 tensor would)
                     if (a.col_sum) reinterpret_cast<half_t*>(a.col_sum)[at] = (half_t)x;
                     if (a.col_sumsq) reinterpret_cast<half_t*>(a.col_sumsq)[at] = (half_t)y;
                 } else {
@@ -606,7 +609,7 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)grid), t(DNW * 64);
 #define TRN_DEC(D_, DS_, N_) hipLaunchKernelGGL((attn_decode_kernel<D_, DS_, N_>), g, t, 0, stream, a)
-#define TRN_DEC_NZ(D_, DS_) do { if (!a.noise) TRN_DEC(D_, DS_, 0); else if (a.io16) TRN_DEC(D_, DS_, 2); else TRN_DEC(D_, DS_, 1); } while (0)
+#define TRN_DEC_NZ(D_, DS_) do { if (!a.noise) TRN_DEC(D_, DS_, 0); else if (a.n16) TRN_DEC(D_, DS_, 2); else TRN_DEC(D_, DS_, 1); } while (0)
     if (head_dim == 128) { if (ds == 4) TRN_DEC_NZ(128, 4); else if (ds == 2) TRN_DEC_NZ(128, 2); else TRN_DEC_NZ(128, 1); }
     else { if (ds == 2) TRN_DEC_NZ(64, 2); else TRN_DEC_NZ(64, 1); }
 #undef TRN_DEC_NZ

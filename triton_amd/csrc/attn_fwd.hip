@@ -25,10 +25,12 @@
 
 namespace trn {
 
-template <int D, int NW, bool NOISE>
-__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer-descriptor types and LDS-load builtins exist in the device pass only;
-                                      // the host pass needs just the launch stub
+                                      // the host pass needs just the launch stubs
+// NZ: 1 fp32 noise, 2 fp16 noise
+template <int D, int NW, int NZ>
+__device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
+    constexpr bool NOISE = NZ != 0, N16 = NZ == 2;
     constexpr int BN = 64;       // keys per LDS stage (two 32-key blocks)
     constexpr int NS = D / 16;   // MFMA slots per phase: k-steps of S^T = K Q^T, and (2 key halves) x (D/32) of P V
     constexpr int NDB = D / 32;  // 32-wide blocks of head_dim in O^T
@@ -123,15 +125,21 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(cons
     // KeyFormer noise: this lane's query row, the 4 x 4 keys of its accumulator layout per 32-key block.  It is
     // the HBM stream that bounds that variant, so each block's 64 bytes per lane are requested two pipeline steps
     // before they are used (buffer loads: keys or rows past the end read as zeros and are masked anyway).
-    const __amdgpu_buffer_rsrc_t nrs = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(NOISE ? a.noise + b * a.nb + head * a.nh : nullptr), 0,
-        NOISE ? (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4) : 0, 0x00020000);
-    const int nvo = NOISE ? (int)(((int64_t)qrow_ld * a.ns + 4 * h) * 4) : 0;
-    float4_t gpre0[4], gpre1[4];       // even / odd 32-key blocks: each refilled two blocks ahead, as soon as it is used
-    auto fetch_noise = [&](int key0, float4_t (&gpre)[4]) __attribute__((always_inline)) {
+    // (fp16 noise: three dwords per 4 keys, widened by the fused multiply-add that uses them.)
+    typedef typename std::conditional<N16, uint3_t, float4_t>::type noise_t;
+    const void* nbase = NOISE ? reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * (N16 ? 2 : 4) : nullptr;
+    const HalfNoise hn(nbase, N16 ? a.Sq : 1, N16 ? a.ns : 0, N16 ? a.Skv : 0);
+    const __amdgpu_buffer_rsrc_t nrs = N16 ? hn.rs : __builtin_amdgcn_make_buffer_rsrc(
+        (void*)nbase, 0, NOISE ? (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4) : 0, 0x00020000);
+    int nsh = 0;
+    const int nvo = N16 ? hn.row((int64_t)qrow_ld * a.ns + 4 * h, nsh) : NOISE ? (int)(((int64_t)qrow_ld * a.ns + 4 * h) * 4) : 0;
+    noise_t gpre0[4], gpre1[4];        // even / odd 32-key blocks: each refilled two blocks ahead, as soon as it is used
+    auto fetch_noise = [&](int key0, noise_t (&gpre)[4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4)
-            gpre[r4] = __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * 32, key0 * 4, 0));
+        for (int r4 = 0; r4 < 4; ++r4) {
+            if constexpr (N16) gpre[r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b96(nrs, nvo + r4 * 16, key0 * 2, 0));
+            else gpre[r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * 32, key0 * 4, 0));
+        }
     };
 
     // ---- staging: direct global -> LDS loads.  Buffer descriptors give zero fill for keys past the end
@@ -159,7 +167,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(cons
     // range, fp32 sums), O and l stay relative to the same m so the final O/l and m + log2(l) are unchanged,
     // and the 16*NDB-multiply rescale of O^T runs on the first block or two only instead of on most blocks.
     // Returns whether a rescale is due (wave-uniform) and the candidate max.
-    auto reduce_block = [&](bool masked, float16_t& sx, int key0, float& smax, float4_t (&gpre)[4]) __attribute__((always_inline)) {
+    auto reduce_block = [&](bool masked, float16_t& sx, int key0, float& smax, noise_t (&gpre)[4]) __attribute__((always_inline)) {
         // `masked` is wave-uniform: the branches below touch only this block's 16 score registers, so the
         // accumulators never meet a control-flow merge.  (Two whole-step variants selected by a branch cost
         // dozens of accumulator register copies per step and broke the in-place MFMA accumulation chains.)
@@ -171,10 +179,11 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(cons
             float16_t d;
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
-                const float4_t gv = gpre[r4];
+                typename std::conditional<N16, half4_t, float4_t>::type gv;
+                if constexpr (N16) gv = half_noise4(gpre[r4], nsh); else gv = gpre[r4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf(gv[e], a.c3, nref));
+                    float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)gv[e], a.c3, nref));
                     if (masked) {
                         const int key = key0 + 8 * r4 + 4 * h + e;
                         dd = (key < a.Skv && (!a.causal || key <= qrow + off)) ? dd : -INFINITY;
@@ -381,15 +390,29 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(cons
         if (qrow < a.Sq && h == 0)
             a.lse_pert[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m2 + fast_log2(l2s)) * kLn2;
     }
+}
+#endif
+
+template <int D, int NW, bool NOISE>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd_body<D, NW, NOISE ? 1 : 0>(a);
+#endif
+}
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_half_noise_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd_body<D, NW, 2>(a);
 #endif
 }
 
-template <int D, int NW, bool NOISE>
+template <int D, int NW>
 static hipError_t launch_fwd(AttnArgs a, hipStream_t s) {
     a.n_qtiles = (a.Sq + 32 * NW - 1) / (32 * NW);
     const int64_t grid = (int64_t)a.n_qtiles * a.B * a.Hq;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((attn_fwd_kernel<D, NW, NOISE>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    if (a.n16) hipLaunchKernelGGL((attn_fwd_half_noise_kernel<D, NW>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    else hipLaunchKernelGGL((attn_fwd_kernel<D, NW, true>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
     return hipGetLastError();
 }
 
@@ -525,14 +548,37 @@ extern "C" int trn_attn_fwd_stats_half_f16(const trn_attn_desc* d, const void* q
     if (!d) return TRN_E_NULL;
     if (!out_sum && !out_sumsq) return TRN_E_NULL;
     if (d->q_norm || d->seq_q > 32) return TRN_E_UNSUPPORTED;
+    if (noise && ((reinterpret_cast<uintptr_t>(noise) & 7u) || (d->noise_stride_s & 3) || (d->noise_stride_h & 3) || (d->noise_stride_b & 3)))
+        return TRN_E_ALIGN;
     return attn_forward(d, q, k, v, o, lse, gamma_q, static_cast<const float*>(noise), lse_pert, nullptr, 0,
-                        static_cast<float*>(out_sum), static_cast<float*>(out_sumsq), stream, nullptr, true);
+                        static_cast<float*>(out_sum), static_cast<float*>(out_sumsq), stream, nullptr, true, true);
+}
+
+extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o,
+                                       const void* noise, int32_t noise_half, float* rows, void* out1, void* out2,
+                                       int32_t out_half, int32_t mean_std, void* workspace, int64_t workspace_bytes,
+                                       void* stream) {
+    using namespace trn;
+    if (!d || !rows || (!out1 && !out2) || (mean_std && !(out1 && out2))) return TRN_E_NULL;
+    if (d->q_norm || (mean_std && noise)) return TRN_E_UNSUPPORTED;
+    const float* n = static_cast<const float*>(noise);
+    float *lse = noise ? nullptr : rows, *lse_pert = noise ? rows : nullptr, *s1 = static_cast<float*>(out1), *s2 = static_cast<float*>(out2);
+    const bool n16 = noise && noise_half, s16 = out_half != 0;
+    const int64_t need = workspace ? trn_attn_stats_workspace_bytes(d) : 0;
+    const bool split = need > 0 && workspace_bytes >= need;
+    // a handful of queries per head and no split of the keys: the statistics are a second sweep inside the same kernel
+    if (d->seq_q <= 32 && !split && !mean_std)
+        return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true);
+    const int st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, split ? workspace : nullptr, split ? workspace_bytes : 0,
+                                nullptr, nullptr, stream, nullptr, n16, false, true);
+    if (st != TRN_OK) return st;
+    return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);
 }
 
 int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                              int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs,
-                             bool io16) {
+                             bool n16, bool s16, bool any_pitch) {
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
     if (!d || !q || !k || !v || !o) return TRN_E_NULL;
     if (noise && !lse_pert) return TRN_E_NULL;
@@ -545,14 +591,13 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         if (d->noise_stride_s < d->seq_kv) return TRN_E_STRIDE;
         // one head's noise is addressed with 32-bit byte offsets
         if ((int64_t)d->seq_q * d->noise_stride_s * 4 + 1024 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
-        if (io16) {     // fp16 noise is fetched 8 bytes at a time
-            if ((reinterpret_cast<uintptr_t>(noise) & 7u) || (d->noise_stride_s & 3) || (d->noise_stride_h & 3) || (d->noise_stride_b & 3))
-                return TRN_E_ALIGN;
+        if (n16 || any_pitch) {   // fp16: whole dwords around the rows are fetched and shifted; fp32: 16-byte loads on any dword
+            if (reinterpret_cast<uintptr_t>(noise) & (n16 ? 1u : 3u)) return TRN_E_ALIGN;
         } else if (!aligned16(noise) || !pitch16(d->noise_stride_s, 4) || !pitch16(d->noise_stride_h, 4) ||
                    !pitch16(d->noise_stride_b, 4))
             return TRN_E_ALIGN;
     }
-    if (io16 && d->seq_q > 32) return TRN_E_UNSUPPORTED;     // fp16 noise and statistics: the decode kernel only
+    if (s16 && d->seq_q > 32) return TRN_E_UNSUPPORTED;      // fp16 statistics of the second sweep: at most 32 queries
     AttnArgs a;
     a.q = (const half_t*)q; a.k = (const half_t*)k; a.v = (const half_t*)v; a.o = (half_t*)o;
     a.lse = lse; a.gamma_q = (const half_t*)gamma_q; a.noise = noise; a.lse_pert = lse_pert;
@@ -567,7 +612,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     const float tau = noise ? d->tau : 1.f;
     a.c2 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.q_eps = d->q_norm_eps; a.causal = d->causal ? 1 : 0; a.q_norm = d->q_norm ? 1 : 0;
-    a.n_split = 1; a.ws = nullptr; a.col_sum = col_sum; a.col_sumsq = col_sumsq; a.probs = probs; a.io16 = io16 ? 1 : 0;
+    a.n_split = 1; a.ws = nullptr; a.col_sum = col_sum; a.col_sumsq = col_sumsq; a.probs = probs; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
     // K/V tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base
     // (with room for the blocks the pipelines request past the end, which must stay representable to read as zeros)
     if (((int64_t)d->seq_kv + 2048) * d->k_stride_s * 2 > 0x7fffffffLL || ((int64_t)d->seq_kv + 2048) * d->v_stride_s * 2 > 0x7fffffffLL)
@@ -584,7 +629,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     // 256 queries) when that still fills the chip -- one workgroup per CU for unmasked attention, two rounds under a
     // causal mask, where workgroups differ in length; otherwise 4 waves x 32 (two workgroups per CU).
     const bool wide = noise_kernel_wide(d);
-#define TRN_LAUNCH(D_, NW_) launch_fwd<D_, NW_, true>(a, s)
+#define TRN_LAUNCH(D_, NW_) launch_fwd<D_, NW_>(a, s)
     if (d->head_dim == 128) e = wide ? TRN_LAUNCH(128, 8) : TRN_LAUNCH(128, 4);
     else e = wide ? TRN_LAUNCH(64, 8) : TRN_LAUNCH(64, 4);
 #undef TRN_LAUNCH

@@ -96,11 +96,20 @@ def _scale(scale: Optional[float], head_dim: int) -> float:
     return head_dim ** -0.5 if scale is None else float(scale)
 
 
+def _noise_operand(mod: "FusedModule", n4: torch.Tensor) -> torch.Tensor:
+    """The noise as the kernels read it: fp32 or fp16 rows of unit innermost stride at any pitch (the reference's noise is
+    fp16 with an arbitrary key count, convert_eval_rms.py:201).  Anything else is copied into an fp32 workspace."""
+    if n4.dtype in (torch.float32, torch.float16) and n4.stride(3) == 1:
+        return n4
+    buf = mod._workspace("noise32", tuple(n4.shape), torch.float32, n4.device)
+    buf.copy_(n4)
+    return buf
+
+
 def _noise_fp32(mod: "FusedModule", n4: torch.Tensor) -> torch.Tensor:
-    """The noise as the kernels read it: fp32, unit innermost stride, base and every pitch a multiple of 16 bytes
-    (they fetch it with 16-byte loads).  The reference's noise is fp16 (convert_eval_rms.py:201) and its key count
-    P + M is arbitrary, so anything else is copied into a workspace whose rows are padded to a multiple of 4 floats;
-    the padding is never read as a key (the kernels mask by key index, with selects)."""
+    """The noise as the un-reduced form reads it: fp32, base and every pitch a multiple of 16 bytes.  Anything else is
+    copied into a workspace whose rows are padded to a multiple of 4 floats; the padding is never read as a key (the
+    kernel masks by key index, with selects)."""
     ok = (n4.dtype == torch.float32 and n4.stride(3) == 1 and n4.data_ptr() % 16 == 0
           and all(n4.stride(i) % 4 == 0 for i in range(3)))
     if ok:
@@ -113,15 +122,12 @@ def _noise_fp32(mod: "FusedModule", n4: torch.Tensor) -> torch.Tensor:
     return view
 
 
-def _half_io_ok(t: torch.Tensor, shape) -> bool:
-    """A caller-owned fp16 statistics tensor that the kernel can write directly."""
-    return t.dtype == torch.float16 and t.is_contiguous() and tuple(t.shape) == tuple(shape)
-
-
-def _half_noise_ok(n3: torch.Tensor) -> bool:
-    """fp16 noise [H, M, P+M] that the decode kernel can read as it is (8-byte pieces)."""
-    return (n3.dtype == torch.float16 and n3.dim() == 3 and n3.stride(2) == 1 and n3.data_ptr() % 8 == 0
-            and n3.stride(0) % 4 == 0 and n3.stride(1) % 4 == 0)
+def _score_outputs(mod: "FusedModule", outs, shape):
+    """The caller's statistics tensors themselves where the kernels can write them (contiguous, one dtype of fp32 and fp16),
+    fp32 workspaces otherwise."""
+    if all(t.dtype == outs[0].dtype and t.is_contiguous() and t.dtype in (torch.float32, torch.float16) for t in outs):
+        return [t.view(shape) for t in outs]
+    return [mod._workspace(f"stat32_{i}", shape, torch.float32, t.device) for i, t in enumerate(outs)]
 
 
 def _store_scores(dst: torch.Tensor, src32: torch.Tensor) -> None:
@@ -192,13 +198,10 @@ class KeyFormerAttention(FusedModule):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
         B, Hq, Sq, D = q.shape
         Skv = k.shape[2]
-        n4 = _noise_fp32(self, _as4(noise, "noise"))
+        n4 = _noise_operand(self, _as4(noise, "noise"))
         lsep = self._workspace("lse_pert", (B, Hq, Sq), torch.float32, q.device)
-        score = C_out.view(B, Hq, Skv) if C_out.dtype == torch.float32 and C_out.is_contiguous() else \
-            self._workspace("score32", (B, Hq, Skv), torch.float32, q.device)
-        sc = _scale(self.scale, D)
-        ops.attention(q, k, v, o, sc, self.causal, noise=n4, tau=self.tau, lse_pert=lsep)
-        ops.attention_colstats(q, k, lsep, sc, self.causal, score, None, noise=n4, tau=self.tau)
+        score, = _score_outputs(self, (C_out,), (B, Hq, Skv))
+        ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lsep, score, noise=n4, tau=self.tau)
         _store_scores(C_out, score)
 
 
@@ -220,16 +223,9 @@ class RoCoAttention(FusedModule):
         B, Hq, Sq, D = q.shape
         Skv = k.shape[2]
         lse = self._workspace("lse", (B, Hq, Sq), torch.float32, q.device)
-        outs = []
-        for i, c in enumerate((C_out1, C_out2)):
-            outs.append(c.view(B, Hq, Skv) if c.dtype == torch.float32 and c.is_contiguous() else
-                        self._workspace(f"stat32_{i}", (B, Hq, Skv), torch.float32, q.device))
-        sc = _scale(self.scale, D)
-        ops.attention(q, k, v, o, sc, self.causal, lse=lse)
-        if self.stats == "sums":
-            ops.attention_colstats(q, k, lse, sc, self.causal, outs[0], outs[1])
-        else:
-            ops.attention_col_mean_std(q, k, lse, sc, self.causal, outs[0], outs[1])
+        outs = _score_outputs(self, (C_out1, C_out2), (B, Hq, Skv))
+        ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lse, outs[0], outs[1],
+                                 mean_std=self.stats == "mean_std")
         _store_scores(C_out1, outs[0]); _store_scores(C_out2, outs[1])
 
 
@@ -353,29 +349,22 @@ class DecodeKeyFormer(_DecodeAppend):
         PM = K_cache.shape[1]
         lsep = self._workspace("lse_pert", (1, H, M), torch.float32, X.device)
         o = self._o_view(O2, H, M, D)
-        # few heads on a long cache: keys split over workgroups, the key scores as a second launch (fp32 on the way)
-        split = ops.attention_stats_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal) \
-            if self.reduce else 0
-        if not split and self.reduce and M <= 32 and _half_io_ok(C_out, (H, PM)) and _half_noise_ok(noise):
-            # everything fp16 as the reference's drivers allocate it: one launch, no copies on the side
-            ops.attention_with_stats_half(q[None], K_cache[None], V_cache[None], self._o_view(O2, H, M, D), self.scale,
-                                          self.causal, C_out.view(1, H, PM), None, noise=noise[None], tau=self.tau,
-                                          lse_pert=lsep)
-            return
-        n4 = _noise_fp32(self, noise[None])
-        shape = (1, H, PM) if self.reduce else (1, H, M, PM)
         if C_out.numel() != H * PM * (1 if self.reduce else M):
-            raise ValueError(f"C_out {tuple(C_out.shape)}: expected {shape[1:]}")
-        score = C_out.view(shape) if C_out.dtype == torch.float32 and C_out.is_contiguous() else \
-            self._workspace("score32", shape, torch.float32, X.device)
+            raise ValueError(f"C_out {tuple(C_out.shape)}: expected {(H, PM) if self.reduce else (H, M, PM)}")
         if self.reduce:
-            # one launch up to 32 new tokens (the key scores are a second sweep inside the attention kernel), two beyond
-            ops.attention_with_stats(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal,
-                                     score, None, noise=n4, tau=self.tau, lse_pert=lsep,
+            # one launch up to 32 new tokens (the key scores are a second sweep inside the attention kernel), unless few heads
+            # on a long cache make the library split the keys; two launches beyond
+            score, = _score_outputs(self, (C_out,), (1, H, PM))
+            split = ops.attention_stats_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
+            ops.attention_key_scores(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal, lsep, score,
+                                     noise=_noise_operand(self, noise[None]), tau=self.tau,
                                      workspace=self._split_ws(split, X.device))
         else:
+            shape = (1, H, M, PM)
+            score = C_out.view(shape) if C_out.dtype == torch.float32 and C_out.is_contiguous() else \
+                self._workspace("score32", shape, torch.float32, X.device)
             ops.attention_with_probs(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal,
-                                     score, noise=n4, tau=self.tau, lse_pert=lsep)
+                                     score, noise=_noise_fp32(self, noise[None]), tau=self.tau, lse_pert=lsep)
         _store_scores(C_out, score)
 
 
@@ -389,18 +378,11 @@ class DecodeRoCo(_DecodeAppend):
         PM = K_cache.shape[1]
         lse = self._workspace("lse", (1, H, M), torch.float32, X.device)
         o = self._o_view(O2, H, M, D)
-        # few heads on a long cache: keys split over workgroups, the statistics as a second launch (fp32 on the way)
+        # (few heads on a long cache: keys split over workgroups, the statistics as a second launch)
         split = ops.attention_stats_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
-        if not split and M <= 32 and _half_io_ok(C_out1, (H, PM)) and _half_io_ok(C_out2, (H, PM)):
-            ops.attention_with_stats_half(q[None], K_cache[None], V_cache[None], o, self.scale,
-                                          self.causal, C_out1.view(1, H, PM), C_out2.view(1, H, PM), lse=lse)
-            return
-        outs = []
-        for i, c in enumerate((C_out1, C_out2)):
-            outs.append(c.view(1, H, PM) if c.dtype == torch.float32 and c.is_contiguous() else
-                        self._workspace(f"stat32_{i}", (1, H, PM), torch.float32, X.device))
-        ops.attention_with_stats(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal,
-                                 outs[0], outs[1], lse=lse, workspace=self._split_ws(split, X.device))
+        outs = _score_outputs(self, (C_out1, C_out2), (1, H, PM))
+        ops.attention_key_scores(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal, lse, outs[0], outs[1],
+                                 workspace=self._split_ws(split, X.device))
         _store_scores(C_out1, outs[0]); _store_scores(C_out2, outs[1])
 
 

@@ -91,7 +91,7 @@ def _attn_desc(q, k, v, o, scale, causal, q_norm, q_eps, noise, tau) -> _lib.Att
     d.scale, d.causal = float(scale), int(bool(causal))
     d.q_norm, d.q_norm_eps = int(bool(q_norm)), float(q_eps)
     if noise is not None:
-        if noise.dtype == torch.float16:        # (only trn_attn_fwd_stats_half_f16 takes it; the strides count halfs)
+        if noise.dtype == torch.float16:        # (for the entry points that take it; the strides count halfs)
             _dev_half(noise, "noise")
         else:
             _dev_float(noise, "noise")
@@ -283,6 +283,33 @@ def attention_with_stats_half(q, k, v, o, scale: float, causal: bool, out_sum: O
     st = lib.trn_attn_fwd_stats_half_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), None, _ptr(noise),
                                          _ptr(lse_pert), _ptr(out_sum), _ptr(out_sumsq), _stream(q))
     _lib.check("trn_attn_fwd_stats_half_f16", st)
+
+
+def attention_key_scores(q, k, v, o, scale: float, causal: bool, rows: torch.Tensor, out1: Optional[torch.Tensor],
+                         out2: Optional[torch.Tensor] = None, noise: Optional[torch.Tensor] = None, tau: float = 1.0,
+                         mean_std: bool = False, workspace: Optional[torch.Tensor] = None) -> None:
+    """`attention_with_stats` for any element types: noise float32 or float16 with unit innermost stride at any pitch, out1 /
+    out2 both float32 or both float16 [B,Hq,Skv] contiguous.  rows float32 [B,Hq,Sq] receives the row normalisers.
+    mean_std: out1 / out2 are the mean and standard deviation (no noise then)."""
+    d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, noise, tau)
+    B, Hq, Sq, _ = q.shape
+    Skv = k.shape[2]
+    _need(rows is not None, "rows is required")
+    _row_stat(rows, "rows", (B, Hq, Sq))
+    outs = [t for t in (out1, out2) if t is not None]
+    _need(len(outs) > 0 and all(t.dtype == outs[0].dtype for t in outs), "expected one or two statistics of one dtype")
+    half = outs[0].dtype == torch.float16
+    for t, n in ((out1, "out1"), (out2, "out2")):
+        if t is not None:
+            (_dev_half if half else _dev_float)(t, n)
+            _need(tuple(t.shape) == (B, Hq, Skv) and t.is_contiguous(), f"{n}: expected contiguous {(B, Hq, Skv)}")
+    if workspace is not None:
+        _need(workspace.is_cuda and workspace.is_contiguous() and workspace.dtype == torch.uint8, "workspace: expected a contiguous uint8 GPU tensor")
+    st = _lib.load().trn_attn_key_scores_f16(
+        C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(noise), int(noise is not None and noise.dtype == torch.float16),
+        _ptr(rows), _ptr(out1), _ptr(out2), int(half), int(mean_std), _ptr(workspace),
+        workspace.numel() if workspace is not None else 0, _stream(q))
+    _lib.check("trn_attn_key_scores_f16", st)
 
 
 def prenorm_qkv(x: torch.Tensor, gamma: Optional[torch.Tensor], wq, wk, wv, q_out, k_out, v_out,
