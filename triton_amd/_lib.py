@@ -111,6 +111,25 @@ def load() -> C.CDLL:
     return lib
 
 
+_host = None
+
+
+def host():
+    """The native host side (_host.so: argument checks and launches of the hot paths), loaded once."""
+    global _host
+    if _host is None:
+        load()                          # (reports a library that is not built)
+        import torch  # noqa: F401      (its shared libraries must be in the process first)
+        try:
+            from . import _host as h
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(HERE, '_host.so')} cannot be loaded ({e}); run `python -m triton_amd.build`. "
+                              "There is no fallback path.") from e
+        h.set_error_class(TrnError)
+        _host = h
+    return _host
+
+
 def check(fn: str, status: int) -> None:
     if status != 0:
         name = load().trn_status_name(status).decode()

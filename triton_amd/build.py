@@ -1,6 +1,6 @@
-"""Build recipe for libtrinity_hip.so: hipcc, gfx950 only, in-tree output.
+"""Build recipe for libtrinity_hip.so (hipcc, gfx950 only) and _host.so (g++), in-tree output.
 
-    python -m triton_amd.build          # compile every csrc/*.hip and link
+    python -m triton_amd.build          # compile every csrc/*.hip and link; compile csrc/host/host.cpp against torch
 
 Packed-FP32 VALU instructions are disabled for all device code (the flag below); the
 host pass prints a harmless "unknown target feature" warning for it.
@@ -11,11 +11,13 @@ import concurrent.futures as cf
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "libtrinity_hip.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -42,6 +44,26 @@ def _compile(src: str) -> str:
     return obj
 
 
+def build_host() -> str:
+    """The host side of the modules (csrc/host/host.cpp): a CPython extension over torch's C++ tensors, linked to
+    libtrinity_hip.so beside it."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           *[f"-isystem{p}" for p in (*include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"])],
+           os.path.join(CSRC, "host", "host.cpp"), "-o", HOST_PATH, f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu",
+           "-ltorch_python", f"-L{HERE}", "-ltrinity_hip", "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{r.stdout}\n{r.stderr}")
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
+    return HOST_PATH
+
+
 def build(verbose: bool = True, jobs: int = 6) -> str:
     os.makedirs(OBJ_DIR, exist_ok=True)
     srcs = sources()
@@ -51,8 +73,9 @@ def build(verbose: bool = True, jobs: int = 6) -> str:
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    build_host()
     if verbose:
-        print(f"built {LIB_PATH} from {len(srcs)} sources")
+        print(f"built {LIB_PATH} from {len(srcs)} sources, and {HOST_PATH}")
     return LIB_PATH
 
 

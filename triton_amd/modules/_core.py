@@ -27,11 +27,40 @@ eager call -- the call the reference's drivers make before capturing a graph.
 """
 from __future__ import annotations
 
+import functools
 from typing import Dict, List, Optional, Tuple
 
 import torch
 
-from .. import ops
+from .. import _lib, ops
+
+
+def _workspace_in(ws: Dict[Tuple, torch.Tensor], owner: str, name: str, shape, dtype, device) -> torch.Tensor:
+    key = (name, tuple(shape), dtype, str(device))
+    t = ws.get(key)
+    if t is None:
+        if torch.cuda.is_current_stream_capturing():
+            raise RuntimeError(
+                f"{owner}.forward: first call for shapes {tuple(shape)} is inside a graph "
+                "capture; call forward once eagerly first (as the reference's drivers do)")
+        t = torch.empty(shape, dtype=dtype, device=device)
+        ws[key] = t
+    return t
+
+
+_HOST_DTYPES = {"Half": torch.float16, "Float": torch.float32, "Byte": torch.uint8}
+
+
+def _workspace_for_host(ws, owner, name, shape, dtype, device_index, zeroed):
+    """The native side's first look-up of a workspace: the module's dictionary is where it lives."""
+    dt, dev = _HOST_DTYPES.get(dtype), torch.device("cuda", device_index)
+    if dt is None:
+        raise ValueError(f"expected float16 tensors, got {dtype}")
+    fresh = (name, tuple(shape), dt, str(dev)) not in ws
+    t = _workspace_in(ws, owner, name, shape, dt, dev)
+    if zeroed and fresh:
+        t.zero_()
+    return t
 
 
 class FusedModule:
@@ -48,38 +77,41 @@ class FusedModule:
 
     def __init__(self) -> None:
         self._ws: Dict[Tuple, torch.Tensor] = {}
+        self._host = None                   # (the native side, loaded with the first forward)
+        self._hws = None                    # its view of these workspaces
 
     def _workspace(self, name: str, shape, dtype, device) -> torch.Tensor:
-        key = (name, tuple(shape), dtype, str(device))
-        t = self._ws.get(key)
-        if t is None:
-            if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError(
-                    f"{type(self).__name__}.forward: first call for shapes {tuple(shape)} is inside a graph "
-                    "capture; call forward once eagerly first (as the reference's drivers do)")
-            t = torch.empty(shape, dtype=dtype, device=device)
-            self._ws[key] = t
-        return t
+        return _workspace_in(self._ws, type(self).__name__, name, shape, dtype, device)
 
     def release(self) -> None:
         """Drop every cached workspace.  Graphs captured from this instance must not be replayed afterwards."""
         self._ws.clear()
+        if self._hws is not None:
+            self._hws.clear()
 
-    def _split(self, args, kwargs):
+    def forward(self, *args, **kwargs) -> None:
         n = len(self.TENSOR_PARAMS)
         if len(args) < n:
             raise TypeError(f"forward expects tensors {self.TENSOR_PARAMS}, got {len(args)} positional arguments")
         for k in kwargs:
             if not k.startswith("block_"):
                 raise TypeError(f"forward got an unexpected keyword argument '{k}'")
-        return dict(zip(self.TENSOR_PARAMS, args[:n]))     # trailing positionals are block sizes: ignored
-
-    def forward(self, *args, **kwargs) -> None:
-        self._run(**self._split(args, kwargs))
+        if len(args) > n:
+            args = args[:n]                                # trailing positionals are block sizes: ignored
+        if self._host is None:
+            self._host = _lib.host()
+            self._hws = self._host.Workspaces(functools.partial(_workspace_for_host, self._ws, type(self).__name__))
+        if not self._native(self._host, self._hws, *args):
+            self._run(*args)
 
     __call__ = forward
 
-    def _run(self, **tensors) -> None:  # pragma: no cover - abstract
+    def _native(self, host, ws, *tensors) -> bool:
+        """The whole forward in one native call (csrc/host/host.cpp); False, with nothing done, for tensors whose layout
+        or type that call does not cover: `_run` then takes them."""
+        return False
+
+    def _run(self, *tensors) -> None:  # pragma: no cover - abstract
         raise NotImplementedError
 
 
@@ -146,6 +178,9 @@ class RMSNorm(FusedModule):
         super().__init__()
         self.eps = eps
 
+    def _native(self, host, ws, X, X_norm, gamma):
+        return host.rmsnorm_forward(self.eps, X, X_norm, gamma)
+
     def _run(self, X, X_norm, gamma):
         ops.rmsnorm(X.view(-1, X.shape[-1]), gamma, X_norm.view(-1, X.shape[-1]), self.eps)
 
@@ -157,6 +192,9 @@ class Attention(FusedModule):
     def __init__(self, scale: Optional[float] = None, causal: bool = True):
         super().__init__()
         self.scale, self.causal = scale, causal
+
+    def _native(self, host, ws, K, O, Q, V):
+        return host.attention_forward(self.scale, self.causal, K, O, Q, V)
 
     def _run(self, K, O, Q, V):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
@@ -172,6 +210,9 @@ class QKNormAttention(FusedModule):
     def __init__(self, scale: Optional[float] = None, causal: bool = True, eps: float = 1e-5):
         super().__init__()
         self.scale, self.causal, self.eps = scale, causal, eps
+
+    def _native(self, host, ws, K, O, Q, V, gamma_k, gamma_q):
+        return host.qknorm_forward(ws, self.scale, self.causal, self.eps, K, O, Q, V, gamma_k, gamma_q)
 
     def _run(self, K, O, Q, V, gamma_k, gamma_q):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
@@ -193,6 +234,9 @@ class KeyFormerAttention(FusedModule):
     def __init__(self, scale: Optional[float] = None, causal: bool = True, tau: float = 1.0):
         super().__init__()
         self.scale, self.causal, self.tau = scale, causal, tau
+
+    def _native(self, host, ws, C_out, K, O, Q, V, noise):
+        return host.key_scores_forward(ws, self.scale, self.causal, self.tau, False, K, O, Q, V, C_out, None, noise)
 
     def _run(self, C_out, K, O, Q, V, noise):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
@@ -218,6 +262,9 @@ class RoCoAttention(FusedModule):
             raise ValueError("stats: expected 'sums' or 'mean_std'")
         self.scale, self.causal, self.stats = scale, causal, stats
 
+    def _native(self, host, ws, C_out1, C_out2, K, O, Q, V):
+        return host.key_scores_forward(ws, self.scale, self.causal, 1.0, self.stats == "mean_std", K, O, Q, V, C_out1, C_out2, None)
+
     def _run(self, C_out1, C_out2, K, O, Q, V):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
         B, Hq, Sq, D = q.shape
@@ -240,6 +287,9 @@ class PreNormBlock(FusedModule):
                  eps: float = 1e-5, norm: bool = True):
         super().__init__()
         self.head_dim, self.scale, self.causal, self.eps, self.norm = head_dim, scale, causal, eps, norm
+
+    def _native(self, host, ws, O, WK, WQ, WV, X, gamma):
+        return host.prenorm_forward(ws, self.head_dim, self.scale, self.causal, self.eps, self.norm, O, WK, WQ, WV, X, gamma)
 
     def _run(self, O, WK, WQ, WV, X, gamma):
         D = self.head_dim
@@ -272,6 +322,10 @@ class _DecodeAppend(FusedModule):
         if o_layout not in ("token_major", "head_major"):
             raise ValueError("o_layout: expected 'token_major' or 'head_major'")
         self.head_dim, self.prenorm, self.scale, self.causal, self.o_layout = head_dim, prenorm, scale, causal, o_layout
+
+    def _native_step(self, host, ws, K_cache, O2, V_cache, WK, WQ, WV, X, q_norm=False, tau=1.0, C1=None, C2=None, noise=None):
+        return host.decode_forward(ws, self.head_dim, self.prenorm, self.scale, self.causal, self.o_layout == "head_major", q_norm,
+                                   tau, K_cache, O2, V_cache, WK, WQ, WV, X, C1, C2, noise)
 
     def _project(self, X, WQ, WK, WV, K_cache, V_cache):
         M, N = X.shape
@@ -316,6 +370,9 @@ class DecodeVanilla(_DecodeAppend):
     """Vanila.forward / PreNorm.forward (ref_rms.py:45-83 / 101-127)."""
     TENSOR_PARAMS = ["K_cache", "O2", "V_cache", "WK", "WQ", "WV", "X"]
 
+    def _native(self, host, ws, K_cache, O2, V_cache, WK, WQ, WV, X):
+        return self._native_step(host, ws, K_cache, O2, V_cache, WK, WQ, WV, X)
+
     def _run(self, K_cache, O2, V_cache, WK, WQ, WV, X):
         q, _ = self._project(X, WQ, WK, WV, K_cache, V_cache)
         self._attend(q, K_cache, V_cache, O2)
@@ -325,6 +382,9 @@ class DecodeQKNorm(_DecodeAppend):
     """QKNorm.forward (ref_rms.py:197-231): q and the newly appended k rows are normalised
     (no eps, no weight); the cached prefix is used as stored."""
     TENSOR_PARAMS = ["K_cache", "O2", "V_cache", "WK", "WQ", "WV", "X"]
+
+    def _native(self, host, ws, K_cache, O2, V_cache, WK, WQ, WV, X):
+        return self._native_step(host, ws, K_cache, O2, V_cache, WK, WQ, WV, X, True)
 
     def _run(self, K_cache, O2, V_cache, WK, WQ, WV, X):
         q, P = self._project(X, WQ, WK, WV, K_cache, V_cache)
@@ -342,6 +402,9 @@ class DecodeKeyFormer(_DecodeAppend):
     def __init__(self, head_dim: int, tau: float = 1.5, reduce: bool = True, **kw):
         super().__init__(head_dim, **kw)
         self.tau, self.reduce = tau, reduce
+
+    def _native(self, host, ws, C_out, K_cache, O2, V_cache, WK, WQ, WV, X, noise):
+        return self.reduce and self._native_step(host, ws, K_cache, O2, V_cache, WK, WQ, WV, X, False, self.tau, C_out, None, noise)
 
     def _run(self, C_out, K_cache, O2, V_cache, WK, WQ, WV, X, noise):
         q, _ = self._project(X, WQ, WK, WV, K_cache, V_cache)
@@ -372,6 +435,9 @@ class DecodeRoCo(_DecodeAppend):
     """RoCo.forward (ref_rms.py:249-280): C_out1 = weights.sum(dim=1), C_out2 = weights.pow(2).sum(dim=1)."""
     TENSOR_PARAMS = ["C_out1", "C_out2", "K_cache", "O2", "V_cache", "WK", "WQ", "WV", "X"]
 
+    def _native(self, host, ws, C_out1, C_out2, K_cache, O2, V_cache, WK, WQ, WV, X):
+        return self._native_step(host, ws, K_cache, O2, V_cache, WK, WQ, WV, X, False, 1.0, C_out1, C_out2)
+
     def _run(self, C_out1, C_out2, K_cache, O2, V_cache, WK, WQ, WV, X):
         q, _ = self._project(X, WQ, WK, WV, K_cache, V_cache)
         H, M, D = q.shape
@@ -391,6 +457,9 @@ class LoRA(FusedModule):
     intermediates C = X W, D = X A, E = D B stay inside: D is a workspace, C and E never leave the kernels).
     Two launches: {O, D} = X {W, A}, then O = D B + O."""
     TENSOR_PARAMS = ["A", "B", "O", "W", "X"]
+
+    def _native(self, host, ws, A, B, O, W, X):
+        return host.lora_forward(ws, A, B, O, W, X)
 
     def _run(self, A, B, O, W, X):
         M, N = X.shape
@@ -413,6 +482,9 @@ class GatedMLP(FusedModule):
         if gate not in ("sigmoid", "silu"):
             raise ValueError("gate: expected 'sigmoid' or 'silu'")
         self.gate = gate
+
+    def _native(self, host, ws, O, W1, W2, X):
+        return host.gmlp_forward(ws, self.gate == "silu", O, W1, W2, X)
 
     def _run(self, O, W1, W2, X):
         M, K = X.shape

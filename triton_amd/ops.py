@@ -43,15 +43,7 @@ def _stream(t: torch.Tensor):
 
 def rmsnorm(x: torch.Tensor, gamma: Optional[torch.Tensor], y: torch.Tensor, eps: float) -> None:
     """y = RMSNorm(x) over the last axis; x, y [rows, cols] (row stride free), gamma [cols] or None."""
-    _dev_half(x, "x"); _dev_half(y, "y")
-    _need(x.dim() == 2 and y.shape == x.shape, f"x {tuple(x.shape)} / y {tuple(y.shape)}: expected equal 2-D shapes")
-    if gamma is not None:
-        _dev_half(gamma, "gamma")
-        _need(gamma.shape == (x.shape[1],), f"gamma {tuple(gamma.shape)}: expected ({x.shape[1]},)")
-    lib = _lib.load()
-    st = lib.trn_rmsnorm_f16(_ptr(x), _ptr(gamma), _ptr(y), 1, x.shape[0], x.shape[1],
-                             0, x.stride(0), 0, y.stride(0), 0, float(eps), _stream(x))
-    _lib.check("trn_rmsnorm_f16", st)
+    _lib.host().rmsnorm(x, gamma, y, eps)
 
 
 def head_rmsnorm(x: torch.Tensor, gamma: Optional[torch.Tensor], y: torch.Tensor, eps: float,
@@ -134,6 +126,9 @@ def attention(q, k, v, o, scale: float, causal: bool, lse: Optional[torch.Tensor
     workspace: optional zero-initialised uint8 tensor of attention_workspace_bytes(...) bytes (decode shapes with
     few heads then split their keys over several workgroups); the string "static" takes the library's own static
     device array instead (nothing is allocated; one such call at a time per GPU)."""
+    if not isinstance(workspace, str):
+        _lib.host().attention(q, k, v, o, scale, causal, lse, q_norm, gamma_q, q_eps, noise, tau, lse_pert, workspace)
+        return
     d = _attn_desc(q, k, v, o, scale, causal, q_norm, q_eps, noise, tau)
     B, Hq, Sq, _ = q.shape
     _row_stat(lse, "lse", (B, Hq, Sq)); _row_stat(lse_pert, "lse_pert", (B, Hq, Sq))
@@ -141,23 +136,11 @@ def attention(q, k, v, o, scale: float, causal: bool, lse: Optional[torch.Tensor
         _dev_half(gamma_q, "gamma_q")
         _need(gamma_q.shape == (q.shape[3],), "gamma_q: expected (head_dim,)")
     _need(noise is None or lse_pert is not None, "noise given without lse_pert")
-    lib = _lib.load()
-    if isinstance(workspace, str):
-        _need(workspace == "static", 'workspace: a uint8 GPU tensor, None, or "static"')
-        _static_scratch_ready(q.device)
-        st = lib.trn_attn_fwd_noalloc_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(gamma_q),
-                                          _ptr(noise), _ptr(lse_pert), _stream(q))
-        _lib.check("trn_attn_fwd_noalloc_f16", st)
-        return
-    if workspace is not None:
-        _need(workspace.is_cuda and workspace.is_contiguous() and workspace.dtype == torch.uint8, "workspace: expected a contiguous uint8 GPU tensor")
-        st = lib.trn_attn_fwd_ws_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(gamma_q),
-                                     _ptr(noise), _ptr(lse_pert), _ptr(workspace), workspace.numel(), _stream(q))
-        _lib.check("trn_attn_fwd_ws_f16", st)
-        return
-    st = lib.trn_attn_fwd_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(gamma_q),
-                              _ptr(noise), _ptr(lse_pert), _stream(q))
-    _lib.check("trn_attn_fwd_f16", st)
+    _need(workspace == "static", 'workspace: a uint8 GPU tensor, None, or "static"')
+    _static_scratch_ready(q.device)
+    st = _lib.load().trn_attn_fwd_noalloc_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(gamma_q),
+                                              _ptr(noise), _ptr(lse_pert), _stream(q))
+    _lib.check("trn_attn_fwd_noalloc_f16", st)
 
 
 def attention_kernel_name(q, k, v, o, scale: float, causal: bool, with_noise: bool = False) -> str:
@@ -317,28 +300,7 @@ def prenorm_qkv(x: torch.Tensor, gamma: Optional[torch.Tensor], wq, wk, wv, q_ou
     """Q,K,V = RMSNorm(x; gamma, eps) @ W{q,k,v}  (norm=False: x @ W).
     x [T, hidden]; w* [hidden, n_*]; *_out indexed [head, token, head_dim] (any view with unit
     innermost stride: a permuted token-major buffer, a head-major buffer, or rows of a KV cache)."""
-    _dev_half(x, "x")
-    _need(x.dim() == 2, "x: expected [tokens, hidden]")
-    T, K = x.shape
-    for w, n in ((wq, "wq"), (wk, "wk"), (wv, "wv")):
-        _dev_half(w, n)
-        _need(w.dim() == 2 and w.shape[0] == K, f"{n}: expected [hidden={K}, n_out], got {tuple(w.shape)}")
-    _need(wk.shape[1] == wv.shape[1], "wk and wv must have the same number of columns")
-    D = q_out.shape[-1]
-    for o, w, n in ((q_out, wq, "q_out"), (k_out, wk, "k_out"), (v_out, wv, "v_out")):
-        _dev_half(o, n)
-        _need(o.dim() == 3 and o.shape[1] == T and o.shape[2] == D and o.shape[0] * D == w.shape[1],
-              f"{n}: expected [heads, {T}, {D}] with heads*{D} == {w.shape[1]}, got {tuple(o.shape)}")
-    if gamma is not None:
-        _dev_half(gamma, "gamma")
-        _need(gamma.shape == (K,), "gamma: expected (hidden,)")
-    lib = _lib.load()
-    st = lib.trn_prenorm_qkv_f16(_ptr(x), _ptr(gamma), _ptr(wq), _ptr(wk), _ptr(wv), _ptr(q_out), _ptr(k_out),
-                                 _ptr(v_out), T, K, wq.shape[1], wk.shape[1], D, x.stride(0), wq.stride(0),
-                                 wk.stride(0), wv.stride(0), q_out.stride(0), q_out.stride(1), k_out.stride(0),
-                                 k_out.stride(1), v_out.stride(0), v_out.stride(1), float(eps), int(bool(norm)),
-                                 _stream(x))
-    _lib.check("trn_prenorm_qkv_f16", st)
+    _lib.host().prenorm_qkv(x, gamma, wq, wk, wv, q_out, k_out, v_out, eps, norm)
 
 
 def linear(x: torch.Tensor, weights, outs, addends=None) -> None:
