@@ -79,9 +79,10 @@ void* attn_static_scratch();
 
 // The forward pass without score perturbation on the 16x16x32 MFMA (attn_fwd16.hip).  Narrow: 4 waves x 32 queries
 // per workgroup; Wide: 8 waves x 32 consecutive queries; Paired: 8 waves, two 128-query tiles from opposite ends of
-// the sequence (causal problems whose grid is a single round).
-enum class Attn16Shape { Narrow, Wide, Paired };
-Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int head_dim, bool causal);
+// the sequence (causal problems whose grid is a single round); Split: 8 waves on 128 queries, two groups of four that
+// take every other 64-key tile each (small grids, long walks).
+enum class Attn16Shape { Narrow, Wide, Paired, Split };
+Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal);
 hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, hipStream_t stream);
 // Name of the kernel instantiation that launch_attn_fwd16 runs for this shape, as a profiler prints it.
 const char* attn_fwd16_kernel_name(int head_dim, Attn16Shape shape);

@@ -457,7 +457,7 @@ extern "C" const char* trn_attn_fwd_kernel_name(const trn_attn_desc* d, int32_t 
     const bool d128 = d->head_dim == 128;
     if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0))
         return attn_decode_kernel_name(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
-    if (!with_noise) return attn_fwd16_kernel_name(d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->head_dim, d->causal != 0));
+    if (!with_noise) return attn_fwd16_kernel_name(d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0));
     const bool wide = noise_kernel_wide(d);
     if (d128) return wide ? "trn::attn_fwd_kernel<128, 8, true>" : "trn::attn_fwd_kernel<128, 4, true>";
     return wide ? "trn::attn_fwd_kernel<64, 8, true>" : "trn::attn_fwd_kernel<64, 4, true>";
@@ -624,7 +624,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         return launch_attn_decode(a, d->head_dim, workspace, workspace_bytes, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     // Without score perturbation: the 16x16x32 kernel, in the workgroup shape its launcher's rule picks.
     if (!noise)
-        return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->head_dim, d->causal != 0), s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+        return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0), s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     // With it: 8 waves x 32 queries per workgroup (one workgroup per CU; each K/V stage is fetched from L2 once per
     // 256 queries) when that still fills the chip -- one workgroup per CU for unmasked attention, two rounds under a
     // causal mask, where workgroups differ in length; otherwise 4 waves x 32 (two workgroups per CU).

@@ -29,6 +29,11 @@
 
 namespace trn {
 
+// What the two groups of four waves of an eight-wave workgroup do: kPlain, the same tile of 256 queries; kPaired, two
+// tiles of 128 queries from the two ends of a causal problem; kSplit, the same 128 queries, each group every other
+// 64-key tile.
+enum { kPlain, kPaired, kSplit };
+
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
@@ -58,25 +63,34 @@ template <int D> __device__ __forceinline__ int swz16(int r) {
 
 struct Scores16 { float4_t s[2][2]; };      // [key half][query block]
 
-template <int D, int NW, bool PAIRED>
-__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(const AttnArgs a) {
-    static_assert(!PAIRED || NW == 8, "paired query tiles are two groups of four waves");
 #if defined(__HIP_DEVICE_COMPILE__)
+template <int D, int NW, int MODE>
+__device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
+    constexpr bool PAIRED = MODE == kPaired, SPLIT = MODE == kSplit;
+    static_assert(MODE == kPlain || NW == 8, "paired query tiles and split keys are two groups of four waves");
+    constexpr int GW = SPLIT ? 4 : NW;       // waves that share the K / V stages
+    constexpr int KSTEP = SPLIT ? 128 : 64;  // keys from one tile of a wave to its next
     constexpr int BN = 64;       // keys per LDS stage (two 32-key blocks)
     constexpr int NS = D / 8;    // MFMA slots per phase: 2 key halves x 2 query blocks x D/32 steps of S^T; D/16 x 2 of P V
     constexpr int NKS = D / 32;  // contraction steps of S^T
     constexpr int NOP = D / 16;  // LDS operands per phase (each feeds the MFMAs of both query blocks)
     constexpr int CPR = D / 8;   // 16-byte chunks per row
     constexpr int RPI = 64 / CPR;            // stage rows covered by one wave-wide 1 KB load
-    constexpr int NI = BN / (RPI * NW);      // such loads per wave per stage (K and V each)
-    constexpr int BM = 32 * NW;              // queries per workgroup
-    __shared__ __attribute__((aligned(1024))) half_t Ks0[BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Ks1[BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Vs0[BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Vs1[BN * D];
+    constexpr int NI = BN / (RPI * GW);      // such loads per wave per stage (K and V each)
+    constexpr int NG = SPLIT ? 2 : 1;        // groups with stages of their own
+    __shared__ __attribute__((aligned(1024))) half_t Ks0_[NG * BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Ks1_[NG * BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Vs0_[NG * BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Vs1_[NG * BN * D];
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = SPLIT ? wave >> 2 : 0, gw = SPLIT ? wave & 3 : wave;
+    half_t* const Ks0 = Ks0_ + grp * BN * D;
+    half_t* const Ks1 = Ks1_ + grp * BN * D;
+    half_t* const Vs0 = Vs0_ + grp * BN * D;
+    half_t* const Vs1 = Vs1_ + grp * BN * D;
+    const int kfirst = grp * BN;             // first key of this wave's first tile
 
     const int BH = a.B * a.Hq;
     const int j = blockIdx.x % BH;
@@ -91,16 +105,14 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
     // same amount of work and each SIMD holds one long and one short wave.  K/V staging follows the later tile; the
     // early waves stop at their own last visible tile as they do in plain mode.
     int q0, q_last, wq0;
-    bool idle = false;
     if constexpr (PAIRED) {
         const int lt = (int)(blockIdx.x / BH), ht = a.n_qtiles - 1 - lt;     // n_qtiles counts 128-query tiles here
         q0 = ht * 128; q_last = q0 + 127;
-        idle = wave >= 4 && lt == ht;                                       // odd tile count: the middle one is alone
         wq0 = (wave < 4 ? ht : lt) * 128 + (wave & 3) * 32;
-        if (idle) wq0 = a.Sq;                                               // loads clamp, stores are predicated off
+        if (wave >= 4 && lt == ht) wq0 = a.Sq;          // odd tile count: the middle one is alone (loads clamp, stores are predicated off)
     } else {
-        q0 = (a.n_qtiles - 1 - (int)(blockIdx.x / BH)) * BM; q_last = q0 + BM - 1;
-        wq0 = q0 + wave * 32;                           // first query of this wave
+        q0 = (a.n_qtiles - 1 - (int)(blockIdx.x / BH)) * (GW * 32); q_last = q0 + GW * 32 - 1;
+        wq0 = q0 + gw * 32;                             // first query of this wave
     }
     int qrow[2];
 #pragma unroll
@@ -132,6 +144,9 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
     // the sum of the block's (fp16-rounded) probabilities of each query in every row of a 16 x 16 accumulator.  Two
     // MFMAs per 32-key block instead of eight dot-product instructions, each of which costs two VALU issue slots.
     float4_t lacc[2] = {zero, zero};
+    // Split keys under a causal mask: a query may see nothing in this group's first tiles.  Its reference then stays 0
+    // with zero sums, and its first visible scores set it (any_fresh: some query of the wave is still in that state).
+    bool fresh[2] = {false, false}, any_fresh = false;
 
     int ntiles = (a.Skv + BN - 1) / BN;
     if (a.causal) ntiles = min(ntiles, (min(q_last, a.Sq - 1) + off) / BN + 1);
@@ -141,14 +156,15 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
         (void*)(a.k + b * a.kb + kvh * a.kh), 0, (int)(((int64_t)(a.Skv - 1) * a.ks + D) * 2), 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.v + b * a.vb + kvh * a.vh), 0, (int)(((int64_t)(a.Skv - 1) * a.vs + D) * 2), 0x00020000);
-    const int st_row = wave * RPI + lane / CPR;
+    const int st_row = gw * RPI + lane / CPR;
     const int st_chunk = (lane % CPR) ^ swz16<D>(st_row);
     const int kvo = (int)(st_row * a.ks * 2) + st_chunk * 16;
     const int vvo = (int)(st_row * a.vs * 2) + st_chunk * 16;
     const int krow_bytes = (int)(RPI * a.ks * 2), vrow_bytes = (int)(RPI * a.vs * 2);
-    const int ktile_bytes = (int)(BN * a.ks * 2), vtile_bytes = (int)(BN * a.vs * 2);
-#define TRN_FETCH_K(jt_, dst_) fetch_tile<NI, D, NW>(krs, &dst_[wave * RPI * D], kvo, (jt_) * ktile_bytes, krow_bytes)
-#define TRN_FETCH_V(jt_, dst_) fetch_tile<NI, D, NW>(vrs, &dst_[wave * RPI * D], vvo, (jt_) * vtile_bytes, vrow_bytes)
+    const int ktile_bytes = (int)(KSTEP * a.ks * 2), vtile_bytes = (int)(KSTEP * a.vs * 2);
+    const int kgrp_bytes = (int)(kfirst * a.ks * 2), vgrp_bytes = (int)(kfirst * a.vs * 2);
+#define TRN_FETCH_K(jt_, dst_) fetch_tile<NI, D, GW>(krs, &dst_[gw * RPI * D], kvo, kgrp_bytes + (jt_) * ktile_bytes, krow_bytes)
+#define TRN_FETCH_V(jt_, dst_) fetch_tile<NI, D, GW>(vrs, &dst_[gw * RPI * D], vvo, vgrp_bytes + (jt_) * vtile_bytes, vrow_bytes)
 
     const int wb = wq0 + off;          // key index bound of this wave's first query
     auto needs_mask = [&](int key0) { return (key0 + 32 > a.Skv) || (a.causal && key0 + 31 > wb); };
@@ -196,8 +212,12 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
         block_max(sx, smax);
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-            const float up = fmaxf(0.f, quad_max(smax[qb]));
-            const float alpha = fast_exp2(-up);
+            float up = fmaxf(0.f, quad_max(smax[qb])), alpha = fast_exp2(-up);
+            if constexpr (SPLIT) {      // a query that has seen no key yet: its first finite maximum is the reference
+                const float qm = quad_max(smax[qb]);
+                if (fresh[qb]) { up = qm == -INFINITY ? 0.f : qm; alpha = 1.f; }
+                fresh[qb] = fresh[qb] && qm == -INFINITY;
+            }
             sx.s[0][qb] = sx.s[0][qb] - up;
             sx.s[1][qb] = sx.s[1][qb] - up;
             negm[qb] = negm[qb] - up;                   // (in place, like the accumulators: a fresh vector here makes
@@ -209,6 +229,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
                                                         // skips the rescale ends up copying every accumulator)
             m[qb] = m[qb] + up;
         }
+        if constexpr (SPLIT) any_fresh = __builtin_amdgcn_ballot_w64(fresh[0] || fresh[1]) != 0;
     };
 
     const half_t one = (half_t)1.f;
@@ -280,7 +301,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
             constexpr int R0 = NS / 2 - (NS >= 16 ? 3 : 2);
             if (i == R0) { if (MAYMASK && masked_next) mask_block(sn, key0_next); }
             if (i >= R0 && i < R0 + 4) mx = max_piece(sn, i - R0, mx);
-            if (i == R0 + 3) due = __builtin_amdgcn_ballot_w64(mx > 0x41000000) != 0;       // 8.0f
+            if (i == R0 + 3) due = __builtin_amdgcn_ballot_w64(mx > 0x41000000) != 0 || (SPLIT && any_fresh);       // 8.0f
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
@@ -291,7 +312,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
     // ---- prologue: K stages 0 and 1 and V stage 0; scores of block 0; first K operands of block 1 ----
     TRN_FETCH_K(0, Ks0);
     TRN_FETCH_V(0, Vs0);
-    if (ntiles > 1) TRN_FETCH_K(1, Ks1);
+    if (SPLIT || ntiles > 1) TRN_FETCH_K(1, Ks1);
 
     // ---- Q^T B-operands: lane holds Q[qrow[qb]][32 ks + 8 g4 .. +7].  The loads go out behind the first K/V stage
     // fetches and all together, so that the workgroup's start-up pays one memory latency, not three in a row.
@@ -349,21 +370,23 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
         for (int i = 0; i < NQ; ++i) load_k(Ks0 + 32 * D, i, i);
         // block 0 sets the reference outright (every query sees key 0, so it is finite from here on)
         float smax[2];
-        mask_block(sA, 0);
+        mask_block(sA, kfirst);
         block_max(sA, smax);
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
             m[qb] = quad_max(smax[qb]);
+            if constexpr (SPLIT) { fresh[qb] = m[qb] == -INFINITY; m[qb] = fresh[qb] ? 0.f : m[qb]; }
             negm[qb] = float4_t{-m[qb], -m[qb], -m[qb], -m[qb]};
             sA.s[0][qb] = sA.s[0][qb] - m[qb];
             sA.s[1][qb] = sA.s[1][qb] - m[qb];
         }
+        if constexpr (SPLIT) any_fresh = __builtin_amdgcn_ballot_w64(fresh[0] || fresh[1]) != 0;
     }
 
     // One 64-key tile jt.  Kc = its own K stage (block 1 still has operands to give), Kn = the next tile's
     // K stage, Vc = its V stage, Vn = the other V stage.
     auto tile = [&](auto maymask_tag, int jt, half_t* Kc, const half_t* Kn, const half_t* Vc, half_t* Vn) __attribute__((always_inline)) {
-        const int kv0 = jt * BN;
+        const int kv0 = kfirst + jt * KSTEP;
         auto handover = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's share of stages Kn and Vc is in LDS
             __syncthreads();                      // ... and everyone's; Kc and Vn have had their last readers
@@ -375,20 +398,22 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
         auto none = [&]() __attribute__((always_inline)) {};
         // (Past the last tile a K stage holds stale rows; scores computed from them are masked away.)
         step(needs_mask(kv0 + 32), maymask_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover);
-        step(needs_mask(kv0 + 64), maymask_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + 64, none);
+        step(needs_mask(kv0 + KSTEP), maymask_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + KSTEP, none);
     };
     // Under a causal mask the waves of a workgroup see different numbers of tiles: a wave computes the tiles that
     // hold a key visible to one of its queries, and for the rest only keeps up the staging it shares with the
     // others (its part of every refill, and the barrier), leaving its SIMD to the wave that still computes.
     int nlive = ntiles;
     if (a.causal) nlive = min(ntiles, (min(wq0 + 31, a.Sq - 1) + off) / BN + 1);
-    if (idle) nlive = 0;
+    const int nloop = SPLIT ? (ntiles + 1) >> 1 : ntiles;
+    if constexpr (SPLIT) nlive = (nlive - grp + 1) >> 1;
+    if (wq0 >= a.Sq) nlive = 0;             // no query of its own: the ragged end of a tile, or the middle tile of an odd count
     // The leading tiles whose blocks (and the first block of the tile after) lie wholly inside the keys and, under a
     // causal mask, before this wave's first query: a loop of their own without the mask test.  needs_mask is monotone
     // in the key index, so they are the tiles jt with 64 jt + 96 <= Skv and 64 jt + 95 <= wb; taken in pairs (the
     // stages alternate), the rest goes through the general loop.
-    int n_plain = (a.Skv - 96 >= 0) ? (a.Skv - 96) / BN + 1 : 0;
-    if (a.causal) n_plain = min(n_plain, wb - 95 >= 0 ? (wb - 95) / BN + 1 : 0);
+    int n_plain = max(0, a.Skv - 32 - kfirst) / KSTEP;
+    if (a.causal) n_plain = min(n_plain, max(0, wb - 31 - kfirst) / KSTEP);
     n_plain = min(n_plain, nlive) & ~1;
     for (int jt = 0; jt < n_plain; jt += 2) {
         tile(std::false_type{}, jt, Ks0, Ks1, Vs0, Vs1);
@@ -398,13 +423,13 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
         tile(std::true_type{}, jt, Ks0, Ks1, Vs0, Vs1);
         if (jt + 1 < nlive) tile(std::true_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
     }
-    for (int jt = nlive; jt < ntiles; ++jt) {
+    for (int jt = nlive; jt < nloop; ++jt) {
         half_t* Kc = (jt & 1) ? Ks1 : Ks0;
         half_t* Vn = (jt & 1) ? Vs0 : Vs1;
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
-        if (jt + 2 < ntiles) TRN_FETCH_K(jt + 2, Kc);
-        if (jt + 1 < ntiles) TRN_FETCH_V(jt + 1, Vn);
+        if (jt + 2 < nloop) TRN_FETCH_K(jt + 2, Kc);
+        if (jt + 1 < nloop) TRN_FETCH_V(jt + 1, Vn);
     }
 #undef TRN_FETCH_K
 #undef TRN_FETCH_V
@@ -417,7 +442,69 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
     for (int qb = 0; qb < 2; ++qb) { l[qb] = lacc[qb][0]; inv[qb] = 1.0f / l[qb]; }
     __builtin_amdgcn_s_waitcnt(0x0f70);                // this wave's last refills (past the end, unread) have landed ...
     __syncthreads();                                   // ... and everyone's; every wave is done with the K/V stages
-    {
+    if constexpr (SPLIT) {
+        // The groups hold partial results of the same queries.  Waves w and w + 4 exchange (m, l) and halves of O^T
+        // lane by lane: group 0 finishes the first D/2 columns, group 1 the others.  A wave that took no tile, or a
+        // query that saw no key of its group, has zero sums and weighs nothing.
+        constexpr int kStat = D == 128 ? 5120 : 2560;   // (floats) the row statistics lie behind the transposing regions
+        float* stat = reinterpret_cast<float*>(Ks1_) + kStat;       // [8 waves][2 query blocks][16 queries] {m, l}
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            if (nlive == 0 || fresh[qb]) m[qb] = -INFINITY;
+            if (g4 == 0) {
+                stat[((wave * 2 + qb) * 16 + n) * 2] = m[qb];
+                stat[((wave * 2 + qb) * 16 + n) * 2 + 1] = l[qb];
+            }
+        }
+        constexpr int NH = NOP / 2;
+        float4_t* mine = reinterpret_cast<float4_t*>(wave < 4 ? Ks0_ : Vs0_) + (wave & 3) * NH * 2 * 64;
+        const float4_t* theirs = reinterpret_cast<const float4_t*>(wave < 4 ? Vs0_ : Ks0_) + (wave & 3) * NH * 2 * 64;
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) mine[(i * 2 + qb) * 64 + lane] = grp == 0 ? oacc[NH + i][qb] : oacc[i][qb];
+        __syncthreads();
+        float wo[2], wt[2];
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            const float mt = stat[(((wave ^ 4) * 2 + qb) * 16 + n) * 2], lt = stat[(((wave ^ 4) * 2 + qb) * 16 + n) * 2 + 1];
+            const float ms = fmaxf(m[qb], mt);            // (finite: every query sees a key)
+            wo[qb] = fast_exp2(m[qb] - ms); wt[qb] = fast_exp2(mt - ms);
+            l[qb] = l[qb] * wo[qb] + lt * wt[qb];
+            m[qb] = ms;
+            inv[qb] = 1.0f / l[qb];
+        }
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                const float4_t own = grp == 0 ? oacc[i][qb] : oacc[NH + i][qb];
+                oacc[i][qb] = own * wo[qb] + theirs[(i * 2 + qb) * 64 + lane] * wt[qb];
+            }
+        constexpr int DP = D / 2, OP = DP + 4, LPRW = DP / 8, RPS = 64 / LPRW;
+        half_t* ot = (wave < 4 ? Vs1_ : Ks1_) + (wave & 3) * 32 * OP;
+        static_assert(4 * 32 * OP * 2 <= kStat * 4 && kStat * 4 + 2048 <= 2 * BN * D * 2, "the stage holds both");
+        const int orow = lane / LPRW, ocol = (lane % LPRW) * 8;
+        half_t* ob = a.o + b * a.ob + head * a.oh + grp * DP;
+#pragma unroll
+        for (int dbl = 0; dbl < NH; ++dbl)
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                half4_t ov;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ov[e] = (half_t)(oacc[dbl][qb][e] * inv[qb]);
+                *reinterpret_cast<half4_t*>(&ot[(16 * qb + n) * OP + dbl * 16 + 4 * g4]) = ov;
+            }
+#pragma unroll
+        for (int jj = 0; jj < 32 / RPS; ++jj) {
+            const int r = jj * RPS + orow;
+            const uint2_t lo = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol]);
+            const uint2_t hi = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol + 4]);
+            if (wq0 + r < a.Sq)
+                *reinterpret_cast<uint4_t*>(ob + (int64_t)(wq0 + r) * a.os + ocol) = uint4_t{lo.x, lo.y, hi.x, hi.y};
+        }
+        if (grp == 1) return;               // (the LSEs are written once)
+    } else {
         // two passes of D/2 columns each, so that NW waves' staging regions fit in the four stage arrays
         constexpr int DP = D / 2, OP = DP + 4;         // row pitch in halfs
         constexpr int LPRW = DP / 8, RPS = 64 / LPRW;  // lanes per output row segment, rows per store instruction
@@ -453,48 +540,78 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(co
         for (int qb = 0; qb < 2; ++qb)
             if (qrow[qb] < a.Sq) a.lse[((int64_t)b * a.Hq + head) * a.Sq + qrow[qb]] = (m[qb] + fast_log2(l[qb])) * kLn2;
     }
+}
+#endif
+
+template <int D, int NW, bool PAIRED>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd16_body<D, NW, PAIRED ? kPaired : kPlain>(a);
 #endif
 }
 
-template <int D, int NW, bool PAIRED = false>
+template <int D>
+__global__ __launch_bounds__(512, 1) void attn_fwd16_split_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd16_body<D, 8, kSplit>(a);
+#endif
+}
+
+template <int D, int NW, int MODE>
 static hipError_t launch16(AttnArgs a, hipStream_t s) {
-    int64_t grid;
-    if (PAIRED) {
-        a.n_qtiles = (a.Sq + 127) / 128;
-        grid = (int64_t)((a.n_qtiles + 1) / 2) * a.B * a.Hq;
-    } else {
-        a.n_qtiles = (a.Sq + 32 * NW - 1) / (32 * NW);
-        grid = (int64_t)a.n_qtiles * a.B * a.Hq;
-    }
+    const int rows = MODE == kPlain ? 32 * NW : 128;
+    a.n_qtiles = (int)(((int64_t)a.Sq + rows - 1) / rows);
+    const int64_t grid = (int64_t)(MODE == kPaired ? (a.n_qtiles + 1) / 2 : a.n_qtiles) * a.B * a.Hq;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((attn_fwd16_kernel<D, NW, PAIRED>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    if constexpr (MODE == kSplit) hipLaunchKernelGGL((attn_fwd16_split_kernel<D>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    else hipLaunchKernelGGL((attn_fwd16_kernel<D, NW, MODE == kPaired>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
     return hipGetLastError();
 }
 
-// Workgroup shape by problem size.  Wide (each K/V stage is fetched from L2 once per 256 queries: a few % less energy,
-// and this kernel is power-limited) when that still fills the chip: one workgroup per CU for unmasked attention; under
-// a causal mask workgroups differ in length by up to n_qtiles x, so at least two rounds are needed to balance (measured
-// at 512 wide workgroups: +2.3 % with head_dim 128; with head_dim 64 the wide form loses 10-20 % at every size).  A
-// causal problem whose narrow workgroups would all be resident at once (a single round: the longest tile sets the time,
-// twice the mean) runs paired instead, which gives every workgroup the same work -- if the pairs still cover the chip.
-Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int head_dim, bool causal) {
+// Workgroup shape by problem size (the figures are us, llama heads = 32 query / 8 KV heads of 128; W counts narrow
+// workgroups).  All four shapes cost the same per wave and 64-key tile, about 0.9 us; what differs is how many waves a
+// CU holds and which of them ends last.
+//  Narrow  128 queries, four waves, two workgroups per CU: the general case.
+//  Split   the same 128 queries by eight waves, which halves the walk over the keys and adds a merge (2 - 3 us).  Pays
+//          when every workgroup has a CU to itself anyway and the walk is long: W <= 256 and 1100 keys or more
+//          (8 heads of 128, 3000 tokens: 42.2 against 46.8; 16 heads of 64, 2000: 21.2 against 23.3; 250 queries on
+//          3250 keys: 46.0 against 51.0; but 1000 tokens, 16 heads of 128: 20.5 against 20.7, 600: 15.6 against 14.9).
+//          A causal triangle's short tiles leave room for a few more: W <= 320 (16 heads of 128, 2500: 40.1 against
+//          41.7 paired; at W = 416: 35.1 against 31.9).
+//  Paired  a causal problem whose narrow workgroups are all resident at once: the longest tile sets the time, twice the
+//          mean, so each workgroup takes two tiles from opposite ends.  Such workgroups are half as many and each needs
+//          a CU of its own: 192 to 256 of them (2048 tokens, llama heads: 40.5 against 44.4 narrow; at 288 workgroups,
+//          71 heads of 64 and 777 tokens: 20.2 against 13.8), and tiles enough for an imbalance to matter (at 12 tiles
+//          30.3 against 31.4, at 11 28.3 against 27.1).
+//  Wide    256 queries per K/V stage (head_dim 128 only; with 64 it loses 10 - 20 % at every size): fewer LDS fills and
+//          a few % less energy, where the chip is full and the power limit sets the pace.  Unmasked, from one workgroup
+//          per CU; causal, where tiles of different lengths must even out over rounds, from 384 workgroups of at least
+//          four tiles per head if the last tile is nearly full (llama heads, 4096: 121 against 133.5; 3500: 92.9 against
+//          101.9; two of 1700: 54 against 58.3; but eight of 512, two tiles: 34.3 against 30.3, and eight of 1300, whose
+//          sixth tile holds 20 rows: 156 against 140).
+Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal) {
     const int64_t bh = (int64_t)batch * n_q_heads;
-    const int64_t n128 = (seq_q + 127) / 128;
-    // (paired workgroups are half as many: below about three quarters of the CUs the idle ones cost more than the
-    // imbalance -- measured at 1024 queries x 32 heads: 22.9 us narrow, 24.8 us paired; at 2048: 46.3 and 43.1)
-    if (causal && n128 * bh <= 512 && ((n128 + 1) / 2) * bh >= 192) return Attn16Shape::Paired;
-    const int64_t n_wide = (int64_t)((seq_q + 255) / 256) * bh;
-    return head_dim == 128 && n_wide >= (causal ? 512 : 256) ? Attn16Shape::Wide : Attn16Shape::Narrow;
+    const int64_t n128 = ((int64_t)seq_q + 127) / 128, W = n128 * bh;
+    if (seq_kv >= 1100 && (W <= 256 || (causal && seq_kv == seq_q && W <= 320))) return Attn16Shape::Split;
+    const int64_t pairs = ((n128 + 1) / 2) * bh;
+    if (causal && W <= 512 && pairs >= 192 && pairs <= 256 && n128 >= 12) return Attn16Shape::Paired;
+    const int64_t n256 = ((int64_t)seq_q + 255) / 256;
+    const bool wide = causal ? n256 * bh >= 384 && n256 >= 4 && n256 * 256 * 16 <= (int64_t)seq_q * 17 : n256 * bh >= 256;
+    return head_dim == 128 && wide ? Attn16Shape::Wide : Attn16Shape::Narrow;
 }
 
 hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, hipStream_t s) {
-    if (shape == Attn16Shape::Paired) return head_dim == 128 ? launch16<128, 8, true>(a, s) : launch16<64, 8, true>(a, s);
-    const bool wide = shape == Attn16Shape::Wide;
-    if (head_dim == 128) return wide ? launch16<128, 8>(a, s) : launch16<128, 4>(a, s);
-    return wide ? launch16<64, 8>(a, s) : launch16<64, 4>(a, s);
+    const bool d128 = head_dim == 128;
+    switch (shape) {
+        case Attn16Shape::Paired: return d128 ? launch16<128, 8, kPaired>(a, s) : launch16<64, 8, kPaired>(a, s);
+        case Attn16Shape::Split:  return d128 ? launch16<128, 8, kSplit>(a, s) : launch16<64, 8, kSplit>(a, s);
+        case Attn16Shape::Wide:   return d128 ? launch16<128, 8, kPlain>(a, s) : launch16<64, 8, kPlain>(a, s);
+        default:                  return d128 ? launch16<128, 4, kPlain>(a, s) : launch16<64, 4, kPlain>(a, s);
+    }
 }
 
 const char* attn_fwd16_kernel_name(int head_dim, Attn16Shape shape) {
+    if (shape == Attn16Shape::Split) return head_dim == 128 ? "trn::attn_fwd16_split_kernel<128>" : "trn::attn_fwd16_split_kernel<64>";
     if (shape == Attn16Shape::Paired) return head_dim == 128 ? "trn::attn_fwd16_kernel<128, 8, true>" : "trn::attn_fwd16_kernel<64, 8, true>";
     const bool wide = shape == Attn16Shape::Wide;
     if (head_dim == 128) return wide ? "trn::attn_fwd16_kernel<128, 8, false>" : "trn::attn_fwd16_kernel<128, 4, false>";
