@@ -368,3 +368,33 @@ def test_key_scores_without_noise_and_as_mean_and_std(Sq, Skv):
         ops.attention_key_scores(q, k, v, o2, 0.1, True, rows, s[4], s[5].half())
     with pytest.raises(_lib.TrnError):           # mean and standard deviation are defined without noise only
         ops.attention_key_scores(q, k, v, o2, 0.1, True, rows, s[4], s[5], noise=torch.zeros(1, 4, Sq, Skv, device="cuda"), mean_std=True)
+
+
+# ---- forward kernel with perturbed scores: the mask-free loop and its late raises of the two running references
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sq,Skv,causal", [(576, 95, False), (577, 96, False), (600, 159, False), (600, 160, False), (600, 225, False),
+                                           (513, 513, True), (640, 640, True), (600, 791, True), (1025, 1025, True)])
+@pytest.mark.parametrize("Hq,Hkv,D", [(2, 1, 128), (2, 2, 64)])
+@pytest.mark.parametrize("noise", ["fp16", "fp32"])
+def test_perturbed_scores_that_grow_along_the_keys(Sq, Skv, causal, Hq, Hkv, D, noise):
+    """Keys whose scores and noise grow with their index, so that both references are raised in every part of the walk:
+    sizes around whole turns of the mask-free loop.  Tolerances as for the other key-score tests (probabilities from fp16
+    products, 1e-3), row normalisers 1e-3."""
+    from triton_amd import ops
+    q, k, v = make(1, Hq, Hkv, Sq, Skv, D, seed=31)
+    ramp = torch.arange(Skv, dtype=torch.float32)
+    # shifts of a key by up to 12 in the scaled scores: a component of q that is 1 everywhere meets the ramp
+    q[..., 0] = 1.0
+    k[..., 0] = (12.0 * D ** 0.5 * ramp / Skv).half()
+    x = (torch.randn(1, Hq, Sq, Skv, generator=torch.Generator().manual_seed(5)) + 60.0 * ramp / Skv).half()
+    nd = x.cuda() if noise == "fp16" else x.float().cuda()
+    scale, qd, kd, vd = D ** -0.5, q.cuda(), k.cuda(), v.cuda()
+    o, rows = torch.zeros_like(qd), torch.zeros(1, Hq, Sq, device="cuda")
+    score = torch.full((1, Hq, Skv), -1.0, device="cuda")
+    ops.attention_key_scores(qd, kd, vd, o, scale, causal, rows, score, None, noise=nd, tau=1.0)
+    torch.cuda.synchronize()
+    wo, wscore = ref.keyformer(q, k, v, x.float(), scale, 1.0, causal)
+    close_scores(score, wscore, atol=1e-6)      # (early keys: e^-60 of a row, below fp32's reach of a column sum)
+    assert (o.float().cpu() - wo.float()).abs().max() < 2e-2
+    s = ref.scores_fp32(q, k, scale, causal)
+    assert torch.allclose(rows.cpu(), torch.logsumexp(s + x.float(), -1), atol=1e-3, rtol=1e-3)

@@ -158,8 +158,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
 #define TRN_FETCH_V(jt_, dst_) fetch_tile<NI, D, NW>(vrs, &dst_[wave * RPI * D], vvo, (jt_) * vtile_bytes, vrow_bytes)
 
     const float16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    const int wb = wq0 + off;          // key index bound of this wave's first query
-    auto needs_mask = [&](int key0) { return (key0 + 32 > a.Skv) || (a.causal && key0 + 31 > wb); };
+    const int last_key = min(a.Skv - 1, a.causal ? qrow + off : a.Skv - 1);    // the last key this lane's query sees
 
     // Scores of a 32-key block starting at key0, just produced: (KeyFormer) fold them into the perturbed
     // row normaliser; mask; block max against the LAZY reference max m.  m is only raised when some row's
@@ -167,10 +166,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // range, fp32 sums), O and l stay relative to the same m so the final O/l and m + log2(l) are unchanged,
     // and the 16*NDB-multiply rescale of O^T runs on the first block or two only instead of on most blocks.
     // Returns whether a rescale is due (wave-uniform) and the candidate max.
-    auto reduce_block = [&](bool masked, float16_t& sx, int key0, float& smax, noise_t (&gpre)[4]) __attribute__((always_inline)) {
-        // `masked` is wave-uniform: the branches below touch only this block's 16 score registers, so the
-        // accumulators never meet a control-flow merge.  (Two whole-step variants selected by a branch cost
-        // dozens of accumulator register copies per step and broke the in-place MFMA accumulation chains.)
+    // (The form for blocks that may need the mask; the steps of the plain loop do the same between their MFMAs.)
+    auto reduce_block = [&](float16_t& sx, int key0, float& smax, noise_t (&gpre)[4]) __attribute__((always_inline)) {
+        const int last = last_key - key0 - 4 * h;      // as an offset from the lane's first key
         if constexpr (NOISE) {
             // Row normaliser of the perturbed scores z = s*c2 + g*c3 (log2 domain), with a lazy reference like the
             // main softmax: d = z - m2 comes straight out of two fused multiply-adds, and m2 is only raised when some d
@@ -183,12 +181,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 if constexpr (N16) gv = half_noise4(gpre[r4], nsh); else gv = gpre[r4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)gv[e], a.c3, nref));
-                    if (masked) {
-                        const int key = key0 + 8 * r4 + 4 * h + e;
-                        dd = (key < a.Skv && (!a.causal || key <= qrow + off)) ? dd : -INFINITY;
-                    }
-                    d[r4 * 4 + e] = dd;
+                    const float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)gv[e], a.c3, nref));
+                    d[r4 * 4 + e] = 8 * r4 + e <= last ? dd : -INFINITY;
                 }
             }
             fetch_noise(key0 + 64, gpre);    // the next block of the same parity, two pipeline steps ahead of its use
@@ -212,14 +206,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
             for (int r = 0; r < 16; ++r) sum += fast_exp2(d[r]);
             l2 += sum;
         }
-        if (masked) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int key = key0 + 8 * (r / 4) + 4 * h + (r % 4);
-                const bool ok = key < a.Skv && (!a.causal || key <= qrow + off);
-                sx[r] = ok ? sx[r] : -INFINITY;      // (a select: stale-LDS garbage past the last block never propagates)
-            }
-        }
+        for (int r = 0; r < 16; ++r)
+            sx[r] = 8 * (r / 4) + (r % 4) <= last ? sx[r] : -INFINITY;      // (a select: stale-LDS garbage past the last block never propagates)
         smax = max16_bare(sx) * a.c1;          // over the lane's own keys; the pair's maximum is formed in rescale()
         return __builtin_amdgcn_ballot_w64(smax > m + 8.0f) != 0;
     };
@@ -252,9 +241,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // then every wave has made its last read of the tile's own K stage (block B+1's last operands) and of the
     // previous tile's V stage, so after the barrier those two stages are refilled (K two tiles ahead, V one
     // tile ahead) and all later LDS reads of this and the next step go to the stages that just became visible.
-    auto step = [&](bool masked_next, auto sync_tag, float16_t& sc, float16_t& sn, const half_t* Vblk, const half_t* K1,
-                    const half_t* K2, int key0_next, auto&& handover) __attribute__((always_inline)) {
-        constexpr bool SYNC = decltype(sync_tag)::value;
+    auto step = [&](auto plain_tag, auto sync_tag, float16_t& sc, float16_t& sn, const half_t* Vblk, const half_t* K1,
+                    const half_t* K2, int key0_next, auto&& handover, noise_t (&gpre)[4]) __attribute__((always_inline)) {
+        constexpr bool SYNC = decltype(sync_tag)::value, PLAIN = decltype(plain_tag)::value;
         // The row sum is taken over the fp16-rounded P (v_dot2_f32_f16 against ones, fp32 accumulate),
         // i.e. over exactly the values that multiply V.
         const half2_t ones = {(half_t)1.f, (half_t)1.f};
@@ -288,13 +277,57 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         // ---- phase B ----
         float smax = 0.f;
         bool due = false;
+        // No mask: the perturbed scores are exponentiated and summed between the MFMAs, two scores at a time, against the
+        // reference as it stands; whether it had to be raised is known at the end, and the block's sum is then formed
+        // again (rare after a row's first block).  In one piece behind the fourth MFMA, as reduce_block() has it, the two
+        // waves of a SIMD left the matrix pipe idle for most of it: 32 heads of 128, 4096 keys, fp32 noise 333 -> 309 us,
+        // fp16 270 -> 251; 1501 keys, fp16 65 -> 51; 284 heads of 64, 392 keys 48 -> 37 (same bits).
+        const float nref = -m2;
+        float down = -INFINITY, top = -INFINITY, sum = 0.f;
+        auto perturbed = [&](int r, float ref) __attribute__((always_inline)) {
+            float g;
+            if constexpr (N16) {
+                const uint3_t w = gpre[r / 4];
+                const uint32_t u = (r & 2) ? __builtin_amdgcn_alignbit(w.z, w.y, nsh) : __builtin_amdgcn_alignbit(w.y, w.x, nsh);
+                g = (float)__builtin_bit_cast(half2_t, u)[r & 1];
+            } else g = gpre[r / 4][r % 4];
+            return __builtin_fmaf(sn[r], a.c2, __builtin_fmaf(g, a.c3, ref));
+        };
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
             oacc[i % NDB] = mfma32(va[i % NQ], pB[i / NDB], oacc[i % NDB]);
             if (i + NQ < NS) load_v(i + NQ, i % NQ);
             else ka[i % NQ] = *reinterpret_cast<const half8_t*>(&K2[koff[i + NQ - NS]]);
-            if (i == NS / 2) due = reduce_block(masked_next, sn, key0_next, smax, SYNC ? gpre1 : gpre0);
+            if constexpr (PLAIN) {
+                // scores [first(i), first(i + 1)) in slot i: none in slot 0, whose MFMA covers the end of the score chain
+                auto first = [](int k) { return NS == 8 ? (k == 8 ? 16 : k < 1 ? 0 : 2 * (k - 1)) : k == 4 ? 16 : k < 2 ? 0 : k == 2 ? 4 : 10; };
+#pragma unroll
+                for (int r = first(i); r < first(i + 1); r += 2) {
+                    const float d0 = perturbed(r, nref), d1 = perturbed(r + 1, nref);
+                    down = max3_after(down, d0, d1, d1);
+                    top = max3_after(top, sn[r], sn[r + 1], d1);
+                    sum += fast_exp2(d0);
+                    sum += fast_exp2(d1);
+                }
+            } else if (i == NS / 2) due = reduce_block(sn, key0_next, smax, gpre);
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (PLAIN) {
+            smax = top * a.c1;
+            if (__builtin_amdgcn_ballot_w64(down > 8.0f || (!have2 && down > -INFINITY) || smax > m + 8.0f) != 0) {
+                const float dmax = half_max(down);
+                const bool seen = dmax > -INFINITY, raise = dmax > 8.0f || (!have2 && seen);
+                const float shift = raise ? dmax : 0.f;
+                l2 *= fast_exp2(-shift);
+                m2 += shift;
+                have2 = have2 || seen;
+                sum = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sum += fast_exp2(perturbed(r, nref) - shift);
+                due = __builtin_amdgcn_ballot_w64(smax > m + 8.0f) != 0;
+            }
+            l2 += sum;
+            fetch_noise(key0_next + 64, gpre);
         }
         if (due) rescale(smax);
     };
@@ -317,12 +350,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
 #pragma unroll
         for (int i = 0; i < NQ; ++i) ka[i] = *reinterpret_cast<const half8_t*>(&Ks0[32 * D + koff[i]]);
         float smax;
-        if (reduce_block(true, sA, 0, smax, gpre0)) rescale(smax);
+        if (reduce_block(sA, 0, smax, gpre0)) rescale(smax);
     }
 
     // One 64-key tile jt.  Kc = its own K stage (block 1 still has operands to give), Kn = the next tile's
     // K stage, Vc = its V stage, Vn = the other V stage.
-    auto tile = [&](int jt, half_t* Kc, const half_t* Kn, const half_t* Vc, half_t* Vn) __attribute__((always_inline)) {
+    auto tile = [&](auto plain_tag, int jt, half_t* Kc, const half_t* Kn, const half_t* Vc, half_t* Vn) __attribute__((always_inline)) {
         const int kv0 = jt * BN;
         auto handover = [&]() __attribute__((always_inline)) {
             // this wave's share of stages Kn and Vc is in LDS: everything but the noise requests of the two
@@ -337,12 +370,21 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         };
         auto none = [&]() __attribute__((always_inline)) {};
         // (Past the last tile a K stage holds stale rows; scores computed from them are masked away.)
-        step(needs_mask(kv0 + 32), std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover);
-        step(needs_mask(kv0 + 64), std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + 64, none);
+        step(plain_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover, gpre1);
+        step(plain_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + 64, none, gpre0);
     };
-    for (int jt = 0; jt < ntiles; jt += 2) {
-        tile(jt, Ks0, Ks1, Vs0, Vs1);
-        if (jt + 1 < ntiles) tile(jt + 1, Ks1, Ks0, Vs1, Vs0);
+    // The tiles whose successors need no mask for any wave of the workgroup have a loop of their own (whole turns of the
+    // two stages), the tiles at the diagonal and at the end of the keys another.
+    const int lim = a.causal ? min(a.Skv, q0 + off + 1) : a.Skv;     // keys that every query of the workgroup sees
+    const int n_plain = lim >= BN + 32 ? ((lim - BN - 32) / BN + 1) & ~1 : 0;
+    int jt = 0;
+    for (; jt < n_plain; jt += 2) {
+        tile(std::true_type{}, jt, Ks0, Ks1, Vs0, Vs1);
+        tile(std::true_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
+    }
+    for (; jt < ntiles; jt += 2) {
+        tile(std::false_type{}, jt, Ks0, Ks1, Vs0, Vs1);
+        if (jt + 1 < ntiles) tile(std::false_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
     }
 #undef TRN_FETCH_K
 #undef TRN_FETCH_V
@@ -350,9 +392,10 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // ---- epilogue: normalise; transpose this wave's 32 x D tile through LDS so that the stores are whole
     // 16-byte-per-lane row segments (the accumulator layout would give 8-byte pieces scattered over 32 rows,
     // i.e. partial-line writes); LSEs ----
-    l = half_sum(l);
+    __builtin_amdgcn_s_waitcnt(0x0f70);                // the refills past the last tile have landed ...
+    __syncthreads();                                   // ... everywhere, and every wave is done with the K/V stages
+    l = half_sum(l); l2 = half_sum(l2);
     const float inv = 1.0f / l;
-    __syncthreads();                                   // every wave is done with the K/V stages
     {
         // two passes of D/2 columns each, so that NW waves' staging regions fit in the four stage arrays
         constexpr int DP = D / 2, OP = DP + 4;         // row pitch in halfs: 8-byte writes of 32 rows spread over all banks
@@ -386,9 +429,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     }
     if (qrow < a.Sq && h == 0 && a.lse) a.lse[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m + fast_log2(l)) * kLn2;
     if constexpr (NOISE) {
-        const float l2s = half_sum(l2);
         if (qrow < a.Sq && h == 0)
-            a.lse_pert[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m2 + fast_log2(l2s)) * kLn2;
+            a.lse_pert[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m2 + fast_log2(l2)) * kLn2;
     }
 }
 #endif

@@ -67,6 +67,13 @@ __device__ __forceinline__ float max3_bare(float a, float b, float c) {
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
+// ... for values that may come straight out of an MFMA: `dep` is one that the compiler computed from the same result, so
+// that its wait states lie before this instruction too
+__device__ __forceinline__ float max3_after(float a, float b, float c, float dep) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c), "v"(dep));
+    return r;
+}
 __device__ __forceinline__ float max16_bare(const float16_t& s) {
     const float a = max3_bare(s[0], s[1], s[2]), b = max3_bare(s[3], s[4], s[5]), c = max3_bare(s[6], s[7], s[8]);
     const float d = max3_bare(s[9], s[10], s[11]), e = max3_bare(s[12], s[13], s[14]);
