@@ -398,3 +398,30 @@ def test_perturbed_scores_that_grow_along_the_keys(Sq, Skv, causal, Hq, Hkv, D, 
     assert (o.float().cpu() - wo.float()).abs().max() < 2e-2
     s = ref.scores_fp32(q, k, scale, causal)
     assert torch.allclose(rows.cpu(), torch.logsumexp(s + x.float(), -1), atol=1e-3, rtol=1e-3)
+
+
+# ---- statistics with noise: one and two groups of waves per workgroup, either side of the rule, ragged group ends
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sq,Skv,causal", [(320, 320, True), (321, 321, True), (385, 130, False), (449, 700, True), (512, 64, False),
+                                           (1537, 1537, True), (1025, 1100, True)])
+@pytest.mark.parametrize("B,Hq,Hkv,D", [(1, 3, 1, 128), (2, 2, 2, 64), (4, 8, 2, 64)])
+@pytest.mark.parametrize("noise", ["fp16", "fp32"])
+def test_key_sums_and_squares_by_one_or_two_groups_of_waves(Sq, Skv, causal, B, Hq, Hkv, D, noise):
+    """Held to float64 sums over the probabilities that the same row normalisers give: 2e-5 relative covers fp32 scores of
+    D products (|score| < 2^4 in the log2 domain: 16 * 2^-24 * sqrt(D) of an exponent) and fp32 sums of 1600 terms."""
+    from triton_amd import ops
+    q, k, _ = (t.cuda() for t in make(B, Hq, Hkv, Sq, Skv, D, seed=41))
+    x = torch.randn(B, Hq, Sq, Skv, generator=torch.Generator(device="cuda").manual_seed(6), device="cuda").half()
+    nd = x if noise == "fp16" else x.float()
+    scale = D ** -0.5
+    s = (q.double() @ k.double().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2).contiguous()) * scale + x.double()
+    if causal:
+        s = s.masked_fill(~torch.ones(Sq, Skv, dtype=torch.bool, device="cuda").tril(Skv - Sq), float("-inf"))
+    o, rows = torch.zeros_like(q), torch.zeros(B, Hq, Sq, device="cuda")
+    s1, s2 = (torch.full((B, Hq, Skv), -1.0, device="cuda") for _ in range(2))
+    v = torch.zeros_like(k)
+    ops.attention_key_scores(q, k, v, o, scale, causal, rows, s1, s2, noise=nd, tau=1.0)
+    torch.cuda.synchronize()
+    p = torch.exp(s - rows.double().unsqueeze(-1))
+    for got, want in ((s1, p.sum(2)), (s2, p.square().sum(2))):
+        assert ((got.double() - want).abs() <= 2e-5 * want + 1e-12).all(), ((got.double() - want).abs() / want).max()

@@ -36,7 +36,6 @@ struct ColArgs {
     int causal;
     int n16;        // noise points at fp16 data (its pitches count halfs)
     int s16;        // the outputs are fp16: the fp32 results rounded once
-    int pair;       // (no-noise kernel) a workgroup takes key tiles i and n-1-i
     int mean_std;   // write the per-key mean and population standard deviation over the queries that see the key
                     // (into out_sum / out_sumsq) instead of the two sums
 };
@@ -47,29 +46,73 @@ __device__ __forceinline__ void store_stat(const ColArgs& a, float* out, int64_t
     else out[at] = v;
 }
 
+// A wave's per-key sums, 16 per lane over the lane's queries, added up over the 32 lanes of each half through 4 KB of LDS:
+// lane 2k + i gets key number k of the wave's 32 from 16 lanes (each key starting at another one: no bank conflicts) and
+// adds its neighbour's.  (In registers, five exchanges of all 16 sums and a division per sum and lane behind them took
+// 1 - 2 us of a launch.)
+__device__ __forceinline__ void put_sums(const float (&v)[16], float* area, int lane) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) area[r * 64 + lane] = v[r];
+}
+__device__ __forceinline__ float key_sum(const float* area, int lane) {
+    const int kh = (lane >> 1) & 1, r = lane >> 2, part = lane & 1;        // key 2r + kh of the wave: half kh, number r of 16
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = area[r * 64 + kh * 32 + part * 16 + ((i + r) & 15)];
+#pragma unroll
+    for (int n = 8; n >= 1; n >>= 1)                                       // (as a tree: a chain's rounding is larger)
+#pragma unroll
+        for (int i = 0; i < n; ++i) x[i] += x[i + n];
+    return x[0] + __shfl_xor(x[0], 1, 64);
+}
+
+// The end of both kernels: x, y = the sums of the lane's key (key_sum's order), turned into mean and deviation if wanted,
+// and stored by the even lanes.
+template <bool SQ>
+__device__ __forceinline__ void finish_columns(const ColArgs& a, float x, float y, int64_t obase, int wkey0, int lane) {
+    const int kh = (lane >> 1) & 1, r = lane >> 2, key = wkey0 + 8 * (r / 4) + 4 * kh + (r % 4);
+    if (SQ && a.mean_std) {
+        // n = queries that see this key: all of them, or under a causal mask those from key - (Skv - Sq) on
+        const float n = (float)(a.causal ? a.Sq - max(0, key - (a.Skv - a.Sq)) : a.Sq);
+        const float mean = x / n;
+        // E p^2 - mean^2 as (y - x mean) / n, the product fused.  The difference is known to about 1e-7 of E p^2, its
+        // root to 3e-4 of the column's root mean square: a key seen by a single query, whose spread is zero by
+        // definition, would come back as that rounding residue, so it is set.
+        y = n > 1.5f ? __builtin_sqrtf(fmaxf(0.f, __builtin_fmaf(-x, mean, y) / n)) : 0.f;
+        x = mean;
+    }
+    if ((lane & 1) == 0 && key < a.Skv) {
+        store_stat(a, a.out_sum, obase + key, x);
+        if (SQ) store_stat(a, a.out_sumsq, obase + key, y);
+    }
+}
+
 constexpr int CBN = 128;  // keys per workgroup
 [[maybe_unused]] constexpr int CBM = 64;   // queries per staged tile
 
 // SQ: the sums of squares are wanted too (RoCo); without them (KeyFormer) their accumulators and one of the five
 // VALU operations per score are not compiled in.
 // NZ: 1 fp32 noise, 2 fp16 noise
-template <int D, int NZ, bool SQ>
-__global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) {
+// NG: groups of four waves on the same 128 keys, each taking every NG-th query tile through stages of its own; the second
+// hands its sums to the first at the end.
+template <int D, int NZ, bool SQ, int NG>
+__global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
     constexpr bool N16 = NZ == 2;
     constexpr int NKS = D / 16;
     constexpr int CPR = D / 8;                 // 16-byte chunks per Q row
     constexpr int RPI = 64 / CPR;              // stage rows covered by one wave-wide 1 KB load
     constexpr int NI = CBM / (RPI * 4);        // such loads per wave per stage
-    __shared__ __attribute__((aligned(1024))) half_t Qs0[CBM * D];
-    __shared__ __attribute__((aligned(1024))) half_t Qs1[CBM * D];
-    __shared__ __attribute__((aligned(1024))) half_t Qs2[CBM * D];
+    __shared__ __attribute__((aligned(1024))) half_t Qs0[NG * CBM * D];
+    __shared__ __attribute__((aligned(1024))) half_t Qs1[NG * CBM * D];
+    __shared__ __attribute__((aligned(1024))) half_t Qs2[NG * CBM * D];
     // KeyFormer: the wave's 32 x 32 block of noise is fetched with whole 128-byte row pieces per 8 lanes (a load
     // instruction then touches 8 cache lines, not 32) and turned into the accumulator layout through this array
-    __shared__ __attribute__((aligned(1024))) float Ns[4 * 1024];
+    __shared__ __attribute__((aligned(1024))) float Ns[NG * 4 * 1024];
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;        // within the group
     const int BH = a.B * a.Hq;
     const int kt = (int)(blockIdx.x / BH);             // key tile 0 sees the most queries: heaviest first
     const int j = blockIdx.x % BH;
@@ -100,7 +143,7 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) 
     const int st_chunk = (lane % CPR) ^ swz<D>(st_row);
     const int qvo = (int)(st_row * a.qs * 2) + st_chunk * 16;
     const int qrow_bytes = (int)(RPI * a.qs * 2), qtile_bytes = (int)(CBM * a.qs * 2);
-#define TRN_FETCH_Q(t_, dst_) fetch_tile<NI, D, 4>(qrs, &dst_[wave * RPI * D], qvo, (t_) * qtile_bytes, qrow_bytes)
+#define TRN_FETCH_Q(t_, dst_) fetch_tile<NI, D, 4>(qrs, &dst_[grp * CBM * D + wave * RPI * D], qvo, (t_) * qtile_bytes, qrow_bytes)
     int qoff[NKS];       // B-operand read: row c (+32 for the second block), logical chunk 2*ks + h
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) qoff[ks] = c * D + (((2 * ks + h) ^ swz<D>(c)) << 3);
@@ -122,7 +165,7 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) 
     const int nrow8 = (int)(8 * a.ns * nsz);
     // transposer: the 16-byte chunk q of row r sits at chunk r*8 + (q ^ ((r/2) % 8)); written as loaded, read as
     // row c, chunks 2*r4 + h (both conflict-free)
-    float* nsw = Ns + wave * 1024;
+    float* nsw = Ns + (grp * 4 + wave) * 1024;
     int ns_wr[4], ns_rd[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -146,7 +189,8 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) 
     };
 
     const int first_q = a.causal ? max(0, kv0 - off) : 0;   // earlier queries see none of this tile's keys
-    const int t0 = first_q / CBM, nt = (a.Sq + CBM - 1) / CBM;
+    // this group's first tile, and a common end: a group whose last tile lies past the queries masks it away
+    const int t0 = first_q / CBM + grp, nt = NG == 1 ? (a.Sq + CBM - 1) / CBM : first_q / CBM + ((a.Sq + CBM - 1) / CBM - first_q / CBM + 1) / 2 * 2 + grp;
 
     // The VALU part of a 32-query block.  Masked and plain blocks are separate loops (one wave-uniform branch
     // per block) so that the plain one is 4 instructions per score: fma, exp2, add, fma.
@@ -213,9 +257,9 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) 
             __builtin_amdgcn_sched_barrier(0);
             if (live0) softmax_sums(acc0, q0, pc.lse[0], pc.g[0]);
         }
-        prefetch(t + 2, 0, pc);              // (unconditional, like every load of the loop: see below)
+        prefetch(t + 2 * NG, 0, pc);              // (unconditional, like every load of the loop: see below)
         if (live1) softmax_sums(acc1, q0 + 32, pc.lse[1], pc.g[1]);
-        prefetch(t + 2, 1, pc);
+        prefetch(t + 2 * NG, 1, pc);
     };
     // Tile t reads stage t % 3; the stage of tile t+2 is requested as soon as the barrier shows that everybody has
     // left tile t-1 (its previous tenant), so a Q stage has two tile times to arrive from L2.  Tile t's stage has
@@ -230,53 +274,48 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) 
         __builtin_amdgcn_s_waitcnt(0x0f70 | (kBehind & 15) | ((kBehind >> 4) << 14));
         __builtin_amdgcn_s_barrier();        // (a bare barrier: nothing else in flight needs draining)
         __builtin_amdgcn_sched_barrier(0);
-        TRN_FETCH_Q(t + 2, Qf);
+        TRN_FETCH_Q(t + 2 * NG, Qf);
         __builtin_amdgcn_sched_barrier(0);
-        blocks(Qc, t, pc);
+        blocks(Qc + grp * CBM * D, t, pc);
     };
     // the same order of requests as in the loop, so that the count above holds from the first tile on
     TRN_FETCH_Q(t0, Qs0);
     prefetch(t0, 0, pa); prefetch(t0, 1, pa);
-    TRN_FETCH_Q(t0 + 1, Qs1);
-    prefetch(t0 + 1, 0, pb); prefetch(t0 + 1, 1, pb);
+    TRN_FETCH_Q(t0 + NG, Qs1);
+    prefetch(t0 + NG, 0, pb); prefetch(t0 + NG, 1, pb);
     // Pin the arrival of the K rows here, ahead of the loop.  Left to the first MFMA that reads them, the wait the
     // compiler inserts sits inside the loop body and, being conservative across the back edge, drains the stage and
     // prefetch loads of every iteration.
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) asm volatile("" ::"v"(kA[ks]));
-    for (int t = t0; t < nt; t += 6) {       // three stages x two register buffers
+    for (int t = t0; t < nt; t += 6 * NG) {       // three stages x two register buffers
         tile(t, Qs0, Qs2, pa);
-        if (t + 1 < nt) tile(t + 1, Qs1, Qs0, pb);
-        if (t + 2 < nt) tile(t + 2, Qs2, Qs1, pa);
-        if (t + 3 < nt) tile(t + 3, Qs0, Qs2, pb);
-        if (t + 4 < nt) tile(t + 4, Qs1, Qs0, pa);
-        if (t + 5 < nt) tile(t + 5, Qs2, Qs1, pb);
+        if (t + NG < nt) tile(t + NG, Qs1, Qs0, pb);
+        if (t + 2 * NG < nt) tile(t + 2 * NG, Qs2, Qs1, pa);
+        if (t + 3 * NG < nt) tile(t + 3 * NG, Qs0, Qs2, pb);
+        if (t + 4 * NG < nt) tile(t + 4 * NG, Qs1, Qs0, pa);
+        if (t + 5 * NG < nt) tile(t + 5 * NG, Qs2, Qs1, pb);
     }
 #undef TRN_FETCH_Q
 
-    // sum over the 32 queries held by lanes c = 0..31 (same h), then lane c == 0 of each half writes
-    const int64_t obase = ((int64_t)b * a.Hq + head) * a.Skv;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        float x = s1[r], y = SQ ? s2[SQ ? r : 0] : 0.f;
-#pragma unroll
-        for (int msk = 1; msk < 32; msk <<= 1) { x += __shfl_xor(x, msk, 64); if constexpr (SQ) y += __shfl_xor(y, msk, 64); }
-        const int key = wkey0 + 8 * (r / 4) + 4 * h + (r % 4);
-        if (SQ && a.mean_std) {
-            // n = queries that see this key: all of them, or under a causal mask those from key - (Skv - Sq) on
-            const float n = (float)(a.causal ? a.Sq - max(0, key - (a.Skv - a.Sq)) : a.Sq);
-            const float mean = x / n;
-            // E p^2 - mean^2 as (y - x mean) / n, the product fused.  The difference is known to about 1e-7 of E p^2, its
-            // root to 3e-4 of the column's root mean square: a key seen by a single query, whose spread is zero by
-            // definition, would come back as that rounding residue, so it is set.
-            y = n > 1.5f ? __builtin_sqrtf(fmaxf(0.f, __builtin_fmaf(-x, mean, y) / n)) : 0.f;
-            x = mean;
+    // (the transposing areas are the waves' own: only the other group's reads and writes need a barrier)
+    const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));     // (the lane, not kept over the walk)
+    auto total = [&](const float (&v)[16]) __attribute__((always_inline)) {
+        put_sums(v, nsw, ln);
+        if constexpr (NG == 1) return key_sum(nsw, ln);
+        else {
+            __syncthreads();
+            const float x = grp == 0 ? key_sum(nsw, ln) + key_sum(nsw + 4 * 1024, ln) : 0.f;
+            if constexpr (SQ) __syncthreads();
+            return x;
         }
-        if (c == 0 && key < a.Skv) {
-            store_stat(a, a.out_sum, obase + key, x);
-            if (SQ) store_stat(a, a.out_sumsq, obase + key, y);
-        }
-    }
+    };
+    const float x = total(s1);
+    float y = 0.f;
+    if constexpr (SQ) y = total(s2);
+    __builtin_amdgcn_s_waitcnt(0x0f70);     // the refills past the last tile have landed before the stages are given up
+    if (NG == 2 && grp == 1) return;
+    finish_columns<SQ>(a, x, y, ((int64_t)b * a.Hq + head) * a.Skv, wkey0, ln);
 #endif
 }
 
@@ -292,7 +331,10 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_kernel(const ColArgs a) 
 //     keys are simply masked away);
 //   * the row normalisers ride along with the Q stage (one 256-byte global->LDS load per wave and tile) instead of
 //     a register prefetch of their own;
-//   * under a causal mask a workgroup takes a heavy and a light key tile in turn, so that all have equal work.
+//   * a workgroup per key tile, the heaviest first.  (A heavy and a light one in turn, equal work for all under a causal
+//     mask, halved the grid: us, paired / as is, 32 heads of 128: 600 keys 27.7 / 17.4, 1501 37 / 29, 2048 44 / 37, 4096
+//     110 / 107; 71 of 64, 639: 25 / 17, 1559: 45 / 41; 8 of 128, 4096: 59 / 49.  With the end of the walk through LDS,
+//     in the same order: 11.6, 23, 31, 91; 10.6, 29; 44.)
 // Ring of four Q stages relative to the first tile.  Tile t+1 is multiplied during step t (the VALU work of tile
 // t); at the barrier that opens step t every wave is done with stage t, which is refilled there with tile t+4 --
 // three steps before its use.
@@ -319,7 +361,7 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int BH = a.B * a.Hq;
-    const int pidx = (int)(blockIdx.x / BH);
+    const int kt = (int)(blockIdx.x / BH);             // key tile 0 sees the most queries: heaviest first
     const int j = blockIdx.x % BH;
     const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
     const int kvslot = j % nkv, g = j / nkv;
@@ -346,16 +388,10 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
     for (int ks = 0; ks < NKS; ++ks) qoff[ks] = c * D + (((2 * ks + h) ^ swz<D>(c)) << 3);
     const int nt = (a.Sq + CBM - 1) / CBM;
 
-    // Under a causal mask key tile kt is seen by the query tiles from its own position on, so the work falls
-    // linearly with kt: a workgroup then takes tile pidx and, after it, tile n-1-pidx (a.pair), and every workgroup
-    // has the same amount to do.
-    for (int pass = 0; pass < 2; ++pass) {
-    int kt = pidx;
-    if (pass == 1) {
-        kt = a.n_kvtiles - 1 - pidx;
-        if (!a.pair || kt <= pidx) break;
-        __builtin_amdgcn_s_barrier();          // everybody has left the stages of the first tile's walk
-    }
+    // (a loop of one turn whose end the compiler cannot see: as straight-line code the walk's running sums and operands take
+    // 20 to 35 registers more, past what two waves per SIMD have)
+    int again = 0;
+    do {
     const int kv0 = kt * CBN;
     const int wkey0 = kv0 + wave * 32;                 // this wave's 32 keys
 
@@ -464,12 +500,14 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
         tile_step(std::false_type{}, std::false_type{}, accA, accB, 0, 0.f, 0.f, accA, accB, Qs0);
     }
     // Three loops of whole turns: masking code up to the first turn whose four tiles are all plain, the code without
-    // masks for the turns of plain tiles, masking code for the rest.  Only the last loop leaves in the middle of a
+    // masks for the turns of plain tiles, masking code for the rest (without a plain turn: for all).  Only the last loop leaves in the middle of a
     // turn; the first may run up to three tiles past the end of the queries (they read as zeros and are masked
     // away).  Every loop is thus entered with the same loads in flight as its own back edge brings -- after a loop
     // that might have ended on another stage, the compiler's own wait before a tile's first LDS read would drain
     // stages still in flight.
-    const int n_pre = (min(tg, nt) - t0 + 3) / 4, n_plain = max(0, tp - (t0 + 4 * n_pre)) / 4;
+    int n_pre = (min(tg, nt) - t0 + 3) / 4;
+    const int n_plain = max(0, tp - (t0 + 4 * n_pre)) / 4;
+    if (n_plain == 0) n_pre = 0;            // the last loop, which ends with the queries, takes it all
     int t = t0;
     auto never = [&](int) { return false; };
     for (int i = 0; i < n_pre; ++i, t += 4) turn(std::true_type{}, t, never);
@@ -478,48 +516,45 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
         if (turn(std::true_type{}, t, [&](int tt) { return tt + 1 >= nt; })) break;
     __builtin_amdgcn_s_waitcnt(0x0f70);     // the refills past the last tile have landed before the stages are given up
 
-    // sum over the 32 queries held by lanes c = 0..31 (same h), then lane c == 0 of each half writes
-    const int64_t obase = ((int64_t)b * a.Hq + head) * a.Skv;
-#pragma unroll
-    for (int r16 = 0; r16 < 16; ++r16) {
-        float x = s1[r16], y = SQ ? s2[SQ ? r16 : 0] : 0.f;
-#pragma unroll
-        for (int msk = 1; msk < 32; msk <<= 1) { x += __shfl_xor(x, msk, 64); if constexpr (SQ) y += __shfl_xor(y, msk, 64); }
-        const int key = wkey0 + 8 * (r16 / 4) + 4 * h + (r16 % 4);
-        if (SQ && a.mean_std) {
-            // n = queries that see this key: all of them, or under a causal mask those from key - (Skv - Sq) on
-            const float n = (float)(a.causal ? a.Sq - max(0, key - (a.Skv - a.Sq)) : a.Sq);
-            const float mean = x / n;
-            // E p^2 - mean^2 as (y - x mean) / n, the product fused.  The difference is known to about 1e-7 of E p^2, its
-            // root to 3e-4 of the column's root mean square: a key seen by a single query, whose spread is zero by
-            // definition, would come back as that rounding residue, so it is set.
-            y = n > 1.5f ? __builtin_sqrtf(fmaxf(0.f, __builtin_fmaf(-x, mean, y) / n)) : 0.f;
-            x = mean;
-        }
-        if (c == 0 && key < a.Skv) {
-            store_stat(a, a.out_sum, obase + key, x);
-            if (SQ) store_stat(a, a.out_sumsq, obase + key, y);
-        }
-    }
-    }   // pass
+    __syncthreads();                        // ... by everybody
+    float* area = reinterpret_cast<float*>(D == 128 || wave < 2 ? Qs0 : Qs1) + (D == 128 ? wave : wave & 1) * 1024;
+    const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));     // (the lane, not kept over the walk)
+    put_sums(s1, area, ln);
+    const float x = key_sum(area, ln);
+    float y = 0.f;
+    if constexpr (SQ) { put_sums(s2, area, ln); y = key_sum(area, ln); }
+    finish_columns<SQ>(a, x, y, ((int64_t)b * a.Hq + head) * a.Skv, wkey0, ln);
+    asm volatile("" : "+s"(again));
+    } while (again != 0);
 #undef TRN_FETCH_QL
 #endif
 }
 
 template <int D>
-static hipError_t launch_col_plain(ColArgs a, hipStream_t s) {
-    a.pair = a.causal && a.n_kvtiles > 1;
-    const unsigned grid = (unsigned)(a.pair ? (a.n_kvtiles + 1) / 2 : a.n_kvtiles) * a.B * a.Hq;
+static hipError_t launch_col_plain(const ColArgs& a, hipStream_t s) {
+    const unsigned grid = (unsigned)a.n_kvtiles * a.B * a.Hq;
     if (a.out_sumsq) hipLaunchKernelGGL((attn_colstats_plain_kernel<D, true>), dim3(grid), dim3(256), 0, s, a);
     else hipLaunchKernelGGL((attn_colstats_plain_kernel<D, false>), dim3(grid), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
+// One or two groups of four waves per workgroup (a CU holds eight waves either way).  Two where one leaves CUs idle, or
+// where a single round of workgroups of unequal walks waits for the longest one; not for short walks, which the start and
+// the merge outweigh, nor where equal walks (no mask) fill the chip.  us, one / two groups, with the number of workgroups of
+// 128 keys: 32 heads of 128, 600 keys 17.9 / 15.2 (160), 1501 43 / 34 (384), 2048 69 / 63 (512), 3126 107 / 128 (800);
+// 8 heads of 128, 250 keys 9.5 / 9.6, 363 12.1 / 11.3, 4096 86 / 73 (256); 16 x 3 heads of 64, 1100 keys 29 / 24 (432);
+// 71 heads of 64, 639 keys 21.0 / 21.5 (355, 10 query tiles); 64 heads of 128, 903 keys 28 / 30 (512, 15 tiles).
+template <int D, int NZ, int NG>
+static void launch_col_ng(const ColArgs& a, unsigned grid, hipStream_t s) {
+    if (a.out_sumsq) hipLaunchKernelGGL((attn_colstats_kernel<D, NZ, true, NG>), dim3(grid), dim3(256 * NG), 0, s, a);
+    else hipLaunchKernelGGL((attn_colstats_kernel<D, NZ, false, NG>), dim3(grid), dim3(256 * NG), 0, s, a);
+}
 template <int D, int NZ>
 static hipError_t launch_col(const ColArgs& a, hipStream_t s) {
     const unsigned grid = (unsigned)a.n_kvtiles * a.B * a.Hq;
-    if (a.out_sumsq) hipLaunchKernelGGL((attn_colstats_kernel<D, NZ, true>), dim3(grid), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((attn_colstats_kernel<D, NZ, false>), dim3(grid), dim3(256), 0, s, a);
+    const int walk = (a.Sq + CBM - 1) / CBM;                     // query tiles of the longest walk
+    const bool two = walk >= 6 && (grid <= 320 || (a.causal && grid <= 512 && walk >= 16));
+    if (two) launch_col_ng<D, NZ, 2>(a, grid, s); else launch_col_ng<D, NZ, 1>(a, grid, s);
     return hipGetLastError();
 }
 
@@ -567,7 +602,7 @@ int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, con
     const float tau = noise ? d->tau : 1.f;
     a.c1 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.causal = d->causal ? 1 : 0;
-    a.mean_std = mean_std; a.pair = 0; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
+    a.mean_std = mean_std; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
     if ((int64_t)a.n_kvtiles * a.B * a.Hq > 0x7fffffffLL) return TRN_E_SHAPE;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
