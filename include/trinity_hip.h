@@ -121,8 +121,14 @@ int trn_attn_fwd_f16(const trn_attn_desc* desc, const void* q, const void* k, co
  *   workspace        device memory, 256-byte aligned, trn_attn_workspace_bytes(desc) bytes, zero-filled ONCE before
  *                    its first use (the kernel returns its counters to zero).  One call at a time may use it.
  * trn_attn_workspace_bytes returns 0 when the shape would not use a workspace.
+ *
+ * A chunk of more than 32 queries per head on a long cache has a workspace of its own, trn_attn_chunk_workspace_bytes(desc)
+ * bytes (0: none), which needs no initial contents: the keys are then shared out over workgroups whose partial results a
+ * second launch merges.  Without it, or with a smaller one, the call is trn_attn_fwd_f16 as above.  No size depends on
+ * seq_kv, so that a cache that grows from call to call keeps its workspace.
  */
 int64_t trn_attn_workspace_bytes(const trn_attn_desc* desc);
+int64_t trn_attn_chunk_workspace_bytes(const trn_attn_desc* desc);
 int trn_attn_fwd_ws_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v,
                         void* o, float* lse, const void* gamma_q,
                         const float* noise, float* lse_pert,

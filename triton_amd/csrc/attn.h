@@ -84,6 +84,10 @@ void* attn_static_scratch();
 enum class Attn16Shape { Narrow, Wide, Paired, Split };
 Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal);
 hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, hipStream_t stream);
+// The keys of a chunk of queries against a long cache shared out over workgroups (attn_fwd16.hip): fp32 partial results in
+// args.ws, attn_share_workspace_bytes of it (0: this problem is not shared out), merged by a second launch.
+int64_t attn_share_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);
+hipError_t launch_attn_shares(const AttnArgs& a, int head_dim, hipStream_t stream);
 // Name of the kernel instantiation that launch_attn_fwd16 runs for this shape, as a profiler prints it.
 const char* attn_fwd16_kernel_name(int head_dim, Attn16Shape shape);
 

@@ -493,6 +493,12 @@ extern "C" int64_t trn_attn_workspace_bytes(const trn_attn_desc* d) {
     return attn_decode_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
 }
 
+extern "C" int64_t trn_attn_chunk_workspace_bytes(const trn_attn_desc* d) {
+    using namespace trn;
+    if (!d || validate_attn(d, true) != TRN_OK) return 0;
+    return attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
+}
+
 extern "C" const char* trn_attn_fwd_kernel_name(const trn_attn_desc* d, int32_t with_noise) {
     using namespace trn;
     if (!d || validate_attn(d, true) != TRN_OK) return "";
@@ -661,6 +667,14 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         return TRN_E_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
+    // a chunk of queries on a long cache, with the workspace for it: the keys shared out over workgroups
+    if (workspace && !noise && !col_sum && !col_sumsq && !probs) {
+        const int64_t need = attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
+        if (need > 0 && workspace_bytes >= need) {
+            a.ws = static_cast<float*>(workspace);
+            return launch_attn_shares(a, d->head_dim, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+        }
+    }
     // few queries per head (decode), or few query tiles in all: one workgroup per head and 32 queries, its waves split the keys
     if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, noise != nullptr))
         return launch_attn_decode(a, d->head_dim, workspace, workspace_bytes, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;

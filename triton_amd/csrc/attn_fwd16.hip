@@ -31,8 +31,8 @@ namespace trn {
 
 // What the two groups of four waves of an eight-wave workgroup do: kPlain, the same tile of 256 queries; kPaired, two
 // tiles of 128 queries from the two ends of a causal problem; kSplit, the same 128 queries, each group every other
-// 64-key tile.
-enum { kPlain, kPaired, kSplit };
+// 64-key tile; kShare, as kSplit on one of a.n_split shares of the keys, whose partial results a second launch merges.
+enum { kPlain, kPaired, kSplit, kShare };
 
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -66,7 +66,7 @@ struct Scores16 { float4_t s[2][2]; };      // [key half][query block]
 #if defined(__HIP_DEVICE_COMPILE__)
 template <int D, int NW, int MODE>
 __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
-    constexpr bool PAIRED = MODE == kPaired, SPLIT = MODE == kSplit;
+    constexpr bool PAIRED = MODE == kPaired, SHARE = MODE == kShare, SPLIT = MODE == kSplit || SHARE;
     static_assert(MODE == kPlain || NW == 8, "paired query tiles and split keys are two groups of four waves");
     constexpr int GW = SPLIT ? 4 : NW;       // waves that share the K / V stages
     constexpr int KSTEP = SPLIT ? 128 : 64;  // keys from one tile of a wave to its next
@@ -90,9 +90,12 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     half_t* const Ks1 = Ks1_ + grp * BN * D;
     half_t* const Vs0 = Vs0_ + grp * BN * D;
     half_t* const Vs1 = Vs1_ + grp * BN * D;
-    const int kfirst = grp * BN;             // first key of this wave's first tile
-
     const int BH = a.B * a.Hq;
+    // The shares of a query tile are consecutive; a share is a whole number of tiles of both groups.
+    const int share = SHARE ? (int)(blockIdx.x / BH) % a.n_split : 0, tile_no = (int)(blockIdx.x / BH) / (SHARE ? a.n_split : 1);
+    const int share_tiles = SHARE ? 2 * (((a.Skv + 2 * BN - 1) / (2 * BN) + a.n_split - 1) / a.n_split) : 0;
+    const int kfirst = grp * BN + share * share_tiles * BN;      // first key of this wave's first tile
+
     const int j = blockIdx.x % BH;
     const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
     const int kvslot = j % nkv, g = j / nkv;
@@ -111,7 +114,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         wq0 = (wave < 4 ? ht : lt) * 128 + (wave & 3) * 32;
         if (wave >= 4 && lt == ht) wq0 = a.Sq;          // odd tile count: the middle one is alone (loads clamp, stores are predicated off)
     } else {
-        q0 = (a.n_qtiles - 1 - (int)(blockIdx.x / BH)) * (GW * 32); q_last = q0 + GW * 32 - 1;
+        q0 = (a.n_qtiles - 1 - tile_no) * (GW * 32); q_last = q0 + GW * 32 - 1;
         wq0 = q0 + gw * 32;                             // first query of this wave
     }
     int qrow[2];
@@ -150,6 +153,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
 
     int ntiles = (a.Skv + BN - 1) / BN;
     if (a.causal) ntiles = min(ntiles, (min(q_last, a.Sq - 1) + off) / BN + 1);
+    if constexpr (SHARE) ntiles = max(0, min(ntiles - share * share_tiles, share_tiles));      // of this share
 
     // ---- staging: direct global -> LDS loads; keys past the end read as zeros
     const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
@@ -404,9 +408,9 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     // hold a key visible to one of its queries, and for the rest only keeps up the staging it shares with the
     // others (its part of every refill, and the barrier), leaving its SIMD to the wave that still computes.
     int nlive = ntiles;
-    if (a.causal) nlive = min(ntiles, (min(wq0 + 31, a.Sq - 1) + off) / BN + 1);
+    if (a.causal) nlive = max(0, min(ntiles, (min(wq0 + 31, a.Sq - 1) + off) / BN + 1 - share * share_tiles));
     const int nloop = SPLIT ? (ntiles + 1) >> 1 : ntiles;
-    if constexpr (SPLIT) nlive = (nlive - grp + 1) >> 1;
+    if constexpr (SPLIT) nlive = (nlive - grp + 1) >> 1;           // (nlive = 0, grp = 1: 0)
     if (wq0 >= a.Sq) nlive = 0;             // no query of its own: the ragged end of a tile, or the middle tile of an odd count
     // The leading tiles whose blocks (and the first block of the tile after) lie wholly inside the keys and, under a
     // causal mask, before this wave's first query: a loop of their own without the mask test.  needs_mask is monotone
@@ -468,7 +472,8 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
             const float mt = stat[(((wave ^ 4) * 2 + qb) * 16 + n) * 2], lt = stat[(((wave ^ 4) * 2 + qb) * 16 + n) * 2 + 1];
-            const float ms = fmaxf(m[qb], mt);            // (finite: every query sees a key)
+            float ms = fmaxf(m[qb], mt);                  // (finite: every query sees a key -- but not of every share)
+            if (SHARE && ms == -INFINITY) ms = 0.f;
             wo[qb] = fast_exp2(m[qb] - ms); wt[qb] = fast_exp2(mt - ms);
             l[qb] = l[qb] * wo[qb] + lt * wt[qb];
             m[qb] = ms;
@@ -481,6 +486,19 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
                 const float4_t own = grp == 0 ? oacc[i][qb] : oacc[NH + i][qb];
                 oacc[i][qb] = own * wo[qb] + theirs[(i * 2 + qb) * 64 + lane] * wt[qb];
             }
+        if constexpr (SHARE) {
+            // this share's {O unnormalised, m, l} per query, fp32: rows of D floats, then the pairs of all rows
+            const int64_t rows = (int64_t)BH * a.n_split * a.Sq, row0 = ((int64_t)(b * a.Hq + head) * a.n_split + share) * a.Sq;
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+                if (qrow[qb] >= a.Sq) continue;
+                float* po = a.ws + (row0 + qrow[qb]) * D + grp * (D / 2) + 4 * g4;
+#pragma unroll
+                for (int i = 0; i < NH; ++i) *reinterpret_cast<float4_t*>(po + 16 * i) = oacc[i][qb];
+                if (g4 == 0 && grp == 0) *reinterpret_cast<float2_t*>(a.ws + rows * D + (row0 + qrow[qb]) * 2) = float2_t{l[qb] > 0.f ? m[qb] : -INFINITY, l[qb]};
+            }
+            return;
+        }
         constexpr int DP = D / 2, OP = DP + 4, LPRW = DP / 8, RPS = 64 / LPRW;
         half_t* ot = (wave < 4 ? Vs1_ : Ks1_) + (wave & 3) * 32 * OP;
         static_assert(4 * 32 * OP * 2 <= kStat * 4 && kStat * 4 + 2048 <= 2 * BN * D * 2, "the stage holds both");
@@ -555,6 +573,93 @@ __global__ __launch_bounds__(512, 1) void attn_fwd16_split_kernel(const AttnArgs
 #if defined(__HIP_DEVICE_COMPILE__)
     attn_fwd16_body<D, 8, kSplit>(a);
 #endif
+}
+
+template <int D>
+__global__ __launch_bounds__(512, 1) void attn_fwd16_share_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd16_body<D, 8, kShare>(a);
+#endif
+}
+
+constexpr int kMaxShares = 16;
+
+// The shares' results of one query per wave: D / 64 columns per lane, the shares in order.  Two memory latencies and the
+// launch, 4 - 5 us (with the shares' maxima and sums read by every lane in a loop of its own, 5 - 8).
+template <int D>
+__global__ __launch_bounds__(256) void attn_merge_shares_kernel(const AttnArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), n_rows = (int64_t)a.B * a.Hq * a.Sq;
+    if (row >= n_rows) return;
+    const int64_t bh = row / a.Sq, qr = row % a.Sq, b = bh / a.Hq, head = bh % a.Hq;
+    const float* parts = a.ws + (bh * a.n_split * a.Sq + qr) * D;                            // share s: + s * Sq * D
+    const float* st = a.ws + n_rows * a.n_split * D + (bh * a.n_split * a.Sq + qr) * 2;      // share s: + s * Sq * 2
+    constexpr int C = D / 64, BATCH = 8;
+    // lane s holds share s's {m, l}; the first rows are requested before they are waited for
+    const float2_t ml = *reinterpret_cast<const float2_t*>(st + (int64_t)min(lane, a.n_split - 1) * a.Sq * 2);
+    float r[BATCH][C];
+    auto fetch = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+#pragma unroll
+            for (int i = 0; i < C; ++i) r[u][i] = parts[(int64_t)min(s0 + u, a.n_split - 1) * a.Sq * D + lane * C + i];
+    };
+    fetch(0);
+    float m = ml.x;
+#pragma unroll
+    for (int k = 1; k < kMaxShares; k <<= 1) m = fmaxf(m, __shfl_xor(m, k, 64));
+    const float w = lane < a.n_split ? fast_exp2(ml.x - m) : 0.f;       // (lanes past the shares repeat the last one's m)
+    float l = lane < kMaxShares ? w * ml.y : 0.f;
+#pragma unroll
+    for (int k = 1; k < kMaxShares; k <<= 1) l += __shfl_xor(l, k, 64);
+    l = __shfl(l, 0, 64); m = __shfl(m, 0, 64);
+    float o[C] = {};
+    for (int s0 = 0; s0 < a.n_split; s0 += BATCH) {
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) {
+            const float wu = s0 + u < a.n_split ? __shfl(w, s0 + u, 64) : 0.f;
+#pragma unroll
+            for (int i = 0; i < C; ++i) o[i] = __builtin_fmaf(r[u][i], wu, o[i]);
+        }
+        if (s0 + BATCH < a.n_split) fetch(s0 + BATCH);
+    }
+    half_t* orow = a.o + b * a.ob + head * a.oh + qr * a.os + lane * C;
+#pragma unroll
+    for (int i = 0; i < C; ++i) orow[i] = (half_t)(o[i] / l);
+    if (lane == 0 && a.lse) a.lse[row] = (m + fast_log2(l)) * kLn2;
+}
+
+// Key shares of the query tiles of 128, one workgroup per CU in all (0: the keys are not shared out).  The other forms are
+// tiles of 32 queries with all the keys each (attn_decode.hip: every tile reads K and V again, twice or more with its column
+// shares) and workgroups of 128 queries (a CU per tile).  Shares read the cache once, at some 10 us + 6 TB/s, and pay about
+// 5 us for the merge: not on short caches.  us without / with shares (both launches): 32 heads of 128: 100 queries on 2.6 k
+// keys 22.1 / 22.1, 128 on 3.1 k 25.6 / 26.1, 40 on 3 k 23.4 / 21.0, 100 on 4.1 k 32.1 / 28.7, 128 on 8.1 k 56.8 / 43.3, 50
+// on 16 k 98 / 57, 300 on 4.3 k 61.5 / 45.4; 8 heads of 128: 100 on 2.6 k 16.2 / 17.7, 40 on 3 k 17.6 / 15.1, 500 on 3.5 k
+// 25.6 / 23.0, 128 on 16 k 73 / 28; 16 heads of 64: 100 on 3.1 k 13.9 / 14.0, 40 on 4 k 15.4 / 12.5, 128 on 9.1 k 30 / 18; 71
+// heads of 64: 64 on 4.1 k 25.1 / 25.8, 40 on 6 k 33.8 / 31.4, and, with more than 256 tiles of 32 queries, 100 on 2.6 k 29.0
+// / 21.5, 128 on 16 k 137 / 70.
+static int key_shares(int64_t bh, int seq_q, int seq_kv, int head_dim) {
+    const int64_t tiles = ((int64_t)seq_q + 127) / 128 * bh, tiles32 = ((int64_t)seq_q + 31) / 32 * bh;
+    if (seq_q <= 32 || tiles > 128 || seq_kv < (head_dim == 128 ? 3072 : tiles32 > 256 ? 2560 : 4096)) return 0;
+    return (int)min((int64_t)kMaxShares, 256 / tiles);
+}
+
+int64_t attn_share_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
+    const int64_t bh = (int64_t)batch * n_q_heads;
+    return bh * key_shares(bh, seq_q, seq_kv, head_dim) * seq_q * (head_dim + 2) * 4;
+}
+
+template <int D>
+static hipError_t launch_shares(AttnArgs a, hipStream_t s) {
+    a.n_qtiles = (a.Sq + 127) / 128;
+    a.n_split = key_shares((int64_t)a.B * a.Hq, a.Sq, a.Skv, D);
+    hipLaunchKernelGGL((attn_fwd16_share_kernel<D>), dim3((unsigned)(a.n_qtiles * a.B * a.Hq * a.n_split)), dim3(512), 0, s, a);
+    if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    hipLaunchKernelGGL((attn_merge_shares_kernel<D>), dim3((unsigned)(((int64_t)a.B * a.Hq * a.Sq + 3) / 4)), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+hipError_t launch_attn_shares(const AttnArgs& a, int head_dim, hipStream_t s) {
+    return head_dim == 128 ? launch_shares<128>(a, s) : launch_shares<64>(a, s);
 }
 
 template <int D, int NW, int MODE>

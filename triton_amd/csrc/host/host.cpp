@@ -404,8 +404,10 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     trn_attn_desc d = attn_desc(q4, k4, v4, o4, scale, causal);
     d.q_norm = q_norm ? 1 : 0;
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[7]));
-    const int64_t need = c1.given ? trn_attn_stats_workspace_bytes(&d) : trn_attn_workspace_bytes(&d);
+    int64_t need = c1.given ? trn_attn_stats_workspace_bytes(&d) : trn_attn_workspace_bytes(&d);
     void* ws = need ? workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true).data_ptr() : nullptr;
+    if (!c1.given && !need && (need = trn_attn_chunk_workspace_bytes(&d)) > 0)
+        ws = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev).data_ptr();
     float* rows = c1.given ? static_cast<float*>(workspace(w, noise.given ? "lse_pert" : "lse", {1, H, M}, c10::ScalarType::Float, X.dev).data_ptr()) : nullptr;
     const View wts[3] = {wq, wk, wv};
     const View outs[3] = {q, make(Kc, Kc.p + 2 * P * Kc.st[1], {H, M, D}, {Kc.st[0], Kc.st[1], Kc.st[2]}),
