@@ -480,10 +480,16 @@ int validate_attn(const trn_attn_desc* d, bool need_v) {
 }  // namespace trn
 
 namespace trn {
-// Workgroup shape of the forward kernel with score perturbation: 8 waves x 32 queries when that still fills the chip.
+// Workgroup shape of the forward kernel with score perturbation: 8 waves x 32 queries (one workgroup per CU; each K/V stage
+// is fetched from L2 once per 256 queries), or 4 waves x 32 (two per CU).  Unmasked, wide from one workgroup per CU.  Causal,
+// where workgroups differ in length: with head_dim 128 from 384 wide workgroups of at least six tiles per head; fewer tiles
+// waste too much of the last one, and head_dim 64 prefers the finer grid throughout.  us, narrow / wide: 32 heads of 128,
+// fp32 noise: 4096 keys 343 / 316, 3600 241 / 230, 3126 201 / 191, 2048 (256 workgroups) 124 / 122; fp16: 2 x 1501 87 / 80,
+// but 2560 (320) 122 / 135, 4 x 777 77 / 85, 8 x 512 55 / 63; 8 x 8 heads, 1448: 97 / 98.  Head_dim 64: 142 heads, 1559 keys
+// 161 / 181; 284 heads, 392 keys 38 / 51; 128 heads, 1448 keys 127 / 130; 48 heads, 2300 keys 148 / 144.
 static bool noise_kernel_wide(const trn_attn_desc* d) {
-    const int64_t n_wide = (int64_t)((d->seq_q + 255) / 256) * d->batch * d->n_q_heads;
-    return n_wide >= (!d->causal ? 256 : d->head_dim == 128 ? 512 : 1024);
+    const int64_t n256 = ((int64_t)d->seq_q + 255) / 256, n_wide = n256 * d->batch * d->n_q_heads;
+    return d->causal ? d->head_dim == 128 && n256 >= 6 && n_wide >= 384 : n_wide >= 256;
 }
 }  // namespace trn
 
@@ -681,9 +687,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     // Without score perturbation: the 16x16x32 kernel, in the workgroup shape its launcher's rule picks.
     if (!noise)
         return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0), s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
-    // With it: 8 waves x 32 queries per workgroup (one workgroup per CU; each K/V stage is fetched from L2 once per
-    // 256 queries) when that still fills the chip -- one workgroup per CU for unmasked attention, two rounds under a
-    // causal mask, where workgroups differ in length; otherwise 4 waves x 32 (two workgroups per CU).
+    // With it: the shape of noise_kernel_wide().
     const bool wide = noise_kernel_wide(d);
 #define TRN_LAUNCH(D_, NW_) launch_fwd<D_, NW_>(a, s)
     if (d->head_dim == 128) e = wide ? TRN_LAUNCH(128, 8) : TRN_LAUNCH(128, 4);
