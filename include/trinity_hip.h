@@ -124,7 +124,8 @@ int trn_attn_fwd_f16(const trn_attn_desc* desc, const void* q, const void* k, co
  *
  * A chunk of more than 32 queries per head on a long cache has a workspace of its own, trn_attn_chunk_workspace_bytes(desc)
  * bytes (0: none), which needs no initial contents: the keys are then shared out over workgroups whose partial results a
- * second launch merges.  Without it, or with a smaller one, the call is trn_attn_fwd_f16 as above.  No size depends on
+ * second launch merges.  (Its first 512 bytes, where the split decode shapes keep their counters, are left alone: one
+ * zero-filled workspace of the larger size may serve both, one call at a time.)  Without it, or with a smaller one, the call is trn_attn_fwd_f16 as above.  No size depends on
  * seq_kv, so that a cache that grows from call to call keeps its workspace.
  */
 int64_t trn_attn_workspace_bytes(const trn_attn_desc* desc);

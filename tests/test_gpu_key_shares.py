@@ -55,7 +55,23 @@ def test_which_problems_share_out_their_keys():
     def need(heads, sq, skv, D):
         q, k = torch.empty(1, heads, sq, D, dtype=torch.float16, device="cuda"), torch.empty(1, 1, skv, D, dtype=torch.float16, device="cuda")
         return chunk_bytes(q, k, q, 1.0, True)
-    assert need(8, 32, 8192, 128) == 0 and need(8, 33, 8192, 128) == need(8, 33, 3072, 128) == 8 * 16 * 33 * 130 * 4
-    assert need(8, 33, 3071, 128) == 0 and need(8, 33, 4095, 64) == 0 and need(8, 33, 4096, 64) == 8 * 16 * 33 * 66 * 4
-    assert need(71, 100, 2560, 64) == 71 * 3 * 100 * 66 * 4 and need(71, 100, 2559, 64) == 0 and need(71, 64, 2560, 64) == 0
+    assert need(8, 32, 8192, 128) == 0 and need(8, 33, 8192, 128) == need(8, 33, 3072, 128) == 512 + 8 * 16 * 33 * 130 * 4
+    assert need(8, 33, 3071, 128) == 0 and need(8, 33, 4095, 64) == 0 and need(8, 33, 4096, 64) == 512 + 8 * 16 * 33 * 66 * 4
+    assert need(71, 100, 2560, 64) == 512 + 71 * 3 * 100 * 66 * 4 and need(71, 100, 2559, 64) == 0 and need(71, 64, 2560, 64) == 0
     assert need(128, 128, 4096, 128) > 0 and need(129, 128, 4096, 128) == 0
+
+
+def test_one_workspace_for_chunks_and_single_tokens():
+    """The split decode shapes find their arrival counters as they left them, whatever a chunk wrote in between."""
+    from triton_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(5)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").half()
+    k, v, chunk, one = r(1, 8, 5000, 128), r(1, 8, 5000, 128), r(1, 8, 100, 128), r(1, 8, 1, 128)
+    n = max(chunk_bytes(chunk, k, chunk, 0.1, False), ops.attention_workspace_bytes(one, k, v, one, 0.1, False))
+    ws, want, got = torch.zeros(n, dtype=torch.uint8, device="cuda"), torch.zeros_like(one), torch.zeros_like(one)
+    ops.attention(one, k, v, want, 0.1, False, workspace=torch.zeros_like(ws))
+    ops.attention(chunk, k, v, torch.zeros_like(chunk), 0.1, False, workspace=ws)
+    assert not ws[:512].any()
+    ops.attention(one, k, v, got, 0.1, False, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)

@@ -644,13 +644,19 @@ static int key_shares(int64_t bh, int seq_q, int seq_kv, int head_dim) {
     return (int)min((int64_t)kMaxShares, 256 / tiles);
 }
 
+// The decode kernel keeps the arrival counters of its key splits (128 heads at most) at the head of a workspace and relies on
+// finding them zero: the shares stay behind them, so that one zero-filled workspace serves both kinds of call.
+constexpr int64_t kCounterBytes = 512;
+
 int64_t attn_share_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
     const int64_t bh = (int64_t)batch * n_q_heads;
-    return bh * key_shares(bh, seq_q, seq_kv, head_dim) * seq_q * (head_dim + 2) * 4;
+    const int shares = key_shares(bh, seq_q, seq_kv, head_dim);
+    return shares == 0 ? 0 : kCounterBytes + bh * shares * seq_q * (head_dim + 2) * 4;
 }
 
 template <int D>
 static hipError_t launch_shares(AttnArgs a, hipStream_t s) {
+    a.ws += kCounterBytes / sizeof(float);
     a.n_qtiles = (a.Sq + 127) / 128;
     a.n_split = key_shares((int64_t)a.B * a.Hq, a.Sq, a.Skv, D);
     hipLaunchKernelGGL((attn_fwd16_share_kernel<D>), dim3((unsigned)(a.n_qtiles * a.B * a.Hq * a.n_split)), dim3(512), 0, s, a);
