@@ -69,3 +69,82 @@ def test_layouts_the_native_forward_declines_still_run(what):
             continue
         assert torch.equal(a[n].to(want[n].dtype).reshape(want[n].shape) if n != "C_out1" else a[n].float(),
                            want[n] if n != "C_out1" or what != "mixed statistics" else want[n].half().float()), n
+
+
+@pytest.mark.parametrize("what", ["five axes", "flat output", "two-axis output of other rows"])
+def test_rmsnorm_of_any_shape_that_flattens(what):
+    """X and X_norm are read as rows of X's last axis, whatever their shapes."""
+    from triton_amd import modules
+    mod = modules.get("rms")
+    a = _tensors(mod)
+    want = {n: t.clone() for n, t in a.items()}
+    mod.forward(*want.values())
+    n = a["X"].numel()
+    if what == "five axes":
+        a["X"], a["X_norm"] = a["X"].view(2, 1, 3, 2, 256), a["X_norm"].view(2, 1, 3, 2, 256)
+    elif what == "flat output":
+        a["X_norm"] = a["X_norm"].view(n)
+    else:
+        a["X_norm"] = a["X_norm"].view(n // 64, 64)
+    mod.forward(*a.values())
+    torch.cuda.synchronize()
+    assert torch.equal(a["X_norm"].view(-1, 256), want["X_norm"])
+
+
+def test_scores_of_any_contiguous_shape():
+    from triton_amd import modules
+    mod = modules.get("roco")
+    a = _tensors(mod)
+    want = {n: t.clone() for n, t in a.items()}
+    mod.forward(*want.values())
+    a["C_out1"] = a["C_out1"].view(1, 1, 2, 2, 70)
+    mod.forward(*a.values())
+    torch.cuda.synchronize()
+    for n in a:
+        assert torch.equal(a[n].reshape(want[n].shape), want[n]), n
+
+
+def test_operators_refuse_five_axes():
+    from triton_amd import ops
+    x = torch.zeros(1, 1, 1, 4, 64, dtype=torch.float16, device="cuda")
+    with pytest.raises(ValueError):
+        ops.rmsnorm(x, None, torch.zeros_like(x), 1e-5)
+
+
+def test_a_module_copies_after_its_first_forward():
+    import copy
+    import pickle
+    from triton_amd import modules
+    mod = modules.get("gmlp", "linear")
+    a = _tensors(mod)
+    mod.forward(*a.values())
+    want = a["O"].clone()
+    for other in (copy.deepcopy(mod), copy.copy(mod), pickle.loads(pickle.dumps(mod))):
+        a["O"].zero_()
+        other.forward(*a.values())
+        torch.cuda.synchronize()
+        assert torch.equal(a["O"], want)
+
+
+@pytest.mark.parametrize("variant,form,kw", [("keyformer", "prefill", {}), ("keyformer", "decode", dict(head_dim=64))])
+@pytest.mark.parametrize("what", ["same row for every query", "rows far apart"])
+def test_noise_that_the_kernels_cannot_address_is_copied(variant, form, kw, what):
+    """fp16 noise expanded along the queries, or with rows further apart than 32-bit offsets within a head reach."""
+    from triton_amd import modules
+    mod = modules.get(variant, form, **kw)
+    a = _tensors(mod)
+    n = a["noise"]
+    if what == "same row for every query":
+        a["noise"] = n[..., :1, :].expand(n.shape)
+    else:
+        pitch = 0x80000000 // (4 * n.shape[-2])
+        wide = torch.empty(n.shape[-2] * pitch, dtype=torch.float16, device="cuda")
+        a["noise"] = wide.as_strided(n.shape, (*[n.shape[-1]] * (n.dim() - 2), pitch, 1))      # (heads side by side)
+        a["noise"].copy_(n)
+    b = {m: t if m == "noise" else t.clone() for m, t in a.items()}
+    b["noise"] = a["noise"].float().contiguous()
+    mod.forward(*a.values())
+    mod.forward(*b.values())
+    torch.cuda.synchronize()
+    for m in a:
+        assert torch.equal(a[m].float(), b[m].float()), m

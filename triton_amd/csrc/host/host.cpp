@@ -26,6 +26,7 @@ namespace {
 struct ValueErr { std::string msg; };
 struct TrnErr { const char* fn; int status; };
 struct PyErrSet {};      // a Python exception is already set
+struct Declined { std::string why; };      // more than four dimensions: the general path may still flatten them
 
 PyObject* g_trn_error = nullptr;      // triton_amd._lib.TrnError
 
@@ -70,7 +71,7 @@ struct View {
 View view_of(const at::Tensor& t, const char* name) {
     View v;
     v.dim = (int)t.dim();
-    NEED(v.dim <= 4, "%s: expected at most 4 dimensions, got %d", name, v.dim);
+    if (v.dim > 4) throw Declined{format("%s: expected at most 4 dimensions, got %d", name, v.dim)};
     const auto sz = t.sizes();
     const auto sd = t.strides();
     for (int i = 0; i < v.dim; ++i) { v.s[i] = sz[i]; v.st[i] = sd[i]; }
@@ -254,12 +255,13 @@ bool f_rmsnorm(Args a, Py_ssize_t n) {                    // x, gamma | None, y,
 bool f_rmsnorm_forward(Args a, Py_ssize_t n) {            // eps, X, X_norm, gamma
     count(n, 4, "rmsnorm_forward");
     View x = arg(a[1], "X"), y = arg(a[2], "X_norm");
-    if (x.dim < 1 || y.dim < 1) return false;
+    // (an output of another shape is read as rows of X's width, and an empty one refused, by the general path)
+    if (x.dim < 1 || y.dim < 1 || x.s[x.dim - 1] != y.s[y.dim - 1] || x.numel() == 0 || y.numel() == 0) return false;
     for (View* t : {&x, &y})
         if (t->dim != 2) {
             if (!t->contiguous()) return false;
-            const int64_t c = t->s[t->dim - 1], r = c ? t->numel() / c : 0;
-            *t = make(*t, t->p, {r, c}, {c, 1});
+            const int64_t c = t->s[t->dim - 1];
+            *t = make(*t, t->p, {t->numel() / c, c}, {c, 1});
         }
     rmsnorm_call(x, opt(a[3], "gamma"), y, num(a[0]));
     return true;
@@ -325,6 +327,15 @@ bool f_qknorm_forward(Args a, Py_ssize_t n) {             // workspaces, scale |
     return true;
 }
 
+// Noise that the kernels read as it is.  fp16 rows and fp32 rows off the 16-byte grid that overlap (an expanded tensor) or lie
+// too far apart for 32-bit offsets within a head are copied by the general path; aligned fp32 has always been passed on.
+bool direct_noise(const View& n) {
+    if (!(n.half() || n.f32()) || !n.unit() || n.dim < 3) return false;
+    bool aligned = n.f32() && reinterpret_cast<uintptr_t>(n.p) % 16 == 0;
+    for (int i = 0; i < n.dim - 1; ++i) aligned = aligned && n.st[i] % 4 == 0;
+    return aligned || (n.st[n.dim - 2] >= n.s[n.dim - 1] && n.s[n.dim - 2] * n.st[n.dim - 2] * 4 + 1024 <= 0x7fffffffLL);
+}
+
 // the statistics tensors the kernels can write themselves
 bool direct_outputs(const View& a, const View* b, int64_t numel) {
     if (!(a.half() || a.f32()) || !a.cuda || !a.contiguous() || a.numel() != numel) return false;
@@ -338,7 +349,7 @@ bool f_key_scores_forward(Args a, Py_ssize_t n) {         // workspaces, scale |
     const View c1 = arg(a[9], "C_out");
     const OptView c2 = opt(a[10], "C_out2"), noise = opt(a[11], "noise");
     if (!q.cuda || !direct_outputs(c1, c2.given ? &c2.v : nullptr, q.s[0] * q.s[1] * k.s[2])) return false;
-    if (noise.given && !((noise.v.half() || noise.v.f32()) && noise.v.unit())) return false;
+    if (noise.given && !direct_noise(noise.v)) return false;
     trn_attn_desc d = attn_desc(q, k, v, o, scale_of(a[1], q.s[3]), flag(a[2]));
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[3]));
     const at::Tensor& rows = workspace(w, noise.given ? "lse_pert" : "lse", {q.s[0], q.s[1], q.s[2]}, c10::ScalarType::Float, q.dev);
@@ -396,7 +407,7 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
          Kc.shape().c_str(), (long long)D);
     if (O2.s[0] != M || O2.s[1] != N || (head_major && !O2.contiguous())) return false;
     if (c1.given && !direct_outputs(c1.v, c2.given ? &c2.v : nullptr, H * PM)) return false;
-    if (noise.given && !(noise.v.dim == 3 && (noise.v.half() || noise.v.f32()) && noise.v.unit())) return false;
+    if (noise.given && !(noise.v.dim == 3 && direct_noise(noise.v))) return false;
     const View q = view_of(workspace(w, "q", {H, M, D}, X.dt, X.dev), "q");
     const View q4 = as4(q, "q"), k4 = as4(Kc, "K_cache"), v4 = as4(Vc, "V_cache");
     const View o4 = head_major ? make(O2, O2.p, {1, H, M, D}, {H * M * D, M * D, D, 1}) : make(O2, O2.p, {1, H, M, D}, {M * O2.st[0], D, O2.st[0], 1});
@@ -458,13 +469,17 @@ PyObject* raise_trn(const char* fn, int status) {
     if (e) { PyErr_SetObject(g_trn_error, e); Py_DECREF(e); }
     return nullptr;
 }
-template <bool (*F)(Args, Py_ssize_t)>
+// OP: an operator of its own, which has no general path behind it.
+template <bool (*F)(Args, Py_ssize_t), bool OP>
 PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n) {
     try {
         if (F(a, n)) Py_RETURN_TRUE;
         Py_RETURN_FALSE;
     } catch (const ValueErr& e) {
         PyErr_SetString(PyExc_ValueError, e.msg.c_str());
+    } catch (const Declined& e) {
+        if (!OP) Py_RETURN_FALSE;
+        PyErr_SetString(PyExc_ValueError, e.why.c_str());
     } catch (const TrnErr& e) {
         return raise_trn(e.fn, e.status);
     } catch (const PyErrSet&) {
@@ -509,9 +524,10 @@ PyObject* set_error_class(PyObject*, PyObject* cls) {
     Py_RETURN_NONE;
 }
 
-#define FN(name) {#name, (PyCFunction)(void (*)(void))entry<f_##name>, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {FN(rmsnorm), FN(rmsnorm_forward), FN(attention), FN(attention_forward), FN(qknorm_forward), FN(key_scores_forward),
-                         FN(prenorm_qkv), FN(prenorm_forward), FN(decode_forward), FN(lora_forward), FN(gmlp_forward),
+#define FN(name) {#name, (PyCFunction)(void (*)(void))entry<f_##name, false>, METH_FASTCALL, nullptr}
+#define OPERATOR(name) {#name, (PyCFunction)(void (*)(void))entry<f_##name, true>, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {OPERATOR(rmsnorm), OPERATOR(attention), OPERATOR(prenorm_qkv), FN(rmsnorm_forward), FN(attention_forward),
+                         FN(qknorm_forward), FN(key_scores_forward), FN(prenorm_forward), FN(decode_forward), FN(lora_forward), FN(gmlp_forward),
                          {"set_error_class", set_error_class, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", "host side of the modules' forward", -1, methods};
 

@@ -80,6 +80,9 @@ class FusedModule:
         self._host = None                   # (the native side, loaded with the first forward)
         self._hws = None                    # its view of these workspaces
 
+    def __getstate__(self):
+        return {**self.__dict__, "_host": None, "_hws": None}      # (a copy makes its own native view)
+
     def _workspace(self, name: str, shape, dtype, device) -> torch.Tensor:
         return _workspace_in(self._ws, type(self).__name__, name, shape, dtype, device)
 
@@ -128,10 +131,18 @@ def _scale(scale: Optional[float], head_dim: int) -> float:
     return head_dim ** -0.5 if scale is None else float(scale)
 
 
+def _noise_aligned(n4: torch.Tensor) -> bool:
+    return (n4.dtype == torch.float32 and n4.stride(3) == 1 and n4.data_ptr() % 16 == 0
+            and all(n4.stride(i) % 4 == 0 for i in range(3)))
+
+
 def _noise_operand(mod: "FusedModule", n4: torch.Tensor) -> torch.Tensor:
     """The noise as the kernels read it: fp32 or fp16 rows of unit innermost stride at any pitch (the reference's noise is
-    fp16 with an arbitrary key count, convert_eval_rms.py:201).  Anything else is copied into an fp32 workspace."""
-    if n4.dtype in (torch.float32, torch.float16) and n4.stride(3) == 1:
+    fp16 with an arbitrary key count, convert_eval_rms.py:201) that do not overlap and that 32-bit byte offsets within a
+    head reach.  Anything else is copied into an fp32 workspace."""
+    pitch = n4.stride(2)
+    if _noise_aligned(n4) or (n4.dtype in (torch.float32, torch.float16) and n4.stride(3) == 1 and pitch >= n4.shape[3]
+                              and n4.shape[2] * pitch * 4 + 1024 <= 0x7fffffff):
         return n4
     buf = mod._workspace("noise32", tuple(n4.shape), torch.float32, n4.device)
     buf.copy_(n4)
@@ -142,9 +153,7 @@ def _noise_fp32(mod: "FusedModule", n4: torch.Tensor) -> torch.Tensor:
     """The noise as the un-reduced form reads it: fp32, base and every pitch a multiple of 16 bytes.  Anything else is
     copied into a workspace whose rows are padded to a multiple of 4 floats; the padding is never read as a key (the
     kernel masks by key index, with selects)."""
-    ok = (n4.dtype == torch.float32 and n4.stride(3) == 1 and n4.data_ptr() % 16 == 0
-          and all(n4.stride(i) % 4 == 0 for i in range(3)))
-    if ok:
+    if _noise_aligned(n4):
         return n4
     B, H, Sq, Skv = n4.shape
     pitch = (Skv + 3) // 4 * 4
