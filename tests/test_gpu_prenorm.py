@@ -109,7 +109,7 @@ def test_projection_reads_and_writes_stay_inside_its_views(T, K, nq, nkv, D):
 def test_projection_tilings_between_decode_and_long_prompts(T, K, nq, nkv, D, norm):
     """Edges of each tile (tokens, columns, ragged hidden, fewer k-tiles than ring stages) with operands cut out of
     NaN-filled buffers and outputs checked for strays.  Tolerance: one fp16 rounding of the output and, with gamma, one of
-    each product gamma * w: 3.6e-4 of the output's spread measured and expected, so 8e-3 of it is more than 20 sigma."""
+    each product gamma * x: 3.6e-4 of the output's spread measured and expected, so 8e-3 of it is more than 20 sigma."""
     from triton_amd import ops
     g = torch.Generator().manual_seed(T + K)
     nan = float("nan")
@@ -147,3 +147,25 @@ def test_weight_stream_at_token_and_hidden_edges(T, K):
     torch.cuda.synchronize()
     for o, w in zip(outs, ref.qkv_project(x[None], gamma, *ws, 1e-5, True)):
         close(o, w[0], atol=8e-3 * float(w.float().std()), rtol=1e-3)
+
+
+@pytest.mark.parametrize("T,nq,nkv", [(20, 1024, 256), (64, 1024, 256), (256, 6144, 1024), (512, 6144, 1024), (700, 6144, 1024)])
+def test_small_gamma_loses_no_precision(T, nq, nkv):
+    """Norm weights around 1e-3 on weights of standard deviation 0.02, every tiling up to two 128 x 128 tiles per CU: the
+    products gamma * x stay normal fp16 numbers where gamma * w would not.  One rounding of each product and one of the output,
+    2^-11 / sqrt(3) relative at most in the root mean square: 4.0e-4 together (2.9e-4 measured; 8.6e-4 with gamma * w)."""
+    from triton_amd import ops
+    K = 1024
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, gamma = r(T, K).half(), (1e-3 * (1 + 0.02 * r(K))).half()
+    ws = [(0.02 * r(K, n)).half() for n in (nq, nkv, nkv)]
+    outs = [torch.zeros(T, n, dtype=torch.float16, device="cuda") for n in (nq, nkv, nkv)]
+    ops.prenorm_qkv(x, gamma, *ws, *[o.unflatten(1, (-1, 64)).permute(1, 0, 2) for o in outs], 1e-5, True)
+    torch.cuda.synchronize()
+    xd = x.double()
+    xn = xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-5) * gamma.double()
+    for o, w in zip(outs, ws):
+        want = xn @ w.double()
+        err = float((o.double() - want).norm() / want.norm())
+        assert err <= 4.0e-4, err

@@ -13,8 +13,9 @@
 // The eight waves are TM token groups x TN column groups x four contraction steps of 16: a wave owns 32 NTB tokens x 64
 // columns of its stage's 16-column step, so that its operands feed 2 NTB MFMAs each stage, and the four partial tiles
 // are added through LDS at the end.  One barrier per stage; the operands of the next stage are read behind the MFMAs of
-// the one in hand.  gamma is multiplied into the W operand, the sum of squares is taken from the X operand by the waves
-// of the first column group (as in the wide kernel).
+// the one in hand.  gamma is multiplied into the X operand, NTB products a stage instead of two: gamma * w falls out of the
+// normal fp16 range where gamma * x does not (distance from float64 with gamma around 1e-3 and weights of 0.02: 8.9e-4
+// against 2.9e-4).  The sum of squares is taken from X as read, by the waves of the first column group.
 //
 // Measured, weights cold in HBM, us before (128 x 128 kernel) / now: 4096 -> 12288 without norm 33 tokens 63 / 26, 64
 // tokens 63 / 29, 100 tokens 70 / 35; 4096 -> 6144 with norm 100 tokens 73 / 25, 256 tokens 73 / 37, 512 tokens 73 / 48;
@@ -137,17 +138,19 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs 
         __builtin_amdgcn_s_waitcnt(0x0070 | (kBehind & 15) | ((kBehind >> 4) << 14));
         __builtin_amdgcn_s_barrier();        // (a bare barrier: the loads in flight must stay in flight)
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NORM == 2) { wa[0] = wa[0] * g; wa[1] = wa[1] * g; }
+        half8_t xg[NTB];                     // (gamma is used up before its slot of the ring is refilled)
+#pragma unroll
+        for (int tb = 0; tb < NTB; ++tb) { if constexpr (NORM == 2) xg[tb] = xb[tb] * g; else xg[tb] = xb[tb]; }
         fetch(s + 4, F, g);
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) {
-            acc[tb][0] = mfma32(wa[0], xb[tb], acc[tb][0]);
+            acc[tb][0] = mfma32(wa[0], xg[tb], acc[tb][0]);
             if (tb == 0) { wn[0] = read_w(Cn, 0); if (NTB == 1) wn[1] = read_w(Cn, 1); }
             if (tb == 1) wn[1] = read_w(Cn, 1);
             if (NTB <= 2) xn[tb] = read_x(Cn, tb);
             else if (tb >= 2) { xn[2 * tb - 4] = read_x(Cn, 2 * tb - 4); xn[2 * tb - 3] = read_x(Cn, 2 * tb - 3); }
             __builtin_amdgcn_sched_barrier(0);
-            acc[tb][1] = mfma32(wa[1], xb[tb], acc[tb][1]);
+            acc[tb][1] = mfma32(wa[1], xg[tb], acc[tb][1]);
             if (stats) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
