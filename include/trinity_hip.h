@@ -238,7 +238,9 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
  * modules call.  As trn_attn_fwd_stats_ws_f16 (one launch with at most 32 queries per head unless the workspace makes it
  * split the keys, two launches otherwise), with
  *   noise       nullable; fp16 when noise_half is set, float otherwise.  Rows at any pitch and any element alignment (the
- *               reference's noise [.., M, P + M] is fp16 with any key count); desc's noise strides count elements.
+ *               reference's noise [.., M, P + M] is fp16 with any key count); desc's noise strides count elements.  One
+ *               head is addressed with 32-bit offsets: (seq_q + TRN_STATS_SPARE_ROWS) * noise_stride_s * 4 < 2^31 where
+ *               the statistics are a launch of their own (a single launch of at most 32 queries takes somewhat more).
  *   rows        float [batch, n_q_heads, seq_q], required: receives the row normalisers of the scores the statistics are
  *               of (perturbed with noise, plain without).
  *   out1, out2  [batch, n_q_heads, seq_kv] contiguous, fp16 when out_half is set (the float result rounded once), float
@@ -246,6 +248,7 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
  *               and standard deviation as trn_attn_colmeanstd_f16.
  *   workspace   nullable: trn_attn_stats_workspace_bytes(desc) zero-initialised bytes, as trn_attn_fwd_stats_ws_f16.
  */
+#define TRN_STATS_SPARE_ROWS 128        /* query rows past the last that the statistics kernels may ask for (as zeros) */
 int trn_attn_key_scores_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v, void* o,
                             const void* noise, int32_t noise_half, float* rows, void* out1, void* out2,
                             int32_t out_half, int32_t mean_std, void* workspace, int64_t workspace_bytes, void* stream);

@@ -127,9 +127,10 @@ def test_a_module_copies_after_its_first_forward():
 
 
 @pytest.mark.parametrize("variant,form,kw", [("keyformer", "prefill", {}), ("keyformer", "decode", dict(head_dim=64))])
-@pytest.mark.parametrize("what", ["same row for every query", "rows far apart"])
+@pytest.mark.parametrize("what", ["same row for every query", "rows far apart", "rows too far apart for the statistics"])
 def test_noise_that_the_kernels_cannot_address_is_copied(variant, form, kw, what):
-    """fp16 noise expanded along the queries, or with rows further apart than 32-bit offsets within a head reach."""
+    """fp16 noise expanded along the queries, or with rows further apart than 32-bit offsets within a head reach: in both
+    launches, or with the spare rows of the statistics only."""
     from triton_amd import modules
     mod = modules.get(variant, form, **kw)
     a = _tensors(mod)
@@ -137,7 +138,7 @@ def test_noise_that_the_kernels_cannot_address_is_copied(variant, form, kw, what
     if what == "same row for every query":
         a["noise"] = n[..., :1, :].expand(n.shape)
     else:
-        pitch = 0x80000000 // (4 * n.shape[-2])
+        pitch = 0x80000000 // (4 * (n.shape[-2] + (64 if "statistics" in what else 0)))
         wide = torch.empty(n.shape[-2] * pitch, dtype=torch.float16, device="cuda")
         a["noise"] = wide.as_strided(n.shape, (*[n.shape[-1]] * (n.dim() - 2), pitch, 1))      # (heads side by side)
         a["noise"].copy_(n)
@@ -148,3 +149,16 @@ def test_noise_that_the_kernels_cannot_address_is_copied(variant, form, kw, what
     torch.cuda.synchronize()
     for m in a:
         assert torch.equal(a[m].float(), b[m].float()), m
+
+
+def test_noise_that_the_statistics_refuse_leaves_the_outputs_alone():
+    """A problem of two launches whose second does not take the noise is refused before the first."""
+    from triton_amd import _lib, ops
+    q = torch.zeros(1, 1, 64, 64, dtype=torch.float16, device="cuda")
+    pitch = 0x80000000 // (4 * 128)
+    noise = torch.zeros(64 * pitch, dtype=torch.float16, device="cuda").as_strided((1, 1, 64, 64), (0, 0, pitch, 1))
+    o, rows, score = torch.full_like(q, 7), torch.full((1, 1, 64), 7.0, device="cuda"), torch.full((1, 1, 64), 7.0, device="cuda")
+    with pytest.raises(_lib.TrnError):
+        ops.attention_key_scores(q, q, q, o, 1.0, False, rows, score, noise=noise)
+    torch.cuda.synchronize()
+    assert all(bool((t == 7).all()) for t in (o, rows, score))

@@ -59,6 +59,10 @@ int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const voi
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
                  bool n16 = false, bool s16 = false, bool any_pitch = false);
 
+// The checks of attn_colstats by themselves, for a caller that launches something else before it.
+int attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
+                        const float* out_sum, const float* out_sumsq, bool n16, bool any_pitch);
+
 // Checks, argument block and kernel choice behind the column statistics (attn_colstats.hip); mean_std: the two outputs
 // are the mean and standard deviation; n16 / s16: fp16 noise / outputs; any_pitch: fp32 noise on any dword (16-byte
 // buffer loads need no more).

@@ -571,8 +571,8 @@ extern "C" int trn_attn_colmeanstd_f16(const trn_attn_desc* d, const void* q, co
     return trn::attn_colstats(d, q, k, lse, nullptr, out_mean, out_std, 1, stream);
 }
 
-int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
-                       float* out_sum, float* out_sumsq, int mean_std, void* stream, bool n16, bool s16, bool any_pitch) {
+int trn::attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
+                             const float* out_sum, const float* out_sumsq, bool n16, bool any_pitch) {
     if (!d || !q || !k || !lse) return TRN_E_NULL;
     if (!out_sum && !out_sumsq) return TRN_E_NULL;
     int st = validate_attn(d, false);
@@ -583,14 +583,22 @@ int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, con
         if (!(d->tau > 0.f)) return TRN_E_UNSUPPORTED;
         if (d->noise_stride_s < d->seq_kv) return TRN_E_STRIDE;
         // one head's noise is addressed with 32-bit byte offsets
-        if (((int64_t)d->seq_q + 128) * d->noise_stride_s * 4 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
+        if (((int64_t)d->seq_q + TRN_STATS_SPARE_ROWS) * d->noise_stride_s * 4 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
         if (n16 || any_pitch ? (reinterpret_cast<uintptr_t>(noise) & (n16 ? 1u : 3u)) != 0
                 : !aligned16(noise) || !pitch16(d->noise_stride_s, 4) || !pitch16(d->noise_stride_h, 4) || !pitch16(d->noise_stride_b, 4))
             return TRN_E_ALIGN;
     }
     // Q tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base (with room for the tile requested
     // past the end, which must stay representable to read as zeros)
-    if (((int64_t)d->seq_q + 128) * d->q_stride_s * 2 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
+    if (((int64_t)d->seq_q + TRN_STATS_SPARE_ROWS) * d->q_stride_s * 2 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
+    if (((int64_t)d->seq_kv + CBN - 1) / CBN * d->batch * d->n_q_heads > 0x7fffffffLL) return TRN_E_SHAPE;
+    return TRN_OK;
+}
+
+int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
+                       float* out_sum, float* out_sumsq, int mean_std, void* stream, bool n16, bool s16, bool any_pitch) {
+    const int st = attn_colstats_check(d, q, k, lse, noise, out_sum, out_sumsq, n16, any_pitch);
+    if (st != TRN_OK) return st;
     ColArgs a;
     a.q = (const half_t*)q; a.k = (const half_t*)k; a.lse = lse; a.noise = noise;
     a.out_sum = out_sum; a.out_sumsq = out_sumsq;
@@ -603,7 +611,6 @@ int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, con
     a.c1 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.causal = d->causal ? 1 : 0;
     a.mean_std = mean_std; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
-    if ((int64_t)a.n_kvtiles * a.B * a.Hq > 0x7fffffffLL) return TRN_E_SHAPE;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
     if (d->head_dim == 128) e = !noise ? launch_col_plain<128>(a, s) : n16 ? launch_col<128, 2>(a, s) : launch_col<128, 1>(a, s);

@@ -623,7 +623,10 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     // a handful of queries per head and no split of the keys: the statistics are a second sweep inside the same kernel
     if (d->seq_q <= 32 && !split && !mean_std)
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true);
-    const int st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, split ? workspace : nullptr, split ? workspace_bytes : 0,
+    // (a problem that the second launch refuses is refused before the first has written anything)
+    int st = attn_colstats_check(d, q, k, rows, n, s1, s2, n16, true);
+    if (st != TRN_OK) return st;
+    st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, split ? workspace : nullptr, split ? workspace_bytes : 0,
                                 nullptr, nullptr, stream, nullptr, n16, false, true);
     if (st != TRN_OK) return st;
     return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);

@@ -328,12 +328,13 @@ bool f_qknorm_forward(Args a, Py_ssize_t n) {             // workspaces, scale |
 }
 
 // Noise that the kernels read as it is.  fp16 rows and fp32 rows off the 16-byte grid that overlap (an expanded tensor) or lie
-// too far apart for 32-bit offsets within a head are copied by the general path; aligned fp32 has always been passed on.
+// too far apart for 32-bit offsets within a head -- by the bound of the statistics launch, the tighter one -- are copied by the
+// general path; aligned fp32 has always been passed on.
 bool direct_noise(const View& n) {
     if (!(n.half() || n.f32()) || !n.unit() || n.dim < 3) return false;
     bool aligned = n.f32() && reinterpret_cast<uintptr_t>(n.p) % 16 == 0;
     for (int i = 0; i < n.dim - 1; ++i) aligned = aligned && n.st[i] % 4 == 0;
-    return aligned || (n.st[n.dim - 2] >= n.s[n.dim - 1] && n.s[n.dim - 2] * n.st[n.dim - 2] * 4 + 1024 <= 0x7fffffffLL);
+    return aligned || (n.st[n.dim - 2] >= n.s[n.dim - 1] && (n.s[n.dim - 2] + TRN_STATS_SPARE_ROWS) * n.st[n.dim - 2] * 4 <= 0x7fffffffLL);
 }
 
 // the statistics tensors the kernels can write themselves

@@ -139,10 +139,10 @@ def _noise_aligned(n4: torch.Tensor) -> bool:
 def _noise_operand(mod: "FusedModule", n4: torch.Tensor) -> torch.Tensor:
     """The noise as the kernels read it: fp32 or fp16 rows of unit innermost stride at any pitch (the reference's noise is
     fp16 with an arbitrary key count, convert_eval_rms.py:201) that do not overlap and that 32-bit byte offsets within a
-    head reach.  Anything else is copied into an fp32 workspace."""
+    head reach, 128 rows past the last included (TRN_STATS_SPARE_ROWS).  Anything else is copied into an fp32 workspace."""
     pitch = n4.stride(2)
     if _noise_aligned(n4) or (n4.dtype in (torch.float32, torch.float16) and n4.stride(3) == 1 and pitch >= n4.shape[3]
-                              and n4.shape[2] * pitch * 4 + 1024 <= 0x7fffffff):
+                              and (n4.shape[2] + 128) * pitch * 4 <= 0x7fffffff):
         return n4
     buf = mod._workspace("noise32", tuple(n4.shape), torch.float32, n4.device)
     buf.copy_(n4)
