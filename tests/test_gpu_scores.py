@@ -425,3 +425,32 @@ def test_key_sums_and_squares_by_one_or_two_groups_of_waves(Sq, Skv, causal, B, 
     p = torch.exp(s - rows.double().unsqueeze(-1))
     for got, want in ((s1, p.sum(2)), (s2, p.square().sum(2))):
         assert ((got.double() - want).abs() <= 2e-5 * want + 1e-12).all(), ((got.double() - want).abs() / want).max()
+
+
+# ---- the furthest rows that the statistics kernels can address: their requests past the last query still read zeros
+@pytest.mark.gpu
+@pytest.mark.parametrize("Sq", [1, 64, 200, 321, 385])
+@pytest.mark.parametrize("noise", [None, "fp16", "fp32"])
+def test_statistics_at_the_largest_row_pitch(Sq, noise):
+    """Query and noise rows as far apart as TRN_STATS_SPARE_ROWS = 128 allows, walks of one and of two groups of waves with
+    short last tiles: the bits of compact tensors."""
+    from triton_amd import ops
+    D, Skv = 64, 130
+
+    def apart(t, elem_bytes):
+        pitch = 0x7fffffff // ((Sq + 128) * elem_bytes) // 8 * 8
+        w = torch.empty((Sq - 1) * pitch + t.shape[-1], dtype=t.dtype, device="cuda").as_strided(t.shape, (0, 0, pitch, 1))
+        return w.copy_(t)
+    q, k, v = (t.cuda() for t in make(1, 1, 1, Sq, Skv, D, seed=51))
+    n = None if noise is None else torch.randn(1, 1, Sq, Skv, device="cuda").to(torch.float16 if noise == "fp16" else torch.float32)
+    got = []
+    for wide in (False, True):
+        qw, nw = (apart(q, 2), None if n is None else apart(n, 4)) if wide else (q, n)
+        o, rows, s1, s2 = torch.zeros_like(q), torch.zeros(1, 1, Sq, device="cuda"), *(torch.zeros(1, 1, Skv, device="cuda") for _ in range(2))
+        if Sq > 32:
+            ops.attention_key_scores(qw, k, v, o, 0.125, False, rows, s1, s2, noise=nw, tau=1.0)
+        elif noise != "fp16":            # (the single launch of a few queries has its own sweep: the statistics alone here)
+            ops.attention_colstats(qw, k, rows, 0.125, False, s1, s2, noise=nw if n is None or wide else torch.nn.functional.pad(n, (0, 2))[..., :Skv])
+        torch.cuda.synchronize()
+        got.append((o, rows, s1, s2))
+    assert all(torch.equal(a, b) for a, b in zip(*got))

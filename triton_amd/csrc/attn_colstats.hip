@@ -143,7 +143,10 @@ __global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArg
     const int st_chunk = (lane % CPR) ^ swz<D>(st_row);
     const int qvo = (int)(st_row * a.qs * 2) + st_chunk * 16;
     const int qrow_bytes = (int)(RPI * a.qs * 2), qtile_bytes = (int)(CBM * a.qs * 2);
-#define TRN_FETCH_Q(t_, dst_) fetch_tile<NI, D, 4>(qrs, &dst_[grp * CBM * D + wave * RPI * D], qvo, (t_) * qtile_bytes, qrow_bytes)
+    // Requests past the last tile are for the one behind it, whose rows read as zeros: no offset lies further out than
+    // TRN_STATS_SPARE_ROWS (64 rows to the end of the last tile at most, and 64 of this one).
+    const int t_end = (a.Sq + CBM - 1) / CBM;
+#define TRN_FETCH_Q(t_, dst_) fetch_tile<NI, D, 4>(qrs, &dst_[grp * CBM * D + wave * RPI * D], qvo, min(t_, t_end) * qtile_bytes, qrow_bytes)
     int qoff[NKS];       // B-operand read: row c (+32 for the second block), logical chunk 2*ks + h
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) qoff[ks] = c * D + (((2 * ks + h) ^ swz<D>(c)) << 3);
@@ -178,7 +181,8 @@ __global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArg
     // wave) are in flight at any time.
     struct Pre { float lse[2]; noise_t g[2][4]; };
     Pre pa, pb;
-    auto prefetch = [&](int t, int qb, Pre& p) __attribute__((always_inline)) {
+    auto prefetch = [&](int tile, int qb, Pre& p) __attribute__((always_inline)) {
+        const int t = min(tile, t_end);
         p.lse[qb] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(lrs, c * 4, (t * CBM + qb * 32) * 4, 0));
         const int so = (int)((t * CBM + qb * 32) * a.ns * nsz);
 #pragma unroll
@@ -190,7 +194,7 @@ __global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArg
 
     const int first_q = a.causal ? max(0, kv0 - off) : 0;   // earlier queries see none of this tile's keys
     // this group's first tile, and a common end: a group whose last tile lies past the queries masks it away
-    const int t0 = first_q / CBM + grp, nt = NG == 1 ? (a.Sq + CBM - 1) / CBM : first_q / CBM + ((a.Sq + CBM - 1) / CBM - first_q / CBM + 1) / 2 * 2 + grp;
+    const int t0 = first_q / CBM + grp, nt = NG == 1 ? t_end : first_q / CBM + (t_end - first_q / CBM + 1) / 2 * 2 + grp;
 
     // The VALU part of a 32-query block.  Masked and plain blocks are separate loops (one wave-uniform branch
     // per block) so that the plain one is 4 instructions per score: fma, exp2, add, fma.
@@ -377,16 +381,17 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
     const int st_chunk = (lane % CPR) ^ swz<D>(st_row);
     const int qvo = (int)(st_row * a.qs * 2) + st_chunk * 16;
     const int qrow_bytes = (int)(RPI * a.qs * 2), qtile_bytes = (int)(CBM * a.qs * 2);
-#define TRN_FETCH_QL(t_, qd_, ld_)                                                                            \
+    const int nt = (a.Sq + CBM - 1) / CBM;
+#define TRN_FETCH_QL(t_, qd_, ld_)      /* (past the last tile: the one behind it, as above) */                \
     do {                                                                                                      \
-        fetch_tile<NI, D, 4>(qrs, &qd_[wave * RPI * D], qvo, (t_) * qtile_bytes, qrow_bytes);                 \
+        const int tt_ = min(t_, nt);                                                                          \
+        fetch_tile<NI, D, 4>(qrs, &qd_[wave * RPI * D], qvo, tt_ * qtile_bytes, qrow_bytes);                  \
         __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                             \
-            lrs, (__attribute__((address_space(3))) void*)(&ld_[wave * CBM]), 4, lane * 4, (t_) * CBM * 4, 0, 0); \
+            lrs, (__attribute__((address_space(3))) void*)(&ld_[wave * CBM]), 4, lane * 4, tt_ * CBM * 4, 0, 0); \
     } while (0)
     int qoff[NKS];       // B-operand read: row c (+32 for the second block), logical chunk 2*ks + h
 #pragma unroll
     for (int ks = 0; ks < NKS; ++ks) qoff[ks] = c * D + (((2 * ks + h) ^ swz<D>(c)) << 3);
-    const int nt = (a.Sq + CBM - 1) / CBM;
 
     // (a loop of one turn whose end the compiler cannot see: as straight-line code the walk's running sums and operands take
     // 20 to 35 registers more, past what two waves per SIMD have)
@@ -589,7 +594,7 @@ int trn::attn_colstats_check(const trn_attn_desc* d, const void* q, const void* 
             return TRN_E_ALIGN;
     }
     // Q tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base (with room for the tile requested
-    // past the end, which must stay representable to read as zeros)
+    // past the end, which must stay representable to read as zeros: the kernels ask for no later one)
     if (((int64_t)d->seq_q + TRN_STATS_SPARE_ROWS) * d->q_stride_s * 2 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
     if (((int64_t)d->seq_kv + CBN - 1) / CBN * d->batch * d->n_q_heads > 0x7fffffffLL) return TRN_E_SHAPE;
     return TRN_OK;
