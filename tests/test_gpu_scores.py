@@ -454,3 +454,29 @@ def test_statistics_at_the_largest_row_pitch(Sq, noise):
         torch.cuda.synchronize()
         got.append((o, rows, s1, s2))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+# ---- a row whose first keys carry a mask: the first reference of the perturbed scores lies far below zero
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hq,Hkv,D,Sq", [(2, 1, 128, 100), (32, 8, 128, 600), (32, 8, 64, 600)])      # 32-query tiles, prefill kernel
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("first,low", [(40, -200.0), (32, -65504.0), (110, -65504.0)])
+def test_noise_that_masks_the_first_keys(Hq, Hkv, D, Sq, dtype, first, low):
+    """Keys [0, first) of every row at `low`, under the causal mask: rows before `first` see nothing else.  Scores next to a
+    reference of the size of `low` carry its rounding, 2^-24 * |low| / ln 2 of an exponent: 0.4 % for -65504, in the block that a
+    row leaves the mask in and, twice, throughout the rows that see nothing else.  Beyond that the 1e-3 of the tests above (2e-3
+    for the normalisers)."""
+    from triton_amd import ops
+    q, k, v = (t.cuda() for t in make(1, Hq, Hkv, Sq, Sq, D, seed=61))
+    n = torch.randn(1, Hq, Sq, Sq, generator=torch.Generator(device="cuda").manual_seed(7), device="cuda").to(dtype)
+    n[..., :first] = low
+    o, rows, score = torch.zeros_like(q), torch.zeros(1, Hq, Sq, device="cuda"), torch.zeros(1, Hq, Sq, device="cuda")
+    ops.attention_key_scores(q, k, v, o, D ** -0.5, True, rows, score, noise=n, tau=1.0)
+    torch.cuda.synchronize()
+    s = q[0].double() @ k[0].double().repeat_interleave(Hq // Hkv, 0).transpose(-1, -2).contiguous() * D ** -0.5 + n[0].double()
+    s = s.masked_fill(~torch.ones(Sq, Sq, dtype=torch.bool, device="cuda").tril(), float("-inf"))
+    lse, p = torch.logsumexp(s, -1), s.softmax(-1).sum(1)
+    spoilt = 2 ** -24 * -low / 0.6931
+    assert ((rows[0].double() - lse).abs() <= 2e-3 + spoilt + 2 ** -23 * lse.abs()).all()
+    assert ((score[0].double() - p).abs()[:, first:] <= (1e-3 + spoilt) * p[:, first:] + 1e-9).all()
+    assert ((score[0].double() - p).abs()[:, :first] <= (1e-3 + 2 * spoilt) * p[:, :first]).all()

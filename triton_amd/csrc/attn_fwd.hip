@@ -195,7 +195,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 const bool seen = dmax > -INFINITY;            // a block can be entirely masked for this row pair
                 const bool raise = dmax > 8.0f || (!have2 && seen);
                 const float shift = raise ? dmax : 0.f;
-                l2 *= fast_exp2(-shift);
+                l2 = have2 ? l2 * fast_exp2(-shift) : 0.f;     // (a first reference below -128 would make the power infinite)
                 m2 += shift;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) d[r] -= shift;
@@ -318,7 +318,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 const float dmax = half_max(down);
                 const bool seen = dmax > -INFINITY, raise = dmax > 8.0f || (!have2 && seen);
                 const float shift = raise ? dmax : 0.f;
-                l2 *= fast_exp2(-shift);
+                l2 = have2 ? l2 * fast_exp2(-shift) : 0.f;     // (as in reduce_block)
                 m2 += shift;
                 have2 = have2 || seen;
                 sum = 0.f;
