@@ -132,21 +132,26 @@ bool same_shape(const View& a, const View& b) {
 
 // ---------------------------------------------------------------------------------------------- workspaces
 // A module's workspaces by name, shape, type and device: found here under the interpreter lock, allocated -- on the first
-// call that asks for one -- and owned by the module through `alloc(name, shape, dtype, device index, zeroed)`.
+// call that asks for one -- and owned by the module through `alloc(name, shape, dtype, device index, zeroed, optional)`, which
+// refuses to under a graph capture, or for an optional one returns None: an undefined tensor here.
 struct Entry { std::string name; std::vector<int64_t> shape; c10::ScalarType dt; int dev; at::Tensor t; };
 struct Workspaces { PyObject_HEAD std::vector<Entry>* e; PyObject* alloc; };
 
-const at::Tensor& workspace(Workspaces* w, const char* name, at::IntArrayRef shape, c10::ScalarType dt, int dev, bool zeroed = false) {
+at::Tensor workspace(Workspaces* w, const char* name, at::IntArrayRef shape, c10::ScalarType dt, int dev, bool zeroed = false, bool optional = false) {
     for (const Entry& e : *w->e)
         if (e.dt == dt && e.dev == dev && at::IntArrayRef(e.shape) == shape && e.name == name) return e.t;
     PyObject* sh = PyTuple_New((Py_ssize_t)shape.size());
     if (!sh) throw PyErrSet{};
     for (size_t i = 0; i < shape.size(); ++i) PyTuple_SET_ITEM(sh, (Py_ssize_t)i, PyLong_FromLongLong(shape[i]));
-    PyObject* t = PyObject_CallFunction(w->alloc, "sNsii", name, sh, c10::toString(dt), dev, (int)zeroed);
+    PyObject* t = PyObject_CallFunction(w->alloc, "sNsiii", name, sh, c10::toString(dt), dev, (int)zeroed, (int)optional);
     if (!t) throw PyErrSet{};
-    w->e->push_back(Entry{name, shape.vec(), dt, dev, THPVariable_Unpack(t)});
+    at::Tensor r;
+    if (t != Py_None) {
+        r = THPVariable_Unpack(t);
+        w->e->push_back(Entry{name, shape.vec(), dt, dev, r});
+    }
     Py_DECREF(t);
-    return w->e->back().t;
+    return r;
 }
 Workspaces* ws_arg(PyObject* o);
 
@@ -353,7 +358,7 @@ bool f_key_scores_forward(Args a, Py_ssize_t n) {         // workspaces, scale |
     if (noise.given && !direct_noise(noise.v)) return false;
     trn_attn_desc d = attn_desc(q, k, v, o, scale_of(a[1], q.s[3]), flag(a[2]));
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[3]));
-    const at::Tensor& rows = workspace(w, noise.given ? "lse_pert" : "lse", {q.s[0], q.s[1], q.s[2]}, c10::ScalarType::Float, q.dev);
+    const at::Tensor rows = workspace(w, noise.given ? "lse_pert" : "lse", {q.s[0], q.s[1], q.s[2]}, c10::ScalarType::Float, q.dev);
     CALL(trn_attn_key_scores_f16, &d, q.p, k.p, v.p, o.p, noise.p(), noise.given && noise.v.half(), static_cast<float*>(rows.data_ptr()),
          c1.p, c2.p(), c1.half(), flag(a[4]), nullptr, 0, stream_of(q));
     return true;
@@ -418,8 +423,11 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[7]));
     int64_t need = c1.given ? trn_attn_stats_workspace_bytes(&d) : trn_attn_workspace_bytes(&d);
     void* ws = need ? workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true).data_ptr() : nullptr;
-    if (!c1.given && !need && (need = trn_attn_chunk_workspace_bytes(&d)) > 0)
-        ws = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev).data_ptr();
+    if (!c1.given && !need && (need = trn_attn_chunk_workspace_bytes(&d)) > 0) {
+        const at::Tensor shares = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev, false, true);
+        ws = shares.defined() ? shares.data_ptr() : nullptr;      // (a cache that has grown long since the eager call: without)
+        if (!ws) need = 0;
+    }
     float* rows = c1.given ? static_cast<float*>(workspace(w, noise.given ? "lse_pert" : "lse", {1, H, M}, c10::ScalarType::Float, X.dev).data_ptr()) : nullptr;
     const View wts[3] = {wq, wk, wv};
     const View outs[3] = {q, make(Kc, Kc.p + 2 * P * Kc.st[1], {H, M, D}, {Kc.st[0], Kc.st[1], Kc.st[2]}),

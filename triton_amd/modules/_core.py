@@ -51,12 +51,15 @@ def _workspace_in(ws: Dict[Tuple, torch.Tensor], owner: str, name: str, shape, d
 _HOST_DTYPES = {"Half": torch.float16, "Float": torch.float32, "Byte": torch.uint8}
 
 
-def _workspace_for_host(ws, owner, name, shape, dtype, device_index, zeroed):
-    """The native side's first look-up of a workspace: the module's dictionary is where it lives."""
+def _workspace_for_host(ws, owner, name, shape, dtype, device_index, zeroed, optional):
+    """The native side's first look-up of a workspace: the module's dictionary is where it lives.  optional: None where a
+    graph capture forbids the allocation."""
     dt, dev = _HOST_DTYPES.get(dtype), torch.device("cuda", device_index)
     if dt is None:
         raise ValueError(f"expected float16 tensors, got {dtype}")
     fresh = (name, tuple(shape), dt, str(dev)) not in ws
+    if optional and fresh and torch.cuda.is_current_stream_capturing():
+        return None
     t = _workspace_in(ws, owner, name, shape, dt, dev)
     if zeroed and fresh:
         t.zero_()
