@@ -125,9 +125,12 @@ int trn_attn_fwd_f16(const trn_attn_desc* desc, const void* q, const void* k, co
  * A chunk of more than 32 queries per head on a long cache has a workspace of its own, trn_attn_chunk_workspace_bytes(desc)
  * bytes (0: none), which needs no initial contents: the keys are then shared out over workgroups whose partial results a
  * second launch merges.  (Its first 512 bytes, where the split decode shapes keep their counters, are left alone: one
- * zero-filled workspace of the larger size may serve both, one call at a time.)  Without it, or with a smaller one, the call is trn_attn_fwd_f16 as above.  No size depends on
- * seq_kv, so that a cache that grows from call to call keeps its workspace.
+ * zero-filled workspace of the larger size may serve both, one call at a time.)  Without it, or with a smaller one, the
+ * call is trn_attn_fwd_f16 as above.  The size does not depend on seq_kv, so that a cache that grows from call to call keeps
+ * its workspace, and never exceeds TRN_ATTN_CHUNK_WORKSPACE_MAX(head_dim) (256 shares of at most 128 queries): one workspace
+ * of that size serves chunks of every length.
  */
+#define TRN_ATTN_CHUNK_WORKSPACE_MAX(head_dim) (512 + (int64_t)256 * 128 * ((head_dim) + 2) * 4)
 int64_t trn_attn_workspace_bytes(const trn_attn_desc* desc);
 int64_t trn_attn_chunk_workspace_bytes(const trn_attn_desc* desc);
 int trn_attn_fwd_ws_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v,

@@ -192,6 +192,23 @@ def test_attention_split_rule_on_the_host(lib):
     assert need(8, 16, 4112) == 256 + 8 * 15 * 32 * 132 * 4
 
 
+def test_no_chunk_workspace_exceeds_the_size_for_all_of_them(lib):
+    """TRN_ATTN_CHUNK_WORKSPACE_MAX against trn_attn_chunk_workspace_bytes over heads and chunk lengths (host arithmetic)."""
+    import re
+    m = re.search(r"#define TRN_ATTN_CHUNK_WORKSPACE_MAX\(head_dim\) \((.*)\)", open(os.path.join(ROOT, "include", "trinity_hip.h")).read())
+    for D in (64, 128):
+        most = eval(m.group(1).replace("(int64_t)", "").replace("head_dim", str(D)))
+        seen = 0
+        for heads in (1, 2, 3, 5, 8, 16, 17, 32, 43, 64, 71, 85, 100, 127, 128, 129):
+            for sq in sorted({33, 34, 64, 100, 127, 128, 129, 250, 256, 257, 300, 511, 512, 513, 1000, 1024, 4000, 4096, 8191, 16384}):
+                skv = max(sq, 65536)
+                d = _desc(batch=1, n_q_heads=heads, n_kv_heads=1, seq_q=sq, seq_kv=skv, head_dim=D, causal=0, q_stride_b=heads * sq * D,
+                          q_stride_h=sq * D, q_stride_s=D, k_stride_b=skv * D, k_stride_h=skv * D, k_stride_s=D, v_stride_b=skv * D,
+                          v_stride_h=skv * D, v_stride_s=D, o_stride_b=heads * sq * D, o_stride_h=sq * D, o_stride_s=D)
+                seen = max(seen, lib.trn_attn_chunk_workspace_bytes(C.byref(d)))
+        assert seen == most, (D, seen, most)
+
+
 def test_statistics_split_rule_on_the_host(lib):
     """trn_attn_stats_workspace_bytes: the long-cache rule (few heads, many keys, at most 32 queries per head) is host
     arithmetic; where it says split, the size is that of the attention's own split workspace."""

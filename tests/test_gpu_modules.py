@@ -350,3 +350,19 @@ def test_a_chunk_on_a_cache_grown_since_the_eager_call_is_captured():
     mod.forward(*args)                        # eagerly, the workspace is made
     torch.cuda.synchronize()
     assert torch.equal(o2, want)
+
+
+def test_chunks_of_every_length_share_one_workspace():
+    from triton_amd import modules
+    g = torch.Generator(device="cuda").manual_seed(10)
+    H, D, keys = 8, 64, 4200
+    N = H * D
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda").half()
+    mod, K, V = modules.get("vanilla", "decode", head_dim=D, scale=0.125), r(H, keys, D), r(H, keys, D)
+    W = [0.04 * r(N, N) for _ in range(3)]
+    for M in (33, 40, 100, 128, 129, 400, 64):
+        X, o2 = r(M, N), torch.zeros(M, N, dtype=torch.float16, device="cuda")
+        mod.forward(K, o2, V, W[0], W[1], W[2], X)
+    torch.cuda.synchronize()
+    held = [t for key, t in mod._ws.items() if key[0] == "attn_shares"]
+    assert len(held) == 1 and held[0].numel() < 9 << 20

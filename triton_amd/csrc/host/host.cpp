@@ -15,6 +15,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/core/Tensor.h>
 #include <c10/hip/HIPStream.h>
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <string>
@@ -424,6 +425,8 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     int64_t need = c1.given ? trn_attn_stats_workspace_bytes(&d) : trn_attn_workspace_bytes(&d);
     void* ws = need ? workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true).data_ptr() : nullptr;
     if (!c1.given && !need && (need = trn_attn_chunk_workspace_bytes(&d)) > 0) {
+        // one for chunks of every length: by exact size each length would keep its own
+        need = std::max<int64_t>(need, TRN_ATTN_CHUNK_WORKSPACE_MAX(D));
         const at::Tensor shares = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev, false, true);
         ws = shares.defined() ? shares.data_ptr() : nullptr;      // (a cache that has grown long since the eager call: without)
         if (!ws) need = 0;
