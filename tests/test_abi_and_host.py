@@ -195,9 +195,11 @@ def test_attention_split_rule_on_the_host(lib):
 def test_no_chunk_workspace_exceeds_the_size_for_all_of_them(lib):
     """TRN_ATTN_CHUNK_WORKSPACE_MAX against trn_attn_chunk_workspace_bytes over heads and chunk lengths (host arithmetic)."""
     import re
+    from triton_amd import ops
     m = re.search(r"#define TRN_ATTN_CHUNK_WORKSPACE_MAX\(head_dim\) \((.*)\)", open(os.path.join(ROOT, "include", "trinity_hip.h")).read())
     for D in (64, 128):
         most = eval(m.group(1).replace("(int64_t)", "").replace("head_dim", str(D)))
+        assert ops.chunk_workspace_max(D) == most
         seen = 0
         for heads in (1, 2, 3, 5, 8, 16, 17, 32, 43, 64, 71, 85, 100, 127, 128, 129):
             for sq in sorted({33, 34, 64, 100, 127, 128, 129, 250, 256, 257, 300, 511, 512, 513, 1000, 1024, 4000, 4096, 8191, 16384}):

@@ -366,3 +366,38 @@ def test_chunks_of_every_length_share_one_workspace():
     torch.cuda.synchronize()
     held = [t for key, t in mod._ws.items() if key[0] == "attn_shares"]
     assert len(held) == 1 and held[0].numel() < 9 << 20
+
+
+@pytest.mark.parametrize("variant", ["vanilla", "prenorm", "qknorm"])
+@pytest.mark.parametrize("layout", ["token_major", "head_major"])
+@pytest.mark.parametrize("causal", [False, True])
+def test_a_chunk_on_a_long_cache(variant, layout, causal):
+    """More than 32 new tokens with their keys shared out over workgroups: the native forward and the general path (which takes
+    the three-axis output) bit for bit, and both against float64 softmax over the module's own projections.  Tolerance as for
+    the kernels: 4e-3 + 1e-3 of the value (one rounding each of Q after the scale, of the probabilities and of the result)."""
+    from triton_amd import modules
+    g = torch.Generator(device="cuda").manual_seed(11)
+    H, D, M, P = 4, 64, 100, 4050
+    N, PM = H * D, P + M
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g, device="cuda") * std).half()
+    t = dict(X=r(M, N), WQ=r(N, N, std=N ** -0.5), WK=r(N, N, std=N ** -0.5), WV=r(N, N, std=N ** -0.5), K_cache=r(H, PM, D),
+             V_cache=r(H, PM, D), O2=torch.zeros(M, N, dtype=torch.float16, device="cuda"))
+    mod = modules.get(variant, "decode", head_dim=D, scale=D ** -0.5, causal=causal, o_layout=layout)
+    u = {n: x.clone() for n, x in t.items()}
+    u["O2"] = u["O2"].view(M, H, D) if layout == "token_major" else u["O2"].view(H, M, D)
+    mod.forward(*[t[p] for p in mod.TENSOR_PARAMS])
+    assert any(key[0] == "attn_shares" for key in mod._ws)
+    mod._ws[next(key for key in mod._ws if key[0] == "attn_shares")].fill_(0xFF)
+    mod.forward(*[u[p] for p in mod.TENSOR_PARAMS])                # (declined by the native side)
+    torch.cuda.synchronize()
+    assert all(torch.equal(t[n], u[n].view(t[n].shape)) for n in t)
+    assert sum(key[0] == "attn_shares" for key in mod._ws) == 1
+    q = next(x for key, x in mod._ws.items() if key[0] == "q").double()
+    if variant == "qknorm":
+        q = q * torch.rsqrt(q.square().mean(-1, keepdim=True))
+    s = q @ t["K_cache"].double().transpose(-1, -2).contiguous() * D ** -0.5
+    if causal:
+        s = s.masked_fill(~torch.ones(M, PM, dtype=torch.bool, device="cuda").tril(P), float("-inf"))
+    want = s.softmax(-1) @ t["V_cache"].double()
+    got = t["O2"].view(M, H, D).permute(1, 0, 2) if layout == "token_major" else t["O2"].view(H, M, D)
+    assert ((got.double() - want).abs() <= 4e-3 + 1e-3 * want.abs()).all()

@@ -35,6 +35,11 @@ import torch
 from .. import _lib, ops
 
 
+def _capture_forbids(ws, name: str, shape, dtype, device) -> bool:
+    """Whether a workspace is missing that a graph capture in progress keeps from being allocated."""
+    return (name, tuple(shape), dtype, str(device)) not in ws and torch.cuda.is_current_stream_capturing()
+
+
 def _workspace_in(ws: Dict[Tuple, torch.Tensor], owner: str, name: str, shape, dtype, device) -> torch.Tensor:
     key = (name, tuple(shape), dtype, str(device))
     t = ws.get(key)
@@ -57,9 +62,9 @@ def _workspace_for_host(ws, owner, name, shape, dtype, device_index, zeroed, opt
     dt, dev = _HOST_DTYPES.get(dtype), torch.device("cuda", device_index)
     if dt is None:
         raise ValueError(f"expected float16 tensors, got {dtype}")
-    fresh = (name, tuple(shape), dt, str(dev)) not in ws
-    if optional and fresh and torch.cuda.is_current_stream_capturing():
+    if optional and _capture_forbids(ws, name, shape, dt, dev):
         return None
+    fresh = (name, tuple(shape), dt, str(dev)) not in ws
     t = _workspace_in(ws, owner, name, shape, dt, dev)
     if zeroed and fresh:
         t.zero_()
@@ -358,12 +363,23 @@ class _DecodeAppend(FusedModule):
 
     def _attend(self, q, K_cache, V_cache, O2, **kw):
         """Attention of the M new queries over the whole cache, with a workspace (allocated and zeroed once per shape;
-        every call leaves its counters at zero again) so that the keys of a head can be split over several workgroups."""
+        every call leaves its counters at zero again) so that the keys of a head can be split over several workgroups, or
+        those of a chunk of more than 32 queries shared out over them."""
         H, M, D = q.shape
         o = self._o_view(O2, H, M, D)
-        nbytes = ops.attention_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
-        ops.attention(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal,
-                      workspace=self._split_ws(nbytes, q.device), **kw)
+        problem = (q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
+        ws = self._split_ws(ops.attention_workspace_bytes(*problem), q.device)
+        if ws is None:
+            ws = self._chunk_ws(ops.attention_chunk_workspace_bytes(*problem), D, q.device)
+        ops.attention(*problem, workspace=ws, **kw)
+
+    def _chunk_ws(self, nbytes: int, head_dim: int, device):
+        """The workspace of the shared-out keys: one for chunks of every length (by exact size each length would keep its
+        own); None when the library would not use one, or a capture finds it missing."""
+        if not nbytes:
+            return None
+        key = ("attn_shares", (max(nbytes, ops.chunk_workspace_max(head_dim)),), torch.uint8, device)
+        return None if _capture_forbids(self._ws, *key) else self._workspace(*key)
 
     def _split_ws(self, nbytes: int, device):
         """The split-key workspace (zeroed once, on the cold call that allocates it; the kernels leave its counters at

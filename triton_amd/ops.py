@@ -155,6 +155,18 @@ def attention_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> int:
     return int(_lib.load().trn_attn_workspace_bytes(C.byref(d)))
 
 
+def attention_chunk_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> int:
+    """Bytes of workspace (no initial contents) with which `attention` would share out the keys of a chunk of more than 32
+    queries over workgroups (0: it would not).  chunk_workspace_max(head_dim) bytes serve chunks of every length."""
+    d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, None, 1.0)
+    return int(_lib.load().trn_attn_chunk_workspace_bytes(C.byref(d)))
+
+
+def chunk_workspace_max(head_dim: int) -> int:
+    """TRN_ATTN_CHUNK_WORKSPACE_MAX of include/trinity_hip.h."""
+    return 512 + 256 * 128 * (head_dim + 2) * 4
+
+
 def attention_stats_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> int:
     """Bytes of workspace with which `attention_with_stats` would split the keys of this problem over several
     workgroups and run the statistics as a second launch (0: it would not -- one launch is faster)."""
