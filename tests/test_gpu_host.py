@@ -162,3 +162,43 @@ def test_noise_that_the_statistics_refuse_leaves_the_outputs_alone():
         ops.attention_key_scores(q, q, q, o, 1.0, False, rows, score, noise=noise)
     torch.cuda.synchronize()
     assert all(bool((t == 7).all()) for t in (o, rows, score))
+
+
+def test_other_threads_run_while_a_launch_waits(tmp_path):
+    """A forward gives up the interpreter lock for its calls into the library, as a ctypes call does.  In a process of its own,
+    with the RMSNorm entry point replaced by one that only sleeps, another thread goes on counting meanwhile."""
+    import os
+    import subprocess
+    import sys
+    (tmp_path / "slow.c").write_text("#include <unistd.h>\nint trn_rmsnorm_f16(void) { usleep(400000); return 0; }\n")
+    slow = str(tmp_path / "slow.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "slow.c"), "-o", slow], check=True)
+    child = f"""
+import ctypes, threading, time
+ctypes.CDLL({slow!r}, mode=ctypes.RTLD_GLOBAL)
+import torch
+from triton_amd import modules
+x = torch.zeros(4, 64, dtype=torch.float16, device="cuda")
+mod = modules.get("rms")
+mod.forward(x, x.clone(), x[0])
+y, n, end = x.clone(), 0, False
+def count():
+    global n
+    while not end:
+        n += 1
+        time.sleep(0.002)
+t = threading.Thread(target=count)
+t.start()
+time.sleep(0.05)
+before, start = n, time.perf_counter()
+mod.forward(x, y, x[0])
+counted, took = n - before, time.perf_counter() - start
+end = True
+t.join()
+print("took", took, "counted", counted)
+assert took > 0.3, "the sleeping entry point was not called"
+assert counted > 20
+"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", child], cwd=root, capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr

@@ -19,6 +19,7 @@
 #include <cmath>
 #include <cstdarg>
 #include <string>
+#include <type_traits>
 #include <vector>
 #include "../../../include/trinity_hip.h"
 
@@ -40,7 +41,17 @@ std::string format(const char* f, ...) {
     return b;
 }
 #define NEED(cond, ...) do { if (__builtin_expect(!(cond), 0)) throw ValueErr{format(__VA_ARGS__)}; } while (0)
-#define CALL(fn, ...) do { const int st_ = fn(__VA_ARGS__); if (__builtin_expect(st_ != 0, 0)) throw TrnErr{#fn, st_}; } while (0)
+
+// A call into libtrinity_hip.so without the interpreter lock, as ctypes makes it: a launch waits while its queue is full, and
+// the process's other Python threads go on.  (The arguments are evaluated before, under the lock.)
+template <class... P>
+int unlocked(int (*fn)(P...), std::common_type_t<P>... args) {
+    PyThreadState* const state = PyEval_SaveThread();
+    const int status = fn(args...);
+    PyEval_RestoreThread(state);
+    return status;
+}
+#define CALL(fn, ...) do { const int st_ = unlocked(fn, __VA_ARGS__); if (__builtin_expect(st_ != 0, 0)) throw TrnErr{#fn, st_}; } while (0)
 
 // A tensor as the C ABI needs it.
 struct View {
@@ -134,7 +145,8 @@ bool same_shape(const View& a, const View& b) {
 // ---------------------------------------------------------------------------------------------- workspaces
 // A module's workspaces by name, shape, type and device: found here under the interpreter lock, allocated -- on the first
 // call that asks for one -- and owned by the module through `alloc(name, shape, dtype, device index, zeroed, optional)`, which
-// refuses to under a graph capture, or for an optional one returns None: an undefined tensor here.
+// refuses to under a graph capture, or for an optional one returns None: an undefined tensor here.  A forward holds the
+// tensors it was given until it returns: between its launches another thread may release the module's.
 struct Entry { std::string name; std::vector<int64_t> shape; c10::ScalarType dt; int dev; at::Tensor t; };
 struct Workspaces { PyObject_HEAD std::vector<Entry>* e; PyObject* alloc; };
 
@@ -319,7 +331,8 @@ bool f_qknorm_forward(Args a, Py_ssize_t n) {             // workspaces, scale |
     NEED(k.contiguous(), "K: expected a contiguous tensor");
     NEED(k.cuda, "K: expected a GPU tensor");
     const double eps = num(a[3]);
-    const View kn = view_of(workspace(w, "k_norm", {k.s[0], k.s[1], k.s[2], k.s[3]}, k.dt, k.dev), "k_norm");
+    const at::Tensor kn_ws = workspace(w, "k_norm", {k.s[0], k.s[1], k.s[2], k.s[3]}, k.dt, k.dev);
+    const View kn = view_of(kn_ws, "k_norm");
     trn_attn_desc d = attn_desc(q, kn, v, o, scale_of(a[1], k.s[3]), flag(a[2]));
     d.q_norm = 1; d.q_norm_eps = (float)eps;
     const OptView gq = opt(a[9], "gamma_q");
@@ -382,7 +395,8 @@ bool f_prenorm_forward(Args a, Py_ssize_t n) {            // workspaces, head_di
     const int64_t B = X.dim == 3 ? X.s[0] : 1, S = X.s[X.dim - 2], K = X.s[X.dim - 1], nq = wq.s[1], nkv = wk.s[1];
     if (D <= 0 || nq % D || nkv % D || O.numel() != B * S * nq) return false;
     const int64_t T = B * S, ld = nq + 2 * nkv;
-    const View qkv = view_of(workspace(w, "qkv", {T, ld}, X.dt, X.dev), "qkv");
+    const at::Tensor qkv_ws = workspace(w, "qkv", {T, ld}, X.dt, X.dev);
+    const View qkv = view_of(qkv_ws, "qkv");
     const View ws[3] = {wq, wk, wv};
     const int64_t off[3] = {0, nq, nq + nkv}, nn[3] = {nq, nkv, nkv};
     View hm[3], b4[3];
@@ -415,7 +429,8 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     if (O2.s[0] != M || O2.s[1] != N || (head_major && !O2.contiguous())) return false;
     if (c1.given && !direct_outputs(c1.v, c2.given ? &c2.v : nullptr, H * PM)) return false;
     if (noise.given && !(noise.v.dim == 3 && direct_noise(noise.v))) return false;
-    const View q = view_of(workspace(w, "q", {H, M, D}, X.dt, X.dev), "q");
+    const at::Tensor q_ws = workspace(w, "q", {H, M, D}, X.dt, X.dev);
+    const View q = view_of(q_ws, "q");
     const View q4 = as4(q, "q"), k4 = as4(Kc, "K_cache"), v4 = as4(Vc, "V_cache");
     const View o4 = head_major ? make(O2, O2.p, {1, H, M, D}, {H * M * D, M * D, D, 1}) : make(O2, O2.p, {1, H, M, D}, {M * O2.st[0], D, O2.st[0], 1});
     NEED(O2.unit(), "O2: innermost stride must be 1");
@@ -423,15 +438,18 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     d.q_norm = q_norm ? 1 : 0;
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[7]));
     int64_t need = c1.given ? trn_attn_stats_workspace_bytes(&d) : trn_attn_workspace_bytes(&d);
-    void* ws = need ? workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true).data_ptr() : nullptr;
-    if (!c1.given && !need && (need = trn_attn_chunk_workspace_bytes(&d)) > 0) {
+    at::Tensor split;
+    if (need) split = workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true);
+    else if (!c1.given && (need = trn_attn_chunk_workspace_bytes(&d)) > 0) {
         // one for chunks of every length: by exact size each length would keep its own
         need = std::max<int64_t>(need, TRN_ATTN_CHUNK_WORKSPACE_MAX(D));
-        const at::Tensor shares = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev, false, true);
-        ws = shares.defined() ? shares.data_ptr() : nullptr;      // (a cache that has grown long since the eager call: without)
-        if (!ws) need = 0;
+        split = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev, false, true);
+        if (!split.defined()) need = 0;             // (captured, the cache grown long since the eager call: without)
     }
-    float* rows = c1.given ? static_cast<float*>(workspace(w, noise.given ? "lse_pert" : "lse", {1, H, M}, c10::ScalarType::Float, X.dev).data_ptr()) : nullptr;
+    void* const ws = need ? split.data_ptr() : nullptr;
+    at::Tensor rows_ws;
+    if (c1.given) rows_ws = workspace(w, noise.given ? "lse_pert" : "lse", {1, H, M}, c10::ScalarType::Float, X.dev);
+    float* const rows = c1.given ? static_cast<float*>(rows_ws.data_ptr()) : nullptr;
     const View wts[3] = {wq, wk, wv};
     const View outs[3] = {q, make(Kc, Kc.p + 2 * P * Kc.st[1], {H, M, D}, {Kc.st[0], Kc.st[1], Kc.st[2]}),
                           make(Vc, Vc.p + 2 * P * Vc.st[1], {H, M, D}, {Vc.st[0], Vc.st[1], Vc.st[2]})};
@@ -453,7 +471,8 @@ bool f_lora_forward(Args a, Py_ssize_t n) {               // workspaces, A, B, O
     const int64_t M = X.s[0], N = X.s[1], R = B.s[0], P = B.s[1];
     NEED(W.s[0] == N && W.s[1] == P && A.s[0] == N && A.s[1] == R && O.s[0] == M && O.s[1] == P,
          "inconsistent shapes: X %s, W %s, A %s, B %s, O %s", X.shape().c_str(), W.shape().c_str(), A.shape().c_str(), B.shape().c_str(), O.shape().c_str());
-    const View d = view_of(workspace(ws, "D", {M, R}, X.dt, X.dev), "D");
+    const at::Tensor d_ws = workspace(ws, "D", {M, R}, X.dt, X.dev);
+    const View d = view_of(d_ws, "D");
     const View w1[2] = {W, A}, o1[2] = {O, d};
     linear_call(X, 2, w1, o1, nullptr);
     linear_call(d, 1, &B, &O, &O);
@@ -467,7 +486,8 @@ bool f_gmlp_forward(Args a, Py_ssize_t n) {               // workspaces, silu, O
     if (O.dim != 2 || W1.dim != 2 || W2.dim != 2 || X.dim != 2 || !X.cuda) return false;
     NEED(W1.s[0] == X.s[1] && same_shape(W1, W2) && O.s[0] == X.s[0] && O.s[1] == W1.s[1], "inconsistent shapes: X %s, W1 %s, W2 %s, O %s",
          X.shape().c_str(), W1.shape().c_str(), W2.shape().c_str(), O.shape().c_str());
-    const View c2 = view_of(workspace(ws, "C2", {O.s[0], O.s[1]}, X.dt, X.dev), "C2");
+    const at::Tensor c2_ws = workspace(ws, "C2", {O.s[0], O.s[1]}, X.dt, X.dev);
+    const View c2 = view_of(c2_ws, "C2");
     const View w[2] = {W1, W2}, o[2] = {O, c2};
     linear_call(X, 2, w, o, nullptr);                     // the first product lands in O and is gated in place
     CALL(trn_gate_f16, O.p, c2.p, O.p, O.s[0], O.s[1], O.st[0], c2.st[0], O.st[0], flag(a[1]) ? 1 : 0, stream_of(X));
