@@ -270,6 +270,30 @@ def test_module_protocol_host_logic():
     assert modules.get("roco", stats="mean_std").TENSOR_PARAMS == modules.get("roco").TENSOR_PARAMS
 
 
+def test_two_threads_may_make_the_first_forward_of_a_module(monkeypatch):
+    """A forward that runs while another is still making the native view of the workspaces makes or finds one itself."""
+    import threading
+    from triton_amd import _lib, modules
+    mod, given = modules.get("vanilla"), []
+
+    class Host:
+        entered = 0
+
+        def Workspaces(self, alloc):
+            Host.entered += 1
+            if Host.entered == 1:          # the first thread is held up here: a second one comes by
+                t = threading.Thread(target=mod.forward, args=(None,) * 4)
+                t.start()
+                t.join()
+            return f"view {Host.entered}"
+
+    monkeypatch.setattr(_lib, "host", lambda: Host.shared)
+    Host.shared = Host()
+    monkeypatch.setattr(type(mod), "_native", lambda self, host, ws, *t: given.append((host, ws)) or True)
+    mod.forward(*(None,) * 4)
+    assert len(given) == 2 and all(host is Host.shared and ws is not None for host, ws in given)
+
+
 def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run(["python", os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0 and "one GPU" in r.stderr

@@ -109,10 +109,12 @@ class FusedModule:
                 raise TypeError(f"forward got an unexpected keyword argument '{k}'")
         if len(args) > n:
             args = args[:n]                                # trailing positionals are block sizes: ignored
-        if self._host is None:
-            self._host = _lib.host()
-            self._hws = self._host.Workspaces(functools.partial(_workspace_for_host, self._ws, type(self).__name__))
-        if not self._native(self._host, self._hws, *args):
+        host = self._host
+        if host is None:
+            host = _lib.host()
+            self._hws = host.Workspaces(functools.partial(_workspace_for_host, self._ws, type(self).__name__))
+            self._host = host               # (last: another thread's forward takes it as the sign that both are there)
+        if not self._native(host, self._hws, *args):
             self._run(*args)
 
     __call__ = forward
