@@ -270,6 +270,19 @@ def test_module_protocol_host_logic():
     assert modules.get("roco", stats="mean_std").TENSOR_PARAMS == modules.get("roco").TENSOR_PARAMS
 
 
+def test_a_module_pickled_without_a_native_side_still_runs():
+    """The state of a module from before it had one: constructor arguments and workspaces only."""
+    import pickle
+    from triton_amd import modules
+    mod = modules.get("vanilla")
+    old = type(mod).__new__(type(mod))
+    old.__dict__.update(_ws={}, scale=None, causal=True)
+    q = torch.zeros(1, 2, 8, 64, dtype=torch.float16)
+    for m in (old, pickle.loads(pickle.dumps(old)), pickle.loads(pickle.dumps(mod))):
+        with pytest.raises(ValueError, match="GPU tensor"):
+            m.forward(q, q, q, q)
+
+
 def test_two_threads_may_make_the_first_forward_of_a_module(monkeypatch):
     """A forward that runs while another is still making the native view of the workspaces makes or finds one itself."""
     import threading

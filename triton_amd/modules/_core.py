@@ -83,13 +83,16 @@ class FusedModule:
     TENSOR_PARAMS: List[str] = []
     BLOCK_PARAMS: List[str] = []
 
+    # the native side, loaded with the first forward, and its view of these workspaces (here, not in __init__: a module pickled
+    # before there was one has neither)
+    _host = None
+    _hws = None
+
     def __init__(self) -> None:
         self._ws: Dict[Tuple, torch.Tensor] = {}
-        self._host = None                   # (the native side, loaded with the first forward)
-        self._hws = None                    # its view of these workspaces
 
     def __getstate__(self):
-        return {**self.__dict__, "_host": None, "_hws": None}      # (a copy makes its own native view)
+        return {k: v for k, v in self.__dict__.items() if k not in ("_host", "_hws")}      # (a copy makes its own native view)
 
     def _workspace(self, name: str, shape, dtype, device) -> torch.Tensor:
         return _workspace_in(self._ws, type(self).__name__, name, shape, dtype, device)
