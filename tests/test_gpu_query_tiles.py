@@ -25,6 +25,10 @@ CASES = [
     (2, 16, 16, 230, 230, 64, True, False, True), (2, 16, 16, 260, 260, 64, False, False, False),
     (1, 71, 1, 100, 1024, 64, False, False, True), (1, 71, 1, 100, 1023, 64, False, False, False),   # 284 tiles, long keys or not
     (1, 32, 32, 100, 1500, 128, False, True, True), (1, 71, 71, 70, 333, 64, True, True, True),      # score perturbation
+    # a few heads, or a number that is no multiple of 8, with so many tiles that they are spread over the XCDs: 4, 2 and 1 column
+    # shares, numbers of tiles that are no multiple of 8, the number of workgroups from which on they are (33 of a head per XCD)
+    (1, 1, 1, 1100, 1100, 64, True, False, True), (1, 3, 1, 530, 530, 128, False, False, True), (1, 12, 4, 300, 300, 128, True, True, True),
+    (3, 3, 3, 800, 830, 64, True, False, True), (1, 1, 1, 512, 600, 64, False, False, True), (1, 1, 1, 513, 600, 64, False, True, True),
     (1, 32, 8, 480, 480, 128, True, True, True), (1, 32, 8, 500, 520, 128, True, True, False),       # 480 tiles and 512
 ]
 

@@ -15,6 +15,7 @@ struct AttnArgs {
     int causal, q_norm;
     // decode kernel only: keys split over n_split workgroups per head, partial results and arrival counters in ws
     int n_split;
+    int spread;    // decode kernel only: the query tiles of a head go to all XCDs
     float* ws;
     // decode kernel only, at most 32 queries: per-key sums (and sums of squares) of the probabilities -- of the
     // perturbed ones when noise is given -- from a second sweep over the keys once the row normalisers are final

@@ -62,12 +62,25 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // workgroup id -> (batch x head j, key share, column share).  The column shares of a head read the same K: their
     // ids are 8 apart, so that they sit on one XCD (ids are dealt to the 8 XCDs in turn) and share its L2.
-    // So do the query tiles of a head; the last one, with the most keys under a causal mask, comes first.
+    // So do the query tiles of a head, unless they are spread (decode_spread()); the last ones, with the most keys under a
+    // causal mask, come first.
     int j, split = 0, dsl = 0, q0 = 0;
-    if (DS > 1 || a.n_qtiles > 1) {
-        const int per_grp = 8 * DS * a.n_qtiles, grp = blockIdx.x / per_grp, rem = blockIdx.x % per_grp;
-        j = grp * 8 + rem % 8; dsl = rem / 8 % DS; q0 = 32 * (a.n_qtiles - 1 - rem / (8 * DS));
-        if (j >= a.B * a.Hq) return;                    // the last group of eight heads may be short
+    const int BH = a.B * a.Hq;
+    if (a.n_qtiles > 1) {
+        int qt;
+        if (a.spread) {
+            const int unit = (int)blockIdx.x / (8 * DS) * 8 + (int)blockIdx.x % 8;
+            j = unit % BH; qt = unit / BH; dsl = (int)blockIdx.x / 8 % DS;
+        } else {
+            const int per_grp = 8 * DS * a.n_qtiles, grp = (int)blockIdx.x / per_grp, rem = (int)blockIdx.x % per_grp;
+            j = grp * 8 + rem % 8; qt = rem / (8 * DS); dsl = rem / 8 % DS;
+        }
+        if (j >= BH || qt >= a.n_qtiles) return;        // the last eight heads, or eight tiles, may be fewer
+        q0 = 32 * (a.n_qtiles - 1 - qt);
+    } else if constexpr (DS > 1) {
+        const int grp = (int)blockIdx.x / (8 * DS), rem = (int)blockIdx.x % (8 * DS);
+        j = grp * 8 + rem % 8; dsl = rem / 8;
+        if (j >= BH) return;
     } else {
         j = blockIdx.x / a.n_split; split = blockIdx.x % a.n_split;
     }
@@ -580,6 +593,16 @@ bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head
     return tiles <= 256 || (tiles < 512 && (noise || (head_dim == 64 && seq_kv >= 1024)));
 }
 
+// Where the query tiles of a head go.  On one XCD they share K and V in its L2, but fewer than eight heads, or a number that
+// leaves the last eight short, then leave XCDs idle: from the point where the others have more than a workgroup per CU the
+// tiles are dealt to all eight instead.  us, together / spread: one head of 128, 845 queries and keys 30.0 / 9.3, 3213 132 /
+// 24, causal 4097 83 / 32; two of 64, causal 5219 68 / 24; four of 128, causal 1529 26.9 / 21.5; twelve of 64, causal 1132 with
+// noise 26.0 / 19.4; but four of 128, 35 queries on 9587 keys (8 workgroups per XCD) 62.0 / 66.3.
+static bool decode_spread(int64_t n_bh, int n_qtiles, int ds) {
+    const int64_t heads8 = (n_bh + 7) / 8;
+    return n_qtiles > 1 && heads8 * 64 > 9 * n_bh && heads8 * n_qtiles * ds > 32;
+}
+
 // Name of the instantiation launched for a problem without a workspace (a measurement aid: what a kernel trace shows).
 const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
     const int ds = decode_col_shares((int64_t)batch * n_q_heads * ((seq_q + 31) / 32), seq_q, seq_kv, head_dim);
@@ -605,7 +628,9 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
     a.n_qtiles = (a.Sq + 31) / 32;
     const int64_t n_bh = (int64_t)a.B * a.Hq;
     const int ds = a.n_split == 1 ? decode_col_shares(n_bh * a.n_qtiles, a.Sq, a.Skv, head_dim) : 1;
-    const int64_t grid = ds > 1 || a.n_qtiles > 1 ? ((n_bh + 7) / 8) * 8 * ds * a.n_qtiles : n_bh * a.n_split;
+    const int64_t heads8 = (n_bh + 7) / 8;
+    a.spread = decode_spread(n_bh, a.n_qtiles, ds) ? 1 : 0;
+    const int64_t grid = a.spread ? (n_bh * a.n_qtiles + 7) / 8 * 8 * ds : ds > 1 || a.n_qtiles > 1 ? heads8 * 8 * ds * a.n_qtiles : n_bh * a.n_split;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)grid), t(DNW * 64);
 #define TRN_DEC(D_, DS_, N_) hipLaunchKernelGGL((attn_decode_kernel<D_, DS_, N_>), g, t, 0, stream, a)
