@@ -19,8 +19,9 @@ def chunk_bytes(q, k, o, scale, causal):
     (1, 4, 2, 700, 4159, 64, True, False), (1, 71, 1, 100, 2600, 64, True, True), (1, 32, 32, 257, 3200, 128, True, False),
     (1, 1, 1, 2300, 4200, 64, True, False), (1, 2, 1, 3100, 3100, 128, True, False), (1, 64, 8, 40, 4097, 64, False, False)])
 def test_shared_out_keys(B, Hq, Hkv, Sq, Skv, D, causal, q_norm):
-    """fp16 results of N(0,1) inputs: 4e-2 of their root mean square covers the rounding of Q after the scale, of the
-    probabilities and of the result (1.1e-2 measured by the other attention tests' distances); row normalisers 2e-3."""
+    """Element by element 4e-3 + 1e-3 of the value, as the other attention kernels are held to on N(0,1) inputs (one fp16 rounding
+    each of the normalised Q, of the probabilities and of the result), so that late rows, whose results are averages over
+    thousands of keys and small, count like the first ones; row normalisers 2e-3."""
     from triton_amd import ops
     g = torch.Generator(device="cuda").manual_seed(3)
     q, k, v = (torch.randn(B, h, s, D, generator=g, device="cuda").half() for h, s in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
@@ -46,7 +47,7 @@ def test_shared_out_keys(B, Hq, Hkv, Sq, Skv, D, causal, q_norm):
                 s = s.masked_fill(~torch.ones(Sq, Skv, dtype=torch.bool, device="cuda").tril(Skv - Sq), float("-inf"))
             want = s.softmax(-1) @ v[b, h // (Hq // Hkv)].double()
             for got in (o, plain):
-                assert (got[b, h].double() - want).abs().max() <= 4e-2 * max(want.square().mean().sqrt(), want.abs().max()), (b, h)
+                assert ((got[b, h].double() - want).abs() <= 4e-3 + 1e-3 * want.abs()).all(), (b, h)
             assert (lse[b, h].double() - torch.logsumexp(s, -1)).abs().max() < 2e-3, (b, h)
 
 
