@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import concurrent.futures as cf
 import os
+import re
 import subprocess
 import sys
 import sysconfig
@@ -25,6 +26,10 @@ FLAGS = [
     "-Wno-unknown-warning-option", "-Wno-unused-command-line-argument",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+# What the compiler says of a kernel's registers, of which the build reports spills: several kernels here are shaped so that
+# their registers just fit, and nothing but the time would tell otherwise.
+RESOURCES = "-Rpass-analysis=kernel-resource-usage"
+_SOURCE_LINE = re.compile(r"\s*\d* \| ")
 
 
 def sources():
@@ -33,14 +38,24 @@ def sources():
 
 def _compile(src: str) -> str:
     obj = os.path.join(OBJ_DIR, os.path.basename(src)[:-4] + ".o")
-    cmd = [HIPCC, *FLAGS, "-c", src, "-o", obj]
+    cmd = [HIPCC, *FLAGS, RESOURCES, "-c", src, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stdout}\n{r.stderr}")
     noise = "packed-fp32-ops' is not a recognized feature"
-    err = "\n".join(l for l in r.stderr.splitlines() if l.strip() and noise not in l)
-    if err.strip():
-        sys.stderr.write(err + "\n")
+    kernel, skip = "", 0
+    for line in r.stderr.splitlines():
+        if f"[{RESOURCES}]" in line:                    # (two lines of source follow the first remark on a kernel)
+            key, _, value = line.split("remark:", 1)[1].split(" [-R")[0].partition(": ")
+            if key.strip() == "Function Name":
+                kernel = value
+            elif key.strip().startswith("ScratchSize") and int(value) > 0:
+                sys.stderr.write(f"{os.path.basename(src)}: {kernel} spills: {value} bytes of scratch per lane\n")
+            skip = 2
+        elif skip and _SOURCE_LINE.match(line):
+            skip -= 1
+        elif line.strip() and noise not in line:
+            sys.stderr.write(line + "\n")
     return obj
 
 
