@@ -281,7 +281,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         // reference as it stands; whether it had to be raised is known at the end, and the block's sum is then formed
         // again (rare after a row's first block).  In one piece behind the fourth MFMA, as reduce_block() has it, the two
         // waves of a SIMD left the matrix pipe idle for most of it: 32 heads of 128, 4096 keys, fp32 noise 333 -> 309 us,
-        // fp16 270 -> 251; 1501 keys, fp16 65 -> 51; 284 heads of 64, 392 keys 48 -> 37 (same bits).
+        // fp16 270 -> 251; 1501 keys, fp16 65 -> 51; 284 heads of 64, 392 keys 48 -> 37 (same bits; short bursts from an idle
+        // board, here and at noise_kernel_wide(): once its clocks have risen 4096 keys take 266).
         const float nref = -m2;
         float down = -INFINITY, top = -INFINITY, sum = 0.f;
         auto perturbed = [&](int r, float ref) __attribute__((always_inline)) {

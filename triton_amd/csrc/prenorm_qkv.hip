@@ -223,7 +223,7 @@ int launch_projections(GemmArgs a, hipStream_t stream) {
     if (prenorm_qkv_wide_tiles(a) >= 128) return launch_prenorm_qkv_wide(a, stream);
     // Below that, the smallest tile that still gives every CU at most one: a tile's time is its chain of k-tiles, nearly
     // the same for all of them up to one per CU, and half as much again or more with a second one beside it (4096 -> 6144,
-    // us 64 x 64 / 128 x 64 / 128 x 128: 100 tokens 25 / 33 / 46, 256 tokens 45 / 37 / 47, 512 tokens 65 / 62 / 48).  When
+    // us 64 x 64 / 128 x 64 / 128 x 128: 100 tokens 26 / 33 / 46, 256 tokens 45 / 37 / 47, 512 tokens 65 / 62 / 50).  When
     // even 128 x 128 tiles exceed the CUs, the kernel of this file takes them two per CU (768 tokens 76 against 87 us).
     if (prenorm_qkv_mid_tiles(a, 64, 64) <= 256) return launch_prenorm_qkv_mid(a, 64, 64, stream);
     if (prenorm_qkv_mid_tiles(a, 128, 64) <= 256) return launch_prenorm_qkv_mid(a, 128, 64, stream);

@@ -18,8 +18,8 @@
 // against 2.9e-4).  The sum of squares is taken from X as read, by the waves of the first column group.
 //
 // Measured, weights cold in HBM, us before (128 x 128 kernel) / now: 4096 -> 12288 without norm 33 tokens 63 / 26, 64
-// tokens 63 / 29, 100 tokens 70 / 35; 4096 -> 6144 with norm 100 tokens 73 / 25, 256 tokens 73 / 37, 512 tokens 73 / 48;
-// 1024 -> 3072 128 tokens 18 / 8.
+// tokens 63 / 29, 100 tokens 64 / 35; 4096 -> 6144 with norm and gamma 100 tokens 74 / 26, 256 tokens 74 / 37.5, 512 tokens
+// 74 / 50; 1024 -> 3072 128 tokens 18 / 8.
 #include "prenorm_qkv.h"
 
 namespace trn {
