@@ -27,10 +27,9 @@ namespace trn {
 
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer-descriptor types and LDS-load builtins exist in the device pass only;
                                       // the host pass needs just the launch stubs
-// NZ: 1 fp32 noise, 2 fp16 noise
-template <int D, int NW, int NZ>
+// N16: fp16 noise (fp32 otherwise)
+template <int D, int NW, bool N16>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
-    constexpr bool NOISE = NZ != 0, N16 = NZ == 2;
     constexpr int BN = 64;       // keys per LDS stage (two 32-key blocks)
     constexpr int NS = D / 16;   // MFMA slots per phase: k-steps of S^T = K Q^T, and (2 key halves) x (D/32) of P V
     constexpr int NDB = D / 32;  // 32-wide blocks of head_dim in O^T
@@ -127,12 +126,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // before they are used (buffer loads: keys or rows past the end read as zeros and are masked anyway).
     // (fp16 noise: three dwords per 4 keys, widened by the fused multiply-add that uses them.)
     typedef typename std::conditional<N16, uint3_t, float4_t>::type noise_t;
-    const void* nbase = NOISE ? reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * (N16 ? 2 : 4) : nullptr;
+    const void* nbase = reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * (N16 ? 2 : 4);
     const HalfNoise hn(nbase, N16 ? a.Sq : 1, N16 ? a.ns : 0, N16 ? a.Skv : 0);
     const __amdgpu_buffer_rsrc_t nrs = N16 ? hn.rs : __builtin_amdgcn_make_buffer_rsrc(
-        (void*)nbase, 0, NOISE ? (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4) : 0, 0x00020000);
+        (void*)nbase, 0, (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4), 0x00020000);
     int nsh = 0;
-    const int nvo = N16 ? hn.row((int64_t)qrow_ld * a.ns + 4 * h, nsh) : NOISE ? (int)(((int64_t)qrow_ld * a.ns + 4 * h) * 4) : 0;
+    const int nvo = N16 ? hn.row((int64_t)qrow_ld * a.ns + 4 * h, nsh) : (int)(((int64_t)qrow_ld * a.ns + 4 * h) * 4);
     noise_t gpre0[4], gpre1[4];        // even / odd 32-key blocks: each refilled two blocks ahead, as soon as it is used
     auto fetch_noise = [&](int key0, noise_t (&gpre)[4]) __attribute__((always_inline)) {
 #pragma unroll
@@ -169,43 +168,41 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // (The form for blocks that may need the mask; the steps of the plain loop do the same between their MFMAs.)
     auto reduce_block = [&](float16_t& sx, int key0, float& smax, noise_t (&gpre)[4]) __attribute__((always_inline)) {
         const int last = last_key - key0 - 4 * h;      // as an offset from the lane's first key
-        if constexpr (NOISE) {
-            // Row normaliser of the perturbed scores z = s*c2 + g*c3 (log2 domain), with a lazy reference like the
-            // main softmax: d = z - m2 comes straight out of two fused multiply-adds, and m2 is only raised when some d
-            // exceeds 8 (the sum lives in fp32: 2^8 of head-room is harmless) or nothing has been summed yet.
-            const float nref = -m2;
-            float16_t d;
+        // Row normaliser of the perturbed scores z = s*c2 + g*c3 (log2 domain), with a lazy reference like the
+        // main softmax: d = z - m2 comes straight out of two fused multiply-adds, and m2 is only raised when some d
+        // exceeds 8 (the sum lives in fp32: 2^8 of head-room is harmless) or nothing has been summed yet.
+        const float nref = -m2;
+        float16_t d;
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                typename std::conditional<N16, half4_t, float4_t>::type gv;
-                if constexpr (N16) gv = half_noise4(gpre[r4], nsh); else gv = gpre[r4];
+        for (int r4 = 0; r4 < 4; ++r4) {
+            typename std::conditional<N16, half4_t, float4_t>::type gv;
+            if constexpr (N16) gv = half_noise4(gpre[r4], nsh); else gv = gpre[r4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)gv[e], a.c3, nref));
-                    d[r4 * 4 + e] = 8 * r4 + e <= last ? dd : -INFINITY;
-                }
+            for (int e = 0; e < 4; ++e) {
+                const float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)gv[e], a.c3, nref));
+                d[r4 * 4 + e] = 8 * r4 + e <= last ? dd : -INFINITY;
             }
-            fetch_noise(key0 + 64, gpre);    // the next block of the same parity, two pipeline steps ahead of its use
-            // The test runs on the lane's own 16 keys; the exchange with the other lane of the query (m2 and have2 are
-            // shared by the pair) is made on the rare path only -- if either lane of a pair wants the raise, the
-            // wave-wide vote takes every lane there.
-            const float down = max16_bare(d);
-            if (__builtin_amdgcn_ballot_w64(down > 8.0f || (!have2 && down > -INFINITY)) != 0) {     // rare after a row's first block
-                const float dmax = half_max(down);
-                const bool seen = dmax > -INFINITY;            // a block can be entirely masked for this row pair
-                const bool raise = dmax > 8.0f || (!have2 && seen);
-                const float shift = raise ? dmax : 0.f;
-                l2 = have2 ? l2 * fast_exp2(-shift) : 0.f;     // (a first reference below -128 would make the power infinite)
-                m2 += shift;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) d[r] -= shift;
-                have2 = have2 || seen;
-            }
-            float sum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sum += fast_exp2(d[r]);
-            l2 += sum;
         }
+        fetch_noise(key0 + 64, gpre);    // the next block of the same parity, two pipeline steps ahead of its use
+        // The test runs on the lane's own 16 keys; the exchange with the other lane of the query (m2 and have2 are
+        // shared by the pair) is made on the rare path only -- if either lane of a pair wants the raise, the
+        // wave-wide vote takes every lane there.
+        const float down = max16_bare(d);
+        if (__builtin_amdgcn_ballot_w64(down > 8.0f || (!have2 && down > -INFINITY)) != 0) {     // rare after a row's first block
+            const float dmax = half_max(down);
+            const bool seen = dmax > -INFINITY;            // a block can be entirely masked for this row pair
+            const bool raise = dmax > 8.0f || (!have2 && seen);
+            const float shift = raise ? dmax : 0.f;
+            l2 = have2 ? l2 * fast_exp2(-shift) : 0.f;     // (a first reference below -128 would make the power infinite)
+            m2 += shift;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) d[r] -= shift;
+            have2 = have2 || seen;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum += fast_exp2(d[r]);
+        l2 += sum;
 #pragma unroll
         for (int r = 0; r < 16; ++r)
             sx[r] = 8 * (r / 4) + (r % 4) <= last ? sx[r] : -INFINITY;      // (a select: stale-LDS garbage past the last block never propagates)
@@ -334,7 +331,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     };
 
     // ---- prologue: K stages 0 and 1 and V stage 0; scores of block 0; first K operands of block 1 ----
-    if constexpr (NOISE) { fetch_noise(0, gpre0); fetch_noise(32, gpre1); }
+    fetch_noise(0, gpre0);
+    fetch_noise(32, gpre1);
     TRN_FETCH_K(0, Ks0);
     TRN_FETCH_V(0, Vs0);
     if (ntiles > 1) TRN_FETCH_K(1, Ks1);
@@ -361,13 +359,13 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         auto handover = [&]() __attribute__((always_inline)) {
             // this wave's share of stages Kn and Vc is in LDS: everything but the noise requests of the two
             // steps since the stages were requested (2 x 4 loads, issued behind them) has returned
-            if constexpr (NOISE) __builtin_amdgcn_s_waitcnt(0x0f78); else __builtin_amdgcn_s_waitcnt(0x0f70);
+            __builtin_amdgcn_s_waitcnt(0x0f78);
             __syncthreads();                      // ... and everyone's; Kc and Vn have had their last readers
-            // With noise in flight the refills are issued unconditionally (tiles past the end just fill stages
+            // The refills are issued unconditionally (tiles past the end just fill stages
             // nobody reads): the compiler sizes its waits for the noise registers by the loads it KNOWS follow
             // them, and a conditional load counts as absent -- every noise use would drain the refills too.
-            if (NOISE || jt + 2 < ntiles) TRN_FETCH_K(jt + 2, Kc);
-            if (NOISE || jt + 1 < ntiles) TRN_FETCH_V(jt + 1, Vn);
+            TRN_FETCH_K(jt + 2, Kc);
+            TRN_FETCH_V(jt + 1, Vn);
         };
         auto none = [&]() __attribute__((always_inline)) {};
         // (Past the last tile a K stage holds stale rows; scores computed from them are masked away.)
@@ -429,23 +427,21 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         }
     }
     if (qrow < a.Sq && h == 0 && a.lse) a.lse[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m + fast_log2(l)) * kLn2;
-    if constexpr (NOISE) {
-        if (qrow < a.Sq && h == 0)
-            a.lse_pert[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m2 + fast_log2(l2)) * kLn2;
-    }
+    if (qrow < a.Sq && h == 0) a.lse_pert[((int64_t)b * a.Hq + head) * a.Sq + qrow] = (m2 + fast_log2(l2)) * kLn2;
 }
 #endif
 
-template <int D, int NW, bool NOISE>
+// (The third parameter only keeps the name that traces and trn_attn_fwd_kernel_name() show.)
+template <int D, int NW, bool>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    attn_fwd_body<D, NW, NOISE ? 1 : 0>(a);
+    attn_fwd_body<D, NW, false>(a);
 #endif
 }
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_half_noise_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    attn_fwd_body<D, NW, 2>(a);
+    attn_fwd_body<D, NW, true>(a);
 #endif
 }
 

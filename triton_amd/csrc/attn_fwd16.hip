@@ -716,7 +716,7 @@ hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape,
     switch (shape) {
         case Attn16Shape::Paired: return d128 ? launch16<128, 8, kPaired>(a, s) : launch16<64, 8, kPaired>(a, s);
         case Attn16Shape::Split:  return d128 ? launch16<128, 8, kSplit>(a, s) : launch16<64, 8, kSplit>(a, s);
-        case Attn16Shape::Wide:   return d128 ? launch16<128, 8, kPlain>(a, s) : launch16<64, 8, kPlain>(a, s);
+        case Attn16Shape::Wide:   return launch16<128, 8, kPlain>(a, s);             // (head_dim 128 only)
         default:                  return d128 ? launch16<128, 4, kPlain>(a, s) : launch16<64, 4, kPlain>(a, s);
     }
 }
@@ -724,9 +724,8 @@ hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape,
 const char* attn_fwd16_kernel_name(int head_dim, Attn16Shape shape) {
     if (shape == Attn16Shape::Split) return head_dim == 128 ? "trn::attn_fwd16_split_kernel<128>" : "trn::attn_fwd16_split_kernel<64>";
     if (shape == Attn16Shape::Paired) return head_dim == 128 ? "trn::attn_fwd16_kernel<128, 8, true>" : "trn::attn_fwd16_kernel<64, 8, true>";
-    const bool wide = shape == Attn16Shape::Wide;
-    if (head_dim == 128) return wide ? "trn::attn_fwd16_kernel<128, 8, false>" : "trn::attn_fwd16_kernel<128, 4, false>";
-    return wide ? "trn::attn_fwd16_kernel<64, 8, false>" : "trn::attn_fwd16_kernel<64, 4, false>";
+    if (shape == Attn16Shape::Wide) return "trn::attn_fwd16_kernel<128, 8, false>";
+    return head_dim == 128 ? "trn::attn_fwd16_kernel<128, 4, false>" : "trn::attn_fwd16_kernel<64, 4, false>";
 }
 
 }  // namespace trn
