@@ -253,11 +253,14 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     //   phase B: MFMA: O^T += V^T P^T                    | VALU: mask + max of block B+1's scores
     // Every LDS operand feeds two consecutive MFMAs (the two query blocks); it is requested NQ operands before its
     // first use, into the register its predecessor has just vacated.  With SYNC (first block of a 64-key tile) the
-    // tile hand-over sits right after the last request to the tile's own K stage.
+    // tile hand-over sits right after the last request to the tile's own K stage, and the refills of the two stages that it
+    // sets free go out one at a time behind the MFMAs of phase B.  A CU takes 64 bytes a clock from L2: requested all at once
+    // behind the barrier, by all waves, 32 KB held up every wave's issue for some 500 of a tile's 2900 - 4300 clocks (32 heads
+    // of 128: 4096 tokens 118.4 -> 117.2 us, 3600 107 -> 104.5, 777 16.8 -> 15.9; 71 of 64, 1574 31.6 -> 30.7).
     // MAYMASK = false: the caller knows that block B+1 needs no mask, and the test and its branch (which would sit in
     // the middle of phase B and split the slot sequence) are not compiled in.
     auto step = [&](bool masked_next, auto maymask_tag, auto sync_tag, Scores16& sc, Scores16& sn, const half_t* Vblk, const half_t* K1,
-                    const half_t* K2, int key0_next, auto&& handover) __attribute__((always_inline)) {
+                    const half_t* K2, int key0_next, auto&& handover, auto&& refill) __attribute__((always_inline)) {
         constexpr bool SYNC = decltype(sync_tag)::value;
         constexpr bool MAYMASK = decltype(maymask_tag)::value;
         half8_t pB[2];
@@ -303,6 +306,11 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
             if (i & 1) {
                 if (db + NQ < NOP) load_v(db + NQ, db % NQ);
                 else load_k(K2, db + NQ - NOP, db % NQ);
+            }
+            if constexpr (SYNC) {
+                constexpr int EVERY = NS / (2 * NI);
+                static_assert(NS % (2 * NI) == 0, "the refills are dealt out evenly");
+                if (i % EVERY == EVERY - 1) refill(i / EVERY);
             }
             constexpr int R0 = NS / 2 - (NS >= 16 ? 3 : 2);
             if (i == R0) { if (MAYMASK && masked_next) mask_block(sn, key0_next); }
@@ -396,15 +404,18 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         auto handover = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's share of stages Kn and Vc is in LDS
             __syncthreads();                      // ... and everyone's; Kc and Vn have had their last readers
-            // (unconditional: tiles past the end of the keys read as zeros into stages nobody reads, and the
-            // hand-over stays free of branches)
-            TRN_FETCH_K(jt + 2, Kc);
-            TRN_FETCH_V(jt + 1, Vn);
+        };
+        // (unconditional: tiles past the end of the keys read as zeros into stages nobody reads, and the
+        // hand-over stays free of branches)
+        auto refill = [&](int i) __attribute__((always_inline)) {
+            if (i < NI) fetch_piece<D, GW>(vrs, &Vn[gw * RPI * D], vvo, vgrp_bytes + (jt + 1) * vtile_bytes, vrow_bytes, i);
+            else fetch_piece<D, GW>(krs, &Kc[gw * RPI * D], kvo, kgrp_bytes + (jt + 2) * ktile_bytes, krow_bytes, i - NI);
         };
         auto none = [&]() __attribute__((always_inline)) {};
+        auto none1 = [&](int) __attribute__((always_inline)) {};
         // (Past the last tile a K stage holds stale rows; scores computed from them are masked away.)
-        step(needs_mask(kv0 + 32), maymask_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover);
-        step(needs_mask(kv0 + KSTEP), maymask_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + KSTEP, none);
+        step(needs_mask(kv0 + 32), maymask_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover, refill);
+        step(needs_mask(kv0 + KSTEP), maymask_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + KSTEP, none, none1);
     };
     // Under a causal mask the waves of a workgroup see different numbers of tiles: a wave computes the tiles that
     // hold a key visible to one of its queries, and for the rest only keeps up the staging it shares with the

@@ -109,13 +109,16 @@ template <int D> __device__ __forceinline__ int swz(int r) {
 // the swizzle; because the row groups of successive loads are a multiple of 16 rows apart the swizzle is the
 // same for all of them, so ONE per-lane offset serves every load and the rest is wave-uniform (soffset).
 #if defined(__HIP_DEVICE_COMPILE__)
+template <int D, int NW>
+__device__ __forceinline__ void fetch_piece(__amdgpu_buffer_rsrc_t rs, half_t* dst_wave, int vo, int soff, int row_step_bytes, int n) {
+    constexpr int RPI = 64 / (D / 8);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst_wave + n * NW * RPI * D), 16, vo,
+                                             soff + n * NW * row_step_bytes, 0, 0);
+}
 template <int NI, int D, int NW>
 __device__ __forceinline__ void fetch_tile(__amdgpu_buffer_rsrc_t rs, half_t* dst_wave, int vo, int soff, int row_step_bytes) {
-    constexpr int RPI = 64 / (D / 8);
 #pragma unroll
-    for (int n = 0; n < NI; ++n)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(dst_wave + n * NW * RPI * D),
-                                                 16, vo, soff + n * NW * row_step_bytes, 0, 0);
+    for (int n = 0; n < NI; ++n) fetch_piece<D, NW>(rs, dst_wave, vo, soff, row_step_bytes, n);
 }
 #endif
 
