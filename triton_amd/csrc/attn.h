@@ -70,6 +70,9 @@ int attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, co
 int attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise, float* out_sum,
                   float* out_sumsq, int mean_std, void* stream, bool n16 = false, bool s16 = false, bool any_pitch = false);
 
+// Whether the kernels that read all of this noise request it past the caches (attn_fwd.hip).
+bool noise_streams(const trn_attn_desc* d, const void* noise, bool n16);
+
 // One workgroup per head and 32 queries, whose eight waves split the keys (attn_decode.hip): at most 32 queries per head
 // (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.
 bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);

@@ -92,7 +92,7 @@ constexpr int CBN = 128;  // keys per workgroup
 
 // SQ: the sums of squares are wanted too (RoCo); without them (KeyFormer) their accumulators and one of the five
 // VALU operations per score are not compiled in.
-// NZ: 1 fp32 noise, 2 fp16 noise
+// NZ: 1 fp32 noise, 2 fp16 noise, 3 fp32 noise requested past the caches (noise_streams())
 // NG: groups of four waves on the same 128 keys, each taking every NG-th query tile through stages of its own; the second
 // hands its sums to the first at the end.
 template <int D, int NZ, bool SQ, int NG>
@@ -188,7 +188,7 @@ __global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArg
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             if constexpr (N16) p.g[qb][r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b96(nrs, nvo + r4 * nrow8, so, 0));
-            else p.g[qb][r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * nrow8, so, 0));
+            else p.g[qb][r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * nrow8, so, NZ == 3 ? 2 : 0));
         }
     };
 
@@ -616,9 +616,10 @@ int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, con
     a.c1 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.causal = d->causal ? 1 : 0;
     a.mean_std = mean_std; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
+    const bool stream_noise = noise_streams(d, noise, n16);
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
-    if (d->head_dim == 128) e = !noise ? launch_col_plain<128>(a, s) : n16 ? launch_col<128, 2>(a, s) : launch_col<128, 1>(a, s);
-    else e = !noise ? launch_col_plain<64>(a, s) : n16 ? launch_col<64, 2>(a, s) : launch_col<64, 1>(a, s);
+    if (d->head_dim == 128) e = !noise ? launch_col_plain<128>(a, s) : n16 ? launch_col<128, 2>(a, s) : stream_noise ? launch_col<128, 3>(a, s) : launch_col<128, 1>(a, s);
+    else e = !noise ? launch_col_plain<64>(a, s) : n16 ? launch_col<64, 2>(a, s) : stream_noise ? launch_col<64, 3>(a, s) : launch_col<64, 1>(a, s);
     return e == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
 }

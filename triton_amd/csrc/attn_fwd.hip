@@ -27,27 +27,42 @@ namespace trn {
 
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer-descriptor types and LDS-load builtins exist in the device pass only;
                                       // the host pass needs just the launch stubs
-// N16: fp16 noise (fp32 otherwise)
-template <int D, int NW, bool N16>
+// N16: fp16 noise (fp32 otherwise).  NT: the noise is requested with the non-temporal hint.  SPLIT: the eight waves are two
+// groups of four on the same 128 queries, each taking every other 64-key tile through stages of its own; their results are
+// merged through LDS at the end.
+template <int D, int NW, bool N16, bool NT, bool SPLIT>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
+    static_assert(!SPLIT || NW == 8, "two groups of four waves");
+    constexpr int GW = SPLIT ? 4 : NW;       // waves that share the K / V stages
+    constexpr int NG = SPLIT ? 2 : 1;        // groups with stages of their own
+    constexpr int KSTEP = SPLIT ? 128 : 64;  // keys from one tile of a wave to its next
     constexpr int BN = 64;       // keys per LDS stage (two 32-key blocks)
     constexpr int NS = D / 16;   // MFMA slots per phase: k-steps of S^T = K Q^T, and (2 key halves) x (D/32) of P V
     constexpr int NDB = D / 32;  // 32-wide blocks of head_dim in O^T
     constexpr int EPI = 16 / NS; // score elements converted per slot
     constexpr int CPR = D / 8;   // 16-byte chunks per row
     constexpr int RPI = 64 / CPR;            // stage rows covered by one wave-wide 1 KB load
-    constexpr int NI = BN / (RPI * NW);      // such loads per wave per stage (K and V each)
-    constexpr int BM = 32 * NW;              // queries per workgroup: NW waves x 32
+    constexpr int NI = BN / (RPI * GW);      // such loads per wave per stage (K and V each)
+    constexpr int BM = 32 * GW;              // queries per workgroup, 32 a wave
     // Two stages each for K and V, as FOUR separate arrays: the compiler orders an LDS read after every
     // outstanding global->LDS load that may alias it, and only distinct variables are provably disjoint --
     // with one [2][..] array every LDS read would wait for the prefetch that was just issued.
-    __shared__ __attribute__((aligned(1024))) half_t Ks0[BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Ks1[BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Vs0[BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Vs1[BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Ks0_[NG * BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Ks1_[NG * BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Vs0_[NG * BN * D];
+    __shared__ __attribute__((aligned(1024))) half_t Vs1_[NG * BN * D];
+    // the waves' noise blocks on their way from whole row pieces, as they are fetched, to the accumulator layout
+    constexpr int NSZ = N16 ? 2 : 4;
+    __shared__ __attribute__((aligned(1024))) char Nt[NW * 1024 * NSZ];
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = SPLIT ? wave >> 2 : 0, gw = SPLIT ? wave & 3 : wave;
+    half_t* const Ks0 = Ks0_ + grp * BN * D;
+    half_t* const Ks1 = Ks1_ + grp * BN * D;
+    half_t* const Vs0 = Vs0_ + grp * BN * D;
+    half_t* const Vs1 = Vs1_ + grp * BN * D;
+    const int kfirst = grp * BN;                        // first key of this wave's first tile
 
     // ---- which (query tile, batch, head): heavy tiles first, KV heads interleaved across ids
     const int BH = a.B * a.Hq;
@@ -59,7 +74,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
 
     const int off = a.Skv - a.Sq;                       // causal: query i sees keys <= i + off
     const int q0 = qt * BM;
-    const int wq0 = q0 + wave * 32;                     // first query of this wave
+    const int wq0 = q0 + gw * 32;                       // first query of this wave
     const int qrow = wq0 + c;                           // this lane's query
     const int qrow_ld = qrow < a.Sq ? qrow : a.Sq - 1;  // clamp loads; stores are predicated
 
@@ -121,24 +136,54 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     int ntiles = (a.Skv + BN - 1) / BN;
     if (a.causal) ntiles = min(ntiles, (min(q0 + BM - 1, a.Sq - 1) + off) / BN + 1);
 
-    // KeyFormer noise: this lane's query row, the 4 x 4 keys of its accumulator layout per 32-key block.  It is
-    // the HBM stream that bounds that variant, so each block's 64 bytes per lane are requested two pipeline steps
-    // before they are used (buffer loads: keys or rows past the end read as zeros and are masked anyway).
-    // (fp16 noise: three dwords per 4 keys, widened by the fused multiply-add that uses them.)
+    // KeyFormer noise, the HBM stream that bounds this kernel: a 32 x 32 block per wave and step, requested two steps before it
+    // is used (buffer loads: keys or rows past the end read as zeros or as another row's and are masked anyway).  A load
+    // takes whole row pieces, eight lanes a row of 32 keys; in the accumulator layout, a row per lane, it touches 32 lines and
+    // a CU serves such loads at 16 bytes a clock instead of 64 -- more than the arithmetic of a step takes, and every wave
+    // waits to issue behind them (71 heads of 64, 2752 keys, fp16: 221 -> 186 us; 32 of 128, 2048, fp32: 124 -> 109, streamed
+    // past the caches 98).  On arrival the block goes through a wave-private part of LDS into the accumulator layout
+    // (LDS operations of one wave execute in order: no barrier).  fp16 noise: three dwords around 4 keys, shifted on arrival.
     typedef typename std::conditional<N16, uint3_t, float4_t>::type noise_t;
-    const void* nbase = reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * (N16 ? 2 : 4);
+    typedef typename std::conditional<N16, half4_t, float4_t>::type nquad_t;
+    const void* nbase = reinterpret_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * NSZ;
     const HalfNoise hn(nbase, N16 ? a.Sq : 1, N16 ? a.ns : 0, N16 ? a.Skv : 0);
     const __amdgpu_buffer_rsrc_t nrs = N16 ? hn.rs : __builtin_amdgcn_make_buffer_rsrc(
         (void*)nbase, 0, (int)(((int64_t)(a.Sq - 1) * a.ns + a.Skv) * 4), 0x00020000);
-    int nsh = 0;
-    const int nvo = N16 ? hn.row((int64_t)qrow_ld * a.ns + 4 * h, nsh) : (int)(((int64_t)qrow_ld * a.ns + 4 * h) * 4);
+    int nsh = 0, nrow[4];              // byte offsets of the wave's rows 0, 8, 16, 24: at most 7 rows past the last are asked for
+    const int64_t nfirst = (lane >> 3) * a.ns + 4 * (lane & 7);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) nrow[i] = (int)(min(wq0 + 8 * i, (a.Sq - 1) & ~7) * a.ns * NSZ);      // (a multiple of 8 rows: dwords)
+    const int nvo = N16 ? hn.row(nfirst, nsh) : (int)(nfirst * 4);
     noise_t gpre0[4], gpre1[4];        // even / odd 32-key blocks: each refilled two blocks ahead, as soon as it is used
     auto fetch_noise = [&](int key0, noise_t (&gpre)[4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4) {
-            if constexpr (N16) gpre[r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b96(nrs, nvo + r4 * 16, key0 * 2, 0));
-            else gpre[r4] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo + r4 * 32, key0 * 4, 0));
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (N16) gpre[i] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b96(nrs, nvo, nrow[i] + key0 * 2, NT ? 2 : 0));
+            else gpre[i] = __builtin_bit_cast(noise_t, __builtin_amdgcn_raw_buffer_load_b128(nrs, nvo, nrow[i] + key0 * 4, NT ? 2 : 0));
         }
+    };
+    // 4 keys of row r at place q ^ (r/2) % 8 of the row's eight (fp16, two rows more to a line of the 64 banks: q ^ (r/4) % 8),
+    // written as fetched, read as row c, quads 2i + h: both conflict-free
+    nquad_t* const nt = reinterpret_cast<nquad_t*>(Nt + wave * 1024 * NSZ);
+    int nt_wr[2], nt_rd[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 8 * i + (lane >> 3);
+        nt_wr[i] = r * 8 + ((lane & 7) ^ ((r >> (N16 ? 2 : 1)) & 7));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) nt_rd[i] = c * 8 + ((2 * i + h) ^ ((c >> (N16 ? 2 : 1)) & 7));
+    auto stash_noise = [&](const noise_t (&gpre)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // (the place of rows 16 further differs in bit 2 where the swizzle counts pairs of rows or fours of them)
+            const int at = N16 ? (i < 2 ? nt_wr[i] : (nt_wr[i & 1] ^ 4) + 128) : nt_wr[i & 1] + (i >> 1) * 128;
+            if constexpr (N16) nt[at] = half_noise4(gpre[i], nsh); else nt[at] = gpre[i];
+        }
+    };
+    auto noise_quads = [&](nquad_t (&g)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) g[i] = nt[nt_rd[i]];
     };
 
     // ---- staging: direct global -> LDS loads.  Buffer descriptors give zero fill for keys past the end
@@ -147,14 +192,15 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         (void*)(a.k + b * a.kb + kvh * a.kh), 0, (int)(((int64_t)(a.Skv - 1) * a.ks + D) * 2), 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.v + b * a.vb + kvh * a.vh), 0, (int)(((int64_t)(a.Skv - 1) * a.vs + D) * 2), 0x00020000);
-    const int st_row = wave * RPI + lane / CPR;                      // this lane's row within each 4*RPI-row group
+    const int st_row = gw * RPI + lane / CPR;                      // this lane's row within each 4*RPI-row group
     const int st_chunk = (lane % CPR) ^ swz<D>(st_row);             // LDS slot lane%CPR of that row holds this logical chunk
     const int kvo = (int)(st_row * a.ks * 2) + st_chunk * 16;       // per-lane byte offsets within a stage
     const int vvo = (int)(st_row * a.vs * 2) + st_chunk * 16;
     const int krow_bytes = (int)(RPI * a.ks * 2), vrow_bytes = (int)(RPI * a.vs * 2);
-    const int ktile_bytes = (int)(BN * a.ks * 2), vtile_bytes = (int)(BN * a.vs * 2);
-#define TRN_FETCH_K(jt_, dst_) fetch_tile<NI, D, NW>(krs, &dst_[wave * RPI * D], kvo, (jt_) * ktile_bytes, krow_bytes)
-#define TRN_FETCH_V(jt_, dst_) fetch_tile<NI, D, NW>(vrs, &dst_[wave * RPI * D], vvo, (jt_) * vtile_bytes, vrow_bytes)
+    const int ktile_bytes = (int)(KSTEP * a.ks * 2), vtile_bytes = (int)(KSTEP * a.vs * 2);
+    const int kgrp_bytes = (int)(kfirst * a.ks * 2), vgrp_bytes = (int)(kfirst * a.vs * 2);
+#define TRN_FETCH_K(jt_, dst_) fetch_tile<NI, D, GW>(krs, &dst_[gw * RPI * D], kvo, kgrp_bytes + (jt_) * ktile_bytes, krow_bytes)
+#define TRN_FETCH_V(jt_, dst_) fetch_tile<NI, D, GW>(vrs, &dst_[gw * RPI * D], vvo, vgrp_bytes + (jt_) * vtile_bytes, vrow_bytes)
 
     const float16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     const int last_key = min(a.Skv - 1, a.causal ? qrow + off : a.Skv - 1);    // the last key this lane's query sees
@@ -166,7 +212,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // and the 16*NDB-multiply rescale of O^T runs on the first block or two only instead of on most blocks.
     // Returns whether a rescale is due (wave-uniform) and the candidate max.
     // (The form for blocks that may need the mask; the steps of the plain loop do the same between their MFMAs.)
-    auto reduce_block = [&](float16_t& sx, int key0, float& smax, noise_t (&gpre)[4]) __attribute__((always_inline)) {
+    auto reduce_block = [&](float16_t& sx, int key0, float& smax, const nquad_t (&g)[4], noise_t (&gpre)[4]) __attribute__((always_inline)) {
         const int last = last_key - key0 - 4 * h;      // as an offset from the lane's first key
         // Row normaliser of the perturbed scores z = s*c2 + g*c3 (log2 domain), with a lazy reference like the
         // main softmax: d = z - m2 comes straight out of two fused multiply-adds, and m2 is only raised when some d
@@ -175,15 +221,13 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
         float16_t d;
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
-            typename std::conditional<N16, half4_t, float4_t>::type gv;
-            if constexpr (N16) gv = half_noise4(gpre[r4], nsh); else gv = gpre[r4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)gv[e], a.c3, nref));
+                const float dd = __builtin_fmaf(sx[r4 * 4 + e], a.c2, __builtin_fmaf((float)g[r4][e], a.c3, nref));
                 d[r4 * 4 + e] = 8 * r4 + e <= last ? dd : -INFINITY;
             }
         }
-        fetch_noise(key0 + 64, gpre);    // the next block of the same parity, two pipeline steps ahead of its use
+        fetch_noise(key0 + KSTEP, gpre); // the next block of the same parity, two pipeline steps ahead of its use
         // The test runs on the lane's own 16 keys; the exchange with the other lane of the query (m2 and have2 are
         // shared by the pair) is made on the rare path only -- if either lane of a pair wants the raise, the
         // wave-wide vote takes every lane there.
@@ -239,7 +283,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     // previous tile's V stage, so after the barrier those two stages are refilled (K two tiles ahead, V one
     // tile ahead) and all later LDS reads of this and the next step go to the stages that just became visible.
     auto step = [&](auto plain_tag, auto sync_tag, float16_t& sc, float16_t& sn, const half_t* Vblk, const half_t* K1,
-                    const half_t* K2, int key0_next, auto&& handover, noise_t (&gpre)[4]) __attribute__((always_inline)) {
+                    const half_t* K2, int key0_next, auto&& handover, auto&& refill, noise_t (&gpre)[4]) __attribute__((always_inline)) {
         constexpr bool SYNC = decltype(sync_tag)::value, PLAIN = decltype(plain_tag)::value;
         // The row sum is taken over the fp16-rounded P (v_dot2_f32_f16 against ones, fp32 accumulate),
         // i.e. over exactly the values that multiply V.
@@ -251,12 +295,15 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
             half4_t hi = lds_read_tr16(vp + voff_hi[op % NDB]);   // keys +8..11
             va[reg] = half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         };
+        nquad_t g[4];
         // ---- phase A ----
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
             if constexpr (SYNC) {
                 if (i == NS - NQ) handover();
             }
+            if (i == NS - 2) stash_noise(gpre);
+            if (i == NS - 1) noise_quads(g);
             sn = mfma32(ka[i % NQ], qB[i], i == 0 ? zero : sn);
             if (i + NQ < NS) ka[i % NQ] = *reinterpret_cast<const half8_t*>(&K1[koff[i + NQ]]);
             else load_v(i + NQ - NS, i % NQ);
@@ -269,52 +316,53 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 l = __builtin_amdgcn_fdot2(pp, ones, l, false);
                 pB[r / 8][r % 8] = pp[0]; pB[r / 8][r % 8 + 1] = pp[1];
             }
+            asm volatile("" : "+v"(l));
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- phase B ----
         float smax = 0.f;
         bool due = false;
         // No mask: the perturbed scores are exponentiated and summed between the MFMAs, two scores at a time, against the
-        // reference as it stands; whether it had to be raised is known at the end, and the block's sum is then formed
-        // again (rare after a row's first block).  In one piece behind the fourth MFMA, as reduce_block() has it, the two
-        // waves of a SIMD left the matrix pipe idle for most of it: 32 heads of 128, 4096 keys, fp32 noise 333 -> 309 us,
-        // fp16 270 -> 251; 1501 keys, fp16 65 -> 51; 284 heads of 64, 392 keys 48 -> 37 (same bits; short bursts from an idle
-        // board, here and at noise_kernel_wide(): once its clocks have risen 4096 keys take 266).
+        // reference as it stands.  That it has to be raised shows in the sum of the lane's 16 (over 256: some score lies more
+        // than 4 above it; none more than 8 otherwise), and the block's sum is then formed again (rare after a row's first).
         const float nref = -m2;
-        float down = -INFINITY, top = -INFINITY, sum = 0.f;
+        float top = -INFINITY, sum = 0.f;
         auto perturbed = [&](int r, float ref) __attribute__((always_inline)) {
-            float g;
-            if constexpr (N16) {
-                const uint3_t w = gpre[r / 4];
-                const uint32_t u = (r & 2) ? __builtin_amdgcn_alignbit(w.z, w.y, nsh) : __builtin_amdgcn_alignbit(w.y, w.x, nsh);
-                g = (float)__builtin_bit_cast(half2_t, u)[r & 1];
-            } else g = gpre[r / 4][r % 4];
-            return __builtin_fmaf(sn[r], a.c2, __builtin_fmaf(g, a.c3, ref));
+            return __builtin_fmaf(sn[r], a.c2, __builtin_fmaf((float)g[r / 4][r % 4], a.c3, ref));
         };
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
             oacc[i % NDB] = mfma32(va[i % NQ], pB[i / NDB], oacc[i % NDB]);
             if (i + NQ < NS) load_v(i + NQ, i % NQ);
             else ka[i % NQ] = *reinterpret_cast<const half8_t*>(&K2[koff[i + NQ - NS]]);
+            if constexpr (SYNC) {
+                if (i < NS / 2) {
+#pragma unroll
+                    for (int k = 0; k < 4 * NI / NS; ++k) refill(i * (4 * NI / NS) + k);
+                }
+            }
             if constexpr (PLAIN) {
                 // scores [first(i), first(i + 1)) in slot i: none in slot 0, whose MFMA covers the end of the score chain
                 auto first = [](int k) { return NS == 8 ? (k == 8 ? 16 : k < 1 ? 0 : 2 * (k - 1)) : k == 4 ? 16 : k < 2 ? 0 : k == 2 ? 4 : 10; };
 #pragma unroll
                 for (int r = first(i); r < first(i + 1); r += 2) {
                     const float d0 = perturbed(r, nref), d1 = perturbed(r + 1, nref);
-                    down = max3_after(down, d0, d1, d1);
                     top = max3_after(top, sn[r], sn[r + 1], d1);
                     sum += fast_exp2(d0);
                     sum += fast_exp2(d1);
+                    asm volatile("" : "+v"(sum));     // (left alone the compiler moves all of this behind the last MFMA)
                 }
-            } else if (i == NS / 2) due = reduce_block(sn, key0_next, smax, gpre);
+            } else if (i == NS / 2) due = reduce_block(sn, key0_next, smax, g, gpre);
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (PLAIN) {
             smax = top * a.c1;
-            if (__builtin_amdgcn_ballot_w64(down > 8.0f || (!have2 && down > -INFINITY) || smax > m + 8.0f) != 0) {
+            if (__builtin_amdgcn_ballot_w64(!have2 || sum > 256.0f || smax > m + 8.0f) != 0) {
+                float down = -INFINITY;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) down = fmaxf(down, perturbed(r, nref));
                 const float dmax = half_max(down);
-                const bool seen = dmax > -INFINITY, raise = dmax > 8.0f || (!have2 && seen);
+                const bool seen = dmax > -INFINITY, raise = dmax > 4.0f || (!have2 && seen);
                 const float shift = raise ? dmax : 0.f;
                 l2 = have2 ? l2 * fast_exp2(-shift) : 0.f;     // (as in reduce_block)
                 m2 += shift;
@@ -325,17 +373,17 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 due = __builtin_amdgcn_ballot_w64(smax > m + 8.0f) != 0;
             }
             l2 += sum;
-            fetch_noise(key0_next + 64, gpre);
+            fetch_noise(key0_next + KSTEP, gpre);
         }
         if (due) rescale(smax);
     };
 
     // ---- prologue: K stages 0 and 1 and V stage 0; scores of block 0; first K operands of block 1 ----
-    fetch_noise(0, gpre0);
-    fetch_noise(32, gpre1);
+    fetch_noise(kfirst, gpre0);
+    fetch_noise(kfirst + 32, gpre1);
     TRN_FETCH_K(0, Ks0);
     TRN_FETCH_V(0, Vs0);
-    if (ntiles > 1) TRN_FETCH_K(1, Ks1);
+    if (SPLIT || ntiles > 1) TRN_FETCH_K(1, Ks1);
     __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0): this wave's loads have landed in LDS
     __syncthreads();
 
@@ -349,13 +397,16 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
 #pragma unroll
         for (int i = 0; i < NQ; ++i) ka[i] = *reinterpret_cast<const half8_t*>(&Ks0[32 * D + koff[i]]);
         float smax;
-        if (reduce_block(sA, 0, smax, gpre0)) rescale(smax);
+        nquad_t g[4];
+        stash_noise(gpre0);
+        noise_quads(g);
+        if (reduce_block(sA, kfirst, smax, g, gpre0)) rescale(smax);
     }
 
     // One 64-key tile jt.  Kc = its own K stage (block 1 still has operands to give), Kn = the next tile's
     // K stage, Vc = its V stage, Vn = the other V stage.
     auto tile = [&](auto plain_tag, int jt, half_t* Kc, const half_t* Kn, const half_t* Vc, half_t* Vn) __attribute__((always_inline)) {
-        const int kv0 = jt * BN;
+        const int kv0 = kfirst + jt * KSTEP;
         auto handover = [&]() __attribute__((always_inline)) {
             // this wave's share of stages Kn and Vc is in LDS: everything but the noise requests of the two
             // steps since the stages were requested (2 x 4 loads, issued behind them) has returned
@@ -364,26 +415,43 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
             // The refills are issued unconditionally (tiles past the end just fill stages
             // nobody reads): the compiler sizes its waits for the noise registers by the loads it KNOWS follow
             // them, and a conditional load counts as absent -- every noise use would drain the refills too.
-            TRN_FETCH_K(jt + 2, Kc);
-            TRN_FETCH_V(jt + 1, Vn);
+        };
+        auto refill = [&](int i) __attribute__((always_inline)) {
+            if (i < NI) fetch_piece<D, GW>(vrs, &Vn[gw * RPI * D], vvo, vgrp_bytes + (jt + 1) * vtile_bytes, vrow_bytes, i);
+            else fetch_piece<D, GW>(krs, &Kc[gw * RPI * D], kvo, kgrp_bytes + (jt + 2) * ktile_bytes, krow_bytes, i - NI);
         };
         auto none = [&]() __attribute__((always_inline)) {};
+        auto none1 = [&](int) __attribute__((always_inline)) {};
         // (Past the last tile a K stage holds stale rows; scores computed from them are masked away.)
-        step(plain_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover, gpre1);
-        step(plain_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + 64, none, gpre0);
+        step(plain_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover, refill, gpre1);
+        step(plain_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + KSTEP, none, none1, gpre0);
     };
-    // The tiles whose successors need no mask for any wave of the workgroup have a loop of their own (whole turns of the
-    // two stages), the tiles at the diagonal and at the end of the keys another.
-    const int lim = a.causal ? min(a.Skv, q0 + off + 1) : a.Skv;     // keys that every query of the workgroup sees
-    const int n_plain = lim >= BN + 32 ? ((lim - BN - 32) / BN + 1) & ~1 : 0;
+    // Under a causal mask a wave computes the tiles that hold a key visible to one of its queries and for the rest only keeps
+    // up the staging that it shares with the others.  The tiles whose successors need no mask have a loop of their own (whole
+    // turns of the two stages), the tiles at the diagonal and at the end of the keys another.
+    int nlive = ntiles;
+    if (a.causal) nlive = min(ntiles, (min(wq0 + 31, a.Sq - 1) + off) / BN + 1);
+    const int nloop = SPLIT ? (ntiles + 1) >> 1 : ntiles;
+    if constexpr (SPLIT) nlive = (nlive - grp + 1) >> 1;
+    if (wq0 >= a.Sq) nlive = 0;
+    const int lim = (a.causal ? min(a.Skv, wq0 + off + 1) : a.Skv) - kfirst;     // keys that every query of the wave sees
+    const int n_plain = min(nlive, lim >= KSTEP + 32 ? (lim - KSTEP - 32) / KSTEP + 1 : 0) & ~1;
     int jt = 0;
     for (; jt < n_plain; jt += 2) {
         tile(std::true_type{}, jt, Ks0, Ks1, Vs0, Vs1);
         tile(std::true_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
     }
-    for (; jt < ntiles; jt += 2) {
+    for (; jt < nlive; jt += 2) {
         tile(std::false_type{}, jt, Ks0, Ks1, Vs0, Vs1);
-        if (jt + 1 < ntiles) tile(std::false_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
+        if (jt + 1 < nlive) tile(std::false_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
+    }
+    for (jt = nlive; jt < nloop; ++jt) {
+        half_t* Kc = (jt & 1) ? Ks1 : Ks0;
+        half_t* Vn = (jt & 1) ? Vs0 : Vs1;
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        __syncthreads();
+        if (jt + 2 < nloop) TRN_FETCH_K(jt + 2, Kc);
+        if (jt + 1 < nloop) TRN_FETCH_V(jt + 1, Vn);
     }
 #undef TRN_FETCH_K
 #undef TRN_FETCH_V
@@ -394,9 +462,59 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     __builtin_amdgcn_s_waitcnt(0x0f70);                // the refills past the last tile have landed ...
     __syncthreads();                                   // ... everywhere, and every wave is done with the K/V stages
     l = half_sum(l); l2 = half_sum(l2);
-    const float inv = 1.0f / l;
-    {
+    if constexpr (SPLIT) {
+        // The groups hold partial results of the same queries: waves w and w + 4 exchange the normalisers and halves of O^T
+        // lane by lane, group 0 finishes the first D/2 columns, group 1 the others.  A query that saw no key of its group (or
+        // none of finite perturbed score) has zero sums and weighs nothing.
+        constexpr int NH = NDB / 2, kStat = D == 128 ? 5120 : 2560;      // (floats) behind the regions of the output's way through LDS
+        if (!have2) m2 = -INFINITY;
+        float4_t* stat = reinterpret_cast<float4_t*>(reinterpret_cast<float*>(Ks1_) + kStat);        // [8 waves][32 queries]
+        if (h == 0) stat[wave * 32 + c] = float4_t{m, l, m2, l2};
+        float4_t* mine = reinterpret_cast<float4_t*>(grp == 0 ? Ks0_ : Vs0_) + gw * NH * 256;
+        const float4_t* theirs = reinterpret_cast<const float4_t*>(grp == 0 ? Vs0_ : Ks0_) + gw * NH * 256;
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const float16_t& o = grp == 0 ? oacc[NH + i] : oacc[i];
+                mine[(i * 4 + r4) * 64 + lane] = float4_t{o[4 * r4], o[4 * r4 + 1], o[4 * r4 + 2], o[4 * r4 + 3]};
+            }
+        __syncthreads();
+        const float4_t t = stat[(wave ^ 4) * 32 + c];
+        const float ms = fmaxf(m, t[0]), m2s = fmaxf(m2, t[2]);
+        const float wo = m == -INFINITY ? 0.f : fast_exp2(m - ms), wt = t[0] == -INFINITY ? 0.f : fast_exp2(t[0] - ms);
+        l = l * wo + t[1] * wt; m = ms;
+        l2 = (m2 == -INFINITY ? 0.f : l2 * fast_exp2(m2 - m2s)) + (t[2] == -INFINITY ? 0.f : t[3] * fast_exp2(t[2] - m2s));
+        m2 = m2s == -INFINITY ? 0.f : m2s;
+        const float inv = 1.0f / l;
+        constexpr int DP = D / 2, OP = DP + 4, LPRW = DP / 8, RPS = 64 / LPRW;
+        half_t* ot = (grp == 0 ? Vs1_ : Ks1_) + gw * 32 * OP;
+        static_assert(4 * 32 * OP * 2 <= kStat * 4 && kStat * 4 + 4096 <= 2 * BN * D * 2, "the stage holds both");
+#pragma unroll
+        for (int i = 0; i < NH; ++i)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+                const float16_t& o = grp == 0 ? oacc[i] : oacc[NH + i];
+                const float4_t u = theirs[(i * 4 + r4) * 64 + lane];
+                half4_t ov;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) ov[e] = (half_t)((o[4 * r4 + e] * wo + u[e] * wt) * inv);
+                *reinterpret_cast<half4_t*>(&ot[c * OP + i * 32 + 8 * r4 + 4 * h]) = ov;
+            }
+        const int orow = lane / LPRW, ocol = (lane % LPRW) * 8;
+        half_t* ob = a.o + b * a.ob + head * a.oh + grp * DP;
+#pragma unroll
+        for (int j = 0; j < 32 / RPS; ++j) {
+            const int r = j * RPS + orow;
+            const uint2_t lo = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol]);
+            const uint2_t hi = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol + 4]);
+            if (wq0 + r < a.Sq)
+                *reinterpret_cast<uint4_t*>(ob + (int64_t)(wq0 + r) * a.os + ocol) = uint4_t{lo.x, lo.y, hi.x, hi.y};
+        }
+        if (grp == 1) return;               // (the normalisers are written once)
+    } else {
         // two passes of D/2 columns each, so that NW waves' staging regions fit in the four stage arrays
+        const float inv = 1.0f / l;
         constexpr int DP = D / 2, OP = DP + 4;         // row pitch in halfs: 8-byte writes of 32 rows spread over all banks
         constexpr int LPRW = DP / 8, RPS = 64 / LPRW;  // lanes per output row segment, rows per store instruction
         static_assert(32 * OP * 2 <= BN * D * 2 / (NW / 4), "staging region too large");
@@ -431,27 +549,58 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
 }
 #endif
 
-// (The third parameter only keeps the name that traces and trn_attn_fwd_kernel_name() show.)
+// Narrow: 4 waves, 128 queries, two workgroups per CU; Wide: 8 waves, 256 queries; Split: 8 waves on 128 queries, two groups
+// that take every other key tile each.
+enum class NoiseShape { Narrow, Wide, Split };
+
+// fp32 noise in the cache policy that goes with the shape (see noise_streams(); the third parameter only keeps the name that
+// traces and trn_attn_fwd_kernel_name() show)
 template <int D, int NW, bool>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    attn_fwd_body<D, NW, false>(a);
+    attn_fwd_body<D, NW, false, D == 128 && NW == 8, false>(a);
+#endif
+}
+// ... in the other policy
+template <int D, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_other_policy_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd_body<D, NW, false, !(D == 128 && NW == 8), false>(a);
 #endif
 }
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_half_noise_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    attn_fwd_body<D, NW, true>(a);
+    attn_fwd_body<D, NW, true, false, false>(a);
+#endif
+}
+template <int D, bool N16, bool NT>
+__global__ __launch_bounds__(512, 1) void attn_fwd_split_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd_body<D, 8, N16, NT, true>(a);
 #endif
 }
 
 template <int D, int NW>
-static hipError_t launch_fwd(AttnArgs a, hipStream_t s) {
-    a.n_qtiles = (a.Sq + 32 * NW - 1) / (32 * NW);
+static void launch_rows(const AttnArgs& a, bool stream_noise, const dim3& g, hipStream_t s) {
+    const dim3 t(NW * 64);
+    if (a.n16) hipLaunchKernelGGL((attn_fwd_half_noise_kernel<D, NW>), g, t, 0, s, a);
+    else if (stream_noise == (D == 128 && NW == 8)) hipLaunchKernelGGL((attn_fwd_kernel<D, NW, true>), g, t, 0, s, a);
+    else hipLaunchKernelGGL((attn_fwd_other_policy_kernel<D, NW>), g, t, 0, s, a);
+}
+
+template <int D>
+static hipError_t launch_fwd(AttnArgs a, NoiseShape shape, bool stream_noise, hipStream_t s) {
+    const int rows = shape == NoiseShape::Wide ? 256 : 128;
+    a.n_qtiles = (int)(((int64_t)a.Sq + rows - 1) / rows);
     const int64_t grid = (int64_t)a.n_qtiles * a.B * a.Hq;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    if (a.n16) hipLaunchKernelGGL((attn_fwd_half_noise_kernel<D, NW>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
-    else hipLaunchKernelGGL((attn_fwd_kernel<D, NW, true>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    const dim3 g((unsigned)grid);
+    if (shape == NoiseShape::Wide) launch_rows<D, 8>(a, stream_noise, g, s);
+    else if (shape == NoiseShape::Narrow) launch_rows<D, 4>(a, stream_noise, g, s);
+    else if (a.n16) hipLaunchKernelGGL((attn_fwd_split_kernel<D, true, false>), g, dim3(512), 0, s, a);
+    else if (stream_noise) hipLaunchKernelGGL((attn_fwd_split_kernel<D, false, true>), g, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((attn_fwd_split_kernel<D, false, false>), g, dim3(512), 0, s, a);
     return hipGetLastError();
 }
 
@@ -477,16 +626,43 @@ int validate_attn(const trn_attn_desc* d, bool need_v) {
 }  // namespace trn
 
 namespace trn {
-// Workgroup shape of the forward kernel with score perturbation: 8 waves x 32 queries (one workgroup per CU; each K/V stage
-// is fetched from L2 once per 256 queries), or 4 waves x 32 (two per CU).  Unmasked, wide from one workgroup per CU.  Causal,
-// where workgroups differ in length: with head_dim 128 from 384 wide workgroups of at least six tiles per head; fewer tiles
-// waste too much of the last one, and head_dim 64 prefers the finer grid throughout.  us, narrow / wide: 32 heads of 128,
-// fp32 noise: 4096 keys 343 / 316, 3600 241 / 230, 3126 201 / 191, 2048 (256 workgroups) 124 / 122; fp16: 2 x 1501 87 / 80,
-// but 2560 (320) 122 / 135, 4 x 777 77 / 85, 8 x 512 55 / 63; 8 x 8 heads, 1448: 97 / 98.  Head_dim 64: 142 heads, 1559 keys
-// 161 / 181; 284 heads, 392 keys 38 / 51; 128 heads, 1448 keys 127 / 130; 48 heads, 2300 keys 148 / 144.
-static bool noise_kernel_wide(const trn_attn_desc* d) {
-    const int64_t n256 = ((int64_t)d->seq_q + 255) / 256, n_wide = n256 * d->batch * d->n_q_heads;
-    return d->causal ? d->head_dim == 128 && n256 >= 6 && n_wide >= 384 : n_wide >= 256;
+// Workgroup shape of the forward kernel with score perturbation (us; W = workgroups of 128 queries).
+//  Narrow  the general case: two workgroups of four waves per CU.
+//  Split   eight waves on 128 queries halve the longest walk of a causal triangle that fills the chip once at most, for a
+//          merge of 2 - 3 us.  Narrow / split: 32 heads of 128: 600 keys 22.7 / 22.3, 1250 43.0 / 39.8, 1501 (fp16) 46.4 /
+//          41.9, 1600 61.6 / 58.9, 1800 (fp16) 60.6 / 58.4; 8 heads 2489 64.8 / 57.0, 4000 (fp16) 96 / 82; 2 x 8 heads, 1500
+//          42.1 / 37.1; 16 heads of 64: 1100 (fp16) 26.8 / 22.4, 2500 (fp16) 55.5 / 43.1, 4034 (fp16) 115 / 90; 32 heads of
+//          64, 1100 29.9 / 27.9, 2000 76 / 72.  Not where many heads bring many short walks, which even out by themselves:
+//          40 heads of 128, 1200 keys (W = 400) 45.0 / 47.6, 64 heads, 700 (384) 26.6 / 33.7, 32 heads, 2048 (512) 109 / 125;
+//          71 heads of 64: 400 (284) 14.7 / 17.9, 700 (426) 21.6 / 26.6.  (A query tile may then hold queries that see no
+//          key of the second group's first tile only if it begins inside one: hence as many queries as keys.)
+//  Wide    256 queries per K/V stage.  Unmasked, from one workgroup per CU.  Causal, where workgroups differ in length:
+//          with head_dim 128 from 384 workgroups of at least six tiles per head; fewer waste too much of the last one, and
+//          head_dim 64 prefers the finer grid throughout.  Narrow / wide: 32 heads of 128: 4096 keys 257 / 244, 4096 (fp16)
+//          231 / 217, 3500 (fp16) 182 / 165, 3107 188 / 175, 3072 149 / 153, 2 x 1706 124 / 114, but 2560 (320) 107 / 117;
+//          6 x 8 heads, 2048 122 / 131; 71 heads of 64, 2048 151 / 158.
+static NoiseShape noise_shape(const trn_attn_desc* d) {
+    const int64_t bh = (int64_t)d->batch * d->n_q_heads, n128 = ((int64_t)d->seq_q + 127) / 128, W = n128 * bh;
+    const int64_t n256 = ((int64_t)d->seq_q + 255) / 256;
+    if (d->causal && d->seq_q == d->seq_kv) {
+        const bool split = d->head_dim == 128 ? (W <= 256 ? n128 >= 5 : bh <= 32 && n128 >= 9 && W < 512) : n128 >= 9 && W <= 512;
+        if (split) return NoiseShape::Split;
+    }
+    const bool wide = d->causal ? d->head_dim == 128 && n256 >= 6 && n256 * bh >= 384 : n256 * bh >= 256;
+    return wide ? NoiseShape::Wide : NoiseShape::Narrow;
+}
+
+// The non-temporal hint for the noise: its lines then don't push K, V and Q out of the L2s, and the last-level cache (256 MB)
+// is not filled with what it cannot keep until the statistics read it again.  For that the rows have to lie on whole lines
+// (elsewhere a line belongs to two row pieces and would be fetched twice) and the visible noise must be more than that cache
+// holds for the second pass.  us, forward + statistics, without / with: 32 heads of 128: 4096 keys 253 + 215 / 244 + 190, 2560
+// 114 + 102 / 107 + 94, 1792 (206 MB) 73 + 43 / 63 + 45; 71 heads of 64, 1536 83 + 73 / 77 + 70; but 1024 keys (67 MB) 35 + 21
+// / 36 + 25, and rows off the lines: 3107 keys 175 + 149 / 219 + 160.
+bool noise_streams(const trn_attn_desc* d, const void* noise, bool n16) {
+    if (!noise || n16 || (reinterpret_cast<uintptr_t>(noise) & 127u)) return false;
+    if ((d->noise_stride_s & 31) || (d->noise_stride_h & 31) || (d->noise_stride_b & 31)) return false;
+    const int64_t per_head = d->causal ? (int64_t)d->seq_q * (2 * (int64_t)d->seq_kv - d->seq_q) * 2 : (int64_t)d->seq_q * d->seq_kv * 4;
+    return (int64_t)d->batch * d->n_q_heads * per_head >= (int64_t)192 << 20;
 }
 }  // namespace trn
 
@@ -509,9 +685,10 @@ extern "C" const char* trn_attn_fwd_kernel_name(const trn_attn_desc* d, int32_t 
     if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0))
         return attn_decode_kernel_name(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
     if (!with_noise) return attn_fwd16_kernel_name(d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0));
-    const bool wide = noise_kernel_wide(d);
-    if (d128) return wide ? "trn::attn_fwd_kernel<128, 8, true>" : "trn::attn_fwd_kernel<128, 4, true>";
-    return wide ? "trn::attn_fwd_kernel<64, 8, true>" : "trn::attn_fwd_kernel<64, 4, true>";
+    const NoiseShape shape = noise_shape(d);       // (fp32 noise in the policy of the shape's usual size; the others have names of their own)
+    if (shape == NoiseShape::Split) return d128 ? "trn::attn_fwd_split_kernel<128, false, false>" : "trn::attn_fwd_split_kernel<64, false, false>";
+    if (d128) return shape == NoiseShape::Wide ? "trn::attn_fwd_kernel<128, 8, true>" : "trn::attn_fwd_kernel<128, 4, true>";
+    return shape == NoiseShape::Wide ? "trn::attn_fwd_kernel<64, 8, true>" : "trn::attn_fwd_kernel<64, 4, true>";
 }
 
 extern "C" int trn_attn_fwd_f16(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o,
@@ -687,11 +864,9 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     // Without score perturbation: the 16x16x32 kernel, in the workgroup shape its launcher's rule picks.
     if (!noise)
         return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0), s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
-    // With it: the shape of noise_kernel_wide().
-    const bool wide = noise_kernel_wide(d);
-#define TRN_LAUNCH(D_, NW_) launch_fwd<D_, NW_>(a, s)
-    if (d->head_dim == 128) e = wide ? TRN_LAUNCH(128, 8) : TRN_LAUNCH(128, 4);
-    else e = wide ? TRN_LAUNCH(64, 8) : TRN_LAUNCH(64, 4);
-#undef TRN_LAUNCH
+    // With it: the shape of noise_shape().
+    const NoiseShape shape = noise_shape(d);
+    const bool stream_noise = noise_streams(d, noise, n16);
+    e = d->head_dim == 128 ? launch_fwd<128>(a, shape, stream_noise, s) : launch_fwd<64>(a, shape, stream_noise, s);
     return e == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
 }
