@@ -5,8 +5,9 @@
 
 namespace trn {
 
-// LPR lanes per row (power of two <= 64), NV 16-byte vectors per lane.
-template <int LPR, int NV>
+// LPR lanes per row (power of two <= 64), NV 16-byte vectors per lane.  All of a row's loads are issued before the first is
+// waited for (with the squares summed in the same loop the compiler waited for each vector in turn); EARLY: gamma's too.
+template <int LPR, int NV, bool EARLY>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
     const half_t* x, const half_t* __restrict__ gamma, half_t* y,     // y may be x (in place): a row is read whole
                                                                      // into registers before any of it is written
@@ -23,13 +24,20 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     const half_t* xr = x + (int64_t)outer * x_outer + ((int64_t)inner + row_start) * ldx;
     half_t* yr = y + (int64_t)outer * y_outer + ((int64_t)inner + row_start) * ldy;
 
-    half8_t v[NV];
+    half8_t v[NV], g[NV];
     float ss = 0.f;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = (i * LPR + sub) * 8;
         if (c < cols) {
             v[i] = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(xr + c));   // streamed once: keep it out of the caches' way
+            if (EARLY && gamma) g[i] = *reinterpret_cast<const half8_t*>(gamma + c);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (i * LPR + sub) * 8;
+        if (c < cols) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) { float f = (float)v[i][e]; ss += f * f; }
         }
@@ -44,9 +52,9 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
         if (c < cols) {
             half8_t o;
             if (gamma) {
-                half8_t g = *reinterpret_cast<const half8_t*>(gamma + c);
+                if (!EARLY) g[i] = *reinterpret_cast<const half8_t*>(gamma + c);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) o[e] = (half_t)((float)g[e] * ((float)v[i][e] * rstd));
+                for (int e = 0; e < 8; ++e) o[e] = (half_t)((float)g[i][e] * ((float)v[i][e] * rstd));
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[e] = (half_t)((float)v[i][e] * rstd);
@@ -56,16 +64,32 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
     }
 }
 
-template <int LPR, int NV>
-static hipError_t launch(const void* x, const void* gamma, void* y, int64_t n_rows, int64_t inner_rows,
+template <int LPR, int NV, bool EARLY>
+static hipError_t launch_form(const void* x, const void* gamma, void* y, int64_t n_rows, int64_t inner_rows,
                          int cols, int64_t xo, int64_t ldx, int64_t yo, int64_t ldy, int64_t row_start,
                          float eps, hipStream_t s) {
     constexpr int RPB = 256 / LPR;
     dim3 grid((unsigned)((n_rows + RPB - 1) / RPB));
-    hipLaunchKernelGGL((rmsnorm_kernel<LPR, NV>), grid, dim3(256), 0, s, (const half_t*)x,
+    hipLaunchKernelGGL((rmsnorm_kernel<LPR, NV, EARLY>), grid, dim3(256), 0, s, (const half_t*)x,
                        (const half_t*)gamma, (half_t*)y, n_rows, inner_rows, cols, xo, ldx, yo, ldy,
                        row_start, eps);
     return hipGetLastError();
+}
+
+// gamma early or late: early is one memory latency instead of two for a row, late leaves the queue to the rows themselves, which
+// matters once the resident waves ask for more than the chip takes at a time.  us, before / late / early: 16 x 4096 5.1 / 4.6 /
+// 3.9, 396 x 5560 10.4 / 6.7 / 5.4, 300 x 8192 13.3 / 7.9 / 6.2, 1929 x 3216 8.6 / 6.7 / 6.4, 3072 x 4096 11.1 / 9.6 / 8.8, 3400 x
+// 4096 11.7 / 10.7 / 12.2, 4096 x 4096 12.8 / 11.4 / 12.5; 1900 x 8192 17.2 / 12.3 / 11.2, 3072 x 6000 17.8 / 14.7 / 14.3, 2500 x
+// 8192 19.7 / 16.4 / 18.2; 9000 x 2048 15.9 / 15.8 / 14.5; 16000 x 1024 12.8 / 13.1 / 12.7, 8000 x 1024 6.6 / 6.3 / 6.7; 12000 x
+// 512 6.8 / 6.8 / 6.5.
+template <int LPR, int NV>
+static hipError_t launch(const void* x, const void* gamma, void* y, int64_t n_rows, int64_t inner_rows,
+                         int cols, int64_t xo, int64_t ldx, int64_t yo, int64_t ldy, int64_t row_start,
+                         float eps, hipStream_t s) {
+    const int64_t bytes = n_rows * cols * 2;
+    const bool early = NV == 2 ? n_rows <= 3072 || n_rows > 9000 : NV == 8 ? bytes <= 26000000 : NV == 16 ? bytes <= 37000000 : NV < 8;
+    if (early) return launch_form<LPR, NV, true>(x, gamma, y, n_rows, inner_rows, cols, xo, ldx, yo, ldy, row_start, eps, s);
+    return launch_form<LPR, NV, false>(x, gamma, y, n_rows, inner_rows, cols, xo, ldx, yo, ldy, row_start, eps, s);
 }
 
 }  // namespace trn
