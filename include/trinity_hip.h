@@ -111,6 +111,17 @@ int trn_attn_fwd_f16(const trn_attn_desc* desc, const void* q, const void* k, co
                      const float* noise, float* lse_pert, void* stream);
 
 /*
+ * QKNorm attention (ref_rms.py:217-228): per-head RMSNorm of K (weight gamma_k, nullable fp16 [head_dim]; k_eps) and of Q (by
+ * desc, weight gamma_q) over head_dim, then trn_attn_fwd_f16.  K is left as it is.  Where few query tiles read the keys they
+ * are normalised on their way into that launch; elsewhere once, by a launch of its own, into
+ *   k_norm     trn_attn_qknorm_workspace_bytes(desc) bytes of device memory, 16-byte aligned; may be NULL if that is 0.
+ * The batches of K must then lie n_kv_heads * k_stride_h apart.
+ */
+int64_t trn_attn_qknorm_workspace_bytes(const trn_attn_desc* desc);
+int trn_attn_qknorm_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v, void* o,
+                        const void* gamma_q, const void* gamma_k, float k_eps, void* k_norm, void* stream);
+
+/*
  * trn_attn_fwd_f16 with a caller-provided workspace.  In the reference every cross-kernel intermediate is a
  * caller-allocated tensor passed to `forward` (C, C_exp, C_sum ... in vanilla_llama_benchmark.py:42-77, zero-filled
  * by the driver, :237-240); this is that convention for the one intermediate these kernels have.  For decode shapes

@@ -19,7 +19,7 @@ EXPORTS = (
     "trn_calibration_mfma", "trn_attn_workspace_bytes", "trn_attn_chunk_workspace_bytes", "trn_attn_fwd_ws_f16", "trn_linear_f16", "trn_gate_f16", "trn_attn_fwd_stats_f16",
     "trn_attn_fwd_noalloc_f16", "trn_attn_fwd_kernel_name", "trn_attn_colmeanstd_f16", "trn_attn_fwd_probs_f16",
     "trn_attn_fwd_stats_half_f16", "trn_attn_fwd_stats_ws_f16", "trn_attn_stats_workspace_bytes",
-    "trn_attn_key_scores_f16",
+    "trn_attn_key_scores_f16", "trn_attn_qknorm_f16", "trn_attn_qknorm_workspace_bytes",
 )
 
 
@@ -93,6 +93,10 @@ def load() -> C.CDLL:
     lib.trn_attn_chunk_workspace_bytes.argtypes = [C.POINTER(AttnDesc)]
     lib.trn_attn_fwd_ws_f16.restype = C.c_int
     lib.trn_attn_fwd_ws_f16.argtypes = [C.POINTER(AttnDesc), vp, vp, vp, vp, vp, vp, vp, vp, vp, C.c_int64, vp]
+    lib.trn_attn_qknorm_workspace_bytes.restype = C.c_int64
+    lib.trn_attn_qknorm_workspace_bytes.argtypes = [C.POINTER(AttnDesc)]
+    lib.trn_attn_qknorm_f16.restype = C.c_int
+    lib.trn_attn_qknorm_f16.argtypes = [C.POINTER(AttnDesc), vp, vp, vp, vp, vp, vp, f32, vp, vp]
     lib.trn_attn_fwd_noalloc_f16.restype = C.c_int
     lib.trn_attn_fwd_noalloc_f16.argtypes = [C.POINTER(AttnDesc), vp, vp, vp, vp, vp, vp, vp, vp, vp]
     lib.trn_attn_fwd_kernel_name.restype = C.c_char_p

@@ -13,6 +13,7 @@ struct AttnArgs {
     float c2, c3;  // scale*log2(e)/tau, log2(e)/tau     : perturbed scores  z2 = s*c2 + g*c3
     float q_eps;
     int causal, q_norm;
+    const half_t* gamma_k; float k_eps; int k_norm;     // decode kernel without noise only: the keys are normalised on arrival
     // decode kernel only: keys split over n_split workgroups per head, partial results and arrival counters in ws
     int n_split;
     int spread;    // decode kernel only: the query tiles of a head go to all XCDs
@@ -58,7 +59,8 @@ __device__ __forceinline__ half4_t half_noise4(const uint3_t& d, int shift) {
 int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                  const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
-                 bool n16 = false, bool s16 = false, bool any_pitch = false);
+                 bool n16 = false, bool s16 = false, bool any_pitch = false, bool k_norm = false, const void* gamma_k = nullptr,
+                 float k_eps = 0.f);
 
 // The checks of attn_colstats by themselves, for a caller that launches something else before it.
 int attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
@@ -77,6 +79,8 @@ bool noise_streams(const trn_attn_desc* d, const void* noise, bool n16);
 // (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.
 bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+// ... and where that launch, without a workspace, also normalises the keys if asked to (args.k_norm).
+bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);
 const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 // Bytes of workspace with which launch_attn_decode splits the keys of this problem over several workgroups (0: it would not).
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);

@@ -30,11 +30,14 @@ template <int DV> __device__ __forceinline__ int swzv(int r) {
 // all of K, but streams only its DV = D / DS columns of V and writes those columns of O).  One CU pulls 40 - 55 GB/s
 // whatever its waves ask for, and with one workgroup per head that rate is what the kernel's time is made of; more
 // workgroups per head without anything to hand over between them means fewer bytes through each CU.
-// NZ: 0 no score perturbation, 1 fp32 noise, 2 fp16 noise
+// NZ: 0 no score perturbation, 1 fp32 noise, 2 fp16 noise, 3 none, and scores of normalised keys: a key's reciprocal root mean
+// square multiplies its scores in fp32, and gamma_k is multiplied into the queries before they are rounded to fp16.  (Normalising
+// the rows themselves costs ten times the vector instructions: us, a norm launch before / rows / scores: 16 heads of 64, 137 keys
+// 9.2 / 7.0 / 6.8, 500 11.1 / 9.5 / 8.5; 32 heads of 128, 128 keys 11.3 / 9.5 / 9.2, 250 13.5 / 15.4 / 11.5.)
 template <int D, int DS, int NZ>
 __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
-    constexpr bool NOISE = NZ != 0, N16 = NZ == 2;
+    constexpr bool NOISE = NZ == 1 || NZ == 2, N16 = NZ == 2, KNORM = NZ == 3;
     constexpr int DV = D / DS;    // columns of V / O this workgroup owns
     constexpr int NS = D / 16;    // k-steps of S^T = K Q^T
     constexpr int NSV = DV / 16;  // (2 key halves) x (DV/32) MFMAs of P V
@@ -98,6 +101,20 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #pragma unroll
         for (int ks = 0; ks < NS; ++ks) qB[ks] = *reinterpret_cast<const half8_t*>(qp + ks * 16);
     }
+    // (the norms' weights along with Q: one memory latency)
+    half8_t gq[NS], gk[KNORM ? NS : 1];
+    const bool use_gq = a.q_norm && a.gamma_q;
+    if (use_gq) {
+#pragma unroll
+        for (int ks = 0; ks < NS; ++ks) gq[ks] = *reinterpret_cast<const half8_t*>(a.gamma_q + ks * 16 + 8 * h);
+    }
+    if constexpr (KNORM) {
+#pragma unroll
+        for (int ks = 0; ks < NS; ++ks) {
+            if (a.gamma_k) gk[ks] = *reinterpret_cast<const half8_t*>(a.gamma_k + ks * 16 + 8 * h);
+            else gk[ks] = half8_t{1, 1, 1, 1, 1, 1, 1, 1};
+        }
+    }
     // ---- K: block rows straight into registers as A operands (lane: key c of the block, columns ks*16 + 8h ..)
     const __amdgpu_buffer_rsrc_t krs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(a.k + b * a.kb + kvh * a.kh), 0, (int)(((int64_t)(a.Skv - 1) * a.ks + D) * 2), 0x00020000);
@@ -128,6 +145,30 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #pragma unroll
             for (int ks = 0; ks < NS; ++ks)
                 ka[ks] = *reinterpret_cast<const half8_t*>(&kt[c * D + (((2 * ks + h) ^ swz<D>(c)) << 3)]);
+        }
+    };
+    // KNORM: the reciprocal root mean squares of a block's keys, through LDS from the lanes that hold the rows (lane and
+    // lane^32 one half each) to the lanes that hold their scores
+    __shared__ __attribute__((aligned(256))) float Kr[KNORM ? DNW * 32 : 4];
+    float gk_unit = 1.f;       // the power of two that gamma_k was divided by
+    auto key_norms = [&](const half8_t (&ka)[NS]) __attribute__((always_inline)) {
+        float ss[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < NS; ++ks)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2) {
+                const half2_t p = {ka[ks][e], ka[ks][e + 1]};
+                ss[e / 2] = __builtin_amdgcn_fdot2(p, p, ss[e / 2], false);
+            }
+        const float rstd = 1.0f / __builtin_sqrtf(half_sum((ss[0] + ss[1]) + (ss[2] + ss[3])) / (float)D + a.k_eps);
+        Kr[wave * 32 + c] = rstd * gk_unit;                // (both lanes of a row write the same)
+    };
+    auto scale_scores = [&](float16_t& s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const float4_t w = *reinterpret_cast<const float4_t*>(&Kr[wave * 32 + 8 * r4 + 4 * h]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[r4 * 4 + e] *= w[e];
         }
     };
     // ---- V: block rows global -> LDS, chunk c of row r stored at c ^ swz<D>(r); load n covers rows n*RPI + lane/CPR
@@ -207,8 +248,10 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] = 0.f;
         k_operands(kc);
+        if constexpr (KNORM) key_norms(kc);
 #pragma unroll
         for (int ks = 0; ks < NS; ++ks) s = mfma32(kc[ks], qB[ks], s);
+        if constexpr (KNORM) scale_scores(s);
         if constexpr (NOISE) fetch_k(blk + DNW, kc);
         // mask (wave-uniform test), block max, running max, probabilities
         const bool masked = (key0 + 32 > a.Skv) || (a.causal && key0 + 31 > q0 + off);
@@ -290,22 +333,36 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     TRN_FETCH_V(blk0 + wave, Vs0);
     if constexpr (NOISE) fetch_noise(blk0 + wave, g0);
     // (the first K / V requests are on their way before Q is waited for: one memory latency instead of two)
-    if (a.q_norm) {
-        float ss = 0.f;
+    if (a.q_norm || KNORM) {
+        if constexpr (KNORM) {
+            // gamma_k over the power of two above its largest element, so that no query grows by it
+            float top = 0.f;
 #pragma unroll
-        for (int ks = 0; ks < NS; ++ks)
+            for (int ks = 0; ks < NS; ++ks) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) { float f = (float)qB[ks][e]; ss += f * f; }
-        ss = half_sum(ss);
-        const float rstd = 1.0f / __builtin_sqrtf(ss / (float)D + a.q_eps);
+                for (int e = 0; e < 8; ++e) top = fmaxf(top, __builtin_fabsf((float)gk[ks][e]));
+            }
+            top = half_max(top);
+            if (top > 0.f && top < INFINITY) gk_unit = __builtin_ldexpf(1.f, __builtin_amdgcn_frexp_expf(top));
+        }
+        float rstd = 1.f;
+        if (a.q_norm) {
+            float ss = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < NS; ++ks)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) { float f = (float)qB[ks][e]; ss += f * f; }
+            ss = half_sum(ss);
+            rstd = 1.0f / __builtin_sqrtf(ss / (float)D + a.q_eps);
+        }
+        const float per_unit = 1.f / gk_unit;
 #pragma unroll
         for (int ks = 0; ks < NS; ++ks) {
-            half8_t gq;
-            if (a.gamma_q) gq = *reinterpret_cast<const half8_t*>(a.gamma_q + ks * 16 + 8 * h);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 float y = (float)qB[ks][e] * rstd;
-                if (a.gamma_q) y = (float)gq[e] * y;
+                if (use_gq) y = (float)gq[ks][e] * y;
+                if constexpr (KNORM) y *= (float)gk[ks][e] * per_unit;
                 qB[ks][e] = (half_t)y;
             }
         }
@@ -471,7 +528,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     // sum over queries is in-lane plus one exchange with lane^32, and a block's 32 sums are one 128-byte store.
     // (One query tile only.  Not with the keys split over workgroups -- the statistics need the normalisers of the whole head; the column
     // shares of a head all have them, and take every DS-th round of blocks of the sweep each.)
-    if (a.col_sum || a.col_sumsq || a.probs) {
+    if (!KNORM && (a.col_sum || a.col_sumsq || a.probs)) {
         __syncthreads();                                   // every thread has read the merge arrays
         if (dg == 0) st_l[0][q] = NOISE ? ms2 + fast_log2(L2) : mstar + fast_log2(L);     // log2 domain
         __syncthreads();
@@ -593,6 +650,12 @@ bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head
     return tiles <= 256 || (tiles < 512 && (noise || (head_dim == 64 && seq_kv >= 1024)));
 }
 
+// Each tile of 32 queries normalises the keys it reads, some 0.25 us per 256 keys against 3 - 5 us for a launch: up to 2048.
+// us, launch / here: 8 heads of 128, 1024 tokens 18.5 / 17.0; 2 x 8, 394 14.0 / 11.9.
+bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
+    return attn_decode_suits(batch, n_q_heads, seq_q, seq_kv, head_dim, false) && seq_kv <= 2048;
+}
+
 // Where the query tiles of a head go.  On one XCD they share K and V in its L2, but fewer than eight heads, or a number that
 // leaves the last eight short, then leave XCDs idle: from the point where the others have more than a workgroup per CU the
 // tiles are dealt to all eight instead.  us, together / spread: one head of 128, 845 queries and keys 30.0 / 9.3, 3213 132 /
@@ -634,7 +697,7 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)grid), t(DNW * 64);
 #define TRN_DEC(D_, DS_, N_) hipLaunchKernelGGL((attn_decode_kernel<D_, DS_, N_>), g, t, 0, stream, a)
-#define TRN_DEC_NZ(D_, DS_) do { if (!a.noise) TRN_DEC(D_, DS_, 0); else if (a.n16) TRN_DEC(D_, DS_, 2); else TRN_DEC(D_, DS_, 1); } while (0)
+#define TRN_DEC_NZ(D_, DS_) do { if (a.k_norm) TRN_DEC(D_, DS_, 3); else if (!a.noise) TRN_DEC(D_, DS_, 0); else if (a.n16) TRN_DEC(D_, DS_, 2); else TRN_DEC(D_, DS_, 1); } while (0)
     if (head_dim == 128) { if (ds == 4) TRN_DEC_NZ(128, 4); else if (ds == 2) TRN_DEC_NZ(128, 2); else TRN_DEC_NZ(128, 1); }
     else { if (ds == 2) TRN_DEC_NZ(64, 2); else TRN_DEC_NZ(64, 1); }
 #undef TRN_DEC_NZ

@@ -806,10 +806,41 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);
 }
 
+// Whether the attention launch takes the norm of the keys along (it needs no workspace then).
+static bool norms_keys(const trn_attn_desc* d) {
+    return trn::attn_decode_norms_keys(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
+}
+
+extern "C" int64_t trn_attn_qknorm_workspace_bytes(const trn_attn_desc* d) {
+    using namespace trn;
+    if (!d || validate_attn(d, true) != TRN_OK || norms_keys(d)) return 0;
+    return (int64_t)d->batch * d->n_kv_heads * d->seq_kv * d->head_dim * 2;
+}
+
+extern "C" int trn_attn_qknorm_f16(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o,
+                                   const void* gamma_q, const void* gamma_k, float k_eps, void* k_norm, void* stream) {
+    using namespace trn;
+    if (!d || !k) return TRN_E_NULL;
+    const int st = validate_attn(d, true);
+    if (st != TRN_OK) return st;
+    if (!aligned16(k) || (gamma_k && !aligned16(gamma_k))) return TRN_E_ALIGN;
+    if (norms_keys(d))
+        return attn_forward(d, q, k, v, o, nullptr, gamma_q, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream, nullptr,
+                            false, false, false, true, gamma_k, k_eps);
+    if (!k_norm) return TRN_E_NULL;
+    if (d->batch > 1 && d->k_stride_b != d->n_kv_heads * d->k_stride_h) return TRN_E_STRIDE;
+    const int64_t rows = d->seq_kv, D = d->head_dim;
+    if (const int e = trn_rmsnorm_f16(k, gamma_k, k_norm, (int64_t)d->batch * d->n_kv_heads, rows, D, d->k_stride_h, d->k_stride_s,
+                                      rows * D, D, 0, k_eps, stream); e != TRN_OK) return e;
+    trn_attn_desc n = *d;
+    n.k_stride_b = d->n_kv_heads * rows * D; n.k_stride_h = rows * D; n.k_stride_s = D;
+    return attn_forward(&n, q, k_norm, v, o, nullptr, gamma_q, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream);
+}
+
 int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                              int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs,
-                             bool n16, bool s16, bool any_pitch) {
+                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps) {
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
     if (!d || !q || !k || !v || !o) return TRN_E_NULL;
     if (noise && !lse_pert) return TRN_E_NULL;
@@ -843,6 +874,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     const float tau = noise ? d->tau : 1.f;
     a.c2 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.q_eps = d->q_norm_eps; a.causal = d->causal ? 1 : 0; a.q_norm = d->q_norm ? 1 : 0;
+    a.gamma_k = (const half_t*)gamma_k; a.k_eps = k_eps; a.k_norm = k_norm ? 1 : 0;
     a.n_split = 1; a.spread = 0; a.ws = nullptr; a.col_sum = col_sum; a.col_sumsq = col_sumsq; a.probs = probs; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
     // K/V tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base
     // (with room for the blocks the pipelines request past the end, which must stay representable to read as zeros)

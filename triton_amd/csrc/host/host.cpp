@@ -331,18 +331,21 @@ bool f_qknorm_forward(Args a, Py_ssize_t n) {             // workspaces, scale |
     NEED(k.contiguous(), "K: expected a contiguous tensor");
     NEED(k.cuda, "K: expected a GPU tensor");
     const double eps = num(a[3]);
-    const at::Tensor kn_ws = workspace(w, "k_norm", {k.s[0], k.s[1], k.s[2], k.s[3]}, k.dt, k.dev);
-    const View kn = view_of(kn_ws, "k_norm");
-    trn_attn_desc d = attn_desc(q, kn, v, o, scale_of(a[1], k.s[3]), flag(a[2]));
+    trn_attn_desc d = attn_desc(q, k, v, o, scale_of(a[1], k.s[3]), flag(a[2]));
     d.q_norm = 1; d.q_norm_eps = (float)eps;
     const OptView gq = opt(a[9], "gamma_q");
     if (gq.given) {
         dev_half(gq.v, "gamma_q");
         NEED(gq.v.dim == 1 && gq.v.s[0] == d.head_dim, "gamma_q: expected (head_dim,)");
     }
-    const int64_t H = k.s[0] * k.s[1], S = k.s[2], D = k.s[3];
-    head_rmsnorm_call(make(k, k.p, {H, S, D}, {S * D, D, 1}), opt(a[8], "gamma_k"), make(kn, kn.p, {H, S, D}, {S * D, D, 1}), eps, 0);
-    CALL(trn_attn_fwd_f16, &d, q.p, kn.p, v.p, o.p, nullptr, gq.p(), nullptr, nullptr, stream_of(q));
+    const OptView gk = opt(a[8], "gamma_k");
+    if (gk.given) {
+        dev_half(gk.v, "gamma");
+        NEED(gk.v.dim == 1 && gk.v.s[0] == d.head_dim, "gamma: expected (head_dim,)");
+    }
+    at::Tensor kn;
+    if (trn_attn_qknorm_workspace_bytes(&d) > 0) kn = workspace(w, "k_norm", {k.s[0], k.s[1], k.s[2], k.s[3]}, k.dt, k.dev);
+    CALL(trn_attn_qknorm_f16, &d, q.p, k.p, v.p, o.p, gq.p(), gk.p(), (float)eps, kn.defined() ? kn.data_ptr() : nullptr, stream_of(q));
     return true;
 }
 

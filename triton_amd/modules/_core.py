@@ -225,8 +225,8 @@ class Attention(FusedModule):
 
 class QKNormAttention(FusedModule):
     """Per-head RMSNorm of Q and K over head_dim, then attention (ref_rms.py:217-228).
-    K is normalised once into a workspace (it is shared by every query head); the Q norm is
-    fused into the attention kernel's prologue."""
+    The Q norm is fused into the attention kernel's prologue.  K is normalised once into a workspace (it is shared by
+    every query head), or, where few query tiles read it, within the attention launch."""
     TENSOR_PARAMS = ["K", "O", "Q", "V", "gamma_k", "gamma_q"]
 
     def __init__(self, scale: Optional[float] = None, causal: bool = True, eps: float = 1e-5):
@@ -240,10 +240,8 @@ class QKNormAttention(FusedModule):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
         if not k.is_contiguous():
             raise ValueError("K: expected a contiguous tensor")
-        B, Hkv, Skv, D = k.shape
-        kn = self._workspace("k_norm", k.shape, k.dtype, k.device)
-        ops.head_rmsnorm(k.view(B * Hkv, Skv, D), gamma_k, kn.view(B * Hkv, Skv, D), self.eps)
-        ops.attention(q, kn, v, o, _scale(self.scale, D), self.causal, q_norm=True, gamma_q=gamma_q, q_eps=self.eps)
+        ops.qknorm_attention(q, k, v, o, _scale(self.scale, k.shape[3]), self.causal, gamma_q, gamma_k, self.eps,
+                             lambda: self._workspace("k_norm", k.shape, k.dtype, k.device))
 
 
 class KeyFormerAttention(FusedModule):

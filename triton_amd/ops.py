@@ -8,7 +8,7 @@ returns None.  Nothing here allocates device memory.
 from __future__ import annotations
 
 import ctypes as C
-from typing import Optional
+from typing import Callable, Optional
 
 import torch
 
@@ -141,6 +141,21 @@ def attention(q, k, v, o, scale: float, causal: bool, lse: Optional[torch.Tensor
     st = _lib.load().trn_attn_fwd_noalloc_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(gamma_q),
                                               _ptr(noise), _ptr(lse_pert), _stream(q))
     _lib.check("trn_attn_fwd_noalloc_f16", st)
+
+
+def qknorm_attention(q, k, v, o, scale: float, causal: bool, gamma_q: Optional[torch.Tensor], gamma_k: Optional[torch.Tensor],
+                     eps: float, k_norm: Callable[[], torch.Tensor]) -> None:
+    """Attention of the RMS-normalised q and k (over head_dim, weights gamma_q and gamma_k), k contiguous.  k_norm gives an
+    fp16 workspace of k's shape; it is asked for one where the keys are normalised by a launch of their own."""
+    d = _attn_desc(q, k, v, o, scale, causal, True, eps, None, 1.0)
+    for t, n in ((gamma_q, "gamma_q"), (gamma_k, "gamma")):
+        if t is not None:
+            _dev_half(t, n)
+            _need(t.shape == (q.shape[3],), f"{n}: expected (head_dim,)")
+    lib = _lib.load()
+    kn = k_norm() if lib.trn_attn_qknorm_workspace_bytes(C.byref(d)) > 0 else None
+    st = lib.trn_attn_qknorm_f16(C.byref(d), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(gamma_q), _ptr(gamma_k), float(eps), _ptr(kn), _stream(q))
+    _lib.check("trn_attn_qknorm_f16", st)
 
 
 def attention_kernel_name(q, k, v, o, scale: float, causal: bool, with_noise: bool = False) -> str:
