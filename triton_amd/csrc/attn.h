@@ -55,6 +55,39 @@ __device__ __forceinline__ half4_t half_noise4(const uint3_t& d, int shift) {
 }
 #endif
 
+// A wave's per-key sums, 16 per lane over the lane's queries, added up over the 32 lanes of each half through 4 KB of LDS:
+// lane 2k + i gets key number k of the wave's 32 from 16 lanes (each key starting at another one: no bank conflicts) and
+// adds its neighbour's.  (In registers, five exchanges of all 16 sums and a division per sum and lane behind them took
+// 1 - 2 us of a launch.)
+// (lo, hi: the first and the second 2 KB)
+__device__ __forceinline__ void put_sums(const float (&v)[16], float* lo, float* hi, int lane) {
+#pragma unroll
+    for (int r = 0; r < 8; ++r) { lo[r * 64 + lane] = v[r]; hi[r * 64 + lane] = v[8 + r]; }
+}
+__device__ __forceinline__ float key_sum(const float* lo, const float* hi, int lane) {
+    const float* area = lane < 32 ? lo : hi - 512;
+    const int kh = (lane >> 1) & 1, r = lane >> 2, part = lane & 1;        // the key's half kh and number r of 16
+    float x[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) x[i] = area[r * 64 + kh * 32 + part * 16 + ((i + r) & 15)];
+#pragma unroll
+    for (int n = 8; n >= 1; n >>= 1)                                       // (as a tree: a chain's rounding is larger)
+#pragma unroll
+        for (int i = 0; i < n; ++i) x[i] += x[i + n];
+    return x[0] + __shfl_xor(x[0], 1, 64);
+}
+// The key, of the block's 32, that a lane has from key_sum.
+__device__ __forceinline__ int key_of_sum(int lane) {
+    const int kh = (lane >> 1) & 1, r = lane >> 2;
+    return 8 * (r / 4) + 4 * kh + (r % 4);
+}
+// (fp16: the fp32 value rounded once, as a copy into the caller's tensor would)
+__device__ __forceinline__ void store_stat(float* out, int s16, int64_t at, float v) {
+    if (!out) return;
+    if (s16) reinterpret_cast<half_t*>(out)[at] = (half_t)v;
+    else out[at] = v;
+}
+
 // Checks, argument block and kernel choice behind every attention entry point of the C ABI.
 int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                  const void* gamma_q, const float* noise, float* lse_pert, void* workspace,

@@ -40,37 +40,11 @@ struct ColArgs {
                     // (into out_sum / out_sumsq) instead of the two sums
 };
 
-__device__ __forceinline__ void store_stat(const ColArgs& a, float* out, int64_t at, float v) {
-    if (!out) return;
-    if (a.s16) reinterpret_cast<half_t*>(out)[at] = (half_t)v;
-    else out[at] = v;
-}
-
-// A wave's per-key sums, 16 per lane over the lane's queries, added up over the 32 lanes of each half through 4 KB of LDS:
-// lane 2k + i gets key number k of the wave's 32 from 16 lanes (each key starting at another one: no bank conflicts) and
-// adds its neighbour's.  (In registers, five exchanges of all 16 sums and a division per sum and lane behind them took
-// 1 - 2 us of a launch.)
-__device__ __forceinline__ void put_sums(const float (&v)[16], float* area, int lane) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) area[r * 64 + lane] = v[r];
-}
-__device__ __forceinline__ float key_sum(const float* area, int lane) {
-    const int kh = (lane >> 1) & 1, r = lane >> 2, part = lane & 1;        // key 2r + kh of the wave: half kh, number r of 16
-    float x[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) x[i] = area[r * 64 + kh * 32 + part * 16 + ((i + r) & 15)];
-#pragma unroll
-    for (int n = 8; n >= 1; n >>= 1)                                       // (as a tree: a chain's rounding is larger)
-#pragma unroll
-        for (int i = 0; i < n; ++i) x[i] += x[i + n];
-    return x[0] + __shfl_xor(x[0], 1, 64);
-}
-
 // The end of both kernels: x, y = the sums of the lane's key (key_sum's order), turned into mean and deviation if wanted,
 // and stored by the even lanes.
 template <bool SQ>
 __device__ __forceinline__ void finish_columns(const ColArgs& a, float x, float y, int64_t obase, int wkey0, int lane) {
-    const int kh = (lane >> 1) & 1, r = lane >> 2, key = wkey0 + 8 * (r / 4) + 4 * kh + (r % 4);
+    const int key = wkey0 + key_of_sum(lane);
     if (SQ && a.mean_std) {
         // n = queries that see this key: all of them, or under a causal mask those from key - (Skv - Sq) on
         const float n = (float)(a.causal ? a.Sq - max(0, key - (a.Skv - a.Sq)) : a.Sq);
@@ -82,8 +56,8 @@ __device__ __forceinline__ void finish_columns(const ColArgs& a, float x, float 
         x = mean;
     }
     if ((lane & 1) == 0 && key < a.Skv) {
-        store_stat(a, a.out_sum, obase + key, x);
-        if (SQ) store_stat(a, a.out_sumsq, obase + key, y);
+        store_stat(a.out_sum, a.s16, obase + key, x);
+        if (SQ) store_stat(a.out_sumsq, a.s16, obase + key, y);
     }
 }
 
@@ -305,11 +279,11 @@ __global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArg
     // (the transposing areas are the waves' own: only the other group's reads and writes need a barrier)
     const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));     // (the lane, not kept over the walk)
     auto total = [&](const float (&v)[16]) __attribute__((always_inline)) {
-        put_sums(v, nsw, ln);
-        if constexpr (NG == 1) return key_sum(nsw, ln);
+        put_sums(v, nsw, nsw + 512, ln);
+        if constexpr (NG == 1) return key_sum(nsw, nsw + 512, ln);
         else {
             __syncthreads();
-            const float x = grp == 0 ? key_sum(nsw, ln) + key_sum(nsw + 4 * 1024, ln) : 0.f;
+            const float x = grp == 0 ? key_sum(nsw, nsw + 512, ln) + key_sum(nsw + 4 * 1024, nsw + 4 * 1024 + 512, ln) : 0.f;
             if constexpr (SQ) __syncthreads();
             return x;
         }
@@ -524,10 +498,10 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
     __syncthreads();                        // ... by everybody
     float* area = reinterpret_cast<float*>(D == 128 || wave < 2 ? Qs0 : Qs1) + (D == 128 ? wave : wave & 1) * 1024;
     const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));     // (the lane, not kept over the walk)
-    put_sums(s1, area, ln);
-    const float x = key_sum(area, ln);
+    put_sums(s1, area, area + 512, ln);
+    const float x = key_sum(area, area + 512, ln);
     float y = 0.f;
-    if constexpr (SQ) { put_sums(s2, area, ln); y = key_sum(area, ln); }
+    if constexpr (SQ) { put_sums(s2, area, area + 512, ln); y = key_sum(area, area + 512, ln); }
     finish_columns<SQ>(a, x, y, ((int64_t)b * a.Hq + head) * a.Skv, wkey0, ln);
     asm volatile("" : "+s"(again));
     } while (again != 0);

@@ -34,10 +34,17 @@ template <int DV> __device__ __forceinline__ int swzv(int r) {
 // square multiplies its scores in fp32, and gamma_k is multiplied into the queries before they are rounded to fp16.  (Normalising
 // the rows themselves costs ten times the vector instructions: us, a norm launch before / rows / scores: 16 heads of 64, 137 keys
 // 9.2 / 7.0 / 6.8, 500 11.1 / 9.5 / 8.5; 32 heads of 128, 128 keys 11.3 / 9.5 / 9.2, 250 13.5 / 15.4 / 11.5.)
+// 4, 5, 6: as 0, 1, 2 with key statistics on at most kept_blocks() key blocks per wave: the scores of a wave's blocks stay in its
+// registers until the row normalisers are final, and the statistics need no second sweep over the keys and the noise.  With
+// noise up to what the registers hold; without, the sums over the lanes cost what the sweep does from 1000 keys on.  Whole
+// decode steps with 8 / 32 new tokens, us, sweep -> kept, 71 heads of 64 with fp16 noise: 200 keys 31.5 -> 30.2 / 35.3 -> 33.4,
+// 1000 keys 37.1 -> 35.6 / 42.7 -> 40.0; 8 heads of 128: 15.1 -> 13.7 / 18.5 -> 16.0, 18.7 -> 17.4 / 22.2 -> 19.8; without noise
+// 200 keys 14.2 -> 13.4 / 16.6 -> 14.9, but 71 heads and 1000 keys 34.7 -> 35.3 / 37.9 -> 38.4.
+constexpr int kept_blocks(int d, int ds, bool noise) { return !noise ? 2 : d == 128 && ds == 1 ? 3 : 6; }
 template <int D, int DS, int NZ>
 __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
-    constexpr bool NOISE = NZ == 1 || NZ == 2, N16 = NZ == 2, KNORM = NZ == 3;
+    constexpr bool KEEP = NZ >= 4, NOISE = NZ % 4 == 1 || NZ % 4 == 2, N16 = NZ % 4 == 2, KNORM = NZ == 3;
     constexpr int DV = D / DS;    // columns of V / O this workgroup owns
     constexpr int NS = D / 16;    // k-steps of S^T = K Q^T
     constexpr int NSV = DV / 16;  // (2 key halves) x (DV/32) MFMAs of P V
@@ -231,8 +238,9 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     half8_t ka0[NS], ka1[NS];
 
     // One 32-key block whose K is in kc and whose V is in stage Vc; the next block's loads go to kn / Vn first.
+    // keep (KEEP only): the block's scores in the log2 domain, the perturbed ones with noise, -inf where masked.
     auto block = [&](int it, half8_t (&kc)[NS], half8_t (&kn)[NS], const half_t* Vc, half_t* Vn, noise_t (&gc)[4],
-                     noise_t (&gn)[4]) __attribute__((always_inline)) {
+                     noise_t (&gn)[4], float16_t& keep) __attribute__((always_inline)) {
         const int blk = blk0 + wave + it * DNW, key0 = blk * 32;
         // (with noise the registers are short: K is then single-buffered, refilled as soon as the scores are issued)
         if constexpr (!NOISE) fetch_k(blk + DNW, kn);
@@ -280,6 +288,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #pragma unroll
                 for (int r = 0; r < 16; ++r) z[r] = s[r] == -INFINITY ? -INFINITY : z[r];
             }
+            if constexpr (KEEP) keep = z;
             const float zmax = fmaxf(m2, half_max(max16(z)));
             if (zmax > -INFINITY) {
                 float sum = 0.f;
@@ -288,6 +297,10 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
                 l2 = l2 * fast_exp2(m2 - zmax) + sum;
                 m2 = zmax;
             }
+        }
+        if constexpr (KEEP && !NOISE) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) keep[r] = s[r] == -INFINITY ? -INFINITY : s[r] * a.c1;
         }
         const float smax = half_max(max16(s)) * a.c1;
         const float mnew = fmaxf(m, smax);
@@ -370,13 +383,32 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     // pin the arrival of Q here: left to the first MFMA in the loop, the compiler's wait would sit in the loop body
 #pragma unroll
     for (int ks = 0; ks < NS; ++ks) asm volatile("" ::"v"(qB[ks]));
-    for (int it = 0; it < nmine; it += 2) {
-        if constexpr (NOISE) {
-            block(it, ka0, ka0, Vs0, VSINGLE ? Vs0 : Vs1, g0, g1);
-            if (it + 1 < nmine) block(it + 1, ka0, ka0, VSINGLE ? Vs0 : Vs1, Vs0, g1, g0);
-        } else {
-            block(it, ka0, ka1, Vs0, VSINGLE ? Vs0 : Vs1, g0, g1);
-            if (it + 1 < nmine) block(it + 1, ka1, ka0, VSINGLE ? Vs0 : Vs1, Vs0, g1, g0);
+    auto even = [&](int it, float16_t& keep) __attribute__((always_inline)) {
+        if constexpr (NOISE) block(it, ka0, ka0, Vs0, VSINGLE ? Vs0 : Vs1, g0, g1, keep);
+        else block(it, ka0, ka1, Vs0, VSINGLE ? Vs0 : Vs1, g0, g1, keep);
+    };
+    auto odd = [&](int it, float16_t& keep) __attribute__((always_inline)) {
+        if constexpr (NOISE) block(it, ka0, ka0, VSINGLE ? Vs0 : Vs1, Vs0, g1, g0, keep);
+        else block(it, ka1, ka0, VSINGLE ? Vs0 : Vs1, Vs0, g1, g0, keep);
+    };
+    constexpr int KB = KEEP ? kept_blocks(D, DS, NOISE) : 1;
+    float16_t kept[KB];
+    if constexpr (KEEP) {
+        // (nested, so that a block's waits are sized on one path only)
+        auto walk = [&](auto&& self, auto at) __attribute__((always_inline)) {
+            constexpr int it = decltype(at)::value;
+            if constexpr (it < KB) {
+                if (it < nmine) {
+                    if constexpr (it % 2 == 0) even(it, kept[it]); else odd(it, kept[it]);
+                    self(self, std::integral_constant<int, it + 1>{});
+                }
+            }
+        };
+        walk(walk, std::integral_constant<int, 0>{});
+    } else {
+        for (int it = 0; it < nmine; it += 2) {
+            even(it, kept[0]);
+            if (it + 1 < nmine) odd(it + 1, kept[0]);
         }
     }
 #undef TRN_FETCH_V
@@ -522,13 +554,43 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
             if (dg == 1 && dsl == 0 && q0 + q < a.Sq) a.lse_pert[(int64_t)bh * a.Sq + q0 + q] = (ms2 + fast_log2(L2)) * kLn2;
         }
     }
-    // ---- column statistics (KeyFormer key scores, RoCo sums): a second sweep over this head's keys now that the
+    // ---- column statistics (KeyFormer key scores, RoCo sums), from the kept scores or by a second sweep over this head's keys now that the
     // row normalisers are final.  The score block is formed the other way round, S[query][key] -- the same two
     // register operands with their roles swapped -- so that a lane owns one KEY and holds 16 of the 32 queries: the
     // sum over queries is in-lane plus one exchange with lane^32, and a block's 32 sums are one 128-byte store.
     // (One query tile only.  Not with the keys split over workgroups -- the statistics need the normalisers of the whole head; the column
     // shares of a head all have them, and take every DS-th round of blocks of the sweep each.)
-    if (!KNORM && (a.col_sum || a.col_sumsq || a.probs)) {
+    if constexpr (KEEP) {
+        __syncthreads();                                   // every thread has read the merge arrays
+        if (dg == 0) st_l[0][q] = NOISE ? ms2 + fast_log2(L2) : mstar + fast_log2(L);     // log2 domain
+        __syncthreads();
+        const float lq = c < a.Sq ? st_l[0][c] : INFINITY;       // (lanes without a query add nothing)
+        // 4 KB of this wave's own for the sums of a block and, in two halves, for those of its squares
+        float* const area = reinterpret_cast<float*>(Kt) + wave * (D * 16);
+        float* const sq_lo = D == 128 ? area + 1024 : reinterpret_cast<float*>(Vs0) + wave * (DV * 16);
+        float* const sq_hi = D == 128 || DV == 64 ? sq_lo + 512 : reinterpret_cast<float*>(Vs1) + wave * (DV * 16);
+#pragma unroll
+        for (int it = 0; it < KB; ++it) {
+            if (it >= nmine || it % DS != dsl) continue;         // (the column shares take every DS-th block each)
+            float p[16], x, y = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) p[r] = kept[it][r] == -INFINITY ? 0.f : fast_exp2(kept[it][r] - lq);
+            put_sums(p, area, area + 512, lane);
+            if (a.col_sumsq) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) p[r] *= p[r];
+                put_sums(p, sq_lo, sq_hi, lane);
+                x = key_sum(area, area + 512, lane);
+                y = key_sum(sq_lo, sq_hi, lane);
+            } else x = key_sum(area, area + 512, lane);
+            const int key = (blk0 + wave + it * DNW) * 32 + key_of_sum(lane);
+            if ((lane & 1) == 0 && key < a.Skv) {
+                const int64_t at = (int64_t)bh * a.Skv + key;
+                store_stat(a.col_sum, a.s16, at, x);
+                store_stat(a.col_sumsq, a.s16, at, y);
+            }
+        }
+    } else if (!KNORM && (a.col_sum || a.col_sumsq || a.probs)) {
         __syncthreads();                                   // every thread has read the merge arrays
         if (dg == 0) st_l[0][q] = NOISE ? ms2 + fast_log2(L2) : mstar + fast_log2(L);     // log2 domain
         __syncthreads();
@@ -581,13 +643,8 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
             x = half_sum(x); y = half_sum(y);
             if (h == 0 && key < a.Skv) {
                 const int64_t at = (int64_t)bh * a.Skv + key;
-                if (a.s16) {        // (the fp32 value rounded once, as a copy into the caller's fp16 tensor would)
-                    if (a.col_sum) reinterpret_cast<half_t*>(a.col_sum)[at] = (half_t)x;
-                    if (a.col_sumsq) reinterpret_cast<half_t*>(a.col_sumsq)[at] = (half_t)y;
-                } else {
-                    if (a.col_sum) a.col_sum[at] = x;
-                    if (a.col_sumsq) a.col_sumsq[at] = y;
-                }
+                store_stat(a.col_sum, a.s16, at, x);
+                store_stat(a.col_sumsq, a.s16, at, y);
             }
         };
         const int first = dsl * DNW + wave;
@@ -656,6 +713,12 @@ bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int
     return attn_decode_suits(batch, n_q_heads, seq_q, seq_kv, head_dim, false) && seq_kv <= 2048;
 }
 
+// Whether the scores of a head's keys fit the registers of one workgroup, for key statistics without a second sweep.
+static bool decode_keeps(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
+    const int ds = decode_col_shares((int64_t)batch * n_q_heads, seq_q, seq_kv, head_dim);
+    return seq_q <= 32 && (seq_kv + 31) / 32 <= kept_blocks(head_dim, ds, noise) * DNW;
+}
+
 // Where the query tiles of a head go.  On one XCD they share K and V in its L2, but fewer than eight heads, or a number that
 // leaves the last eight short, then leave XCDs idle: from the point where the others have more than a workgroup per CU the
 // tiles are dealt to all eight instead.  us, together / spread: one head of 128, 845 queries and keys 30.0 / 9.3, 3213 132 /
@@ -697,7 +760,9 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     const dim3 g((unsigned)grid), t(DNW * 64);
 #define TRN_DEC(D_, DS_, N_) hipLaunchKernelGGL((attn_decode_kernel<D_, DS_, N_>), g, t, 0, stream, a)
-#define TRN_DEC_NZ(D_, DS_) do { if (a.k_norm) TRN_DEC(D_, DS_, 3); else if (!a.noise) TRN_DEC(D_, DS_, 0); else if (a.n16) TRN_DEC(D_, DS_, 2); else TRN_DEC(D_, DS_, 1); } while (0)
+    // (as the kernel deals them out: blocks of 32 keys to the eight waves in turn; the un-reduced probabilities come from the sweep)
+    const bool keep = decode_keeps(a.B, a.Hq, a.Sq, a.Skv, head_dim, a.noise != nullptr) && a.n_split == 1 && (a.col_sum || a.col_sumsq) && !a.probs;
+#define TRN_DEC_NZ(D_, DS_) do { if (keep) { if (!a.noise) TRN_DEC(D_, DS_, 4); else if (a.n16) TRN_DEC(D_, DS_, 6); else TRN_DEC(D_, DS_, 5); } else if (a.k_norm) TRN_DEC(D_, DS_, 3); else if (!a.noise) TRN_DEC(D_, DS_, 0); else if (a.n16) TRN_DEC(D_, DS_, 2); else TRN_DEC(D_, DS_, 1); } while (0)
     if (head_dim == 128) { if (ds == 4) TRN_DEC_NZ(128, 4); else if (ds == 2) TRN_DEC_NZ(128, 2); else TRN_DEC_NZ(128, 1); }
     else { if (ds == 2) TRN_DEC_NZ(64, 2); else TRN_DEC_NZ(64, 1); }
 #undef TRN_DEC_NZ

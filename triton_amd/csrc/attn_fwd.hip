@@ -794,7 +794,7 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     const bool n16 = noise && noise_half, s16 = out_half != 0;
     const int64_t need = workspace ? trn_attn_stats_workspace_bytes(d) : 0;
     const bool split = need > 0 && workspace_bytes >= need;
-    // a handful of queries per head and no split of the keys: the statistics are a second sweep inside the same kernel
+    // a handful of queries per head and no split of the keys: the statistics are part of the same kernel
     if (d->seq_q <= 32 && !split && !mean_std)
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true);
     // (a problem that the second launch refuses is refused before the first has written anything)

@@ -446,7 +446,7 @@ class DecodeKeyFormer(_DecodeAppend):
         if C_out.numel() != H * PM * (1 if self.reduce else M):
             raise ValueError(f"C_out {tuple(C_out.shape)}: expected {(H, PM) if self.reduce else (H, M, PM)}")
         if self.reduce:
-            # one launch up to 32 new tokens (the key scores are a second sweep inside the attention kernel), unless few heads
+            # one launch up to 32 new tokens (the key scores are part of the attention kernel), unless few heads
             # on a long cache make the library split the keys; two launches beyond
             score, = _score_outputs(self, (C_out,), (1, H, PM))
             split = ops.attention_stats_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
