@@ -218,7 +218,7 @@ int trn_attn_fwd_stats_f16(const trn_attn_desc* desc, const void* q, const void*
  * unit of that product -- 8192 keys for 8 heads of 128, 16384 for 16 -- but never fewer than 4096) and how many bytes
  * that takes, 0 otherwise.  Given a zero-initialised workspace of at least
  * that many bytes (256-byte aligned, as for trn_attn_fwd_ws_f16) the attention runs with its keys split over
- * workgroups, and the statistics -- which need the merged row normalisers -- follow as a second launch over all keys
+ * workgroups, and the statistics -- which need the merged row normalisers -- follow in a second launch, over all keys
  * at once; lse (lse_pert with noise) is then required as the buffer that carries the normalisers between the two.
  * Without a workspace, with one that is too small, without that buffer, or for a problem that would not be split,
  * the call is trn_attn_fwd_stats_f16.  Results as trn_attn_fwd_stats_f16 to the stated tolerances (the shares are
@@ -260,9 +260,13 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
  *   out1, out2  [batch, n_q_heads, seq_kv] contiguous, fp16 when out_half is set (the float result rounded once), float
  *               otherwise: sum and sum of squares (one may be NULL) or, with mean_std (without noise; both required), mean
  *               and standard deviation as trn_attn_colmeanstd_f16.
- *   workspace   nullable: trn_attn_stats_workspace_bytes(desc) zero-initialised bytes, as trn_attn_fwd_stats_ws_f16.
+ *   workspace   nullable: trn_attn_key_scores_workspace_bytes(desc, noise given) bytes (0: none), 256-byte aligned, no initial
+ *               contents needed: the keys of at most 32 queries are then split over workgroups, and the launch that merges
+ *               their results sweeps over the keys for the statistics.  With fewer bytes, but those of
+ *               trn_attn_workspace_bytes(desc), over as many as these are for; with less than that, not at all.
  */
 #define TRN_STATS_SPARE_ROWS 128        /* query rows past the last that the statistics kernels may ask for (as zeros) */
+int64_t trn_attn_key_scores_workspace_bytes(const trn_attn_desc* desc, int32_t with_noise);
 int trn_attn_key_scores_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v, void* o,
                             const void* noise, int32_t noise_half, float* rows, void* out1, void* out2,
                             int32_t out_half, int32_t mean_std, void* workspace, int64_t workspace_bytes, void* stream);

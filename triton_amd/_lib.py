@@ -19,7 +19,7 @@ EXPORTS = (
     "trn_calibration_mfma", "trn_attn_workspace_bytes", "trn_attn_chunk_workspace_bytes", "trn_attn_fwd_ws_f16", "trn_linear_f16", "trn_gate_f16", "trn_attn_fwd_stats_f16",
     "trn_attn_fwd_noalloc_f16", "trn_attn_fwd_kernel_name", "trn_attn_colmeanstd_f16", "trn_attn_fwd_probs_f16",
     "trn_attn_fwd_stats_half_f16", "trn_attn_fwd_stats_ws_f16", "trn_attn_stats_workspace_bytes",
-    "trn_attn_key_scores_f16", "trn_attn_qknorm_f16", "trn_attn_qknorm_workspace_bytes",
+    "trn_attn_key_scores_f16", "trn_attn_key_scores_workspace_bytes", "trn_attn_qknorm_f16", "trn_attn_qknorm_workspace_bytes",
 )
 
 
@@ -78,6 +78,8 @@ def load() -> C.CDLL:
     lib.trn_attn_stats_workspace_bytes.argtypes = [C.POINTER(AttnDesc)]
     lib.trn_attn_fwd_stats_ws_f16.restype = C.c_int
     lib.trn_attn_fwd_stats_ws_f16.argtypes = [C.POINTER(AttnDesc), vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i64, vp]
+    lib.trn_attn_key_scores_workspace_bytes.restype = C.c_int64
+    lib.trn_attn_key_scores_workspace_bytes.argtypes = [C.POINTER(AttnDesc), i32]
     lib.trn_attn_key_scores_f16.restype = C.c_int
     lib.trn_attn_key_scores_f16.argtypes = [C.POINTER(AttnDesc), vp, vp, vp, vp, vp, i32, vp, vp, vp, i32, i32, vp, i64, vp]
     lib.trn_attn_fwd_stats_half_f16.restype = C.c_int

@@ -16,6 +16,7 @@ struct AttnArgs {
     const half_t* gamma_k; float k_eps; int k_norm;     // decode kernel without noise only: the keys are normalised on arrival
     // decode kernel only: keys split over n_split workgroups per head, partial results and arrival counters in ws
     int n_split;
+    int partial;   // ... which the next launch merges
     int spread;    // decode kernel only: the query tiles of a head go to all XCDs
     float* ws;
     // decode kernel only, at most 32 queries: per-key sums (and sums of squares) of the probabilities -- of the
@@ -117,6 +118,9 @@ bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int
 const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 // Bytes of workspace with which launch_attn_decode splits the keys of this problem over several workgroups (0: it would not).
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);
+
+// ... and of that with which it does for key statistics, merged and summed up by a second launch.
+int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 
 // Device address, on the current device, of the library's static scratch array (TRN_ATTN_NOALLOC_SCRATCH_BYTES bytes)
 // behind trn_attn_fwd_noalloc_f16; looked up once per device.  nullptr if the runtime refuses.

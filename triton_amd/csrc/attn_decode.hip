@@ -44,7 +44,7 @@ constexpr int kept_blocks(int d, int ds, bool noise) { return !noise ? 2 : d == 
 template <int D, int DS, int NZ>
 __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
-    constexpr bool KEEP = NZ >= 4, NOISE = NZ % 4 == 1 || NZ % 4 == 2, N16 = NZ % 4 == 2, KNORM = NZ == 3;
+    constexpr bool SWEEP = NZ >= 8, KEEP = NZ >= 4 && !SWEEP, NOISE = NZ % 4 == 1 || NZ % 4 == 2, N16 = NZ % 4 == 2, KNORM = NZ == 3;
     constexpr int DV = D / DS;    // columns of V / O this workgroup owns
     constexpr int NS = D / 16;    // k-steps of S^T = K Q^T
     constexpr int NSV = DV / 16;  // (2 key halves) x (DV/32) MFMAs of P V
@@ -57,8 +57,8 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     // (With the whole head dimension of V in one workgroup at head_dim 128 a V stage is 64 KB: one stage then, refilled
     // as soon as its block's P V is issued, so that the K area below still fits.)
     constexpr bool VSINGLE = D == 128 && DS == 1;
-    __shared__ __attribute__((aligned(1024))) half_t Vs0[DNW * 32 * DV];
-    __shared__ __attribute__((aligned(1024))) half_t Vs1[VSINGLE ? 8 : DNW * 32 * DV];
+    __shared__ __attribute__((aligned(1024))) half_t Vs0[SWEEP ? 8 : DNW * 32 * DV];
+    __shared__ __attribute__((aligned(1024))) half_t Vs1[SWEEP || VSINGLE ? 8 : DNW * 32 * DV];
     __shared__ float st_m[DNW][32], st_l[DNW][32], st_m2[DNW][32], st_l2[DNW][32];
     // K blocks are fetched as whole rows (a wave-wide load = 1 KB of consecutive bytes) and turned into MFMA operands
     // through a wave-private LDS area: a load whose lanes each take 16 bytes of their own row -- the operand layout --
@@ -236,6 +236,11 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     const int blk0 = split * bps, nblk = max(0, min(nblk_all, blk0 + bps) - blk0);
     const int nmine = nblk > wave ? (nblk - wave + DNW - 1) / DNW : 0;          // blocks blk0 + wave, + 8, ...
     half8_t ka0[NS], ka1[NS];
+    const int q = tid & 31, dg = tid >> 5;                // merges: 16 groups of threads share out the DV/4 quads of a query
+    const int bh = b * a.Hq + head;
+    constexpr int KB = KEEP ? kept_blocks(D, DS, NOISE) : 1;
+    float16_t kept[KB];
+    float mstar = -INFINITY, L = 0.f, ms2 = -INFINITY, L2 = 0.f;      // of the merged partial results
 
     // One 32-key block whose K is in kc and whose V is in stage Vc; the next block's loads go to kn / Vn first.
     // keep (KEEP only): the block's scores in the log2 domain, the perturbed ones with noise, -inf where masked.
@@ -342,6 +347,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
             TRN_FETCH_V(blk + DNW, Vn);
         }
     };
+    if constexpr (!SWEEP) {
     fetch_k(blk0 + wave, ka0);
     TRN_FETCH_V(blk0 + wave, Vs0);
     if constexpr (NOISE) fetch_noise(blk0 + wave, g0);
@@ -391,8 +397,6 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         if constexpr (NOISE) block(it, ka0, ka0, VSINGLE ? Vs0 : Vs1, Vs0, g1, g0, keep);
         else block(it, ka1, ka0, VSINGLE ? Vs0 : Vs1, Vs0, g1, g0, keep);
     };
-    constexpr int KB = KEEP ? kept_blocks(D, DS, NOISE) : 1;
-    float16_t kept[KB];
     if constexpr (KEEP) {
         // (nested, so that a block's waits are sized on one path only)
         auto walk = [&](auto&& self, auto at) __attribute__((always_inline)) {
@@ -434,12 +438,10 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         }
     }
     __syncthreads();
-    const int q = tid & 31, dg = tid >> 5;                // 16 groups of threads share out the DV/4 quads of a query
     constexpr int NQD = (DV / 4 + 15) / 16;               // quads per thread (with 8 quads, half the groups have none)
-    float mstar = st_m[0][q];
+    mstar = st_m[0][q];
 #pragma unroll
     for (int w = 1; w < DNW; ++w) mstar = fmaxf(mstar, st_m[w][q]);
-    float L = 0.f;
     float4_t acc[NQD];
     {
         float wgt[DNW];
@@ -458,14 +460,12 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
             for (int w = 0; w < DNW; ++w) acc[qi] += reinterpret_cast<const float4_t*>(base + w * 32 * DV)[ql * 32 + q] * wgt[w];
         }
     }
-    float ms2 = -INFINITY, L2 = 0.f;
     if constexpr (NOISE) {
 #pragma unroll
         for (int w = 0; w < DNW; ++w) ms2 = fmaxf(ms2, st_m2[w][q]);
 #pragma unroll
         for (int w = 0; w < DNW; ++w) L2 += ms2 == -INFINITY ? 0.f : st_l2[w][q] * fast_exp2(st_m2[w][q] - ms2);
     }
-    const int bh = b * a.Hq + head;
     if (DS == 1 && a.n_split > 1) {
         // ---- keys split over workgroups: publish (m, l, unnormalised O) of this share; the workgroup that arrives
         // last at the head's counter merges all shares.  Workspace: [arrival counters, 256-byte aligned][bh][split]
@@ -477,6 +477,13 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         const int n_bh = a.B * a.Hq;
         unsigned* counters = reinterpret_cast<unsigned*>(a.ws);
         float* parts = a.ws + ((n_bh + 63) / 64) * 64;
+        if (a.partial) {                       // (the merge is the next launch's: ordinary stores)
+            float* p = parts + ((int64_t)bh * a.n_split + split) * PART;
+#pragma unroll
+            for (int qi = 0; qi < NQD; ++qi) *reinterpret_cast<float4_t*>(p + ((dg + 16 * qi) * 32 + q) * 4) = acc[qi];
+            if (dg == 0) *reinterpret_cast<float4_t*>(p + 32 * D + 4 * q) = float4_t{mstar, L, ms2, L2};
+            return;
+        }
         float* mine = parts + ((int64_t)bh * a.n_split + split) * PART;
         auto publish = [](float* p, float4_t v) __attribute__((always_inline)) {
             const ulong2_t u = __builtin_bit_cast(ulong2_t, v);
@@ -552,6 +559,46 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         if (dg == 0 && dsl == 0 && q0 + q < a.Sq && a.lse) a.lse[(int64_t)bh * a.Sq + q0 + q] = (mstar + fast_log2(L)) * kLn2;
         if constexpr (NOISE) {
             if (dg == 1 && dsl == 0 && q0 + q < a.Sq) a.lse_pert[(int64_t)bh * a.Sq + q0 + q] = (ms2 + fast_log2(L2)) * kLn2;
+        }
+    }
+    } else {
+        // ---- the launch behind a.partial: every workgroup of a head merges the row normalisers of all its shares, each a
+        // part of the output columns, and sweeps over its own share of the keys below
+        constexpr int PART = 32 * (D + 4), BATCH = 8;
+        const float* parts = a.ws + ((a.B * a.Hq + 63) / 64) * 64 + (int64_t)bh * a.n_split * PART;
+        const int quads = (D / 4 + a.n_split - 1) / a.n_split, quad = split * quads + dg;     // at most 16: two shares or more
+        const bool merges = dg < quads && quad < D / 4;
+        const float* op = parts + (min(quad, D / 4 - 1) * 32 + q) * 4;
+        float4_t d[BATCH];
+        auto fetch_o = [&](int s0) __attribute__((always_inline)) {
+#pragma unroll
+            for (int u = 0; u < BATCH; ++u) d[u] = *reinterpret_cast<const float4_t*>(op + min(s0 + u, a.n_split - 1) * PART);
+        };
+        if (merges) fetch_o(0);
+        float4_t* const st = reinterpret_cast<float4_t*>(Kt);            // [share][query]: 16 KB for kMaxStatSplits
+        for (int s = dg; s < a.n_split; s += 16) st[s * 32 + q] = *reinterpret_cast<const float4_t*>(parts + s * PART + 32 * D + 4 * q);
+        __syncthreads();
+        for (int s = 0; s < a.n_split; ++s) { mstar = fmaxf(mstar, st[s * 32 + q][0]); ms2 = fmaxf(ms2, st[s * 32 + q][2]); }
+        for (int s = 0; s < a.n_split; ++s) {
+            const float4_t v = st[s * 32 + q];
+            if (mstar > -INFINITY) L += v[1] * fast_exp2(v[0] - mstar);
+            if (NOISE && ms2 > -INFINITY) L2 += v[3] * fast_exp2(v[2] - ms2);
+        }
+        if (merges) {
+            float4_t o = {0.f, 0.f, 0.f, 0.f};
+            for (int s0 = 0; s0 < a.n_split; s0 += BATCH) {
+                if (s0 > 0) fetch_o(s0);
+#pragma unroll
+                for (int u = 0; u < BATCH; ++u)
+                    if (s0 + u < a.n_split && mstar > -INFINITY) o += d[u] * fast_exp2(st[(s0 + u) * 32 + q][0] - mstar);
+            }
+            const float inv = 1.0f / L;
+            const half4_t ov = {(half_t)(o[0] * inv), (half_t)(o[1] * inv), (half_t)(o[2] * inv), (half_t)(o[3] * inv)};
+            if (q < a.Sq) *reinterpret_cast<half4_t*>(a.o + b * a.ob + head * a.oh + (int64_t)q * a.os + 4 * quad) = ov;
+        }
+        if (split == 0 && dg == 0 && q < a.Sq) {
+            if (a.lse) a.lse[(int64_t)bh * a.Sq + q] = (mstar + fast_log2(L)) * kLn2;
+            if constexpr (NOISE) a.lse_pert[(int64_t)bh * a.Sq + q] = (ms2 + fast_log2(L2)) * kLn2;
         }
     }
     // ---- column statistics (KeyFormer key scores, RoCo sums), from the kept scores or by a second sweep over this head's keys now that the
@@ -675,12 +722,14 @@ static int decode_splits(int batch, int n_q_heads, int seq_kv, int head_dim) {
     return (nblk + bps - 1) / bps;                        // no empty share: the last one starts inside the keys
 }
 
+// Arrival counters and the shares' partial results.
+static int64_t split_bytes(int64_t n_bh, int ns, int head_dim) { return ns <= 1 ? 0 : ((n_bh + 63) / 64) * 256 + n_bh * ns * 32 * (head_dim + 4) * 4; }
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
     if (seq_q > 32) return 0;
     const int ns = decode_splits(batch, n_q_heads, seq_kv, head_dim);
     if (ns <= 1) return 0;
     const int64_t n_bh = (int64_t)batch * n_q_heads;
-    return ((n_bh + 63) / 64) * 256 + n_bh * ns * 32 * (head_dim + 4) * 4;
+    return split_bytes(n_bh, ns, head_dim);
 }
 
 // Column shares of a head for `units` = heads x query tiles: as many as leave 32 columns per workgroup and at most one
@@ -729,6 +778,34 @@ static bool decode_spread(int64_t n_bh, int n_qtiles, int ds) {
     return n_qtiles > 1 && heads8 * 64 > 9 * n_bh && heads8 * n_qtiles * ds > 32;
 }
 
+// Key shares of a problem with key statistics, for the two launches; 0: the statistics are part of the one launch, which runs
+// on one workgroup per head and column share.  The second launch and what the first hands to it cost 4 - 6 us.  us one launch /
+// two, 8 (32) queries with fp16 noise; without: 16 heads of 64, 1600 keys 17.4 / 14.3 (20.6 / 15.9); 12.7 / 12.4, 2064 20.5 / 14.4
+// (22.5 / 15.8); 15.5 / 12.9, 16400 127 / 31 (163 / 37); 103 / 29; 8 heads of 128, 1600 17.8 / 17.0 (22.0 / 20.0); 14.3 / 15.1, 4112
+// 32.8 / 18.9 (39.0 / 21.9); 27.4 / 17.6; 32 heads of 128, 2064 21.5 / 25.3 (24.6 / 28.8); 17.3 / 23.4, 4112 40.8 / 35.0 (49.7 /
+// 42.4); 34.6 / 33.1, 16400 152 / 83 (185 / 94); 136 / 79; 71 of 64, 2064 21.0 / 21.4 (27.2 / 25.3); 16.3 / 19.1, 4112 40.3 / 31.5
+// (50.0 / 37.5); 33.9 / 29.3; 64 of 128, 4112 49.9 / 48.2 (59.5 / 58.1); 43.5 / 46.5, 8208 92.9 / 84.9; 82.9 / 78.6.
+constexpr int kMaxStatSplits = 32;
+static int stats_splits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
+    const int64_t n_bh = (int64_t)batch * n_q_heads, per_key = n_bh * head_dim;
+    const int nblk = (seq_kv + 31) / 32;
+    const int from = n_bh <= 16 ? (noise ? 1537 : 2048) : per_key <= 5120 ? (noise ? 3072 : 3712) : 8192;
+    if (seq_q > 32 || n_bh > 128 || seq_kv < from) return 0;
+    const int ns = max(1, min(min(kMaxStatSplits, (int)(256 / n_bh)), nblk / 8));
+    const int bps = (nblk + ns - 1) / ns, n = (nblk + bps - 1) / bps;
+    return n > 1 ? n : 0;
+}
+int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
+    return split_bytes((int64_t)batch * n_q_heads, stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), head_dim);
+}
+// ... that a workspace holds: with the plain attention's, as many as that has.
+static int stat_shares_in(const AttnArgs& a, int head_dim, int64_t workspace_bytes) {
+    if (a.Sq > 32) return 0;
+    for (const int ns : {stats_splits(a.B, a.Hq, a.Sq, a.Skv, head_dim, a.noise != nullptr), decode_splits(a.B, a.Hq, a.Skv, head_dim)})
+        if (ns > 1 && split_bytes((int64_t)a.B * a.Hq, ns, head_dim) <= workspace_bytes) return ns;
+    return 0;
+}
+
 // Name of the instantiation launched for a problem without a workspace (a measurement aid: what a kernel trace shows).
 const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
     const int ds = decode_col_shares((int64_t)batch * n_q_heads * ((seq_q + 31) / 32), seq_q, seq_kv, head_dim);
@@ -742,11 +819,22 @@ const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq
 }
 
 hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
-    a.n_split = 1; a.ws = nullptr;
+    a.n_split = 1; a.ws = nullptr; a.partial = 0;
     const int64_t need = attn_decode_workspace_bytes(a.B, a.Hq, a.Sq, a.Skv, head_dim);
     if (workspace && need > 0 && workspace_bytes >= need && !a.col_sum && !a.col_sumsq && !a.probs) {
         a.n_split = decode_splits(a.B, a.Hq, a.Skv, head_dim);
         a.ws = static_cast<float*>(workspace);
+    }
+    const int stat_shares = workspace && (a.col_sum || a.col_sumsq) && !a.probs && !a.k_norm ? stat_shares_in(a, head_dim, workspace_bytes) : 0;
+    if (stat_shares > 0) {
+        a.n_split = stat_shares; a.ws = static_cast<float*>(workspace); a.partial = 1; a.n_qtiles = 1;
+        const dim3 g((unsigned)(a.B * a.Hq * stat_shares)), t(DNW * 64);
+        const int nz = !a.noise ? 0 : a.n16 ? 2 : 1;
+#define TRN_DEC_PAIR(D_, N_) do { hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_>), g, t, 0, stream, a); hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_ + 8>), g, t, 0, stream, a); } while (0)
+        if (head_dim == 128) { if (nz == 0) TRN_DEC_PAIR(128, 0); else if (nz == 1) TRN_DEC_PAIR(128, 1); else TRN_DEC_PAIR(128, 2); }
+        else { if (nz == 0) TRN_DEC_PAIR(64, 0); else if (nz == 1) TRN_DEC_PAIR(64, 1); else TRN_DEC_PAIR(64, 2); }
+#undef TRN_DEC_PAIR
+        return hipGetLastError();
     }
     // Without a key split: share V's columns out over workgroups while that still leaves every workgroup 32 columns
     // and the grid within one workgroup per CU (32 heads of 128: 4 shares; 71 heads of 64: 2).  Few queries on a short

@@ -733,18 +733,19 @@ extern "C" int trn_attn_fwd_stats_f16(const trn_attn_desc* d, const void* q, con
     return trn_attn_colstats_f16(d, q, k, rows, noise, out_sum, out_sumsq, stream);
 }
 
-// Where two launches (keys split over workgroups, then the statistics over all keys at once) beat the single launch
-// whose two sweeps run with one workgroup per head and column share.  Measured, 16 queries per head, microseconds one
-// launch / two launches, RoCo (KeyFormer): 8 heads of 128: 27 / 35 (33 / 30) at 4 k keys, 47 / 38 (59 / 39) at 8 k, 163 /
-// 78 (209 / 77) at 32 k; 16 heads of 64: 24 / 30 (33 / 31) at 4 k, 44 / 41 (60 / 42) at 8 k; 16 heads of 128: 48 / 55
-// (61 / 55) at 8 k, 87 / 81 (112 / 79) at 16 k; 32 heads of 128: 48 / 65 (59 / 64) at 8 k, 165 / 189 (207 / 183) at 32 k;
-// 48 heads: the single launch at every length.  The crossover follows the work per key, heads x head_dim: up to 2048 of
-// it, from 8 keys per unit (1024: 8192 keys, 2048: 16384), never below 4096 keys.
+// (attention_with_stats and its C entry split where heads x head_dim is at most 2048, from 8 keys per unit of it and 4096 on;
+// the key scores of the modules where their own rule says so)
 extern "C" int64_t trn_attn_stats_workspace_bytes(const trn_attn_desc* d) {
     const int64_t need = trn_attn_workspace_bytes(d);
     if (need == 0) return 0;
     const int64_t per_key = (int64_t)d->batch * d->n_q_heads * d->head_dim;
     return per_key <= 2048 && d->seq_kv >= (8 * per_key > 4096 ? 8 * per_key : 4096) ? need : 0;
+}
+
+extern "C" int64_t trn_attn_key_scores_workspace_bytes(const trn_attn_desc* d, int32_t with_noise) {
+    using namespace trn;
+    if (!d || validate_attn(d, true) != TRN_OK) return 0;
+    return attn_decode_stats_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
 }
 
 extern "C" int trn_attn_fwd_stats_ws_f16(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o,
@@ -756,16 +757,13 @@ extern "C" int trn_attn_fwd_stats_ws_f16(const trn_attn_desc* d, const void* q, 
     if (!out_sum && !out_sumsq) return TRN_E_NULL;
     if (d->q_norm) return TRN_E_UNSUPPORTED;
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
-    // Few queries and few heads on a long cache: the keys are split over workgroups (which needs the workspace), and
-    // the statistics, which need the merged row normalisers, follow as a launch of their own over all keys at once --
-    // if the caller gave the buffer that carries the normalisers.  Everything else runs as trn_attn_fwd_stats_f16.
+    // Few queries on a long cache: the keys are split over workgroups (which needs the workspace), and the statistics, which
+    // need the merged row normalisers, follow in a second launch -- if the caller gave the buffer that carries the
+    // normalisers.  Everything else runs as trn_attn_fwd_stats_f16.
     const int64_t need = trn_attn_stats_workspace_bytes(d);
     float* rows = noise ? lse_pert : lse;
-    if (workspace && need > 0 && workspace_bytes >= need && rows) {
-        const int st = attn_forward(d, q, k, v, o, lse, gamma_q, noise, lse_pert, workspace, workspace_bytes, nullptr, nullptr, stream);
-        if (st != TRN_OK) return st;
-        return trn_attn_colstats_f16(d, q, k, rows, noise, out_sum, out_sumsq, stream);
-    }
+    if (workspace && need > 0 && workspace_bytes >= need && rows)
+        return attn_forward(d, q, k, v, o, lse, gamma_q, noise, lse_pert, workspace, workspace_bytes, out_sum, out_sumsq, stream);
     return trn_attn_fwd_stats_f16(d, q, k, v, o, lse, gamma_q, noise, lse_pert, out_sum, out_sumsq, stream);
 }
 
@@ -792,16 +790,13 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     const float* n = static_cast<const float*>(noise);
     float *lse = noise ? nullptr : rows, *lse_pert = noise ? rows : nullptr, *s1 = static_cast<float*>(out1), *s2 = static_cast<float*>(out2);
     const bool n16 = noise && noise_half, s16 = out_half != 0;
-    const int64_t need = workspace ? trn_attn_stats_workspace_bytes(d) : 0;
-    const bool split = need > 0 && workspace_bytes >= need;
-    // a handful of queries per head and no split of the keys: the statistics are part of the same kernel
-    if (d->seq_q <= 32 && !split && !mean_std)
-        return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true);
+    // a handful of queries per head: the statistics are part of the same kernel, or of the launch that merges the key shares
+    if (d->seq_q <= 32 && !mean_std)
+        return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, workspace, workspace_bytes, s1, s2, stream, nullptr, n16, s16, true);
     // (a problem that the second launch refuses is refused before the first has written anything)
     int st = attn_colstats_check(d, q, k, rows, n, s1, s2, n16, true);
     if (st != TRN_OK) return st;
-    st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, split ? workspace : nullptr, split ? workspace_bytes : 0,
-                                nullptr, nullptr, stream, nullptr, n16, false, true);
+    st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, d->seq_q <= 32 ? workspace : nullptr, workspace_bytes, nullptr, nullptr, stream, nullptr, n16, false, true);
     if (st != TRN_OK) return st;
     return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);
 }

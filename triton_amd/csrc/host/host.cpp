@@ -440,11 +440,11 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     trn_attn_desc d = attn_desc(q4, k4, v4, o4, scale, causal);
     d.q_norm = q_norm ? 1 : 0;
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[7]));
-    int64_t need = c1.given ? trn_attn_stats_workspace_bytes(&d) : trn_attn_workspace_bytes(&d);
+    int64_t need = c1.given ? 0 : trn_attn_workspace_bytes(&d);
     at::Tensor split;
     if (need) split = workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true);
-    else if (!c1.given && (need = trn_attn_chunk_workspace_bytes(&d)) > 0) {
-        // one for chunks of every length: by exact size each length would keep its own
+    else if ((need = c1.given ? trn_attn_key_scores_workspace_bytes(&d, noise.given) : trn_attn_chunk_workspace_bytes(&d)) > 0) {
+        // one for chunks and caches of every length: by exact size each length would keep its own
         need = std::max<int64_t>(need, TRN_ATTN_CHUNK_WORKSPACE_MAX(D));
         split = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev, false, true);
         if (!split.defined()) need = 0;             // (captured, the cache grown long since the eager call: without)

@@ -377,7 +377,7 @@ class _DecodeAppend(FusedModule):
         ops.attention(*problem, workspace=ws, **kw)
 
     def _chunk_ws(self, nbytes: int, head_dim: int, device):
-        """The workspace of the shared-out keys: one for chunks of every length (by exact size each length would keep its
+        """The workspace of the shared-out keys: one for chunks and caches of every length (by exact size each would keep its
         own); None when the library would not use one, or a capture finds it missing."""
         if not nbytes:
             return None
@@ -446,13 +446,13 @@ class DecodeKeyFormer(_DecodeAppend):
         if C_out.numel() != H * PM * (1 if self.reduce else M):
             raise ValueError(f"C_out {tuple(C_out.shape)}: expected {(H, PM) if self.reduce else (H, M, PM)}")
         if self.reduce:
-            # one launch up to 32 new tokens (the key scores are part of the attention kernel), unless few heads
-            # on a long cache make the library split the keys; two launches beyond
+            # one launch up to 32 new tokens (the key scores are part of the attention kernel), unless a long cache makes the
+            # library split the keys; two launches beyond
             score, = _score_outputs(self, (C_out,), (1, H, PM))
-            split = ops.attention_stats_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
+            split = ops.attention_key_scores_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal, True)
             ops.attention_key_scores(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal, lsep, score,
                                      noise=_noise_operand(self, noise[None]), tau=self.tau,
-                                     workspace=self._split_ws(split, X.device))
+                                     workspace=self._chunk_ws(split, D, X.device))
         else:
             shape = (1, H, M, PM)
             score = C_out.view(shape) if C_out.dtype == torch.float32 and C_out.is_contiguous() else \
@@ -475,11 +475,11 @@ class DecodeRoCo(_DecodeAppend):
         PM = K_cache.shape[1]
         lse = self._workspace("lse", (1, H, M), torch.float32, X.device)
         o = self._o_view(O2, H, M, D)
-        # (few heads on a long cache: keys split over workgroups, the statistics as a second launch)
-        split = ops.attention_stats_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
+        # (a long cache: keys split over workgroups, the statistics as a second launch)
+        split = ops.attention_key_scores_workspace_bytes(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal, False)
         outs = _score_outputs(self, (C_out1, C_out2), (1, H, PM))
         ops.attention_key_scores(q[None], K_cache[None], V_cache[None], o, self.scale, self.causal, lse, outs[0], outs[1],
-                                 workspace=self._split_ws(split, X.device))
+                                 workspace=self._chunk_ws(split, D, X.device))
         _store_scores(C_out1, outs[0]); _store_scores(C_out2, outs[1])
 
 

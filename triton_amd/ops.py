@@ -189,6 +189,13 @@ def attention_stats_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> i
     return int(_lib.load().trn_attn_stats_workspace_bytes(C.byref(d)))
 
 
+def attention_key_scores_workspace_bytes(q, k, v, o, scale: float, causal: bool, with_noise: bool) -> int:
+    """Bytes of workspace with which `attention_key_scores` would split the keys of this problem over several workgroups
+    and run the statistics with the merge of their results as a second launch (0: it would not)."""
+    d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, None, 1.0)
+    return int(_lib.load().trn_attn_key_scores_workspace_bytes(C.byref(d), int(with_noise)))
+
+
 def attention_colstats(q, k, lse, scale: float, causal: bool, out_sum: Optional[torch.Tensor],
                        out_sumsq: Optional[torch.Tensor] = None, noise: Optional[torch.Tensor] = None,
                        tau: float = 1.0) -> None:
