@@ -250,7 +250,7 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
 /*
  * Attention and per-key statistics for every shape and element type in one entry point: what the KeyFormer and RoCo
  * modules call.  As trn_attn_fwd_stats_ws_f16 (one launch with at most 32 queries per head unless the workspace makes it
- * split the keys, two launches otherwise), with
+ * split the keys, and with at most 128 queries and 128 keys; two launches otherwise), with
  *   noise       nullable; fp16 when noise_half is set, float otherwise.  Rows at any pitch and any element alignment (the
  *               reference's noise [.., M, P + M] is fp16 with any key count); desc's noise strides count elements.  One
  *               head is addressed with 32-bit offsets: (seq_q + TRN_STATS_SPARE_ROWS) * noise_stride_s * 4 < 2^31 where

@@ -22,10 +22,11 @@ struct AttnArgs {
     // decode kernel only, at most 32 queries: per-key sums (and sums of squares) of the probabilities -- of the
     // perturbed ones when noise is given -- from a second sweep over the keys once the row normalisers are final
     float* col_sum; float* col_sumsq;
+    int mean_std;  // short kernel only: ... turned into mean and standard deviation
     // ... and the probabilities themselves, un-reduced: float [B, Hq, Sq, Skv] contiguous
     float* probs;
     int n16;       // noise points at fp16 data (its pitches count halfs; any alignment: see HalfNoise)
-    int s16;       // decode kernel only: col_sum and col_sumsq point at fp16 data
+    int s16;       // decode and short kernels: col_sum and col_sumsq point at fp16 data
 };
 
 // fp16 noise as the kernels fetch it.  Its rows may start at any element (the reference's [.., M, P + M] tensors have any
@@ -82,6 +83,15 @@ __device__ __forceinline__ int key_of_sum(int lane) {
     const int kh = (lane >> 1) & 1, r = lane >> 2;
     return 8 * (r / 4) + 4 * kh + (r % 4);
 }
+// The sums x, y of a key's probabilities and their squares over the n queries that see it, into mean and standard deviation.
+__device__ __forceinline__ void mean_std_of(float& x, float& y, float n) {
+    const float mean = x / n;
+    // E p^2 - mean^2 as (y - x mean) / n, the product fused.  The difference is known to about 1e-7 of E p^2, its
+    // root to 3e-4 of the column's root mean square: a key seen by a single query, whose spread is zero by
+    // definition, would come back as that rounding residue, so it is set.
+    y = n > 1.5f ? __builtin_sqrtf(fmaxf(0.f, __builtin_fmaf(-x, mean, y) / n)) : 0.f;
+    x = mean;
+}
 // (fp16: the fp32 value rounded once, as a copy into the caller's tensor would)
 __device__ __forceinline__ void store_stat(float* out, int s16, int64_t at, float v) {
     if (!out) return;
@@ -94,7 +104,7 @@ int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const voi
                  const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
                  bool n16 = false, bool s16 = false, bool any_pitch = false, bool k_norm = false, const void* gamma_k = nullptr,
-                 float k_eps = 0.f);
+                 float k_eps = 0.f, bool mean_std = false);
 
 // The checks of attn_colstats by themselves, for a caller that launches something else before it.
 int attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
@@ -125,6 +135,10 @@ int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, i
 // Device address, on the current device, of the library's static scratch array (TRN_ATTN_NOALLOC_SCRATCH_BYTES bytes)
 // behind trn_attn_fwd_noalloc_f16; looked up once per device.  nullptr if the runtime refuses.
 void* attn_static_scratch();
+
+// Attention and key statistics of at most 128 queries and keys in one launch (attn_short.hip).
+bool attn_short_suits(int seq_q, int seq_kv);
+hipError_t launch_attn_short(const AttnArgs& a, int head_dim, hipStream_t s);
 
 // The forward pass without score perturbation on the 16x16x32 MFMA (attn_fwd16.hip).  Narrow: 4 waves x 32 queries
 // per workgroup; Wide: 8 waves x 32 consecutive queries; Paired: 8 waves, two 128-query tiles from opposite ends of

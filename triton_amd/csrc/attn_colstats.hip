@@ -45,16 +45,8 @@ struct ColArgs {
 template <bool SQ>
 __device__ __forceinline__ void finish_columns(const ColArgs& a, float x, float y, int64_t obase, int wkey0, int lane) {
     const int key = wkey0 + key_of_sum(lane);
-    if (SQ && a.mean_std) {
-        // n = queries that see this key: all of them, or under a causal mask those from key - (Skv - Sq) on
-        const float n = (float)(a.causal ? a.Sq - max(0, key - (a.Skv - a.Sq)) : a.Sq);
-        const float mean = x / n;
-        // E p^2 - mean^2 as (y - x mean) / n, the product fused.  The difference is known to about 1e-7 of E p^2, its
-        // root to 3e-4 of the column's root mean square: a key seen by a single query, whose spread is zero by
-        // definition, would come back as that rounding residue, so it is set.
-        y = n > 1.5f ? __builtin_sqrtf(fmaxf(0.f, __builtin_fmaf(-x, mean, y) / n)) : 0.f;
-        x = mean;
-    }
+    // (queries that see a key: all of them, or under a causal mask those from key - (Skv - Sq) on)
+    if (SQ && a.mean_std) mean_std_of(x, y, (float)(a.causal ? a.Sq - max(0, key - (a.Skv - a.Sq)) : a.Sq));
     if ((lane & 1) == 0 && key < a.Skv) {
         store_stat(a.out_sum, a.s16, obase + key, x);
         if (SQ) store_stat(a.out_sumsq, a.s16, obase + key, y);

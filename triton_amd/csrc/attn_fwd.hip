@@ -796,6 +796,8 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     // (a problem that the second launch refuses is refused before the first has written anything)
     int st = attn_colstats_check(d, q, k, rows, n, s1, s2, n16, true);
     if (st != TRN_OK) return st;
+    if (attn_short_suits(d->seq_q, d->seq_kv))
+        return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, mean_std != 0);
     st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, d->seq_q <= 32 ? workspace : nullptr, workspace_bytes, nullptr, nullptr, stream, nullptr, n16, false, true);
     if (st != TRN_OK) return st;
     return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);
@@ -835,7 +837,7 @@ extern "C" int trn_attn_qknorm_f16(const trn_attn_desc* d, const void* q, const 
 int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                              int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs,
-                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps) {
+                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps, bool mean_std) {
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
     if (!d || !q || !k || !v || !o) return TRN_E_NULL;
     if (noise && !lse_pert) return TRN_E_NULL;
@@ -854,7 +856,6 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
                    !pitch16(d->noise_stride_b, 4))
             return TRN_E_ALIGN;
     }
-    if (s16 && d->seq_q > 32) return TRN_E_UNSUPPORTED;      // fp16 statistics of the second sweep: at most 32 queries
     AttnArgs a;
     a.q = (const half_t*)q; a.k = (const half_t*)k; a.v = (const half_t*)v; a.o = (half_t*)o;
     a.lse = lse; a.gamma_q = (const half_t*)gamma_q; a.noise = noise; a.lse_pert = lse_pert;
@@ -870,13 +871,15 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     a.c2 = d->scale * kLog2e / tau; a.c3 = kLog2e / tau;
     a.q_eps = d->q_norm_eps; a.causal = d->causal ? 1 : 0; a.q_norm = d->q_norm ? 1 : 0;
     a.gamma_k = (const half_t*)gamma_k; a.k_eps = k_eps; a.k_norm = k_norm ? 1 : 0;
-    a.n_split = 1; a.spread = 0; a.ws = nullptr; a.col_sum = col_sum; a.col_sumsq = col_sumsq; a.probs = probs; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
+    a.n_split = 1; a.spread = 0; a.ws = nullptr; a.col_sum = col_sum; a.col_sumsq = col_sumsq; a.probs = probs; a.mean_std = mean_std ? 1 : 0; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
     // K/V tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base
     // (with room for the blocks the pipelines request past the end, which must stay representable to read as zeros)
     if (((int64_t)d->seq_kv + 2048) * d->k_stride_s * 2 > 0x7fffffffLL || ((int64_t)d->seq_kv + 2048) * d->v_stride_s * 2 > 0x7fffffffLL)
         return TRN_E_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
+    if ((col_sum || col_sumsq) && d->seq_q > 32)
+        return launch_attn_short(a, d->head_dim, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;      // (attn_short_suits: the callers see to it)
     // a chunk of queries on a long cache, with the workspace for it: the keys shared out over workgroups
     if (workspace && !noise && !col_sum && !col_sumsq && !probs) {
         const int64_t need = attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
