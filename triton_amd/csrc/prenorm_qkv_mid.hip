@@ -19,7 +19,7 @@
 //
 // Measured, weights cold in HBM, us before (128 x 128 kernel) / now: 4096 -> 12288 without norm 33 tokens 63 / 26, 64
 // tokens 63 / 29, 100 tokens 64 / 35; 4096 -> 6144 with norm and gamma 100 tokens 74 / 26, 256 tokens 74 / 37.5, 512 tokens
-// 74 / 50; 1024 -> 3072 128 tokens 18 / 8.
+// 74 / 43; 1024 -> 3072 128 tokens 18 / 8.
 #include "prenorm_qkv.h"
 
 namespace trn {
@@ -76,21 +76,23 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs 
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(NORM == 2 ? a.gamma : a.x), 0, NORM == 2 ? a.K * 2 : 0, 0x00020000);
     half8_t g0, g1, g2, g3;
-    // All requests of stage s; past the last stage they read rows past hidden, i.e. zeros.
-    auto fetch = [&](int s, half_t* D, half8_t& g) __attribute__((always_inline)) {
-        const int st = min(s, nst);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (NORM == 2)
+    // Request n of a stage's NL (gamma, W, X); past the last stage they read rows past hidden, i.e. zeros.
+    auto request = [&](int n, int s, half_t* D, half8_t& g) __attribute__((always_inline)) {
+        const int st = min(s, nst), i = n - (NL - XI - WI);
+        if (i < 0)
             g = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(grs, (kq * 16 + 8 * h) * 2, st * SK * 2, 0));
-#pragma unroll
-        for (int i = 0; i < WI; ++i)
+        else if (i < WI)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 wrs, (__attribute__((address_space(3))) void*)(D + MT * SK + (wave * WI + i) * 512), 16, w_vo[i], st * w_stage, 0, 0);
-#pragma unroll
-        for (int i = 0; i < XI; ++i)      // columns past hidden hold the next row's data: read zeros instead
+        else              // columns past hidden hold the next row's data: read zeros instead
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                xrs, (__attribute__((address_space(3))) void*)(D + (XI * wave + i) * 512), 16,
-                st * SK + 8 * x_ch[i] >= a.K ? kOut : x_vo[i], st * SK * 2, 0, 0);
+                xrs, (__attribute__((address_space(3))) void*)(D + (XI * wave + i - WI) * 512), 16,
+                st * SK + 8 * x_ch[i - WI] >= a.K ? kOut : x_vo[i - WI], st * SK * 2, 0, 0);
+    };
+    auto fetch = [&](int s, half_t* D, half8_t& g) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < NL; ++n) request(n, s, D, g);
         __builtin_amdgcn_sched_barrier(0);
     };
 
@@ -141,7 +143,17 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs 
         half8_t xg[NTB];                     // (gamma is used up before its slot of the ring is refilled)
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) { if constexpr (NORM == 2) xg[tb] = xb[tb] * g; else xg[tb] = xb[tb]; }
-        fetch(s + 4, F, g);
+        // With eight MFMAs a stage its requests go out one by one behind them: all at once they keep the wave from issuing
+        // anything else (4096 -> 6144, us at once / dealt out, with norm and gamma; without: 300 tokens 45.4 / 41.3; 30.4 / 29.1, 512
+        // 46.0 / 43.3; 39.8 / 38.6, 640 51.3 / 49.2; 40.2 / 39.0; the tiles of two and four MFMAs: the same).
+        constexpr bool kDeal = NTB == 4;
+        if constexpr (!kDeal) fetch(s + 4, F, g);
+        auto deal = [&](int mfma) __attribute__((always_inline)) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int n = 0; n < NL; ++n) if (kDeal && n * 2 * NTB / NL == mfma) request(n, s + 4, F, g);
+            __builtin_amdgcn_sched_barrier(0);
+        };
 #pragma unroll
         for (int tb = 0; tb < NTB; ++tb) {
             acc[tb][0] = mfma32(wa[0], xg[tb], acc[tb][0]);
@@ -149,7 +161,7 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs 
             if (tb == 1) wn[1] = read_w(Cn, 1);
             if (NTB <= 2) xn[tb] = read_x(Cn, tb);
             else if (tb >= 2) { xn[2 * tb - 4] = read_x(Cn, 2 * tb - 4); xn[2 * tb - 3] = read_x(Cn, 2 * tb - 3); }
-            __builtin_amdgcn_sched_barrier(0);
+            deal(2 * tb);
             acc[tb][1] = mfma32(wa[1], xg[tb], acc[tb][1]);
             if (stats) {
 #pragma unroll
@@ -158,7 +170,7 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs 
                     ss[tb] = __builtin_amdgcn_fdot2(p, p, ss[tb], false);
                 }
             }
-            __builtin_amdgcn_sched_barrier(0);
+            deal(2 * tb + 1);
         }
     };
     half8_t waA[2], xbA[NTB], waB[2], xbB[NTB];
