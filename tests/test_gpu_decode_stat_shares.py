@@ -12,11 +12,17 @@ CASES = [(1, 8, 2, 128, 8, 8193), (1, 2, 2, 64, 32, 8192), (1, 16, 16, 64, 5, 20
          (2, 12, 4, 128, 3, 4097), (1, 71, 71, 64, 16, 4100), (1, 100, 10, 64, 17, 8200), (1, 128, 8, 64, 16, 8192)]
 
 
-@pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", CASES)
+# chunks of more than 32 queries, without noise: the forward's shares
+CHUNKS = [(1, 32, 8, 128, 100, 4100), (1, 16, 16, 64, 33, 8193), (1, 71, 1, 64, 128, 9000)]
+
+
+@pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", CASES + CHUNKS)
 @pytest.mark.parametrize("noise_type", [None, torch.float16, torch.float32])
 @pytest.mark.parametrize("causal", [False, True])
 def test_shared_out_statistics(B, H, Hkv, D, Sq, Skv, noise_type, causal):
     from triton_amd import ops
+    if Sq > 32 and noise_type is not None:
+        pytest.skip("chunks are shared out without noise only")
     g = torch.Generator(device="cuda").manual_seed(Skv + Sq)
     q, k, v = (torch.randn(B, h, s, D, generator=g, device="cuda").half() for h, s in ((H, Sq), (Hkv, Skv), (Hkv, Skv)))
     noise = None
@@ -61,4 +67,5 @@ def test_rule(H, D, noise, keys):
             assert (ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, True, noise) > 0) == want
             if keys:
                 q = torch.empty(1, H, 33, D, dtype=torch.half, device="cuda")
-                assert ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, True, noise) == 0
+                want = 0 if noise else ops.attention_chunk_workspace_bytes(q, k, k, q, 0.1, True)
+                assert ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, True, noise) == want

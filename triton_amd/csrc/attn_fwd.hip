@@ -745,6 +745,8 @@ extern "C" int64_t trn_attn_stats_workspace_bytes(const trn_attn_desc* d) {
 extern "C" int64_t trn_attn_key_scores_workspace_bytes(const trn_attn_desc* d, int32_t with_noise) {
     using namespace trn;
     if (!d || validate_attn(d, true) != TRN_OK) return 0;
+    // a chunk of more than 32 queries without noise: its forward shares out the keys as it does without the statistics
+    if (d->seq_q > 32 && !with_noise) return attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
     return attn_decode_stats_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
 }
 
@@ -798,7 +800,7 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     if (st != TRN_OK) return st;
     if (attn_short_suits(d->seq_q, d->seq_kv))
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, mean_std != 0);
-    st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, d->seq_q <= 32 ? workspace : nullptr, workspace_bytes, nullptr, nullptr, stream, nullptr, n16, false, true);
+    st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, workspace, workspace_bytes, nullptr, nullptr, stream, nullptr, n16, false, true);
     if (st != TRN_OK) return st;
     return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);
 }
