@@ -200,8 +200,8 @@ int trn_attn_colmeanstd_f16(const trn_attn_desc* desc, const void* q, const void
  * trn_attn_fwd_f16 and trn_attn_colstats_f16 in one call: the attention output plus the per-key statistics of its
  * probabilities -- of the perturbed probabilities when noise is given -- i.e. what one forward of the reference's
  * KeyFormer (ref_rms.py:147-179, C_out of keyformer_llama_benchmark.py:79) or RoCo (ref_rms.py:249-280) computes.
- * With at most 32 queries per head (the reference's decode-append problem) the statistics are a second sweep over
- * the keys inside the attention kernel -- one launch; otherwise the two kernels are launched one after the other,
+ * With at most 32 queries per head (the reference's decode-append problem) the statistics come from the attention
+ * kernel itself -- one launch; otherwise the two kernels are launched one after the other,
  * and lse (lse_pert with noise) is required as the buffer that carries the row normalisers between them.
  * q_norm is not supported here.  out_sum / out_sumsq as in trn_attn_colstats_f16 (one of them may be NULL).
  */
