@@ -69,3 +69,42 @@ def test_rule(H, D, noise, keys):
                 q = torch.empty(1, H, 33, D, dtype=torch.half, device="cuda")
                 want = 0 if noise else ops.attention_chunk_workspace_bytes(q, k, k, q, 0.1, True)
                 assert ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, True, noise) == want
+
+
+# the shares by the statistics' rule, by that of the plain attention's workspace too (4112 keys, 16 heads), and none of either
+@pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", [(1, 8, 8, 128, 8, 4112), (1, 16, 16, 64, 5, 4112), (1, 8, 2, 128, 32, 8193), (1, 100, 10, 64, 17, 9000),
+                                              (1, 2, 1, 64, 1, 2049), (1, 8, 8, 128, 8, 700)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("half", [False, True])
+def test_mean_and_deviation_of_shared_out_keys(B, H, Hkv, D, Sq, Skv, causal, half):
+    """At most 32 queries, mean and standard deviation, a workspace of any contents: against float64.
+
+    Bounds: the normaliser sums probabilities rounded to fp16 (2^-12 relative at most, each), hence 2.5e-4 on the means; a
+    difference of the two sums that is known to 1e-7 of E p^2 gives its root to 3e-4 of the root mean square; fp16 results
+    are rounded once more (2^-11, and half of the smallest fp16 number)."""
+    from triton_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(Skv + Sq)
+    q, k, v = (torch.randn(B, h, s, D, generator=g, device="cuda").half() for h, s in ((H, Sq), (Hkv, Skv), (Hkv, Skv)))
+    scale = D ** -0.5
+    size = max(ops.attention_key_scores_workspace_bytes(q, k, v, q, scale, causal, False), ops.attention_workspace_bytes(q, k, v, q, scale, causal))
+    ws = torch.full((max(size, 256),), 255, dtype=torch.uint8, device="cuda")
+    rows, o = torch.full((B, H, Sq), -1.0, device="cuda"), torch.full_like(q, 7.0)
+    out = [torch.full((B, H, Skv), -1.0, device="cuda", dtype=torch.half if half else torch.float) for _ in range(2)]
+    ops.attention_key_scores(q, k, v, o, scale, causal, rows, *out, mean_std=True, workspace=ws)
+    torch.cuda.synchronize()
+    seen = torch.ones(Sq, Skv, dtype=torch.bool, device="cuda")
+    if causal:
+        seen = seen.tril(Skv - Sq)
+    n = seen.sum(0).double()
+    rounded, least = (2.0 ** -11, 2.0 ** -25) if half else (0.0, 0.0)
+    for h in range(H):
+        kk, vv = (t[0, h * Hkv // H].double() for t in (k, v))
+        s = (q[0, h].double() @ kk.T.contiguous() * scale).masked_fill(~seen, float("-inf"))
+        p = s.softmax(-1)
+        want = p @ vv
+        assert (o[0, h].double() - want).norm() <= 1e-3 * want.norm() and (rows[0, h].double() - s.logsumexp(-1)).abs().max() <= 2.5e-4
+        mean, square = p.sum(0) / n, p.pow(2).sum(0) / n
+        std = (square - mean * mean).clamp(min=0).sqrt()
+        std[n == 1] = 0
+        assert ((out[0][0, h].double() - mean).abs() <= (2.5e-4 + rounded) * mean + least).all()
+        assert ((out[1][0, h].double() - std).abs() <= 2.5e-4 * std + 3e-4 * square.sqrt() + rounded * std + least).all()

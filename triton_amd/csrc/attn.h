@@ -22,7 +22,7 @@ struct AttnArgs {
     // decode kernel only, at most 32 queries: per-key sums (and sums of squares) of the probabilities -- of the
     // perturbed ones when noise is given -- from a second sweep over the keys once the row normalisers are final
     float* col_sum; float* col_sumsq;
-    int mean_std;  // short kernel only: ... turned into mean and standard deviation
+    int mean_std;  // short kernel, and decode kernel with shared-out keys: ... turned into mean and standard deviation
     // ... and the probabilities themselves, un-reduced: float [B, Hq, Sq, Skv] contiguous
     float* probs;
     int n16;       // noise points at fp16 data (its pitches count halfs; any alignment: see HalfNoise)
@@ -131,6 +131,8 @@ int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq
 
 // ... and of that with which it does for key statistics, merged and summed up by a second launch.
 int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
+// ... over how many workgroups a head with a workspace of so many bytes (0: the statistics are part of a single launch).
+int attn_decode_stat_shares(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes);
 
 // Device address, on the current device, of the library's static scratch array (TRN_ATTN_NOALLOC_SCRATCH_BYTES bytes)
 // behind trn_attn_fwd_noalloc_f16; looked up once per device.  nullptr if the runtime refuses.

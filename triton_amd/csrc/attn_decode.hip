@@ -688,6 +688,10 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
                 y = __builtin_fmaf(p, p, y);
             }
             x = half_sum(x); y = half_sum(y);
+            // (the statistics kernels' other form: the second launch has every query's probabilities of its keys too)
+            if constexpr (SWEEP && !NOISE) {
+                if (a.mean_std) mean_std_of(x, y, (float)(a.causal ? a.Sq - max(0, key - off) : a.Sq));
+            }
             if (h == 0 && key < a.Skv) {
                 const int64_t at = (int64_t)bh * a.Skv + key;
                 store_stat(a.col_sum, a.s16, at, x);
@@ -799,10 +803,10 @@ int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, i
     return split_bytes((int64_t)batch * n_q_heads, stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), head_dim);
 }
 // ... that a workspace holds: with the plain attention's, as many as that has.
-static int stat_shares_in(const AttnArgs& a, int head_dim, int64_t workspace_bytes) {
-    if (a.Sq > 32) return 0;
-    for (const int ns : {stats_splits(a.B, a.Hq, a.Sq, a.Skv, head_dim, a.noise != nullptr), decode_splits(a.B, a.Hq, a.Skv, head_dim)})
-        if (ns > 1 && split_bytes((int64_t)a.B * a.Hq, ns, head_dim) <= workspace_bytes) return ns;
+int attn_decode_stat_shares(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes) {
+    if (seq_q > 32) return 0;
+    for (const int ns : {stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), decode_splits(batch, n_q_heads, seq_kv, head_dim)})
+        if (ns > 1 && split_bytes((int64_t)batch * n_q_heads, ns, head_dim) <= workspace_bytes) return ns;
     return 0;
 }
 
@@ -825,7 +829,9 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
         a.n_split = decode_splits(a.B, a.Hq, a.Skv, head_dim);
         a.ws = static_cast<float*>(workspace);
     }
-    const int stat_shares = workspace && (a.col_sum || a.col_sumsq) && !a.probs && !a.k_norm ? stat_shares_in(a, head_dim, workspace_bytes) : 0;
+    const int stat_shares = workspace && (a.col_sum || a.col_sumsq) && !a.probs && !a.k_norm ?
+        attn_decode_stat_shares(a.B, a.Hq, a.Sq, a.Skv, head_dim, a.noise != nullptr, workspace_bytes) : 0;
+    if (a.mean_std && stat_shares == 0) return hipErrorInvalidValue;      // (the single launch has the sums only)
     if (stat_shares > 0) {
         a.n_split = stat_shares; a.ws = static_cast<float*>(workspace); a.partial = 1; a.n_qtiles = 1;
         const dim3 g((unsigned)(a.B * a.Hq * stat_shares)), t(DNW * 64);

@@ -800,6 +800,13 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     if (st != TRN_OK) return st;
     if (attn_short_suits(d->seq_q, d->seq_kv))
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, mean_std != 0);
+    // mean and deviation of a handful of queries: by the launch that merges the key shares; elsewhere the workspace stays
+    // out of it (the plain attention would split the keys by counters in it that have to be zero)
+    if (d->seq_q <= 32) {
+        if (workspace && attn_decode_stat_shares(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, false, workspace_bytes) > 0)
+            return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, workspace, workspace_bytes, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, true);
+        workspace = nullptr; workspace_bytes = 0;
+    }
     st = attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, workspace, workspace_bytes, nullptr, nullptr, stream, nullptr, n16, false, true);
     if (st != TRN_OK) return st;
     return attn_colstats(d, q, k, rows, n, s1, s2, mean_std ? 1 : 0, stream, n16, s16, true);
