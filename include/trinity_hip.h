@@ -115,7 +115,7 @@ int trn_attn_fwd_f16(const trn_attn_desc* desc, const void* q, const void* k, co
  * desc, weight gamma_q) over head_dim, then trn_attn_fwd_f16.  K is left as it is.  Where few query tiles read the keys they
  * are normalised on their way into that launch; elsewhere once, by a launch of its own, into
  *   k_norm     trn_attn_qknorm_workspace_bytes(desc) bytes of device memory, 16-byte aligned; may be NULL if that is 0.
- * The batches of K must then lie n_kv_heads * k_stride_h apart.
+ * The batches of K must then lie n_kv_heads * k_stride_h apart (with a single KV head: anywhere).
  */
 int64_t trn_attn_qknorm_workspace_bytes(const trn_attn_desc* desc);
 int trn_attn_qknorm_f16(const trn_attn_desc* desc, const void* q, const void* k, const void* v, void* o,

@@ -68,3 +68,32 @@ def test_ranges(D):
     o, _ = run(q, k, v, gq, gk * 0, 1e-5)
     w = want(q, k, v, gq, gk * 0, 1e-5)
     assert not ((o.double() - w).abs() > 2e-2 + 1e-2 * w.abs()).any()
+
+
+# the keys normalised within the attention launch, and by a launch of their own
+@pytest.mark.parametrize("B,Hq,S,D", [(2, 8, 100, 128), (2, 71, 300, 64), (3, 40, 515, 128)])
+@pytest.mark.parametrize("native", [True, False])
+def test_contiguous_keys_of_any_stride_along_an_axis_of_one(B, Hq, S, D, native):
+    """A contiguous K may have any stride along an axis of one element: a single KV head seen through the token-major tensor
+    that a projection writes, one batch or one key out of a larger buffer."""
+    from triton_amd import modules
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (ref.randn_half((B, h, S, D), g).cuda() for h in (Hq, 1, 1))
+    gq, gk = (ref.randn_half((D,), g, 1.0, 0.02).cuda() for _ in range(2))
+    m = modules.get("qknorm")
+
+    def out(q, k, v):
+        t = dict(Q=q, K=k, V=v, O=torch.full_like(q, 7.0), gamma_q=gq, gamma_k=gk)
+        (m.forward if native else m._run)(*[t[p] for p in m.TENSOR_PARAMS])
+        torch.cuda.synchronize()
+        return t["O"]
+
+    token_major = k.view(B, S, 1, D).transpose(1, 2)
+    odd_batch = torch.as_strided(k, (1, 1, S, D), (S * D + 4, 4, D, 1))
+    odd_key = torch.as_strided(k, (B, 1, 1, D), (D, 12, 4, 1))
+    for odd in (token_major, odd_batch, odd_key):
+        b, _, s, _ = odd.shape
+        plain = torch.empty(b, 1, s, D, dtype=torch.half, device="cuda").copy_(odd)
+        assert odd.is_contiguous() and odd.stride() != plain.stride()
+        qs, vs = q[:b, :, :s].contiguous(), v[:b, :, :s].contiguous()
+        assert torch.equal(out(qs, odd, vs), out(qs, plain, vs))

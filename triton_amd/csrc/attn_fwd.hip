@@ -834,9 +834,11 @@ extern "C" int trn_attn_qknorm_f16(const trn_attn_desc* d, const void* q, const 
         return attn_forward(d, q, k, v, o, nullptr, gamma_q, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream, nullptr,
                             false, false, false, true, gamma_k, k_eps);
     if (!k_norm) return TRN_E_NULL;
-    if (d->batch > 1 && d->k_stride_b != d->n_kv_heads * d->k_stride_h) return TRN_E_STRIDE;
+    // (the stride from one head's keys to the next, batch by batch; a single head has none of its own)
+    const int64_t head = d->n_kv_heads == 1 ? d->k_stride_b : d->k_stride_h;
+    if (d->batch > 1 && d->k_stride_b != d->n_kv_heads * head) return TRN_E_STRIDE;
     const int64_t rows = d->seq_kv, D = d->head_dim;
-    if (const int e = trn_rmsnorm_f16(k, gamma_k, k_norm, (int64_t)d->batch * d->n_kv_heads, rows, D, d->k_stride_h, d->k_stride_s,
+    if (const int e = trn_rmsnorm_f16(k, gamma_k, k_norm, (int64_t)d->batch * d->n_kv_heads, rows, D, head, d->k_stride_s,
                                       rows * D, D, 0, k_eps, stream); e != TRN_OK) return e;
     trn_attn_desc n = *d;
     n.k_stride_b = d->n_kv_heads * rows * D; n.k_stride_h = rows * D; n.k_stride_s = D;

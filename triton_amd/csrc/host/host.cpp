@@ -327,8 +327,11 @@ bool f_attention_forward(Args a, Py_ssize_t n) {          // scale | None, causa
 bool f_qknorm_forward(Args a, Py_ssize_t n) {             // workspaces, scale | None, causal, eps, K, O, Q, V, gamma_k, gamma_q
     count(n, 10, "qknorm_forward");
     Workspaces* w = ws_arg(a[0]);
-    const View k = as4(arg(a[4], "K"), "K"), o = as4(arg(a[5], "O"), "O"), q = as4(arg(a[6], "Q"), "Q"), v = as4(arg(a[7], "V"), "V");
+    View k = as4(arg(a[4], "K"), "K");
+    const View o = as4(arg(a[5], "O"), "O"), q = as4(arg(a[6], "Q"), "Q"), v = as4(arg(a[7], "V"), "V");
     NEED(k.contiguous(), "K: expected a contiguous tensor");
+    // (whose strides along axes of one element may be anything: a single KV head of a token-major tensor)
+    k = make(k, k.p, {k.s[0], k.s[1], k.s[2], k.s[3]}, {k.s[1] * k.s[2] * k.s[3], k.s[2] * k.s[3], k.s[3], 1});
     NEED(k.cuda, "K: expected a GPU tensor");
     const double eps = num(a[3]);
     trn_attn_desc d = attn_desc(q, k, v, o, scale_of(a[1], k.s[3]), flag(a[2]));

@@ -240,6 +240,8 @@ class QKNormAttention(FusedModule):
         q, k, v, o = _as4(Q, "Q"), _as4(K, "K"), _as4(V, "V"), _as4(O, "O")
         if not k.is_contiguous():
             raise ValueError("K: expected a contiguous tensor")
+        B, Hkv, Skv, D = k.shape            # (a contiguous tensor's strides along axes of one element may be anything)
+        k = k.as_strided(k.shape, (Hkv * Skv * D, Skv * D, D, 1))
         ops.qknorm_attention(q, k, v, o, _scale(self.scale, k.shape[3]), self.causal, gamma_q, gamma_k, self.eps,
                              lambda: self._workspace("k_norm", k.shape, k.dtype, k.device))
 
