@@ -108,3 +108,39 @@ def test_mean_and_deviation_of_shared_out_keys(B, H, Hkv, D, Sq, Skv, causal, ha
         std[n == 1] = 0
         assert ((out[0][0, h].double() - mean).abs() <= (2.5e-4 + rounded) * mean + least).all()
         assert ((out[1][0, h].double() - std).abs() <= 2.5e-4 * std + 3e-4 * square.sqrt() + rounded * std + least).all()
+
+
+# problems that use no workspace, that use one, that share out a chunk's keys, and prompts with two launches
+@pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", [(1, 8, 8, 128, 8, 200), (1, 8, 8, 128, 8, 4112), (1, 16, 16, 64, 5, 2064), (1, 8, 8, 128, 100, 4100),
+                                              (1, 4, 2, 64, 300, 300), (1, 4, 2, 128, 64, 64)])
+@pytest.mark.parametrize("mean_std", [False, True])
+def test_a_misaligned_workspace_is_not_used(B, H, Hkv, D, Sq, Skv, mean_std):
+    """Off 256 bytes: the call is the one without a workspace, and nothing is written there."""
+    from triton_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(Skv)
+    q, k, v = (torch.randn(B, h, s, D, generator=g, device="cuda").half() for h, s in ((H, Sq), (Hkv, Skv), (Hkv, Skv)))
+    assert ops.attention_stats_workspace_bytes(q, k, v, q, D ** -0.5, True) == 0
+    need = max(256, ops.attention_key_scores_workspace_bytes(q, k, v, q, D ** -0.5, True, False), ops.attention_workspace_bytes(q, k, v, q, D ** -0.5, True))
+    store = torch.full((need + 16,), 255, dtype=torch.uint8, device="cuda")
+    assert store.data_ptr() % 256 == 0
+    results = []
+    for ws in (None, store[16:]):
+        rows, o = torch.zeros(B, H, Sq, device="cuda"), torch.full_like(q, 7.0)
+        x, y = (torch.full((B, H, Skv), -1.0, device="cuda") for _ in range(2))
+        ops.attention_key_scores(q, k, v, o, D ** -0.5, True, rows, x, y, mean_std=mean_std, workspace=ws)
+        results.append((o, rows, x, y))
+    torch.cuda.synchronize()
+    assert (store == 255).all()
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+
+
+def test_a_misaligned_workspace_is_refused_where_it_was():
+    """The sizes and problems of attention_stats_workspace_bytes."""
+    from triton_amd import ops
+    q, k = torch.zeros(1, 8, 8, 128, dtype=torch.half, device="cuda"), torch.zeros(1, 8, 8192, 128, dtype=torch.half, device="cuda")
+    need = ops.attention_stats_workspace_bytes(q, k, k, q, 0.1, True)
+    assert need > 0
+    rows, x = torch.zeros(1, 8, 8, device="cuda"), torch.zeros(1, 8, 8192, device="cuda")
+    with pytest.raises(Exception, match="ALIGN"):
+        ops.attention_key_scores(q, k, k, torch.empty_like(q), 0.1, True, rows, x, workspace=torch.zeros(need + 16, dtype=torch.uint8, device="cuda")[16:])

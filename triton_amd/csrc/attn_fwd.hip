@@ -792,6 +792,13 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     const float* n = static_cast<const float*>(noise);
     float *lse = noise ? nullptr : rows, *lse_pert = noise ? rows : nullptr, *s1 = static_cast<float*>(out1), *s2 = static_cast<float*>(out2);
     const bool n16 = noise && noise_half, s16 = out_half != 0;
+    // A workspace that cannot be used is as good as none: the keys are not split then.  Misaligned ones of the size and problems
+    // that trn_attn_stats_workspace_bytes() names have always been refused.
+    if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) || workspace_bytes < 0)) {
+        const int64_t named = trn_attn_stats_workspace_bytes(d);
+        if (named > 0 && workspace_bytes >= named) return TRN_E_ALIGN;
+        workspace = nullptr; workspace_bytes = 0;
+    }
     // a handful of queries per head: the statistics are part of the same kernel, or of the launch that merges the key shares
     if (d->seq_q <= 32 && !mean_std)
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, workspace, workspace_bytes, s1, s2, stream, nullptr, n16, s16, true);
