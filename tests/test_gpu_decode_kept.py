@@ -1,7 +1,9 @@
 """GPU parity of the decode attention with key statistics where the scores stay in registers (at most six key blocks of 32 per
 wave, three with the whole head dimension of 128 in one workgroup, two without noise) and one key past it, in every number of column shares.
 
-Tolerances as in test_gpu_scores.py: 2e-2 on outputs of fp16 probabilities, 1e-3 relative on fp32 key scores."""
+Tolerances: outputs to 2e-3 of each query's 2-norm (fp16 probabilities and one fp16 rounding, 2^-11 each at most, are some 3e-4 of a
+norm; an element of an output is 0.02 to 0.05 at these lengths, so that an absolute bound of that size would see nothing),
+1e-3 relative on fp32 key scores as in test_gpu_scores.py."""
 import pytest
 import torch
 
@@ -42,7 +44,8 @@ def test_kept_scores(B, H, Hkv, D, Sq, Skv, noise_type, causal):
     if causal:
         hidden = ~torch.ones(Sq, Skv, dtype=torch.bool, device="cuda").tril(Skv - Sq)
     s = s.masked_fill(hidden, float("-inf"))
-    assert (o.float() - s.softmax(-1) @ vv).abs().max() < 2e-2
+    want = s.softmax(-1) @ vv
+    assert ((o.float() - want).norm(dim=-1) <= 2e-3 * want.norm(dim=-1)).all()
     z = s if noise is None else ((s + noise.float().masked_fill(hidden, 0)) / tau)
     p = z.softmax(-1)
     assert (rows - z.logsumexp(-1)).abs().max() < 1e-3

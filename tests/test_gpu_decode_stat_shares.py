@@ -1,7 +1,9 @@
 """GPU parity of the decode attention with key statistics over keys split over workgroups (the partial results merged, and the
 statistics summed, by a second launch), against fp32 sums and against the single launch.
 
-Tolerances as in test_gpu_scores.py: 2e-2 on outputs of fp16 probabilities, 1e-3 relative on fp32 key scores."""
+Tolerances: outputs to 2e-3 of each query's 2-norm (fp16 probabilities and one fp16 rounding, 2^-11 each at most, are some 3e-4 of a
+norm; an element of an output is 0.02 to 0.05 at these lengths, so that an absolute bound of that size would see nothing),
+1e-3 relative on fp32 key scores as in test_gpu_scores.py."""
 import pytest
 import torch
 
@@ -52,7 +54,7 @@ def test_shared_out_statistics(B, H, Hkv, D, Sq, Skv, noise_type, causal):
         p = z.softmax(-1)
         want = s.softmax(-1) @ vv, z.logsumexp(-1), p.sum(1), (p * p).sum(1)
         for o, rows, x, y in outs:
-            assert (o[b] - want[0]).abs().max() < 2e-2 and (rows[b] - want[1]).abs().max() < 1e-3
+            assert ((o[b] - want[0]).norm(dim=-1) <= 2e-3 * want[0].norm(dim=-1)).all() and (rows[b] - want[1]).abs().max() < 1e-3
             for got, w in ((x[b], want[2]), (y[b], want[3])):
                 assert ((got - w).abs() <= 1e-3 * w + 1e-12).all(), ((got - w).abs() / w).max()
 
@@ -102,7 +104,7 @@ def test_mean_and_deviation_of_shared_out_keys(B, H, Hkv, D, Sq, Skv, causal, ha
         s = (q[0, h].double() @ kk.T.contiguous() * scale).masked_fill(~seen, float("-inf"))
         p = s.softmax(-1)
         want = p @ vv
-        assert (o[0, h].double() - want).norm() <= 1e-3 * want.norm() and (rows[0, h].double() - s.logsumexp(-1)).abs().max() <= 2.5e-4
+        assert ((o[0, h].double() - want).norm(dim=-1) <= 2e-3 * want.norm(dim=-1)).all() and (rows[0, h].double() - s.logsumexp(-1)).abs().max() <= 2.5e-4
         mean, square = p.sum(0) / n, p.pow(2).sum(0) / n
         std = (square - mean * mean).clamp(min=0).sqrt()
         std[n == 1] = 0

@@ -1,7 +1,9 @@
 """GPU parity of the KeyFormer pair (forward with score perturbation, key statistics) in the workgroup shapes and cache policies
 of the forward, with the noise at every row alignment: keys split over two groups of waves, 128 and 256 queries a workgroup.
 
-Tolerances as in test_gpu_scores.py: 2e-2 on outputs of fp16 probabilities, 1e-3 relative on fp32 key scores."""
+Tolerances: outputs to 2e-3 of each query's 2-norm (fp16 probabilities and one fp16 rounding, 2^-11 each at most, are some 3e-4 of a
+norm; an element of an output is 0.02 to 0.05 at these lengths, so that an absolute bound of that size would see nothing),
+1e-3 relative on fp32 key scores as in test_gpu_scores.py."""
 import pytest
 import torch
 
@@ -59,8 +61,9 @@ def test_keyformer_in_every_shape_and_row_alignment(B, Hq, Hkv, S, D, half, spar
     for b in range(B):
         for h in range(Hq):
             s = (q[b, h].float() @ k[b, h * Hkv // Hq].float().T * scale).masked_fill(~keep, float("-inf"))
-            err = (o[b, h].float() - s.softmax(-1) @ v[b, h * Hkv // Hq].float()).abs().max()
-            assert err < 2e-2, f"batch {b} head {h}: output off by {err:.3g}"
+            want = s.softmax(-1) @ v[b, h * Hkv // Hq].float()
+            err = ((o[b, h].float() - want).norm(dim=-1) / want.norm(dim=-1)).max()
+            assert err <= 2e-3, f"batch {b} head {h}: a query's output off by {err:.3g} of its norm"
             want = ((s + noise[b, h].float().masked_fill(~keep, 0)) / tau).softmax(-1).sum(0)
             rel = ((c[b, h] - want).abs() / want).max()
             assert rel < 1e-3, f"batch {b} head {h}: scores off by {rel:.3g} relative"

@@ -1,7 +1,7 @@
 """GPU parity of attention with key statistics in one launch on short prompts (33 to 128 queries, at most 128 keys) and one past.
 
-Tolerances as in test_gpu_scores.py: 2e-2 on outputs of fp16 probabilities, 1e-3 relative on fp32 key scores; a deviation is
-known to 1e-3 of its column's root mean square."""
+Tolerances: outputs to 2e-3 of each query's 2-norm (fp16 probabilities and one fp16 rounding, 2^-11 each at most, are some 3e-4
+of a norm), 1e-3 relative on fp32 key scores as in test_gpu_scores.py; a deviation is known to 1e-3 of its column's root mean square."""
 import pytest
 import torch
 
@@ -39,7 +39,8 @@ def test_short_prompts(B, H, Hkv, D, Sq, Skv, noise_type, causal):
     assert torch.equal(half[0], o) and torch.equal(half[1], rows) and torch.equal(half[2], x.half()) and (half[3] == -1).all()
     kk, vv = (t.double().repeat_interleave(H // Hkv, 1) for t in (k, v))
     s = (q.double() @ kk.transpose(2, 3).contiguous() * scale).masked_fill(hidden, float("-inf"))
-    assert (o.double() - s.softmax(-1) @ vv).abs().max() < 2e-2
+    want = s.softmax(-1) @ vv
+    assert ((o.double() - want).norm(dim=-1) <= 2e-3 * want.norm(dim=-1)).all()
     z = s if noise is None else ((s + noise.double()) / tau).masked_fill(hidden, float("-inf"))
     p = z.softmax(-1)
     assert (rows - z.logsumexp(-1)).abs().max() < 1e-3
