@@ -334,11 +334,13 @@ int trn_gate_f16(const void* c1, const void* c2, void* out, int64_t rows, int64_
 /*
  * Measurement aid, no counterpart in the reference: the name (as a profiler's kernel trace prints it) of the kernel
  * instantiation that trn_attn_fwd_f16 launches for this problem -- decided by the same rules as the launch itself,
- * so that a benchmark can say which kernel its timing belongs to.  with_noise: as if a noise tensor were passed.
- * It speaks for trn_attn_fwd_f16 only: fp32 noise, no workspace.  With at most 32 queries per head the other entry
- * points launch the same kernel template with other last arguments -- fp16 noise (trn_attn_fwd_stats_half_f16) shows
- * as <..., 2> where this function says <..., 1>, and a workspace that splits the keys turns the column shares
- * (the middle argument) back to 1.  Returns "" for an invalid descriptor.  The string is static.
+ * so that a benchmark can say which kernel its timing belongs to.  with_noise: as if a noise tensor were passed, with
+ * the noise strides of desc (all three zero: a contiguous one), at an address that is a multiple of 128 (1) or not (2):
+ * noise rows on whole lines may be requested past the caches.
+ * It speaks for trn_attn_fwd_f16 only: fp32 noise, no workspace, no statistics.  The other entry points launch other
+ * instantiations: fp16 noise and statistics change the last argument of the decode kernel, a workspace that splits the keys
+ * turns its column shares (the middle argument) back to 1, fp16 noise on prompts and short prompts with statistics have
+ * kernels of their own.  Returns "" for an invalid descriptor.  The string is static.
  */
 const char* trn_attn_fwd_kernel_name(const trn_attn_desc* desc, int32_t with_noise);
 

@@ -118,6 +118,16 @@ def test_kernel_name_follows_the_launch_rules(lib):
     assert name(seq_q=2048, n_q_heads=71, n_kv_heads=1, head_dim=64) == "trn::attn_fwd16_kernel<64, 4, false>"
     assert name(1, seq_q=4096, **llama) == "trn::attn_fwd_kernel<128, 8, true>"
     assert name(1, seq_q=512, **llama) == "trn::attn_fwd_kernel<128, 4, true>"
+    # noise past the caches: more than the last-level cache holds, rows on whole 128-byte lines
+    noise = lambda pitch: dict(noise_stride_s=pitch, noise_stride_h=pitch * 2048, noise_stride_b=32 * pitch * 2048)
+    assert name(1, seq_q=2048, **llama) == "trn::attn_fwd_kernel<128, 4, false>"
+    assert name(2, seq_q=2048, **llama) == "trn::attn_fwd_kernel<128, 4, true>"
+    assert name(1, seq_q=2048, **noise(2080), **llama) == "trn::attn_fwd_kernel<128, 4, false>"
+    assert name(1, seq_q=2048, **noise(2052), **llama) == "trn::attn_fwd_kernel<128, 4, true>"
+    assert name(2, seq_q=4096, **llama) == "trn::attn_fwd_kernel<128, 8, false>"
+    assert name(1, seq_q=1792, **llama) == "trn::attn_fwd_split_kernel<128, false, true>"
+    assert name(1, seq_q=1800, **llama) == "trn::attn_fwd_split_kernel<128, false, false>"
+    assert name(1, seq_q=1536, n_q_heads=71, n_kv_heads=1) == "trn::attn_fwd_kernel<64, 4, false>"
     assert name(seq_q=16, seq_kv=1040, causal=0, **llama) == "trn::attn_decode_kernel<128, 4, 0>"
     assert name(1, seq_q=16, seq_kv=1040, causal=0, n_q_heads=71, n_kv_heads=71, head_dim=64) == "trn::attn_decode_kernel<64, 2, 1>"
     assert name(seq_q=16, seq_kv=100, causal=0, **llama) == "trn::attn_decode_kernel<128, 1, 0>"    # short cache

@@ -553,19 +553,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
 // that take every other key tile each.
 enum class NoiseShape { Narrow, Wide, Split };
 
-// fp32 noise in the cache policy that goes with the shape (see noise_streams(); the third parameter only keeps the name that
-// traces and trn_attn_fwd_kernel_name() show)
-template <int D, int NW, bool>
+// fp32 noise.  USUAL: in the cache policy of the shape's usual sizes -- past the caches for 256 queries of 128, through them
+// elsewhere -- or in the other one (see noise_streams()).
+template <int D, int NW, bool USUAL>
 __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    attn_fwd_body<D, NW, false, D == 128 && NW == 8, false>(a);
-#endif
-}
-// ... in the other policy
-template <int D, int NW>
-__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd_other_policy_kernel(const AttnArgs a) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    attn_fwd_body<D, NW, false, !(D == 128 && NW == 8), false>(a);
+    attn_fwd_body<D, NW, false, (D == 128 && NW == 8) == USUAL, false>(a);
 #endif
 }
 template <int D, int NW>
@@ -586,7 +579,7 @@ static void launch_rows(const AttnArgs& a, bool stream_noise, const dim3& g, hip
     const dim3 t(NW * 64);
     if (a.n16) hipLaunchKernelGGL((attn_fwd_half_noise_kernel<D, NW>), g, t, 0, s, a);
     else if (stream_noise == (D == 128 && NW == 8)) hipLaunchKernelGGL((attn_fwd_kernel<D, NW, true>), g, t, 0, s, a);
-    else hipLaunchKernelGGL((attn_fwd_other_policy_kernel<D, NW>), g, t, 0, s, a);
+    else hipLaunchKernelGGL((attn_fwd_kernel<D, NW, false>), g, t, 0, s, a);
 }
 
 template <int D>
@@ -685,10 +678,21 @@ extern "C" const char* trn_attn_fwd_kernel_name(const trn_attn_desc* d, int32_t 
     if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0))
         return attn_decode_kernel_name(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
     if (!with_noise) return attn_fwd16_kernel_name(d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0));
-    const NoiseShape shape = noise_shape(d);       // (fp32 noise in the policy of the shape's usual size; the others have names of their own)
-    if (shape == NoiseShape::Split) return d128 ? "trn::attn_fwd_split_kernel<128, false, false>" : "trn::attn_fwd_split_kernel<64, false, false>";
-    if (d128) return shape == NoiseShape::Wide ? "trn::attn_fwd_kernel<128, 8, true>" : "trn::attn_fwd_kernel<128, 4, true>";
-    return shape == NoiseShape::Wide ? "trn::attn_fwd_kernel<64, 8, true>" : "trn::attn_fwd_kernel<64, 4, true>";
+    trn_attn_desc n = *d;
+    if (!n.noise_stride_s && !n.noise_stride_h && !n.noise_stride_b) {       // (no noise described: a contiguous one)
+        n.noise_stride_s = n.seq_kv; n.noise_stride_h = n.seq_q * n.noise_stride_s; n.noise_stride_b = n.n_q_heads * n.noise_stride_h;
+    }
+    const bool stream = noise_streams(&n, reinterpret_cast<const void*>((uintptr_t)(with_noise == 2 ? 16 : 128)), false);
+    const NoiseShape shape = noise_shape(d);
+    if (shape == NoiseShape::Split) {
+        if (d128) return stream ? "trn::attn_fwd_split_kernel<128, false, true>" : "trn::attn_fwd_split_kernel<128, false, false>";
+        return stream ? "trn::attn_fwd_split_kernel<64, false, true>" : "trn::attn_fwd_split_kernel<64, false, false>";
+    }
+    const bool wide = shape == NoiseShape::Wide, usual = stream == (d128 && wide);
+    if (d128) return wide ? (usual ? "trn::attn_fwd_kernel<128, 8, true>" : "trn::attn_fwd_kernel<128, 8, false>")
+                          : (usual ? "trn::attn_fwd_kernel<128, 4, true>" : "trn::attn_fwd_kernel<128, 4, false>");
+    return wide ? (usual ? "trn::attn_fwd_kernel<64, 8, true>" : "trn::attn_fwd_kernel<64, 8, false>")
+                : (usual ? "trn::attn_fwd_kernel<64, 4, true>" : "trn::attn_fwd_kernel<64, 4, false>");
 }
 
 extern "C" int trn_attn_fwd_f16(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o,

@@ -8,7 +8,7 @@ returns None.  Nothing here allocates device memory.
 from __future__ import annotations
 
 import ctypes as C
-from typing import Callable, Optional
+from typing import Callable, Optional, Union
 
 import torch
 
@@ -158,10 +158,15 @@ def qknorm_attention(q, k, v, o, scale: float, causal: bool, gamma_q: Optional[t
     _lib.check("trn_attn_qknorm_f16", st)
 
 
-def attention_kernel_name(q, k, v, o, scale: float, causal: bool, with_noise: bool = False) -> str:
-    """Name of the kernel instantiation `attention` launches for these tensors, as a profiler prints it."""
-    d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, None, 1.0)
-    return _lib.load().trn_attn_fwd_kernel_name(C.byref(d), 1 if with_noise else 0).decode()
+def attention_kernel_name(q, k, v, o, scale: float, causal: bool, with_noise: Union[bool, torch.Tensor] = False) -> str:
+    """Name of the kernel instantiation `attention` launches for these tensors, as a profiler prints it.  with_noise: the
+    noise, or True for a contiguous one on whole cache lines."""
+    noise = with_noise if isinstance(with_noise, torch.Tensor) else None
+    if noise is not None:
+        _dev_float(noise, "noise")
+    d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, noise, 1.0)
+    kind = int(bool(with_noise)) if noise is None else 2 if noise.data_ptr() % 128 else 1
+    return _lib.load().trn_attn_fwd_kernel_name(C.byref(d), kind).decode()
 
 
 def attention_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> int:
