@@ -7,7 +7,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,cols", [(3072, 1024), (3073, 1024), (9000, 520), (9001, 1016), (3173, 4096), (3174, 4096), (40, 2056), (6000, 2064),
-                                       (2258, 8192), (2259, 8192), (33, 4104), (4400, 4208), (700, 2048), (5, 8200), (20000, 24)])
+                                       (2258, 8192), (2259, 8192), (33, 4104), (4400, 4208), (700, 2048), (5, 8200), (20000, 24),
+                                       (4150, 1024), (4151, 1024), (8192, 520), (8193, 520), (8192, 1016), (8193, 1016)])
 @pytest.mark.parametrize("in_place", [False, True])
 def test_rmsnorm_forms(rows, cols, in_place):
     from triton_amd import ops

@@ -1,6 +1,7 @@
 // RMSNorm over rows of fp16 data: one pass, the row held in registers between the mean-square
 // reduction and the scale.  HBM-bound: 16-byte loads, LPR lanes cooperate on one row and reduce
 // with cross-lane shuffles; rows*cols*2 bytes read, the same written.
+#include <type_traits>
 #include "common.h"
 
 namespace trn {
@@ -80,16 +81,24 @@ static hipError_t launch_form(const void* x, const void* gamma, void* y, int64_t
 // matters once the resident waves ask for more than the chip takes at a time.  us, before / late / early: 16 x 4096 5.1 / 4.6 /
 // 3.9, 396 x 5560 10.4 / 6.7 / 5.4, 300 x 8192 13.3 / 7.9 / 6.2, 1929 x 3216 8.6 / 6.7 / 6.4, 3072 x 4096 11.1 / 9.6 / 8.8, 3400 x
 // 4096 11.7 / 10.7 / 12.2, 4096 x 4096 12.8 / 11.4 / 12.5; 1900 x 8192 17.2 / 12.3 / 11.2, 3072 x 6000 17.8 / 14.7 / 14.3, 2500 x
-// 8192 19.7 / 16.4 / 18.2; 9000 x 2048 15.9 / 15.8 / 14.5; 16000 x 1024 12.8 / 13.1 / 12.7, 8000 x 1024 6.6 / 6.3 / 6.7; 12000 x
-// 512 6.8 / 6.8 / 6.5.
+// 8192 19.7 / 16.4 / 18.2; 9000 x 2048 15.9 / 15.8 / 14.5; 12000 x 512 6.8 / 6.8 / 6.5.
+// Two vectors a lane: 8192 rows are the waves that the chip holds at once (8 workgroups of 4 rows on each of 256 CUs).  Up to
+// there all rows ask at the same moment, and from some 8.5 MB on gamma is better left for later; with more rows the workgroups
+// start one by one as others end, and it is not.  late / early: 5000 x 1024 5.06 / 5.06, 7000 x 640 5.25 / 5.31, 7000 x 896 5.78 /
+// 6.20, 8192 x 520 5.52 / 5.57, 8192 x 768 5.89 / 6.30, 8192 x 1024 6.96 / 7.90; 8200 x 520 6.45 / 5.96, 8200 x 768 7.46 / 6.78, 8200 x
+// 1024 8.36 / 7.87, 12000 x 1016 11.74 / 11.09, 16000 x 1024 14.29 / 13.37; but 2500 x 1024 4.13 / 3.97, 3500 x 520 4.22 / 4.20.
 template <int LPR, int NV>
 static hipError_t launch(const void* x, const void* gamma, void* y, int64_t n_rows, int64_t inner_rows,
                          int cols, int64_t xo, int64_t ldx, int64_t yo, int64_t ldy, int64_t row_start,
                          float eps, hipStream_t s) {
-    const int64_t bytes = n_rows * cols * 2;
-    const bool early = NV == 2 ? n_rows <= 3072 || n_rows > 9000 : NV == 8 ? bytes <= 26000000 : NV == 16 ? bytes <= 37000000 : NV < 8;
-    if (early) return launch_form<LPR, NV, true>(x, gamma, y, n_rows, inner_rows, cols, xo, ldx, yo, ldy, row_start, eps, s);
-    return launch_form<LPR, NV, false>(x, gamma, y, n_rows, inner_rows, cols, xo, ldx, yo, ldy, row_start, eps, s);
+    auto form = [&](auto early) { return launch_form<LPR, NV, decltype(early)::value>(x, gamma, y, n_rows, inner_rows, cols, xo, ldx, yo, ldy, row_start, eps, s); };
+    if constexpr (NV == 1 || NV == 4) return form(std::true_type{});
+    else if constexpr (NV == 32) return form(std::false_type{});        // (gamma's 32 vectors beside the row's: registers)
+    else {
+        const int64_t bytes = n_rows * cols * 2;
+        const bool early = NV == 2 ? n_rows > 8192 || bytes <= 8500000 : bytes <= (NV == 8 ? 26000000 : 37000000);
+        return early ? form(std::true_type{}) : form(std::false_type{});
+    }
 }
 
 }  // namespace trn
