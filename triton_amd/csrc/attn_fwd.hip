@@ -900,8 +900,11 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         return TRN_E_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
-    if ((col_sum || col_sumsq) && d->seq_q > 32)
-        return launch_attn_short(a, d->head_dim, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;      // (attn_short_suits: the callers see to it)
+    if ((col_sum || col_sumsq) && d->seq_q > 32) {
+        // (what that kernel does not do: the callers see to it)
+        if (!attn_short_suits(d->seq_q, d->seq_kv) || d->q_norm || k_norm || probs) return TRN_E_UNSUPPORTED;
+        return launch_attn_short(a, d->head_dim, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+    }
     // a chunk of queries on a long cache, with the workspace for it: the keys shared out over workgroups
     if (workspace && !noise && !col_sum && !col_sumsq && !probs) {
         const int64_t need = attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
