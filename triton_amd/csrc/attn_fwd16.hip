@@ -415,8 +415,10 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         auto handover = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's share of stages Kn and Vc is in LDS
             __syncthreads();                      // ... and everyone's; Kc and Vn have had their last readers
-            // (the shares of a long cache wait for HBM, not for issue: all at once, 100 queries on 4100 keys, whole step 66.5 ->
-            // 66.2 us)
+            // (the shares of a long cache wait for HBM, not for issue: all at once, which tells where many heads of 64 share a
+            // long one.  Whole steps, us, dealt out / at once: 71 heads of 64, 100 on 16000 104.7 / 101.7, 100 on 4000 49.8 / 49.0,
+            // 64 on 6000 50.3 / 50.3; 32 of 128, 100 on 4000 48.7 / 49.1, 128 on 16000 102.5 / 103.1, 64 on 8000 49.7 / 49.9; 16 of
+            // 64, 100 on 8000 22.0 / 22.6, 128 on 16000 27.8 / 27.8; 8 of 128, 100 on 8000 25.9 / 26.2)
             if constexpr (SHARE) {
 #pragma unroll
                 for (int i = 0; i < 2 * NI; ++i) refill(i);
