@@ -218,9 +218,9 @@ int trn_attn_fwd_stats_f16(const trn_attn_desc* desc, const void* q, const void*
  * unit of that product -- 8192 keys for 8 heads of 128, 16384 for 16 -- but never fewer than 4096) and how many bytes
  * that takes, 0 otherwise.  Given a zero-initialised workspace of at least
  * that many bytes (256-byte aligned, as for trn_attn_fwd_ws_f16) the attention runs with its keys split over
- * workgroups, and the statistics -- which need the merged row normalisers -- follow in a second launch, over all keys
- * at once; lse (lse_pert with noise) is then required as the buffer that carries the normalisers between the two.
- * Without a workspace, with one that is too small, without that buffer, or for a problem that would not be split,
+ * workgroups, and the second launch merges their results and sums up the statistics, a share of the keys per workgroup.
+ * The split is taken by calls that ask for the row normalisers of their scores (lse, or lse_pert with noise).
+ * Without a workspace, with one that is too small, without that output, or for a problem that would not be split,
  * the call is trn_attn_fwd_stats_f16.  Results as trn_attn_fwd_stats_f16 to the stated tolerances (the shares are
  * merged in a fixed order: the result does not depend on the run).  Neither has a counterpart in the reference, whose
  * generated kernels load the whole key axis in one tile (TritonGen.py:2474-2547).

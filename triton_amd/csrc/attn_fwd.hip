@@ -763,9 +763,9 @@ extern "C" int trn_attn_fwd_stats_ws_f16(const trn_attn_desc* d, const void* q, 
     if (!out_sum && !out_sumsq) return TRN_E_NULL;
     if (d->q_norm) return TRN_E_UNSUPPORTED;
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
-    // Few queries on a long cache: the keys are split over workgroups (which needs the workspace), and the statistics, which
-    // need the merged row normalisers, follow in a second launch -- if the caller gave the buffer that carries the
-    // normalisers.  Everything else runs as trn_attn_fwd_stats_f16.
+    // Few queries on a long cache: the keys are split over workgroups (which needs the workspace), and a second launch merges
+    // them and sums up the statistics -- in calls that ask for the row normalisers.  Everything else runs as
+    // trn_attn_fwd_stats_f16.
     const int64_t need = trn_attn_stats_workspace_bytes(d);
     float* rows = noise ? lse_pert : lse;
     if (workspace && need > 0 && workspace_bytes >= need && rows)

@@ -250,7 +250,7 @@ class KeyFormerAttention(FusedModule):
     """Attention plus key scores C_out[h,j] = sum_i softmax_i((scale*QK^T + noise)/tau)[j]
     (ref_rms.py:171-176; reduced over queries as the generated kernel's C_out is,
     keyformer_llama_benchmark.py:79).  Two launches: forward (+ perturbed row normaliser),
-    then the column-owner pass."""
+    then the column-owner pass; one launch for at most 32 queries or 128 queries and keys."""
     TENSOR_PARAMS = ["C_out", "K", "O", "Q", "V", "noise"]
 
     def __init__(self, scale: Optional[float] = None, causal: bool = True, tau: float = 1.0):
