@@ -1,0 +1,121 @@
+"""GPU parity of KeyFormer's prompts whose row normalisers and key scores come from one pass over the noise (32 queries at a
+time, their exponentials kept in registers): held keys and those beyond, strips and blocks cut off by the end, noise at every
+row alignment, references that have to rise.
+
+Tolerance on the scores against float64: their exponents z are good to a few roundings of |z| log2 e in fp32 (2^-24 relative
+each), a probability to 4 x 2^-24 x |z| ln 2, some 5e-6 at |z| = 30 and 1.7e-4 at 1000; the sums over queries add less than that.  The row normalisers: as the
+exponents, 3e-7 of the largest |z| (a reference that rises by as much leaves its rounding), and a rounding of what lies around 1."""
+import pytest
+import torch
+
+from oracle import ref
+
+pytestmark = pytest.mark.gpu
+
+
+def problem(B, Hq, Hkv, S, D, half, spare, first, seed=1):
+    g = torch.Generator().manual_seed(seed + S)
+    q, k, v = (ref.randn_half((B, h, S, D), g).cuda() for h in (Hq, Hkv, Hkv))
+    pitch = S + spare
+    flat = torch.full((B * Hq * S * pitch + first,), float("nan"), dtype=torch.float16 if half else torch.float32, device="cuda")
+    n = torch.as_strided(flat, (B, Hq, S, S), (Hq * S * pitch, S * pitch, pitch, 1), first)
+    gg = torch.Generator(device="cuda").manual_seed(seed)
+    for b in range(B):
+        n[b] = -torch.log(torch.empty(Hq, S, S, device="cuda").exponential_(generator=gg))
+    return q, k, v, n
+
+
+def scores(q, k, v, n, tau, with_workspace=True):
+    from triton_amd import ops
+    B, H, S, D = q.shape
+    o, rows, c = torch.empty_like(q), torch.full((B, H, S), 9.0, device="cuda"), torch.full((B, H, S), -1.0, device="cuda")
+    need = ops.attention_key_scores_workspace_bytes(q, k, v, o, D ** -0.5, True, True)
+    assert need > 0
+    ws = torch.full((need,), 255, dtype=torch.uint8, device="cuda") if with_workspace else None      # (any contents: NaN here)
+    ops.attention_key_scores(q, k, v, o, D ** -0.5, True, rows, c, noise=n, tau=tau, workspace=ws)
+    torch.cuda.synchronize()
+    return o, rows, c
+
+
+def check(q, k, n, rows, c, tau, tol, heads, largest=0.0):
+    B, H, S, D = q.shape
+    mask = torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1)
+    for b, h in heads:
+        z = (q[b, h].double() @ k[b, h * k.shape[1] // H].double().t() * D ** -0.5 + n[b, h].double()) / tau
+        z.masked_fill_(mask, float("-inf"))
+        lse = z.logsumexp(1)
+        want = (z - lse[:, None]).exp().sum(0)
+        assert ((rows[b, h] - lse).abs() <= 4e-6 + 3e-7 * lse.abs().clamp(min=largest)).all(), (rows[b, h] - lse).abs().max()
+        assert ((c[b, h] - want).abs() <= tol * want + 1e-30).all(), ((c[b, h] - want).abs() / want).max()
+
+
+# B, Hq, Hkv, S, D, fp16 noise, spare elements per row, first element
+CASES = [
+    (9, 72, 1, 161, 64, False, 0, 0), (16, 64, 8, 129, 64, False, 3, 1), (6, 71, 1, 256, 64, True, 0, 0), (5, 71, 71, 287, 64, True, 1, 1),
+    (13, 32, 8, 255, 128, False, 1, 0), (13, 32, 8, 289, 128, True, 0, 1),                     # strips and blocks cut short
+    (2, 24, 6, 1024, 128, False, 0, 0), (2, 24, 6, 1057, 128, True, 0, 1), (1, 40, 8, 1056, 64, False, 32, 0),     # at the end of the held keys
+    (1, 4, 1, 2048, 64, False, 0, 0), (1, 5, 5, 2081, 64, False, 0, 2), (1, 8, 2, 2305, 128, True, 1, 0), (1, 6, 3, 2113, 128, False, 3, 0),
+    (1, 3, 1, 4801, 128, False, 0, 0), (1, 2, 2, 4830, 64, True, 2, 1),                        # the longest rows
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half,spare,first", CASES)
+def test_one_pass_over_the_noise(B, Hq, Hkv, S, D, half, spare, first):
+    tau = 1.5
+    q, k, v, n = problem(B, Hq, Hkv, S, D, half, spare, first)
+    o, rows, c = scores(q, k, v, n, tau)
+    heads = [(0, 0), (B - 1, Hq - 1), (B // 2, Hq // 2)]
+    check(q, k, n, rows, c, tau, 2e-5, heads)
+    # the attention is the plain one, and a second call gives the same bits
+    from triton_amd import ops
+    plain = torch.empty_like(q)
+    ops.attention(q, k, v, plain, D ** -0.5, True)
+    o2, rows2, c2 = scores(q, k, v, n, tau)
+    assert torch.equal(o, plain) and torch.equal(rows, rows2) and torch.equal(c, c2) and torch.equal(o, o2)
+    # without the workspace: forward and statistics with a pass each
+    o1, rows1, c1 = scores(q, k, v, n, tau, with_workspace=False)
+    assert ((o1 - o).float().norm(dim=-1) <= 4e-3 * o.float().norm(dim=-1)).all()
+    assert (c1 - c).norm() <= 1e-4 * c.norm() and (rows1 - rows).abs().max() < 1e-3
+
+
+@pytest.mark.parametrize("S,D,Hq", [(1100, 128, 32), (2200, 64, 8), (1090, 64, 71)])
+def test_references_that_rise_and_rows_without_noise(S, D, Hq):
+    """Scores that jump by hundreds within a row, before and beyond the held keys; keys that are all but masked (-1000), keys that
+    are (-inf), from the first one on, for some rows of a strip and for all."""
+    q, k, v, n = problem(1, Hq, Hq, S, D, False, 0, 0, seed=3)
+    n[0, 0, :, 40:] += 300.0
+    n[0, 0, :, S // 2:] += 300.0
+    n[0, 1, :, :200] = -1e3
+    n[0, 1, 3::5, :10] = 0.0
+    n[0, 2, 300:, :299] = float("-inf")
+    n[0, 2, 7::3, 20:260] = float("-inf")
+    n[0, 3, :, ::2] += 500.0
+    o, rows, c = scores(q, k, v, n, 1.0)
+    check(q, k, n, rows, c, 1.0, 4e-4, [(0, h) for h in range(5)], 1000.0)
+
+
+def test_captured_module_and_where_the_rule_lies():
+    from triton_amd import modules, ops
+    # fp32 from 32 MB (head_dim 64) and 48 to 640 MB (128), causal squares of more than 128 queries only
+    def need(B, H, S, D, causal=True, Skv=None):
+        q, k = (torch.as_strided(torch.empty(1 << 20, device="cuda", dtype=torch.half), (B, H, s, D), (0, 0, D, 1)) for s in (S, Skv or S))
+        return ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, causal, True)
+    assert need(1, 71, 600, 64) > 0 and need(1, 71, 300, 64) == 0 and need(1, 32, 1024, 128) > 0 and need(1, 8, 1536, 128) == 0 and need(1, 8, 2050, 128) > 0
+    assert need(1, 32, 4096, 128) == 0 and need(1, 71, 600, 64, causal=False) == 0 and need(1, 71, 600, 64, Skv=700) == 0
+    assert need(64, 71, 128, 64) == 0 and need(1, 71, 4900, 64) == 0
+    q, k, v, n = problem(1, 71, 1, 608, 64, False, 0, 0)
+    c, o = torch.empty(1, 71, 608, device="cuda"), torch.empty_like(q)
+    m = modules.get("keyformer")
+    t = dict(Q=q, K=k, V=v, O=o, noise=n, C_out=c)
+    args = [t[p] for p in m.TENSOR_PARAMS]
+    m.forward(*args)
+    want_c, want_o = c.clone(), o.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        m.forward(*args)
+    for _ in range(3):
+        c.fill_(-1.0); o.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(c, want_c) and torch.equal(o, want_o)

@@ -119,6 +119,13 @@ int attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const fl
 // Whether the kernels that read all of this noise request it past the caches (attn_fwd.hip).
 bool noise_streams(const trn_attn_desc* d, const void* noise, bool n16);
 
+// KeyFormer's row normalisers and key scores in one pass over the noise (attn_noise_strips.hip): in how many workgroups per head
+// (0: this problem does not suit it), and with how much workspace, of any contents, for noise of either type.
+int noise_strip_slots(const trn_attn_desc* d, bool n16);
+int64_t noise_strips_workspace_bytes(const trn_attn_desc* d);
+hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void* k, const void* noise, bool n16, float* lse, void* out,
+                               bool s16, void* workspace, hipStream_t s);
+
 // One workgroup per head and 32 queries, whose eight waves split the keys (attn_decode.hip): at most 32 queries per head
 // (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.
 bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);

@@ -1,0 +1,521 @@
+// KeyFormer's perturbed row normalisers and key scores in one pass over the noise:
+//
+//     lse_i = log sum_j exp(z_ij),   out_j = sum_i exp(z_ij - lse_i),   z = (scale * Q K^T + noise) / tau
+//
+// A column sum needs the finished row normalisers, so that two passes -- the forward's, row by row, and the statistics', column
+// by column -- read all of the noise twice, at the rate of HBM both times (the last-level cache returns lines no faster than
+// HBM: a 128 MB buffer read over and over 7.0 - 7.4 TB/s, 2 GB 6.3 - 7.1).  Here a workgroup takes 32 queries at a time and keeps their
+// exponentials in registers, 32 x 2048 of them in fp32 -- half of a CU's register file --, until the rows are summed up; the
+// scores then follow without another look at the noise.  Only what a row has beyond 2048 keys is read, and multiplied, again.
+// The attention itself, which does not depend on the noise, runs on the plain kernel of attn_fwd16.hip.
+//
+// Eight waves take a strip's 32-key blocks in turn, each through a private part of LDS (K one block ahead, noise two), so that
+// the walk has no barrier.  S[query][key], a lane one key and 16 of the 32 queries: the scores' sums over the queries are then
+// sums within a lane, the blocks of a wave are the same columns in every strip, and a workgroup adds them up in LDS without
+// atomics; the second launch adds the workgroups of a head in a fixed order.  Results repeat bit for bit.
+//
+// What bounds it: a wave's block is a chain -- K and noise out of LDS, eight MFMAs that wait for each other, the exponentials --
+// that two waves a SIMD overlap only in part, and 32 to 64 KB of noise in flight a CU.  71 heads of 64, 1536 keys, fp32: 79 us for
+// 0.37 GB (4.7 TB/s; 59 with the noise in the caches, 51 without its and K's requests at all); 32 heads of 128, 2048: 80 us, where
+// the forward's noise and the statistics took 121 beside the attention's 40.
+//
+// All requests are global -> LDS loads issued as inline assembly and counted by hand: a wave's requests run ahead over the end
+// of a strip into the next, and the compiler, which cannot see which of them a read depends on, would wait for all.
+#include "attn.h"
+
+namespace trn {
+
+struct StripArgs {
+    const half_t* q; const half_t* k; const void* noise; float* lse; float* out; float* part;
+    int B, Hq, Hkv, S, n_strips, n_slots;
+    int64_t qb, qh, qs, kb, kh, ks, nb, nh, ns;
+    float c2, c3;      // scale*log2(e)/tau, log2(e)/tau
+    int s16;
+};
+
+[[maybe_unused]] constexpr int kHeldBlocks = 8;      // of 32 keys, per wave
+// keys whose column sums fit beside the stages, of 8 waves a CU in one workgroup or two
+constexpr int strip_keys(int waves, int head_dim) { return waves == 8 ? 4864 : head_dim == 128 ? 1664 : 5120; }
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// Four of a wave's global -> LDS loads of BYTES a lane, LSTEP bytes of LDS and `step` bytes of memory from each to the next:
+// lane l's land at lds + 4 l (16 l), offsets past the range as zeros.  lds and so end up where a fifth would go.
+template <int BYTES, bool NT, int LSTEP>
+__device__ __forceinline__ void request4(uint4_t rs, uint32_t& lds, int vo0, int vo1, int vo2, int vo3, int& so, int step) {
+#define TRN_NEXT "s_add_u32 m0, m0, %8\n\ts_add_u32 %0, %0, %7\n\t"
+#define TRN_REQ(op_, mod_)                                                                                                      \
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\t" op_ " %2, %6, %0 offen " mod_ "\n\t" TRN_NEXT op_ " %3, %6, %0 offen " mod_ "\n\t" TRN_NEXT    \
+                 op_ " %4, %6, %0 offen " mod_ "\n\t" TRN_NEXT op_ " %5, %6, %0 offen " mod_ "\n\ts_add_u32 %0, %0, %7"         \
+                 : "+s"(so) : "s"(lds), "v"(vo0), "v"(vo1), "v"(vo2), "v"(vo3), "s"(rs), "s"(step), "n"(LSTEP) : "memory", "scc")
+    if constexpr (BYTES == 16) { if constexpr (NT) TRN_REQ("buffer_load_dwordx4", "nt lds"); else TRN_REQ("buffer_load_dwordx4", "lds"); }
+    else if constexpr (BYTES == 4) TRN_REQ("buffer_load_dword", "lds");
+    else TRN_REQ("buffer_load_ushort", "lds");
+#undef TRN_REQ
+#undef TRN_NEXT
+    lds += 4 * LSTEP;
+}
+__device__ __forceinline__ void request1(uint4_t rs, uint32_t lds, int vo, int so) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" :: "s"(lds), "v"(vo), "s"(rs), "s"(so) : "memory");
+}
+template <int N> __device__ __forceinline__ void wait_requests() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
+__device__ __forceinline__ half8_t operand(uint32_t at) { return *(__attribute__((address_space(3))) const half8_t*)(uintptr_t)at; }
+__device__ __forceinline__ uint4_t descriptor(const void* p, int64_t bytes) {
+    const uint64_t u = reinterpret_cast<uint64_t>(p);
+    return uint4_t{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u), (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32)),
+                   (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
+template <int CTRL> __device__ __forceinline__ float dpp(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+// The lane, where it is not worth a register over the walk.
+__device__ __forceinline__ int lane_now() {
+    int r;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(r));
+    return r;
+}
+// f over the 32 lanes of each half, of 16 values a lane: lane l ends with that of value l % 16.  Each step hands half of the
+// values to a lane that differs in one more bit of its number (ror 8, half mirror, two quad permutations) and keeps the others.
+template <class F>
+__device__ __forceinline__ float reduce_keys(const float (&v)[16], int lane, F f) {
+    float a[8], b[4], c[2];
+    const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2, b0 = lane & 1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = f(b3 ? v[i + 8] : v[i], dpp<0x128>(b3 ? v[i] : v[i + 8]));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) b[i] = f(b2 ? a[i + 4] : a[i], dpp<0x141>(b2 ? a[i] : a[i + 4]));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) c[i] = f(b1 ? b[i + 2] : b[i], dpp<0x4e>(b1 ? b[i] : b[i + 2]));
+    float x = f(b0 ? c[1] : c[0], dpp<0xb1>(b0 ? c[0] : c[1])), y = x;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+    return f(x, y);
+}
+#endif
+
+// NB: bytes of noise a lane requests at a time: 16 fp32 rows on 16-byte addresses, 4 fp32, 2 fp16.
+template <int D, int NB, bool NT, int NW>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_kernel(const StripArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int NKS = D / 16, CPR = D / 8, RPI = 64 / CPR;
+    constexpr int NK = 32 / RPI;                 // requests of a block's K
+    constexpr int NN = NB == 16 ? 4 : 16;        // ... and of its noise
+    constexpr int nsz = NB == 2 ? 2 : 4, NQW = 8 / NW, kKeys = strip_keys(NW, D);
+    __shared__ __attribute__((aligned(1024))) half_t Ks[NW * 32 * D];
+    __shared__ __attribute__((aligned(1024))) float Ns[NW * 2 * 1024];
+    __shared__ __attribute__((aligned(1024))) half_t Qs[32 * D];
+    __shared__ __attribute__((aligned(256))) float2_t St[NW * 32];       // a strip's row references and sums, by wave
+    __shared__ __attribute__((aligned(256))) float Wr[NW * 32];          // a value per row: the references, or what one lane has for all
+    __shared__ __attribute__((aligned(256))) float Cs[kKeys];                // the column sums
+
+    const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int BH = a.B * a.Hq;
+    const int slot = (int)(blockIdx.x / BH), j = blockIdx.x % BH;
+    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
+    const int kvslot = j % nkv, g = j / nkv;
+    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+
+    const uint4_t qrs = descriptor(a.q + b * a.qb + head * a.qh, ((int64_t)(a.S - 1) * a.qs + D) * 2);
+    const uint4_t krs = descriptor(a.k + b * a.kb + kvh * a.kh, ((int64_t)(a.S - 1) * a.ks + D) * 2);
+    const uint4_t nrs = descriptor(static_cast<const char*>(a.noise) + (b * a.nb + head * a.nh) * nsz, ((int64_t)(a.S - 1) * a.ns + a.S) * nsz);
+
+    // ---- K and Q: RPI rows a request, the 16-byte chunks of a row swizzled by its number on their way in
+    const int krow = lane / CPR;
+    int kvo[D == 128 ? 4 : 2];                   // (the swizzle's part that differs from request to request)
+#pragma unroll
+    for (int p = 0; p < (D == 128 ? 4 : 2); ++p) kvo[p] = (int)(krow * a.ks * 2) + (((lane % CPR) ^ swz<D>(p * RPI + krow)) << 4);
+    // ---- noise: row 8p + 4h + i of a block at 1024 p + 256 i + 128 h bytes, its keys in order: what a lane reads of row number r
+    // of its 16 lies at 256 r + 4 lane
+    const int nvo = NB == 16 ? (int)((4 * ((lane >> 3) & 1) + (lane >> 4)) * a.ns * 4) + 16 * (lane & 7) : (int)((4 * h * a.ns + c) * nsz);
+    float* const nst = Ns + wave * 2 * 1024;
+    const uint32_t klds = lds_address(Ks + wave * 32 * D), nlds = lds_address(nst), qlds = lds_address(Qs) + wave * 1024;
+    const uint32_t kplace = klds + (c * D + ((h ^ swz<D>(c)) << 3)) * 2;      // operand ks of row c: 16-byte chunk 2 ks + h, at kplace ^ (ks << 5)
+
+    // ---- the wave's list of blocks: of strip after strip, those beyond the last kHeldBlocks first, then these, then the first
+    // ones again
+    struct Cursor { int k, i, n, q0, again; };
+    auto open = [&](Cursor& x) __attribute__((always_inline)) {      // strip number x.k of this workgroup: long and short ones in turn
+        const int idx = x.k * a.n_slots + ((x.k & 1) ? a.n_slots - 1 - slot : slot);
+        if (idx >= a.n_strips) { x.q0 = -1; x.n = 0; return; }
+        x.q0 = 32 * idx;
+        const int blocks = (min(a.S, x.q0 + 32) + 31) >> 5;
+        x.n = max(0, (blocks - wave + NW - 1) / NW);
+    };
+    auto advance = [&](Cursor& x) __attribute__((always_inline)) {
+        if (x.q0 < 0) return;
+        ++x.i;
+        const int early = x.n - kHeldBlocks;
+        if (x.i < (x.again ? early : x.n)) return;
+        x.i = 0;
+        if (!x.again && early > 0) { x.again = 1; return; }
+        x.again = 0;
+        do { ++x.k; open(x); } while (x.q0 >= 0 && x.n == 0);
+    };
+    // (past the end of the list the first block is asked for: its stage has no reader)
+    const int kkey = (int)(a.ks * 2), kstep = RPI * kkey, nkey = (int)(a.ns * nsz);       // bytes from key to key, request to request, row to row
+    auto key_of = [&](const Cursor& x) __attribute__((always_inline)) { return x.q0 < 0 ? 0 : 32 * (wave + NW * x.i); };
+    auto fetch_k = [&](uint32_t& at, int& so) __attribute__((always_inline)) {       // four requests, of NK
+        request4<16, false, 1024>(krs, at, kvo[0], kvo[1], kvo[D == 128 ? 2 : 0], kvo[D == 128 ? 3 : 1], so, kstep);
+    };
+    auto noise_at = [&](const Cursor& x) __attribute__((always_inline)) { return max(x.q0, 0) * nkey + key_of(x) * nsz; };
+    auto fetch_noise = [&](uint32_t& at, int& so) __attribute__((always_inline)) {   // four requests, of NN
+        if constexpr (NB == 16) request4<16, NT, 1024>(nrs, at, nvo, nvo, nvo, nvo, so, 8 * nkey);
+        else {
+            request4<NB, false, 256>(nrs, at, nvo, nvo, nvo, nvo, so, nkey);
+            so += 4 * nkey;                      // (rows 4 to 7 of eight are those of the other half of the lanes)
+        }
+    };
+    const int qrow = (int)(a.qs * 2);
+    auto fetch_q = [&](int q0) __attribute__((always_inline)) {      // eight requests or, of head_dim 64, four hold a strip's queries
+#pragma unroll
+        for (int i = 0; i < (D == 128 ? NQW : 1); ++i) {
+            const int ln = lane_now(), row = (NW * i + wave) * RPI + ln / CPR;
+            if (D == 128 || wave < 4) request1(qrs, qlds + i * NW * 1024, row * qrow + (((ln % CPR) ^ swz<D>(row)) << 4), q0 * qrow);
+        }
+    };
+
+    // the noise runs two blocks ahead, K one: k_next is the key of the block that the noise was last asked for
+    Cursor cn{0, 0, 0, 0, 0}, now{0, 0, 0, 0, 0};
+    open(cn);
+    if (cn.q0 >= 0 && cn.n == 0) { cn.i = -1; advance(cn); }
+    open(now);
+    fetch_q(max(now.q0, 0));
+    auto fetch_block = [&](int stage) __attribute__((always_inline)) {
+        uint32_t at = nlds + stage * 4096;
+        int so = noise_at(cn);
+#pragma unroll
+        for (int i = 0; i < NN; i += 4) fetch_noise(at, so);
+    };
+    fetch_block(0);
+    {
+        uint32_t at = klds;
+        int so = key_of(cn) * kkey;
+#pragma unroll
+        for (int i = 0; i < NK; i += 4) fetch_k(at, so);
+    }
+    advance(cn);
+    fetch_block(1);
+    int k_next = key_of(cn);
+    advance(cn);
+    int stage = 0;
+    for (int i = tid; i < a.S + 31 && i < kKeys; i += NW * 64) Cs[i] = 0.f;
+    wait_requests<2 * NN + NK>();
+    wait_lds();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+
+    constexpr float kNone = -1e30f;              // the reference of a row that has seen no finite score
+    half8_t qA[NKS];
+    float mlane = kNone, lsum = 0.f;             // of the one row a lane keeps: reference and sum
+    auto row_of = [](int ln) __attribute__((always_inline)) { return 8 * ((ln & 15) >> 2) + 4 * (ln >> 5) + (ln & 3); };
+    auto spread = [&](float x, float (&v)[16]) __attribute__((always_inline)) {      // the row's value from one lane to all
+        const int ln = lane_now();
+        float* const wr = Wr + wave * 32;
+        wr[row_of(ln)] = x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4_t t = *reinterpret_cast<const float4_t*>(wr + 8 * i + 4 * (ln >> 5));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[4 * i + e] = t[e];
+        }
+    };
+    bool unseen = true;                          // some row's reference is still to come
+    float16_t held[kHeldBlocks];
+
+    // z - ref of a block, the rows' references being in wr; requests the blocks ahead.  All that can be done before the scores
+    // are there is done between the MFMAs, which wait for each other.
+    auto differences = [&](bool first, int q_next, int key0, int q0, float (&e)[16]) __attribute__((always_inline)) {
+        wait_requests<NN>();                     // this block's K and noise: only the noise of the next was asked for behind them
+        uint32_t at = kplace;
+        if (D == 128) asm volatile("" : "+v"(at));      // (the eight places are not kept in registers)
+        const float16_t zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        constexpr int NQ = 4;                    // operands in registers at a time
+        half8_t kB[NQ];
+#pragma unroll
+        for (int ks = 0; ks < NQ; ++ks) kB[ks] = operand(at ^ (ks << 5));
+        const float* np = nst + stage * 1024 + lane;
+        const float* const rp = Wr + wave * 32 + 4 * h;
+        float gn[16];
+        float16_t s;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            if constexpr (NB == 2) gn[r] = (float)*reinterpret_cast<const half_t*>(np + 64 * r);
+            else gn[r] = np[64 * r];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        uint32_t kat = klds, nat = nlds + stage * 4096;
+        int kso = k_next * kkey, nso = noise_at(cn);
+        constexpr int READ = D == 128 ? NKS - NQ : 1;      // slot from which the stages have been read
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            s = mfma32(qA[ks], kB[ks % NQ], ks == 0 ? zero : s);
+            if (ks + NQ < NKS) kB[ks % NQ] = operand(at ^ ((ks + NQ) << 5));
+            if (ks == READ) wait_lds();
+            if (ks == READ && first) fetch_q(q_next);
+            if (ks >= READ && ks < READ + NK / 4) fetch_k(kat, kso);
+            if (ks == READ + NK / 4) {
+#pragma unroll
+                for (int i = 0; i < NN; i += 4) fetch_noise(nat, nso);
+            }
+            if (ks == READ + NK / 4) { k_next = key_of(cn); advance(cn); stage ^= 1; }
+            if (ks >= NKS / 2) {
+                constexpr int PER = 16 / (NKS / 2);
+                const int first_r = (ks - NKS / 2) * PER;
+#pragma unroll
+                for (int r4 = first_r / 4; r4 < (first_r + PER) / 4; ++r4) {
+                    const float4_t t = *reinterpret_cast<const float4_t*>(rp + 8 * r4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) gn[4 * r4 + i] = __builtin_fmaf(gn[4 * r4 + i], a.c3, -t[i]);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) e[r] = __builtin_fmaf(s[r], a.c2, gn[r]);
+        if (key0 + 31 > q0) {
+            // the first of the strip's rows that sees the lane's key, counted from the lane's first row
+            const int from = key0 + c >= a.S ? 64 : key0 + c - q0 - 4 * h;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) e[r] = 8 * (r / 4) + (r % 4) >= from ? e[r] : -INFINITY;
+        }
+    };
+    // The exponentials of a block relative to references (the first block's maxima) that only rise where a score exceeds them
+    // by 64 -- in fp32 that costs no precision --; what was summed and held is scaled then.
+    auto exponentials = [&](bool first, int q_next, int key0, int q0, int n_held, float (&e)[16], float* l) __attribute__((always_inline)) {
+        differences(first, q_next, key0, q0, e);
+        float top = max3(max3(e[0], e[1], e[2]), e[3], e[4]);
+#pragma unroll
+        for (int r = 5; r < 15; r += 2) top = max3(top, e[r], e[r + 1]);
+        top = fmaxf(top, e[15]);
+        if (unseen || __builtin_amdgcn_ballot_w64(top > 64.0f) != 0) {
+            float f[16];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float4_t t = *reinterpret_cast<const float4_t*>(Wr + wave * 32 + 8 * i + 4 * h);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) e[4 * i + j] += t[j];
+            }
+            const float zmax = reduce_keys(e, lane_now(), [](float x, float y) __attribute__((always_inline)) { return fmaxf(x, y); });
+            const float mn = mlane == kNone ? fmaxf(zmax, kNone) : zmax > mlane + 64.0f ? zmax : mlane;
+            const float fl = fast_exp2(mlane - mn);
+            spread(fl, f);
+            lsum *= fl;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (l) l[r] *= f[r];
+#pragma unroll
+            for (int i = 0; i < kHeldBlocks; ++i)
+                if (i < n_held)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) held[i][r] *= f[r];
+            mlane = mn;
+            unseen = __builtin_amdgcn_ballot_w64(mn == kNone) != 0;
+            spread(mn == kNone ? 0.f : mn, f);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) e[r] -= f[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) e[r] = fast_exp2(e[r]);
+    };
+
+    for (; now.q0 >= 0; ++now.k, open(now)) {
+        const int q0 = now.q0, n = now.n, early = max(0, n - kHeldBlocks), nh = n - early;
+        Cursor nx{now.k + 1, 0, 0, 0, 0};
+        open(nx);
+        const int q_next = max(nx.q0, 0);
+        uint32_t qat = kplace;
+        asm volatile("" : "+v"(qat));            // (as above)
+        qat += lds_address(Qs) - klds;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) qA[ks] = operand(qat ^ (ks << 5));
+        wait_lds();
+        __builtin_amdgcn_s_barrier();            // every wave has its queries: the next strip's may come in
+        asm volatile("" ::: "memory");
+        if (n == 0) fetch_q(q_next);
+        if (lane < 32) Wr[wave * 32 + lane] = 0.f;
+        mlane = kNone; lsum = 0.f; unseen = true;
+        const auto plus = [](float x, float y) __attribute__((always_inline)) { return x + y; };
+        if (early > 0) {
+            float l[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) l[r] = 0.f;
+            for (int i = 0; i < early; ++i) {
+                float e[16];
+                exponentials(i == 0, q_next, 32 * (wave + NW * i), q0, 0, e, l);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) l[r] += e[r];
+            }
+            lsum = reduce_keys(l, lane_now(), plus);
+        }
+#pragma unroll
+        for (int i = 0; i < kHeldBlocks; ++i)
+            if (i < nh) {
+                float e[16];
+                exponentials(i == 0 && early == 0, q_next, 32 * (wave + NW * (early + i)), q0, i, e, nullptr);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) held[i][r] = e[r];
+            }
+        // ---- the rows' normalisers, of all eight waves
+        {
+            float l[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) l[r] = 0.f;
+#pragma unroll
+            for (int i = 0; i < kHeldBlocks; ++i)
+                if (i < nh)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) l[r] += held[i][r];
+            lsum += reduce_keys(l, lane_now(), plus);
+        }
+        const int row = row_of(lane_now());
+        St[wave * 32 + row] = float2_t{mlane, lsum};
+        if (n == 0) wait_requests<0>(); else wait_requests<NK + NN>();      // the next strip's queries
+        wait_lds();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        float mx = kNone, ls = 0.f;
+#pragma unroll
+        for (int half = 0; half < NW; half += 4) {
+            float2_t st[4];
+            float top = mx;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) { st[w] = St[(half + w) * 32 + row]; top = fmaxf(top, st[w][0]); }
+            ls *= fast_exp2(mx - top);
+            mx = top;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) ls = __builtin_fmaf(st[w][1], fast_exp2(st[w][0] - mx), ls);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const float lse2 = mx + fast_log2(ls);
+        const bool real = q0 + row < a.S;
+        if (wave == 0 && (lane & 16) == 0 && real) a.lse[((int64_t)b * a.Hq + head) * a.S + q0 + row] = lse2 * kLn2;
+        // ---- the held blocks' column sums
+        float w[16];
+        spread(real ? fast_exp2(mlane - lse2) : 0.f, w);
+#pragma unroll
+        for (int i = 0; i < kHeldBlocks; ++i)
+            if (i < nh) {
+                float x = held[i][0] * w[0];
+#pragma unroll
+                for (int r = 1; r < 16; ++r) x = __builtin_fmaf(held[i][r], w[r], x);
+                x = half_sum(x);
+                if (h == 0) Cs[32 * (wave + NW * (early + i)) + c] += x;
+            }
+        // ---- ... and the others', once more from K and the noise
+        if (early > 0) {
+            Wr[wave * 32 + row] = real ? lse2 : INFINITY;
+            for (int i = 0; i < early; ++i) {
+                const int key0 = 32 * (wave + NW * i);
+                float e[16];
+                differences(false, 0, key0, q0, e);
+                float x = 0.f;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) x += fast_exp2(e[r]);
+                x = half_sum(x);
+                if (h == 0) Cs[key0 + c] += x;
+            }
+        }
+    }
+    wait_requests<0>();                          // (nothing lands in these stages once they are given up)
+    const int64_t bh = (int64_t)b * a.Hq + head;
+    if (lane < 32)
+        for (int key = 32 * wave + c; key < a.S; key += 32 * NW) {
+            if (a.n_slots == 1) store_stat(a.out, a.s16, bh * a.S + key, Cs[key]);
+            else a.part[(bh * a.n_slots + slot) * a.S + key] = Cs[key];
+        }
+#endif
+}
+
+// The column sums of a head's workgroups, in their order.
+__global__ __launch_bounds__(256) void attn_add_slots_kernel(const float* part, float* out, int n_slots, int Skv, int64_t n, int s16) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int64_t bh = i / Skv, key = i % Skv;
+    const float* p = part + bh * n_slots * Skv + key;
+    float x = 0.f;
+    for (int s = 0; s < n_slots; ++s) x += p[(int64_t)s * Skv];
+    store_stat(out, s16, i, x);
+}
+
+// Where the two launches here -- one where a head has one workgroup -- and the plain attention are faster than the forward with
+// noise and the column statistics: causal prompts whose noise is large enough to pay for the third launch, and for head_dim 128,
+// where a block's K is twice its noise, not those that keep the two passes at the rate of HBM all the time.  us, two passes / here:
+//   fp32  71 heads of 64: 300 keys (13 MB) 22.3 / 22.6, 600 40.6 / 33.4, 1100 106 / 78, 1536 151 / 113, 2050 301 / 235, 2752 457 /
+//         337; 16 of 64: 600 24.2 / 25.7, 1100 (39 MB) 43.6 / 37.3, 2050 89 / 76, 4096 210 / 186; 32 of 128: 1024 (67 MB) 51.9 /
+//         48.7, 1501 94 / 89, 2048 163 / 129, 3000 (576 MB) 298 / 277, 4096 449 / 461; 8 of 128: 1100 40 / 48, 1536 (38 MB) 50 / 55,
+//         2050 (67 MB) 83 / 72, 4096 172 / 150
+//   fp16  71 of 64: 600 (26 MB) 37.7 / 34.4, 1100 77 / 64, 1536 128 / 111, 2752 349 / 318; 16 of 64: 1536 (38 MB) 52 / 42, 2050 (67
+//         MB) 68 / 65, 2752 91 / 100; 32 of 128: 1024 (34 MB) 49.5 / 45.9, 1501 (72 MB) 74.1 / 77.0, 3000 231 / 245; 8 of 128: 2050 (34
+//         MB) 80 / 71, 4096 157 / 139
+static bool strips_suit(const trn_attn_desc* d, bool n16) {
+    if (!d->causal || d->seq_q != d->seq_kv || d->seq_q <= 128) return false;
+    const int64_t bh = (int64_t)d->batch * d->n_q_heads, mb = (bh * d->seq_q * d->seq_q * (n16 ? 1 : 2)) >> 20;
+    if (d->head_dim == 64) return n16 ? mb >= 24 && (bh >= 32 || mb <= 80) : mb >= 32;
+    return n16 ? mb >= 32 && (bh <= 16 || mb <= 64) : mb >= 48 && mb <= 640;
+}
+// Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
+// and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
+// 1536 113 / 124, 2050 243 / 235; 32 of 128: 1024 48.7 / 50.3, 1501 91.6 / 89.1; 16 of 64: 1100 43.9 / 37.3, 1536 50.3 / 44.2.
+static int strip_waves(const trn_attn_desc* d) {
+    return (int64_t)d->batch * d->n_q_heads >= 32 && d->seq_q + 31 <= strip_keys(4, 128) ? 4 : 8;
+}
+
+// Workgroups per head: a workgroup's time is its start and its share of the head's strips, and the chip takes so many at once.
+int noise_strip_slots(const trn_attn_desc* d, bool n16) {
+    const int waves = strip_waves(d);
+    if (!strips_suit(d, n16) || d->seq_q + 31 > strip_keys(waves, d->head_dim)) return 0;
+    const int64_t bh = (int64_t)d->batch * d->n_q_heads, at_once = waves == 8 ? 256 : 512;
+    const int n_strips = (d->seq_q + 31) / 32;
+    const double work = 0.06 * n_strips * (n_strips + 1) + 0.7 * n_strips, start = 3.0;      // (us)
+    int best = 1;
+    double least = 1e30;
+    for (int n = 1; n <= n_strips && n <= 64; ++n) {
+        const double t = (double)((bh * n + at_once - 1) / at_once) * (start + work / n) + 0.02 * n;
+        if (t < least) { least = t; best = n; }
+    }
+    return best;
+}
+
+int64_t noise_strips_workspace_bytes(const trn_attn_desc* d) {
+    const int64_t n = noise_strip_slots(d, false) > 0 ? noise_strip_slots(d, false) : noise_strip_slots(d, true);
+    return n * d->batch * d->n_q_heads * d->seq_kv * 4;
+}
+
+template <int D, int NW>
+static void launch_strips(const StripArgs& a, int nb, bool nt, unsigned grid, hipStream_t s) {
+    const dim3 g(grid), t(NW * 64);
+    if (nb == 2) hipLaunchKernelGGL((attn_noise_strips_kernel<D, 2, false, NW>), g, t, 0, s, a);
+    else if (nb == 4) hipLaunchKernelGGL((attn_noise_strips_kernel<D, 4, false, NW>), g, t, 0, s, a);
+    else if (nt) hipLaunchKernelGGL((attn_noise_strips_kernel<D, 16, true, NW>), g, t, 0, s, a);
+    else hipLaunchKernelGGL((attn_noise_strips_kernel<D, 16, false, NW>), g, t, 0, s, a);
+}
+
+hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void* k, const void* noise, bool n16, float* lse, void* out,
+                               bool s16, void* workspace, hipStream_t s) {
+    StripArgs a;
+    a.q = (const half_t*)q; a.k = (const half_t*)k; a.noise = noise; a.lse = lse; a.out = (float*)out; a.part = (float*)workspace;
+    a.B = d->batch; a.Hq = d->n_q_heads; a.Hkv = d->n_kv_heads; a.S = d->seq_q;
+    a.n_strips = (d->seq_q + 31) / 32; a.n_slots = noise_strip_slots(d, n16);
+    a.qb = d->q_stride_b; a.qh = d->q_stride_h; a.qs = d->q_stride_s;
+    a.kb = d->k_stride_b; a.kh = d->k_stride_h; a.ks = d->k_stride_s;
+    a.nb = d->noise_stride_b; a.nh = d->noise_stride_h; a.ns = d->noise_stride_s;
+    a.c2 = d->scale * kLog2e / d->tau; a.c3 = kLog2e / d->tau;
+    a.s16 = s16 ? 1 : 0;
+    const int64_t bh = (int64_t)a.B * a.Hq;
+    const bool grid16 = aligned16(noise) && pitch16(a.ns, 4) && pitch16(a.nh, 4) && pitch16(a.nb, 4);
+    const int nb = n16 ? 2 : grid16 ? 16 : 4;
+    const bool nt = (reinterpret_cast<uintptr_t>(noise) & 127u) == 0 && !(a.ns & 31) && !(a.nh & 31) && !(a.nb & 31);
+    const unsigned grid = (unsigned)(bh * a.n_slots);
+    const bool wide = strip_waves(d) == 8;
+    if (d->head_dim == 128) { if (wide) launch_strips<128, 8>(a, nb, nt, grid, s); else launch_strips<128, 4>(a, nb, nt, grid, s); }
+    else { if (wide) launch_strips<64, 8>(a, nb, nt, grid, s); else launch_strips<64, 4>(a, nb, nt, grid, s); }
+    if (a.n_slots > 1) {
+        const int64_t n = bh * a.S;
+        hipLaunchKernelGGL(attn_add_slots_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.part, a.out, a.n_slots, a.S, n, a.s16);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace trn

@@ -250,7 +250,8 @@ class KeyFormerAttention(FusedModule):
     """Attention plus key scores C_out[h,j] = sum_i softmax_i((scale*QK^T + noise)/tau)[j]
     (ref_rms.py:171-176; reduced over queries as the generated kernel's C_out is,
     keyformer_llama_benchmark.py:79).  Two launches: forward (+ perturbed row normaliser),
-    then the column-owner pass; one launch for at most 32 queries or 128 queries and keys."""
+    then the column-owner pass; one launch for at most 32 queries or 128 queries and keys; on prompts with
+    much noise the plain attention and then normalisers and scores in one pass over it."""
     TENSOR_PARAMS = ["C_out", "K", "O", "Q", "V", "noise"]
 
     def __init__(self, scale: Optional[float] = None, causal: bool = True, tau: float = 1.0):
@@ -267,7 +268,9 @@ class KeyFormerAttention(FusedModule):
         n4 = _noise_operand(self, _as4(noise, "noise"))
         lsep = self._workspace("lse_pert", (B, Hq, Sq), torch.float32, q.device)
         score, = _score_outputs(self, (C_out,), (B, Hq, Skv))
-        ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lsep, score, noise=n4, tau=self.tau)
+        need = ops.attention_key_scores_workspace_bytes(q, k, v, o, _scale(self.scale, D), self.causal, True)
+        parts = self._workspace("key_parts", (need,), torch.uint8, q.device) if need else None
+        ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lsep, score, noise=n4, tau=self.tau, workspace=parts)
         _store_scores(C_out, score)
 
 
