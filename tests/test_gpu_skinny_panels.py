@@ -37,8 +37,21 @@ def test_linear_panels(T, K, cols):
     assert close(outs[0], product + add[0].double(), product)
 
 
+@pytest.mark.parametrize("T", [33, 48, 49, 63, 64, 65])
+@pytest.mark.parametrize("K,cols", [(8, (8,)), (264, (480, 8, 32)), (1000, (136, 1000, 24)), (96, (8200,))])
+def test_linear_panels_of_two_token_blocks(T, K, cols):
+    test_linear_panels(T, K, cols)
+
+
+# 64 MB of weights and more: read past the caches, up to 32 tokens and by the tilings of one tile of tokens
+@pytest.mark.parametrize("T,K,cols", [(16, 4104, (8200,)), (32, 4096, (4096, 4096, 40)), (64, 4096, (8200,)), (100, 4096, (8192, 64))])
+def test_large_weights(T, K, cols):
+    test_linear_panels(T, K, cols)
+
+
 @pytest.mark.parametrize("T,K,nq,nkv,D,gamma", [(1, 256, 256, 64, 64, True), (16, 1024, 1024, 1024, 64, False), (17, 512, 384, 128, 128, True),
-                                                (32, 1032, 1024, 256, 128, True), (24, 328, 64, 64, 64, False)])
+                                                (32, 1032, 1024, 256, 128, True), (24, 328, 64, 64, 64, False),
+                                                (50, 512, 512, 128, 128, True), (64, 1032, 1024, 1024, 64, False)])
 def test_normalised_projection_panels(T, K, nq, nkv, D, gamma):
     from triton_amd import ops
     g = torch.Generator().manual_seed(K + T)

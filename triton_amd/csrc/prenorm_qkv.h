@@ -24,11 +24,23 @@ struct GemmArgs {
 // chunks (one phase of the transposing read) touch every bank once.
 __device__ __forceinline__ int wswz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
+// Whether weights that one workgroup each reads once are requested past the caches (the non-temporal hint): 64 MB and more,
+// of which the last-level cache (256 MB) keeps nothing until the same layer comes round again but would evict what it holds
+// for each line.  us, without / with, weights and cache cold (three sets in turn): whole decode step, 16 tokens on 1024, 4096 ->
+// 12288 (101 MB) 35.3 / 32.9, 4544 -> 13632 31.7 / 28.8, one token 33.1 / 30.0; the projection of 100 tokens 36.4 / 35.0.  The other
+// side: one layer's step again and again, its weights then out of that cache, 27.2 / 32.3 and 26.7 / 28.1; and weights of 6 MB,
+// of which the caches hold many layers, 11.0 / 13.0.
+inline bool weights_stream(const GemmArgs& a) {
+    int64_t columns = 0;
+    for (int i = 0; i < 3; ++i) columns += a.p[i].n;
+    return columns * a.K * 2 >= (int64_t)64 << 20;
+}
+
 // 256 x 256 workgroup tiles, for problems large enough to fill the chip with them (prenorm_qkv_wide.hip).
 int launch_prenorm_qkv_wide(GemmArgs a, hipStream_t stream);
 int64_t prenorm_qkv_wide_tiles(const GemmArgs& a);
 
-// At most 32 tokens: 64-column panels streamed by eight waves that split the contraction (prenorm_qkv_skinny.hip).
+// At most 64 tokens: panels of 64 or 32 columns streamed by eight waves that split the contraction (prenorm_qkv_skinny.hip).
 int launch_prenorm_qkv_skinny(GemmArgs a, hipStream_t stream);
 
 // 64 x 64, 128 x 64 or 128 x 128 tiles (tokens x columns) whose waves split the contraction, for problems that leave the

@@ -219,6 +219,12 @@ __global__ __launch_bounds__(256, 2) void prenorm_qkv_kernel(const GemmArgs a) {
 int launch_projections(GemmArgs a, hipStream_t stream) {
     // a handful of tokens (decode): the weight stream is everything
     if (a.T <= 32) return launch_prenorm_qkv_skinny(a, stream);
+    // Up to 64 tokens on few weights too: there the tiling of prenorm_qkv_mid.hip is a chain of stages on a few CUs.  us, that / the
+    // stream, 33 and 64 tokens: 1024 deep, 576 columns and a second product of 64 deep 10.9 / 9.4, 10.9 / 9.4; 4096 deep, 1056 columns
+    // 16.1 / 14.5, 16.3 / 14.6; 1024 -> 3072 with an attention 12.4 / 11.6; but 4096 deep, 2048 columns (16 MB) 16.2 / 16.3, 17.9 / 18.4
+    int64_t columns = 0;
+    for (int i = 0; i < 3; ++i) columns += a.p[i].n;
+    if (a.T <= 64 && columns * a.K * 2 <= (int64_t)12 << 20) return launch_prenorm_qkv_skinny(a, stream);
     // 256-token tiles once they alone occupy at least half of the 256 CUs
     if (prenorm_qkv_wide_tiles(a) >= 128) return launch_prenorm_qkv_wide(a, stream);
     // Below that, the smallest tile that still gives every CU at most one: a tile's time is its chain of k-tiles, nearly

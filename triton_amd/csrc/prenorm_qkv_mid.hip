@@ -24,7 +24,7 @@
 
 namespace trn {
 
-template <int NTB, int TM, int TN, int NORM>      // NORM: 0 none, 1 without gamma, 2 with gamma
+template <int NTB, int TM, int TN, int NORM, bool STREAM>      // NORM: 0 none, 1 without gamma, 2 with gamma; STREAM: W past the caches
 __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
     static_assert(TM * TN == 2, "eight waves: two tiles x four contraction steps");
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_mid_kernel(const GemmArgs 
             g = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(grs, (kq * 16 + 8 * h) * 2, st * SK * 2, 0));
         else if (i < WI)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                wrs, (__attribute__((address_space(3))) void*)(D + MT * SK + (wave * WI + i) * 512), 16, w_vo[i], st * w_stage, 0, 0);
+                wrs, (__attribute__((address_space(3))) void*)(D + MT * SK + (wave * WI + i) * 512), 16, w_vo[i], st * w_stage, 0, STREAM ? 2 : 0);
         else              // columns past hidden hold the next row's data: read zeros instead
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
                 xrs, (__attribute__((address_space(3))) void*)(D + (XI * wave + i - WI) * 512), 16,
@@ -257,7 +257,7 @@ int64_t prenorm_qkv_mid_tiles(const GemmArgs& a, int mt, int nt) {
     return ((int64_t)a.T + mt - 1) / mt * panels;
 }
 
-template <int NTB, int TM, int TN>
+template <int NTB, int TM, int TN, bool STREAM>
 static int launch_mid(GemmArgs a, hipStream_t stream) {
     constexpr int MT = TM * NTB * 32, NT = TN * 64;
     a.n_mtiles = (a.T + MT - 1) / MT;
@@ -266,15 +266,16 @@ static int launch_mid(GemmArgs a, hipStream_t stream) {
     a.n_panels = t0;
     const int64_t grid = (int64_t)8 * ((t0 + 7) / 8) * a.n_mtiles;
     if (grid > 0x7fffffffLL) return TRN_E_SHAPE;
-    auto* kernel = !a.norm ? prenorm_qkv_mid_kernel<NTB, TM, TN, 0> : !a.gamma ? prenorm_qkv_mid_kernel<NTB, TM, TN, 1>
-                                                                               : prenorm_qkv_mid_kernel<NTB, TM, TN, 2>;
+    auto* kernel = !a.norm ? prenorm_qkv_mid_kernel<NTB, TM, TN, 0, STREAM> : !a.gamma ? prenorm_qkv_mid_kernel<NTB, TM, TN, 1, STREAM>
+                                                                                   : prenorm_qkv_mid_kernel<NTB, TM, TN, 2, STREAM>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), 0, stream, a);
     return hipGetLastError() == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
 }
 
 int launch_prenorm_qkv_mid(const GemmArgs& a, int mt, int nt, hipStream_t stream) {
-    if (nt == 128) return launch_mid<4, 1, 2>(a, stream);
-    return mt == 128 ? launch_mid<2, 2, 1>(a, stream) : launch_mid<1, 2, 1>(a, stream);
+    if (nt == 128) return launch_mid<4, 1, 2, false>(a, stream);
+    if (a.T <= mt && weights_stream(a)) return mt == 128 ? launch_mid<2, 2, 1, true>(a, stream) : launch_mid<1, 2, 1, true>(a, stream);
+    return mt == 128 ? launch_mid<2, 2, 1, false>(a, stream) : launch_mid<1, 2, 1, false>(a, stream);
 }
 
 }  // namespace trn

@@ -1,8 +1,8 @@
-// Fused RMSNorm + Q/K/V projection for a handful of tokens (decode: at most 32), where the GEMM is a stream of the
+// Fused RMSNorm + Q/K/V projection for a handful of tokens (decode: at most 32; 64 on few weights), where the GEMM is a stream of the
 // weight matrices through HBM and nothing else matters: 100 MB of W for 16 tokens at the Llama3-8B widths.
 //
-// Same arithmetic and MFMA mapping as the larger tilings (C^T = W^T X^T, 32x32x16 fp16 MFMAs, tokens padded to one
-// 32-wide block).  A workgroup owns a 64-column panel of one projection -- full 128-byte lines of every W row -- and
+// Same arithmetic and MFMA mapping as the larger tilings (C^T = W^T X^T, 32x32x16 fp16 MFMAs, tokens padded to
+// 32-wide blocks).  A workgroup owns a 64-column panel of one projection -- full 128-byte lines of every W row -- and
 // its eight waves take the contraction in turns of SK rows: wave w's k-tiles are w, w + 8, ...  Nothing in the loop is
 // shared between waves, so it has no barrier: a wave loads a k-tile of W and X into registers while it multiplies the
 // one before, writes it to its private part of LDS when it arrives, and reads it back as MFMA operands (LDS operations
@@ -20,19 +20,20 @@
 namespace trn {
 
 // XL: wave-wide loads that cover the tokens of a k-tile (rows of SK columns); NORM: 0 none, 1 without gamma, 2 with gamma
-// SN: columns of a panel
-template <int SK, int XL, int NORM, int SN>
+// SN: columns of a panel; NT: W is requested past the caches
+template <int SK, int XL, int NORM, int SN, bool NT>
 __global__ __launch_bounds__(512, 2) void prenorm_qkv_skinny_kernel(const GemmArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors exist in the device pass only
     constexpr int NW = 8, NB = SN / 32, WC = SN / 8, WR = 64 / WC, WL = SK / WR;      // waves, column blocks; W: chunks per row, rows per load, loads
     constexpr int XC = SK / 8, XR = 64 / XC;                                           // X: chunks per row, rows per load
-    static_assert((SK == 32 || SK == 64) && (SN == 32 || SN == 64) && XL * XR <= 32, "k-tiles of 32 or 64 rows, at most 32 tokens");
+    constexpr int TB = (XL * XR + 31) / 32;                                            // blocks of 32 tokens
+    static_assert((SK == 32 || SK == 64) && (SN == 32 || SN == 64) && TB <= 2, "k-tiles of 32 or 64 rows, at most 64 tokens");
     // [NW] W k-tiles, then [NW] X k-tiles (reads of token rows past the loaded ones stay inside: their results are never
     // stored); at the end the partial accumulators, 8 KB per wave
-    constexpr int WSZ = NW * SK * SN, XSZ = NW * XL * XR * SK + (32 - XL * XR) * SK, RSZ = NW * 16 * NB * 64 * 2;
+    constexpr int WSZ = NW * SK * SN, XSZ = NW * XL * XR * SK + (32 * TB - XL * XR) * SK, RSZ = NW * 16 * NB * 64 * 2;
     __shared__ __attribute__((aligned(1024))) half_t smem[WSZ + XSZ > RSZ ? WSZ + XSZ : RSZ];
     __shared__ __attribute__((aligned(256))) half_t Gs[NORM == 2 ? NW * SK : 8];
-    __shared__ float ss_part[NW][32];
+    __shared__ float ss_part[NW][32 * TB];
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -62,7 +63,7 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_skinny_kernel(const GemmAr
     half8_t wreg[WL], xreg[XL], greg;
     auto fetch = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < WL; ++i) wreg[i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(wrs, w_vo, (s * WL + i) * w_step, 0));
+        for (int i = 0; i < WL; ++i) wreg[i] = __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(wrs, w_vo, (s * WL + i) * w_step, NT ? 2 : 0));
         // columns past hidden hold the next row's data: read zeros instead
         const bool drop = s * SK + 8 * xc >= a.K;
 #pragma unroll
@@ -97,12 +98,16 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_skinny_kernel(const GemmAr
         for (int ks = 0; ks < SK / 16; ++ks) xoff[ks] = c * SK + (((2 * ks + h) ^ xsw(c)) << 3);
     }
 
-    float16_t acc[NB];
+    float16_t acc[TB][NB];
+    float ss[TB];
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
+    for (int tb = 0; tb < TB; ++tb) {
+        ss[tb] = 0.f;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[nb][r] = 0.f;
-    float ss = 0.f;
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[tb][nb][r] = 0.f;
+    }
 
     if (wave < nkt) fetch(wave);
     for (int kt = wave; kt < nkt; kt += NW) {
@@ -124,63 +129,73 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_skinny_kernel(const GemmAr
                 const half4_t hi = lds_read_tr16(&Wm[ks * 16 * SN + woff_hi[nb]]);
                 wa[nb] = half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
             }
-            half8_t xv = *reinterpret_cast<const half8_t*>(&Xm[xoff[ks]]);
-            if constexpr (NORM > 0) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const half2_t p = {xv[2 * e], xv[2 * e + 1]};
-                    ss = __builtin_amdgcn_fdot2(p, p, ss, false);
+            for (int tb = 0; tb < TB; ++tb) {
+                half8_t xv = *reinterpret_cast<const half8_t*>(&Xm[tb * 32 * SK + xoff[ks]]);
+                if constexpr (NORM > 0) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const half2_t p = {xv[2 * e], xv[2 * e + 1]};
+                        ss[tb] = __builtin_amdgcn_fdot2(p, p, ss[tb], false);
+                    }
+                    if constexpr (NORM == 2) xv = xv * *reinterpret_cast<const half8_t*>(&Gm[ks * 16 + 8 * h]);
                 }
-                if constexpr (NORM == 2) xv = xv * *reinterpret_cast<const half8_t*>(&Gm[ks * 16 + 8 * h]);
-            }
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc[nb] = mfma32(wa[nb], xv, acc[nb]);
+                for (int nb = 0; nb < NB; ++nb) acc[tb][nb] = mfma32(wa[nb], xv, acc[tb][nb]);
+            }
         }
     }
 
     // ---- add the eight waves' partial results through LDS
-    __syncthreads();
-    float* red = reinterpret_cast<float*>(smem);             // [NW][16 NB registers][64 lanes]
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) red[((wave * NB + nb) * 16 + r) * 64 + lane] = acc[nb][r];
+    float* red = reinterpret_cast<float*>(smem);             // [NW][16 NB registers][64 lanes], a block of 32 tokens at a time
     if constexpr (NORM > 0) {
-        const float s = half_sum(ss);                        // both halves of a token's columns
-        if (h == 0) ss_part[wave][c] = s;
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            const float s = half_sum(ss[tb]);                // both halves of a token's columns
+            if (h == 0) ss_part[wave][32 * tb + c] = s;
+        }
     }
-    __syncthreads();
     // wave w finishes accumulator registers FIN w .. FIN w + FIN-1: of column block w / (8 / NB), rows 8*(r/4) + 4h + r%4, token c
     constexpr int FIN = 2 * NB;
     typedef _Float16 fin_t __attribute__((ext_vector_type(FIN)));
-    float rstd = 1.0f;
-    if constexpr (NORM > 0) {
-        float sq = 0.f;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) sq += ss_part[w][c];
-        rstd = 1.0f / __builtin_sqrtf(sq / (float)a.K + a.eps);
-    }
     const int r0 = FIN * wave % 16, n = n0 + FIN * wave / 16 * 32 + 8 * (r0 / 4) + 4 * h + r0 % 4;
-    if (c < a.T && n < P.n) {
-        const int64_t o_off = (int64_t)(n / a.head_dim) * P.stride_h + (int64_t)c * P.stride_s + (n % a.head_dim);
-        fin_t ad = {};
-        if (P.addend) ad = *reinterpret_cast<const fin_t*>(P.addend + o_off);
-        fin_t ov;
 #pragma unroll
-        for (int e = 0; e < FIN; ++e) {
-            float v = 0.f;
+    for (int tb = 0; tb < TB; ++tb) {
+        __syncthreads();
 #pragma unroll
-            for (int w = 0; w < NW; ++w) v += red[(w * 16 * NB + FIN * wave + e) * 64 + lane];
-            ov[e] = (half_t)((float)(half_t)(v * rstd) + (float)ad[e]);     // the product rounded to fp16 first, as a separate GEMM would leave it
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) red[((wave * NB + nb) * 16 + r) * 64 + lane] = acc[tb][nb][r];
+        __syncthreads();
+        const int t = 32 * tb + c;
+        float rstd = 1.0f;
+        if constexpr (NORM > 0) {
+            float sq = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) sq += ss_part[w][t];
+            rstd = 1.0f / __builtin_sqrtf(sq / (float)a.K + a.eps);
         }
-        *reinterpret_cast<fin_t*>(P.out + o_off) = ov;
+        if (t < a.T && n < P.n) {
+            const int64_t o_off = (int64_t)(n / a.head_dim) * P.stride_h + (int64_t)t * P.stride_s + (n % a.head_dim);
+            fin_t ad = {};
+            if (P.addend) ad = *reinterpret_cast<const fin_t*>(P.addend + o_off);
+            fin_t ov;
+#pragma unroll
+            for (int e = 0; e < FIN; ++e) {
+                float v = 0.f;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) v += red[(w * 16 * NB + FIN * wave + e) * 64 + lane];
+                ov[e] = (half_t)((float)(half_t)(v * rstd) + (float)ad[e]);     // the product rounded to fp16 first, as a separate GEMM would leave it
+            }
+            *reinterpret_cast<fin_t*>(P.out + o_off) = ov;
+        }
     }
 #endif
 }
 
 // k-tiles of 32 rows up to 16 tokens (a shorter chain where hidden is small), of 64 beyond: 32 tokens x 64 bytes are half
 // lines of X, and fetching those costs more than the shorter chain gains (4096 -> 12288, 32 tokens: 27.3 against 25.5 us).
-template <int SN>
+template <int SN, bool NT>
 static int launch_panels(GemmArgs a, hipStream_t stream) {
     int t0 = 0;
     for (int i = 0; i < 3; ++i) { a.p[i].tile0 = t0; t0 += (a.p[i].n + SN - 1) / SN; }
@@ -189,13 +204,14 @@ static int launch_panels(GemmArgs a, hipStream_t stream) {
     const int norm = !a.norm ? 0 : a.gamma ? 2 : 1;
 #define TRN_SKINNY(SK_, XL_)                                                                                              \
     do {                                                                                                                  \
-        if (norm == 0) hipLaunchKernelGGL((prenorm_qkv_skinny_kernel<SK_, XL_, 0, SN>), g, t, 0, stream, a);              \
-        else if (norm == 1) hipLaunchKernelGGL((prenorm_qkv_skinny_kernel<SK_, XL_, 1, SN>), g, t, 0, stream, a);         \
-        else hipLaunchKernelGGL((prenorm_qkv_skinny_kernel<SK_, XL_, 2, SN>), g, t, 0, stream, a);                        \
+        if (norm == 0) hipLaunchKernelGGL((prenorm_qkv_skinny_kernel<SK_, XL_, 0, SN, NT>), g, t, 0, stream, a);              \
+        else if (norm == 1) hipLaunchKernelGGL((prenorm_qkv_skinny_kernel<SK_, XL_, 1, SN, NT>), g, t, 0, stream, a);         \
+        else hipLaunchKernelGGL((prenorm_qkv_skinny_kernel<SK_, XL_, 2, SN, NT>), g, t, 0, stream, a);                        \
     } while (0)
     if (a.T <= 16) TRN_SKINNY(32, 1);
     else if (a.T <= 24) TRN_SKINNY(64, 3);
-    else TRN_SKINNY(64, 4);
+    else if (SN == 64 || a.T <= 32) TRN_SKINNY(64, 4);
+    else TRN_SKINNY(32, 4);
 #undef TRN_SKINNY
     return hipGetLastError() == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
 }
@@ -209,7 +225,8 @@ static int launch_panels(GemmArgs a, hipStream_t stream) {
 int launch_prenorm_qkv_skinny(GemmArgs a, hipStream_t stream) {
     int panels = 0;
     for (int i = 0; i < 3; ++i) panels += (a.p[i].n + 63) / 64;
-    return panels <= 128 ? launch_panels<32>(a, stream) : launch_panels<64>(a, stream);
+    if (a.T > 32) return launch_panels<32, false>(a, stream);
+    return panels <= 128 ? launch_panels<32, false>(a, stream) : weights_stream(a) ? launch_panels<64, true>(a, stream) : launch_panels<64, false>(a, stream);
 }
 
 }  // namespace trn
