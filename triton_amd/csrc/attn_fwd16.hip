@@ -78,22 +78,28 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     constexpr int RPI = 64 / CPR;            // stage rows covered by one wave-wide 1 KB load
     constexpr int NI = BN / (RPI * GW);      // such loads per wave per stage (K and V each)
     constexpr int NG = SPLIT ? 2 : 1;        // groups with stages of their own
-    __shared__ __attribute__((aligned(1024))) half_t Ks0_[NG * BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Ks1_[NG * BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Vs0_[NG * BN * D];
-    __shared__ __attribute__((aligned(1024))) half_t Vs1_[NG * BN * D];
+    constexpr int SR = SHARE ? 32 : BN;      // keys per stage of the ring: two stages of a tile, or four of a block (see share_tile)
+    __shared__ __attribute__((aligned(1024))) half_t Ks0_[NG * SR * D];
+    __shared__ __attribute__((aligned(1024))) half_t Ks1_[NG * SR * D];
+    __shared__ __attribute__((aligned(1024))) half_t Vs0_[NG * SR * D];
+    __shared__ __attribute__((aligned(1024))) half_t Vs1_[NG * SR * D];
+    __shared__ __attribute__((aligned(1024))) half_t Ks2_[SHARE ? NG * SR * D : 1];
+    __shared__ __attribute__((aligned(1024))) half_t Ks3_[SHARE ? NG * SR * D : 1];
+    __shared__ __attribute__((aligned(1024))) half_t Vs2_[SHARE ? NG * SR * D : 1];
+    __shared__ __attribute__((aligned(1024))) half_t Vs3_[SHARE ? NG * SR * D : 1];
 
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g4 = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = SPLIT ? wave >> 2 : 0, gw = SPLIT ? wave & 3 : wave;
-    half_t* const Ks0 = Ks0_ + grp * BN * D;
-    half_t* const Ks1 = Ks1_ + grp * BN * D;
-    half_t* const Vs0 = Vs0_ + grp * BN * D;
-    half_t* const Vs1 = Vs1_ + grp * BN * D;
+    half_t* const Ks0 = Ks0_ + grp * SR * D;
+    half_t* const Ks1 = Ks1_ + grp * SR * D;
+    half_t* const Vs0 = Vs0_ + grp * SR * D;
+    half_t* const Vs1 = Vs1_ + grp * SR * D;
     const int BH = a.B * a.Hq;
-    // The shares of a query tile are consecutive; a share is a whole number of tiles of both groups.
+    // The shares of a query tile are consecutive; a share is a whole number of tiles, which the groups take in turns (not of pairs of
+    // tiles: 4100 keys in eight shares would be seven of 640, and are eight of at most 576).
     const int share = SHARE ? (int)(blockIdx.x / BH) % a.n_split : 0, tile_no = (int)(blockIdx.x / BH) / (SHARE ? a.n_split : 1);
-    const int share_tiles = SHARE ? 2 * (((a.Skv + 2 * BN - 1) / (2 * BN) + a.n_split - 1) / a.n_split) : 0;
+    const int share_tiles = SHARE ? ((a.Skv + BN - 1) / BN + a.n_split - 1) / a.n_split : 0;
     const int kfirst = grp * BN + share * share_tiles * BN;      // first key of this wave's first tile
 
     const int j = blockIdx.x % BH;
@@ -238,6 +244,8 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         if constexpr (SPLIT) any_fresh = __builtin_amdgcn_ballot_w64(fresh[0] || fresh[1]) != 0;
     };
 
+    bool more = true;       // shares: the block whose scores a step leaves is one of the wave's own (the stage of the block past its
+                            // last is not its keys: scores from it must not move the reference)
     const half_t one = (half_t)1.f;
     const half8_t ones8 = {one, one, one, one, one, one, one, one};
     constexpr int NQ = 2;   // operand look-ahead, in operands (= 2 NQ MFMA slots; 4 measured no better, twice)
@@ -320,13 +328,29 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         }
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) lacc[qb] = mfma16(ones8, pB[qb], lacc[qb]);
-        if (due) rescale(sn);
+        if (SHARE ? due && more : due) rescale(sn);
+    };
+
+    // Shares: 32-key block B of this group's keys (two per tile) to its stage; past the share's last block nothing is read.
+    const int n_blocks = 2 * ((ntiles - grp + 1) >> 1);
+    auto request_k = [&](int blk, half_t* dst) __attribute__((always_inline)) {
+        fetch_tile<(NI + 1) / 2, D, GW>(krs, dst + grp * SR * D + gw * RPI * D, blk < n_blocks ? kvo : 0x7ffffff0,
+                                        kgrp_bytes + (blk >> 1) * ktile_bytes + (blk & 1) * (ktile_bytes / 4), krow_bytes);
+    };
+    auto request_v = [&](int blk, half_t* dst) __attribute__((always_inline)) {
+        fetch_tile<(NI + 1) / 2, D, GW>(vrs, dst + grp * SR * D + gw * RPI * D, blk < n_blocks ? vvo : 0x7ffffff0,
+                                        vgrp_bytes + (blk >> 1) * vtile_bytes + (blk & 1) * (vtile_bytes / 4), vrow_bytes);
     };
 
     // ---- prologue: K stages 0 and 1 and V stage 0; scores of block 0; first K operands of block 1 ----
-    TRN_FETCH_K(0, Ks0);
-    TRN_FETCH_V(0, Vs0);
-    if (SPLIT || ntiles > 1) TRN_FETCH_K(1, Ks1);
+    if constexpr (SHARE) {
+        request_k(0, Ks0_); request_k(1, Ks1_);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        TRN_FETCH_K(0, Ks0);
+        TRN_FETCH_V(0, Vs0);
+        if (SPLIT || ntiles > 1) TRN_FETCH_K(1, Ks1);
+    }
 
     // ---- Q^T B-operands: lane holds Q[qrow[qb]][32 ks + 8 g4 .. +7].  The loads go out behind the first K/V stage
     // fetches and all together, so that the workgroup's start-up pays one memory latency, not three in a row.
@@ -344,6 +368,11 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     if (use_gq) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) gq[ks] = *reinterpret_cast<const half8_t*>(a.gamma_q + ks * 32 + 8 * g4);
+    }
+    if constexpr (SHARE) {      // (the rest of the ring behind Q, whose wait would otherwise be for all of it)
+        __builtin_amdgcn_sched_barrier(0);
+        request_v(0, Vs0_); request_k(2, Ks2_); request_v(1, Vs1_); request_k(3, Ks3_); request_v(2, Vs2_);
+        __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
@@ -372,8 +401,15 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
             for (int e = 0; e < 8; ++e) qB[qb][ks][e] = (half_t)((float)qB[qb][ks][e] * a.c1);
     }
 
-    __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0): this wave's loads have landed in LDS
-    __syncthreads();
+    if constexpr (SHARE) {
+        constexpr int kBehind = 5 * NI / 2;             // K blocks 0 and 1 have landed
+        __builtin_amdgcn_s_waitcnt(0x0070 | (kBehind & 15) | ((kBehind >> 4) << 14));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0): this wave's loads have landed in LDS
+        __syncthreads();
+    }
 
     Scores16 sA, sB;                        // scores of the current / next 32-key block (ping-pong)
     {
@@ -386,7 +422,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
                 for (int qb = 0; qb < 2; ++qb) sA.s[kb][qb] = mfma16(k0, qB[qb][ks], ks == 0 ? zero : sA.s[kb][qb]);
             }
 #pragma unroll
-        for (int i = 0; i < NQ; ++i) load_k(Ks0 + 32 * D, i, i);
+        for (int i = 0; i < NQ; ++i) load_k(SHARE ? Ks1 : Ks0 + 32 * D, i, i);
         // block 0 sets the reference outright (every query sees key 0, so it is finite from here on)
         float smax[2];
         mask_block(sA, kfirst);
@@ -415,20 +451,41 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         auto handover = [&]() __attribute__((always_inline)) {
             __builtin_amdgcn_s_waitcnt(0x0f70);   // this wave's share of stages Kn and Vc is in LDS
             __syncthreads();                      // ... and everyone's; Kc and Vn have had their last readers
-            // (the shares of a long cache wait for HBM, not for issue: all at once, which tells where many heads of 64 share a
-            // long one.  Whole steps, us, dealt out / at once: 71 heads of 64, 100 on 16000 104.7 / 101.7, 100 on 4000 49.8 / 49.0,
-            // 64 on 6000 50.3 / 50.3; 32 of 128, 100 on 4000 48.7 / 49.1, 128 on 16000 102.5 / 103.1, 64 on 8000 49.7 / 49.9; 16 of
-            // 64, 100 on 8000 22.0 / 22.6, 128 on 16000 27.8 / 27.8; 8 of 128, 100 on 8000 25.9 / 26.2)
-            if constexpr (SHARE) {
-#pragma unroll
-                for (int i = 0; i < 2 * NI; ++i) refill(i);
-            }
         };
         auto none = [&]() __attribute__((always_inline)) {};
         auto none1 = [&](int) __attribute__((always_inline)) {};
         // (Past the last tile a K stage holds stale rows; scores computed from them are masked away.)
-        step(needs_mask(kv0 + 32), maymask_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover, [&](int i) __attribute__((always_inline)) { if constexpr (!SHARE) refill(i); });
+        step(needs_mask(kv0 + 32), maymask_tag, std::true_type{}, sA, sB, Vc, Kc + 32 * D, Kn, kv0 + 32, handover, refill);
         step(needs_mask(kv0 + KSTEP), maymask_tag, std::false_type{}, sB, sA, Vc + 32 * D, Kn, Kn + 32 * D, kv0 + KSTEP, none, none1);
+    };
+    // Tile jt of a share: K0 .. K3 and V0 .. V3 are the ring's stages from the tile's first block on.  What bounds it is how much is
+    // under way from HBM: with the two stages of 64 keys above all of it had to land before the next was asked for, a tile of
+    // 64 KB every 3 - 4 us.  Here block B's hand-over asks for V of block B + 3 and K of block B + 5, into the stages that block
+    // B - 1 and block B + 1 have just vacated, and waits for what the one three blocks ago asked for.
+    // us, two stages and shares of whole pairs of tiles / ring and shares of single tiles, without the merge: 32 heads of 128: 100
+    // queries on 4.1 k keys 25.2 / 19.4, 128 on 3.2 k 22.7 / 18.3, 40 on 3.1 k 17.5 / 14.8, 128 on 8.1 k 38.5 / 33.5, 50 on 16 k
+    // 52.2 / 50.4; 8 of 128: 100 on 8.1 k 16.6 / 16.4, 128 on 16 k 23.7 / 23.1; 71 of 64: 40 on 6 k 26.7 / 24.2, 64 on 6 k 27.4 / 24.7,
+    // 128 on 3.1 k 20.0 / 17.0, 100 on 2.7 k 17.8 / 15.7; 16 of 64, three tiles a group at most: 60 on 4.3 k 9.8 / 9.9, 5.1 k 9.5 /
+    // 10.1; 12 k 13.7 / 13.7.  (Of those, writing the partial results past the caches: 128 on 8.1 k 37.4 / 33.2, 100 on 4.1 k 20.4 / 19.3.)
+    auto share_handover = [&](int blk, half_t* Kf, half_t* Vf) __attribute__((always_inline)) {
+        constexpr int kBehind = 2 * NI;      // V of blk and K of blk + 2 have landed: behind them only two hand-overs' requests
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0x0070 | (kBehind & 15) | ((kBehind >> 4) << 14));      // lgkmcnt(0): the vacated stages have been read
+        __builtin_amdgcn_s_barrier();        // (a bare barrier: the loads in flight must stay in flight)
+        __builtin_amdgcn_sched_barrier(0);
+        request_v(blk + 3, Vf);
+        request_k(blk + 5, Kf);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto share_tile = [&](auto maymask_tag, int jt, int nlive, half_t* K0, half_t* K1, half_t* K2, half_t* K3, half_t* V0, half_t* V1,
+                          half_t* V3) __attribute__((always_inline)) {
+        const int kv0 = kfirst + jt * KSTEP, g0 = grp * SR * D;
+        auto none1 = [&](int) __attribute__((always_inline)) {};
+        step(needs_mask(kv0 + 32), maymask_tag, std::true_type{}, sA, sB, V0 + g0, K1 + g0, K2 + g0, kv0 + 32,
+             [&]() __attribute__((always_inline)) { share_handover(2 * jt, K1, V3); }, none1);
+        more = jt + 1 < nlive;
+        step(needs_mask(kv0 + KSTEP), maymask_tag, std::true_type{}, sB, sA, V1 + g0, K2 + g0, K3 + g0, kv0 + KSTEP,
+             [&]() __attribute__((always_inline)) { share_handover(2 * jt + 1, K2, V0); }, none1);
     };
     // Under a causal mask the waves of a workgroup see different numbers of tiles: a wave computes the tiles that
     // hold a key visible to one of its queries, and for the rest only keeps up the staging it shares with the
@@ -445,21 +502,42 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     int n_plain = max(0, a.Skv - 32 - kfirst) / KSTEP;
     if (a.causal) n_plain = min(n_plain, max(0, wb - 31 - kfirst) / KSTEP);
     n_plain = min(n_plain, nlive) & ~1;
-    for (int jt = 0; jt < n_plain; jt += 2) {
-        tile(std::false_type{}, jt, Ks0, Ks1, Vs0, Vs1);
-        tile(std::false_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
-    }
-    for (int jt = n_plain; jt < nlive; jt += 2) {
-        tile(std::true_type{}, jt, Ks0, Ks1, Vs0, Vs1);
-        if (jt + 1 < nlive) tile(std::true_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
-    }
-    for (int jt = nlive; jt < nloop; ++jt) {
-        half_t* Kc = (jt & 1) ? Ks1 : Ks0;
-        half_t* Vn = (jt & 1) ? Vs0 : Vs1;
-        __builtin_amdgcn_s_waitcnt(0x0f70);
-        __syncthreads();
-        if (jt + 2 < nloop) TRN_FETCH_K(jt + 2, Kc);
-        if (jt + 1 < nloop) TRN_FETCH_V(jt + 1, Vn);
+    if constexpr (SHARE) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xc07f);     // lgkmcnt(0): K block 0 has been read ...
+        __builtin_amdgcn_s_barrier();           // ... by everyone
+        __builtin_amdgcn_sched_barrier(0);
+        request_k(4, Ks0_);
+        __builtin_amdgcn_sched_barrier(0);
+        for (int jt = 0; jt < n_plain; jt += 2) {
+            share_tile(std::false_type{}, jt, nlive, Ks0_, Ks1_, Ks2_, Ks3_, Vs0_, Vs1_, Vs3_);
+            share_tile(std::false_type{}, jt + 1, nlive, Ks2_, Ks3_, Ks0_, Ks1_, Vs2_, Vs3_, Vs1_);
+        }
+        for (int jt = n_plain; jt < nlive; jt += 2) {
+            share_tile(std::true_type{}, jt, nlive, Ks0_, Ks1_, Ks2_, Ks3_, Vs0_, Vs1_, Vs3_);
+            if (jt + 1 < nlive) share_tile(std::true_type{}, jt + 1, nlive, Ks2_, Ks3_, Ks0_, Ks1_, Vs2_, Vs3_, Vs1_);
+        }
+        for (int jt = nlive; jt < nloop; ++jt) {
+            share_handover(2 * jt, (jt & 1) ? Ks3_ : Ks1_, (jt & 1) ? Vs1_ : Vs3_);
+            share_handover(2 * jt + 1, (jt & 1) ? Ks0_ : Ks2_, (jt & 1) ? Vs2_ : Vs0_);
+        }
+    } else {
+        for (int jt = 0; jt < n_plain; jt += 2) {
+            tile(std::false_type{}, jt, Ks0, Ks1, Vs0, Vs1);
+            tile(std::false_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
+        }
+        for (int jt = n_plain; jt < nlive; jt += 2) {
+            tile(std::true_type{}, jt, Ks0, Ks1, Vs0, Vs1);
+            if (jt + 1 < nlive) tile(std::true_type{}, jt + 1, Ks1, Ks0, Vs1, Vs0);
+        }
+        for (int jt = nlive; jt < nloop; ++jt) {
+            half_t* Kc = (jt & 1) ? Ks1 : Ks0;
+            half_t* Vn = (jt & 1) ? Vs0 : Vs1;
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+            __syncthreads();
+            if (jt + 2 < nloop) TRN_FETCH_K(jt + 2, Kc);
+            if (jt + 1 < nloop) TRN_FETCH_V(jt + 1, Vn);
+        }
     }
 #undef TRN_FETCH_K
 #undef TRN_FETCH_V
@@ -477,7 +555,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         // lane by lane: group 0 finishes the first D/2 columns, group 1 the others.  A wave that took no tile, or a
         // query that saw no key of its group, has zero sums and weighs nothing.
         constexpr int kStat = D == 128 ? 5120 : 2560;   // (floats) the row statistics lie behind the transposing regions
-        float* stat = reinterpret_cast<float*>(Ks1_) + kStat;       // [8 waves][2 query blocks][16 queries] {m, l}
+        float* stat = SHARE ? reinterpret_cast<float*>(Ks2_) : reinterpret_cast<float*>(Ks1_) + kStat;   // [8 waves][2 query blocks][16 queries] {m, l}
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
             if (nlive == 0 || fresh[qb]) m[qb] = -INFINITY;
@@ -489,6 +567,11 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         constexpr int NH = NOP / 2;
         float4_t* mine = reinterpret_cast<float4_t*>(wave < 4 ? Ks0_ : Vs0_) + (wave & 3) * NH * 2 * 64;
         const float4_t* theirs = reinterpret_cast<const float4_t*>(wave < 4 ? Vs0_ : Ks0_) + (wave & 3) * NH * 2 * 64;
+        if constexpr (SHARE) {          // (a stage of the ring holds two waves' halves)
+            half_t *const ka_ = wave & 2 ? Ks1_ : Ks0_, *const va_ = wave & 2 ? Vs1_ : Vs0_;
+            mine = reinterpret_cast<float4_t*>(wave < 4 ? ka_ : va_) + (wave & 1) * NH * 2 * 64;
+            theirs = reinterpret_cast<const float4_t*>(wave < 4 ? va_ : ka_) + (wave & 1) * NH * 2 * 64;
+        }
 #pragma unroll
         for (int i = 0; i < NH; ++i)
 #pragma unroll
@@ -520,7 +603,8 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
                 if (qrow[qb] >= a.Sq) continue;
                 float* po = a.ws + (row0 + qrow[qb]) * D + grp * (D / 2) + 4 * g4;
 #pragma unroll
-                for (int i = 0; i < NH; ++i) *reinterpret_cast<float4_t*>(po + 16 * i) = oacc[i][qb];
+                for (int i = 0; i < NH; ++i)       // (16 MB in all that this launch does not read: past the caches)
+                    __builtin_nontemporal_store(oacc[i][qb], reinterpret_cast<float4_t*>(po + 16 * i));
                 if (g4 == 0 && grp == 0) *reinterpret_cast<float2_t*>(a.ws + rows * D + (row0 + qrow[qb]) * 2) = float2_t{l[qb] > 0.f ? m[qb] : -INFINITY, l[qb]};
             }
             return;
@@ -657,13 +741,13 @@ __global__ __launch_bounds__(256) void attn_merge_shares_kernel(const AttnArgs a
 
 // Key shares of the query tiles of 128, one workgroup per CU in all (0: the keys are not shared out).  The other forms are
 // tiles of 32 queries with all the keys each (attn_decode.hip: every tile reads K and V again, twice or more with its column
-// shares) and workgroups of 128 queries (a CU per tile).  Shares read the cache once, at some 10 us + 6 TB/s, and pay about
+// shares) and workgroups of 128 queries (a CU per tile).  Shares read the cache once, at some 8 us + 6 TB/s, and pay about
 // 5 us for the merge: not on short caches.  us without / with shares (both launches): 32 heads of 128: 100 queries on 2.6 k
-// keys 22.1 / 22.1, 128 on 3.1 k 25.6 / 26.1, 40 on 3 k 23.4 / 21.0, 100 on 4.1 k 32.1 / 28.7, 128 on 8.1 k 56.8 / 43.3, 50
-// on 16 k 98 / 57, 300 on 4.3 k 61.5 / 45.4; 8 heads of 128: 100 on 2.6 k 16.2 / 17.7, 40 on 3 k 17.6 / 15.1, 500 on 3.5 k
-// 25.6 / 23.0, 128 on 16 k 73 / 28; 16 heads of 64: 100 on 3.1 k 13.9 / 14.0, 40 on 4 k 15.4 / 12.5, 128 on 9.1 k 30 / 18; 71
-// heads of 64: 64 on 4.1 k 25.1 / 25.8, 40 on 6 k 33.8 / 31.4, and, with more than 256 tiles of 32 queries, 100 on 2.6 k 29.0
-// / 21.5, 128 on 16 k 137 / 70.
+// keys 20.7 / 20.8, 128 on 2.8 k 21.1 / 22.7, 128 on 3.1 k 25.6 / 23.9, 40 on 2.7 k 19.3 / 18.1, 3 k 23.4 / 19.5, 100 on 4.1 k
+// 32.1 / 24.1, 128 on 8.1 k 56.8 / 41, 50 on 16 k 98 / 55, 300 on 4.3 k 61.5 / 48; 8 heads of 128: 100 on 2.6 k 16.2 / 16.0, 40
+// on 3 k 17.6 / 15.5, 500 on 3.5 k 25.6 / 23.0, 128 on 16 k 73 / 28; 16 heads of 64: 100 on 2.1 k 10.5 / 13.5, 3.1 k 13.9 / 13.4,
+// 40 on 4 k 15.4 / 13.6, 128 on 9.1 k 30 / 18; 71 heads of 64: 64 on 3.1 k 16.2 / 20.2, 4.1 k 25.1 / 23.0, 40 on 6 k 33.8 / 29.3,
+// and, with more than 256 tiles of 32 queries, 100 on 1.3 k 16.7 / 16.4, 1.6 k 18.8 / 16.9, 2.6 k 29.0 / 19.9, 128 on 16 k 137 / 65.
 static int key_shares(int64_t bh, int seq_q, int seq_kv, int head_dim) {
     const int64_t tiles = ((int64_t)seq_q + 127) / 128 * bh, tiles32 = ((int64_t)seq_q + 31) / 32 * bh;
     if (seq_q <= 32 || tiles > 128 || seq_kv < (head_dim == 128 ? 3072 : tiles32 > 256 ? 2560 : 4096)) return 0;
