@@ -29,6 +29,14 @@ struct AttnArgs {
     int s16;       // decode and short kernels: col_sum and col_sumsq point at fp16 data
 };
 
+// 16 bytes of the output, past the caches: what a launch leaves dirty in the L2s is written back before it ends, and the next
+// layer's rows come from the last-level cache no faster than from HBM.  Attention launches, us, through the caches / past them: 8 x 500
+// tokens, 32 heads of 128 34.0 / 29.0, 4 x 777 35.4 / 33.9, 1100 21.4 / 20.7, 4096 138.2 / 136.3; 8 x 300, 16 heads of 64 8.5 / 8.3;
+// 71 of 64, 1000 tokens 18.7 / 17.7, 400 8.65 / 8.52; with key scores, whole calls: 4096 tokens 448 / 441, 71 of 64, 1500 129 / 126;
+// outputs of 1 MB and less the same.  (Not for the projections, whose outputs the next launch reads: a block of 2000 tokens, 16 heads of
+// 64 46.5 / 50.5.)
+__device__ __forceinline__ void store_out(half_t* p, uint4_t v) { __builtin_nontemporal_store(v, reinterpret_cast<uint4_t*>(p)); }
+
 // fp16 noise as the kernels fetch it.  Its rows may start at any element (the reference's [.., M, P + M] tensors have any
 // key count), so a lane reads the whole dwords around its 4 keys -- three of them cover both cases -- and shifts by half a
 // dword where its row starts on an odd element.  Nothing outside the dword that holds a row's last key is ever read: the

@@ -509,7 +509,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
             const uint2_t lo = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol]);
             const uint2_t hi = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol + 4]);
             if (wq0 + r < a.Sq)
-                *reinterpret_cast<uint4_t*>(ob + (int64_t)(wq0 + r) * a.os + ocol) = uint4_t{lo.x, lo.y, hi.x, hi.y};
+                store_out(ob + (int64_t)(wq0 + r) * a.os + ocol, uint4_t{lo.x, lo.y, hi.x, hi.y});
         }
         if (grp == 1) return;               // (the normalisers are written once)
     } else {
@@ -540,7 +540,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 const uint2_t lo = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol]);
                 const uint2_t hi = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol + 4]);
                 if (wq0 + r < a.Sq)
-                    *reinterpret_cast<uint4_t*>(ob + (int64_t)(wq0 + r) * a.os + pass * DP + ocol) = uint4_t{lo.x, lo.y, hi.x, hi.y};
+                    store_out(ob + (int64_t)(wq0 + r) * a.os + pass * DP + ocol, uint4_t{lo.x, lo.y, hi.x, hi.y});
             }
         }
     }
