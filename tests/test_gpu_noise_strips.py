@@ -94,6 +94,34 @@ def test_references_that_rise_and_rows_without_noise(S, D, Hq):
     check(q, k, n, rows, c, 1.0, 4e-4, [(0, h) for h in range(5)], 1000.0)
 
 
+@pytest.mark.parametrize("S,D,Hq,half", [(1100, 128, 32, False), (620, 64, 71, False), (2200, 64, 8, False), (1030, 64, 71, True)])
+def test_rows_without_a_normaliser(S, D, Hq, half):
+    """A row without a finite score, or with +inf or NaN among them, has no probabilities: the scores of the keys that it sees are
+    NaN, and only these.  A row whose scores are all the same huge negative number is uniform as long as that is finite (and its keys
+    held; beyond them the last place of the normaliser is more than log n).  At 6e4 the exponents of a row's first block, which has
+    no reference yet, are rounded to 2^-8 and the probabilities to 2^-8 of themselves."""
+    r = 300
+    for what in ("-inf", "+inf", "nan", "low"):
+        q, k, v, n = problem(1, Hq, Hq, S, D, half, 0, 0, seed=5)
+        _, _, base = scores(q, k, v, n, 1.0)
+        seen = lambda: (n[0, 0, r].double() + k[0, 0].double() @ q[0, 0, r].double() * D ** -0.5)[: r + 1].softmax(0)
+        before = seen()
+        if what == "low":
+            n[0, 0, r] = -6e4 if half else -1e38
+        elif what == "-inf":
+            n[0, 0, r] = float("-inf")
+        else:
+            n[0, 0, r, 5] = float(what)
+        _, rows, c = scores(q, k, v, n, 1.0)
+        assert torch.equal(c[:, 1:], base[:, 1:])
+        assert ((c[0, 0, r + 1:] - base[0, 0, r + 1:]).abs() <= 2e-5 * base[0, 0, r + 1:]).all(), what
+        if what == "low":
+            want = base[0, 0, : r + 1].double() - before + seen()
+            assert ((c[0, 0, : r + 1] - want).abs() <= 2e-5 * want + (2.0 ** -7 * seen() if half else 0)).all()
+        else:
+            assert c[0, 0, : r + 1].isnan().all(), what
+
+
 def test_captured_module_and_where_the_rule_lies():
     from triton_amd import modules, ops
     # fp32 from 32 MB (head_dim 64) and 48 to 640 MB (128), causal squares of more than 128 queries only

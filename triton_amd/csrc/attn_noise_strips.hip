@@ -206,7 +206,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 
-    constexpr float kNone = -1e30f;              // the reference of a row that has seen no finite score
+    constexpr float kNone = -3e38f;              // the reference of a row that has seen no finite score
     half8_t qA[NKS];
     float mlane = kNone, lsum = 0.f;             // of the one row a lane keeps: reference and sum
     auto row_of = [](int ln) __attribute__((always_inline)) { return 8 * ((ln & 15) >> 2) + 4 * (ln >> 5) + (ln & 3); };
@@ -391,17 +391,27 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
         const float lse2 = mx + fast_log2(ls);
         const bool real = q0 + row < a.S;
         if (wave == 0 && (lane & 16) == 0 && real) a.lse[((int64_t)b * a.Hq + head) * a.S + q0 + row] = lse2 * kLn2;
-        // ---- the held blocks' column sums
+        // ---- the held blocks' column sums.  (Weights without lse2, whose rounding at 1e8 and more would be a factor.  A row without
+        // a normaliser -- no finite score, or +inf or NaN among them -- makes a NaN of every key that it sees; of the others, whose
+        // exponentials are zeros, it must not: they are left out where a block has any.)
         float w[16];
-        spread(real ? fast_exp2(mlane - lse2) : 0.f, w);
+        spread(real ? fast_exp2(mlane - mx) * __builtin_amdgcn_rcpf(ls) : 0.f, w);
 #pragma unroll
         for (int i = 0; i < kHeldBlocks; ++i)
             if (i < nh) {
+                const int key0 = 32 * (wave + NW * (early + i));
                 float x = held[i][0] * w[0];
+                if (key0 == q0) {
+                    const int ln = lane_now(), from = (ln & 31) - 4 * (ln >> 5);      // (compared here and not once for all blocks)
+                    if (from > 0) x = 0.f;
 #pragma unroll
-                for (int r = 1; r < 16; ++r) x = __builtin_fmaf(held[i][r], w[r], x);
+                    for (int r = 1; r < 16; ++r) x = 8 * (r / 4) + (r % 4) >= from ? __builtin_fmaf(held[i][r], w[r], x) : x;
+                } else {
+#pragma unroll
+                    for (int r = 1; r < 16; ++r) x = __builtin_fmaf(held[i][r], w[r], x);
+                }
                 x = half_sum(x);
-                if (h == 0) Cs[32 * (wave + NW * (early + i)) + c] += x;
+                if (h == 0) Cs[key0 + c] += x;
             }
         // ---- ... and the others', once more from K and the noise
         if (early > 0) {
