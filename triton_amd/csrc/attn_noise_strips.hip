@@ -445,7 +445,14 @@ __global__ __launch_bounds__(256) void attn_add_slots_kernel(const float* part, 
     const int64_t bh = i / Skv, key = i % Skv;
     const float* p = part + bh * n_slots * Skv + key;
     float x = 0.f;
-    for (int s = 0; s < n_slots; ++s) x += p[(int64_t)s * Skv];
+    for (int s = 0; s < n_slots; s += 8) {       // (eight on their way at once.  Whole calls, us, one after the other / so: 8 heads of 128, 4096 keys (32
+                                                 // slots) 144.3 / 137.8; 16 of 64, 1536 41.9 / 39.4; 32 of 128, 1024 44.6 / 41.9)
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[(int64_t)min(s + e, n_slots - 1) * Skv];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x += s + e < n_slots ? v[e] : 0.f;
+    }
     store_stat(out, s16, i, x);
 }
 
