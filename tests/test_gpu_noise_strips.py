@@ -51,9 +51,10 @@ def check(q, k, n, rows, c, tau, tol, heads, largest=0.0):
 
 # B, Hq, Hkv, S, D, fp16 noise, spare elements per row, first element
 CASES = [
-    (9, 72, 1, 161, 64, False, 0, 0), (16, 64, 8, 129, 64, False, 3, 1), (6, 71, 1, 256, 64, True, 0, 0), (5, 71, 71, 287, 64, True, 1, 1),
-    (13, 32, 8, 255, 128, False, 1, 0), (13, 32, 8, 289, 128, True, 0, 1),                     # strips and blocks cut short
-    (2, 24, 6, 1024, 128, False, 0, 0), (2, 24, 6, 1057, 128, True, 0, 1), (1, 40, 8, 1056, 64, False, 32, 0),     # at the end of the held keys
+    (2, 72, 1, 321, 64, False, 0, 0), (4, 64, 8, 353, 64, False, 3, 1), (1, 71, 1, 352, 64, True, 0, 0), (1, 71, 71, 351, 64, True, 1, 1),
+    (3, 32, 8, 351, 128, False, 1, 0), (1, 32, 8, 321, 128, True, 0, 1), (1, 32, 8, 300, 128, True, 3, 1), (1, 32, 4, 415, 128, False, 0, 0),    # strips and blocks cut short
+    (1, 8, 2, 800, 128, True, 0, 0), (2, 32, 8, 625, 128, True, 1, 1), (1, 16, 16, 703, 64, True, 0, 0), (1, 16, 4, 737, 64, False, 0, 0),    # the rule's lines
+    (2, 24, 6, 1024, 128, False, 0, 0), (1, 32, 8, 1057, 128, True, 0, 1), (1, 40, 8, 1056, 64, False, 32, 0),     # at the end of the held keys
     (1, 4, 1, 2048, 64, False, 0, 0), (1, 5, 5, 2081, 64, False, 0, 2), (1, 8, 2, 2305, 128, True, 1, 0), (1, 6, 3, 2113, 128, False, 3, 0),
     (1, 3, 1, 4801, 128, False, 0, 0), (1, 2, 2, 4830, 64, True, 2, 1),                        # the longest rows
 ]
@@ -124,11 +125,12 @@ def test_rows_without_a_normaliser(S, D, Hq, half):
 
 def test_captured_module_and_where_the_rule_lies():
     from triton_amd import modules, ops
-    # fp32 from 32 MB (head_dim 64) and 48 to 640 MB (128), causal squares of more than 128 queries only
+    # from 300 keys and some MB of noise; the workspace serves either type
     def need(B, H, S, D, causal=True, Skv=None):
         q, k = (torch.as_strided(torch.empty(1 << 20, device="cuda", dtype=torch.half), (B, H, s, D), (0, 0, D, 1)) for s in (S, Skv or S))
         return ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, causal, True)
-    assert need(1, 71, 600, 64) > 0 and need(1, 71, 300, 64) == 0 and need(1, 32, 1024, 128) > 0 and need(1, 8, 1536, 128) == 0 and need(1, 8, 2050, 128) > 0
+    assert need(1, 71, 300, 64) > 0 and need(1, 71, 299, 64) == 0 and need(1, 16, 600, 64) == 0 and need(1, 16, 700, 64) > 0
+    assert need(1, 32, 300, 128) > 0 and need(1, 8, 600, 128) == 0 and need(1, 8, 800, 128) > 0 and need(1, 32, 3000, 128) > 0
     assert need(1, 32, 4096, 128) == 0 and need(1, 71, 600, 64, causal=False) == 0 and need(1, 71, 600, 64, Skv=700) == 0
     assert need(64, 71, 128, 64) == 0 and need(1, 71, 4900, 64) == 0
     q, k, v, n = problem(1, 71, 1, 608, 64, False, 0, 0)

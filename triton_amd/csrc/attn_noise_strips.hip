@@ -457,20 +457,28 @@ __global__ __launch_bounds__(256) void attn_add_slots_kernel(const float* part, 
 }
 
 // Where the two launches here -- one where a head has one workgroup -- and the plain attention are faster than the forward with
-// noise and the column statistics: causal prompts whose noise is large enough to pay for the third launch, and for head_dim 128,
-// where a block's K is twice its noise, not those that keep the two passes at the rate of HBM all the time.  us, two passes / here:
-//   fp32  71 heads of 64: 300 keys (13 MB) 22.3 / 22.6, 600 40.6 / 33.4, 1100 106 / 78, 1536 151 / 113, 2050 301 / 235, 2752 457 /
-//         337; 16 of 64: 600 24.2 / 25.7, 1100 (39 MB) 43.6 / 37.3, 2050 89 / 76, 4096 210 / 186; 32 of 128: 1024 (67 MB) 51.9 /
-//         48.7, 1501 94 / 89, 2048 163 / 129, 3000 (576 MB) 298 / 277, 4096 449 / 461; 8 of 128: 1100 40 / 48, 1536 (38 MB) 50 / 55,
-//         2050 (67 MB) 83 / 72, 4096 172 / 150
-//   fp16  71 of 64: 600 (26 MB) 37.7 / 34.4, 1100 77 / 64, 1536 128 / 111, 2752 349 / 318; 16 of 64: 1536 (38 MB) 52 / 42, 2050 (67
-//         MB) 68 / 65, 2752 91 / 100; 32 of 128: 1024 (34 MB) 49.5 / 45.9, 1501 (72 MB) 74.1 / 77.0, 3000 231 / 245; 8 of 128: 2050 (34
-//         MB) 80 / 71, 4096 157 / 139
+// noise and the column statistics.  A third launch and the strips' ends have to be paid for: causal prompts of 300 keys and more
+// with some MB of (visible) noise, the fewer heads the more of it; and for head_dim 128, where a block's K is twice its noise, not
+// those that keep the two passes at the rate of HBM all the time, nor fp16 noise of many heads beyond 44 MB, where the strips are
+// at the rate of their arithmetic; short fp16 rows of many heads; and few heads with little more than one strip a CU.  us, two
+// passes / here (MB):
+//   D = 64, fp32   71 heads: 250 keys (9) 20.0 / 21.2, 300 (12) 21.6 / 21.0, 420 28.5 / 24.2, 600 40.6 / 33.4, 1100 106 / 78, 1536 151 / 112,
+//         2752 457 / 333; 16: 600 (11) 24.2 / 24.3, 700 (15) 27.8 / 24.7, 1100 43.6 / 37.3, 4096 210 / 186; 8 x 16, 200 19.9 / 19.8
+//   D = 64, fp16   71: 250 (4) 19.4 / 20.7, 360 (9) 24.0 / 23.1, 500 30.0 / 28.3, 1100 77 / 64, 2752 344 / 311; 2 x 71, 350 30.2 / 31.4; 8 x 16, 310 23.2 / 24.4; 16: 600
+//         (5) 24.8 / 25.0, 700 (7) 27.5 / 25.7, 1100 41.7 / 35.2, 1536 52 / 39, 2500 (95) 84 / 79, 2752 (115) 94 / 103, 4000 161 / 169
+//   D = 128, fp32  32: 400 keys (10) 32.1 / 24.0, 600 36.1 / 33.2, 777 44.5 / 38.8, 1024 51.9 / 42, 2048 163 / 124, 3000 (549) 288 / 270, 3600 (791)
+//         389 / 395, 4096 439 / 457; 4 x 32, 401 41.4 / 39.6; 8 x 32, 200 (20) 29.7 / 31.5; 2 x 8, 1000 (31) 48.3 / 36.4; 8: 1100 (18) 39.9 / 41.3,
+//         1536 (36) 49.2 / 49.6, 1650 (42) 57.5 / 49.3, 1800 63 / 50, 4096 172 / 143
+//   D = 128, fp16  32: 300 (3) 27.5 / 20.9, 500 31.7 / 26.6, 777 42.5 / 37.7, 1000 49.8 / 42.6, 1201 (44) 56.6 / 56.0, 1350 (56) 64.3 / 68.4, 1633 84 /
+//         97, 2500 169 / 174; 2 x 32, 700 47.0 / 42.7; 4 x 32, 401 36.4 / 38.5; 8: 800 (5) 32.3 / 25.8, 1000 35.7 / 28.2, 1101 (280 strips) 39.4 / 41.9, 1350 (344) 46.7 / 44.4, 1536 51.6 / 46.6, 2050 80 /
+//         69, 4096 157 / 138
 static bool strips_suit(const trn_attn_desc* d, bool n16) {
-    if (!d->causal || d->seq_q != d->seq_kv || d->seq_q <= 128) return false;
+    if (!d->causal || d->seq_q != d->seq_kv || d->seq_q < 300) return false;
     const int64_t bh = (int64_t)d->batch * d->n_q_heads, mb = (bh * d->seq_q * d->seq_q * (n16 ? 1 : 2)) >> 20;
-    if (d->head_dim == 64) return n16 ? mb >= 24 && (bh >= 32 || mb <= 80) : mb >= 32;
-    return n16 ? mb >= 32 && (bh <= 16 || mb <= 64) : mb >= 48 && mb <= 640;
+    if (d->head_dim == 64) return n16 ? mb >= 7 && (bh >= 32 || mb <= 96) && (bh <= 80 || d->seq_q >= 600) : mb >= 12;
+    const int64_t strips = bh * ((d->seq_q + 31) / 32);
+    if (n16) return bh <= 16 ? mb >= 4 && (strips <= 256 || strips > 320) : mb <= 44 && (bh <= 32 || d->seq_q >= 600);
+    return mb >= (bh >= 32 ? 9 : bh >= 16 ? 28 : 38) && mb <= 640;
 }
 // Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
 // and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
