@@ -250,7 +250,7 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
 /*
  * Attention and per-key statistics for every shape and element type in one entry point: what the KeyFormer and RoCo
  * modules call.  As trn_attn_fwd_stats_ws_f16 (one launch with at most 32 queries per head unless the workspace makes it
- * split the keys, and with at most 128 queries and 128 keys; two launches otherwise), with
+ * split the keys, and with at most 128 queries and 128 keys; two launches otherwise, up to three with noise and a workspace), with
  *   noise       nullable; fp16 when noise_half is set, float otherwise.  Rows at any pitch and any element alignment (the
  *               reference's noise [.., M, P + M] is fp16 with any key count); desc's noise strides count elements.  One
  *               head is addressed with 32-bit offsets: (seq_q + TRN_STATS_SPARE_ROWS) * noise_stride_s * 4 < 2^31 where
@@ -260,13 +260,14 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
  *   out1, out2  [batch, n_q_heads, seq_kv] contiguous, fp16 when out_half is set (the float result rounded once), float
  *               otherwise: sum and sum of squares (one may be NULL) or, with mean_std (without noise; both required), mean
  *               and standard deviation as trn_attn_colmeanstd_f16.
- *   workspace   nullable: trn_attn_key_scores_workspace_bytes(desc, noise given) bytes (0: none), 256-byte aligned, no initial
- *               contents needed: the keys of at most 32 queries are then split over workgroups, and the launch that merges
- *               their results sweeps over the keys for the statistics.  With fewer bytes, but those of
- *               trn_attn_workspace_bytes(desc), over as many as these are for; with less than that, not at all.  Without noise it
- *               serves a chunk of more than 32 queries too, as trn_attn_chunk_workspace_bytes does without statistics; with noise
- *               a prompt whose scores are then formed in one pass over the noise.  One that
- *               is not 256-byte aligned is not used (TRN_E_ALIGN where trn_attn_stats_workspace_bytes names a size that it has).
+ *   workspace   nullable: trn_attn_key_scores_workspace_bytes(desc, with_noise) bytes (0: none; with_noise 0 without noise, 1
+ *               with noise of either type, 2 fp16, 3 float), 256-byte aligned, no initial contents needed.  The keys of at most
+ *               32 queries are then split over workgroups, and the launch that merges their results sweeps over the keys for
+ *               the statistics; with fewer bytes, but those of trn_attn_workspace_bytes(desc), over as many as these are for;
+ *               with less than that, not at all.  Without noise it serves a chunk of more than 32 queries too, as
+ *               trn_attn_chunk_workspace_bytes does without statistics; with noise a prompt, whose scores are then formed in
+ *               one pass over the noise.  One that is not 256-byte aligned is not used (TRN_E_ALIGN where
+ *               trn_attn_stats_workspace_bytes names a size that it has).
  */
 #define TRN_STATS_SPARE_ROWS 128        /* query rows past the last that the statistics kernels may ask for (as zeros) */
 int64_t trn_attn_key_scores_workspace_bytes(const trn_attn_desc* desc, int32_t with_noise);

@@ -126,10 +126,11 @@ def test_rows_without_a_normaliser(S, D, Hq, half):
 def test_captured_module_and_where_the_rule_lies():
     from triton_amd import modules, ops
     # from 300 keys and some MB of noise; the workspace serves either type
-    def need(B, H, S, D, causal=True, Skv=None):
+    def need(B, H, S, D, causal=True, Skv=None, noise=True):
         q, k = (torch.as_strided(torch.empty(1 << 20, device="cuda", dtype=torch.half), (B, H, s, D), (0, 0, D, 1)) for s in (S, Skv or S))
-        return ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, causal, True)
+        return ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, causal, noise)
     assert need(1, 71, 300, 64) > 0 and need(1, 71, 299, 64) == 0 and need(1, 16, 600, 64) == 0 and need(1, 16, 700, 64) > 0
+    assert need(1, 8, 1000, 128, noise=2) > 0 and need(1, 8, 1000, 128, noise=3) == 0 and need(1, 32, 1501, 128, noise=2) == 0 and need(1, 32, 1501, 128, noise=3) > 0
     assert need(1, 32, 300, 128) > 0 and need(1, 8, 600, 128) == 0 and need(1, 8, 800, 128) > 0 and need(1, 32, 3000, 128) > 0
     assert need(1, 32, 4096, 128) == 0 and need(1, 71, 600, 64, causal=False) == 0 and need(1, 71, 600, 64, Skv=700) == 0
     assert need(64, 71, 128, 64) == 0 and need(1, 71, 4900, 64) == 0

@@ -750,7 +750,7 @@ extern "C" int64_t trn_attn_key_scores_workspace_bytes(const trn_attn_desc* d, i
     using namespace trn;
     if (!d || validate_attn(d, true) != TRN_OK) return 0;
     // a chunk of more than 32 queries without noise: its forward shares out the keys as it does without the statistics
-    if (d->seq_q > 32 && with_noise) return noise_strips_workspace_bytes(d);
+    if (d->seq_q > 32 && with_noise) return noise_strips_workspace_bytes(d, with_noise);
     if (d->seq_q > 32) return attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
     return attn_decode_stats_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
 }
@@ -813,7 +813,7 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     if (attn_short_suits(d->seq_q, d->seq_kv))
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, mean_std != 0);
     // The scores of a prompt in one pass over the noise, and its attention, which needs none, on the plain kernel
-    if (n && s1 && !s2 && workspace && noise_strip_slots(d, n16) > 0 && workspace_bytes >= noise_strips_workspace_bytes(d)) {
+    if (n && s1 && !s2 && workspace && noise_strip_slots(d, n16) > 0 && workspace_bytes >= noise_strips_workspace_bytes(d, n16 ? 2 : 3)) {
         st = attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream);
         if (st != TRN_OK) return st;
         return launch_noise_strips(d, q, k, noise, n16, rows, out1, s16, workspace, (hipStream_t)stream) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;

@@ -503,8 +503,9 @@ int noise_strip_slots(const trn_attn_desc* d, bool n16) {
     return best;
 }
 
-int64_t noise_strips_workspace_bytes(const trn_attn_desc* d) {
-    const int64_t n = noise_strip_slots(d, false) > 0 ? noise_strip_slots(d, false) : noise_strip_slots(d, true);
+int64_t noise_strips_workspace_bytes(const trn_attn_desc* d, int with_noise) {
+    const int n32 = with_noise == 2 ? 0 : noise_strip_slots(d, false), n16 = with_noise == 3 ? 0 : noise_strip_slots(d, true);
+    const int64_t n = n32 > 0 ? n32 : n16;       // (the same number where both suit)
     return n * d->batch * d->n_q_heads * d->seq_kv * 4;
 }
 

@@ -268,7 +268,7 @@ class KeyFormerAttention(FusedModule):
         n4 = _noise_operand(self, _as4(noise, "noise"))
         lsep = self._workspace("lse_pert", (B, Hq, Sq), torch.float32, q.device)
         score, = _score_outputs(self, (C_out,), (B, Hq, Skv))
-        need = ops.attention_key_scores_workspace_bytes(q, k, v, o, _scale(self.scale, D), self.causal, True)
+        need = ops.attention_key_scores_workspace_bytes(q, k, v, o, _scale(self.scale, D), self.causal, 2 if n4.dtype == torch.float16 else 3)
         parts = self._workspace("key_parts", (need,), torch.uint8, q.device) if need else None
         ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lsep, score, noise=n4, tau=self.tau, workspace=parts)
         _store_scores(C_out, score)

@@ -194,10 +194,10 @@ def attention_stats_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> i
     return int(_lib.load().trn_attn_stats_workspace_bytes(C.byref(d)))
 
 
-def attention_key_scores_workspace_bytes(q, k, v, o, scale: float, causal: bool, with_noise: bool) -> int:
+def attention_key_scores_workspace_bytes(q, k, v, o, scale: float, causal: bool, with_noise) -> int:
     """Bytes of workspace with which `attention_key_scores` would split the keys of this problem over several workgroups
     and run the statistics with the merge of their results as a second launch, or form a prompt's scores in one pass over
-    its noise (0: it would not)."""
+    its noise (0: it would not).  with_noise: False, True (noise of either type), 2 (fp16) or 3 (fp32)."""
     d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, None, 1.0)
     return int(_lib.load().trn_attn_key_scores_workspace_bytes(C.byref(d), int(with_noise)))
 
