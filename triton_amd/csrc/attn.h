@@ -107,12 +107,13 @@ __device__ __forceinline__ void store_stat(float* out, int s16, int64_t at, floa
     else out[at] = v;
 }
 
-// Checks, argument block and kernel choice behind every attention entry point of the C ABI.
+// Checks, argument block and kernel choice behind every attention entry point of the C ABI.  given_q: without noise too the queries
+// are not multiplied by the scale, and rounded, before the products (attn_fwd16.hip; the other kernels never do).
 int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                  const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
                  bool n16 = false, bool s16 = false, bool any_pitch = false, bool k_norm = false, const void* gamma_k = nullptr,
-                 float k_eps = 0.f, bool mean_std = false);
+                 float k_eps = 0.f, bool mean_std = false, bool given_q = false);
 
 // The checks of attn_colstats by themselves, for a caller that launches something else before it.
 int attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
@@ -163,7 +164,7 @@ hipError_t launch_attn_short(const AttnArgs& a, int head_dim, hipStream_t s);
 // take every other 64-key tile each (small grids, long walks).
 enum class Attn16Shape { Narrow, Wide, Paired, Split };
 Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal);
-hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, hipStream_t stream);
+hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, bool given_q, hipStream_t stream);
 // The keys of a chunk of queries against a long cache shared out over workgroups (attn_fwd16.hip): fp32 partial results in
 // args.ws, attn_share_workspace_bytes of it (0: this problem is not shared out), merged by a second launch.
 int64_t attn_share_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);

@@ -812,9 +812,11 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     if (st != TRN_OK) return st;
     if (attn_short_suits(d->seq_q, d->seq_kv))
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, mean_std != 0);
-    // The scores of a prompt in one pass over the noise, and its attention, which needs none, on the plain kernel
+    // The scores of a prompt in one pass over the noise, and its attention, which needs none, on the kernels without it (the queries
+    // as given, as the forward with noise takes them)
     if (n && s1 && !s2 && workspace && noise_strip_slots(d, n16) > 0 && workspace_bytes >= noise_strips_workspace_bytes(d, n16 ? 2 : 3)) {
-        st = attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream);
+        st = attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream, nullptr, false, false, false, false,
+                          nullptr, 0.f, false, true);
         if (st != TRN_OK) return st;
         return launch_noise_strips(d, q, k, noise, n16, rows, out1, s16, workspace, (hipStream_t)stream) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     }
@@ -866,7 +868,7 @@ extern "C" int trn_attn_qknorm_f16(const trn_attn_desc* d, const void* q, const 
 int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                              int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs,
-                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps, bool mean_std) {
+                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps, bool mean_std, bool given_q) {
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
     if (!d || !q || !k || !v || !o) return TRN_E_NULL;
     if (noise && !lse_pert) return TRN_E_NULL;
@@ -925,7 +927,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         return launch_attn_decode(a, d->head_dim, workspace, workspace_bytes, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     // Without score perturbation: the 16x16x32 kernel, in the workgroup shape its launcher's rule picks.
     if (!noise)
-        return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0), s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+        return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0), given_q, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     // With it: the shape of noise_shape().
     const NoiseShape shape = noise_shape(d);
     const bool stream_noise = noise_streams(d, noise, n16);

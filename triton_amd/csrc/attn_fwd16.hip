@@ -64,7 +64,12 @@ template <int D> __device__ __forceinline__ int swz16(int r) {
 struct Scores16 { float4_t s[2][2]; };      // [key half][query block]
 
 #if defined(__HIP_DEVICE_COMPILE__)
-template <int D, int NW, int MODE>
+// GIVEN: the queries enter the products as they are given, and the fp32 scores are multiplied by scale * log2(e) -- one FMA a score,
+// behind the MFMAs of phase B, which also subtracts m (the chains start from zero then).  Q times scale * log2(e) rounded to fp16
+// is another rounding of the queries: O against float64, 1024 tokens, 32 heads of 128: 3.1e-4 for N(0,1), 4.0e-4 and 6.1e-4 for queries
+// twice and eight times as large, where the queries as given leave 2.5e-4, 2.5e-4 and 2.1e-4.  For KeyFormer's prompts whose noise has a
+// pass of its own, as the kernel that takes the noise along does.
+template <int D, int NW, int MODE, bool GIVEN = false>
 __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     constexpr bool PAIRED = MODE == kPaired, SHARE = MODE == kShare, SPLIT = MODE == kSplit || SHARE;
     static_assert(MODE == kPlain || NW == 8, "paired query tiles and split keys are two groups of four waves");
@@ -295,7 +300,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
             if constexpr (SYNC) {
                 if (i == NS - 2 * NQ) handover();
             }
-            sn.s[kb][qb] = mfma16(ka[op % NQ], qB[qb][ks], ks == 0 ? negm[qb] : sn.s[kb][qb]);
+            sn.s[kb][qb] = mfma16(ka[op % NQ], qB[qb][ks], ks == 0 ? (GIVEN ? zero : negm[qb]) : sn.s[kb][qb]);
             if (i & 1) {
                 if (op + NQ < NOP) load_k(K1, op + NQ, op % NQ);
                 else load_v(op + NQ - NOP, op % NQ);
@@ -321,6 +326,15 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
                 if (i % EVERY == EVERY - 1) refill(i / EVERY);
             }
             constexpr int R0 = NS / 2 - (NS >= 16 ? 3 : 2);
+            if constexpr (GIVEN) {      // the block's four quads of scores in the slots before R0, those of the last MFMAs last
+                constexpr int PER = NS >= 16 ? 1 : 2, FIRST = R0 - 4 / PER;
+                if (i >= FIRST && i < R0)
+#pragma unroll
+                    for (int u = PER * (i - FIRST); u < PER * (i - FIRST + 1); ++u)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            sn.s[u >> 1][u & 1][e] = __builtin_fmaf(sn.s[u >> 1][u & 1][e], a.c1, negm[u & 1][0]);
+            }
             if (i == R0) { if (MAYMASK && masked_next) mask_block(sn, key0_next); }
             if (i >= R0 && i < R0 + 4) mx = max_piece(sn, i - R0, mx);
             if (i == R0 + 3) due = __builtin_amdgcn_ballot_w64(mx > 0x41000000) != 0 || (SPLIT && any_fresh);       // 8.0f
@@ -395,6 +409,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
             }
         }
         // the softmax scale and log2(e) go into Q once, so that the scores leave the matrix pipe ready for exp2
+        if constexpr (!GIVEN)
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks)
 #pragma unroll
@@ -424,6 +439,9 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
 #pragma unroll
         for (int i = 0; i < NQ; ++i) load_k(SHARE ? Ks1 : Ks0 + 32 * D, i, i);
         // block 0 sets the reference outright (every query sees key 0, so it is finite from here on)
+        if constexpr (GIVEN)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sA.s[i >> 1][i & 1] = sA.s[i >> 1][i & 1] * a.c1;
         float smax[2];
         mask_block(sA, kfirst);
         block_max(sA, smax);
@@ -685,6 +703,13 @@ __global__ __launch_bounds__(512, 1) void attn_fwd16_split_kernel(const AttnArgs
 #endif
 }
 
+template <int D, int NW, int MODE>
+__global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_fwd16_given_kernel(const AttnArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    attn_fwd16_body<D, NW, MODE, true>(a);
+#endif
+}
+
 template <int D>
 __global__ __launch_bounds__(512, 1) void attn_fwd16_share_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -778,13 +803,14 @@ hipError_t launch_attn_shares(const AttnArgs& a, int head_dim, hipStream_t s) {
     return head_dim == 128 ? launch_shares<128>(a, s) : launch_shares<64>(a, s);
 }
 
-template <int D, int NW, int MODE>
+template <int D, int NW, int MODE, bool GIVEN>
 static hipError_t launch16(AttnArgs a, hipStream_t s) {
     const int rows = MODE == kPlain ? 32 * NW : 128;
     a.n_qtiles = (int)(((int64_t)a.Sq + rows - 1) / rows);
     const int64_t grid = (int64_t)(MODE == kPaired ? (a.n_qtiles + 1) / 2 : a.n_qtiles) * a.B * a.Hq;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
-    if constexpr (MODE == kSplit) hipLaunchKernelGGL((attn_fwd16_split_kernel<D>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    if constexpr (GIVEN) hipLaunchKernelGGL((attn_fwd16_given_kernel<D, NW, MODE>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+    else if constexpr (MODE == kSplit) hipLaunchKernelGGL((attn_fwd16_split_kernel<D>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
     else hipLaunchKernelGGL((attn_fwd16_kernel<D, NW, MODE == kPaired>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
     return hipGetLastError();
 }
@@ -821,14 +847,17 @@ Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, in
     return head_dim == 128 && wide ? Attn16Shape::Wide : Attn16Shape::Narrow;
 }
 
-hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, hipStream_t s) {
-    const bool d128 = head_dim == 128;
+template <bool GIVEN>
+static hipError_t launch_shape(const AttnArgs& a, bool d128, Attn16Shape shape, hipStream_t s) {
     switch (shape) {
-        case Attn16Shape::Paired: return d128 ? launch16<128, 8, kPaired>(a, s) : launch16<64, 8, kPaired>(a, s);
-        case Attn16Shape::Split:  return d128 ? launch16<128, 8, kSplit>(a, s) : launch16<64, 8, kSplit>(a, s);
-        case Attn16Shape::Wide:   return launch16<128, 8, kPlain>(a, s);             // (head_dim 128 only)
-        default:                  return d128 ? launch16<128, 4, kPlain>(a, s) : launch16<64, 4, kPlain>(a, s);
+        case Attn16Shape::Paired: return d128 ? launch16<128, 8, kPaired, GIVEN>(a, s) : launch16<64, 8, kPaired, GIVEN>(a, s);
+        case Attn16Shape::Split:  return d128 ? launch16<128, 8, kSplit, GIVEN>(a, s) : launch16<64, 8, kSplit, GIVEN>(a, s);
+        case Attn16Shape::Wide:   return launch16<128, 8, kPlain, GIVEN>(a, s);             // (head_dim 128 only)
+        default:                  return d128 ? launch16<128, 4, kPlain, GIVEN>(a, s) : launch16<64, 4, kPlain, GIVEN>(a, s);
     }
+}
+hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, bool given_q, hipStream_t s) {
+    return given_q ? launch_shape<true>(a, head_dim == 128, shape, s) : launch_shape<false>(a, head_dim == 128, shape, s);
 }
 
 const char* attn_fwd16_kernel_name(int head_dim, Attn16Shape shape) {
