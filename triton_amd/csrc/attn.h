@@ -27,15 +27,25 @@ struct AttnArgs {
     float* probs;
     int n16;       // noise points at fp16 data (its pitches count halfs; any alignment: see HalfNoise)
     int s16;       // decode and short kernels: col_sum and col_sumsq point at fp16 data
+    int o_nt;      // prefill kernels: the output goes past the caches (outputs_stream)
 };
 
-// 16 bytes of the output, past the caches: what a launch leaves dirty in the L2s is written back before it ends, and the next
-// layer's rows come from the last-level cache no faster than from HBM.  Attention launches, us, through the caches / past them: 8 x 500
-// tokens, 32 heads of 128 34.0 / 29.0, 4 x 777 35.4 / 33.9, 1100 21.4 / 20.7, 4096 138.2 / 136.3; 8 x 300, 16 heads of 64 8.5 / 8.3;
-// 71 of 64, 1000 tokens 18.7 / 17.7, 400 8.65 / 8.52; with key scores, whole calls: 4096 tokens 448 / 441, 71 of 64, 1500 129 / 126;
-// outputs of 1 MB and less the same.  (Not for the projections, whose outputs the next launch reads: a block of 2000 tokens, 16 heads of
-// 64 46.5 / 50.5.)
-__device__ __forceinline__ void store_out(half_t* p, uint4_t v) { __builtin_nontemporal_store(v, reinterpret_cast<uint4_t*>(p)); }
+// Whether a launch of so many outputs stores them past the caches.  What it leaves dirty in the L2s is written back before it ends, on
+// top of the launch; but the projection behind an attention reads what the caches still hold.  us, through the caches / past them:
+//   the launch alone: 32 heads of 128: 4 x 777 tokens (25 MB) 36.1 / 33.1, 8 x 500 34.3 / 30.4, 4096 122.2 / 117.7, 2 x 2048 74.7 / 67.7
+//   and a projection to the same width behind it, by the library's product; by ours: 4 x 777 133.8 / 132.8; 152.1 / 151.7, 12 x 260 (26 MB)
+//     125.9 / 127.0; 143.8 / 143.6, 8 x 500 (33 MB) 144.1 / 142.5; 167.4 / 165.0, 4 x 1024 158.8 / 158.4; 183.3 / 181.5, 4096 233.6 / 233.8; 258.2 / 258.0
+//   the losses: 300 tokens (2.5 MB) 45.5 / 45.5; 32.4 / 37.4, 777 (6 MB) 56 / 56; 51.7 / 55.1, and an addition behind 2048 (17 MB) 51.1 / 52.3,
+//     2800 (23 MB) 78.3 / 78.9 (26 MB and more the same); 71 heads of 64: 400 (4 MB) 45.2 / 49.7; 40.6 / 51.7, 3 x 1000 (27 MB) 159 / 163.4; 277.5 / 277.8
+inline bool outputs_stream(int64_t rows, int head_dim) { return head_dim == 128 && rows * head_dim * 2 >= (int64_t)24 << 20; }
+// 16 bytes of the output
+__device__ __forceinline__ void store_out(half_t* p, uint4_t v, int past) {
+    if (past) {
+        asm volatile("" ::: "memory");      // (the two stores would be merged into one without the hint)
+        __builtin_nontemporal_store(v, reinterpret_cast<uint4_t*>(p));
+        asm volatile("" ::: "memory");
+    } else *reinterpret_cast<uint4_t*>(p) = v;
+}
 
 // fp16 noise as the kernels fetch it.  Its rows may start at any element (the reference's [.., M, P + M] tensors have any
 // key count), so a lane reads the whole dwords around its 4 keys -- three of them cover both cases -- and shifts by half a

@@ -509,7 +509,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
             const uint2_t lo = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol]);
             const uint2_t hi = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol + 4]);
             if (wq0 + r < a.Sq)
-                store_out(ob + (int64_t)(wq0 + r) * a.os + ocol, uint4_t{lo.x, lo.y, hi.x, hi.y});
+                store_out(ob + (int64_t)(wq0 + r) * a.os + ocol, uint4_t{lo.x, lo.y, hi.x, hi.y}, a.o_nt);
         }
         if (grp == 1) return;               // (the normalisers are written once)
     } else {
@@ -540,7 +540,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
                 const uint2_t lo = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol]);
                 const uint2_t hi = *reinterpret_cast<const uint2_t*>(&ot[r * OP + ocol + 4]);
                 if (wq0 + r < a.Sq)
-                    store_out(ob + (int64_t)(wq0 + r) * a.os + pass * DP + ocol, uint4_t{lo.x, lo.y, hi.x, hi.y});
+                    store_out(ob + (int64_t)(wq0 + r) * a.os + pass * DP + ocol, uint4_t{lo.x, lo.y, hi.x, hi.y}, a.o_nt);
             }
         }
     }
@@ -903,6 +903,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     a.q_eps = d->q_norm_eps; a.causal = d->causal ? 1 : 0; a.q_norm = d->q_norm ? 1 : 0;
     a.gamma_k = (const half_t*)gamma_k; a.k_eps = k_eps; a.k_norm = k_norm ? 1 : 0;
     a.n_split = 1; a.spread = 0; a.ws = nullptr; a.col_sum = col_sum; a.col_sumsq = col_sumsq; a.probs = probs; a.mean_std = mean_std ? 1 : 0; a.n16 = n16 ? 1 : 0; a.s16 = s16 ? 1 : 0;
+    a.o_nt = outputs_stream((int64_t)d->batch * d->n_q_heads * d->seq_q, d->head_dim) ? 1 : 0;
     // K/V tiles are fetched with 32-bit buffer offsets relative to the (batch, head) base
     // (with room for the blocks the pipelines request past the end, which must stay representable to read as zeros)
     if (((int64_t)d->seq_kv + 2048) * d->k_stride_s * 2 > 0x7fffffffLL || ((int64_t)d->seq_kv + 2048) * d->v_stride_s * 2 > 0x7fffffffLL)
