@@ -458,27 +458,40 @@ __global__ __launch_bounds__(256) void attn_add_slots_kernel(const float* part, 
 
 // Where the two launches here -- one where a head has one workgroup -- and the plain attention are faster than the forward with
 // noise and the column statistics.  A third launch and the strips' ends have to be paid for: causal prompts of 300 keys and more
-// with some MB of (visible) noise, the fewer heads the more of it; and for head_dim 128, where a block's K is twice its noise, not
-// those that keep the two passes at the rate of HBM all the time, nor fp16 noise of many heads beyond 44 MB, where the strips are
-// at the rate of their arithmetic; short fp16 rows of many heads; and few heads with little more than one strip a CU.  us, two
-// passes / here (MB):
-//   D = 64, fp32   71 heads: 250 keys (9) 20.0 / 21.2, 300 (12) 21.6 / 21.0, 420 28.5 / 24.2, 600 40.6 / 33.4, 1100 106 / 78, 1536 151 / 112,
-//         2752 457 / 333; 16: 600 (11) 24.2 / 24.3, 700 (15) 27.8 / 24.7, 1100 43.6 / 37.3, 4096 210 / 186; 8 x 16, 200 19.9 / 19.8
-//   D = 64, fp16   71: 250 (4) 19.4 / 20.7, 360 (9) 24.0 / 23.1, 500 30.0 / 28.3, 1100 77 / 64, 2752 344 / 311; 2 x 71, 350 30.2 / 31.4; 8 x 16, 310 23.2 / 24.4; 16: 600
-//         (5) 24.8 / 25.0, 700 (7) 27.5 / 25.7, 1100 41.7 / 35.2, 1536 52 / 39, 2500 (95) 84 / 79, 2752 (115) 94 / 103, 4000 161 / 169
-//   D = 128, fp32  32: 400 keys (10) 32.1 / 24.0, 600 36.1 / 33.2, 777 44.5 / 38.8, 1024 51.9 / 42, 2048 163 / 124, 3000 (549) 288 / 270, 3600 (791)
-//         389 / 395, 4096 439 / 457; 4 x 32, 401 41.4 / 39.6; 8 x 32, 200 (20) 29.7 / 31.5; 2 x 8, 1000 (31) 48.3 / 36.4; 8: 1100 (18) 39.9 / 41.3,
-//         1536 (36) 49.2 / 49.6, 1650 (42) 57.5 / 49.3, 1800 63 / 50, 4096 172 / 143
-//   D = 128, fp16  32: 300 (3) 27.5 / 20.9, 500 31.7 / 26.6, 777 42.5 / 37.7, 1000 49.8 / 42.6, 1201 (44) 56.6 / 56.0, 1350 (56) 64.3 / 68.4, 1633 84 /
-//         97, 2500 169 / 174; 2 x 32, 700 47.0 / 42.7; 4 x 32, 401 36.4 / 38.5; 8: 800 (5) 32.3 / 25.8, 1000 35.7 / 28.2, 1101 (280 strips) 39.4 / 41.9, 1350 (344) 46.7 / 44.4, 1536 51.6 / 46.6, 2050 80 /
-//         69, 4096 157 / 138
+// with some MB of (visible) noise, the fewer heads the more of it, and not
+//   -- few heads of short prompts with little more than one strip a CU: some CUs then have two strips, most of them one;
+//   -- the longest rows, of which 2048 keys are held and the rest is read and multiplied twice;
+//   -- head_dim 128, where a block's K is twice its fp32 noise, once the two passes keep the rate of HBM all the time;
+//   -- fp16 noise, half as much to read for the same arithmetic, of long rows: with head_dim 64 only few heads, and many, whose
+//      workgroups are full rounds; with head_dim 128 up to 44 MB, of up to 16 heads 70, 10 heads 95;
+//   -- long prompts of 64 to 319 heads with keys of their own, when the heads' count is no multiple of the 8 XCDs: a head's
+//      workgroups are then on all of them, and each L2 reads all of K.
+// Whole calls, here / two passes in per cent of time (1600 sizes; minus: faster here):
+//   D = 64, fp32   71 heads: 300 keys -1, 570 -13, 1100 -26, 2700 -23; 32: 500 -17, 1001 -19, 2000 -15; 8: 1001 -18, 2000 -27, 4000 -22.  Left out:
+//         9 and 10 heads, 900 and 1001 keys (261 to 320 strips) +2 to +9, 12, 800 +6; 4800 keys: 12 +10, 16 -3, 8 (kept) -7
+//   D = 64, fp16   71: 340 -5, 640 -13, 1100 -15, 2000 -7; 16: 1001 -26, 2000 -17; 4 x 71, 1001 -12, 2450 -10; 256, 2000 -12.  Left out: 24 heads, 1650
+//         to 2000 keys +6 to +9 (1100 kept, -6), 32, 1400 +5, 48, 1650 +4; 142 heads with keys of their own, 1650 +9
+//   D = 128, fp32  32: 390 -22, 1001 -17, 2000 -11, 3000 -6; 8: 1800 -20, 3000 -22; 71 on one KV head, 1001 -15; 256, 1001 -19.  Left out: 4400 and 4800
+//         keys -8 to +20; 16 heads, 2700 to 3640 +3 to +9; 142 with keys of their own, 1190 to 1500 +1 to +15
+//   D = 128, fp16  32: 300 -25, 640 -4, 1001 -12; 8: 1001 -20, 2000 -18, 4000 -11; 16: 1501 -18, 2000 -13; 14: 2000 -12.  Left out: 16 heads, 2200 +2,
+//         2700 to 3640 +6 to +17; 12, 2700 +3, 3640 +13; 8 and 9, 4400 +5; 32, 1350 (56 MB) +6, 2500 +3
+// Inside the lines one size in forty loses 1 to 5 %, where the strips fall badly on the CUs: 24 heads of 128, 2000 keys, fp32 +5; 48 of 64, 1001,
+// fp16 +4; 56 of 128, 300, fp32 +4.
 static bool strips_suit(const trn_attn_desc* d, bool n16) {
     if (!d->causal || d->seq_q != d->seq_kv || d->seq_q < 300) return false;
     const int64_t bh = (int64_t)d->batch * d->n_q_heads, mb = (bh * d->seq_q * d->seq_q * (n16 ? 1 : 2)) >> 20;
-    if (d->head_dim == 64) return n16 ? mb >= 7 && (bh >= 32 || mb <= 96) && (bh <= 80 || d->seq_q >= 600) : mb >= 12;
     const int64_t strips = bh * ((d->seq_q + 31) / 32);
-    if (n16) return bh <= 16 ? mb >= 4 && (strips <= 256 || strips > 320) : mb <= 44 && (bh <= 32 || d->seq_q >= 600);
-    return mb >= (bh >= 32 ? 9 : bh >= 16 ? 28 : 38) && mb <= 640;
+    const bool second_strips = bh <= 16 && strips > 256 && strips <= 320;
+    const bool scattered = bh % 8 != 0 && bh < 320 && (int64_t)d->batch * d->n_kv_heads >= 64;
+    if (d->head_dim == 64) {
+        if ((second_strips && d->seq_q <= 1024) || (d->seq_q > 4500 && bh > 8)) return false;
+        if (!n16) return mb >= 12;
+        if (d->seq_q > 1250 && !(bh < 22 ? mb <= 96 : bh >= 64 && !scattered)) return false;
+        return mb >= 7 && (bh <= 80 || d->seq_q >= 600);
+    }
+    if (d->seq_q > 4200) return false;
+    if (n16) return bh <= 16 ? mb >= 4 && !second_strips && (bh <= 8 || mb <= (bh <= 10 ? 95 : 70)) : mb <= 44 && (bh <= 32 || d->seq_q >= 600);
+    return mb >= (bh >= 32 ? 9 : bh >= 16 ? 28 : 38) && mb <= (bh > 12 && bh < 18 ? 200 : 640) && (!scattered || d->seq_q <= 700);
 }
 // Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
 // and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
