@@ -156,6 +156,33 @@ def test_rows_without_a_normaliser(S, D, Hq, half):
             assert c[0, 0, : r + 1].isnan().all(), what
 
 
+@pytest.mark.parametrize("general", [False, True])
+def test_capture_with_noise_of_the_other_type(general):
+    """One eager call per shape is what a capture needs, with noise of either type: where only fp16 noise has the single pass, a
+    capture with it after an eager call with fp32 noise goes without its workspace, in two passes.  general: scores that the kernels
+    do not write themselves (the path in Python)."""
+    from triton_amd import modules
+    q, k, v, n = problem(1, 8, 2, 1000, 128, True, 0, 0)
+    c, o = torch.empty(1, 8, 2000, dtype=torch.half, device="cuda")[..., ::2] if general else torch.empty(1, 8, 1000, dtype=torch.half, device="cuda"), torch.empty_like(q)
+    m = modules.get("keyformer")
+    t = dict(Q=q, K=k, V=v, O=o, noise=n.float(), C_out=c)
+    m.forward(*[t[p] for p in m.TENSOR_PARAMS])
+    t["noise"] = n
+    args = [t[p] for p in m.TENSOR_PARAMS]
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        m.forward(*args)
+    for _ in range(3):
+        c.fill_(-1.0); o.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        check_outputs(q, k, v, o, [(0, 0), (0, 7)])
+        rows = torch.stack([((q[0, h].double() @ k[0, h // 4].double().t() * 128 ** -0.5 + n[0, h].double())
+                             .masked_fill(torch.ones(1000, 1000, dtype=torch.bool, device="cuda").triu(1), float("-inf"))).softmax(1).sum(0) for h in range(8)])
+        assert ((c[0] - rows).abs() <= 2.0 ** -11 * rows + 2e-5 * rows + 2.0 ** -24).all()
+
+
 def test_captured_module_and_where_the_rule_lies():
     from triton_amd import modules, ops
     # from 300 keys and some MB of noise; the workspace serves either type

@@ -380,8 +380,11 @@ bool f_key_scores_forward(Args a, Py_ssize_t n) {         // workspaces, scale |
     if (noise.given) add_noise(d, as4(noise.v, "noise"), num(a[3]));
     const at::Tensor rows = workspace(w, noise.given ? "lse_pert" : "lse", {q.s[0], q.s[1], q.s[2]}, c10::ScalarType::Float, q.dev);
     at::Tensor parts;
-    const int64_t need = noise.given ? trn_attn_key_scores_workspace_bytes(&d, noise.v.half() ? 2 : 3) : 0;
-    if (need) parts = workspace(w, "key_parts", {need}, c10::ScalarType::Byte, q.dev);
+    int64_t need = noise.given ? trn_attn_key_scores_workspace_bytes(&d, noise.v.half() ? 2 : 3) : 0;
+    if (need) {
+        parts = workspace(w, "key_parts", {need}, c10::ScalarType::Byte, q.dev, false, true);
+        if (!parts.defined()) need = 0;             // (captured with noise of another type than the eager call's: without)
+    }
     CALL(trn_attn_key_scores_f16, &d, q.p, k.p, v.p, o.p, noise.p(), noise.given && noise.v.half(), static_cast<float*>(rows.data_ptr()),
          c1.p, c2.p(), c1.half(), flag(a[4]), need ? parts.data_ptr() : nullptr, need, stream_of(q));
     return true;

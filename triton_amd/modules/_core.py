@@ -269,7 +269,9 @@ class KeyFormerAttention(FusedModule):
         lsep = self._workspace("lse_pert", (B, Hq, Sq), torch.float32, q.device)
         score, = _score_outputs(self, (C_out,), (B, Hq, Skv))
         need = ops.attention_key_scores_workspace_bytes(q, k, v, o, _scale(self.scale, D), self.causal, 2 if n4.dtype == torch.float16 else 3)
-        parts = self._workspace("key_parts", (need,), torch.uint8, q.device) if need else None
+        key = ("key_parts", (need,), torch.uint8, q.device)
+        # (a capture with noise of another type than the eager call's: without)
+        parts = self._workspace(*key) if need and not _capture_forbids(self._ws, *key) else None
         ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lsep, score, noise=n4, tau=self.tau, workspace=parts)
         _store_scores(C_out, score)
 
