@@ -266,8 +266,9 @@ int trn_attn_fwd_stats_half_f16(const trn_attn_desc* desc, const void* q, const 
  *               the statistics; with fewer bytes, but those of trn_attn_workspace_bytes(desc), over as many as these are for;
  *               with less than that, not at all.  Without noise it serves a chunk of more than 32 queries too, as
  *               trn_attn_chunk_workspace_bytes does without statistics; with noise a prompt, whose scores are then formed in
- *               one pass over the noise.  One that is not 256-byte aligned is not used (TRN_E_ALIGN where
- *               trn_attn_stats_workspace_bytes names a size that it has).
+ *               one pass over the noise (where one workgroup a head takes all of it, without a workspace too).  One that
+ *               is not 256-byte aligned is not used (TRN_E_ALIGN where trn_attn_stats_workspace_bytes names a size that
+ *               it has).
  */
 #define TRN_STATS_SPARE_ROWS 128        /* query rows past the last that the statistics kernels may ask for (as zeros) */
 int64_t trn_attn_key_scores_workspace_bytes(const trn_attn_desc* desc, int32_t with_noise);

@@ -25,12 +25,12 @@ def problem(B, Hq, Hkv, S, D, half, spare, first, seed=1):
     return q, k, v, n
 
 
-def scores(q, k, v, n, tau, with_workspace=True):
+def scores(q, k, v, n, tau, with_workspace=True, one_workgroup=False, out=torch.float32):
     from triton_amd import ops
     B, H, S, D = q.shape
-    o, rows, c = torch.empty_like(q), torch.full((B, H, S), 9.0, device="cuda"), torch.full((B, H, S), -1.0, device="cuda")
-    need = ops.attention_key_scores_workspace_bytes(q, k, v, o, D ** -0.5, True, True)
-    assert need > 0
+    o, rows, c = torch.empty_like(q), torch.full((B, H, S), 9.0, device="cuda"), torch.full((B, H, S), -1.0, dtype=out, device="cuda")
+    need = ops.attention_key_scores_workspace_bytes(q, k, v, o, D ** -0.5, True, 2 if n.dtype == torch.half else 3)
+    assert (need == 0) == one_workgroup          # (one workgroup a head needs none)
     ws = torch.full((need,), 255, dtype=torch.uint8, device="cuda") if with_workspace else None      # (any contents: NaN here)
     ops.attention_key_scores(q, k, v, o, D ** -0.5, True, rows, c, noise=n, tau=tau, workspace=ws)
     torch.cuda.synchronize()
@@ -110,6 +110,46 @@ def test_one_pass_over_the_noise(B, Hq, Hkv, S, D, half, spare, first):
     o1, rows1, c1 = scores(q, k, v, n, tau, with_workspace=False)
     assert ((o1 - o).float().norm(dim=-1) <= 4e-3 * o.float().norm(dim=-1)).all()
     assert (c1 - c).norm() <= 1e-4 * c.norm() and (rows1 - rows).abs().max() < 1e-3
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half,one", [(6, 71, 1, 333, 64, False, True), (6, 71, 1, 633, 64, True, True), (8, 64, 8, 401, 128, False, True), (4, 64, 8, 1650, 64, True, True),
+                                                   (1, 71, 1, 333, 64, False, False), (1, 32, 8, 701, 128, True, False)])
+def test_one_workgroup_a_head_and_scores_in_half(B, Hq, Hkv, S, D, half, one):
+    """A head of one workgroup, which writes its column sums itself, and several, whose sums a second launch adds; as fp16 the
+    fp32 scores rounded once in both.  The row normalisers do not depend on how many there are: those of one batch entry alone, whose heads have several
+    workgroups, are the same bits (those of the two passes are not)."""
+    q, k, v, n = problem(B, Hq, Hkv, S, D, half, 1, 1, seed=9)
+    o, rows, c = scores(q, k, v, n, 1.5, with_workspace=not one, one_workgroup=one)
+    check(q, k, n, rows, c, 1.5, 2e-5, [(0, 0), (B - 1, Hq - 1), (B // 2, Hq // 2)])
+    check_outputs(q, k, v, o, [(0, 0), (B - 1, Hq - 1)])
+    _, rows16, c16 = scores(q, k, v, n, 1.5, with_workspace=not one, one_workgroup=one, out=torch.half)
+    assert torch.equal(c16, c.half()) and torch.equal(rows16, rows)
+    if one:
+        _, rows1, c1 = scores(q[-1:], k[-1:], v[-1:], n[-1:], 1.5)
+        assert torch.equal(rows1, rows[-1:]) and (c1 - c[-1:]).abs().max() <= 1e-5 * c.abs().max()
+
+
+def test_workspaces_of_many_lengths():
+    """Prompts of every length in an instance share the workspaces of the single pass: powers of two, so that all of them hold at
+    most twice the largest of them, and none where a head has one workgroup."""
+    from triton_amd import modules, ops
+    m, most = modules.get("keyformer"), 0
+    q = torch.randn(1, 8, 2400, 128, device="cuda").half()
+    kv = torch.randn(1, 2, 2400, 128, device="cuda").half()
+    n = torch.randn(8 * 2400 * 2400, device="cuda").half()
+    for S in list(range(801, 2400, 97)):
+        t = dict(Q=q[:, :, :S].contiguous(), K=kv[:, :, :S].contiguous(), V=kv[:, :, :S].contiguous(), O=torch.empty(1, 8, S, 128, dtype=torch.half, device="cuda"),
+                 noise=n[: 8 * S * S].view(1, 8, S, S), C_out=torch.empty(1, 8, S, dtype=torch.half, device="cuda"))
+        m.forward(*[t[p] for p in m.TENSOR_PARAMS])
+        most = max(most, ops.attention_key_scores_workspace_bytes(t["Q"], t["K"], t["V"], t["O"], 0.1, True, 2))
+    sizes = [w.numel() for key, w in m._ws.items() if key[0] == "key_parts"]
+    assert most > 1 << 20 and sizes and all(x & (x - 1) == 0 for x in sizes) and sum(sizes) <= 4 * most
+    m = modules.get("keyformer")
+    t = dict(Q=torch.randn(6, 71, 333, 64, device="cuda").half(), K=torch.randn(6, 1, 333, 64, device="cuda").half(), V=torch.randn(6, 1, 333, 64, device="cuda").half(),
+             O=torch.empty(6, 71, 333, 64, dtype=torch.half, device="cuda"), noise=torch.randn(6, 71, 333, 333, device="cuda"), C_out=torch.empty(6, 71, 333, device="cuda"))
+    m.forward(*[t[p] for p in m.TENSOR_PARAMS])
+    torch.cuda.synchronize()
+    assert not [key for key in m._ws if key[0] == "key_parts"]
 
 
 @pytest.mark.parametrize("S,D,Hq", [(1100, 128, 32), (2200, 64, 8), (1090, 64, 71)])

@@ -139,7 +139,7 @@ int attn_colstats(const trn_attn_desc* d, const void* q, const void* k, const fl
 bool noise_streams(const trn_attn_desc* d, const void* noise, bool n16);
 
 // KeyFormer's row normalisers and key scores in one pass over the noise (attn_noise_strips.hip): in how many workgroups per head
-// (0: this problem does not suit it), and with how much workspace, of any contents, for noise of either type (1), fp16 (2), fp32 (3).
+// (0: this problem does not suit it), and with how much workspace, of any contents, for noise of either type (1), fp16 (2), fp32 (3); none with one workgroup a head.
 int noise_strip_slots(const trn_attn_desc* d, bool n16);
 int64_t noise_strips_workspace_bytes(const trn_attn_desc* d, int with_noise);
 hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void* k, const void* noise, bool n16, float* lse, void* out,

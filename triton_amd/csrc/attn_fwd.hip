@@ -814,7 +814,8 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
         return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, nullptr, 0, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, mean_std != 0);
     // The scores of a prompt in one pass over the noise, and its attention, which needs none, on the kernels without it (the queries
     // as given, as the forward with noise takes them)
-    if (n && s1 && !s2 && workspace && noise_strip_slots(d, n16) > 0 && workspace_bytes >= noise_strips_workspace_bytes(d, n16 ? 2 : 3)) {
+    const int64_t parts = n && s1 && !s2 && noise_strip_slots(d, n16) > 0 ? noise_strips_workspace_bytes(d, n16 ? 2 : 3) : -1;
+    if (parts == 0 || (parts > 0 && workspace && workspace_bytes >= parts)) {
         st = attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream, nullptr, false, false, false, false,
                           nullptr, 0.f, false, true);
         if (st != TRN_OK) return st;

@@ -519,7 +519,7 @@ int noise_strip_slots(const trn_attn_desc* d, bool n16) {
 int64_t noise_strips_workspace_bytes(const trn_attn_desc* d, int with_noise) {
     const int n32 = with_noise == 2 ? 0 : noise_strip_slots(d, false), n16 = with_noise == 3 ? 0 : noise_strip_slots(d, true);
     const int64_t n = n32 > 0 ? n32 : n16;       // (the same number where both suit)
-    return n * d->batch * d->n_q_heads * d->seq_kv * 4;
+    return n <= 1 ? 0 : n * d->batch * d->n_q_heads * d->seq_kv * 4;         // (one workgroup a head writes its sums itself)
 }
 
 template <int D, int NW>

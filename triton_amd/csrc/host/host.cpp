@@ -167,6 +167,13 @@ at::Tensor workspace(Workspaces* w, const char* name, at::IntArrayRef shape, c10
     return r;
 }
 Workspaces* ws_arg(PyObject* o);
+// Size at which a workspace of so many bytes is kept: the next power of two from 1 MB on, so that lengths share one (by exact
+// size each length met would keep its own; all of them together are at most twice the largest).
+int64_t kept_bytes(int64_t need) {
+    int64_t n = (int64_t)1 << 20;
+    while (n < need) n <<= 1;
+    return n;
+}
 
 // ---------------------------------------------------------------------------------------------- operators
 void rmsnorm_call(const View& x, const OptView& gamma, const View& y, double eps) {
@@ -382,6 +389,7 @@ bool f_key_scores_forward(Args a, Py_ssize_t n) {         // workspaces, scale |
     at::Tensor parts;
     int64_t need = noise.given ? trn_attn_key_scores_workspace_bytes(&d, noise.v.half() ? 2 : 3) : 0;
     if (need) {
+        need = kept_bytes(need);
         parts = workspace(w, "key_parts", {need}, c10::ScalarType::Byte, q.dev, false, true);
         if (!parts.defined()) need = 0;             // (captured with noise of another type than the eager call's: without)
     }
@@ -454,7 +462,7 @@ bool f_decode_forward(Args a, Py_ssize_t n) {
     if (need) split = workspace(w, "attn_ws", {need}, c10::ScalarType::Byte, X.dev, true);
     else if ((need = c1.given ? trn_attn_key_scores_workspace_bytes(&d, noise.given) : trn_attn_chunk_workspace_bytes(&d)) > 0) {
         // one for chunks and caches of every length: by exact size each length would keep its own
-        need = std::max<int64_t>(need, TRN_ATTN_CHUNK_WORKSPACE_MAX(D));
+        need = need <= TRN_ATTN_CHUNK_WORKSPACE_MAX(D) ? TRN_ATTN_CHUNK_WORKSPACE_MAX(D) : kept_bytes(need);
         split = workspace(w, "attn_shares", {need}, c10::ScalarType::Byte, X.dev, false, true);
         if (!split.defined()) need = 0;             // (captured, the cache grown long since the eager call: without)
     }

@@ -40,6 +40,11 @@ def _capture_forbids(ws, name: str, shape, dtype, device) -> bool:
     return (name, tuple(shape), dtype, str(device)) not in ws and torch.cuda.is_current_stream_capturing()
 
 
+def _kept_bytes(need: int) -> int:
+    """Size at which a workspace of `need` bytes is kept: the next power of two from 1 MB on, so that lengths share one."""
+    return max(1 << 20, 1 << (need - 1).bit_length()) if need else 0
+
+
 def _workspace_in(ws: Dict[Tuple, torch.Tensor], owner: str, name: str, shape, dtype, device) -> torch.Tensor:
     key = (name, tuple(shape), dtype, str(device))
     t = ws.get(key)
@@ -250,8 +255,9 @@ class KeyFormerAttention(FusedModule):
     """Attention plus key scores C_out[h,j] = sum_i softmax_i((scale*QK^T + noise)/tau)[j]
     (ref_rms.py:171-176; reduced over queries as the generated kernel's C_out is,
     keyformer_llama_benchmark.py:79).  Two launches: forward (+ perturbed row normaliser),
-    then the column-owner pass; one launch for at most 32 queries or 128 queries and keys; on prompts with
-    much noise the plain attention and then normalisers and scores in one pass over it."""
+    then the column-owner pass; one launch for at most 32 queries (two on a long cache, whose keys are split
+    over workgroups) or 128 queries and keys; on prompts with much noise the attention without it and then
+    normalisers and scores in one pass over it."""
     TENSOR_PARAMS = ["C_out", "K", "O", "Q", "V", "noise"]
 
     def __init__(self, scale: Optional[float] = None, causal: bool = True, tau: float = 1.0):
@@ -269,7 +275,7 @@ class KeyFormerAttention(FusedModule):
         lsep = self._workspace("lse_pert", (B, Hq, Sq), torch.float32, q.device)
         score, = _score_outputs(self, (C_out,), (B, Hq, Skv))
         need = ops.attention_key_scores_workspace_bytes(q, k, v, o, _scale(self.scale, D), self.causal, 2 if n4.dtype == torch.float16 else 3)
-        key = ("key_parts", (need,), torch.uint8, q.device)
+        key = ("key_parts", (_kept_bytes(need),), torch.uint8, q.device)
         # (a capture with noise of another type than the eager call's: without)
         parts = self._workspace(*key) if need and not _capture_forbids(self._ws, *key) else None
         ops.attention_key_scores(q, k, v, o, _scale(self.scale, D), self.causal, lsep, score, noise=n4, tau=self.tau, workspace=parts)
@@ -388,7 +394,8 @@ class _DecodeAppend(FusedModule):
         own); None when the library would not use one, or a capture finds it missing."""
         if not nbytes:
             return None
-        key = ("attn_shares", (max(nbytes, ops.chunk_workspace_max(head_dim)),), torch.uint8, device)
+        most = ops.chunk_workspace_max(head_dim)
+        key = ("attn_shares", (most if nbytes <= most else _kept_bytes(nbytes),), torch.uint8, device)
         return None if _capture_forbids(self._ws, *key) else self._workspace(*key)
 
     def _split_ws(self, nbytes: int, device):
