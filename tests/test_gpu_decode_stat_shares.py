@@ -146,3 +146,27 @@ def test_a_misaligned_workspace_is_refused_where_it_was():
     rows, x = torch.zeros(1, 8, 8, device="cuda"), torch.zeros(1, 8, 8192, device="cuda")
     with pytest.raises(Exception, match="ALIGN"):
         ops.attention_key_scores(q, k, k, torch.empty_like(q), 0.1, True, rows, x, workspace=torch.zeros(need + 16, dtype=torch.uint8, device="cuda")[16:])
+
+
+@pytest.mark.parametrize("general", [False, True])
+@pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", CASES[:4] + [(1, 16, 16, 64, 20, 2100)])
+def test_the_keyformer_module_shares_out_the_keys_of_few_queries(B, H, Hkv, D, Sq, Skv, general):
+    """A few queries on a long cache through the module: split over workgroups as by the call that is given a workspace -- the same
+    bits -- with one of its own.  general: scores that the kernels do not write themselves (the path in Python)."""
+    from triton_amd import modules, ops
+    g = torch.Generator(device="cuda").manual_seed(Skv + Sq)
+    q, k, v = (torch.randn(B, h, s, D, generator=g, device="cuda").half() for h, s in ((H, Sq), (Hkv, Skv), (Hkv, Skv)))
+    noise = -torch.log(torch.empty(B, H, Sq, Skv, device="cuda").exponential_(generator=g))
+    c = torch.empty(B, H, 2 * Skv, device="cuda")[..., ::2] if general else torch.empty(B, H, Skv, device="cuda")
+    m, o = modules.get("keyformer", tau=1.5), torch.empty_like(q)
+    t = dict(Q=q, K=k, V=v, O=o, noise=noise, C_out=c)
+    m.forward(*[t[p] for p in m.TENSOR_PARAMS])
+    outs = []
+    need = ops.attention_key_scores_workspace_bytes(q, k, v, o, D ** -0.5, True, True)
+    for ws in (torch.empty(need, dtype=torch.uint8, device="cuda"), None):
+        rows, x, ow = torch.empty(B, H, Sq, device="cuda"), torch.empty(B, H, Skv, device="cuda"), torch.empty_like(q)
+        ops.attention_key_scores(q, k, v, ow, D ** -0.5, True, rows, x, noise=noise, tau=1.5, workspace=ws)
+        outs.append((ow, x))
+    torch.cuda.synchronize()
+    assert torch.equal(o, outs[0][0]) and torch.equal(c, outs[0][1]) and any(key[0] == "key_parts" for key in m._ws)
+    assert (c - outs[1][1]).abs().max() <= 1e-4 * c.abs().max()
