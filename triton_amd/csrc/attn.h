@@ -38,13 +38,12 @@ struct AttnArgs {
 //   the losses: 300 tokens (2.5 MB) 45.5 / 45.5; 32.4 / 37.4, 777 (6 MB) 56 / 56; 51.7 / 55.1, and an addition behind 2048 (17 MB) 51.1 / 52.3,
 //     2800 (23 MB) 78.3 / 78.9 (26 MB and more the same); 71 heads of 64: 400 (4 MB) 45.2 / 49.7; 40.6 / 51.7, 3 x 1000 (27 MB) 159 / 163.4; 277.5 / 277.8
 inline bool outputs_stream(int64_t rows, int head_dim) { return head_dim == 128 && rows * head_dim * 2 >= (int64_t)24 << 20; }
-// 16 bytes of the output
-__device__ __forceinline__ void store_out(half_t* p, uint4_t v, int past) {
+template <class V> __device__ __forceinline__ void store_out(void* p, V v, int past) {
     if (past) {
         asm volatile("" ::: "memory");      // (the two stores would be merged into one without the hint)
-        __builtin_nontemporal_store(v, reinterpret_cast<uint4_t*>(p));
+        __builtin_nontemporal_store(v, static_cast<V*>(p));
         asm volatile("" ::: "memory");
-    } else *reinterpret_cast<uint4_t*>(p) = v;
+    } else *static_cast<V*>(p) = v;
 }
 
 // fp16 noise as the kernels fetch it.  Its rows may start at any element (the reference's [.., M, P + M] tensors have any

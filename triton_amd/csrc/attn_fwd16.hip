@@ -485,7 +485,8 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     // queries on 4.1 k keys 25.2 / 19.4, 128 on 3.2 k 22.7 / 18.3, 40 on 3.1 k 17.5 / 14.8, 128 on 8.1 k 38.5 / 33.5, 50 on 16 k
     // 52.2 / 50.4; 8 of 128: 100 on 8.1 k 16.6 / 16.4, 128 on 16 k 23.7 / 23.1; 71 of 64: 40 on 6 k 26.7 / 24.2, 64 on 6 k 27.4 / 24.7,
     // 128 on 3.1 k 20.0 / 17.0, 100 on 2.7 k 17.8 / 15.7; 16 of 64, three tiles a group at most: 60 on 4.3 k 9.8 / 9.9, 5.1 k 9.5 /
-    // 10.1; 12 k 13.7 / 13.7.  (Of those, writing the partial results past the caches: 128 on 8.1 k 37.4 / 33.2, 100 on 4.1 k 20.4 / 19.3.)
+    // 10.1; 12 k 13.7 / 13.7.  With the merge, K and V out of the caches: 100 on 4.1 k 26.4 / 25.2, 128 on 8.1 k 32.0 / 32.3, 8 heads of 128, 100 on
+    // 3.4 k 19.4 / 17.8, 71 of 64, 64 on 6 k 32.4 / 29.9, 100 on 2.7 k 22.1 / 21.5, 16 of 64, 100 on 4.1 k 16.3 / 15.6, 40 on 4.1 k 14.0 / 14.4.
     auto share_handover = [&](int blk, half_t* Kf, half_t* Vf) __attribute__((always_inline)) {
         constexpr int kBehind = 2 * NI;      // V of blk and K of blk + 2 have landed: behind them only two hand-overs' requests
         __builtin_amdgcn_sched_barrier(0);
@@ -616,14 +617,19 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
             }
         if constexpr (SHARE) {
             // this share's {O unnormalised, m, l} per query, fp32: rows of D floats, then the pairs of all rows
+            // (3 MB and more of them past the caches, as far as the L2s would be written back at the end of the launch: with the merge,
+            // us, through / past, K and V out of the caches: 32 heads of 128: 100 queries on 4.1 k keys (13 MB) 26.8 / 25.4, 128 on 3.2 k 28.0 /
+            // 26.1, 40 on 3.1 k (5.3) 19.8 / 19.1; 16 of 64: 100 on 4.1 k 16.9 / 15.8, 60 on 4.3 k (4.1) 14.85 / 14.55, 50 on 4.2 k (3.4) 14.41 /
+            // 14.31, 40 on 4.1 k (2.7) 14.34 / 14.56; 8 of 128: 40 on 3.1 k (2.7) 15.64 / 15.94; 71 of 64: 64 on 6 k (3.6) 29.9 / 29.9, 40 on 6 k (2.2)
+            // 29.1 / 29.4)
             const int64_t rows = (int64_t)BH * a.n_split * a.Sq, row0 = ((int64_t)(b * a.Hq + head) * a.n_split + share) * a.Sq;
+            const int past = rows * D * 4 >= (int64_t)3 << 20 ? 1 : 0;
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb) {
                 if (qrow[qb] >= a.Sq) continue;
                 float* po = a.ws + (row0 + qrow[qb]) * D + grp * (D / 2) + 4 * g4;
 #pragma unroll
-                for (int i = 0; i < NH; ++i)       // (16 MB in all that this launch does not read: past the caches)
-                    __builtin_nontemporal_store(oacc[i][qb], reinterpret_cast<float4_t*>(po + 16 * i));
+                for (int i = 0; i < NH; ++i) store_out(po + 16 * i, oacc[i][qb], past);
                 if (g4 == 0 && grp == 0) *reinterpret_cast<float2_t*>(a.ws + rows * D + (row0 + qrow[qb]) * 2) = float2_t{l[qb] > 0.f ? m[qb] : -INFINITY, l[qb]};
             }
             return;
