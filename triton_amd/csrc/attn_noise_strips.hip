@@ -40,13 +40,15 @@ constexpr int strip_keys(int waves, int head_dim) { return waves == 8 ? 4864 : h
 #if defined(__HIP_DEVICE_COMPILE__)
 // Four of a wave's global -> LDS loads of BYTES a lane, LSTEP bytes of LDS and `step` bytes of memory from each to the next:
 // lane l's land at lds + 4 l (16 l), offsets past the range as zeros.  lds and so end up where a fifth would go.
+// (m0, which both functions write, is a reserved register that a clobber list does not take: this kernel has no other user of it --
+// no global -> LDS load by a builtin, no message, no indexed register.  so is written before the last inputs are read.)
 template <int BYTES, bool NT, int LSTEP>
 __device__ __forceinline__ void request4(uint4_t rs, uint32_t& lds, int vo0, int vo1, int vo2, int vo3, int& so, int step) {
 #define TRN_NEXT "s_add_u32 m0, m0, %8\n\ts_add_u32 %0, %0, %7\n\t"
 #define TRN_REQ(op_, mod_)                                                                                                      \
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\t" op_ " %2, %6, %0 offen " mod_ "\n\t" TRN_NEXT op_ " %3, %6, %0 offen " mod_ "\n\t" TRN_NEXT    \
                  op_ " %4, %6, %0 offen " mod_ "\n\t" TRN_NEXT op_ " %5, %6, %0 offen " mod_ "\n\ts_add_u32 %0, %0, %7"         \
-                 : "+s"(so) : "s"(lds), "v"(vo0), "v"(vo1), "v"(vo2), "v"(vo3), "s"(rs), "s"(step), "n"(LSTEP) : "memory", "scc")
+                 : "+&s"(so) : "s"(lds), "v"(vo0), "v"(vo1), "v"(vo2), "v"(vo3), "s"(rs), "s"(step), "n"(LSTEP) : "memory", "scc")
     if constexpr (BYTES == 16) { if constexpr (NT) TRN_REQ("buffer_load_dwordx4", "nt lds"); else TRN_REQ("buffer_load_dwordx4", "lds"); }
     else if constexpr (BYTES == 4) TRN_REQ("buffer_load_dword", "lds");
     else TRN_REQ("buffer_load_ushort", "lds");
