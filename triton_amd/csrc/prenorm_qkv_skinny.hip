@@ -43,6 +43,7 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_skinny_kernel(const GemmAr
     const int pi = panel >= a.p[2].tile0 ? 2 : (panel >= a.p[1].tile0 ? 1 : 0);
     const ProjOut P = a.p[pi];
     const int n0 = (panel - P.tile0) * SN;
+    if (SN == 32 && n0 >= P.n) return;               // (the place between an odd number of panels and the next matrix)
     const int nkt = (a.K + SK - 1) / SK;
     constexpr int kOut = 0x7ffffff0;                 // a byte offset past every buffer: the load returns zeros
 
@@ -198,7 +199,13 @@ __global__ __launch_bounds__(512, 2) void prenorm_qkv_skinny_kernel(const GemmAr
 template <int SN, bool NT>
 static int launch_panels(GemmArgs a, hipStream_t stream) {
     int t0 = 0;
-    for (int i = 0; i < 3; ++i) { a.p[i].tile0 = t0; t0 += (a.p[i].n + SN - 1) / SN; }
+    for (int i = 0; i < 3; ++i) {
+        // (a matrix begins with a whole pair, which one XCD has.  us, 16 tokens, weights cold, one behind the other / so: two matrices 4096 deep of
+        // 4000 columns whose rows begin on whole lines 23.9 / 23.0, of 2080 17.5 / 17.15; rows at odd half lines and 1056 and fewer columns the same)
+        if (SN == 32 && a.p[i].n > 0) t0 = (t0 + 1) & ~1;
+        a.p[i].tile0 = t0;
+        t0 += (a.p[i].n + SN - 1) / SN;
+    }
     a.n_panels = t0;
     const dim3 g((unsigned)(SN == 64 ? t0 : (t0 + 15) / 16 * 16)), t(512);
     const int norm = !a.norm ? 0 : a.gamma ? 2 : 1;
