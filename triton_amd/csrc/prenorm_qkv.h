@@ -25,11 +25,18 @@ struct GemmArgs {
 __device__ __forceinline__ int wswz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
 // Whether weights that one workgroup each reads once are requested past the caches (the non-temporal hint): 64 MB and more,
-// of which the last-level cache (256 MB) keeps nothing until the same layer comes round again but would evict what it holds
-// for each line.  us, without / with, weights and cache cold (three sets in turn): whole decode step, 16 tokens on 1024, 4096 ->
-// 12288 (101 MB) 35.3 / 32.9, 4544 -> 13632 31.7 / 28.8, one token 33.1 / 30.0; the projection of 100 tokens 36.4 / 35.0.  The other
-// side: one layer's step again and again, its weights then out of that cache, 27.2 / 32.3 and 26.7 / 28.1; and weights of 6 MB,
-// of which the caches hold many layers, 11.0 / 13.0.
+// of which the last-level cache (256 MB) holds four layers at most and keeps nothing until the same layer comes round again, but would
+// evict what it holds for each line.  A trade: a model whose layers come in turn gains, one layer's step again and again on the same
+// weights, which then come from HBM each time, loses.  us, whole decode steps, without / with, weights and cache cold (1.4 GB of layers
+// in turn); one layer repeated:
+//   4096 -> 12288 (96 MB): 1 token on 1024 34.9 / 31.7; 27.2 / 30.0, 16 37.6 / 34.6; 28.3 / 34.0, 32 on 2048 45.0 / 44.1; 33.8 / 40.2, 48 on 1024
+//     42.3 / 40.9; 32.6 / 39.2, 64 on 2048 50.0 / 49.3; 38.0 / 47.2, 100 on 4000 67.2 / 67.0; 49.6 / 60.8, 128 on 1024 53.5 / 53.0; 41.0 / 51.0
+//   4544 -> 13632 (118 MB): 1 33.9 / 30.2; 27.1 / 28.7, 16 34.6 / 31.0; 27.6 / 30.1, 32 39.8 / 38.9; 31.2 / 34.2, 48 39.0 / 36.1; 30.7 / 35.4, 64 45.7 /
+//     44.8; 35.7 / 41.4, 128 58.7 / 56.0; 43.5 / 54.7
+//   3584 -> 10752 (73 MB): 1 31.8 / 29.2; 23.8 / 27.1, 16 33.5 / 31.7; 24.9 / 30.4, 64 46.7 / 46.1; 34.0 / 43.0, 128 49.8 / 49.0; 35.3 / 47.0
+//   5120 -> 15360 (150 MB): 1 46.6 / 42.3; 35.9 / 40.6, 16 48.4 / 44.7; 36.9 / 43.7, 48 55.0 / 52.2; 40.5 / 50.8, 128 71.0 / 68.7; 51.2 / 67.3
+// Below the line a projection alone would go the same way (2816 -> 8448, 45 MB, 16 tokens 15.9 / 15.1; 10.3 / 14.1, 3328 -> 9984, 63 MB 18.5 /
+// 17.9; 12.9 / 16.9), but the cache then holds so many layers that a small model's step finds them there.
 inline bool weights_stream(const GemmArgs& a) {
     int64_t columns = 0;
     for (int i = 0; i < 3; ++i) columns += a.p[i].n;
