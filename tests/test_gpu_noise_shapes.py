@@ -39,9 +39,20 @@ def noise_tensor(B, H, S, half, spare, first, seed):
 
 
 def run(q, k, v, noise, scale, tau):
-    from triton_amd import modules
+    """The two launches by themselves: without a workspace the single pass over the noise is not taken (but where a head has one
+    workgroup, which takes some 240 heads)."""
+    from triton_amd import ops
+    assert q.shape[0] * q.shape[1] <= 128
     c = torch.full(q.shape[:3], -1.0, dtype=torch.float32, device="cuda")
     o = torch.full_like(q, 7.0)
+    ops.attention_key_scores(q, k, v, o, scale, True, torch.empty_like(c), c, noise=noise, tau=tau)
+    torch.cuda.synchronize()
+    return o, c
+
+
+def through_the_module(q, k, v, noise, tau):
+    from triton_amd import modules
+    c, o = torch.full(q.shape[:3], -1.0, dtype=torch.float32, device="cuda"), torch.full_like(q, 7.0)
     m = modules.get("keyformer", tau=tau)
     t = dict(Q=q, K=k, V=v, O=o, noise=noise, C_out=c)
     m.forward(*[t[p] for p in m.TENSOR_PARAMS])
@@ -60,6 +71,8 @@ def test_keyformer_in_every_shape_and_row_alignment(B, Hq, Hkv, S, D, half, spar
     launched = ops.attention_kernel_name(q, k, v, torch.empty_like(q), scale, True, half or noise)
     assert launched.rsplit(",", 1)[0] == "trn::" + name.rsplit(",", 1)[0] and (half or launched == "trn::" + name)
     o, c = run(q, k, v, noise, scale, tau)
+    if ops.attention_key_scores_workspace_bytes(q, k, v, o, scale, True, 2 if half else 3) == 0:       # (elsewhere the module takes the single pass)
+        assert all(torch.equal(x, y) for x, y in zip((o, c), through_the_module(q, k, v, noise, tau)))
     keep = torch.ones(S, S, dtype=torch.bool, device="cuda").tril()
     for b in range(B):
         for h in range(Hq):
