@@ -7,7 +7,7 @@
 // HBM: a 128 MB buffer read over and over 7.0 - 7.4 TB/s, 2 GB 6.3 - 7.1).  Here a workgroup takes 32 queries at a time and keeps their
 // exponentials in registers, 32 x 2048 of them in fp32 -- half of a CU's register file --, until the rows are summed up; the
 // scores then follow without another look at the noise.  Only what a row has beyond 2048 keys is read, and multiplied, again.
-// The attention itself, which does not depend on the noise, runs on the plain kernel of attn_fwd16.hip.
+// The attention itself, which does not depend on the noise, runs on the kernels of attn_fwd16.hip with the queries as given.
 //
 // Eight waves take a strip's 32-key blocks in turn, each through a private part of LDS (K one block ahead, noise two), so that
 // the walk has no barrier.  S[query][key], a lane one key and 16 of the 32 queries: the scores' sums over the queries are then
@@ -16,8 +16,8 @@
 //
 // What bounds it: a wave's block is a chain -- K and noise out of LDS, eight MFMAs that wait for each other, the exponentials --
 // that two waves a SIMD overlap only in part, and 32 to 64 KB of noise in flight a CU.  71 heads of 64, 1536 keys, fp32: 79 us for
-// 0.37 GB (4.7 TB/s; 59 with the noise in the caches, 51 without its and K's requests at all); 32 heads of 128, 2048: 80 us, where
-// the forward's noise and the statistics took 121 beside the attention's 40.
+// 0.37 GB (4.7 TB/s; 59 with the noise in the caches, 51 without its and K's requests at all); 32 heads of 128, 2048: 83 us, where
+// the forward's noise and the statistics took 121 beside the attention's 42.
 //
 // All requests are global -> LDS loads issued as inline assembly and counted by hand: a wave's requests run ahead over the end
 // of a strip into the next, and the compiler, which cannot see which of them a read depends on, would wait for all.

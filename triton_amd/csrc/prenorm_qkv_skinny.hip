@@ -227,8 +227,10 @@ static int launch_panels(GemmArgs a, hipStream_t stream) {
 // of its waves ask, so the time of few panels is their bytes per CU (X's among them).  The two panels of a 128-byte line go to
 // one XCD, whose L2 then has the line for both; dealt out singly each line is fetched from HBM twice (4096 deep, 1056 columns,
 // 16 tokens, with a second product of 32: 12.6 us in panels of 64, 15.5 of 32 dealt out singly, 9.5 so).  us, 64 / 32 columns, 16
-// tokens: 1024 deep, 576 columns (and a second product) 8.0 / 6.7; 2048, 2112 9.6 / 7.7; 4096, 4160 16.2 / 14.9; 4096, 8192
-// 15.6 / 14.9 (the last with 128 panels of 64); but 4096, 12288 (192) 24.4 / 35.6, when the panels no longer run all at once.
+// tokens, weights cold, launches in a graph: 1024 deep, 512 + 64 columns 5.5 / 4.8; 2048, 2080 + 2080 12.1 / 9.65; 4096, 4000 + 64 20.5 /
+// 15.5, 4096 + 4096 25.2 / 22.9 (the last with 128 panels of 64); whole LoRA of 1024 x 512, rank 64, which is two launches, 9.3 / 8.4, and
+// called one by one, where the host sets the pace as well, 10.1 / 8.2 to 9.7; but 4096, 12288 (192) 24.4 / 35.6, when the panels no longer
+// run all at once.
 int launch_prenorm_qkv_skinny(GemmArgs a, hipStream_t stream) {
     int panels = 0;
     for (int i = 0; i < 3; ++i) panels += (a.p[i].n + 63) / 64;
