@@ -31,13 +31,15 @@ struct AttnArgs {
 };
 
 // Whether a launch of so many outputs stores them past the caches.  What it leaves dirty in the L2s is written back before it ends, on
-// top of the launch; but the projection behind an attention reads what the caches still hold.  us, through the caches / past them:
-//   the launch alone: 32 heads of 128: 4 x 777 tokens (25 MB) 36.1 / 33.1, 8 x 500 34.3 / 30.4, 4096 122.2 / 117.7, 2 x 2048 74.7 / 67.7
-//   and a projection to the same width behind it, by the library's product; by ours: 4 x 777 133.8 / 132.8; 152.1 / 151.7, 12 x 260 (26 MB)
-//     125.9 / 127.0; 143.8 / 143.6, 8 x 500 (33 MB) 144.1 / 142.5; 167.4 / 165.0, 4 x 1024 158.8 / 158.4; 183.3 / 181.5, 4096 233.6 / 233.8; 258.2 / 258.0
-//   the losses: 300 tokens (2.5 MB) 45.5 / 45.5; 32.4 / 37.4, 777 (6 MB) 56 / 56; 51.7 / 55.1, and an addition behind 2048 (17 MB) 51.1 / 52.3,
-//     2800 (23 MB) 78.3 / 78.9 (26 MB and more the same); 71 heads of 64: 400 (4 MB) 45.2 / 49.7; 40.6 / 51.7, 3 x 1000 (27 MB) 159 / 163.4; 277.5 / 277.8
-inline bool outputs_stream(int64_t rows, int head_dim) { return head_dim == 128 && rows * head_dim * 2 >= (int64_t)24 << 20; }
+// top of the launch; but the output projection behind an attention reads what the caches still hold.  us, through the caches / past them:
+//   the launch alone: 32 heads of 128: 4 x 777 tokens (25 MB) 36.1 / 33.1, 8 x 500 34.3 / 30.4, 4096 122.2 / 117.7; 71 of 64, 2048 (19 MB) 46.0 / 45.6
+//   projection of Q, K, V, attention, output projection by the library's product; by ours (runs of one side differ by 1 %):
+//     small ones lose: 32 heads of 128, 300 tokens (2.5 MB) 82.3 / 82.3; 67.0 / 70.5, 777 (6 MB) 127.2 / 127.1; 120.7 / 122.8; 71 of 64, 400 (4 MB) 81.8 / 83.9;
+//       72.0 / 83.8; 16 of 64, 1000 (2 MB) 37.2 / 39.6; 35.5 / 36.0
+//     from 8 MB on they are the same: 1442 (12 MB) 173.8 / 173.7; 189.0 / 187.9, 2048 (17 MB) 219.7 / 221.9; 241.2 / 242.1; 71 of 64, 1000 (9 MB) 149.6 / 150.9;
+//       172.9 / 171.8, 2048 262.0 / 261.2; 267.0 / 263.3, 4 x 777 396.4 / 394.2; 508.3 / 507.0; 16 of 64, 8 x 1000 (16 MB) 121.3 / 121.2; 130.8 / 129.6; with
+//       KeyFormer's scores, fp32 noise, 2048 311.9 / 311.8; 330.5 / 329.9, 71 of 64, 1442 289.0 / 287.5; 295.9 / 295.9
+inline bool outputs_stream(int64_t rows, int head_dim) { return rows * head_dim * 2 >= (int64_t)8 << 20; }
 template <class V> __device__ __forceinline__ void store_out(void* p, V v, int past) {
     if (past) {
         asm volatile("" ::: "memory");      // (the two stores would be merged into one without the hint)
