@@ -168,6 +168,21 @@ def test_references_that_rise_and_rows_without_noise(S, D, Hq):
     check(q, k, n, rows, c, 1.0, 4e-4, [(0, h) for h in range(5)], 1000.0)
 
 
+@pytest.mark.parametrize("S,D,Hq,half,mask", [(1100, 128, 32, False, -1e4), (1100, 64, 71, False, -1e9), (2200, 64, 8, False, -1e9), (2200, 64, 8, False, -1e30), (2200, 64, 8, True, -65504.0),
+                                              (1030, 64, 71, True, -1e4), (3100, 64, 4, False, -1e6)])
+def test_keys_masked_by_finite_numbers(S, D, Hq, half, mask):
+    """Keys that later rows are kept from by a large negative number, whole blocks of them and the first that some waves see among
+    these, before the held keys (2200, 3100) and within: the scores of the others are as exact as without.  (A reference of -1e9
+    has a last place of 64.)"""
+    q, k, v, n = problem(1, Hq, Hq, S, D, half, 0, 0, seed=11)
+    for h, first in enumerate((0, 32, 100, 1)):
+        n[0, h, 400:, first:400] = mask
+    n[0, 3, 700:, 400:640] = mask
+    n[0, 3, 900::3, 128:800] = mask
+    o, rows, c = scores(q, k, v, n, 1.0)
+    check(q, k, n, rows, c, 1.0, 2e-5, [(0, h) for h in range(4)])
+
+
 @pytest.mark.parametrize("S,D,Hq,half", [(1100, 128, 32, False), (620, 64, 71, False), (2200, 64, 8, False), (1030, 64, 71, True)])
 def test_rows_without_a_normaliser(S, D, Hq, half):
     """A row without a finite score, or with +inf or NaN among them, has no probabilities: the scores of the keys that it sees are

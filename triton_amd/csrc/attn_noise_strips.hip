@@ -223,7 +223,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
             for (int e = 0; e < 4; ++e) v[4 * i + e] = t[e];
         }
     };
-    bool unseen = true;                          // some row's reference is still to come
+    bool unseen = true;                          // some row's reference is still to come, or lies far below zero
     float16_t held[kHeldBlocks];
 
     // z - ref of a block, the rows' references being in wr; requests the blocks ahead.  All that can be done before the scores
@@ -313,10 +313,14 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
 #pragma unroll
                     for (int r = 0; r < 16; ++r) held[i][r] *= f[r];
             mlane = mn;
-            unseen = __builtin_amdgcn_ballot_w64(mn == kNone) != 0;
             spread(mn == kNone ? 0.f : mn, f);
 #pragma unroll
             for (int r = 0; r < 16; ++r) e[r] -= f[r];
+            // A row whose reference lies far below zero -- its first keys masked by -1e4 or -1e9, say -- takes its next differences
+            // from zero again: relative to that reference an ordinary score would be rounded to the reference's last place, and lost.
+            const bool low = mn < -64.0f;
+            unseen = __builtin_amdgcn_ballot_w64(low) != 0;
+            if (low) Wr[wave * 32 + row_of(lane_now())] = 0.f;
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) e[r] = fast_exp2(e[r]);
