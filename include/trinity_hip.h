@@ -335,6 +335,19 @@ int trn_gate_f16(const void* c1, const void* c2, void* out, int64_t rows, int64_
                  int64_t ld1, int64_t ld2, int64_t ldo, int32_t kind, void* stream);
 
 /*
+ * LoRA (lora_benchmark.py:41-53), out = x w + (x a) b, and the gated MLP (gmlp_benchmark.py:53-64), out = gate(x w1) * (x w2), as a
+ * whole: one launch for at most 32 tokens on little weight, otherwise the launches of trn_linear_f16 and trn_gate_f16 in turn, whose
+ * operands, pitches, roundings and refusals these are.  d [tokens, r] and c2 [tokens, n] are scratch memory of any contents, which the single
+ * launch leaves alone; kind as in trn_gate_f16.
+ */
+int trn_lora_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, const void* w, int64_t n, int64_t ldw,
+                 const void* a, int64_t r, int64_t lda, const void* b, int64_t ldb, void* out, int64_t ldo,
+                 void* d, int64_t ldd, void* stream);
+int trn_gated_mlp_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, const void* w1, int64_t ldw1,
+                      const void* w2, int64_t ldw2, int64_t n, void* out, int64_t ldo, void* c2, int64_t ldc,
+                      int32_t kind, void* stream);
+
+/*
  * Measurement aid, no counterpart in the reference: the name (as a profiler's kernel trace prints it) of the kernel
  * instantiation that trn_attn_fwd_f16 launches for this problem -- decided by the same rules as the launch itself,
  * so that a benchmark can say which kernel its timing belongs to.  with_noise: as if a noise tensor were passed, with

@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(HERE, "libtrinity_hip.so")
 EXPORTS = (
     "trn_version", "trn_status_name", "trn_check_device", "trn_rmsnorm_f16",
     "trn_attn_fwd_f16", "trn_attn_colstats_f16", "trn_prenorm_qkv_f16", "trn_calibration_copy",
-    "trn_calibration_mfma", "trn_attn_workspace_bytes", "trn_attn_chunk_workspace_bytes", "trn_attn_fwd_ws_f16", "trn_linear_f16", "trn_gate_f16", "trn_attn_fwd_stats_f16",
+    "trn_calibration_mfma", "trn_attn_workspace_bytes", "trn_attn_chunk_workspace_bytes", "trn_attn_fwd_ws_f16", "trn_linear_f16", "trn_gate_f16", "trn_lora_f16", "trn_gated_mlp_f16", "trn_attn_fwd_stats_f16",
     "trn_attn_fwd_noalloc_f16", "trn_attn_fwd_kernel_name", "trn_attn_colmeanstd_f16", "trn_attn_fwd_probs_f16",
     "trn_attn_fwd_stats_half_f16", "trn_attn_fwd_stats_ws_f16", "trn_attn_stats_workspace_bytes",
     "trn_attn_key_scores_f16", "trn_attn_key_scores_workspace_bytes", "trn_attn_qknorm_f16", "trn_attn_qknorm_workspace_bytes",
@@ -89,6 +89,10 @@ def load() -> C.CDLL:
                                    C.POINTER(C.c_int64), C.POINTER(vp), C.POINTER(C.c_int64), C.POINTER(vp), vp]
     lib.trn_gate_f16.restype = C.c_int
     lib.trn_gate_f16.argtypes = [vp, vp, vp, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int32, vp]
+    lib.trn_lora_f16.restype = C.c_int
+    lib.trn_lora_f16.argtypes = [vp, i64, i64, i64, vp, i64, i64, vp, i64, i64, vp, i64, vp, i64, vp, i64, vp]
+    lib.trn_gated_mlp_f16.restype = C.c_int
+    lib.trn_gated_mlp_f16.argtypes = [vp, i64, i64, i64, vp, i64, vp, i64, i64, vp, i64, vp, i64, i32, vp]
     lib.trn_attn_workspace_bytes.restype = C.c_int64
     lib.trn_attn_workspace_bytes.argtypes = [C.POINTER(AttnDesc)]
     lib.trn_attn_chunk_workspace_bytes.restype = C.c_int64

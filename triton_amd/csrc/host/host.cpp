@@ -250,23 +250,6 @@ void prenorm_qkv_call(const View& x, const OptView& gamma, const View (&w)[3], c
          norm ? 1 : 0, stream_of(x));
 }
 
-void linear_call(const View& x, int k, const View* w, const View* o, const View* add) {
-    dev_half(x, "x");
-    NEED(x.dim == 2, "x: expected [tokens, hidden]");
-    const void *wp[3], *ap[3];
-    void* op[3];
-    int64_t n[3], lw[3], lo[3];
-    for (int i = 0; i < k; ++i) {
-        dev_half(w[i], "weights"); dev_half(o[i], "outs");
-        NEED(w[i].dim == 2 && w[i].s[0] == x.s[1], "weights[%d]: expected [hidden=%lld, n], got %s", i, (long long)x.s[1], w[i].shape().c_str());
-        NEED(o[i].dim == 2 && o[i].s[0] == x.s[0] && o[i].s[1] == w[i].s[1], "outs[%d]: expected [%lld, %lld], got %s", i,
-             (long long)x.s[0], (long long)w[i].s[1], o[i].shape().c_str());
-        wp[i] = w[i].p; op[i] = o[i].p; ap[i] = add ? add[i].p : nullptr;
-        n[i] = w[i].s[1]; lw[i] = w[i].st[0]; lo[i] = o[i].st[0];
-    }
-    CALL(trn_linear_f16, x.p, x.s[0], x.s[1], x.st[0], k, wp, n, lw, op, lo, ap, stream_of(x));
-}
-
 // ---------------------------------------------------------------------------------------------- functions
 using Args = PyObject* const*;
 
@@ -493,9 +476,10 @@ bool f_lora_forward(Args a, Py_ssize_t n) {               // workspaces, A, B, O
          "inconsistent shapes: X %s, W %s, A %s, B %s, O %s", X.shape().c_str(), W.shape().c_str(), A.shape().c_str(), B.shape().c_str(), O.shape().c_str());
     const at::Tensor d_ws = workspace(ws, "D", {M, R}, X.dt, X.dev);
     const View d = view_of(d_ws, "D");
-    const View w1[2] = {W, A}, o1[2] = {O, d};
-    linear_call(X, 2, w1, o1, nullptr);
-    linear_call(d, 1, &B, &O, &O);
+    dev_half(X, "x");
+    for (const View* t : {&W, &A, &B}) dev_half(*t, "weights");
+    dev_half(O, "outs"); dev_half(d, "outs");
+    CALL(trn_lora_f16, X.p, M, N, X.st[0], W.p, P, W.st[0], A.p, R, A.st[0], B.p, B.st[0], O.p, O.st[0], d.p, d.st[0], stream_of(X));
     return true;
 }
 
@@ -508,9 +492,9 @@ bool f_gmlp_forward(Args a, Py_ssize_t n) {               // workspaces, silu, O
          X.shape().c_str(), W1.shape().c_str(), W2.shape().c_str(), O.shape().c_str());
     const at::Tensor c2_ws = workspace(ws, "C2", {O.s[0], O.s[1]}, X.dt, X.dev);
     const View c2 = view_of(c2_ws, "C2");
-    const View w[2] = {W1, W2}, o[2] = {O, c2};
-    linear_call(X, 2, w, o, nullptr);                     // the first product lands in O and is gated in place
-    CALL(trn_gate_f16, O.p, c2.p, O.p, O.s[0], O.s[1], O.st[0], c2.st[0], O.st[0], flag(a[1]) ? 1 : 0, stream_of(X));
+    dev_half(X, "x"); dev_half(W1, "weights"); dev_half(W2, "weights"); dev_half(O, "outs"); dev_half(c2, "outs");
+    CALL(trn_gated_mlp_f16, X.p, X.s[0], X.s[1], X.st[0], W1.p, W1.st[0], W2.p, W2.st[0], W1.s[1], O.p, O.st[0], c2.p, c2.st[0],
+         flag(a[1]) ? 1 : 0, stream_of(X));
     return true;
 }
 

@@ -1,0 +1,253 @@
+// LoRA and the gated MLP of at most 32 tokens on little weight in one launch:
+//
+//     O = X W + (X A) B        O = gate(X W1) * (X W2)
+//
+// Two launches -- {O, D} = X {W, A} and O += D B; both products and their gate -- are two chains of memory latencies of 3 to 4 us
+// each, however small, and the second waits for the first.  Here a workgroup owns 32 columns of O and forms what they need besides: all
+// of D = X A, which its neighbours form as well (A and X come from L2), or the same columns of the second product.
+//
+// What bounds it: the latency of the first loads and, from some 100 KB a workgroup on, what a CU takes in.  Eight waves take the
+// contraction in turns of 32 rows, as in prenorm_qkv_skinny.hip, but with up to four turns' loads on their way at once: so little
+// weight has no order of DRAM pages to lose.  The last four turns have no loads behind them, so that 1024 rows pass without a loop.
+// 16x16x32 MFMAs: at most 16 tokens fill half of a 32x32 one, and the sums of eight waves that pass through LDS are half as many (16
+// tokens, 1024 x 512, rank 64 in 32x32x16 7.0 us, in 16x16x32 6.3, without the loads behind the last turns 5.9).
+#include "prenorm_qkv.h"
+
+namespace trn {
+
+struct FewArgs {
+    const half_t* x; const half_t* w; const half_t* a; const half_t* b; half_t* o;
+    int T, K, n, r, n_panels, silu;
+    int64_t ldx, ldw, lda, ldb, ldo;
+};
+
+// NR: blocks of 32 columns of the second matrix (A, or the panel of W2); TB: blocks of 16 tokens; PD: turns on their way
+template <int NR, int TB, int PD, bool GATE>
+__global__ __launch_bounds__(512, 2) void linear_few_kernel(const FewArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int NW = 8, NB = 1 + NR;                                 // waves, column blocks
+    constexpr int CPR = 4 * NR, RPL = 64 / CPR, AL = 32 / RPL;         // second matrix: chunks per row, rows per load, loads
+    constexpr int STAGE = NB * 1024 + TB * 512, DP = NR * 32 + 8;      // halfs of a wave's k-tile; pitch of D
+    constexpr int SSZ = NW * STAGE * 2, RSZ = NW * NB * 8 * 64 * 4;
+    __shared__ __attribute__((aligned(1024))) char smem[SSZ > RSZ ? SSZ : RSZ];
+    __shared__ __attribute__((aligned(256))) half_t Dm[GATE ? 8 : TB * 16 * DP];
+    __shared__ __attribute__((aligned(256))) half_t Bs[GATE ? 8 : NR * 32 * 32];
+
+    const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // (the two panels of a 128-byte line go to one XCD, whose L2 then has the line for both)
+    const int id = blockIdx.x, panel = 16 * (id >> 4) + 2 * (id & 7) + ((id >> 3) & 1);
+    if (panel >= a.n_panels) return;
+    const int n0 = 32 * panel, nkt = (a.K + 31) / 32;
+    constexpr int kOut = 0x7ffffff0;                 // a byte offset past every buffer: the load returns zeros
+    auto rows_of = [](const half_t* p, int64_t rows, int64_t pitch, int64_t cols) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(((rows - 1) * pitch + cols) * 2), 0x00020000);
+    };
+    const __amdgpu_buffer_rsrc_t xrs = rows_of(a.x, a.T, a.ldx, a.K), wrs = rows_of(a.w, a.K, a.ldw, a.n);
+    const __amdgpu_buffer_rsrc_t ars = rows_of(a.a, a.K, a.lda, GATE ? a.n : a.r);
+    const int wr = lane >> 2, wc = lane & 3, ar = lane / CPR, ac = lane % CPR;
+    const int w_pitch = (int)a.ldw * 2, a_pitch = (int)a.lda * 2, acol = (GATE ? n0 : 0) + 8 * ac;
+    const int w_vo = wr * w_pitch + (n0 + 8 * wc) * 2, a_vo = acol < (GATE ? a.n : a.r) ? ar * a_pitch + acol * 2 : kOut;
+    int x_vo[TB];
+#pragma unroll
+    for (int i = 0; i < TB; ++i) x_vo[i] = 16 * i + wr < a.T ? (int)((16 * i + wr) * a.ldx * 2) + wc * 16 : kOut;
+
+    // (unconditional, past the end as zeros: a load that may not be issued counts as absent when the compiler sizes its waits)
+    half8_t wreg[PD][2], areg[PD][AL], xreg[PD][TB], breg;
+    auto load = [](__amdgpu_buffer_rsrc_t rs, int vo, int so) __attribute__((always_inline)) {
+        return __builtin_bit_cast(half8_t, __builtin_amdgcn_raw_buffer_load_b128(rs, vo, so, 0));
+    };
+    auto fetch = [&](int j, int kt) __attribute__((always_inline)) {
+        const int k = 32 * min(kt, nkt), none = kt < nkt ? 0 : kOut;
+        const bool drop = k + 8 * wc >= a.K;                   // (columns past hidden hold the next row's data)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wreg[j][i] = load(wrs, w_vo | none, (k + 16 * i) * w_pitch);
+#pragma unroll
+        for (int i = 0; i < AL; ++i) areg[j][i] = load(ars, a_vo | none, (k + RPL * i) * a_pitch);
+#pragma unroll
+        for (int i = 0; i < TB; ++i) xreg[j][i] = load(xrs, drop ? kOut : x_vo[i], k * 2);
+    };
+
+    // ---- this wave's part of LDS: the blocks of 32 rows of 64 bytes each, then X in rows of 64 bytes, chunk j at j ^ ((r/4) % 4)
+    half_t* const Wm = reinterpret_cast<half_t*>(smem) + wave * STAGE;
+    half_t* const Xm = Wm + NB * 1024;
+    const int w_st = lane * 8, a_st = (1 + (ac >> 2)) * 1024 + ar * 32 + (ac & 3) * 8, x_st = wr * 32 + ((wc ^ ((wr >> 2) & 3)) << 3);
+    const int x_ld = c * 32 + ((g ^ ((c >> 2) & 3)) << 3);
+    // W^T through the transposing read: 16 columns, rows 8g + c/4 [+4]
+    const int w_ld = (8 * g + (c >> 2)) * 32 + (c & 3) * 4;
+    auto operand = [&](const half_t* block) __attribute__((always_inline)) {
+        const half4_t lo = lds_read_tr16(block + w_ld), hi = lds_read_tr16(block + w_ld + 4 * 32);
+        return half8_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    };
+    auto mfma16 = [](half8_t x, half8_t y, float4_t z) __attribute__((always_inline)) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(x, y, z, 0, 0, 0); };
+
+    const float4_t zero = {0.f, 0.f, 0.f, 0.f};
+    float4_t acc[TB][2 * NB];
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int nb = 0; nb < 2 * NB; ++nb) acc[tb][nb] = zero;
+
+    if constexpr (!GATE) {                           // this panel's columns of B: 16 rows a wave
+        const __amdgpu_buffer_rsrc_t brs = rows_of(a.b, a.r, a.ldb, a.n);
+        const int k = 16 * wave + wr;
+        breg = load(brs, wave < 2 * NR && k < a.r ? (int)(k * a.ldb * 2) + (n0 + 8 * wc) * 2 : kOut, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < PD; ++j) {
+        fetch(j, wave + NW * j);
+        __builtin_amdgcn_sched_barrier(0);           // (in this order: the loop's first wait is for the first turn alone)
+    }
+    auto turn = [&](int j, int ahead) __attribute__((always_inline)) {       // ahead: the turn to ask for in its place, -1: none
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *reinterpret_cast<half8_t*>(Wm + i * 512 + w_st) = wreg[j][i];
+#pragma unroll
+        for (int i = 0; i < AL; ++i) *reinterpret_cast<half8_t*>(Wm + i * RPL * 32 + a_st) = areg[j][i];
+#pragma unroll
+        for (int i = 0; i < TB; ++i) *reinterpret_cast<half8_t*>(Xm + i * 512 + x_st) = xreg[j][i];
+        __builtin_amdgcn_sched_barrier(0);
+        if (ahead >= 0) fetch(j, ahead);
+        __builtin_amdgcn_sched_barrier(0);
+        half8_t xv[TB];
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) xv[tb] = *reinterpret_cast<const half8_t*>(Xm + tb * 512 + x_ld);
+#pragma unroll
+        for (int nb = 0; nb < 2 * NB; ++nb) {
+            const half8_t wv = operand(Wm + (nb >> 1) * 1024 + (nb & 1) * 16);
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) acc[tb][nb] = mfma16(wv, xv[tb], acc[tb][nb]);
+        }
+    };
+    int kt = wave;
+    for (; kt + NW * PD < nkt; kt += NW * PD)
+#pragma unroll
+        for (int j = 0; j < PD; ++j) turn(j, kt + NW * (j + PD));
+#pragma unroll
+    for (int j = 0; j < PD; ++j)
+        if (kt + NW * j < nkt) turn(j, -1);
+    if constexpr (!GATE)
+        if (wave < 2 * NR) *reinterpret_cast<half8_t*>(Bs + wave * 512 + w_st) = breg;
+
+    // ---- the eight waves' partial results: wave w finishes register w % 4 of the blocks' 16 columns number w / 4, which is column
+    // col of them
+    float* const red = reinterpret_cast<float*>(smem);
+    const int col = 16 * (wave >> 2) + 4 * g + (wave & 3);
+    float sum[TB][NB];
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < 2 * NB; ++nb)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[((wave * NB * 2 + nb) * 4 + r) * 64 + lane] = acc[tb][nb][r];
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) v += red[((w * NB + nb) * 8 + wave) * 64 + lane];
+            sum[tb][nb] = v;
+        }
+    }
+    // ---- every product is rounded to fp16, as a separate one would leave it
+    if constexpr (!GATE) {
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+            for (int nb = 1; nb < NB; ++nb) {
+                const int d = 32 * (nb - 1) + col;   // (columns past the rank: zeros also where X is no number)
+                Dm[(16 * tb + c) * DP + d] = d < a.r ? (half_t)sum[tb][nb] : (half_t)0.f;
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        half_t o;
+        if constexpr (GATE) {
+            const float u = (float)(half_t)sum[tb][0], sg = 1.0f / (1.0f + fast_exp2(-u * kLog2e));
+            o = (half_t)((a.silu ? u * sg : sg) * (float)(half_t)sum[tb][1]);
+        } else {
+            float4_t p = zero;
+#pragma unroll
+            for (int ks = 0; ks < NR; ++ks)
+                p = mfma16(operand(Bs + ks * 1024 + 16 * (wave >> 2)), *reinterpret_cast<const half8_t*>(Dm + (16 * tb + c) * DP + 32 * ks + 8 * g), p);
+            const float q = wave & 2 ? (wave & 1 ? p[3] : p[2]) : (wave & 1 ? p[1] : p[0]);
+            o = (half_t)((float)(half_t)q + (float)(half_t)sum[tb][0]);
+        }
+        const int t = 16 * tb + c;
+        if (t < a.T && n0 + col < a.n) a.o[t * a.ldo + n0 + col] = o;
+    }
+#endif
+}
+
+// Where that is faster than two launches: up to what depth, by what a workgroup takes in beside its own panel (all of A; the second
+// panel, of which there are half as many workgroups as the two launches have).  Up to 4096 columns; us, two launches / one, forwards
+// back to back, the lower of several runs (the host's share of two launches varies from box to box, up to 2 us more):
+//   LoRA, rank 64   16 tokens: 1024 x 512 6.8 / 5.9, 1024 x 4096 7.0 / 6.0, 1280 x 2048 7.1 / 6.9, 1448 x 1024 7.4 / 7.3; but 2048 x 2048 7.8 / 8.5
+//                   32 tokens: 1024 x 512 7.5 / 7.2, 1088 x 512 7.7 / 7.5; but 24 tokens, 1280 x 2048 7.5 / 8.2
+//   rank 8 to 32    16 tokens: 256 x 256 5.9 / 3.8, 2048 x 1024 7.8 / 6.4, 3248 x 1160 12.4 / 9.9; but 4096 x 504 10.8 / 11.2
+//                   32 tokens: 1024 x 4096 7.6 / 5.8, 2048 x 4096 11.2 / 9.9; but 3000 x 2048 11.2 / 11.7, 4096 x 1024 10.9 / 11.7
+//   rank 128        16 tokens: 512 x 512 6.4 / 5.7, 704 x 4096 6.8 / 6.7; but 896 x 2048 6.9 / 7.3, 4096 x 1024 9.8 / 20.7
+//                   32 tokens: 512 x 512 7.0 / 7.1, 640 x 2048 7.2 / 7.9
+//   gated MLP       16 tokens: 1024 -> 1024 6.2 / 4.6, 1024 -> 4096 7.1 / 6.2, 1280 -> 4096 8.3 / 8.1, 1640 -> 2008 9.6 / 9.5, 1800 -> 1000 9.2 / 9.0; but 1536 ->
+//                   4096 8.9 / 9.1, 2048 -> 2048 8.9 / 9.5, 2200 -> 1000 10.2 / 10.8 (rows at odd half lines; 2400 -> 1024 7.4 / 6.8)
+//                   32 tokens: 1024 -> 4096 7.7 / 7.4, 1088 -> 2008 8.9 / 7.8, 1280 -> 1000 8.7 / 8.3; but 1200 -> 1400 7.9 / 8.6, 1280 -> 4096 8.8 / 9.5
+static bool few_suits(int64_t tokens, int64_t hidden, int64_t n, int64_t rank, bool gate) {
+    if (tokens > 32 || n > 4096) return false;
+    const bool one = tokens <= 16;
+    if (gate) return hidden <= (n <= 1024 ? (one ? 1800 : 1280) : n <= 2048 ? (one ? 1600 : 1088) : (one ? 1280 : 1024));
+    return hidden <= (rank <= 32 ? (one ? 3584 : 2560) : rank <= 64 ? (one ? 1448 : 1088) : rank <= 128 ? (one ? 704 : 448) : 0);
+}
+
+template <int NR, int PD, bool GATE>
+static int launch_few(FewArgs a, hipStream_t stream) {
+    a.n_panels = (a.n + 31) / 32;
+    const dim3 g((unsigned)((a.n_panels + 15) / 16 * 16)), t(512);
+    if (a.T <= 16) hipLaunchKernelGGL((linear_few_kernel<NR, 1, PD, GATE>), g, t, 0, stream, a);
+    else hipLaunchKernelGGL((linear_few_kernel<NR, 2, PD, GATE>), g, t, 0, stream, a);
+    return hipGetLastError() == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+}
+
+}  // namespace trn
+
+extern "C" int trn_lora_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, const void* w, int64_t n, int64_t ldw,
+                            const void* a, int64_t r, int64_t lda, const void* b, int64_t ldb, void* out, int64_t ldo,
+                            void* d, int64_t ldd, void* stream) {
+    using namespace trn;
+    GemmArgs first, second;
+    const void *w1[] = {w, a}, *w2[] = {b}, *ad[] = {out};
+    void *o1[] = {out, d}, *o2[] = {out};
+    const int64_t n1[] = {n, r}, l1[] = {ldw, lda}, p1[] = {ldo, ldd}, n2[] = {n}, l2[] = {ldb}, p2[] = {ldo};
+    int st = linear_args(first, x, tokens, hidden, ldx, 2, w1, n1, l1, o1, p1, nullptr);
+    if (st != TRN_OK) return st;
+    st = linear_args(second, d, tokens, r, ldd, 1, w2, n2, l2, o2, p2, ad);
+    if (st != TRN_OK || tokens == 0) return st;
+    if (few_suits(tokens, hidden, n, r, false)) {
+        const FewArgs f{(const half_t*)x, (const half_t*)w, (const half_t*)a, (const half_t*)b, (half_t*)out,
+                        (int)tokens, (int)hidden, (int)n, (int)r, 0, 0, ldx, ldw, lda, ldb, ldo};
+        hipStream_t s = (hipStream_t)stream;
+        return r <= 32 ? launch_few<1, 4, false>(f, s) : r <= 64 ? launch_few<2, 4, false>(f, s) : launch_few<4, 2, false>(f, s);
+    }
+    st = launch_projections(first, (hipStream_t)stream);
+    return st != TRN_OK ? st : launch_projections(second, (hipStream_t)stream);
+}
+
+extern "C" int trn_gated_mlp_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, const void* w1, int64_t ldw1,
+                                 const void* w2, int64_t ldw2, int64_t n, void* out, int64_t ldo, void* c2, int64_t ldc,
+                                 int32_t kind, void* stream) {
+    using namespace trn;
+    GemmArgs both;
+    const void* w[] = {w1, w2};
+    void* o[] = {out, c2};
+    const int64_t ns[] = {n, n}, lw[] = {ldw1, ldw2}, lo[] = {ldo, ldc};
+    if (kind != 0 && kind != 1) return TRN_E_SHAPE;
+    int st = linear_args(both, x, tokens, hidden, ldx, 2, w, ns, lw, o, lo, nullptr);
+    if (st != TRN_OK || tokens == 0) return st;
+    if (few_suits(tokens, hidden, n, 0, true)) {
+        const FewArgs f{(const half_t*)x, (const half_t*)w1, (const half_t*)w2, nullptr, (half_t*)out,
+                        (int)tokens, (int)hidden, (int)n, 0, 0, kind, ldx, ldw1, ldw2, 0, ldo};
+        return launch_few<1, 4, true>(f, (hipStream_t)stream);
+    }
+    st = launch_projections(both, (hipStream_t)stream);
+    return st != TRN_OK ? st : trn_gate_f16(out, c2, out, tokens, n, ldo, ldc, ldo, kind, stream);
+}

@@ -58,4 +58,8 @@ int64_t prenorm_qkv_mid_tiles(const GemmArgs& a, int mt, int nt);
 // The 128 x 128 tiling with two workgroups per CU, and the choice between them all (prenorm_qkv.hip).
 int launch_projections(GemmArgs a, hipStream_t stream);
 
+// The checks of trn_linear_f16, and its argument block (not filled in for no tokens).
+int linear_args(GemmArgs& a, const void* x, int64_t tokens, int64_t hidden, int64_t ldx, int32_t n_mats, const void* const* w,
+                const int64_t* n, const int64_t* ldw, void* const* out, const int64_t* ldo, const void* const* addend);
+
 }  // namespace trn

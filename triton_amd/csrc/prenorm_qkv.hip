@@ -297,10 +297,8 @@ extern "C" int trn_prenorm_qkv_f16(const void* x, const void* gamma, const void*
     return launch_projections(a, (hipStream_t)stream);
 }
 
-extern "C" int trn_linear_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, int32_t n_mats,
-                              const void* const* w, const int64_t* n, const int64_t* ldw, void* const* out,
-                              const int64_t* ldo, const void* const* addend, void* stream) {
-    using namespace trn;
+int trn::linear_args(GemmArgs& a, const void* x, int64_t tokens, int64_t hidden, int64_t ldx, int32_t n_mats, const void* const* w,
+                     const int64_t* n, const int64_t* ldw, void* const* out, const int64_t* ldo, const void* const* addend) {
     if (tokens < 0 || hidden <= 0 || n_mats < 1 || n_mats > 3) return TRN_E_SHAPE;
     if (!x || !w || !n || !ldw || !out || !ldo) return TRN_E_NULL;
     if (tokens == 0) return TRN_OK;
@@ -308,7 +306,6 @@ extern "C" int trn_linear_f16(const void* x, int64_t tokens, int64_t hidden, int
     if (ldx < hidden) return TRN_E_STRIDE;
     if (!aligned16(x) || !pitch16(ldx, 2)) return TRN_E_ALIGN;
     if ((tokens + 256) * ldx * 2 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
-    GemmArgs a;
     a.x = (const half_t*)x; a.gamma = nullptr;
     a.T = (int)tokens; a.K = (int)hidden; a.ldx = ldx; a.eps = 0.f; a.norm = 0;
     // plain row-major outputs [tokens, n_i]: "heads" of 8 columns at a pitch of 8 put column n at offset n
@@ -323,7 +320,15 @@ extern "C" int trn_linear_f16(const void* x, int64_t tokens, int64_t hidden, int
         if ((hidden + 512) * ldw[i] * 2 > 0x7fffffffLL) return TRN_E_UNSUPPORTED;
         a.p[i] = ProjOut{(const half_t*)w[i], (half_t*)out[i], ldw[i], 8, ldo[i], (int)n[i], 0, (const half_t*)ad};
     }
-    return launch_projections(a, (hipStream_t)stream);
+    return TRN_OK;
+}
+
+extern "C" int trn_linear_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, int32_t n_mats,
+                              const void* const* w, const int64_t* n, const int64_t* ldw, void* const* out,
+                              const int64_t* ldo, const void* const* addend, void* stream) {
+    trn::GemmArgs a;
+    const int st = trn::linear_args(a, x, tokens, hidden, ldx, n_mats, w, n, ldw, out, ldo, addend);
+    return st != TRN_OK || tokens == 0 ? st : trn::launch_projections(a, (hipStream_t)stream);
 }
 
 extern "C" int trn_gate_f16(const void* c1, const void* c2, void* out, int64_t rows, int64_t cols, int64_t ld1,
