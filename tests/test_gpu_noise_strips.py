@@ -271,3 +271,16 @@ def test_captured_module_and_where_the_rule_lies():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(c, want_c) and torch.equal(o, want_o)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("first,later", [(43.0, 43.0), (-43.0, -43.0), (-43.0, 43.0), (43.0, -43.0), (-46.0, 46.0), (60.0, -60.0), (-90.0, 90.0)])
+def test_rows_without_a_reference(first, later, half):
+    """Scores within 64 of zero, in the log2 domain (44.4), need no reference: rows on both sides of that line, whose first keys and
+    whose later ones lie on the same side of zero or on different ones, next to ordinary rows.  In fp16 noise of 32 and more is rounded to 2^-5, which is its value."""
+    q, k, v, n = problem(1, 71, 1, 641, 64, half, 0, 0, seed=3)
+    n[:, :, 1::3, :256] += first
+    n[:, :, 1::3, 256:] += later
+    n[:, :, 2::7] += first
+    _, rows, c = scores(q, k, v, n, 1.0)
+    check(q, k, n, rows, c, 1.0, 5e-5, [(0, 0), (0, 35), (0, 70)], largest=max(abs(first), abs(later)) * 2)
