@@ -8,6 +8,7 @@ struct AttnArgs {
     const half_t* q; const half_t* k; const half_t* v; half_t* o;
     float* lse; const half_t* gamma_q; const float* noise; float* lse_pert;
     int B, Hq, Hkv, Sq, Skv, n_qtiles;
+    int even;      // prefill kernels with split keys: two tiles of 64 queries a workgroup (attn_fwd16.hip)
     int64_t qb, qh, qs, kb, kh, ks, vb, vh, vs, ob, oh, os, nb, nh, ns;
     float c1;      // scale * log2(e)                    : plain scores in the log2 domain
     float c2, c3;  // scale*log2(e)/tau, log2(e)/tau     : perturbed scores  z2 = s*c2 + g*c3
@@ -172,7 +173,7 @@ hipError_t launch_attn_short(const AttnArgs& a, int head_dim, hipStream_t s);
 // The forward pass without score perturbation on the 16x16x32 MFMA (attn_fwd16.hip).  Narrow: 4 waves x 32 queries
 // per workgroup; Wide: 8 waves x 32 consecutive queries; Paired: 8 waves, two 128-query tiles from opposite ends of
 // the sequence (causal problems whose grid is a single round); Split: 8 waves on 128 queries, two groups of four that
-// take every other 64-key tile each (small grids, long walks).
+// take every other 64-key tile each (small grids, long walks), of a causal problem 64 from either end.
 enum class Attn16Shape { Narrow, Wide, Paired, Split };
 Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal);
 hipError_t launch_attn_fwd16(const AttnArgs& a, int head_dim, Attn16Shape shape, bool given_q, hipStream_t stream);

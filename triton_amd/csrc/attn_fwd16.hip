@@ -31,7 +31,7 @@ namespace trn {
 
 // What the two groups of four waves of an eight-wave workgroup do: kPlain, the same tile of 256 queries; kPaired, two
 // tiles of 128 queries from the two ends of a causal problem; kSplit, the same 128 queries, each group every other
-// 64-key tile; kShare, as kSplit on one of a.n_split shares of the keys, whose partial results a second launch merges.
+// 64-key tile -- of 128 consecutive queries or, under a causal mask, of two tiles of 64 from the two ends (a.even) --; kShare, as kSplit on one of a.n_split shares of the keys, whose partial results a second launch merges.
 enum { kPlain, kPaired, kSplit, kShare };
 
 __device__ __forceinline__ float4_t mfma16(half8_t a, half8_t b, float4_t c) {
@@ -119,12 +119,20 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     // 0-3 own the 128-query tile h, waves 4-7 the tile n - 1 - h from the other end, so that every workgroup has the
     // same amount of work and each SIMD holds one long and one short wave.  K/V staging follows the later tile; the
     // early waves stop at their own last visible tile as they do in plain mode.
+    // Split mode on two tiles of 64 (even): waves 0, 1, 6, 7 own the later one.
+    const bool even = MODE == kSplit && a.even != 0;
     int q0, q_last, wq0;
     if constexpr (PAIRED) {
         const int lt = (int)(blockIdx.x / BH), ht = a.n_qtiles - 1 - lt;     // n_qtiles counts 128-query tiles here
         q0 = ht * 128; q_last = q0 + 127;
         wq0 = (wave < 4 ? ht : lt) * 128 + (wave & 3) * 32;
         if (wave >= 4 && lt == ht) wq0 = a.Sq;          // odd tile count: the middle one is alone (loads clamp, stores are predicated off)
+    } else if (even) {              // (a SIMD has waves w and w + 4: one of the later tile and one of the earlier)
+        const int ht = a.n_qtiles - 1 - tile_no;                             // n_qtiles counts 64-query tiles here
+        const bool early = ((gw >> 1) ^ grp) != 0;
+        q0 = ht * 64; q_last = q0 + 63;
+        wq0 = (early ? tile_no : ht) * 64 + (gw & 1) * 32;
+        if (early && tile_no == ht) wq0 = a.Sq;
     } else {
         q0 = (a.n_qtiles - 1 - tile_no) * (GW * 32); q_last = q0 + GW * 32 - 1;
         wq0 = q0 + gw * 32;                             // first query of this wave
@@ -571,9 +579,10 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     __builtin_amdgcn_s_waitcnt(0x0f70);                // this wave's last refills (past the end, unread) have landed ...
     __syncthreads();                                   // ... and everyone's; every wave is done with the K/V stages
     if constexpr (SPLIT) {
-        // The groups hold partial results of the same queries.  Waves w and w + 4 exchange (m, l) and halves of O^T
-        // lane by lane: group 0 finishes the first D/2 columns, group 1 the others.  A wave that took no tile, or a
+        // The groups hold partial results of the same queries.  Waves w and w + 4 (of two tiles, w and w ^ 6) exchange (m, l) and
+        // halves of O^T lane by lane: group 0 finishes the first D/2 columns, group 1 the others.  A wave that took no tile, or a
         // query that saw no key of its group, has zero sums and weighs nothing.
+        const int other = wave ^ (even ? 6 : 4);
         constexpr int kStat = D == 128 ? 5120 : 2560;   // (floats) the row statistics lie behind the transposing regions
         float* stat = SHARE ? reinterpret_cast<float*>(Ks2_) : reinterpret_cast<float*>(Ks1_) + kStat;   // [8 waves][2 query blocks][16 queries] {m, l}
 #pragma unroll
@@ -586,7 +595,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         }
         constexpr int NH = NOP / 2;
         float4_t* mine = reinterpret_cast<float4_t*>(wave < 4 ? Ks0_ : Vs0_) + (wave & 3) * NH * 2 * 64;
-        const float4_t* theirs = reinterpret_cast<const float4_t*>(wave < 4 ? Vs0_ : Ks0_) + (wave & 3) * NH * 2 * 64;
+        const float4_t* theirs = reinterpret_cast<const float4_t*>(wave < 4 ? Vs0_ : Ks0_) + (other & 3) * NH * 2 * 64;
         if constexpr (SHARE) {          // (a stage of the ring holds two waves' halves)
             half_t *const ka_ = wave & 2 ? Ks1_ : Ks0_, *const va_ = wave & 2 ? Vs1_ : Vs0_;
             mine = reinterpret_cast<float4_t*>(wave < 4 ? ka_ : va_) + (wave & 1) * NH * 2 * 64;
@@ -600,7 +609,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         float wo[2], wt[2];
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-            const float mt = stat[(((wave ^ 4) * 2 + qb) * 16 + n) * 2], lt = stat[(((wave ^ 4) * 2 + qb) * 16 + n) * 2 + 1];
+            const float mt = stat[((other * 2 + qb) * 16 + n) * 2], lt = stat[((other * 2 + qb) * 16 + n) * 2 + 1];
             float ms = fmaxf(m[qb], mt);                  // (finite: every query sees a key -- but not of every share)
             if (SHARE && ms == -INFINITY) ms = 0.f;
             wo[qb] = fast_exp2(m[qb] - ms); wt[qb] = fast_exp2(mt - ms);
@@ -810,11 +819,21 @@ hipError_t launch_attn_shares(const AttnArgs& a, int head_dim, hipStream_t s) {
     return head_dim == 128 ? launch_shares<128>(a, s) : launch_shares<64>(a, s);
 }
 
+// Whether a workgroup with split keys takes two tiles of 64 queries from the two ends of a causal problem instead of 128 consecutive
+// ones: as many workgroups, all of the same work.  Where they run all at once (each needs a CU), the longest of the others sets the time.
+// us, one tile / two: 8 heads of 128: 1300 keys 21.1 / 18.8, 2048 28.8 / 24.4, 3000 39.3 / 32.8, 4096 50.7 / 43.6; 16: 1500 23.5 / 21.0, 2000
+// 29.0 / 26.3; 24: 1200 21.5 / 19.7; 16 heads of 64: 1300 14.1 / 12.6, 2048 19.1 / 16.7, and against narrow workgroups (Attn16Shape) 600
+// 9.6 / 9.4, 777 11.1 / 10.2, 32 heads: 640 9.8 / 9.6, 900 12.5 / 11.1, 1020 13.8 / 11.7, but 520 9.0 / 9.1; 16 heads, 3000 keys (384 workgroups) 27.3 / 34.6.
+static bool split_in_two(int64_t batch, int64_t n_q_heads, int64_t seq_q, int64_t seq_kv, bool causal) {
+    return causal && seq_q == seq_kv && (seq_q + 127) / 128 * batch * n_q_heads <= 256;
+}
+
 template <int D, int NW, int MODE, bool GIVEN>
 static hipError_t launch16(AttnArgs a, hipStream_t s) {
-    const int rows = MODE == kPlain ? 32 * NW : 128;
+    a.even = MODE == kSplit && split_in_two(a.B, a.Hq, a.Sq, a.Skv, a.causal != 0);
+    const int rows = MODE == kPlain ? 32 * NW : a.even ? 64 : 128;
     a.n_qtiles = (int)(((int64_t)a.Sq + rows - 1) / rows);
-    const int64_t grid = (int64_t)(MODE == kPaired ? (a.n_qtiles + 1) / 2 : a.n_qtiles) * a.B * a.Hq;
+    const int64_t grid = (int64_t)(MODE == kPaired || a.even ? (a.n_qtiles + 1) / 2 : a.n_qtiles) * a.B * a.Hq;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     if constexpr (GIVEN) hipLaunchKernelGGL((attn_fwd16_given_kernel<D, NW, MODE>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
     else if constexpr (MODE == kSplit) hipLaunchKernelGGL((attn_fwd16_split_kernel<D>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
@@ -831,7 +850,8 @@ static hipError_t launch16(AttnArgs a, hipStream_t s) {
 //          (8 heads of 128, 3000 tokens: 42.2 against 46.8; 16 heads of 64, 2000: 21.2 against 23.3; 250 queries on
 //          3250 keys: 46.0 against 51.0; but 1000 tokens, 16 heads of 128: 20.5 against 20.7, 600: 15.6 against 14.9).
 //          A causal triangle's short tiles leave room for a few more: W <= 320 (16 heads of 128, 2500: 40.1 against
-//          41.7 paired; at W = 416: 35.1 against 31.9).
+//          41.7 paired; at W = 416: 35.1 against 31.9).  Up to 256 a causal problem's workgroups take two short tiles each
+//          (split_in_two), which with head_dim 64 pays from 600 keys on.
 //  Paired  a causal problem whose narrow workgroups are all resident at once: the longest tile sets the time, twice the
 //          mean, so each workgroup takes two tiles from opposite ends.  Such workgroups are half as many and each needs
 //          a CU of its own: 192 to 256 of them (2048 tokens, llama heads: 40.5 against 44.4 narrow; at 288 workgroups,
@@ -847,6 +867,7 @@ Attn16Shape attn_fwd16_shape(int batch, int n_q_heads, int seq_q, int seq_kv, in
     const int64_t bh = (int64_t)batch * n_q_heads;
     const int64_t n128 = ((int64_t)seq_q + 127) / 128, W = n128 * bh;
     if (seq_kv >= 1100 && (W <= 256 || (causal && seq_kv == seq_q && W <= 320))) return Attn16Shape::Split;
+    if (head_dim == 64 && seq_kv >= 600 && split_in_two(batch, n_q_heads, seq_q, seq_kv, causal)) return Attn16Shape::Split;
     const int64_t pairs = ((n128 + 1) / 2) * bh;
     if (causal && W <= 512 && pairs >= 192 && pairs <= 256 && n128 >= 12) return Attn16Shape::Paired;
     const int64_t n256 = ((int64_t)seq_q + 255) / 256;
