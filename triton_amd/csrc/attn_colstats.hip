@@ -30,6 +30,7 @@ struct ColArgs {
     const half_t* q; const half_t* k; const float* lse; const float* noise;
     float* out_sum; float* out_sumsq;
     int B, Hq, Hkv, Sq, Skv, n_kvtiles;
+    HeadMap heads;
     int64_t qb, qh, qs, kb, kh, ks, nb, nh, ns;
     float c1;   // log2-domain multiplier of the raw score: scale*log2e (RoCo) or scale*log2e/tau (KeyFormer)
     float c3;   // log2e/tau multiplier of the noise
@@ -79,12 +80,10 @@ __global__ __launch_bounds__(NG * 256, 2) void attn_colstats_kernel(const ColArg
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int grp = NG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;        // within the group
-    const int BH = a.B * a.Hq;
-    const int kt = (int)(blockIdx.x / BH);             // key tile 0 sees the most queries: heaviest first
-    const int j = blockIdx.x % BH;
-    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
-    const int kvslot = j % nkv, g = j / nkv;
-    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+    const int kt = a.heads.all.of(blockIdx.x);         // key tile 0 sees the most queries: heaviest first
+    int b, kvh, g;
+    a.heads.find(blockIdx.x - kt * a.heads.all.d, b, kvh, g);
+    const int head = kvh * a.heads.G + g;
     const int off = a.Skv - a.Sq;
     const int kv0 = kt * CBN;
     const int wkey0 = kv0 + wave * 32;                 // this wave's 32 keys
@@ -330,12 +329,10 @@ __global__ __launch_bounds__(256, 2) void attn_colstats_plain_kernel(const ColAr
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int BH = a.B * a.Hq;
-    const int kt = (int)(blockIdx.x / BH);             // key tile 0 sees the most queries: heaviest first
-    const int j = blockIdx.x % BH;
-    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
-    const int kvslot = j % nkv, g = j / nkv;
-    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+    const int kt = a.heads.all.of(blockIdx.x);         // key tile 0 sees the most queries: heaviest first
+    int b, kvh, g;
+    a.heads.find(blockIdx.x - kt * a.heads.all.d, b, kvh, g);
+    const int head = kvh * a.heads.G + g;
     const int off = a.Skv - a.Sq;
 
     // ---- stages: Q rows and normalisers, direct global -> LDS; queries past the end read as zeros
@@ -575,6 +572,7 @@ int trn::attn_colstats(const trn_attn_desc* d, const void* q, const void* k, con
     a.out_sum = out_sum; a.out_sumsq = out_sumsq;
     a.B = d->batch; a.Hq = d->n_q_heads; a.Hkv = d->n_kv_heads; a.Sq = d->seq_q; a.Skv = d->seq_kv;
     a.n_kvtiles = (d->seq_kv + CBN - 1) / CBN;
+    a.heads = HeadMap(a.B, a.Hq, a.Hkv);
     a.qb = d->q_stride_b; a.qh = d->q_stride_h; a.qs = d->q_stride_s;
     a.kb = d->k_stride_b; a.kh = d->k_stride_h; a.ks = d->k_stride_s;
     a.nb = d->noise_stride_b; a.nh = d->noise_stride_h; a.ns = d->noise_stride_s;

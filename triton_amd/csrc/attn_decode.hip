@@ -75,12 +75,12 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     // So do the query tiles of a head, unless they are spread (decode_spread()); the last ones, with the most keys under a
     // causal mask, come first.
     int j, split = 0, dsl = 0, q0 = 0;
-    const int BH = a.B * a.Hq;
+    const int BH = a.heads.all.d;
     if (a.n_qtiles > 1) {
         int qt;
         if (a.spread) {
             const int unit = (int)blockIdx.x / (8 * DS) * 8 + (int)blockIdx.x % 8;
-            j = unit % BH; qt = unit / BH; dsl = (int)blockIdx.x / 8 % DS;
+            qt = a.heads.all.of(unit); j = unit - qt * BH; dsl = (int)blockIdx.x / 8 % DS;
         } else {
             const int per_grp = 8 * DS * a.n_qtiles, grp = (int)blockIdx.x / per_grp, rem = (int)blockIdx.x % per_grp;
             j = grp * 8 + rem % 8; qt = rem / (8 * DS); dsl = rem / 8 % DS;
@@ -94,9 +94,9 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     } else {
         j = blockIdx.x / a.n_split; split = blockIdx.x % a.n_split;
     }
-    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
-    const int kvslot = j % nkv, g = j / nkv;
-    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+    int b, kvh, g;
+    a.heads.find(j, b, kvh, g);
+    const int head = kvh * a.heads.G + g;
     const int off = a.Skv - a.Sq;                       // causal: query i sees keys <= i + off
     const int qrow = q0 + c;                            // this lane's query
     const int qrow_ld = qrow < a.Sq ? qrow : a.Sq - 1;

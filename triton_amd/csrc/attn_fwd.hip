@@ -65,12 +65,10 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a) {
     const int kfirst = grp * BN;                        // first key of this wave's first tile
 
     // ---- which (query tile, batch, head): heavy tiles first, KV heads interleaved across ids
-    const int BH = a.B * a.Hq;
-    const int qt = a.n_qtiles - 1 - (int)(blockIdx.x / BH);
-    const int j = blockIdx.x % BH;
-    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
-    const int kvslot = j % nkv, g = j / nkv;
-    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+    const int tile_no = a.heads.all.of(blockIdx.x), qt = a.n_qtiles - 1 - tile_no;
+    int b, kvh, g;
+    a.heads.find(blockIdx.x - tile_no * a.heads.all.d, b, kvh, g);
+    const int head = kvh * a.heads.G + g;
 
     const int off = a.Skv - a.Sq;                       // causal: query i sees keys <= i + off
     const int q0 = qt * BM;
@@ -893,6 +891,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     a.lse = lse; a.gamma_q = (const half_t*)gamma_q; a.noise = noise; a.lse_pert = lse_pert;
     a.B = d->batch; a.Hq = d->n_q_heads; a.Hkv = d->n_kv_heads; a.Sq = d->seq_q; a.Skv = d->seq_kv;
     a.n_qtiles = 0;   // set per tile shape at launch
+    a.heads = HeadMap(a.B, a.Hq, a.Hkv);
     a.qb = d->q_stride_b; a.qh = d->q_stride_h; a.qs = d->q_stride_s;
     a.kb = d->k_stride_b; a.kh = d->k_stride_h; a.ks = d->k_stride_s;
     a.vb = d->v_stride_b; a.vh = d->v_stride_h; a.vs = d->v_stride_s;

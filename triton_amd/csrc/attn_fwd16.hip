@@ -101,17 +101,16 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     half_t* const Ks1 = Ks1_ + grp * SR * D;
     half_t* const Vs0 = Vs0_ + grp * SR * D;
     half_t* const Vs1 = Vs1_ + grp * SR * D;
-    const int BH = a.B * a.Hq;
+    const int units = a.heads.all.of(blockIdx.x);
     // The shares of a query tile are consecutive; a share is a whole number of tiles, which the groups take in turns (not of pairs of
     // tiles: 4100 keys in eight shares would be seven of 640, and are eight of at most 576).
-    const int share = SHARE ? (int)(blockIdx.x / BH) % a.n_split : 0, tile_no = (int)(blockIdx.x / BH) / (SHARE ? a.n_split : 1);
+    const int share = SHARE ? units % a.n_split : 0, tile_no = SHARE ? units / a.n_split : units;
     const int share_tiles = SHARE ? ((a.Skv + BN - 1) / BN + a.n_split - 1) / a.n_split : 0;
     const int kfirst = grp * BN + share * share_tiles * BN;      // first key of this wave's first tile
 
-    const int j = blockIdx.x % BH;
-    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
-    const int kvslot = j % nkv, g = j / nkv;
-    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+    int b, kvh, g;
+    a.heads.find(blockIdx.x - units * a.heads.all.d, b, kvh, g);
+    const int head = kvh * a.heads.G + g;
 
     const int off = a.Skv - a.Sq;                       // causal: query i sees keys <= i + off
     // Query rows.  Plain mode: the workgroup owns BM consecutive queries, latest (heaviest under a causal mask) tiles
@@ -123,7 +122,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     const bool even = MODE == kSplit && a.even != 0;
     int q0, q_last, wq0;
     if constexpr (PAIRED) {
-        const int lt = (int)(blockIdx.x / BH), ht = a.n_qtiles - 1 - lt;     // n_qtiles counts 128-query tiles here
+        const int lt = tile_no, ht = a.n_qtiles - 1 - lt;     // n_qtiles counts 128-query tiles here
         q0 = ht * 128; q_last = q0 + 127;
         wq0 = (wave < 4 ? ht : lt) * 128 + (wave & 3) * 32;
         if (wave >= 4 && lt == ht) wq0 = a.Sq;          // odd tile count: the middle one is alone (loads clamp, stores are predicated off)
@@ -631,7 +630,7 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
             // 26.1, 40 on 3.1 k (5.3) 19.8 / 19.1; 16 of 64: 100 on 4.1 k 16.9 / 15.8, 60 on 4.3 k (4.1) 14.85 / 14.55, 50 on 4.2 k (3.4) 14.41 /
             // 14.31, 40 on 4.1 k (2.7) 14.34 / 14.56; 8 of 128: 40 on 3.1 k (2.7) 15.64 / 15.94; 71 of 64: 64 on 6 k (3.6) 29.9 / 29.9, 40 on 6 k (2.2)
             // 29.1 / 29.4)
-            const int64_t rows = (int64_t)BH * a.n_split * a.Sq, row0 = ((int64_t)(b * a.Hq + head) * a.n_split + share) * a.Sq;
+            const int64_t rows = (int64_t)a.heads.all.d * a.n_split * a.Sq, row0 = ((int64_t)(b * a.Hq + head) * a.n_split + share) * a.Sq;
             const int past = rows * D * 4 >= (int64_t)3 << 20 ? 1 : 0;
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb) {

@@ -28,6 +28,7 @@ namespace trn {
 struct StripArgs {
     const half_t* q; const half_t* k; const void* noise; float* lse; float* out; float* part;
     int B, Hq, Hkv, S, n_strips, n_slots;
+    HeadMap heads;
     int64_t qb, qh, qs, kb, kh, ks, nb, nh, ns;
     float c2, c3;      // scale*log2(e)/tau, log2(e)/tau
     int s16;
@@ -113,11 +114,10 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int BH = a.B * a.Hq;
-    const int slot = (int)(blockIdx.x / BH), j = blockIdx.x % BH;
-    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
-    const int kvslot = j % nkv, g = j / nkv;
-    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
+    const int slot = a.heads.all.of(blockIdx.x);
+    int b, kvh, g;
+    a.heads.find(blockIdx.x - slot * a.heads.all.d, b, kvh, g);
+    const int head = kvh * a.heads.G + g;
 
     const uint4_t qrs = descriptor(a.q + b * a.qb + head * a.qh, ((int64_t)(a.S - 1) * a.qs + D) * 2);
     const uint4_t krs = descriptor(a.k + b * a.kb + kvh * a.kh, ((int64_t)(a.S - 1) * a.ks + D) * 2);
@@ -550,6 +550,7 @@ hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void
     StripArgs a;
     a.q = (const half_t*)q; a.k = (const half_t*)k; a.noise = noise; a.lse = lse; a.out = (float*)out; a.part = (float*)workspace;
     a.B = d->batch; a.Hq = d->n_q_heads; a.Hkv = d->n_kv_heads; a.S = d->seq_q;
+    a.heads = HeadMap(a.B, a.Hq, a.Hkv);
     a.n_strips = (d->seq_q + 31) / 32; a.n_slots = noise_strip_slots(d, n16);
     a.qb = d->q_stride_b; a.qh = d->q_stride_h; a.qs = d->q_stride_s;
     a.kb = d->k_stride_b; a.kh = d->k_stride_h; a.ks = d->k_stride_s;

@@ -20,6 +20,31 @@ constexpr int kWave = 64;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
+// Division of numbers below 2^31 by one that the host knows: n / d = n m / 2^s with m the next whole number above 2^s / d, which at s = 31 +
+// ceil(log2 d) is exact and fits 32 bits.  A division of which the compiler knows nothing is some twenty dependent instructions at the
+// head of a kernel, before its first load.
+struct Div {
+    uint32_t m; int s, d;
+    Div() = default;
+    explicit Div(int64_t by) : s(31), d((int)by) {
+        while (((int64_t)1 << (s - 31)) < by) ++s;
+        m = (uint32_t)((((unsigned __int128)1 << s) / (uint64_t)by) + 1);
+    }
+    __host__ __device__ __forceinline__ int of(int n) const { return (int)(((uint64_t)(uint32_t)n * m) >> s); }
+};
+// Which head a workgroup has, of B x Hq numbered with the KV heads interleaved (those that share one lie on one XCD).
+struct HeadMap {
+    Div all, kv, hkv; int G;
+    HeadMap() = default;
+    HeadMap(int B, int Hq, int Hkv) : all((int64_t)B * Hq), kv((int64_t)B * Hkv), hkv(Hkv), G(Hq / Hkv) {}
+    __host__ __device__ __forceinline__ void find(int j, int& b, int& kvh, int& g) const {
+        g = kv.of(j);
+        const int slot = j - g * kv.d;
+        b = hkv.of(slot);
+        kvh = slot - b * hkv.d;
+    }
+};
+
 // D(32x32) += A(32x16) * B(16x32), fp16 in, fp32 out.  Lane l supplies A[l%32][8*(l/32)..+7]
 // and B[8*(l/32)..+7][l%32]; it receives D[8*(r/4) + 4*(l/32) + r%4][l%32] in element r.
 __device__ __forceinline__ float16_t mfma32(half8_t a, half8_t b, float16_t c) {
