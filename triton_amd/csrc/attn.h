@@ -9,6 +9,7 @@ struct AttnArgs {
     float* lse; const half_t* gamma_q; const float* noise; float* lse_pert;
     int B, Hq, Hkv, Sq, Skv, n_qtiles;
     HeadMap heads;
+    int pack;      // prefill kernels: 2^pack heads of a KV head to a workgroup (attn_fwd16.hip)
     int even;      // prefill kernels with split keys: two tiles of 64 queries a workgroup (attn_fwd16.hip)
     int64_t qb, qh, qs, kb, kh, ks, vb, vh, vs, ob, oh, os, nb, nh, ns;
     float c1;      // scale * log2(e)                    : plain scores in the log2 domain

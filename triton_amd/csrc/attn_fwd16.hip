@@ -101,6 +101,8 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     half_t* const Ks1 = Ks1_ + grp * SR * D;
     half_t* const Vs0 = Vs0_ + grp * SR * D;
     half_t* const Vs1 = Vs1_ + grp * SR * D;
+    // Query heads of one KV head: a group of waves is 2^pack of them times as many blocks of 32 queries (see packed_heads).
+    const int pack = MODE == kPlain ? a.pack : 0, lead = gw >> pack, QW = GW >> pack;
     const int units = a.heads.all.of(blockIdx.x);
     // The shares of a query tile are consecutive; a share is a whole number of tiles, which the groups take in turns (not of pairs of
     // tiles: 4100 keys in eight shares would be seven of 640, and are eight of at most 576).
@@ -110,7 +112,8 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
 
     int b, kvh, g;
     a.heads.find(blockIdx.x - units * a.heads.all.d, b, kvh, g);
-    const int head = kvh * a.heads.G + g;
+    if constexpr (MODE == kPlain) g = (g << pack) + (gw & ((1 << pack) - 1));
+    const int head = kvh * a.heads.G + (MODE == kPlain ? min(g, a.heads.G - 1) : g);
 
     const int off = a.Skv - a.Sq;                       // causal: query i sees keys <= i + off
     // Query rows.  Plain mode: the workgroup owns BM consecutive queries, latest (heaviest under a causal mask) tiles
@@ -133,8 +136,9 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         wq0 = (early ? tile_no : ht) * 64 + (gw & 1) * 32;
         if (early && tile_no == ht) wq0 = a.Sq;
     } else {
-        q0 = (a.n_qtiles - 1 - tile_no) * (GW * 32); q_last = q0 + GW * 32 - 1;
-        wq0 = q0 + gw * 32;                             // first query of this wave
+        q0 = (a.n_qtiles - 1 - tile_no) * (QW * 32); q_last = q0 + QW * 32 - 1;
+        wq0 = q0 + lead * 32;                           // first query of this wave
+        if (MODE == kPlain && g >= a.heads.G) wq0 = a.Sq;      // (no head for it)
     }
     int qrow[2];
 #pragma unroll
@@ -818,6 +822,24 @@ hipError_t launch_attn_shares(const AttnArgs& a, int head_dim, hipStream_t s) {
     return head_dim == 128 ? launch_shares<128>(a, s) : launch_shares<64>(a, s);
 }
 
+// How many heads of a KV head a narrow workgroup takes, as a power of two: 2^pack heads times 4 / 2^pack blocks of 32 queries instead of
+// four blocks of one head.  The tiles are then shorter by as much, their waves see the same keys, and a last tile of few queries, whose
+// walk is the longest, is a quarter as large.  Where workgroups come in more than one round, up to 2048 keys; not where one round holds them, since
+// the longest tile then has four waves with a full walk each.  us, one head / two / four:
+//   32 heads of 128 on 8: 4 x 520 tokens 20.9 / 19.0 / 16.9, 4 x 777 30.8 / 30.2 / 29.8, 3 x 777 26.4 / 24.3 / 24.4, 8 x 400 23.5 / 21.8 / 21.5, 2 x 1600
+//     49.5 / 46.8 / 46.8, 2250 47.4 / 46.9 / 47.2; 8 x 8 on 2, 1300 36.5 / 33.6 / 33.8; left out: 2 x 700 (384 workgroups of one head) 15.9 / 16.4 / 16.4, 8 x 250
+//     (512) 11.8 / 11.9 / 11.9, 8 x 8 on 2, 777 (448) 17.8 / 18.1 / 18.6, 4 x 8 on 2, 2600 55.9 / 57.0 / 56.8
+//   71 of 64 on one: 700 (426) 11.7 / 11.2 / 11.2, 2 x 300 (426) 9.0 / 7.8 / 7.9, 8 x 130 11.8 / 9.7 / 7.9, 4 x 400 16.2 / 13.8 / 13.5, 1600 30.7 / 29.4 / 29.2, 3600
+//     121 / 118 / 117; left out: 520 (355) 9.4 / 9.3 / 9.5, 300 (213) 7.1 / 7.2 / 7.5
+// (heads that do not fill the last workgroup leave its waves idle: a sixteenth of them at most)
+static int packed_heads(int batch, int n_kv_heads, int group, int seq_q, int seq_kv, int head_dim, bool causal) {
+    const int64_t narrow = ((int64_t)seq_q + 127) / 128 * batch * n_kv_heads * group;
+    if (!causal || seq_q != seq_kv || !(head_dim == 128 ? narrow > 512 && seq_kv <= 2048 : narrow >= 400)) return 0;
+    int p = 2;
+    while (p > 0 && (((int64_t)(group - 1) >> p) + 1) * 16 << p > (int64_t)group * 17) --p;
+    return p;
+}
+
 // Whether a workgroup with split keys takes two tiles of 64 queries from the two ends of a causal problem instead of 128 consecutive
 // ones: as many workgroups, all of the same work.  Where they run all at once (each needs a CU), the longest of the others sets the time.
 // us, one tile / two: 8 heads of 128: 1300 keys 21.1 / 18.8, 2048 28.8 / 24.4, 3000 39.3 / 32.8, 4096 50.7 / 43.6; 16: 1500 23.5 / 21.0, 2000
@@ -830,9 +852,11 @@ static bool split_in_two(int64_t batch, int64_t n_q_heads, int64_t seq_q, int64_
 template <int D, int NW, int MODE, bool GIVEN>
 static hipError_t launch16(AttnArgs a, hipStream_t s) {
     a.even = MODE == kSplit && split_in_two(a.B, a.Hq, a.Sq, a.Skv, a.causal != 0);
-    const int rows = MODE == kPlain ? 32 * NW : a.even ? 64 : 128;
+    a.pack = MODE == kPlain && NW == 4 ? packed_heads(a.B, a.Hkv, a.heads.G, a.Sq, a.Skv, D, a.causal != 0) : 0;
+    if (a.pack) a.heads.all = Div((int64_t)a.B * a.Hkv * (((a.heads.G - 1) >> a.pack) + 1));
+    const int rows = MODE == kPlain ? 32 * NW >> a.pack : a.even ? 64 : 128;
     a.n_qtiles = (int)(((int64_t)a.Sq + rows - 1) / rows);
-    const int64_t grid = (int64_t)(MODE == kPaired || a.even ? (a.n_qtiles + 1) / 2 : a.n_qtiles) * a.B * a.Hq;
+    const int64_t grid = (int64_t)(MODE == kPaired || a.even ? (a.n_qtiles + 1) / 2 : a.n_qtiles) * a.heads.all.d;
     if (grid > 0x7fffffffLL) return hipErrorInvalidValue;
     if constexpr (GIVEN) hipLaunchKernelGGL((attn_fwd16_given_kernel<D, NW, MODE>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
     else if constexpr (MODE == kSplit) hipLaunchKernelGGL((attn_fwd16_split_kernel<D>), dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
