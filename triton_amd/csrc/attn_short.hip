@@ -34,9 +34,9 @@ __global__ __launch_bounds__(256, 2) void attn_short_kernel(const AttnArgs a) {
 
     const int tid = threadIdx.x, lane = tid & 63, c = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int b, kvh, g;
-    a.heads.find(blockIdx.x, b, kvh, g);
-    const int head = kvh * a.heads.G + g;
+    const int G = a.Hq / a.Hkv, nkv = a.B * a.Hkv;
+    const int kvslot = blockIdx.x % nkv, g = blockIdx.x / nkv;
+    const int b = kvslot / a.Hkv, kvh = kvslot % a.Hkv, head = kvh * G + g;
     const int off = a.Skv - a.Sq, q0 = 32 * wave, qrow = q0 + c;
     const int64_t bh = (int64_t)b * a.Hq + head;
     // this wave's key blocks: none without queries, and under a causal mask none past its last query's last key
