@@ -374,12 +374,14 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         __builtin_amdgcn_sched_barrier(0);
     } else {
         TRN_FETCH_K(0, Ks0);
-        TRN_FETCH_V(0, Vs0);
-        if (SPLIT || ntiles > 1) TRN_FETCH_K(1, Ks1);
+        if constexpr (PAIRED) { TRN_FETCH_V(0, Vs0); TRN_FETCH_K(1, Ks1); }
+        __builtin_amdgcn_sched_barrier(0);
     }
 
-    // ---- Q^T B-operands: lane holds Q[qrow[qb]][32 ks + 8 g4 .. +7].  The loads go out behind the first K/V stage
-    // fetches and all together, so that the workgroup's start-up pays one memory latency, not three in a row.
+    // ---- Q^T B-operands: lane holds Q[qrow[qb]][32 ks + 8 g4 .. +7].  The loads go out behind the first K stage
+    // fetch and all together, so that the workgroup's start-up pays one memory latency, not three in a row; the other two stages
+    // behind them, for the first tile's hand-over.  us, in front of them / behind: 32 heads of 128, 300 tokens 9.3 / 8.95, 8 x 250 11.9 / 11.55,
+    // 4 x 777 29.9 / 29.3; 71 of 64, 300 7.07 / 6.71, 4 x 200 7.83 / 7.54, 2048 46.4 / 46.2; but paired tiles, 2048 of 32 heads 37.8 / 38.3.
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
         const int qrow_ld = qrow[qb] < a.Sq ? qrow[qb] : a.Sq - 1;       // clamp loads; stores are predicated
@@ -394,6 +396,12 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
     if (use_gq) {
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) gq[ks] = *reinterpret_cast<const half8_t*>(a.gamma_q + ks * 32 + 8 * g4);
+    }
+    if constexpr (!SHARE && !PAIRED) {
+        __builtin_amdgcn_sched_barrier(0);
+        TRN_FETCH_V(0, Vs0);
+        TRN_FETCH_K(1, Ks1);    // (also of a single tile, whose hand-over waits for it: the compiler takes a conditional load for absent)
+        __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (SHARE) {      // (the rest of the ring behind Q, whose wait would otherwise be for all of it)
         __builtin_amdgcn_sched_barrier(0);
@@ -434,8 +442,10 @@ __device__ __forceinline__ void attn_fwd16_body(const AttnArgs& a) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     } else {
-        __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0): this wave's loads have landed in LDS
-        __syncthreads();
+        constexpr int kBehind = PAIRED ? 0 : 2 * NI;    // K stage 0 has landed
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (kBehind & 15) | ((kBehind >> 4) << 14));
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
     }
 
     Scores16 sA, sB;                        // scores of the current / next 32-key block (ping-pong)
