@@ -4,6 +4,10 @@
 
 namespace trn {
 
+// Column sums of a head's workgroups that are still to be added, in their order: part [heads][n_slots][keys] fp32 into out
+// [heads][keys] (KeyFormer's single pass: attn_noise_strips.hip).  n_slots = 0: none.
+struct SlotSums { const float* part; void* out; int64_t n; int n_slots, keys, s16; Div by_keys; };
+
 struct AttnArgs {
     const half_t* q; const half_t* k; const half_t* v; half_t* o;
     float* lse; const half_t* gamma_q; const float* noise; float* lse_pert;
@@ -31,6 +35,7 @@ struct AttnArgs {
     int n16;       // noise points at fp16 data (its pitches count halfs; any alignment: see HalfNoise)
     int s16;       // decode and short kernels: col_sum and col_sumsq point at fp16 data
     int o_nt;      // prefill kernels: the output goes past the caches (outputs_stream)
+    SlotSums sums; int n_main;     // prefill kernels with the queries as given: sums to add, by the workgroups from n_main on
 };
 
 // Whether a launch of so many outputs stores them past the caches.  What it leaves dirty in the L2s is written back before it ends, on
@@ -121,13 +126,31 @@ __device__ __forceinline__ void store_stat(float* out, int s16, int64_t at, floa
     else out[at] = v;
 }
 
+// One element a thread.
+__device__ __forceinline__ void add_slots(const SlotSums& a, int64_t i) {
+    if (i >= a.n) return;
+    const int bh = a.by_keys.of((int)i), key = (int)i - bh * a.keys;
+    const float* p = a.part + (int64_t)bh * a.n_slots * a.keys + key;
+    float x = 0.f;
+    for (int s = 0; s < a.n_slots; s += 8) {     // (eight on their way at once.  Whole calls, us, one after the other / so: 8 heads of 128, 4096 keys (32
+                                                 // slots) 144.3 / 137.8; 16 of 64, 1536 41.9 / 39.4; 32 of 128, 1024 44.6 / 41.9)
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = p[(int64_t)min(s + e, a.n_slots - 1) * a.keys];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x += s + e < a.n_slots ? v[e] : 0.f;
+    }
+    store_stat(static_cast<float*>(a.out), a.s16, i, x);
+}
+
 // Checks, argument block and kernel choice behind every attention entry point of the C ABI.  given_q: without noise too the queries
-// are not multiplied by the scale, and rounded, before the products (attn_fwd16.hip; the other kernels never do).
+// are not multiplied by the scale, and rounded, before the products (attn_fwd16.hip; the other kernels never do).  sums: taken along by the
+// same launch, or added by one behind it.  check_only: nothing is launched.
 int attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                  const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                  int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs = nullptr,
                  bool n16 = false, bool s16 = false, bool any_pitch = false, bool k_norm = false, const void* gamma_k = nullptr,
-                 float k_eps = 0.f, bool mean_std = false, bool given_q = false);
+                 float k_eps = 0.f, bool mean_std = false, bool given_q = false, const SlotSums* sums = nullptr, bool check_only = false);
 
 // The checks of attn_colstats by themselves, for a caller that launches something else before it.
 int attn_colstats_check(const trn_attn_desc* d, const void* q, const void* k, const float* lse, const float* noise,
@@ -147,7 +170,8 @@ bool noise_streams(const trn_attn_desc* d, const void* noise, bool n16);
 int noise_strip_slots(const trn_attn_desc* d, bool n16);
 int64_t noise_strips_workspace_bytes(const trn_attn_desc* d, int with_noise);
 hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void* k, const void* noise, bool n16, float* lse, void* out,
-                               bool s16, void* workspace, hipStream_t s);
+                               bool s16, void* workspace, SlotSums& left, hipStream_t s);       // left: what the caller has to have added
+hipError_t launch_add_slots(const SlotSums& a, hipStream_t s);
 
 // One workgroup per head and 32 queries, whose eight waves split the keys (attn_decode.hip): at most 32 queries per head
 // (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.

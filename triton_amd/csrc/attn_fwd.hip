@@ -825,10 +825,14 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     // as given, as the forward with noise takes them)
     const int64_t parts = n && s1 && !s2 && noise_strip_slots(d, n16) > 0 ? noise_strips_workspace_bytes(d, n16 ? 2 : 3) : -1;
     if (parts == 0 || (parts > 0 && workspace && workspace_bytes >= parts)) {
-        st = attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream, nullptr, false, false, false, false,
-                          nullptr, 0.f, false, true);
-        if (st != TRN_OK) return st;
-        return launch_noise_strips(d, q, k, noise, n16, rows, out1, s16, workspace, (hipStream_t)stream) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+        // (in this order, so that the attention takes the sums of a head's workgroups along, 3 us as a launch of their own; what the attention refuses is
+        // refused before anything is written)
+        if (st = attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, false, false, false, false,
+                              nullptr, 0.f, false, true, nullptr, true); st != TRN_OK) return st;
+        SlotSums sums;
+        if (launch_noise_strips(d, q, k, noise, n16, rows, out1, s16, workspace, sums, (hipStream_t)stream) != hipSuccess) return TRN_E_LAUNCH;
+        return attn_forward(d, q, k, v, o, nullptr, nullptr, nullptr, nullptr, nullptr, 0, nullptr, nullptr, stream, nullptr, false, false, false, false,
+                            nullptr, 0.f, false, true, &sums);
     }
     // mean and deviation of a handful of queries: by the launch that merges the key shares; elsewhere the workspace stays
     // out of it (the plain attention would split the keys by counters in it that have to be zero)
@@ -878,7 +882,8 @@ extern "C" int trn_attn_qknorm_f16(const trn_attn_desc* d, const void* q, const 
 int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, const void* v, void* o, float* lse,
                              const void* gamma_q, const float* noise, float* lse_pert, void* workspace,
                              int64_t workspace_bytes, float* col_sum, float* col_sumsq, void* stream, float* probs,
-                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps, bool mean_std, bool given_q) {
+                             bool n16, bool s16, bool any_pitch, bool k_norm, const void* gamma_k, float k_eps, bool mean_std, bool given_q,
+                             const SlotSums* sums, bool check_only) {
     if (workspace && ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0 || workspace_bytes < 0)) return TRN_E_ALIGN;
     if (!d || !q || !k || !v || !o) return TRN_E_NULL;
     if (noise && !lse_pert) return TRN_E_NULL;
@@ -919,6 +924,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
     // (with room for the blocks the pipelines request past the end, which must stay representable to read as zeros)
     if (((int64_t)d->seq_kv + 2048) * d->k_stride_s * 2 > 0x7fffffffLL || ((int64_t)d->seq_kv + 2048) * d->v_stride_s * 2 > 0x7fffffffLL)
         return TRN_E_UNSUPPORTED;
+    if (check_only) return TRN_OK;
     hipStream_t s = (hipStream_t)stream;
     hipError_t e;
     if ((col_sum || col_sumsq) && d->seq_q > 32) {
@@ -935,8 +941,11 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         }
     }
     // few queries per head (decode), or few query tiles in all: one workgroup per head and 32 queries, its waves split the keys
-    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, noise != nullptr))
+    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, noise != nullptr)) {
+        if (sums && sums->n_slots > 0 && launch_add_slots(*sums, s) != hipSuccess) return TRN_E_LAUNCH;
         return launch_attn_decode(a, d->head_dim, workspace, workspace_bytes, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
+    }
+    if (sums) a.sums = *sums; else a.sums.n_slots = 0;
     // Without score perturbation: the 16x16x32 kernel, in the workgroup shape its launcher's rule picks.
     if (!noise)
         return launch_attn_fwd16(a, d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0), given_q, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;

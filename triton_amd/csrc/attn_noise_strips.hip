@@ -12,7 +12,7 @@
 // Eight waves take a strip's 32-key blocks in turn, each through a private part of LDS (K one block ahead, noise two), so that
 // the walk has no barrier.  S[query][key], a lane one key and 16 of the 32 queries: the scores' sums over the queries are then
 // sums within a lane, the blocks of a wave are the same columns in every strip, and a workgroup adds them up in LDS without
-// atomics; the second launch adds the workgroups of a head in a fixed order.  Results repeat bit for bit.
+// atomics; the launch of the attention behind this one adds the workgroups of a head in a fixed order.  Results repeat bit for bit.
 //
 // What bounds it: a wave's block is a chain -- K and noise out of LDS, eight MFMAs that wait for each other, the exponentials --
 // that two waves a SIMD overlap only in part, and 32 to 64 KB of noise in flight a CU.  71 heads of 64, 1536 keys, fp32: 79 us for
@@ -452,26 +452,14 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
 #endif
 }
 
-// The column sums of a head's workgroups, in their order.
-__global__ __launch_bounds__(256) void attn_add_slots_kernel(const float* part, float* out, int n_slots, int Skv, int64_t n, int s16) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int64_t bh = i / Skv, key = i % Skv;
-    const float* p = part + bh * n_slots * Skv + key;
-    float x = 0.f;
-    for (int s = 0; s < n_slots; s += 8) {       // (eight on their way at once.  Whole calls, us, one after the other / so: 8 heads of 128, 4096 keys (32
-                                                 // slots) 144.3 / 137.8; 16 of 64, 1536 41.9 / 39.4; 32 of 128, 1024 44.6 / 41.9)
-        float v[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = p[(int64_t)min(s + e, n_slots - 1) * Skv];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) x += s + e < n_slots ? v[e] : 0.f;
-    }
-    store_stat(out, s16, i, x);
+__global__ __launch_bounds__(256) void attn_add_slots_kernel(const SlotSums a) { add_slots(a, (int64_t)blockIdx.x * 256 + threadIdx.x); }
+hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
+    hipLaunchKernelGGL(attn_add_slots_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s, a);
+    return hipGetLastError();
 }
 
-// Where the two launches here -- one where a head has one workgroup -- and the plain attention are faster than the forward with
-// noise and the column statistics.  A third launch and the strips' ends have to be paid for: causal prompts of 300 keys and more
+// Where this launch and the plain attention, which adds the sums of a head's workgroups, are faster than the forward with
+// noise and the column statistics.  The strips' ends have to be paid for: causal prompts of 300 keys and more
 // with some MB of (visible) noise, the fewer heads the more of it, and not
 //   -- few heads of short prompts with little more than one strip a CU: some CUs then have two strips, most of them one;
 //   -- the longest rows, of which 2048 keys are held and the rest is read and multiplied twice;
@@ -546,7 +534,7 @@ static void launch_strips(const StripArgs& a, int nb, bool nt, unsigned grid, hi
 }
 
 hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void* k, const void* noise, bool n16, float* lse, void* out,
-                               bool s16, void* workspace, hipStream_t s) {
+                               bool s16, void* workspace, SlotSums& left, hipStream_t s) {
     StripArgs a;
     a.q = (const half_t*)q; a.k = (const half_t*)k; a.noise = noise; a.lse = lse; a.out = (float*)out; a.part = (float*)workspace;
     a.B = d->batch; a.Hq = d->n_q_heads; a.Hkv = d->n_kv_heads; a.S = d->seq_q;
@@ -565,10 +553,7 @@ hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void
     const bool wide = strip_waves(d) == 8;
     if (d->head_dim == 128) { if (wide) launch_strips<128, 8>(a, nb, nt, grid, s); else launch_strips<128, 4>(a, nb, nt, grid, s); }
     else { if (wide) launch_strips<64, 8>(a, nb, nt, grid, s); else launch_strips<64, 4>(a, nb, nt, grid, s); }
-    if (a.n_slots > 1) {
-        const int64_t n = bh * a.S;
-        hipLaunchKernelGGL(attn_add_slots_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a.part, a.out, a.n_slots, a.S, n, a.s16);
-    }
+    left = SlotSums{a.part, out, bh * a.S, a.n_slots > 1 ? a.n_slots : 0, a.S, a.s16, Div(a.S)};
     return hipGetLastError();
 }
 
