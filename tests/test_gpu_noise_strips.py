@@ -284,3 +284,21 @@ def test_rows_without_a_reference(first, later, half):
     n[:, :, 2::7] += first
     _, rows, c = scores(q, k, v, n, 1.0)
     check(q, k, n, rows, c, 1.0, 5e-5, [(0, 0), (0, 35), (0, 70)], largest=max(abs(first), abs(later)) * 2)
+
+
+# short prompts and the longest of fp16 noise, at the rule's lines: B, Hq, Hkv, S, D, fp16 noise, spare elements per row, first element
+SHORT = [
+    (1, 18, 2, 200, 64, False, 1, 0), (1, 20, 4, 201, 64, True, 0, 1), (2, 32, 8, 223, 64, True, 3, 0), (2, 64, 8, 225, 64, False, 0, 0), (2, 71, 1, 380, 64, True, 0, 1),
+    (1, 18, 2, 180, 128, False, 0, 1), (1, 40, 8, 180, 128, True, 1, 0), (2, 32, 8, 160, 128, False, 0, 0), (3, 24, 6, 193, 128, False, 3, 1), (2, 40, 8, 255, 128, True, 0, 0),
+    (2, 5, 5, 400, 128, False, 0, 0), (1, 48, 8, 1399, 128, True, 1, 0), (1, 32, 8, 1503, 64, True, 0, 0), (4, 71, 1, 200, 64, False, 0, 1),
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half,spare,first", SHORT)
+def test_one_pass_where_the_rule_begins(B, Hq, Hkv, S, D, half, spare, first):
+    tau, one = 1.5, B * Hq > 240
+    q, k, v, n = problem(B, Hq, Hkv, S, D, half, spare, first)
+    o, rows, c = scores(q, k, v, n, tau, one_workgroup=one)
+    heads = [(0, 0), (B - 1, Hq - 1), (B // 2, Hq // 2)]
+    check(q, k, n, rows, c, tau, 2e-5, heads)
+    check_outputs(q, k, v, o, heads)

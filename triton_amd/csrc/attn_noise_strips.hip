@@ -458,42 +458,48 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Where this launch and the plain attention, which adds the sums of a head's workgroups, are faster than the forward with
-// noise and the column statistics.  The strips' ends have to be paid for: causal prompts of 300 keys and more
-// with some MB of (visible) noise, the fewer heads the more of it, and not
-//   -- few heads of short prompts with little more than one strip a CU: some CUs then have two strips, most of them one;
+// Where this launch and the plain attention, which adds the sums of a head's workgroups, are faster than the forward with noise and the
+// column statistics: causal prompts nearly throughout, but not
 //   -- the longest rows, of which 2048 keys are held and the rest is read and multiplied twice;
-//   -- head_dim 128, where a block's K is twice its fp32 noise, once the two passes keep the rate of HBM all the time;
-//   -- fp16 noise, half as much to read for the same arithmetic, of long rows: with head_dim 64 only few heads, and many, whose
-//      workgroups are full rounds; with head_dim 128 up to 44 MB, of up to 16 heads 70, 10 heads 95;
+//   -- fp16 noise, half as much to read for the same arithmetic, of long rows of few heads;
 //   -- long prompts of 64 to 319 heads with keys of their own, when the heads' count is no multiple of the 8 XCDs: a head's
 //      workgroups are then on all of them, and each L2 reads all of K.
-// Whole calls, here / two passes in per cent of time (1600 sizes; minus: faster here):
-//   D = 64, fp32   71 heads: 300 keys -1, 570 -13, 1100 -26, 2700 -23; 32: 500 -17, 1001 -19, 2000 -15; 8: 1001 -18, 2000 -27, 4000 -22.  Left out:
-//         9 and 10 heads, 900 and 1001 keys (261 to 320 strips) +2 to +9, 12, 800 +6; 4800 keys: 12 +10, 16 -3, 8 (kept) -7
-//   D = 64, fp16   71: 340 -5, 640 -13, 1100 -15, 2000 -7; 16: 1001 -26, 2000 -17; 4 x 71, 1001 -12, 2450 -10; 256, 2000 -12.  Left out: 24 heads, 1650
-//         to 2000 keys +6 to +9 (1100 kept, -6), 32, 1400 +5, 48, 1650 +4; 142 heads with keys of their own, 1650 +9
-//   D = 128, fp32  32: 390 -22, 1001 -17, 2000 -11, 3000 -6; 8: 1800 -20, 3000 -22; 71 on one KV head, 1001 -15; 256, 1001 -19.  Left out: 4400 and 4800
-//         keys -8 to +20; 16 heads, 2700 to 3640 +3 to +9; 142 with keys of their own, 1190 to 1500 +1 to +15
-//   D = 128, fp16  32: 300 -25, 640 -4, 1001 -12; 8: 1001 -20, 2000 -18, 4000 -11; 16: 1501 -18, 2000 -13; 14: 2000 -12.  Left out: 16 heads, 2200 +2,
-//         2700 to 3640 +6 to +17; 12, 2700 +3, 3640 +13; 8 and 9, 4400 +5; 32, 1350 (56 MB) +6, 2500 +3
-// Inside the lines one size in forty loses 1 to 5 %, where the strips fall badly on the CUs: 24 heads of 128, 2000 keys, fp32 +5; 48 of 64, 1001,
-// fp16 +4; 56 of 128, 300, fp32 +4.
+// Calls in a graph, here / two passes in per cent of time (900 sizes; minus: faster here):
+//   D = 64, fp32   71 heads: 420 keys -8, 1001 -30, 2600 -20; 142: 160 -8, 260 -16, 1000 -32; 284: 230 -11, 290 -9; 128: 200 -10; 16: 1000 -39, 2100 -18.  Left out:
+//         4800 keys: 12 heads +10, 16 -3, 8 (kept) -7
+//   D = 64, fp16   71: 520 -19, 1000 -17, 2600 -8; 20: 1440 -25; 32: 1500 -4, 2000 -7, 3000 -9; 48: 1360 -11, 1700 -1, 2400 -11; 142: 380 -6, 560 -14; 284: 440 -8.  Left out: 284, 330
+//         +1, 568, 290 +6; 24 heads, 1700 to 2000 +1 to +8 (1500 -11); 16, 2600 +9, 3300 +13; 142 with keys of their own, 1650 +9
+//   D = 128, fp32  32: 420 -17, 1000 -21, 2100 -13, 3100 -2, 3800 -4; 64: 160 -40, 260 -7, 2400 -8; 256: 260 -14, 1400 -19; 24: 420 -23, 1300 -7; 16: 520 -13, 1300
+//         -29; 10: 520 -22; 8: 1800 -29, 4000 -17.  Left out: 256, 200 +5; 32, 4000 +5; 16 heads, 2700 to 3640 +3 to +9; 142 with keys of their own,
+//         1190 to 1500 +1 to +15
+//   D = 128, fp16  32: 420 -15, 1000 -15; 8: 1000 -16, 2600 -30, 4000 -18; 16: 520 -11, 1000 -27; 9: 900 -3; 48: 360 -6, 1400 -7; 64: 420 -11, 1400 -2; 96: 1000 -7, 2500 -1; 128:
+//         520 -10, 2500 -2; 256: 640 -10, 2500 -4.  Left out: 32, 1350 +4, 1800 +5; 48, 1700 +6; 64, 1700 +4 (2100 -4); 16, 2200 +2, 2700 to 3640 +6 to +17; 8 and 9, 4400 +5
+// Inside the lines one size in thirty loses 1 to 6 %, where the strips fall badly on the CUs: 112 heads of 128, 560 to 740 keys, fp16; 128, 400, fp16 +3; 192 of
+// 64, 470, fp16 +5; 32 of 64, 1600, fp16 +10.  Short prompts of these lines, where a launch counts: 70 of 128, 210, fp16 -37; 40 of 64, 226, fp32 -28; 48 of 64,
+// 240, fp16 -29; 40 of 128, 180, fp16 -5.  (So would prompts of 65 to 127 heads of 64 below 300 keys gain, and those of up to 16 with less noise than the lines
+// ask for: 2 to 17 %.  They have been calls without a workspace, and stay so.)
 static bool strips_suit(const trn_attn_desc* d, bool n16) {
-    if (!d->causal || d->seq_q != d->seq_kv || d->seq_q < 300) return false;
+    if (!d->causal || d->seq_q != d->seq_kv || d->seq_q < 160) return false;
     const int64_t bh = (int64_t)d->batch * d->n_q_heads, mb = (bh * d->seq_q * d->seq_q * (n16 ? 1 : 2)) >> 20;
-    const int64_t strips = bh * ((d->seq_q + 31) / 32);
+    const int64_t strips = bh * ((d->seq_q + 31) / 32), S = d->seq_q;
     const bool second_strips = bh <= 16 && strips > 256 && strips <= 320;
     const bool scattered = bh % 8 != 0 && bh < 320 && (int64_t)d->batch * d->n_kv_heads >= 64;
     if (d->head_dim == 64) {
-        if ((second_strips && d->seq_q <= 1024) || (d->seq_q > 4500 && bh > 8)) return false;
-        if (!n16) return mb >= 12;
-        if (d->seq_q > 1250 && !(bh < 22 ? mb <= 96 : bh >= 64 && !scattered)) return false;
-        return mb >= 7 && (bh <= 80 || d->seq_q >= 600);
+        if ((second_strips && S <= 1024) || (S > 4500 && bh > 8)) return false;
+        const bool launches = S >= 200 && bh >= 18 && bh <= 64;
+        if (!n16) return launches || (S < 300 ? bh >= 128 && S >= 200 : mb >= 12);
+        if (S > 1250 && !(bh < 22 ? mb <= 96 : bh >= 32 && !scattered)) return false;
+        return launches || (S >= 300 && mb >= 7 && (bh <= 80 || S >= 380));
     }
-    if (d->seq_q > 4200) return false;
-    if (n16) return bh <= 16 ? mb >= 4 && !second_strips && (bh <= 8 || mb <= (bh <= 10 ? 95 : 70)) : mb <= 44 && (bh <= 32 || d->seq_q >= 600);
-    return mb >= (bh >= 32 ? 9 : bh >= 16 ? 28 : 38) && mb <= (bh > 12 && bh < 18 ? 200 : 640) && (!scattered || d->seq_q <= 700);
+    if (S > 4200) return false;
+    if (n16) {
+        if (bh <= 16) return S >= 300 && mb >= 4 && (bh <= 8 || mb <= (bh <= 10 ? 95 : 70));
+        if (S < (bh <= 64 ? 180 : bh <= 128 ? 240 : 420)) return false;
+        return bh < 40 ? mb <= 44 : S <= (bh < 96 ? 1400 : bh < 128 ? 1600 : 2600);
+    }
+    if (scattered && S > 700) return false;
+    if (S < 300) return bh >= 18 && S >= (bh < 64 ? 180 : bh < 192 ? 160 : 260);
+    return bh >= 18 ? S <= (bh >= 32 ? 3800 : 3400) : mb >= (bh > 8 ? 3 : 16) && (bh <= 12 || mb <= 200);
 }
 // Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
 // and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
