@@ -292,10 +292,16 @@ SHORT = [
     (1, 18, 2, 180, 128, False, 0, 1), (1, 40, 8, 180, 128, True, 1, 0), (2, 32, 8, 160, 128, False, 0, 0), (3, 24, 6, 193, 128, False, 3, 1), (2, 40, 8, 255, 128, True, 0, 0),
     (2, 5, 5, 400, 128, False, 0, 0), (1, 48, 8, 1399, 128, True, 1, 0), (1, 32, 8, 1503, 64, True, 0, 0), (4, 71, 1, 200, 64, False, 0, 1),
 ]
+# strips that are no multiple of a head's workgroups: missing from the first round (of one workgroup a CU and of two, an odd and an even number of
+# rounds), and from the last
+DEALT = [
+    (1, 8, 2, 2170, 64, False, 0, 0), (1, 24, 6, 1390, 64, False, 1, 0), (1, 32, 8, 514, 128, False, 0, 0), (1, 44, 4, 743, 64, True, 0, 1), (1, 71, 1, 505, 64, False, 0, 0),
+    (1, 71, 1, 820, 128, False, 3, 0), (4, 16, 16, 613, 64, True, 0, 0), (3, 48, 8, 400, 128, False, 0, 1),
+]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,S,D,half,spare,first", SHORT)
-def test_one_pass_where_the_rule_begins(B, Hq, Hkv, S, D, half, spare, first):
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half,spare,first", SHORT + DEALT)
+def test_one_pass_where_the_rule_begins_and_strips_are_missing(B, Hq, Hkv, S, D, half, spare, first):
     tau, one = 1.5, B * Hq > 240
     q, k, v, n = problem(B, Hq, Hkv, S, D, half, spare, first)
     o, rows, c = scores(q, k, v, n, tau, one_workgroup=one)

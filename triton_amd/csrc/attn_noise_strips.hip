@@ -27,7 +27,7 @@ namespace trn {
 
 struct StripArgs {
     const half_t* q; const half_t* k; const void* noise; float* lse; float* out; float* part;
-    int B, Hq, Hkv, S, n_strips, n_slots;
+    int B, Hq, Hkv, S, n_strips, n_slots, missing;
     HeadMap heads;
     int64_t qb, qh, qs, kb, kh, ks, nb, nh, ns;
     float c2, c3;      // scale*log2(e)/tau, log2(e)/tau
@@ -138,8 +138,9 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
     // ---- the wave's list of blocks: of strip after strip, those beyond the last kHeldBlocks first, then these, then the first
     // ones again
     struct Cursor { int k, i, n, q0, again; };
-    auto open = [&](Cursor& x) __attribute__((always_inline)) {      // strip number x.k of this workgroup: long and short ones in turn
-        const int idx = x.k * a.n_slots + ((x.k & 1) ? a.n_slots - 1 - slot : slot);
+    const int first_round = slot < a.missing ? 1 : 0;
+    auto open = [&](Cursor& x) __attribute__((always_inline)) {      // the strip of round x.k: long and short ones in turn
+        const int idx = x.k * a.n_slots + ((x.k & 1) ? a.n_slots - 1 - slot : slot) - a.missing;
         if (idx >= a.n_strips) { x.q0 = -1; x.n = 0; return; }
         x.q0 = 32 * idx;
         const int blocks = (min(a.S, x.q0 + 32) + 31) >> 5;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(NW * 64, NW == 8 ? 1 : 2) void attn_noise_strips_ke
     };
 
     // the noise runs two blocks ahead, K one: k_next is the key of the block that the noise was last asked for
-    Cursor cn{0, 0, 0, 0, 0}, now{0, 0, 0, 0, 0};
+    Cursor cn{first_round, 0, 0, 0, 0}, now{first_round, 0, 0, 0, 0};
     open(cn);
     if (cn.q0 >= 0 && cn.n == 0) { cn.i = -1; advance(cn); }
     open(now);
@@ -475,7 +476,7 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
 //   D = 128, fp16  32: 420 -15, 1000 -15; 8: 1000 -16, 2600 -30, 4000 -18; 16: 520 -11, 1000 -27; 9: 900 -3; 48: 360 -6, 1400 -7; 64: 420 -11, 1400 -2; 96: 1000 -7, 2500 -1; 128:
 //         520 -10, 2500 -2; 256: 640 -10, 2500 -4.  Left out: 32, 1350 +4, 1800 +5; 48, 1700 +6; 64, 1700 +4 (2100 -4); 16, 2200 +2, 2700 to 3640 +6 to +17; 8 and 9, 4400 +5
 // Inside the lines one size in thirty loses 1 to 6 %, where the strips fall badly on the CUs: 112 heads of 128, 560 to 740 keys, fp16; 128, 400, fp16 +3; 192 of
-// 64, 470, fp16 +5; 32 of 64, 1600, fp16 +10.  Short prompts of these lines, where a launch counts: 70 of 128, 210, fp16 -37; 40 of 64, 226, fp32 -28; 48 of 64,
+// 64, 470, fp16 +5; 32 of 128, 1260, fp32 +2.  Short prompts of these lines, where a launch counts: 70 of 128, 210, fp16 -37; 40 of 64, 226, fp32 -28; 48 of 64,
 // 240, fp16 -29; 40 of 128, 180, fp16 -5.  (So would prompts of 65 to 127 heads of 64 below 300 keys gain, and those of up to 16 with less noise than the lines
 // ask for: 2 to 17 %.  They have been calls without a workspace, and stay so.)
 static bool strips_suit(const trn_attn_desc* d, bool n16) {
@@ -524,6 +525,19 @@ int noise_strip_slots(const trn_attn_desc* d, bool n16) {
     return best;
 }
 
+// A head's strips are dealt to its workgroups in rounds of n_slots, in turns of direction.  Where the last round is not full, strips
+// are taken as missing from the first one, the shortest, instead of from the last, the longest: the sums of strips are then equal
+// after an even number of rounds, and a short strip apart after an odd one.  Of two workgroups a CU, whose sum counts, the odd numbers
+// gain little, and of more than 56 heads nothing.  us, missing from the last / first: one workgroup: 8 of 64: 2170 keys 49.0 / 41.3; 8 of 128: 2103
+// 60.6 / 51.1; 16 of 64: 2116 75.2 / 65.4; 32 of 64: 1600 69.6 / 56.3; 40 of 64: 2327 179 / 163; 64 of 64: 3337 512 / 491; 71 of 64: 2600 342 / 332; two, even: 32 of 128: 514
+// 30.8 / 24.7, 1600 95.4 / 83.3; 64 of 128: 1300 107 / 97; 48 of 128: 993 -11 %; 71 of 64: 777 39.7 / 37.9; odd: 44 of 128: 1603 130 / 123; 40 of 64: 953 35.9 / 37.6; left out:
+// 64 of 64: 578 28.9 / 30.2; 80: 1227 +8 %; 71: 948 53.1 / 54.5, 601 31.6 / 30.8.
+static int strips_missing(const trn_attn_desc* d, int n_strips, int n_slots) {
+    const int rounds = (n_strips + n_slots - 1) / n_slots;
+    if (strip_waves(d) == 4 && (int64_t)d->batch * d->n_q_heads > 56 && (rounds & 1)) return 0;
+    return rounds * n_slots - n_strips;
+}
+
 int64_t noise_strips_workspace_bytes(const trn_attn_desc* d, int with_noise) {
     const int n32 = with_noise == 2 ? 0 : noise_strip_slots(d, false), n16 = with_noise == 3 ? 0 : noise_strip_slots(d, true);
     const int64_t n = n32 > 0 ? n32 : n16;       // (the same number where both suit)
@@ -545,7 +559,7 @@ hipError_t launch_noise_strips(const trn_attn_desc* d, const void* q, const void
     a.q = (const half_t*)q; a.k = (const half_t*)k; a.noise = noise; a.lse = lse; a.out = (float*)out; a.part = (float*)workspace;
     a.B = d->batch; a.Hq = d->n_q_heads; a.Hkv = d->n_kv_heads; a.S = d->seq_q;
     a.heads = HeadMap(a.B, a.Hq, a.Hkv);
-    a.n_strips = (d->seq_q + 31) / 32; a.n_slots = noise_strip_slots(d, n16);
+    a.n_strips = (d->seq_q + 31) / 32; a.n_slots = noise_strip_slots(d, n16); a.missing = strips_missing(d, a.n_strips, a.n_slots);
     a.qb = d->q_stride_b; a.qh = d->q_stride_h; a.qs = d->q_stride_s;
     a.kb = d->k_stride_b; a.kh = d->k_stride_h; a.ks = d->k_stride_s;
     a.nb = d->noise_stride_b; a.nh = d->noise_stride_h; a.ns = d->noise_stride_s;
