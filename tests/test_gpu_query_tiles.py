@@ -33,7 +33,16 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,with_noise,tiles", CASES)
+# few heads of 128 under a causal mask: past a tile a CU
+FEW = [
+    (1, 4, 1, 3584, 3584, 128, True, False, True), (1, 4, 1, 3585, 3585, 128, True, False, False), (1, 8, 2, 1025, 1025, 128, True, False, True),
+    (1, 8, 2, 1600, 1600, 128, True, False, True), (1, 8, 2, 1601, 1601, 128, True, False, False), (1, 8, 2, 1200, 1201, 128, True, False, False),
+    (1, 8, 8, 1100, 1100, 128, False, False, False), (2, 5, 5, 1117, 1117, 128, True, False, True), (1, 10, 2, 1121, 1121, 128, True, False, False),
+    (1, 12, 4, 861, 861, 128, True, False, True), (1, 12, 4, 865, 865, 128, True, False, False), (1, 13, 1, 700, 700, 128, True, False, False),
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,with_noise,tiles", CASES + FEW)
 def test_attention_on_both_sides_of_the_query_tile_rule(B, Hq, Hkv, Sq, Skv, D, causal, with_noise, tiles):
     from triton_amd import ops
     g = torch.Generator().manual_seed(Sq * Skv)

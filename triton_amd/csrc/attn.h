@@ -175,7 +175,7 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s);
 
 // One workgroup per head and 32 queries, whose eight waves split the keys (attn_decode.hip): at most 32 queries per head
 // (decode), and problems with so few query tiles that the prefill kernels would leave most of the chip idle.
-bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
+bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal, bool noise);
 hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 // ... and where that launch, without a workspace, also normalises the keys if asked to (args.k_norm).
 bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);

@@ -754,16 +754,23 @@ static int decode_col_shares(int64_t units, int seq_q, int seq_kv, int head_dim)
 // tiles than CUs: head_dim 64 on long caches (71 heads, 100 queries: 4100 keys 42 / 35, 1124 keys 15.6 / 15.6, 164 keys
 // 6.8 / 10.2); with score perturbation, where the prefill kernel is slower, any (32 heads of 128, causal 350 on 350 22 /
 // 19; 71 heads of 64, 128 queries on 4128 keys 114 / 83; but 781 tiles 20 / 25).
-bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
+// Few heads of 128 under a causal mask have long tiles, which come first, and the CUs of the short ones take those past 256:
+// us, split keys (narrow workgroups below 1100 keys) / here: one head of 4: 2071 keys (260 tiles) 24.1 / 19.6, 2807 30.0 / 24.7, 3575 (448) 35.6 / 33.6, 4055
+// (508) 39.6 / 39.5; of 8: 1143 (288) 17.3 / 14.5, 1399 19.4 / 18.2, 1591 (400) 21.2 / 20.9, 1783 22.4 / 22.8; of 10: 823 (260) 15.4 / 12.9,
+// 1015 18.5 / 16.4, 1111 (350) 17.8 / 17.5, 1271 18.7 / 19.2; of 12: 727 (276) 15.0 / 13.8, 855 (324) 16.7 / 15.4; of 14: 695 (308) 14.0 / 14.1; of 16: 567 (288) 12.3 / 13.1.
+// (Not the attention that adds the sums of KeyFormer's single pass: this launch does not.)
+bool attn_decode_suits(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool causal, bool noise) {
     if (seq_q <= 32) return true;
-    const int64_t tiles = (int64_t)batch * n_q_heads * ((seq_q + 31) / 32);
+    const int64_t bh = (int64_t)batch * n_q_heads, tiles = bh * ((seq_q + 31) / 32);
+    if (head_dim == 128 && causal && seq_q == seq_kv && bh <= 12 && tiles <= (bh <= 4 ? 448 : bh <= 8 ? 400 : bh <= 10 ? 350 : 330)) return true;
     return tiles <= 256 || (tiles < 512 && (noise || (head_dim == 64 && seq_kv >= 1024)));
 }
 
 // Each tile of 32 queries normalises the keys it reads, some 0.25 us per 256 keys against 3 - 5 us for a launch: up to 2048.
-// us, launch / here: 8 heads of 128, 1024 tokens 18.5 / 17.0; 2 x 8, 394 14.0 / 11.9.
+// us, launch / here: 8 heads of 128, 1024 tokens 18.5 / 17.0; 2 x 8, 394 14.0 / 11.9.  (Not where a CU has a second tile of head_dim 128:
+// 8 heads, 1399 22.9 / 25.5; 10, 1015 21.0 / 23.0.)
 bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
-    return attn_decode_suits(batch, n_q_heads, seq_q, seq_kv, head_dim, false) && seq_kv <= 2048;
+    return attn_decode_suits(batch, n_q_heads, seq_q, seq_kv, head_dim, false, false) && seq_kv <= 2048;
 }
 
 // Whether the scores of a head's keys fit the registers of one workgroup, for key statistics without a second sweep.

@@ -684,7 +684,7 @@ extern "C" const char* trn_attn_fwd_kernel_name(const trn_attn_desc* d, int32_t 
     using namespace trn;
     if (!d || validate_attn(d, true) != TRN_OK) return "";
     const bool d128 = d->head_dim == 128;
-    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0))
+    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0, with_noise != 0))
         return attn_decode_kernel_name(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, with_noise != 0);
     if (!with_noise) return attn_fwd16_kernel_name(d->head_dim, attn_fwd16_shape(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal != 0));
     trn_attn_desc n = *d;
@@ -941,7 +941,7 @@ int trn::attn_forward(const trn_attn_desc* d, const void* q, const void* k, cons
         }
     }
     // few queries per head (decode), or few query tiles in all: one workgroup per head and 32 queries, its waves split the keys
-    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, noise != nullptr)) {
+    if (attn_decode_suits(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, d->causal && !(sums && sums->n_slots > 0), noise != nullptr)) {
         if (sums && sums->n_slots > 0 && launch_add_slots(*sums, s) != hipSuccess) return TRN_E_LAUNCH;
         return launch_attn_decode(a, d->head_dim, workspace, workspace_bytes, s) == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
     }
