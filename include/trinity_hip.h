@@ -126,19 +126,20 @@ int trn_attn_qknorm_f16(const trn_attn_desc* desc, const void* q, const void* k,
  * caller-allocated tensor passed to `forward` (C, C_exp, C_sum ... in vanilla_llama_benchmark.py:42-77, zero-filled
  * by the driver, :237-240); this is that convention for the one intermediate these kernels have.  For decode shapes
  * (seq_q <= 32) with fewer than 128 heads on a long cache (4096 keys or more with at most 16 heads, 8192 or more
- * otherwise) the keys are then split over several workgroups per head, whose partial results and
- * arrival counters live in the workspace; for every other shape, or with workspace == NULL or too small, the call is
- * exactly trn_attn_fwd_f16.
+ * otherwise) the keys are then split over several workgroups per head, whose partial results (and, with noise,
+ * arrival counters) live in the workspace; for every other shape but the chunks below, or with workspace == NULL or too
+ * small, the call is exactly trn_attn_fwd_f16.
  *   workspace        device memory, 256-byte aligned, trn_attn_workspace_bytes(desc) bytes, zero-filled ONCE before
  *                    its first use (the kernel returns its counters to zero).  One call at a time may use it.
  * trn_attn_workspace_bytes returns 0 when the shape would not use a workspace.
  *
  * A chunk of more than 32 queries per head on a long cache has a workspace of its own, trn_attn_chunk_workspace_bytes(desc)
  * bytes (0: none), which needs no initial contents: the keys are then shared out over workgroups whose partial results a
- * second launch merges.  (Its first 512 bytes, where the split decode shapes keep their counters, are left alone: one
+ * second launch merges.  So have up to 32 queries without noise on caches of some 2000 keys and more (of many KV heads, up to 8000) for which
+ * trn_attn_workspace_bytes is 0.  (Its first 512 bytes, where the split decode shapes keep their counters, are left alone: one
  * zero-filled workspace of the larger size may serve both, one call at a time.)  Without it, or with a smaller one, the
- * call is trn_attn_fwd_f16 as above.  The size does not depend on seq_kv, so that a cache that grows from call to call keeps
- * its workspace, and never exceeds TRN_ATTN_CHUNK_WORKSPACE_MAX(head_dim) (256 shares of at most 128 queries): one workspace
+ * call is trn_attn_fwd_f16 as above.  The size does not depend on seq_kv (of up to 32 queries: by the shares' rounding alone), so that a
+ * cache that grows from call to call keeps its workspace, and never exceeds TRN_ATTN_CHUNK_WORKSPACE_MAX(head_dim) (256 shares of at most 128 queries): one workspace
  * of that size serves chunks of every length.
  */
 #define TRN_ATTN_CHUNK_WORKSPACE_MAX(head_dim) (512 + (int64_t)256 * 128 * ((head_dim) + 2) * 4)

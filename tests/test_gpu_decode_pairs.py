@@ -1,0 +1,57 @@
+"""GPU parity of up to 32 queries whose keys are shared out in two launches, on both sides of the lines from which they are: shares
+that see no key of a query, rows past the last query, workspaces with any contents.
+
+Tolerance against float64: a probability and an output are rounded to fp16 once each, by 2^-11 / sqrt(3) of their size in root mean square at
+most, 4.0e-4 in 2-norm; a row has up to twice that.  Row normalisers
+are sums of the rounded probabilities, of 2000 and more of scores of standard deviation 1: 2^-11 / sqrt(3) x sqrt(e / 2000) = 1.04e-5 in root mean
+square, asked for as six times that."""
+import pytest
+import torch
+
+from oracle import ref
+
+pytestmark = pytest.mark.gpu
+
+# B, Hq, Hkv, Sq, Skv, D, causal, shared out
+CASES = [
+    (1, 8, 2, 16, 2000, 128, False, True), (1, 8, 2, 16, 1999, 128, False, False), (1, 32, 8, 32, 2245, 128, True, True),      # (2245: a last share of five keys)
+    (1, 32, 32, 16, 2400, 128, True, True), (1, 32, 32, 16, 2399, 128, True, False), (1, 64, 8, 1, 3000, 128, True, True),
+    (1, 120, 8, 5, 2716, 128, True, True), (1, 120, 8, 5, 2715, 128, True, False), (1, 128, 8, 5, 4000, 128, False, False),
+    (1, 16, 16, 17, 2340, 64, True, True), (1, 16, 16, 17, 2339, 64, True, False), (1, 71, 1, 32, 2674, 64, True, True), (1, 71, 1, 32, 2673, 64, True, False),
+    (1, 71, 71, 2, 7854, 64, True, True), (1, 71, 71, 2, 7853, 64, True, False), (3, 32, 4, 3, 3588, 64, True, True), (3, 32, 4, 3, 3587, 64, True, False),
+    (2, 2, 1, 32, 3999, 128, True, True), (1, 8, 2, 33, 2500, 128, True, False),
+    (1, 8, 2, 16, 4100, 128, True, None), (1, 4, 4, 32, 9997, 128, True, None), (1, 16, 4, 1, 12000, 64, True, None), (1, 71, 1, 9, 8193, 64, False, None),      # (their own workspace)
+]
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,shared", CASES)
+def test_keys_shared_out_in_two_launches(B, Hq, Hkv, Sq, Skv, D, causal, shared):
+    from triton_amd import ops
+    g = torch.Generator().manual_seed(Skv)
+    q, k, v = (ref.randn_half((B, h, s, D), g).cuda() for h, s in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    scale = D ** -0.5
+    o, plain = torch.full((B, Hq, 40, D), 7.0, dtype=torch.half, device="cuda"), torch.empty_like(q)
+    need = ops.attention_chunk_workspace_bytes(q, k, v, plain, scale, causal)
+    if shared is None:
+        assert need == 0
+        need = ops.attention_workspace_bytes(q, k, v, plain, scale, causal)
+    assert (need > 0) == (shared is not False)
+    ws = torch.full((max(need, 1024) + 512,), 255, dtype=torch.uint8, device="cuda")       # (NaN)
+    lse, lse1 = torch.zeros(B, Hq, Sq, device="cuda"), torch.zeros(B, Hq, Sq, device="cuda")
+    ops.attention(q, k, v, o[:, :, :Sq], scale, causal, lse=lse, workspace=ws)
+    ops.attention(q, k, v, plain, scale, causal, lse=lse1)
+    assert (ws[:256] == 255).all() and (ws[max(need, 1024):] == 255).all() and (o[:, :, Sq:] == 7).all()
+    assert (ws[512:need] != 255).any() == (shared is not False)
+    small = torch.full((max(need - 256, 256),), 255, dtype=torch.uint8, device="cuda")
+    again = torch.empty_like(q)
+    ops.attention(q, k, v, again, scale, causal, workspace=small)
+    assert torch.equal(again, plain) and (small == 255).all()
+    mask = torch.ones(Sq, Skv, dtype=torch.bool, device="cuda").triu(Skv - Sq + 1)
+    for b, h in {(0, 0), (B - 1, Hq - 1), (B // 2, Hq // 2)}:
+        s = q[b, h].double() @ k[b, h * Hkv // Hq].double().t() * scale
+        if causal:
+            s = s.masked_fill(mask, float("-inf"))
+        want = s.softmax(1) @ v[b, h * Hkv // Hq].double()
+        rows = (o[b, h, :Sq] - want).norm(dim=1) / want.norm(dim=1)
+        assert (o[b, h, :Sq] - want).norm() <= 4e-4 * want.norm() and rows.max() <= 8e-4, (rows.max(), rows.argmax())
+        assert ((lse[b, h] - s.logsumexp(1)).abs() <= 6.2e-5).all() and ((lse1[b, h] - s.logsumexp(1)).abs() <= 6.2e-5).all()

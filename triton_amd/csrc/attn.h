@@ -23,7 +23,7 @@ struct AttnArgs {
     const half_t* gamma_k; float k_eps; int k_norm;     // decode kernel without noise only: the keys are normalised on arrival
     // decode kernel only: keys split over n_split workgroups per head, partial results and arrival counters in ws
     int n_split;
-    int partial;   // ... which the next launch merges
+    int partial;   // ... which the next launch merges (2: of the queries there are alone)
     int spread;    // decode kernel only: the query tiles of a head go to all XCDs
     float* ws;
     // decode kernel only, at most 32 queries: per-key sums (and sums of squares) of the probabilities -- of the
@@ -182,6 +182,7 @@ bool attn_decode_norms_keys(int batch, int n_q_heads, int seq_q, int seq_kv, int
 const char* attn_decode_kernel_name(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 // Bytes of workspace with which launch_attn_decode splits the keys of this problem over several workgroups (0: it would not).
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim);
+int64_t attn_few_query_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim);      // ... where that is 0, for two launches
 
 // ... and of that with which it does for key statistics, merged and summed up by a second launch.
 int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);

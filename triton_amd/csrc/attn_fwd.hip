@@ -677,6 +677,7 @@ extern "C" int64_t trn_attn_workspace_bytes(const trn_attn_desc* d) {
 extern "C" int64_t trn_attn_chunk_workspace_bytes(const trn_attn_desc* d) {
     using namespace trn;
     if (!d || validate_attn(d, true) != TRN_OK) return 0;
+    if (d->seq_q <= 32) return attn_few_query_workspace_bytes(d->batch, d->n_q_heads, d->n_kv_heads, d->seq_q, d->seq_kv, d->head_dim);
     return attn_share_workspace_bytes(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim);
 }
 

@@ -176,8 +176,8 @@ def attention_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> int:
 
 
 def attention_chunk_workspace_bytes(q, k, v, o, scale: float, causal: bool) -> int:
-    """Bytes of workspace (no initial contents) with which `attention` would share out the keys of a chunk of more than 32
-    queries over workgroups (0: it would not).  chunk_workspace_max(head_dim) bytes serve chunks of every length."""
+    """Bytes of workspace (no initial contents) with which `attention` would share out the keys of a chunk of queries, or of
+    up to 32 where attention_workspace_bytes is 0, over workgroups (0: it would not).  chunk_workspace_max(head_dim) bytes serve chunks of every length."""
     d = _attn_desc(q, k, v, o, scale, causal, False, 0.0, None, 1.0)
     return int(_lib.load().trn_attn_chunk_workspace_bytes(C.byref(d)))
 
