@@ -75,7 +75,8 @@ def test_rule(H, D, noise, keys):
 
 # the shares by the statistics' rule, by that of the plain attention's workspace too (4112 keys, 16 heads), and none of either
 @pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", [(1, 8, 8, 128, 8, 4112), (1, 16, 16, 64, 5, 4112), (1, 8, 2, 128, 32, 8193), (1, 100, 10, 64, 17, 9000),
-                                              (1, 2, 1, 64, 1, 2049), (1, 8, 8, 128, 8, 700)])
+                                              (1, 2, 1, 64, 1, 2049), (1, 8, 8, 128, 8, 700),
+                                              (1, 32, 32, 128, 3, 3800), (1, 5, 5, 64, 9, 7001)])        # six shares of eight, sixteen of 32
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("half", [False, True])
 def test_mean_and_deviation_of_shared_out_keys(B, H, Hkv, D, Sq, Skv, causal, half):

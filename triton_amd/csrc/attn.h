@@ -187,7 +187,7 @@ int64_t attn_few_query_workspace_bytes(int batch, int n_q_heads, int n_kv_heads,
 // ... and of that with which it does for key statistics, merged and summed up by a second launch.
 int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise);
 // ... over how many workgroups a head with a workspace of so many bytes (0: the statistics are part of a single launch).
-int attn_decode_stat_shares(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes);
+int attn_decode_stat_shares(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes);
 
 // Device address, on the current device, of the library's static scratch array (TRN_ATTN_NOALLOC_SCRATCH_BYTES bytes)
 // behind trn_attn_fwd_noalloc_f16; looked up once per device.  nullptr if the runtime refuses.

@@ -843,11 +843,21 @@ static int stats_splits(int batch, int n_q_heads, int seq_q, int seq_kv, int hea
 int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
     return split_bytes((int64_t)batch * n_q_heads, stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), head_dim);
 }
-// ... that a workspace holds: with the plain attention's, as many as that has.
-int attn_decode_stat_shares(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes) {
+// ... that a workspace holds: with the plain attention's, as many as that has; but sixteen at most, and not many more than 192 that read keys of
+// their own, of 3 to 32 heads.  us of a decode step of one token, as many as stats_splits() / 24 / 16 / 12 / 8 / 6 / 4: KeyFormer, 8 heads of 128: 4500 keys (32) 23.1 /
+// 23.2 / 23.1 / 23.4, 10000 33.0 / 29.9 / 28.4 / 29.6, 15000 37.9 / 34.1 / 34.1 / 36.3; 16 of 64 (16): 4500 21.4 / - / - / 19.9 / 20.6, 15000 32.6 / - / - / 32.3 / 34.1; 32 of
+// 128 (8): 3200 51.0 / - / - / - / - / 47.5 / 47.0, 10000 76.0 / - / - / - / - / 73.8 / 73.4; RoCo, 8 of 128: 10000 32.6 / 29.0 / 27.2 / 28.1 / 31.3.
+// Left out: 2 of 128, KeyFormer, 10000 22.3 / - / 23.2; 4, 15000 27.2 / - / 30.7; 40 of 64 (6 / 4 shares), 10000 45.8 / 47.5.
+int attn_decode_stat_shares(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes) {
     if (seq_q > 32) return 0;
+    const int nblk = (seq_kv + 31) / 32;
     for (const int ns : {stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), decode_splits(batch, n_q_heads, seq_kv, head_dim)})
-        if (ns > 1 && split_bytes((int64_t)batch * n_q_heads, ns, head_dim) <= workspace_bytes) return ns;
+        if (ns > 1 && split_bytes((int64_t)batch * n_q_heads, ns, head_dim) <= workspace_bytes) {
+            const int n_bh = batch * n_q_heads, n_bkv = batch * n_kv_heads;
+            const int cap = n_bkv > 32 || n_bh <= 2 || (n_bh <= 4 && seq_kv >= 12000) ? ns : min(16, 192 / n_bkv);
+            const int n = min(ns, cap), bps = (nblk + n - 1) / n;
+            return (nblk + bps - 1) / bps;
+        }
     return 0;
 }
 
@@ -927,7 +937,7 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
         }
     }
     const int stat_shares = workspace && (a.col_sum || a.col_sumsq) && !a.probs && !a.k_norm ?
-        attn_decode_stat_shares(a.B, a.Hq, a.Sq, a.Skv, head_dim, a.noise != nullptr, workspace_bytes) : 0;
+        attn_decode_stat_shares(a.B, a.Hq, a.Hkv, a.Sq, a.Skv, head_dim, a.noise != nullptr, workspace_bytes) : 0;
     if (a.mean_std && stat_shares == 0) return hipErrorInvalidValue;      // (the single launch has the sums only)
     if (stat_shares > 0) {
         a.n_split = stat_shares; a.ws = static_cast<float*>(workspace); a.partial = 1; a.n_qtiles = 1;

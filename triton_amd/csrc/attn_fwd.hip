@@ -838,7 +838,7 @@ extern "C" int trn_attn_key_scores_f16(const trn_attn_desc* d, const void* q, co
     // mean and deviation of a handful of queries: by the launch that merges the key shares; elsewhere the workspace stays
     // out of it (the plain attention would split the keys by counters in it that have to be zero)
     if (d->seq_q <= 32) {
-        if (workspace && attn_decode_stat_shares(d->batch, d->n_q_heads, d->seq_q, d->seq_kv, d->head_dim, false, workspace_bytes) > 0)
+        if (workspace && attn_decode_stat_shares(d->batch, d->n_q_heads, d->n_kv_heads, d->seq_q, d->seq_kv, d->head_dim, false, workspace_bytes) > 0)
             return attn_forward(d, q, k, v, o, lse, nullptr, n, lse_pert, workspace, workspace_bytes, s1, s2, stream, nullptr, n16, s16, true, false, nullptr, 0.f, true);
         workspace = nullptr; workspace_bytes = 0;
     }
