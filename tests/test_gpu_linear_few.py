@@ -1,4 +1,4 @@
-"""GPU parity of LoRA and the gated MLP of at most 32 tokens on little weight, which are one launch each: partial panels, ranks around
+"""GPU parity of LoRA and the gated MLP of few tokens on little weight, which are one launch each: partial panels, ranks around
 the blocks of 32, depths around the turns of eight waves and around the lines between one launch and two, rows at a pitch.
 
 Tolerance: fp16 operands, fp32 sums, every product rounded to fp16 (2^-11 of itself): LoRA's output is the sum of two roundings and its
@@ -71,3 +71,14 @@ def test_no_numbers_stay_in_their_token(T):
     assert torch.equal(o.isfinite(), want.isfinite()) and o.isfinite().sum() == (T - 1) * P
     keep = [t for t in range(T) if t != 3]
     close(o[keep], want[keep].double())
+
+
+@pytest.mark.parametrize("T,K,P,R,pad", [(34, 512, 1000, 16, 0), (64, 1512, 1256, 64, 8), (65, 40, 24, 8, 0), (512, 264, 512, 24, 8), (513, 264, 512, 24, 0), (63, 704, 520, 128, 0),
+                                         (70, 328, 2848, 16, 0), (1024, 1000, 504, 32, 8), (1025, 40, 504, 32, 0), (96, 4096, 200, 40, 0), (97, 4104, 200, 40, 0)])
+def test_lora_in_tiles_of_tokens(T, K, P, R, pad):
+    test_lora(T, K, P, R, pad)
+
+
+@pytest.mark.parametrize("T,K,N,pad", [(34, 424, 288, 0), (64, 1352, 3024, 8), (65, 8, 8, 0), (512, 384, 416, 8), (513, 384, 416, 0), (95, 4096, 640, 0), (33, 40, 4096, 0), (64, 3072, 40, 0), (64, 3080, 40, 0)])
+def test_gated_mlp_in_tiles_of_tokens(T, K, N, pad):
+    test_gated_mlp(T, K, N, pad, "silu" if T % 2 else "sigmoid")

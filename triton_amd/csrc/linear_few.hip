@@ -1,4 +1,4 @@
-// LoRA and the gated MLP of at most 32 tokens on little weight in one launch:
+// LoRA and the gated MLP of few tokens on little weight in one launch:
 //
 //     O = X W + (X A) B        O = gate(X W1) * (X W2)
 //
@@ -39,18 +39,20 @@ __global__ __launch_bounds__(512, 2) void linear_few_kernel(const FewArgs a) {
     const int id = blockIdx.x, panel = 16 * (id >> 4) + 2 * (id & 7) + ((id >> 3) & 1);
     if (panel >= a.n_panels) return;
     const int n0 = 32 * panel, nkt = (a.K + 31) / 32;
+    const int64_t t0 = (int64_t)blockIdx.y * (16 * TB);                // (the token tiles of a panel are on one XCD as well)
+    const int T = min((int)(a.T - t0), 16 * TB);
     constexpr int kOut = 0x7ffffff0;                 // a byte offset past every buffer: the load returns zeros
     auto rows_of = [](const half_t* p, int64_t rows, int64_t pitch, int64_t cols) __attribute__((always_inline)) {
         return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(((rows - 1) * pitch + cols) * 2), 0x00020000);
     };
-    const __amdgpu_buffer_rsrc_t xrs = rows_of(a.x, a.T, a.ldx, a.K), wrs = rows_of(a.w, a.K, a.ldw, a.n);
+    const __amdgpu_buffer_rsrc_t xrs = rows_of(a.x + t0 * a.ldx, T, a.ldx, a.K), wrs = rows_of(a.w, a.K, a.ldw, a.n);
     const __amdgpu_buffer_rsrc_t ars = rows_of(a.a, a.K, a.lda, GATE ? a.n : a.r);
     const int wr = lane >> 2, wc = lane & 3, ar = lane / CPR, ac = lane % CPR;
     const int w_pitch = (int)a.ldw * 2, a_pitch = (int)a.lda * 2, acol = (GATE ? n0 : 0) + 8 * ac;
     const int w_vo = wr * w_pitch + (n0 + 8 * wc) * 2, a_vo = acol < (GATE ? a.n : a.r) ? ar * a_pitch + acol * 2 : kOut;
     int x_vo[TB];
 #pragma unroll
-    for (int i = 0; i < TB; ++i) x_vo[i] = 16 * i + wr < a.T ? (int)((16 * i + wr) * a.ldx * 2) + wc * 16 : kOut;
+    for (int i = 0; i < TB; ++i) x_vo[i] = 16 * i + wr < T ? (int)((16 * i + wr) * a.ldx * 2) + wc * 16 : kOut;
 
     // (unconditional, past the end as zeros: a load that may not be issued counts as absent when the compiler sizes its waits)
     half8_t wreg[PD][2], areg[PD][AL], xreg[PD][TB], breg;
@@ -175,7 +177,7 @@ __global__ __launch_bounds__(512, 2) void linear_few_kernel(const FewArgs a) {
             o = (half_t)((float)(half_t)q + (float)(half_t)sum[tb][0]);
         }
         const int t = 16 * tb + c;
-        if (t < a.T && n0 + col < a.n) a.o[t * a.ldo + n0 + col] = o;
+        if (t < T && n0 + col < a.n) a.o[(t0 + t) * a.ldo + n0 + col] = o;
     }
 #endif
 }
@@ -192,8 +194,21 @@ __global__ __launch_bounds__(512, 2) void linear_few_kernel(const FewArgs a) {
 //   gated MLP       16 tokens: 1024 -> 1024 6.2 / 4.6, 1024 -> 4096 7.1 / 6.2, 1280 -> 4096 8.3 / 8.1, 1640 -> 2008 9.6 / 9.5, 1800 -> 1000 9.2 / 9.0; but 1536 ->
 //                   4096 8.9 / 9.1, 2048 -> 2048 8.9 / 9.5, 2200 -> 1000 10.2 / 10.8 (rows at odd half lines; 2400 -> 1024 7.4 / 6.8)
 //                   32 tokens: 1024 -> 4096 7.7 / 7.4, 1088 -> 2008 8.9 / 7.8, 1280 -> 1000 8.7 / 8.3; but 1200 -> 1400 7.9 / 8.6, 1280 -> 4096 8.8 / 9.5
+// More than 32 tokens are tiles of 32, of which every CU has one at most (a panel's read its weights from the same L2): the two launches then
+// take several us longer, and only all of A for a large rank makes up for it.  Ranks of up to 32 on little depth bear two a CU.
+//   LoRA, rank 8 to 24   53 tokens, 328 x 272 8.0 / 4.9; 72, 1064 x 272 11.3 / 6.1; 145, 3816 x 328 25.4 / 15.0; 401, 576 x 432 10.6 / 5.6; 76, 688 x 2064 10.9 / 6.0; two a CU:
+//                        71, 328 x 2848 10.2 / 7.6, 497, 568 x 816 11.1 / 9.5, 178, 968 x 1904 12.8 / 11.3; but 361, 1984 x 824 17.3 / 17.8, 449, 712 x 1240 (720 tiles) 12.1 / 14.1
+//   rank 33 to 64        62 tokens, 512 x 1000 8.3 / 5.1; 177, 2984 x 448 16.1 / 14.4; 55, 1512 x 1256 11.1 / 10.6; 36, 4064 x 576 14.0 / 16.0; two a CU 317, 672 x 1056 10.8 / 12.4
+//   rank 65 to 128       52 tokens, 304 x 784 8.5 / 6.7; 180, 472 x 504 10.4 / 7.5; 149, 656 x 1160 10.9 / 9.5; but 36, 824 x 512 8.6 / 9.1, 118, 2712 x 360 16.1 / 17.8
+//   gated MLP            50 tokens, 424 -> 288 6.4 / 4.8; 88, 4000 -> 640 18.5 / 16.6; 47, 1352 -> 3024 12.9 / 10.2; 34, 4064 -> 728 17.8 / 18.6; 476, 384 -> 416 7.5 / 5.2; two a CU 365, 488 -> 608 7.7 / 8.8,
+//                        82, 1264 -> 3248 13.2 / 16.7
 static bool few_suits(int64_t tokens, int64_t hidden, int64_t n, int64_t rank, bool gate) {
-    if (tokens > 32 || n > 4096) return false;
+    if (n > 4096) return false;
+    if (tokens > 32) {
+        const int64_t tiles = (n + 511) / 512 * 16 * ((tokens + 31) / 32);      // (as launch_few() has them)
+        const int64_t deep = tokens <= 64 && (gate || rank > 32) ? 3072 : 4096;
+        return hidden <= deep && (tiles <= 256 ? gate || rank <= 64 || (rank <= 128 && hidden <= 704) : !gate && rank <= 32 && hidden <= 1000 && tiles <= 512);
+    }
     const bool one = tokens <= 16;
     if (gate) return hidden <= (n <= 1024 ? (one ? 1800 : 1280) : n <= 2048 ? (one ? 1600 : 1088) : (one ? 1280 : 1024));
     return hidden <= (rank <= 32 ? (one ? 3584 : 2560) : rank <= 64 ? (one ? 1448 : 1088) : rank <= 128 ? (one ? 704 : 448) : 0);
@@ -202,7 +217,7 @@ static bool few_suits(int64_t tokens, int64_t hidden, int64_t n, int64_t rank, b
 template <int NR, int PD, bool GATE>
 static int launch_few(FewArgs a, hipStream_t stream) {
     a.n_panels = (a.n + 31) / 32;
-    const dim3 g((unsigned)((a.n_panels + 15) / 16 * 16)), t(512);
+    const dim3 g((unsigned)((a.n_panels + 15) / 16 * 16), (unsigned)((a.T + 31) / 32)), t(512);
     if (a.T <= 16) hipLaunchKernelGGL((linear_few_kernel<NR, 1, PD, GATE>), g, t, 0, stream, a);
     else hipLaunchKernelGGL((linear_few_kernel<NR, 2, PD, GATE>), g, t, 0, stream, a);
     return hipGetLastError() == hipSuccess ? TRN_OK : TRN_E_LAUNCH;
