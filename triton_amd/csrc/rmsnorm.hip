@@ -1,12 +1,12 @@
 // RMSNorm over rows of fp16 data: one pass, the row held in registers between the mean-square
-// reduction and the scale.  HBM-bound: 16-byte loads, LPR lanes cooperate on one row and reduce
-// with cross-lane shuffles; rows*cols*2 bytes read, the same written.
+// reduction and the scale.  HBM-bound (few rows: the latency of a row's loads): 16-byte loads, LPR lanes cooperate on one row and reduce
+// with cross-lane shuffles, of four waves through LDS; rows*cols*2 bytes read, the same written.
 #include <type_traits>
 #include "common.h"
 
 namespace trn {
 
-// LPR lanes per row (power of two <= 64), NV 16-byte vectors per lane.  All of a row's loads are issued before the first is
+// LPR lanes per row (power of two <= 64, or the workgroup's 256), NV 16-byte vectors per lane.  All of a row's loads are issued before the first is
 // waited for (with the squares summed in the same loop the compiler waited for each vector in turn); EARLY: gamma's too.
 template <int LPR, int NV, bool EARLY>
 __global__ __launch_bounds__(256) void rmsnorm_kernel(
@@ -44,7 +44,13 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(
         }
     }
 #pragma unroll
-    for (int m = LPR / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    for (int m = (LPR < 64 ? LPR : 64) / 2; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+    if constexpr (LPR == 256) {
+        __shared__ float part[4];
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = (part[0] + part[1]) + (part[2] + part[3]);
+    }
     const float rstd = 1.0f / __builtin_sqrtf(ss / (float)cols + eps);
 
 #pragma unroll
@@ -77,7 +83,7 @@ static hipError_t launch_form(const void* x, const void* gamma, void* y, int64_t
     return hipGetLastError();
 }
 
-// gamma early or late: early is one memory latency instead of two for a row, late leaves the queue to the rows themselves, which
+// gamma early or late, of a wave's rows: early is one memory latency instead of two for a row, late leaves the queue to the rows themselves, which
 // matters once the resident waves ask for more than the chip takes at a time.  us, before / late / early: 16 x 4096 5.1 / 4.6 /
 // 3.9, 396 x 5560 10.4 / 6.7 / 5.4, 300 x 8192 13.3 / 7.9 / 6.2, 1929 x 3216 8.6 / 6.7 / 6.4, 3072 x 4096 11.1 / 9.6 / 8.8, 3400 x
 // 4096 11.7 / 10.7 / 12.2, 4096 x 4096 12.8 / 11.4 / 12.5; 1900 x 8192 17.2 / 12.3 / 11.2, 3072 x 6000 17.8 / 14.7 / 14.3, 2500 x
@@ -92,7 +98,7 @@ static hipError_t launch(const void* x, const void* gamma, void* y, int64_t n_ro
                          int cols, int64_t xo, int64_t ldx, int64_t yo, int64_t ldy, int64_t row_start,
                          float eps, hipStream_t s) {
     auto form = [&](auto early) { return launch_form<LPR, NV, decltype(early)::value>(x, gamma, y, n_rows, inner_rows, cols, xo, ldx, yo, ldy, row_start, eps, s); };
-    if constexpr (NV == 1 || NV == 4) return form(std::true_type{});
+    if constexpr (NV == 1 || NV == 4 || LPR == 256) return form(std::true_type{});
     else if constexpr (NV == 32) return form(std::false_type{});        // (gamma's 32 vectors beside the row's: registers)
     else {
         const int64_t bytes = n_rows * cols * 2;
@@ -122,12 +128,20 @@ extern "C" int trn_rmsnorm_f16(const void* x, const void* gamma, void* y, int64_
     hipStream_t s = (hipStream_t)stream;
     const int vecs = (int)(cols / 8);
     hipError_t e;
+    // Few long rows: a workgroup has one, whose loads are a quarter as many a lane, instead of four waves one each.  us, wave / workgroup:
+    // 1 x 2048 2.60 / 2.22, 64 x 4096 3.88 / 2.59, 1 x 8192 4.68 / 2.91, 200 x 8192 5.89 / 3.99, 64 x 16384 13.2 / 4.2, 400 x 1032 2.97 / 2.95, 400 x 3072 4.44 / 3.34; 1200 x 2048
+    // 4.51 / 4.02, 1200 x 4104 6.33 / 5.59, 1200 x 12000 14.3 / 13.7; left out: 800 x 1032 3.18 / 3.24, 2048 x 4096 6.40 / 6.93, 1600 x 8192 9.93 / 10.93, 3000 x 2048 5.39 / 6.32.
+    const bool spread = vecs > 128 && n_rows <= (vecs < 160 ? 400 : 1200);
 #define TRN_RMS(LPR, NV) e = launch<LPR, NV>(x, gamma, y, n_rows, inner_rows, (int)cols, x_outer_stride, ldx, y_outer_stride, ldy, row_start, eps, s)
     if (vecs <= 8) TRN_RMS(8, 1);
     else if (vecs <= 16) TRN_RMS(16, 1);
     else if (vecs <= 32) TRN_RMS(32, 1);
     else if (vecs <= 64) TRN_RMS(64, 1);
     else if (vecs <= 128) TRN_RMS(64, 2);
+    else if (spread && vecs <= 256) TRN_RMS(256, 1);
+    else if (spread && vecs <= 512) TRN_RMS(256, 2);
+    else if (spread && vecs <= 1024) TRN_RMS(256, 4);
+    else if (spread) TRN_RMS(256, 8);
     else if (vecs <= 256) TRN_RMS(64, 4);
     else if (vecs <= 512) TRN_RMS(64, 8);
     else if (vecs <= 1024) TRN_RMS(64, 16);
