@@ -55,3 +55,53 @@ def test_keys_shared_out_in_two_launches(B, Hq, Hkv, Sq, Skv, D, causal, shared)
         rows = (o[b, h, :Sq] - want).norm(dim=1) / want.norm(dim=1)
         assert (o[b, h, :Sq] - want).norm() <= 4e-4 * want.norm() and rows.max() <= 8e-4, (rows.max(), rows.argmax())
         assert ((lse[b, h] - s.logsumexp(1)).abs() <= 6.2e-5).all() and ((lse1[b, h] - s.logsumexp(1)).abs() <= 6.2e-5).all()
+
+
+# head_dim 64, as many KV heads, three shares: around the line of the launches without a workspace of their own (2600 + 74 x heads) and the
+# 8192 keys from which that workspace is there: B, H, Sq, Skv
+@pytest.mark.parametrize("B,H,Sq,Skv", [(1, 80, 2, 8192), (1, 80, 2, 8519), (1, 80, 2, 8520), (1, 76, 32, 8192), (1, 76, 1, 8224), (1, 85, 1, 8192), (1, 85, 1, 8889),
+                                        (1, 85, 1, 8890), (5, 16, 16, 8519), (5, 16, 3, 8191)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_what_the_workspace_held_before_does_not_matter(B, H, Sq, Skv, causal):
+    """The workspace as allocated (zeros), full of NaN, with another call's shares in it, and the library's own after another call."""
+    import ctypes as C
+    from triton_amd import _lib, ops
+    g = torch.Generator().manual_seed(Skv + H)
+    D, scale = 64, 0.125
+    q, k, v = (ref.randn_half((B, H, s, D), g).cuda() for s in (Sq, Skv, Skv))
+    o = torch.zeros_like(q)
+    need = ops.attention_workspace_bytes(q, k, v, o, scale, causal)
+    assert (need > 0) == (Skv >= 8192)
+    ws = torch.zeros(max(need, ops.attention_chunk_workspace_bytes(q, k, v, o, scale, causal), 256), dtype=torch.uint8, device="cuda")
+    lib = _lib.load()
+
+    def call(how, q, k, v, o, lse):
+        if how != "own":
+            return ops.attention(q, k, v, o, scale, causal, lse=lse, workspace=ws)
+        d = ops._attn_desc(q, k, v, o, scale, causal, False, 0.0, None, 1.0)
+        st = lib.trn_attn_fwd_noalloc_f16(C.byref(d), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), None, None, None,
+                                          torch.cuda.current_stream().cuda_stream)
+        assert st == 0
+
+    heads = [(0, 0), (B - 1, H - 1), (B // 2, H // 2)]
+    mask = torch.ones(Sq, Skv, dtype=torch.bool, device="cuda").triu(Skv - Sq + 1)
+    want = {}
+    for b, h in heads:
+        s = q[b, h].double() @ k[b, h].double().t() * scale
+        if causal:
+            s = s.masked_fill(mask, float("-inf"))
+        want[b, h] = s.softmax(1) @ v[b, h].double(), s.logsumexp(1)
+    first = None
+    for how in ("zeros", "nan", "used", "own"):
+        if how == "nan":
+            ws.fill_(255)
+        elif how in ("used", "own"):                    # another problem's results in the same places: keys twice as large, other values
+            call(how, q, k * 2, v + 8, torch.zeros_like(q), torch.zeros(B, H, Sq, device="cuda"))
+        o, lse = torch.full_like(q, 7.0), torch.full((B, H, Sq), 7.0, device="cuda")
+        call(how, q, k, v, o, lse)
+        for at in heads:
+            w, l = want[at]
+            assert (o[at] - w).norm() <= 4e-4 * w.norm() and ((lse[at] - l).abs() <= 6.2e-5).all(), how
+        if need > 0:                                    # (the library's own serves the same shares)
+            first = first or (o, lse)
+            assert torch.equal(o, first[0]) and torch.equal(lse, first[1]), how

@@ -11,6 +11,7 @@
 // loop has no barrier; every load is issued unconditionally (blocks past the end read zeros, which are masked) so
 // that the waits can be counted.
 #include "attn.h"
+#include "attn_decode_rules.h"
 #include <mutex>
 #include <type_traits>
 
@@ -714,50 +715,11 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #endif
 }
 
-// Key shares that trn_attn_workspace_bytes has room for, and as many as one launch with score perturbation has, whose workgroup that
-// arrives last at a head's counter collects the others' results (4 - 5 us and more for more shares).  Measured with 16 queries per
-// head, unsplit / split, us: 32 heads of 128: 2064 keys 13.9 / 22.2, 4112 keys 21.5 / 27.1, 8208 keys 36.7 / 35.8, 16400 keys 69 / 57, 65552
-// keys 406 / 198; 8 heads of 128: 4112 keys 20.0 / 18.1, 8208 keys 35 / 22, 65552 keys 232 / 59; 71 heads of 64: 4112 keys 14.1 / 14.5, 8208
-// keys 23.9 / 18.9.  Hence: from 4096 keys with at most 16 heads, from 8192 with more, never with 128 heads or more.  The caller provides
-// the workspace.
-static int decode_splits(int batch, int n_q_heads, int seq_kv, int head_dim) {
-    const int n_bh = batch * n_q_heads, nblk = (seq_kv + 31) / 32;
-    (void)head_dim;
-    if (n_bh >= 128 || seq_kv < (n_bh <= 16 ? 4096 : 8192)) return 1;
-    const int ns = max(1, min(min(16, 256 / n_bh), nblk / 4));
-    const int bps = (nblk + ns - 1) / ns;                 // blocks per share, as the kernel computes it
-    return (nblk + bps - 1) / bps;                        // no empty share: the last one starts inside the keys
-}
-
-// Key shares of up to 32 queries in two launches, the second of which adds the shares up (attn_decode_merge_kernel): some 3 us more than a
-// launch without shares, against 5 to 7 for arriving and collecting in one, and hardly more for more shares.  Eight of them, or one
-// workgroup per CU in all, or some 144 that read keys of their own, which are what the memory takes; sixteen where few heads have many
-// keys.  us, 16 queries per head, K and V from beyond the L2s, unsplit / 2 / 4 / 6 / 8 / 16 shares (in brackets: arriving and collecting, as many as
-// decode_splits()):
-//   128, 8 heads: 1500 keys 11.3 / 14.4 / 12.0 / 11.9 / 11.3, 2200 14.3 / 16.3 / 13.3 / 12.2 / 11.9, 4200 21.5 / 21.7 / 16.3 / 14.7 / 13.6 / 13.6 (18.1), 16000 66 / 53 / 33 / 25.6 / 22.7
-//       / 20.4; 32 on 8 KV heads: 1900 12.7 / 15.7 / 13.2 / 12.2 / 12.2, 4200 21.7 / 21.5 / 16.2 / 14.9 / 14.0, 16000 67 / 53 / 33 / 26.3 / 24.5 (26.7); 120 on 8: 2600 18.6 / 18.4,
-//       8300 46 / 35 (37.7)
-//     24: 1900 12.7 / 16.0 / 13.6 / 13.1, 2200 15.0 / 16.7 / 13.7 / 13.5 / 14.6; 32: 2200 15.2 / 16.6 / 14.5 / 15.3 / 17.3, 4200 22.7 / 22.3 / 18.9 / 19.7 / 21.5, 16000 104 / 86 / 55 / 51 / 52;
-//       40: 2600 16.8 / 18.2 / 17.4, 3000 18.9 / 19.6 / 18.2; 64 (three): 3500 24.9 / 25.7, 4200 31.9 / 29.2; 96: 4200 43.4 / 43.7, 5000 52.3 / 50.9
-//   64, 16: 1900 8.9 / 11.3 / 9.8 / 9.3 / 9.6, 2200 10.2 / 11.3 / 9.8 / 9.4 / 9.6, 4200 14.8 / 14.5 / 11.7 / 11.0 / 10.8 / 12.6 (15.3), 16000 45 / 34 / 22 / 17.4 / 17.1 / 19.2; 32: 2600
-//       11.1 / 12.3 / 11.4 / 11.5, 3000 12.5 / 13.3 / 11.7 / 11.6 / 12.7; 48: 3000 12.9 / 13.5 / 13.2, 3500 14.5 / 14.5 / 14.0; 71 (three): 6000 21.8 / 22.8, 8000 39.4 / 28.4; on
-//       one KV head 2600 11.1 / 11.0, 6000 19.8 / 15.3; 100 (two): 5000 25.1 / 26.0, 6000 37.4 / 30.7; 96 on 8: 3000 12.3 / 12.4, 3500 13.8 / 13.2
-static int pair_shares(int n_bh, int n_bkv, int seq_kv, int head_dim) {
-    if (n_bh >= 128) return 1;
-    const int nblk = (seq_kv + 31) / 32, most = 256 / n_bh;
-    const int from = head_dim == 128 ? (most == 2 ? 2500 + 27 * n_bkv : 2000 + 50 * max(0, n_bkv - 24))
-                                     : most == 2 ? 3300 + 24 * n_bkv : most == 3 ? 2600 + 74 * n_bkv : 2200 + 35 * max(0, n_bkv - 12);
-    if (seq_kv < from) return 1;
-    const bool many = n_bh <= 8 ? (int64_t)seq_kv * head_dim >= 5000 * 128 : n_bh <= 16 && head_dim == 128 && seq_kv >= 10000;
-    const int ns = min(min(many ? 16 : 8, most), max(3, 144 / n_bkv)), bps = (nblk + ns - 1) / ns;      // (blocks per share, as the kernel computes it)
-    return (nblk + bps - 1) / bps;
-}
-
 // Arrival counters and the shares' partial results.
 static int64_t split_bytes(int64_t n_bh, int ns, int head_dim) { return ns <= 1 ? 0 : ((n_bh + 63) / 64) * 256 + n_bh * ns * 32 * (head_dim + 4) * 4; }
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
     if (seq_q > 32) return 0;
-    const int ns = decode_splits(batch, n_q_heads, seq_kv, head_dim);
+    const int ns = decode_splits(batch * n_q_heads, seq_kv);
     if (ns <= 1) return 0;
     const int64_t n_bh = (int64_t)batch * n_q_heads;
     return split_bytes(n_bh, ns, head_dim);
@@ -765,9 +727,8 @@ int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq
 
 // The shares' partial results alone, of two launches below that rule's lines.
 int64_t attn_few_query_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim) {
-    if (seq_q > 32 || decode_splits(batch, n_q_heads, seq_kv, head_dim) > 1) return 0;
-    const int ns = pair_shares(batch * n_q_heads, batch * n_kv_heads, seq_kv, head_dim);
-    return split_bytes((int64_t)batch * n_q_heads, ns, head_dim);
+    if (seq_q > 32 || decode_splits(batch * n_q_heads, seq_kv) > 1) return 0;
+    return split_bytes((int64_t)batch * n_q_heads, few_query_shares(batch * n_q_heads, batch * n_kv_heads, seq_kv, head_dim), head_dim);
 }
 
 // Column shares of a head for `units` = heads x query tiles: as many as leave 32 columns per workgroup and at most one
@@ -851,7 +812,7 @@ int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, i
 int attn_decode_stat_shares(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes) {
     if (seq_q > 32) return 0;
     const int nblk = (seq_kv + 31) / 32;
-    for (const int ns : {stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), decode_splits(batch, n_q_heads, seq_kv, head_dim)})
+    for (const int ns : {stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), decode_splits(batch * n_q_heads, seq_kv)})
         if (ns > 1 && split_bytes((int64_t)batch * n_q_heads, ns, head_dim) <= workspace_bytes) {
             const int n_bh = batch * n_q_heads, n_bkv = batch * n_kv_heads;
             const int cap = n_bkv > 32 || n_bh <= 2 || (n_bh <= 4 && seq_kv >= 12000) ? ns : min(16, 192 / n_bkv);
@@ -922,18 +883,12 @@ static hipError_t launch_share_pair(AttnArgs a, int head_dim, hipStream_t s) {
 
 hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
     a.n_split = 1; a.ws = nullptr; a.partial = 0;
-    const int64_t need = attn_decode_workspace_bytes(a.B, a.Hq, a.Sq, a.Skv, head_dim);
-    if (workspace && !a.col_sum && !a.col_sumsq && !a.probs) {
-        const bool pair = !a.noise && !a.k_norm;
-        const int64_t bytes = need > 0 ? need : pair ? attn_few_query_workspace_bytes(a.B, a.Hq, a.Hkv, a.Sq, a.Skv, head_dim) : 0;
-        if (bytes > 0 && workspace_bytes >= bytes) {
-            a.ws = static_cast<float*>(workspace);
-            if (need > 0) a.n_split = decode_splits(a.B, a.Hq, a.Skv, head_dim);
-            if (pair) {
-                const int ns = pair_shares(a.B * a.Hq, a.B * a.Hkv, a.Skv, head_dim);
-                a.n_split = need > 0 ? min(a.n_split, ns) : ns;
-                return launch_share_pair(a, head_dim, stream);
-            }
+    if (workspace && a.Sq <= 32 && !a.col_sum && !a.col_sumsq && !a.probs && !a.k_norm) {
+        const int64_t need = attn_decode_workspace_bytes(a.B, a.Hq, a.Sq, a.Skv, head_dim);
+        const int ns = a.noise ? decode_splits(a.B * a.Hq, a.Skv) : few_query_shares(a.B * a.Hq, a.B * a.Hkv, a.Skv, head_dim);
+        if (ns > 1 && workspace_bytes >= (need > 0 ? need : split_bytes((int64_t)a.B * a.Hq, ns, head_dim))) {
+            a.n_split = ns; a.ws = static_cast<float*>(workspace);
+            if (!a.noise) return launch_share_pair(a, head_dim, stream);
         }
     }
     const int stat_shares = workspace && (a.col_sum || a.col_sumsq) && !a.probs && !a.k_norm ?
