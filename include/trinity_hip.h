@@ -130,7 +130,9 @@ int trn_attn_qknorm_f16(const trn_attn_desc* desc, const void* q, const void* k,
  * arrival counters) live in the workspace; for every other shape but the chunks below, or with workspace == NULL or too
  * small, the call is exactly trn_attn_fwd_f16.
  *   workspace        device memory, 256-byte aligned, trn_attn_workspace_bytes(desc) bytes, zero-filled ONCE before
- *                    its first use (the kernel returns its counters to zero).  One call at a time may use it.
+ *                    its first use (the kernel returns its counters to zero).  One call at a time may use it.  The shares'
+ *                    results lie behind the counters of the batch x n_q_heads heads, so that problems with more heads need
+ *                    one of their own (or a fresh zero-fill).
  * trn_attn_workspace_bytes returns 0 when the shape would not use a workspace.
  *
  * A chunk of more than 32 queries per head on a long cache has a workspace of its own, trn_attn_chunk_workspace_bytes(desc)

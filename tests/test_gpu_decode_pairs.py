@@ -40,7 +40,8 @@ def test_keys_shared_out_in_two_launches(B, Hq, Hkv, Sq, Skv, D, causal, shared)
     lse, lse1 = torch.zeros(B, Hq, Sq, device="cuda"), torch.zeros(B, Hq, Sq, device="cuda")
     ops.attention(q, k, v, o[:, :, :Sq], scale, causal, lse=lse, workspace=ws)
     ops.attention(q, k, v, plain, scale, causal, lse=lse1)
-    assert (ws[:256] == 255).all() and (ws[max(need, 1024):] == 255).all() and (o[:, :, Sq:] == 7).all()
+    front = 512 if shared else (B * Hq + 63) // 64 * 256      # (counters of these heads; of any number in a workspace for chunks)
+    assert (ws[:front] == 255).all() and (ws[max(need, 1024):] == 255).all() and (o[:, :, Sq:] == 7).all()
     assert (ws[512:need] != 255).any() == (shared is not False)
     small = torch.full((max(need - 256, 256),), 255, dtype=torch.uint8, device="cuda")
     again = torch.empty_like(q)
@@ -105,3 +106,30 @@ def test_what_the_workspace_held_before_does_not_matter(B, H, Sq, Skv, causal):
         if need > 0:                                    # (the library's own serves the same shares)
             first = first or (o, lse)
             assert torch.equal(o, first[0]) and torch.equal(lse, first[1]), how
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_one_workspace_for_counters_and_chunks(D):
+    """One zero-filled workspace: keys shared out in two launches, then a call with noise of more heads, whose counters have to be zero still."""
+    from triton_amd import ops
+    g = torch.Generator().manual_seed(D)
+    scale = D ** -0.5
+    q, k, v = (ref.randn_half((1, 71, s, D), g).cuda() for s in (2, 8200, 8200))
+    noise = torch.randn(1, 71, 2, 8200, generator=g).cuda()
+    few = [t[:, :32, :2, :].contiguous() if t is q else t[:, :32, :3700].contiguous() for t in (q, k, v)]
+    o, o1 = torch.full_like(q, 7.0), torch.full_like(q, 7.0)
+    lse, lse1 = torch.full((1, 71, 2), 7.0, device="cuda"), torch.full((1, 71, 2), 7.0, device="cuda")
+    small = ops.attention_chunk_workspace_bytes(*few, torch.zeros_like(few[0]), scale, True)
+    big = ops.attention_workspace_bytes(q, k, v, o, scale, True)
+    assert small > 0 and big > 0
+    ws = torch.zeros(max(small, big), dtype=torch.uint8, device="cuda")
+    ops.attention(q, k, v, o, scale, True, noise=noise, tau=1.0, lse_pert=lse, workspace=ws)
+    got, alone = torch.zeros_like(few[0]), torch.zeros_like(few[0])
+    ops.attention(*few, got, scale, True, workspace=ws)
+    ops.attention(*few, alone, scale, True)
+    assert not torch.equal(got, alone) and (got.double() - alone.double()).norm() <= 8e-4 * alone.double().norm()      # (shared out)
+    assert (ws[:512] == 0).all()
+    for _ in range(2):
+        ops.attention(q, k, v, o1, scale, True, noise=noise, tau=1.0, lse_pert=lse1, workspace=ws)
+        assert torch.equal(o, o1) and torch.equal(lse, lse1)
+        o1.fill_(7.0)

@@ -469,7 +469,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     }
     if (DS == 1 && a.n_split > 1) {
         // ---- keys split over workgroups: publish (m, l, unnormalised O) of this share; the workgroup that arrives
-        // last at the head's counter merges all shares.  Workspace: [arrival counters, 256-byte aligned][bh][split]
+        // last at the head's counter merges all shares.  Workspace: [arrival counters, 256-byte aligned][bh][split] (two launches: without the counters)
         // {O as quads [D/4][32 queries][4], (m, l, m2, l2) [32]} floats.  The shares travel as device-scope atomic stores and loads, which
         // go to the memory all L2 slices agree on (a fence that makes ordinary stores visible writes back and
         // invalidates a whole L2, and with one per wave that took several times the kernel's own time); the arrival
@@ -477,7 +477,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         constexpr int PART = 32 * (D + 4);
         const int n_bh = a.B * a.Hq;
         unsigned* counters = reinterpret_cast<unsigned*>(a.ws);
-        float* parts = a.ws + ((n_bh + 63) / 64) * 64;
+        float* parts = a.partial ? a.ws : a.ws + ((n_bh + 63) / 64) * 64;
         const bool query = q < a.Sq;
         if (a.partial) {                       // (the merge is the next launch's: ordinary stores)
             float* p = parts + ((int64_t)bh * a.n_split + split) * PART;
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         // ---- the launch behind a.partial: every workgroup of a head merges the row normalisers of all its shares, each a
         // part of the output columns, and sweeps over its own share of the keys below
         constexpr int PART = 32 * (D + 4), BATCH = 8;
-        const float* parts = a.ws + ((a.B * a.Hq + 63) / 64) * 64 + (int64_t)bh * a.n_split * PART;
+        const float* parts = a.ws + (int64_t)bh * a.n_split * PART;
         const int quads = (D / 4 + a.n_split - 1) / a.n_split, quad = split * quads + dg;     // at most 16: two shares or more
         const bool merges = dg < quads && quad < D / 4;
         const float* op = parts + (min(quad, D / 4 - 1) * 32 + q) * 4;
@@ -715,8 +715,10 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #endif
 }
 
-// Arrival counters and the shares' partial results.
-static int64_t split_bytes(int64_t n_bh, int ns, int head_dim) { return ns <= 1 ? 0 : ((n_bh + 63) / 64) * 256 + n_bh * ns * 32 * (head_dim + 4) * 4; }
+// Arrival counters, and the shares' partial results behind them.
+static int64_t counter_bytes(int64_t n_bh) { return (n_bh + 63) / 64 * 256; }
+static int64_t share_bytes(int64_t n_bh, int ns, int head_dim) { return n_bh * ns * 32 * (head_dim + 4) * 4; }
+static int64_t split_bytes(int64_t n_bh, int ns, int head_dim) { return ns <= 1 ? 0 : counter_bytes(n_bh) + share_bytes(n_bh, ns, head_dim); }
 int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim) {
     if (seq_q > 32) return 0;
     const int ns = decode_splits(batch * n_q_heads, seq_kv);
@@ -725,10 +727,13 @@ int64_t attn_decode_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq
     return split_bytes(n_bh, ns, head_dim);
 }
 
-// The shares' partial results alone, of two launches below that rule's lines.
+// The shares' partial results alone, of two launches below that rule's lines: behind as many bytes as the counters of any number of heads that has
+// some take, so that a workspace with counters in it serves these calls too.
+constexpr int kCounterRoom = 512;
 int64_t attn_few_query_workspace_bytes(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim) {
     if (seq_q > 32 || decode_splits(batch * n_q_heads, seq_kv) > 1) return 0;
-    return split_bytes((int64_t)batch * n_q_heads, few_query_shares(batch * n_q_heads, batch * n_kv_heads, seq_kv, head_dim), head_dim);
+    const int ns = few_query_shares(batch * n_q_heads, batch * n_kv_heads, seq_kv, head_dim);
+    return ns > 1 ? kCounterRoom + share_bytes((int64_t)batch * n_q_heads, ns, head_dim) : 0;
 }
 
 // Column shares of a head for `units` = heads x query tiles: as many as leave 32 columns per workgroup and at most one
@@ -841,7 +846,7 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(const AttnArgs a
     constexpr int PART = 32 * (D + 4), BATCH = 8;
     const int bh = blockIdx.x / (D / 32), q = threadIdx.x & 31, quad = (int)(blockIdx.x % (D / 32)) * 8 + (threadIdx.x >> 5);
     if (q >= a.Sq) return;
-    const float* const parts = a.ws + ((a.B * a.Hq + 63) / 64) * 64 + (int64_t)bh * a.n_split * PART;
+    const float* const parts = a.ws + (int64_t)bh * a.n_split * PART;
     float m = -INFINITY, l = 0.f;
     float4_t o = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < a.n_split; s0 += BATCH) {
@@ -872,8 +877,8 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(const AttnArgs a
     *reinterpret_cast<half4_t*>(orow + 4 * quad) = half4_t{(half_t)(o[0] * inv), (half_t)(o[1] * inv), (half_t)(o[2] * inv), (half_t)(o[3] * inv)};
     if (quad == 0 && a.lse) a.lse[(int64_t)bh * a.Sq + q] = (m + fast_log2(l)) * kLn2;
 }
-static hipError_t launch_share_pair(AttnArgs a, int head_dim, hipStream_t s) {
-    a.n_qtiles = 1; a.partial = 2;
+static hipError_t launch_share_pair(AttnArgs a, int64_t at, int head_dim, hipStream_t s) {      // at: byte of the workspace from which on the shares' results lie
+    a.n_qtiles = 1; a.partial = 2; a.ws += at / 4;
     const dim3 g((unsigned)(a.B * a.Hq * a.n_split)), t(DNW * 64), m((unsigned)(a.B * a.Hq * head_dim / 32));
     if (head_dim == 128) hipLaunchKernelGGL((attn_decode_kernel<128, 1, 0>), g, t, 0, s, a); else hipLaunchKernelGGL((attn_decode_kernel<64, 1, 0>), g, t, 0, s, a);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
@@ -883,19 +888,23 @@ static hipError_t launch_share_pair(AttnArgs a, int head_dim, hipStream_t s) {
 
 hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
     a.n_split = 1; a.ws = nullptr; a.partial = 0;
+    const int64_t counters = counter_bytes((int64_t)a.B * a.Hq);
     if (workspace && a.Sq <= 32 && !a.col_sum && !a.col_sumsq && !a.probs && !a.k_norm) {
-        const int64_t need = attn_decode_workspace_bytes(a.B, a.Hq, a.Sq, a.Skv, head_dim);
-        const int ns = a.noise ? decode_splits(a.B * a.Hq, a.Skv) : few_query_shares(a.B * a.Hq, a.B * a.Hkv, a.Skv, head_dim);
-        if (ns > 1 && workspace_bytes >= (need > 0 ? need : split_bytes((int64_t)a.B * a.Hq, ns, head_dim))) {
-            a.n_split = ns; a.ws = static_cast<float*>(workspace);
-            if (!a.noise) return launch_share_pair(a, head_dim, stream);
+        const int64_t own = attn_decode_workspace_bytes(a.B, a.Hq, a.Sq, a.Skv, head_dim);
+        const int64_t need = own > 0 ? own : a.noise ? 0 : attn_few_query_workspace_bytes(a.B, a.Hq, a.Hkv, a.Sq, a.Skv, head_dim);
+        if (need > 0 && workspace_bytes >= need) {
+            a.ws = static_cast<float*>(workspace);
+            if (!a.noise) {
+                a.n_split = few_query_shares(a.B * a.Hq, a.B * a.Hkv, a.Skv, head_dim);
+                if (a.n_split > 1) return launch_share_pair(a, own > 0 ? counters : kCounterRoom, head_dim, stream);
+            } else a.n_split = decode_splits(a.B * a.Hq, a.Skv);
         }
     }
     const int stat_shares = workspace && (a.col_sum || a.col_sumsq) && !a.probs && !a.k_norm ?
         attn_decode_stat_shares(a.B, a.Hq, a.Hkv, a.Sq, a.Skv, head_dim, a.noise != nullptr, workspace_bytes) : 0;
     if (a.mean_std && stat_shares == 0) return hipErrorInvalidValue;      // (the single launch has the sums only)
     if (stat_shares > 0) {
-        a.n_split = stat_shares; a.ws = static_cast<float*>(workspace); a.partial = 1; a.n_qtiles = 1;
+        a.n_split = stat_shares; a.ws = static_cast<float*>(workspace) + counters / 4; a.partial = 1; a.n_qtiles = 1;
         const dim3 g((unsigned)(a.B * a.Hq * stat_shares)), t(DNW * 64);
         const int nz = !a.noise ? 0 : a.n16 ? 2 : 1;
 #define TRN_DEC_PAIR(D_, N_) do { hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_>), g, t, 0, stream, a); hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_ + 8>), g, t, 0, stream, a); } while (0)
