@@ -133,3 +133,33 @@ def test_one_workspace_for_counters_and_chunks(D):
         ops.attention(q, k, v, o1, scale, True, noise=noise, tau=1.0, lse_pert=lse1, workspace=ws)
         assert torch.equal(o, o1) and torch.equal(lse, lse1)
         o1.fill_(7.0)
+
+
+# 2245 and 4100 keys: shares of 288 (the last of 5) and of 320 (of 260); 8200 of 64 with its own workspace, shares of 1056
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D", [(1, 32, 8, 17, 2245, 128), (1, 8, 2, 32, 4100, 128), (1, 16, 16, 1, 2400, 64), (1, 71, 1, 5, 8200, 64)])
+@pytest.mark.parametrize("first,last", [(0, None), (0, 400), (1056, 2200), (-3, None), (-300, None)])
+def test_scores_that_are_no_numbers(B, Hq, Hkv, Sq, Skv, D, first, last):
+    """NaN keys in a part of a share, in a whole one and in several, and a NaN query: the same outputs and normalisers are NaN as without shares."""
+    from triton_amd import ops
+    g = torch.Generator().manual_seed(Skv)
+    q, k, v = (ref.randn_half((B, h, s, D), g).cuda() for h, s in ((Hq, Sq), (Hkv, Skv), (Hkv, Skv)))
+    k[:, 0, first:last] = float("nan")
+    q[:, -1, Sq // 2] = float("nan")
+    scale, outs = D ** -0.5, []
+    need = max(ops.attention_workspace_bytes(q, k, v, q, scale, True), ops.attention_chunk_workspace_bytes(q, k, v, q, scale, True))
+    assert need > 0
+    for ws in (None, torch.zeros(need, dtype=torch.uint8, device="cuda")):
+        o, lse = torch.full_like(q, 7.0), torch.full((B, Hq, Sq), 7.0, device="cuda")
+        ops.attention(q, k, v, o, scale, True, lse=lse, workspace=ws)
+        outs.append((o, lse))
+    (o1, l1), (o2, l2) = outs
+    visible = torch.arange(Skv, device="cuda")[None] <= torch.arange(Sq, device="cuda")[:, None] + Skv - Sq
+    poisoned = torch.zeros(Skv, dtype=torch.bool, device="cuda")
+    poisoned[first:last] = True
+    rows = torch.zeros(B, Hq, Sq, dtype=torch.bool, device="cuda")
+    rows[:, :Hq // Hkv] = (visible & poisoned).any(1)
+    rows[:, -1, Sq // 2] = True
+    assert torch.equal(o1.isnan().all(3), rows) and torch.equal(l1.isnan(), rows)
+    assert torch.equal(o1.isnan(), o2.isnan()) and torch.equal(l1.isnan(), l2.isnan())
+    d = (o1 - o2)[~rows].double()
+    assert d.norm() <= 8e-4 * o1[~rows].double().norm() and ((l1 - l2)[~rows].abs() <= 1.24e-4).all()      # (twice the distance of each from float64)

@@ -864,8 +864,9 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(const AttnArgs a
         l *= wa; o *= wa; m = top;
 #pragma unroll
         for (int u = 0; u < BATCH; ++u) {
-            if (s0 + u < a.n_split && st[u][0] > -INFINITY) {            // (-inf: a share that saw no key of this query)
-                const float w = fast_exp2(st[u][0] - top);
+            if (s0 + u < a.n_split) {
+                // (-inf: a share that saw no key of this query, whose sums are zero, or nothing but NaN scores, whose sums are that)
+                const float w = st[u][0] > -INFINITY ? fast_exp2(st[u][0] - top) : 0.f;
                 l = __builtin_fmaf(st[u][1], w, l);
                 o += d[u] * w;
             }
