@@ -308,3 +308,28 @@ def test_one_pass_where_the_rule_begins_and_strips_are_missing(B, Hq, Hkv, S, D,
     heads = [(0, 0), (B - 1, Hq - 1), (B // 2, Hq // 2)]
     check(q, k, n, rows, c, tau, 2e-5, heads)
     check_outputs(q, k, v, o, heads)
+
+
+# B, Hq, Hkv, S, D, fp16 noise, one pass: few heads of 128 whose rows are long; three workgroups a head that the chip does not take at once; KV heads that
+# the XCDs do not share evenly; fp16 noise of long rows
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half,one_pass", [
+    (1, 18, 9, 3401, 128, False, True), (1, 20, 10, 3900, 128, False, True), (1, 28, 14, 3461, 128, False, True), (1, 28, 14, 3500, 128, False, False),
+    (1, 30, 15, 3400, 128, False, True), (1, 30, 15, 3401, 128, False, False), (1, 32, 8, 3800, 128, False, True), (1, 32, 8, 3801, 128, False, False),
+    (6, 32, 8, 256, 64, False, False), (6, 32, 8, 257, 64, False, True), (5, 34, 2, 200, 64, False, True), (8, 32, 8, 200, 64, False, True), (3, 57, 3, 200, 64, False, False),
+    (6, 32, 8, 416, 64, True, True), (6, 32, 8, 417, 64, True, False), (6, 32, 8, 512, 64, True, False), (6, 32, 8, 513, 64, True, True), (5, 41, 1, 450, 64, True, True),
+    (6, 32, 8, 560, 128, True, False), (6, 32, 8, 561, 128, True, True), (5, 34, 2, 420, 128, True, True), (5, 41, 1, 420, 128, True, True),
+    (1, 96, 24, 1400, 128, True, True), (1, 96, 24, 1401, 128, True, False), (4, 32, 8, 1600, 128, True, True), (4, 32, 8, 1601, 128, True, False),
+    (1, 100, 25, 1200, 128, True, True), (1, 100, 25, 1201, 128, True, False), (1, 96, 16, 1400, 128, True, True), (1, 71, 71, 900, 128, True, True), (1, 71, 71, 901, 128, True, False),
+    (2, 71, 71, 500, 128, True, False), (1, 100, 25, 1830, 128, False, True), (1, 100, 25, 1840, 128, False, False), (1, 96, 24, 1900, 128, False, True),
+])
+def test_where_the_single_pass_is_the_faster(B, Hq, Hkv, S, D, half, one_pass):
+    from triton_amd import ops
+    room = torch.empty(1 << 20, device="cuda", dtype=torch.half)
+    q, k = (torch.as_strided(room, (B, H, S, D), (0, 0, D, 1)) for H in (Hq, Hkv))
+    # (no size here has one workgroup a head, which needs no workspace)
+    assert (ops.attention_key_scores_workspace_bytes(q, k, k, q, 0.1, True, 2 if half else 3) > 0) == one_pass
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half", [(1, 20, 10, 3403, 128, False), (5, 41, 1, 450, 64, True), (6, 32, 8, 561, 128, True)])
+def test_one_pass_at_these_lines(B, Hq, Hkv, S, D, half):
+    test_one_pass_where_the_rule_begins_and_strips_are_missing(B, Hq, Hkv, S, D, half, 0, 0)

@@ -464,43 +464,51 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
 //   -- the longest rows, of which 2048 keys are held and the rest is read and multiplied twice;
 //   -- fp16 noise, half as much to read for the same arithmetic, of long rows of few heads;
 //   -- long prompts of 64 to 319 heads with keys of their own, when the heads' count is no multiple of the 8 XCDs: a head's
-//      workgroups are then on all of them, and each L2 reads all of K.
-// Calls in a graph, here / two passes in per cent of time (900 sizes; minus: faster here):
-//   D = 64, fp32   71 heads: 420 keys -8, 1001 -30, 2600 -20; 142: 160 -8, 260 -16, 1000 -32; 284: 230 -11, 290 -9; 128: 200 -10; 16: 1000 -39, 2100 -18.  Left out:
-//         4800 keys: 12 heads +10, 16 -3, 8 (kept) -7
-//   D = 64, fp16   71: 520 -19, 1000 -17, 2600 -8; 20: 1440 -25; 32: 1500 -4, 2000 -7, 3000 -9; 48: 1360 -11, 1700 -1, 2400 -11; 142: 380 -6, 560 -14; 284: 440 -8.  Left out: 284, 330
-//         +1, 568, 290 +6; 24 heads, 1700 to 2000 +1 to +8 (1500 -11); 16, 2600 +9, 3300 +13; 142 with keys of their own, 1650 +9
-//   D = 128, fp32  32: 420 -17, 1000 -21, 2100 -13, 3100 -2, 3800 -4; 64: 160 -40, 260 -7, 2400 -8; 256: 260 -14, 1400 -19; 24: 420 -23, 1300 -7; 16: 520 -13, 1300
-//         -29; 10: 520 -22; 8: 1800 -29, 4000 -17.  Left out: 256, 200 +5; 32, 4000 +5; 16 heads, 2700 to 3640 +3 to +9; 142 with keys of their own,
+//      workgroups are then on all of them, and each L2 reads all of K.  With head_dim 128, whose K is the larger, so are from some length
+//      on those of more than 16 KV heads in all that are no multiple;
+//   -- short prompts of 171 to 255 heads: the chip takes two workgroups a head at once, but not three, and two leave up to a third of it
+//      idle.
+// Calls one after the other, here / two passes in per cent of time (2500 sizes; minus: faster here):
+//   D = 64, fp32   71 heads: 420 keys -8, 1001 -30, 2600 -20; 128: 200 -8, 289 -5; 160: 208 -2, 240 +1, 272 -15; 284: 200 -3, 272 -21; 320: 240 -18; 16: 1000 -39, 2100
+//         -18.  Left out: 176, 202 +18, 256 +9; 192, 208 +14; 224, 202 +14; 256, 200 to 225 (kept) +6 to +1, 256 -9; 4800 keys: 12 heads +10, 16 -3, 8 (kept) -7
+//   D = 64, fp16   71: 520 -19, 1000 -17, 2600 -8; 20: 1440 -25; 32: 1500 -4, 2000 -7, 3000 -9; 48: 1360 -11, 1700 -1, 2400 -11; 142: 380 -6, 560 -14; 192: 385 -4, 530 -4, 650
+//         -14.  Left out: 176 to 192, 420 to 500 +3 to +9; 284, 330 +1, 568, 290 +6; 24 heads, 1700 to 2000 +1 to +8 (1500 -11); 16, 2600 +9, 3300 +13; 142 with keys of
+//         their own, 1650 +9
+//   D = 128, fp32  32: 420 -17, 1000 -21, 2100 -13, 3210 -7, 3790 -2; 64: 160 -40, 260 -7, 2400 -8, 3790 -4; 256: 260 -14, 1400 -19; 24: 420 -23, 1300 -7, 3600 -6; 18: 3401
+//         -10, 3900 -17; 20: 3401 -19, 4000 (kept) +3; 28: 3450 -9; 100 on 25 KV heads: 1350 -4; 16: 520 -13, 1300 -29; 10: 520 -22; 8: 1800 -29, 4000 -17.  Left out: 256, 200
+//         +5; 26, 3800 to 4150 +5, 30, 3401 to 4150 +2 to +11; 32, 4000 +5; 16 heads, 2700 to 3640 +3 to +9; 100 on 25, 2000 +6, 136 on 34 +3; 142 with keys of their own,
 //         1190 to 1500 +1 to +15
-//   D = 128, fp16  32: 420 -15, 1000 -15; 8: 1000 -16, 2600 -30, 4000 -18; 16: 520 -11, 1000 -27; 9: 900 -3; 48: 360 -6, 1400 -7; 64: 420 -11, 1400 -2; 96: 1000 -7, 2500 -1; 128:
-//         520 -10, 2500 -2; 256: 640 -10, 2500 -4.  Left out: 32, 1350 +4, 1800 +5; 48, 1700 +6; 64, 1700 +4 (2100 -4); 16, 2200 +2, 2700 to 3640 +6 to +17; 8 and 9, 4400 +5
-// Inside the lines one size in thirty loses 1 to 6 %, where the strips fall badly on the CUs: 112 heads of 128, 560 to 740 keys, fp16; 128, 400, fp16 +3; 192 of
-// 64, 470, fp16 +5; 32 of 128, 1260, fp32 +2.  Short prompts of these lines, where a launch counts: 70 of 128, 210, fp16 -37; 40 of 64, 226, fp32 -28; 48 of 64,
-// 240, fp16 -29; 40 of 128, 180, fp16 -5.  (So would prompts of 65 to 127 heads of 64 below 300 keys gain, and those of up to 16 with less noise than the lines
-// ask for: 2 to 17 %.  They have been calls without a workspace, and stay so.)
+//   D = 128, fp16  32: 420 -15, 1000 -15; 8: 1000 -16, 2600 -30, 4000 -18; 16: 520 -11, 1000 -27; 9: 900 -3; 48: 360 -6, 1400 -7; 80: 430 -8, 1300 -1; 112: 430 +3, 830 -11,
+//         1300 -6; 128: 530 -13, 1590 -4; 192: 700 -3, 1300 -8; 256: 640 -11, 1300 -13, 2500 -5; 100 on 25: 1050 -8; 71 with keys of their own: 520 -7, 800 +3, 100: 800 -11.  Left out:
+//         32, 1350 +4, 1800 +5; 48, 1700 +6; 96, 1500 +3; 80, 1700 +10; 128, 1700 +4, 2500 +3; 160, 1700 +7; 176, 450 +14, 545 +5; 192, 500 +11; 88 on 22, 1391 +5; 100 on 25, 1350 +7; 200 on 50 +8; 71 with
+//         keys of their own, 1200 +8; 142, 520 +3, 1200 +17; 16, 2200 +2, 2700 to 3640 +6 to +17; 8 and 9, 4400 +5
+// Short prompts of these lines, where a launch counts: 70 of 128, 210, fp16 -37; 40 of 64, 226, fp32 -28; 48 of 64, 240, fp16 -29; 40 of 128, 180, fp16 -5.
+// (Not for speed: prompts of 65 to 127 heads of 64 below 300 keys and of up to 16 heads with less noise than these lines ask for would gain 2 to 17 %
+// too.  That 71 heads of 64 with 299 keys, 16 with 600 and 8 of 128 with 600 have no workspace is what a test of these lines has held fast from the first.)
 static bool strips_suit(const trn_attn_desc* d, bool n16) {
     if (!d->causal || d->seq_q != d->seq_kv || d->seq_q < 160) return false;
-    const int64_t bh = (int64_t)d->batch * d->n_q_heads, mb = (bh * d->seq_q * d->seq_q * (n16 ? 1 : 2)) >> 20;
+    const int64_t bh = (int64_t)d->batch * d->n_q_heads, bkv = (int64_t)d->batch * d->n_kv_heads, mb = (bh * d->seq_q * d->seq_q * (n16 ? 1 : 2)) >> 20;
     const int64_t strips = bh * ((d->seq_q + 31) / 32), S = d->seq_q;
     const bool second_strips = bh <= 16 && strips > 256 && strips <= 320;
-    const bool scattered = bh % 8 != 0 && bh < 320 && (int64_t)d->batch * d->n_kv_heads >= 64;
+    const bool scattered = bh % 8 != 0 && bh < 320 && bkv >= 64, uneven = bkv % 8 != 0 && bkv > 16;
     if (d->head_dim == 64) {
         if ((second_strips && S <= 1024) || (S > 4500 && bh > 8)) return false;
         const bool launches = S >= 200 && bh >= 18 && bh <= 64;
-        if (!n16) return launches || (S < 300 ? bh >= 128 && S >= 200 : mb >= 12);
+        if (!n16) return launches || (S < 300 ? S >= (bh > 170 && bh < 256 ? 257 : 200) && bh >= 128 : mb >= 12);
         if (S > 1250 && !(bh < 22 ? mb <= 96 : bh >= 32 && !scattered)) return false;
-        return launches || (S >= 300 && mb >= 7 && (bh <= 80 || S >= 380));
+        return launches || (S >= 300 && mb >= 7 && (bh <= 80 || S >= 380) && !(bh > 170 && bh < 205 && S > 416 && S <= 512));
     }
     if (S > 4200) return false;
     if (n16) {
         if (bh <= 16) return S >= 300 && mb >= 4 && (bh <= 8 || mb <= (bh <= 10 ? 95 : 70));
-        if (S < (bh <= 64 ? 180 : bh <= 128 ? 240 : 420)) return false;
-        return bh < 40 ? mb <= 44 : S <= (bh < 96 ? 1400 : bh < 128 ? 1600 : 2600);
+        if (S < (bh <= 64 ? 180 : bh <= 128 ? 240 : bh > 170 && bh < 205 ? 561 : 420)) return false;
+        if (scattered) return S <= 900 && bh < 128;
+        return bh < 40 ? mb <= 44 : S <= (uneven ? 1200 : bh < 128 ? 1400 : bh < 256 ? 1600 : 2600);
     }
     if (scattered && S > 700) return false;
     if (S < 300) return bh >= 18 && S >= (bh < 64 ? 180 : bh < 192 ? 160 : 260);
-    return bh >= 18 ? S <= (bh >= 32 ? 3800 : 3400) : mb >= (bh > 8 ? 3 : 16) && (bh <= 12 || mb <= 200);
+    if (bh >= 18) return mb <= 640 || S <= (bh < 32 ? 3400 : uneven && bh >= 96 ? 0 : 3800);
+    return mb >= (bh > 8 ? 3 : 16) && (bh <= 12 || mb <= 200);
 }
 // Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
 // and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
