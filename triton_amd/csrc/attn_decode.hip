@@ -41,11 +41,13 @@ template <int DV> __device__ __forceinline__ int swzv(int r) {
 // decode steps with 8 / 32 new tokens, us, sweep -> kept, 71 heads of 64 with fp16 noise: 200 keys 31.5 -> 30.2 / 35.3 -> 33.4,
 // 1000 keys 37.1 -> 35.6 / 42.7 -> 40.0; 8 heads of 128: 15.1 -> 13.7 / 18.5 -> 16.0, 18.7 -> 17.4 / 22.2 -> 19.8; without noise
 // 200 keys 14.2 -> 13.4 / 16.6 -> 14.9, but 71 heads and 1000 keys 34.7 -> 35.3 / 37.9 -> 38.4.
+// 7: as 0, a workgroup one of n_split key shares, whose results the next launch merges.  (A form of its own: beside the unsplit one in
+// the same kernel it cost that 0.1 of 4.3 us, 20 to 180 heads of 64, 30 tokens.)
 constexpr int kept_blocks(int d, int ds, bool noise) { return !noise ? 2 : d == 128 && ds == 1 ? 3 : 6; }
 template <int D, int DS, int NZ>
 __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)   // buffer descriptors and LDS-load builtins exist in the device pass only
-    constexpr bool SWEEP = NZ >= 8, KEEP = NZ >= 4 && !SWEEP, NOISE = NZ % 4 == 1 || NZ % 4 == 2, N16 = NZ % 4 == 2, KNORM = NZ == 3;
+    constexpr bool SWEEP = NZ >= 8, PARTS = NZ == 7, KEEP = NZ >= 4 && !PARTS && !SWEEP, NOISE = NZ % 4 == 1 || NZ % 4 == 2, N16 = NZ % 4 == 2, KNORM = NZ == 3;
     constexpr int DV = D / DS;    // columns of V / O this workgroup owns
     constexpr int NS = D / 16;    // k-steps of S^T = K Q^T
     constexpr int NSV = DV / 16;  // (2 key halves) x (DV/32) MFMAs of P V
@@ -75,6 +77,10 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     // ids are 8 apart, so that they sit on one XCD (ids are dealt to the 8 XCDs in turn) and share its L2.
     // So do the query tiles of a head, unless they are spread (decode_spread()); the last ones, with the most keys under a
     // causal mask, come first.
+    // (the arguments of the start in one go: by itself the compiler asks for them where they are first needed, three memory latencies in a
+    // row, of which divisions by the number of heads once hid one.  us, with the divisions / without / so: 8 heads of 64, 100 tokens 3.98 /
+    // 4.23 / 3.90, 66, 30 tokens 4.20 / 4.45 / 4.16)
+    asm volatile("" : : "s"(a.q), "s"(a.qb), "s"(a.q_norm), "s"(a.spread));
     int j, split = 0, dsl = 0, q0 = 0;
     const int BH = a.heads.all.d;
     if (a.n_qtiles > 1) {
@@ -93,7 +99,8 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         j = grp * 8 + rem % 8; dsl = rem / 8;
         if (j >= BH) return;
     } else {
-        j = blockIdx.x / a.n_split; split = blockIdx.x % a.n_split;
+        j = blockIdx.x;
+        if constexpr (PARTS || NOISE || SWEEP) { j = blockIdx.x / a.n_split; split = blockIdx.x % a.n_split; }
     }
     int b, kvh, g;
     a.heads.find(j, b, kvh, g);
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
     // this workgroup's blocks: a contiguous share of the keys when they are split over several workgroups
     int visible = a.Skv;                                // keys that some query of the tile sees
     if (a.causal) visible = min(visible, min(q0 + 31, a.Sq - 1) + off + 1);
-    const int nblk_all = (visible + 31) / 32, bps = (nblk_all + a.n_split - 1) / a.n_split;
+    const int nblk_all = (visible + 31) / 32, bps = PARTS || NOISE || SWEEP ? (nblk_all + a.n_split - 1) / a.n_split : nblk_all;
     const int blk0 = split * bps, nblk = max(0, min(nblk_all, blk0 + bps) - blk0);
     const int nmine = nblk > wave ? (nblk - wave + DNW - 1) / DNW : 0;          // blocks blk0 + wave, + 8, ...
     half8_t ka0[NS], ka1[NS];
@@ -467,9 +474,9 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
 #pragma unroll
         for (int w = 0; w < DNW; ++w) L2 += ms2 == -INFINITY ? 0.f : st_l2[w][q] * fast_exp2(st_m2[w][q] - ms2);
     }
-    if (DS == 1 && a.n_split > 1) {
-        // ---- keys split over workgroups: publish (m, l, unnormalised O) of this share; the workgroup that arrives
-        // last at the head's counter merges all shares.  Workspace: [arrival counters, 256-byte aligned][bh][split] (two launches: without the counters)
+    if (DS == 1 && (PARTS || (NOISE && !KEEP && a.n_split > 1))) {
+        // ---- keys split over workgroups: publish (m, l, unnormalised O) of this share; the next launch merges all shares or, in one launch
+        // with score perturbation, the workgroup that arrives last at the head's counter.  Workspace: [arrival counters, 256-byte aligned][bh][split] (two launches: without the counters)
         // {O as quads [D/4][32 queries][4], (m, l, m2, l2) [32]} floats.  The shares travel as device-scope atomic stores and loads, which
         // go to the memory all L2 slices agree on (a fence that makes ordinary stores visible writes back and
         // invalidates a whole L2, and with one per wave that took several times the kernel's own time); the arrival
@@ -477,9 +484,9 @@ __global__ __launch_bounds__(DNW * 64, 1) void attn_decode_kernel(const AttnArgs
         constexpr int PART = 32 * (D + 4);
         const int n_bh = a.B * a.Hq;
         unsigned* counters = reinterpret_cast<unsigned*>(a.ws);
-        float* parts = a.partial ? a.ws : a.ws + ((n_bh + 63) / 64) * 64;
+        float* parts = !NOISE || a.partial ? a.ws : a.ws + ((n_bh + 63) / 64) * 64;
         const bool query = q < a.Sq;
-        if (a.partial) {                       // (the merge is the next launch's: ordinary stores)
+        if (!NOISE || a.partial) {             // (the merge is the next launch's: ordinary stores)
             float* p = parts + ((int64_t)bh * a.n_split + split) * PART;
             if (a.partial == 2 && !query) return;
 #pragma unroll
@@ -881,7 +888,7 @@ __global__ __launch_bounds__(256) void attn_decode_merge_kernel(const AttnArgs a
 static hipError_t launch_share_pair(AttnArgs a, int64_t at, int head_dim, hipStream_t s) {      // at: byte of the workspace from which on the shares' results lie
     a.n_qtiles = 1; a.partial = 2; a.ws += at / 4;
     const dim3 g((unsigned)(a.B * a.Hq * a.n_split)), t(DNW * 64), m((unsigned)(a.B * a.Hq * head_dim / 32));
-    if (head_dim == 128) hipLaunchKernelGGL((attn_decode_kernel<128, 1, 0>), g, t, 0, s, a); else hipLaunchKernelGGL((attn_decode_kernel<64, 1, 0>), g, t, 0, s, a);
+    if (head_dim == 128) hipLaunchKernelGGL((attn_decode_kernel<128, 1, 7>), g, t, 0, s, a); else hipLaunchKernelGGL((attn_decode_kernel<64, 1, 7>), g, t, 0, s, a);
     if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     if (head_dim == 128) hipLaunchKernelGGL(attn_decode_merge_kernel<128>, m, dim3(256), 0, s, a); else hipLaunchKernelGGL(attn_decode_merge_kernel<64>, m, dim3(256), 0, s, a);
     return hipGetLastError();
@@ -908,7 +915,7 @@ hipError_t launch_attn_decode(AttnArgs a, int head_dim, void* workspace, int64_t
         a.n_split = stat_shares; a.ws = static_cast<float*>(workspace) + counters / 4; a.partial = 1; a.n_qtiles = 1;
         const dim3 g((unsigned)(a.B * a.Hq * stat_shares)), t(DNW * 64);
         const int nz = !a.noise ? 0 : a.n16 ? 2 : 1;
-#define TRN_DEC_PAIR(D_, N_) do { hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_>), g, t, 0, stream, a); hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_ + 8>), g, t, 0, stream, a); } while (0)
+#define TRN_DEC_PAIR(D_, N_) do { hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_ ? N_ : 7>), g, t, 0, stream, a); hipLaunchKernelGGL((attn_decode_kernel<D_, 1, N_ + 8>), g, t, 0, stream, a); } while (0)
         if (head_dim == 128) { if (nz == 0) TRN_DEC_PAIR(128, 0); else if (nz == 1) TRN_DEC_PAIR(128, 1); else TRN_DEC_PAIR(128, 2); }
         else { if (nz == 0) TRN_DEC_PAIR(64, 0); else if (nz == 1) TRN_DEC_PAIR(64, 1); else TRN_DEC_PAIR(64, 2); }
 #undef TRN_DEC_PAIR
@@ -986,8 +993,8 @@ extern "C" int trn_attn_fwd_noalloc_f16(const trn_attn_desc* d, const void* q, c
     void* ws = attn_static_scratch();
     if (!ws) return TRN_E_LAUNCH;
     // The array keeps whatever the last call on this device left.  The shares are rewritten by every launch before
-    // they are read; the arrival counters must start at zero, so they are cleared here (the kernel also leaves them
-    // at zero, but a launch that failed half way would not have).
+    // they are read; the arrival counters, of calls with noise, must start at zero, so they are cleared here (the kernel also
+    // leaves them at zero, but a launch that failed half way would not have).
     const int n_counters = (int)(((int64_t)d->batch * d->n_q_heads + 63) / 64) * 64;
     hipLaunchKernelGGL(fill_zero_kernel, dim3((n_counters + 255) / 256), dim3(256), 0, (hipStream_t)stream,
                        static_cast<unsigned*>(ws), n_counters);
