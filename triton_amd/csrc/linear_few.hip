@@ -183,17 +183,33 @@ __global__ __launch_bounds__(512, 2) void linear_few_kernel(const FewArgs a) {
 }
 
 // Where that is faster than two launches: up to what depth, by what a workgroup takes in beside its own panel (all of A; the second
-// panel, of which there are half as many workgroups as the two launches have).  Up to 4096 columns; us, two launches / one, forwards
-// back to back, the lower of several runs (the host's share of two launches varies from box to box, up to 2 us more):
-//   LoRA, rank 64   16 tokens: 1024 x 512 6.8 / 5.9, 1024 x 4096 7.0 / 6.0, 1280 x 2048 7.1 / 6.9, 1448 x 1024 7.4 / 7.3; but 2048 x 2048 7.8 / 8.5
-//                   32 tokens: 1024 x 512 7.5 / 7.2, 1088 x 512 7.7 / 7.5; but 24 tokens, 1280 x 2048 7.5 / 8.2
-//   rank 8 to 32    16 tokens: 256 x 256 5.9 / 3.8, 2048 x 1024 7.8 / 6.4, 3248 x 1160 12.4 / 9.9; but 4096 x 504 10.8 / 11.2
-//                   32 tokens: 1024 x 4096 7.6 / 5.8, 2048 x 4096 11.2 / 9.9; but 3000 x 2048 11.2 / 11.7, 4096 x 1024 10.9 / 11.7
-//   rank 128        16 tokens: 512 x 512 6.4 / 5.7, 704 x 4096 6.8 / 6.7; but 896 x 2048 6.9 / 7.3, 4096 x 1024 9.8 / 20.7
-//                   32 tokens: 512 x 512 7.0 / 7.1, 640 x 2048 7.2 / 7.9
-//   gated MLP       16 tokens: 1024 -> 1024 6.2 / 4.6, 1024 -> 4096 7.1 / 6.2, 1280 -> 4096 8.3 / 8.1, 1640 -> 2008 9.6 / 9.5, 1800 -> 1000 9.2 / 9.0; but 1536 ->
-//                   4096 8.9 / 9.1, 2048 -> 2048 8.9 / 9.5, 2200 -> 1000 10.2 / 10.8 (rows at odd half lines; 2400 -> 1024 7.4 / 6.8)
-//                   32 tokens: 1024 -> 4096 7.7 / 7.4, 1088 -> 2008 8.9 / 7.8, 1280 -> 1000 8.7 / 8.3; but 1200 -> 1400 7.9 / 8.6, 1280 -> 4096 8.8 / 9.5
+// panel, of which there are half as many workgroups as the two launches have).  Up to 4096 columns; us in a graph, weights from beyond the
+// L2s, tokens: depth x columns two launches / one (called one by one, the two take up to 2 us more of the host's time):
+//   LoRA, rank 33 to 64   12: 968 x 512 5.8 / 5.6, 1112 x 3712 8.1 / 7.3, 4: 1320 x 1920 8.4 / 7.8; but 12: 1096 x 384 5.8 / 6.6, 16: 1176 x 64 5.4 / 6.2
+//                         24: 600 x 768 6.0 / 5.9, 32: 1048 x 3864 10.1 / 9.6; but 24: 920 x 640 6.2 / 7.2, 1040 x 256 6.3 / 6.9
+//   rank 8 to 32          16: 256 x 256 5.9 / 3.8, 2048 x 1024 7.8 / 6.4, 3248 x 1160 12.4 / 9.9; but 8: 3104 x 72 8.3 / 9.1, 12: 2640 x 256 7.2 / 9.1
+//                         32: 1024 x 4096 7.6 / 5.8, 31: 2088 x 752 11.8 / 10.2; but 32: 1592 x 384 7.3 / 8.1, 17: 2240 x 128 6.9 / 9.0
+//   rank 65 to 128        3: 696 x 3552 7.9 / 7.7; but 12: 648 x 128 5.3 / 6.1, 16: 4096 x 1024 9.8 / 20.7; 20: 256 x 3800 7.4 / 6.6; but 17: 328 x 128 5.2 / 6.0
+//   gated MLP             4: 936 -> 1024 5.8 / 4.2, 1: 968 -> 3928 9.0 / 6.9, 9: 1336 -> 256 5.5 / 4.9; but 16: 1536 -> 4096 8.9 / 9.1
+//                         28: 1088 -> 128 5.9 / 5.3, 25: 968 -> 4008 9.7 / 8.3; but 24: 952 -> 768 6.2 / 6.9
+//                         rows that do not begin on whole lines, where few panels take in two lines a row: 4: 936 -> 240 5.2 / 4.5, 32: 720 -> 224 5.5 / 5.2;
+//                         but 1: 1056 -> 184 5.4 / 6.0, 12: 1584 -> 176 6.7 / 8.1, 8: 1504 -> 120 5.5 / 7.6, 24: 1048 -> 168 5.7 / 7.2
+// By columns up to 64, 128, 256, ... 4096; tokens up to 16, 32; rows of W at a pitch of whole lines, or not.
+static int few_depth(int64_t tokens, int64_t n, int64_t ldw, int64_t rank, bool gate) {
+    static constexpr short gated[2][7][2] = {{{1640, 1640}, {1640, 1080}, {1400, 800}, {1590, 1100}, {1340, 1260}, {1340, 1400}, {1280, 1280}},
+                                             {{1040, 1040}, {1090, 1030}, {1040, 740}, {1090, 760}, {760, 860}, {1050, 1050}, {1024, 1024}}};
+    static constexpr short r32[2][7][2] = {{{2480, 2480}, {2250, 2480}, {2250, 3584}, {2500, 3584}, {3584, 3584}, {3584, 3584}, {3584, 3584}},
+                                           {{1550, 1550}, {1400, 1690}, {1400, 1800}, {1400, 1800}, {2360, 2360}, {2360, 2360}, {2360, 2560}}};
+    static constexpr short r64[2][7][2] = {{{910, 910}, {1000, 1000}, {950, 950}, {1040, 1040}, {1070, 1300}, {1440, 1448}, {1448, 1448}},
+                                           {{430, 430}, {640, 640}, {600, 760}, {640, 640}, {600, 700}, {640, 1080}, {1050, 1050}}};
+    static constexpr short r128[2][7][2] = {{{420, 420}, {500, 500}, {500, 540}, {520, 520}, {480, 500}, {440, 600}, {560, 704}},
+                                            {{0, 0}, {0, 0}, {0, 0}, {0, 0}, {0, 280}, {0, 320}, {0, 448}}};
+    if (!gate && rank > 128) return 0;
+    int wide = 0;
+    while (wide < 6 && n > 64 << wide) ++wide;
+    return (gate ? gated : rank <= 32 ? r32 : rank <= 64 ? r64 : r128)[tokens > 16][wide][ldw % 64 != 0];
+}
+
 // More than 32 tokens are tiles of 32, of which every CU has one at most (a panel's read its weights from the same L2): the two launches then
 // take several us longer, and only all of A for a large rank makes up for it.  Ranks of up to 32 on little depth bear two a CU.
 //   LoRA, rank 8 to 24   53 tokens, 328 x 272 8.0 / 4.9; 72, 1064 x 272 11.3 / 6.1; 145, 3816 x 328 25.4 / 15.0; 401, 576 x 432 10.6 / 5.6; 76, 688 x 2064 10.9 / 6.0; two a CU:
@@ -202,16 +218,14 @@ __global__ __launch_bounds__(512, 2) void linear_few_kernel(const FewArgs a) {
 //   rank 65 to 128       52 tokens, 304 x 784 8.5 / 6.7; 180, 472 x 504 10.4 / 7.5; 149, 656 x 1160 10.9 / 9.5; but 36, 824 x 512 8.6 / 9.1, 118, 2712 x 360 16.1 / 17.8
 //   gated MLP            50 tokens, 424 -> 288 6.4 / 4.8; 88, 4000 -> 640 18.5 / 16.6; 47, 1352 -> 3024 12.9 / 10.2; 34, 4064 -> 728 17.8 / 18.6; 476, 384 -> 416 7.5 / 5.2; two a CU 365, 488 -> 608 7.7 / 8.8,
 //                        82, 1264 -> 3248 13.2 / 16.7
-static bool few_suits(int64_t tokens, int64_t hidden, int64_t n, int64_t rank, bool gate) {
+static bool few_suits(int64_t tokens, int64_t hidden, int64_t n, int64_t ldw, int64_t rank, bool gate) {
     if (n > 4096) return false;
     if (tokens > 32) {
         const int64_t tiles = (n + 511) / 512 * 16 * ((tokens + 31) / 32);      // (as launch_few() has them)
         const int64_t deep = tokens <= 64 && (gate || rank > 32) ? 3072 : 4096;
         return hidden <= deep && (tiles <= 256 ? gate || rank <= 64 || (rank <= 128 && hidden <= 704) : !gate && rank <= 32 && hidden <= 1000 && tiles <= 512);
     }
-    const bool one = tokens <= 16;
-    if (gate) return hidden <= (n <= 1024 ? (one ? 1800 : 1280) : n <= 2048 ? (one ? 1600 : 1088) : (one ? 1280 : 1024));
-    return hidden <= (rank <= 32 ? (one ? 3584 : 2560) : rank <= 64 ? (one ? 1448 : 1088) : rank <= 128 ? (one ? 704 : 448) : 0);
+    return hidden <= few_depth(tokens, n, ldw, rank, gate);
 }
 
 template <int NR, int PD, bool GATE>
@@ -237,7 +251,7 @@ extern "C" int trn_lora_f16(const void* x, int64_t tokens, int64_t hidden, int64
     if (st != TRN_OK) return st;
     st = linear_args(second, d, tokens, r, ldd, 1, w2, n2, l2, o2, p2, ad);
     if (st != TRN_OK || tokens == 0) return st;
-    if (few_suits(tokens, hidden, n, r, false)) {
+    if (few_suits(tokens, hidden, n, ldw, r, false)) {
         const FewArgs f{(const half_t*)x, (const half_t*)w, (const half_t*)a, (const half_t*)b, (half_t*)out,
                         (int)tokens, (int)hidden, (int)n, (int)r, 0, 0, ldx, ldw, lda, ldb, ldo};
         hipStream_t s = (hipStream_t)stream;
@@ -258,7 +272,7 @@ extern "C" int trn_gated_mlp_f16(const void* x, int64_t tokens, int64_t hidden, 
     if (kind != 0 && kind != 1) return TRN_E_SHAPE;
     int st = linear_args(both, x, tokens, hidden, ldx, 2, w, ns, lw, o, lo, nullptr);
     if (st != TRN_OK || tokens == 0) return st;
-    if (few_suits(tokens, hidden, n, 0, true)) {
+    if (few_suits(tokens, hidden, n, ldw1, 0, true)) {
         const FewArgs f{(const half_t*)x, (const half_t*)w1, (const half_t*)w2, nullptr, (half_t*)out,
                         (int)tokens, (int)hidden, (int)n, 0, 0, kind, ldx, ldw1, ldw2, 0, ldo};
         return launch_few<1, 4, true>(f, (hipStream_t)stream);
