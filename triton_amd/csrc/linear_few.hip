@@ -218,12 +218,15 @@ static int few_depth(int64_t tokens, int64_t n, int64_t ldw, int64_t rank, bool 
 //   rank 65 to 128       52 tokens, 304 x 784 8.5 / 6.7; 180, 472 x 504 10.4 / 7.5; 149, 656 x 1160 10.9 / 9.5; but 36, 824 x 512 8.6 / 9.1, 118, 2712 x 360 16.1 / 17.8
 //   gated MLP            50 tokens, 424 -> 288 6.4 / 4.8; 88, 4000 -> 640 18.5 / 16.6; 47, 1352 -> 3024 12.9 / 10.2; 34, 4064 -> 728 17.8 / 18.6; 476, 384 -> 416 7.5 / 5.2; two a CU 365, 488 -> 608 7.7 / 8.8,
 //                        82, 1264 -> 3248 13.2 / 16.7
+//   few columns of up to 64 tokens, where the two launches do not take longer yet: LoRA, rank 64 54, 1296 x 128 8.4 / 9.4, 43, 1552 x 320 9.4 / 10.5; rank 128 50, 688 x 320
+//                        7.9 / 8.5, 41, 552 x 1408 7.5 / 7.9; gated MLP 39, 1184 -> 144 7.1 / 8.1, 56, 1376 -> 80 7.4 / 8.5
 static bool few_suits(int64_t tokens, int64_t hidden, int64_t n, int64_t ldw, int64_t rank, bool gate) {
     if (n > 4096) return false;
     if (tokens > 32) {
         const int64_t tiles = (n + 511) / 512 * 16 * ((tokens + 31) / 32);      // (as launch_few() has them)
-        const int64_t deep = tokens <= 64 && (gate || rank > 32) ? 3072 : 4096;
-        return hidden <= deep && (tiles <= 256 ? gate || rank <= 64 || (rank <= 128 && hidden <= 704) : !gate && rank <= 32 && hidden <= 1000 && tiles <= 512);
+        int64_t deep = 4096;
+        if (tokens <= 64 && (gate || rank > 32)) deep = gate ? (n <= 256 ? 1000 : 3072) : n <= 384 ? 1100 : 3072;
+        return hidden <= deep && (tiles <= 256 ? gate || rank <= 64 || (rank <= 128 && hidden <= (tokens <= 64 ? 540 : 704)) : !gate && rank <= 32 && hidden <= 1000 && tiles <= 512);
     }
     return hidden <= few_depth(tokens, n, ldw, rank, gate);
 }
