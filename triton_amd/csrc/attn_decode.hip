@@ -817,10 +817,12 @@ static int stats_splits(int batch, int n_q_heads, int seq_q, int seq_kv, int hea
 int64_t attn_decode_stats_workspace_bytes(int batch, int n_q_heads, int seq_q, int seq_kv, int head_dim, bool noise) {
     return split_bytes((int64_t)batch * n_q_heads, stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), head_dim);
 }
-// ... that a workspace holds: with the plain attention's, as many as that has; but sixteen at most, and not many more than 192 that read keys of
-// their own, of 3 to 32 heads.  us of a decode step of one token, as many as stats_splits() / 24 / 16 / 12 / 8 / 6 / 4: KeyFormer, 8 heads of 128: 4500 keys (32) 23.1 /
-// 23.2 / 23.1 / 23.4, 10000 33.0 / 29.9 / 28.4 / 29.6, 15000 37.9 / 34.1 / 34.1 / 36.3; 16 of 64 (16): 4500 21.4 / - / - / 19.9 / 20.6, 15000 32.6 / - / - / 32.3 / 34.1; 32 of
-// 128 (8): 3200 51.0 / - / - / - / - / 47.5 / 47.0, 10000 76.0 / - / - / - / - / 73.8 / 73.4; RoCo, 8 of 128: 10000 32.6 / 29.0 / 27.2 / 28.1 / 31.3.
+// ... that a workspace holds: with the plain attention's, as many as that has; but sixteen at most -- 24 of up to 10 heads on long caches --, and not many
+// more than 192 that read keys of their own, of 3 to 32 heads.  us of a decode step of one token, as many as stats_splits() / 24 / 16 / 12 / 8 / 6 / 4: KeyFormer, 8
+// heads of 128: 4500 keys (32) 23.1 / 23.2 / 23.1 / 23.4, 10000 33.0 / 29.9 / 28.4 / 29.6, 15000 37.9 / 34.1 / 34.1 / 36.3; 16 of 64 (16): 4500 21.4 / - / - / 19.9 / 20.6, 15000
+// 32.6 / - / - / 32.3 / 34.1; 32 of 128 (8): 3200 51.0 / - / - / - / - / 47.5 / 47.0, 10000 76.0 / - / - / - / - / 73.8 / 73.4; RoCo, 8 of 128: 10000 32.6 / 29.0 / 27.2 / 28.1 / 31.3.
+// Of the two launches alone: 8 of 128 on 2, 19989 25.1 / 25.4 / 29.4 / 34.6, 5 of 128, 15891 28.7 / 29.3 / 32.2, 9 of 64 on one, 23227 25.2 / 24.4 / 28.0, 3 of 128, 11471 22.4 /
+// 21.8 / 23.4; 26 of 64, 22142 49.5 / - / - / - / 49.9 / 53.4, 28 of 64, 13191 40.1 / - / - / - / 38.5 / 42.2; 17 of 64, 21902 37.0 / - / - / 36.5 / 41.8.
 // Left out: 2 of 128, KeyFormer, 10000 22.3 / - / 23.2; 4, 15000 27.2 / - / 30.7; 40 of 64 (6 / 4 shares), 10000 45.8 / 47.5.
 int attn_decode_stat_shares(int batch, int n_q_heads, int n_kv_heads, int seq_q, int seq_kv, int head_dim, bool noise, int64_t workspace_bytes) {
     if (seq_q > 32) return 0;
@@ -828,7 +830,9 @@ int attn_decode_stat_shares(int batch, int n_q_heads, int n_kv_heads, int seq_q,
     for (const int ns : {stats_splits(batch, n_q_heads, seq_q, seq_kv, head_dim, noise), decode_splits(batch * n_q_heads, seq_kv)})
         if (ns > 1 && split_bytes((int64_t)batch * n_q_heads, ns, head_dim) <= workspace_bytes) {
             const int n_bh = batch * n_q_heads, n_bkv = batch * n_kv_heads;
-            const int cap = n_bkv > 32 || n_bh <= 2 || (n_bh <= 4 && seq_kv >= 12000) ? ns : min(16, 192 / n_bkv);
+            int cap = ns;
+            if (n_bh > 10 && n_bkv <= 32) cap = min(16, max((seq_kv >= 10000 ? 208 : 192) / n_bkv, head_dim == 64 ? 8 : 1));
+            else if (n_bh > 2 && n_bh <= 10 && (n_bh > 4 || seq_kv < 12000)) cap = seq_kv >= (n_bh <= 4 ? 9000 : 11000) ? 24 : 16;
             const int n = min(ns, cap), bps = (nblk + n - 1) / n;
             return (nblk + bps - 1) / bps;
         }
