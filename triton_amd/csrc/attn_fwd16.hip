@@ -848,12 +848,14 @@ hipError_t launch_attn_shares(const AttnArgs& a, int head_dim, hipStream_t s) {
 //   71 of 64 on one: 700 (426) 11.7 / 11.2 / 11.2, 2 x 300 (426) 9.0 / 7.8 / 7.9, 8 x 130 11.8 / 9.7 / 7.9, 4 x 400 16.2 / 13.8 / 13.5, 1600 30.7 / 29.4 / 29.2, 3600
 //     121 / 118 / 117; left out: 520 (355) 9.4 / 9.3 / 9.5, 300 (213) 7.1 / 7.2 / 7.5, 3 x 223 (426)
 //     7.7 against 7.9 of four (4 x 256 9.5 and 8.45)
-// (heads that do not fill the last workgroup leave its waves idle: a sixteenth of them at most)
+// (heads that do not fill the last workgroup leave its waves idle: a sixteenth of them at most, and hardly any of short prompts without a ragged
+// last tile to gain from: 12 groups of 21 heads of 64, 383 tokens, one head / two 11.8 / 12.7, 28 of 35 of 128, 255 50.3 / 54.7 of four)
 static int packed_heads(int batch, int n_kv_heads, int group, int seq_q, int seq_kv, int head_dim, bool causal) {
     const int64_t narrow = ((int64_t)seq_q + 127) / 128 * batch * n_kv_heads * group;
     if (!causal || seq_q != seq_kv || !(head_dim == 128 ? narrow > 512 && seq_kv <= 2048 : narrow >= (seq_q > 256 ? 400 : 512))) return 0;
     int p = 2;
-    while (p > 0 && (((int64_t)(group - 1) >> p) + 1) * 16 << p > (int64_t)group * 17) --p;
+    const int64_t part = seq_q <= 384 && (seq_q - 1) % 128 >= 96 ? 50 : 16;
+    while (p > 0 && (((int64_t)(group - 1) >> p) + 1) * part << p > (int64_t)group * (part + 1)) --p;
     return p;
 }
 
