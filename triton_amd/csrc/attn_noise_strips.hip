@@ -459,6 +459,30 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
+// and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
+// 1536 113 / 124, 2050 243 / 235; 32 of 128: 1024 48.7 / 50.3, 1501 91.6 / 89.1; 16 of 64: 1100 43.9 / 37.3, 1536 50.3 / 44.2.
+static int strip_waves(const trn_attn_desc* d) {
+    return (int64_t)d->batch * d->n_q_heads >= 32 && d->seq_q + 31 <= strip_keys(4, 128) ? 4 : 8;
+}
+
+// Workgroups per head: a workgroup's time is its start and its share of the head's strips, and the chip takes so many at once.  fill: of these places
+// in all rounds, the percentage that is taken.
+static int strip_slots(const trn_attn_desc* d, int64_t& fill) {
+    const int waves = strip_waves(d);
+    const int64_t bh = (int64_t)d->batch * d->n_q_heads, at_once = waves == 8 ? 256 : 512;
+    const int n_strips = (d->seq_q + 31) / 32;
+    const double work = 0.06 * n_strips * (n_strips + 1) + 0.7 * n_strips, start = 3.0;      // (us)
+    int best = 1;
+    double least = 1e30;
+    for (int n = 1; n <= n_strips && n <= 64; ++n) {
+        const double t = (double)((bh * n + at_once - 1) / at_once) * (start + work / n) + 0.02 * n;
+        if (t < least) { least = t; best = n; }
+    }
+    fill = bh * best * 100 / ((bh * best + at_once - 1) / at_once * at_once);
+    return best;
+}
+
 // Where this launch and the plain attention, which adds the sums of a head's workgroups, are faster than the forward with noise and the
 // column statistics: causal prompts nearly throughout, but not
 //   -- the longest rows, of which 2048 keys are held and the rest is read and multiplied twice;
@@ -467,7 +491,8 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
 //      workgroups are then on all of them, and each L2 reads all of K.  With head_dim 128, whose K is the larger, so are from some length
 //      on those of more than 16 KV heads in all that are no multiple;
 //   -- short prompts of 171 to 255 heads: the chip takes two workgroups a head at once, but not three, and two leave up to a third of it
-//      idle.
+//      idle.  With head_dim 128 and fp16 noise, where there is the least to gain, so it is with every number of 128 heads and more that leaves
+//      a fifth of the places empty (an eighth, from 256 on), and with 48 KV heads in all that are no multiple, or 64.
 // Calls one after the other, here / two passes in per cent of time (2500 sizes; minus: faster here):
 //   D = 64, fp32   71 heads: 420 keys -8, 1001 -30, 2600 -20; 128: 200 -8, 289 -5; 160: 208 -2, 240 +1, 272 -15; 284: 200 -3, 272 -21; 320: 240 -18; 16: 1000 -39, 2100
 //         -18.  Left out: 176, 202 +18, 256 +9; 192, 208 +14; 224, 202 +14; 256, 200 to 225 (kept) +6 to +1, 256 -9; 4800 keys: 12 heads +10, 16 -3, 8 (kept) -7
@@ -476,12 +501,12 @@ hipError_t launch_add_slots(const SlotSums& a, hipStream_t s) {
 //         their own, 1650 +9
 //   D = 128, fp32  32: 420 -17, 1000 -21, 2100 -13, 3210 -7, 3790 -2; 64: 160 -40, 260 -7, 2400 -8, 3790 -4; 256: 260 -14, 1400 -19; 24: 420 -23, 1300 -7, 3600 -6; 18: 3401
 //         -10, 3900 -17; 20: 3401 -19, 4000 (kept) +3; 28: 3450 -9; 100 on 25 KV heads: 1350 -4; 16: 520 -13, 1300 -29; 10: 520 -22; 8: 1800 -29, 4000 -17.  Left out: 256, 200
-//         +5; 26, 3800 to 4150 +5, 30, 3401 to 4150 +2 to +11; 32, 4000 +5; 16 heads, 2700 to 3640 +3 to +9; 100 on 25, 2000 +6, 136 on 34 +3; 142 with keys of their own,
+//         +5; 37 with keys of their own, 3777 +27, 39, 3186 +12, 40, 3648 +11, 56, 2944 +8, 34 on 17, 3619 +9; 26, 3800 to 4150 +5, 30, 3401 to 4150 +2 to +11; 32, 4000 +5; 16 heads, 2700 to 3640 +3 to +9; 100 on 25, 2000 +6, 136 on 34 +3; 142 with keys of their own,
 //         1190 to 1500 +1 to +15
 //   D = 128, fp16  32: 420 -15, 1000 -15; 8: 1000 -16, 2600 -30, 4000 -18; 16: 520 -11, 1000 -27; 9: 900 -3; 48: 360 -6, 1400 -7; 80: 430 -8, 1300 -1; 112: 430 +3, 830 -11,
-//         1300 -6; 128: 530 -13, 1590 -4; 192: 700 -3, 1300 -8; 256: 640 -11, 1300 -13, 2500 -5; 100 on 25: 1050 -8; 71 with keys of their own: 520 -7, 800 +3, 100: 800 -11.  Left out:
+//         1300 -6; 128: 530 -13, 1590 -4; 192: 700 -3, 1300 -8; 256: 640 -11, 1300 -13, 2500 -5; 155: 411 -14; 204: 650 -9; 336: 534 -8; 300: 780 -9; 480: 918 -11; 168 with keys of their own: 538 -10; 100 on 25: 1050 -8; 71 with keys of their own: 520 -7, 800 +3, 100: 800 -11.  Left out:
 //         32, 1350 +4, 1800 +5; 48, 1700 +6; 96, 1500 +3; 80, 1700 +10; 128, 1700 +4, 2500 +3; 160, 1700 +7; 176, 450 +14, 545 +5; 192, 500 +11; 88 on 22, 1391 +5; 100 on 25, 1350 +7; 200 on 50 +8; 71 with
-//         keys of their own, 1200 +8; 142, 520 +3, 1200 +17; 16, 2200 +2, 2700 to 3640 +6 to +17; 8 and 9, 4400 +5
+//         keys of their own, 1200 +8; 77, 838 +6, 95, 745 +9; 142, 520 +3, 1200 +17; 189 on 63, 941 +16; 264 on 24, 496 +13, 288, 554 +8, 312, 1223 +8, 405, 638 +8; 264 to 495 of their own +1 to +17; 16, 2200 +2, 2700 to 3640 +6 to +17; 8 and 9, 4400 +5
 // Short prompts of these lines, where a launch counts: 70 of 128, 210, fp16 -37; 40 of 64, 226, fp32 -28; 48 of 64, 240, fp16 -29; 40 of 128, 180, fp16 -5.
 // (Not for speed: prompts of 65 to 127 heads of 64 below 300 keys and of up to 16 heads with less noise than these lines ask for would gain 2 to 17 %
 // too.  That 71 heads of 64 with 299 keys, 16 with 600 and 8 of 128 with 600 have no workspace is what a test of these lines has held fast from the first.)
@@ -502,35 +527,23 @@ static bool strips_suit(const trn_attn_desc* d, bool n16) {
     if (n16) {
         if (bh <= 16) return S >= 300 && mb >= 4 && (bh <= 8 || mb <= (bh <= 10 ? 95 : 70));
         if (S < (bh <= 64 ? 180 : bh <= 128 ? 240 : bh > 170 && bh < 205 ? 561 : 420)) return false;
-        if (scattered) return S <= 900 && bh < 128;
-        return bh < 40 ? mb <= 44 : S <= (uneven ? 1200 : bh < 128 ? 1400 : bh < 256 ? 1600 : 2600);
+        if (bh < 40) return mb <= 44;
+        if (bh < 128) return S <= (scattered ? (bh < 76 ? 900 : bh < 88 ? 780 : 560) : uneven ? 1200 : 1400);
+        if (bkv >= 64) return bh % 8 == 0 && bkv % 8 == 0 && bh < 176 && S <= 1000;
+        if (bkv >= 48 && bkv % 8 != 0) return false;
+        int64_t fill;
+        strip_slots(d, fill);
+        if (bh < 256) return fill >= 80 && S <= (fill >= 99 ? 1600 : bkv < 32 ? 1300 : 900);
+        return fill >= 87 && S <= (fill >= 99 ? 2600 : 1000);
     }
     if (scattered && S > 700) return false;
     if (S < 300) return bh >= 18 && S >= (bh < 64 ? 180 : bh < 192 ? 160 : 260);
-    if (bh >= 18) return mb <= 640 || S <= (bh < 32 ? 3400 : uneven && bh >= 96 ? 0 : 3800);
+    if (bh >= 18) return mb <= 640 || (!uneven && S <= (bh < 32 ? 3400 : bh > 32 && bkv == bh ? 2500 : 3800));
     return mb >= (bh > 8 ? 3 : 16) && (bh <= 12 || mb <= 200);
 }
-// Two workgroups of four waves a CU instead of one of eight: the waves that wait for the end of a strip are then half as many,
-// and the other workgroup's go on; but 1024 held keys instead of 2048.  us, four / eight waves: 71 heads of 64: 600 33.4 / 41.0,
-// 1536 113 / 124, 2050 243 / 235; 32 of 128: 1024 48.7 / 50.3, 1501 91.6 / 89.1; 16 of 64: 1100 43.9 / 37.3, 1536 50.3 / 44.2.
-static int strip_waves(const trn_attn_desc* d) {
-    return (int64_t)d->batch * d->n_q_heads >= 32 && d->seq_q + 31 <= strip_keys(4, 128) ? 4 : 8;
-}
-
-// Workgroups per head: a workgroup's time is its start and its share of the head's strips, and the chip takes so many at once.
 int noise_strip_slots(const trn_attn_desc* d, bool n16) {
-    const int waves = strip_waves(d);
-    if (!strips_suit(d, n16) || d->seq_q + 31 > strip_keys(waves, d->head_dim)) return 0;
-    const int64_t bh = (int64_t)d->batch * d->n_q_heads, at_once = waves == 8 ? 256 : 512;
-    const int n_strips = (d->seq_q + 31) / 32;
-    const double work = 0.06 * n_strips * (n_strips + 1) + 0.7 * n_strips, start = 3.0;      // (us)
-    int best = 1;
-    double least = 1e30;
-    for (int n = 1; n <= n_strips && n <= 64; ++n) {
-        const double t = (double)((bh * n + at_once - 1) / at_once) * (start + work / n) + 0.02 * n;
-        if (t < least) { least = t; best = n; }
-    }
-    return best;
+    int64_t fill;
+    return strips_suit(d, n16) && d->seq_q + 31 <= strip_keys(strip_waves(d), d->head_dim) ? strip_slots(d, fill) : 0;
 }
 
 // A head's strips are dealt to its workgroups in rounds of n_slots, in turns of direction.  Where the last round is not full, strips
