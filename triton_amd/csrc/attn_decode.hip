@@ -1000,9 +1000,11 @@ extern "C" int trn_attn_fwd_noalloc_f16(const trn_attn_desc* d, const void* q, c
     // The array keeps whatever the last call on this device left.  The shares are rewritten by every launch before
     // they are read; the arrival counters, of calls with noise, must start at zero, so they are cleared here (the kernel also
     // leaves them at zero, but a launch that failed half way would not have).
-    const int n_counters = (int)(((int64_t)d->batch * d->n_q_heads + 63) / 64) * 64;
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((n_counters + 255) / 256), dim3(256), 0, (hipStream_t)stream,
-                       static_cast<unsigned*>(ws), n_counters);
-    if (hipGetLastError() != hipSuccess) return TRN_E_LAUNCH;
+    if (noise) {
+        const int n_counters = (int)(((int64_t)d->batch * d->n_q_heads + 63) / 64) * 64;
+        hipLaunchKernelGGL(fill_zero_kernel, dim3((n_counters + 255) / 256), dim3(256), 0, (hipStream_t)stream,
+                           static_cast<unsigned*>(ws), n_counters);
+        if (hipGetLastError() != hipSuccess) return TRN_E_LAUNCH;
+    }
     return attn_forward(d, q, k, v, o, lse, gamma_q, noise, lse_pert, ws, TRN_ATTN_NOALLOC_SCRATCH_BYTES, nullptr, nullptr, stream);
 }
