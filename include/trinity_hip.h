@@ -339,9 +339,9 @@ int trn_gate_f16(const void* c1, const void* c2, void* out, int64_t rows, int64_
 
 /*
  * LoRA (lora_benchmark.py:41-53), out = x w + (x a) b, and the gated MLP (gmlp_benchmark.py:53-64), out = gate(x w1) * (x w2), as a
- * whole: one launch for at most 32 tokens on little weight, otherwise the launches of trn_linear_f16 and trn_gate_f16 in turn, whose
- * operands, pitches, roundings and refusals these are.  d [tokens, r] and c2 [tokens, n] are scratch memory of any contents, which the single
- * launch leaves alone; kind as in trn_gate_f16.
+ * whole: one launch on little weight -- at most 32 tokens, and more in tiles of 32 as long as every compute unit has one of them, with a rank
+ * of at most 32 two --, otherwise the launches of trn_linear_f16 and trn_gate_f16 in turn, whose operands, pitches, roundings and refusals these
+ * are.  d [tokens, r] and c2 [tokens, n] are scratch memory of any contents, which may be left as they are at any size; kind as in trn_gate_f16.
  */
 int trn_lora_f16(const void* x, int64_t tokens, int64_t hidden, int64_t ldx, const void* w, int64_t n, int64_t ldw,
                  const void* a, int64_t r, int64_t lda, const void* b, int64_t ldb, void* out, int64_t ldo,

@@ -379,8 +379,8 @@ class _DecodeAppend(FusedModule):
 
     def _attend(self, q, K_cache, V_cache, O2, **kw):
         """Attention of the M new queries over the whole cache, with a workspace (allocated and zeroed once per shape;
-        every call leaves its counters at zero again) so that the keys of a head can be split over several workgroups, or
-        those of a chunk of more than 32 queries shared out over them."""
+        every call leaves its counters at zero again) so that the keys of a head can be split over several workgroups, or with
+        one for chunks, by which those of more than 32 queries, and of fewer on caches too short for the first, are shared out."""
         H, M, D = q.shape
         o = self._o_view(O2, H, M, D)
         problem = (q[None], K_cache[None], V_cache[None], o, self.scale, self.causal)
@@ -500,7 +500,7 @@ class DecodeRoCo(_DecodeAppend):
 class LoRA(FusedModule):
     """O = X W + (X A) B  (lora_benchmark.py:41-53: X [M,N], W [N,P], A [N,R], B [R,P], O [M,P]; the driver's
     intermediates C = X W, D = X A, E = D B stay inside: D is a workspace, C and E never leave the kernels).
-    Two launches: {O, D} = X {W, A}, then O = D B + O."""
+    One launch on little weight, otherwise two: {O, D} = X {W, A}, then O = D B + O."""
     TENSOR_PARAMS = ["A", "B", "O", "W", "X"]
 
     def _native(self, host, ws, A, B, O, W, X):
@@ -519,7 +519,8 @@ class LoRA(FusedModule):
 class GatedMLP(FusedModule):
     """O = gate(X W1) * (X W2)  (gmlp_benchmark.py:53-64: X [M,K], W1, W2 [K,N], O [M,N]; intermediates C1, C1_exp,
     C2).  gate = 'sigmoid' (sigmoid(C1)) or 'silu' (C1 sigmoid(C1)): the reference names the tensors and has a sigmoid
-    operator, but the IR that combines them is not in its tree.  One GEMM launch for both products, one for the gate."""
+    operator, but the IR that combines them is not in its tree.  One launch on little weight, otherwise one for both products
+    and one for the gate."""
     TENSOR_PARAMS = ["O", "W1", "W2", "X"]
 
     def __init__(self, gate: str = "sigmoid"):
