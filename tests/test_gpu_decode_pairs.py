@@ -163,3 +163,14 @@ def test_scores_that_are_no_numbers(B, Hq, Hkv, Sq, Skv, D, first, last):
     assert torch.equal(o1.isnan(), o2.isnan()) and torch.equal(l1.isnan(), l2.isnan())
     d = (o1 - o2)[~rows].double()
     assert d.norm() <= 8e-4 * o1[~rows].double().norm() and ((l1 - l2)[~rows].abs() <= 1.24e-4).all()      # (twice the distance of each from float64)
+
+
+# KV groups that the 8 XCDs do not share evenly -- two shares where there is room for three, four of six, none yet --, and long caches: B, Hq, Hkv, Sq,
+# Skv, D, causal, shared out, as above
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D,causal,shared", [
+    (1, 72, 9, 4, 3600, 64, True, True), (1, 72, 9, 4, 3599, 64, True, False), (2, 21, 3, 9, 3041, 128, False, True), (1, 42, 21, 9, 3040, 128, True, True),
+    (1, 42, 21, 9, 3039, 128, True, False), (1, 100, 25, 2, 6000, 64, True, True), (1, 100, 25, 2, 5999, 64, True, False), (1, 122, 61, 3, 8191, 128, True, False),
+    (1, 122, 61, 3, 8192, 128, True, None), (1, 38, 38, 32, 16000, 64, True, None), (1, 70, 10, 1, 10001, 64, False, None), (1, 36, 6, 17, 9000, 128, True, None),
+])
+def test_keys_of_uneven_groups(B, Hq, Hkv, Sq, Skv, D, causal, shared):
+    test_keys_shared_out_in_two_launches(B, Hq, Hkv, Sq, Skv, D, causal, shared)

@@ -171,3 +171,10 @@ def test_the_keyformer_module_shares_out_the_keys_of_few_queries(B, H, Hkv, D, S
     torch.cuda.synchronize()
     assert torch.equal(o, outs[0][0]) and torch.equal(c, outs[0][1]) and any(key[0] == "key_parts" for key in m._ws)
     assert (c - outs[1][1]).abs().max() <= 1e-4 * c.abs().max()
+
+
+# 24 shares and the 16 below that line, eight of head_dim 64, twelve on a longer cache
+@pytest.mark.parametrize("B,H,Hkv,D,Sq,Skv", [(1, 8, 2, 128, 3, 11000), (1, 10, 10, 64, 32, 10999), (1, 3, 1, 128, 2, 9001), (1, 26, 26, 64, 5, 8200), (1, 17, 17, 64, 1, 10000)])
+@pytest.mark.parametrize("noise_type", [None, torch.float16])
+def test_numbers_of_shares(B, H, Hkv, D, Sq, Skv, noise_type):
+    test_shared_out_statistics(B, H, Hkv, D, Sq, Skv, noise_type, True)

@@ -333,3 +333,18 @@ def test_where_the_single_pass_is_the_faster(B, Hq, Hkv, S, D, half, one_pass):
 @pytest.mark.parametrize("B,Hq,Hkv,S,D,half", [(1, 20, 10, 3403, 128, False), (5, 41, 1, 450, 64, True), (6, 32, 8, 561, 128, True)])
 def test_one_pass_at_these_lines(B, Hq, Hkv, S, D, half):
     test_one_pass_where_the_rule_begins_and_strips_are_missing(B, Hq, Hkv, S, D, half, 0, 0)
+
+
+# B, Hq, Hkv, S, fp16 noise, one pass, all of head_dim 128: places that stay empty, KV heads that the XCDs do not share evenly, keys of their own
+@pytest.mark.parametrize("B,Hq,Hkv,S,half,one_pass", [
+    (4, 66, 6, 496, True, False), (7, 48, 4, 534, True, True), (5, 81, 9, 638, True, False), (7, 27, 9, 941, True, False), (2, 84, 84, 538, True, True), (2, 84, 84, 1001, True, False),
+    (2, 66, 66, 538, True, False), (1, 77, 77, 780, True, True), (1, 77, 77, 781, True, False), (1, 95, 95, 560, True, True), (1, 95, 95, 561, True, False),
+    (1, 39, 39, 2900, False, True), (1, 39, 39, 3100, False, False), (1, 56, 56, 2500, False, True), (1, 56, 56, 2501, False, False),
+])
+def test_where_two_passes_are_the_faster(B, Hq, Hkv, S, half, one_pass):
+    test_where_the_single_pass_is_the_faster(B, Hq, Hkv, S, 128, half, one_pass)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,D,half", [(4, 51, 3, 650, 128, True), (1, 95, 95, 545, 128, True)])
+def test_one_pass_of_many_heads(B, Hq, Hkv, S, D, half):
+    test_one_pass_where_the_rule_begins_and_strips_are_missing(B, Hq, Hkv, S, D, half, 0, 0)

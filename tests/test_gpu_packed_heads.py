@@ -55,3 +55,9 @@ def test_norms_and_given_queries(D, B, Hq, Hkv, S):
     o.fill_(7.0)
     ops.attention_key_scores(q, k, v, o, D ** -0.5, True, torch.empty(B, Hq, S, device="cuda"), torch.empty(B, Hq, S, device="cuda"), noise=n, tau=1.0, workspace=ws)
     compare(q, k, v, o)
+
+
+# short prompts whose last tile is nearly full: odd groups a head at a time, even ones in pairs, and the sizes on either side
+@pytest.mark.parametrize("B,Hq,Hkv,S,D", [(6, 42, 2, 383, 64), (6, 42, 2, 352, 64), (4, 84, 2, 255, 128), (4, 35, 1, 256, 128), (6, 42, 2, 385, 64), (10, 35, 1, 353, 64)])
+def test_groups_with_little_to_gain(B, Hq, Hkv, S, D):
+    test_heads_that_share_a_workgroup(B, Hq, Hkv, S, D)
